@@ -161,6 +161,13 @@ int spion_pattern_generate(const float* Score, int n_maps, int seq_len, int bloc
                            int conv_ksize, int mode, double param,
                            float* Mat, float* Pooled, float* Thresh, void* stream);
 
+/* The same for maps that lie anywhere (the reference keeps one tensor per layer, models/model_transformer.py:137):
+ * Score is a HOST array of n_maps device pointers, and Mat [replicas][n_maps][nb][nb] receives the same masks
+ * `replicas` times (one copy per data-parallel replica, main_conv_ff.py:298-299). */
+int spion_pattern_generate_maps(const float* const* Score, int n_maps, int seq_len, int block_size,
+                                int conv_ksize, int mode, double param,
+                                float* Mat, int replicas, float* Pooled, float* Thresh, void* stream);
+
 /* ------------------------------------------------------------------------------------------------
  * Score map of a layer for pattern discovery: the mean of the dense phase's probability maps over the
  * batch and then over the heads -- models/model_transformer.py:136-137

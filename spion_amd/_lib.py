@@ -125,6 +125,8 @@ def core() -> ctypes.CDLL:
     lib.spion_version.argtypes = []
     lib.spion_pattern_generate.argtypes = [_P, c_int, c_int, c_int, c_int, c_int, c_double, _P, _P, _P, _P]
     lib.spion_pattern_generate.restype = c_int
+    lib.spion_pattern_generate_maps.argtypes = [_P, c_int, c_int, c_int, c_int, c_int, c_double, _P, c_int, _P, _P, _P]
+    lib.spion_pattern_generate_maps.restype = c_int
     lib.spion_score_map_mean.argtypes = [_P, c_int, c_int, c_int, c_int, _P, _P]
     lib.spion_score_map_mean.restype = c_int
     for fam, extra in (("block", 0), ("blockmask", 1)):

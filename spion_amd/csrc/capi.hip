@@ -90,6 +90,7 @@ void dense_forward(void*, const float*, const float*, const float*, const float*
 void dense_backward(void*, const float*, const float*, const float*, const float*, const float*, float*, float*,
                     float*);
 int pattern_generate(const float*, int, int, int, int, int, double, float*, float*, float*, hipStream_t);
+int pattern_generate_maps(const float* const*, int, int, int, int, int, double, float*, int, float*, float*, hipStream_t);
 int score_map_mean(const float*, int, int, int, int, float*, hipStream_t, float post = 1.0f);
 void dense_forward_strided_mean(void*, const float*, const float*, const float*, const float*, float*, float*, float*, int,
                                 const HeadLayout&, const HeadLayout&);
@@ -217,6 +218,14 @@ void spion_densemask_attn_backward(void* h, const float* Qt, const float* Kt, co
 void spion_densemask_destroy(void* h) { dense_destroy(h); }
 
 // ---- pattern discovery ---------------------------------------------------------------------------
+int spion_pattern_generate_maps(const float* const* Score, int n_maps, int seq_len, int block_size, int conv_ksize,
+                                int mode, double param, float* Mat, int replicas, float* Pooled, float* Thresh,
+                                void* stream) {
+    note_current_handle(nullptr);
+    return pattern_generate_maps(Score, n_maps, seq_len, block_size, conv_ksize, mode, param, Mat, replicas, Pooled,
+                                 Thresh, static_cast<hipStream_t>(stream));
+}
+
 int spion_pattern_generate(const float* Score, int n_maps, int seq_len, int block_size, int conv_ksize, int mode,
                            double param, float* Mat, float* Pooled, float* Thresh, void* stream) {
     note_current_handle(nullptr);

@@ -4,11 +4,13 @@
 // Restates what the reference does on the host CPU with PyTorch ops and a recursive Python function
 // (main_conv_ff.py:35-62 and :254-278; top-k variant main_conv.py:236-256; pool-only main_ff.py:253-272).
 #include "common.h"
+#include "tile_ops.h"
 #include "../../include/spion_hip.h"
 
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <vector>
 
 namespace spion {
 
@@ -16,14 +18,22 @@ constexpr int POOL_THREADS = 256;
 constexpr int WALK_THREADS = 1024;
 constexpr int POOLED_LDS = 36864;  // block grids up to 192 x 192 are walked from LDS (144 KB of the CU's 160)
 
+// The score maps of one launch, wherever they lie (the reference's attn_lst holds one tensor per layer,
+// models/model_transformer.py:137): reading them in place spares the copy that stacks them, a quarter of the whole
+// discovery at four maps of 2048 x 2048.  More maps take further launches.
+constexpr int MAPS_PER_LAUNCH = 16;
+struct ScoreMaps {
+    const float* p[MAPS_PER_LAUNCH];
+};
+
 // pooled[I][J] = (1/bs^2) sum_{i in I, j in J} sum_{t=-hk..hk} A[i+t][j+t]  (zero outside the map).
 // Regrouped per source element A[p][q]: its weight is the number of shifts t that land in the block.
 // fp64 accumulation in a fixed order, one rounding to fp32.
-__global__ __launch_bounds__(POOL_THREADS) void conv_pool_kernel(const float* __restrict__ A, float* __restrict__ pooled,
-                                                                 int L, int bs, int nb, int hk) {
+__global__ __launch_bounds__(POOL_THREADS) void conv_pool_kernel(ScoreMaps maps, float* __restrict__ pooled, int L,
+                                                                 int bs, int nb, int hk) {
     __shared__ double red[POOL_THREADS];
     const int I = blockIdx.y, J = blockIdx.x, map = blockIdx.z;
-    const float* Am = A + (size_t)map * L * L;
+    const float* Am = maps.p[map];
     const int p0 = max(0, I * bs - hk), p1 = min(L, I * bs + bs + hk);
     const int q0 = max(0, J * bs - hk), q1 = min(L, J * bs + bs + hk);
     const int w = q1 - q0, total = (p1 - p0) * w;
@@ -50,45 +60,61 @@ __global__ __launch_bounds__(POOL_THREADS) void conv_pool_kernel(const float* __
 // keeps two fp64 sums, for the column's own block and for the neighbour it reaches into; one wavefront per block
 // then adds the block's partial sums in a fixed order.  Every element is read once per block row it touches
 // ((bs + 2 hk) / bs times, the repeats from L2) instead of once per block, and in full rows.
-constexpr int CP_COLS = 256, CP_RG = 4;
-__global__ __launch_bounds__(CP_COLS* CP_RG) void conv_pool_cols_kernel(const float* __restrict__ A,
-                                                                         float* __restrict__ pooled, int L, int bs,
-                                                                         int nb, int hk, int gb) {
+// A column's filter shifts t form an interval [lo, hi]; element row dp (from the block's first row) counts for those
+// of them in [dp - bs + 1, dp], a trapezoid in dp: min(dp + 1 - lo, hi - lo + 1, hi + bs - dp), not below zero.  Small
+// whole numbers, so it is formed in fp32 (four instructions, the integer form took eight comparisons per element), and
+// for one of the two sums only: the shifts of a column's own block and of its neighbour make up all of them, so the
+// neighbour's sum is that over the full trapezoid, the same for every column and looked up per row, less the own one.
+// A batch of loads is issued before any of them is used, with the row clamped instead of a remainder loop whose loads
+// would each wait alone.  Four maps of 2048 x 2048, block 32: 52.7 -> 25.2 us.
+constexpr int CP_COLS = 256, CP_RG = 2, CP_BATCH = 16;
+__global__ __launch_bounds__(CP_COLS* CP_RG) void conv_pool_cols_kernel(ScoreMaps maps, float* __restrict__ pooled, int L,
+                                                                         int bs, int nb, int hk, int gb) {
     __shared__ double part[CP_RG][2][CP_COLS];
-    const int I = blockIdx.y, map = blockIdx.z;
-    const int Jg = blockIdx.x * gb;  // first block of this group
-    const float* Am = A + (size_t)map * L * L;
-    const int cc = threadIdx.x % CP_COLS, rg = threadIdx.x / CP_COLS;
+    __shared__ double full[CP_COLS];  // full trapezoid of row dp at [dp + hk]
+    // consecutive items -- the groups of a block row, then the next block row of the same map, whose rows overlap --
+    // run on one die, whose L2 then serves the bs + 2 hk rows' overlap
+    const int groups = (nb + gb - 1) / gb;
+    const int item = xcd_remap(blockIdx.x, gridDim.x);
+    const int I = item / groups % nb, map = item / groups / nb;
+    const int Jg = item % groups * gb;  // first block of this group
+    const float* Am = maps.p[map];
+    const int cc = threadIdx.x % CP_COLS;
+    const int rg = __builtin_amdgcn_readfirstlane((int)threadIdx.x / CP_COLS);  // a wavefront's columns share their rows
     const int ncols = gb * bs + 2 * hk;
     const int q = Jg * bs - hk + cc;
     const int p0 = max(0, I * bs - hk), p1 = min(L, I * bs + bs + hk);
-    double a0 = 0.0, a1 = 0.0;
+    const auto trapezoid = [&](float dp, float lo1, float n, float top) {
+        return fmaxf(0.f, fminf(fminf(dp + lo1, n), top - dp));
+    };
+    if ((int)threadIdx.x < bs + 2 * hk)
+        full[threadIdx.x] = (double)trapezoid((float)((int)threadIdx.x - hk), (float)(1 + hk),
+                                              (float)min(2 * hk + 1, bs), (float)(hk + bs));
+    __syncthreads();
+    double a0 = 0.0, all = 0.0;
     if (cc < ncols && q >= 0 && q < L) {
-        const int J0 = q / bs, c = q - J0 * bs;
-        int dq1 = 0;
-        bool has1 = false;
-        if (c < hk) {  // reaches into the block on the left
-            dq1 = c + bs;
-            has1 = J0 > 0;
-        } else if (c >= bs - hk) {  // ... on the right
-            dq1 = c - bs;
-            has1 = J0 + 1 < nb;
-        }
-        auto weight = [&](int dp, int dq) {  // shifts t with dp - t and dq - t inside the block
-            const int lo = max(-hk, max(dp, dq) - bs + 1), hi = min(hk, min(dp, dq));
-            return max(0, hi - lo + 1);
-        };
+        const int c = q % bs;
+        const int lo = max(-hk, c - bs + 1), hi = min(hk, c);
+        const float lo1 = (float)(1 - lo), n = (float)min(hi - lo + 1, bs), top = (float)(hi + bs);
         const float* col = Am + q;
-#pragma unroll 8
-        for (int p = p0 + rg; p < p1; p += CP_RG) {
-            const int dp = p - I * bs;
-            const double v = (double)col[(size_t)p * L];
-            a0 += v * (double)weight(dp, c);
-            if (has1) a1 += v * (double)weight(dp, dq1);
+        for (int pb = p0 + rg; pb < p1; pb += CP_RG * CP_BATCH) {
+            float v[CP_BATCH];
+#pragma unroll
+            for (int k = 0; k < CP_BATCH; ++k) v[k] = col[(size_t)min(pb + k * CP_RG, p1 - 1) * L];
+#pragma unroll
+            for (int k = 0; k < CP_BATCH; ++k) {
+                const int p = pb + k * CP_RG;
+                if (p < p1) {
+                    const int dp = p - I * bs;
+                    const double x = (double)v[k];
+                    a0 += x * (double)trapezoid((float)dp, lo1, n, top);
+                    all += x * full[dp + hk];
+                }
+            }
         }
     }
     part[rg][0][cc] = a0;
-    part[rg][1][cc] = a1;
+    part[rg][1][cc] = all - a0;
     __syncthreads();
     // wavefront b adds up block b: entries e = 0 .. CP_RG (bs + 2 hk) - 1, lane-strided, then a butterfly
     const int b = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -155,77 +181,301 @@ __device__ uint32_t block_select(const float* __restrict__ v, int N, int rank, i
     return prefix;
 }
 
-// One work-group per map.
+// Wavefront reductions and sums over the lanes below, by DPP moves (a shuffle goes through the LDS and takes its latency
+// at every one of the six steps).  The result of a reduction is in the last lane.
+template <class Op>
+__device__ __forceinline__ uint32_t dpp_scan(uint32_t v, uint32_t none, Op op) {
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x111, 0xf, 0xf, false));  // row_shr:1
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x112, 0xf, 0xf, false));  // row_shr:2
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x114, 0xf, 0xf, false));  // row_shr:4
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x118, 0xf, 0xf, false));  // row_shr:8
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return v;
+}
+__device__ __forceinline__ uint32_t wave_min_last(uint32_t v) {
+    return dpp_scan(v, 0xffffffffu, [](uint32_t a, uint32_t b) { return min(a, b); });
+}
+__device__ __forceinline__ uint32_t wave_max_last(uint32_t v) {
+    return dpp_scan(v, 0u, [](uint32_t a, uint32_t b) { return max(a, b); });
+}
+
+// f(element, index) for every i < N, four of a thread's elements loaded before the first is used.
+template <class F>
+__device__ __forceinline__ void for_elements(const float* __restrict__ v, int N, F f) {
+    for (int i0 = threadIdx.x; i0 < N; i0 += 4 * WALK_THREADS) {
+        float x[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = v[min(i0 + k * WALK_THREADS, N - 1)];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (i0 + k * WALK_THREADS < N) f(x[k], i0 + k * WALK_THREADS);
+    }
+}
+
+// Key of the element of ascending rank `rank` among v[0..N), and of rank + 1 (unspecified for the last).  The range of
+// the keys is found first and cut into 2048 equal parts: one histogram (the keys of one map share their leading bits,
+// so the digits of a plain radix pass put them all into a few bins and serialise the LDS atomics), then the elements
+// of the part the rank falls into are collected and ranked against each other.  More than SEL_CAND of them:
+// block_select over the whole map.
+constexpr int SEL_BINS = 2 * WALK_THREADS, SEL_CAND = 512;
+struct SelectSpace {
+    int bins[SEL_BINS];
+    uint32_t cand[SEL_CAND];
+    int hist[256];
+    int wave[WALK_THREADS / 64];
+    uint32_t key_min, key_max, above, key, next;
+    int part, rank, cnt, n_cand, sh[2];
+};
+struct Ranked {
+    uint32_t key, next;
+};
+__device__ Ranked range_select(const float* __restrict__ v, int N, int rank, SelectSpace& S) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t mn = 0xffffffffu, mx = 0u;
+    for_elements(v, N, [&](float x, int) {
+        const uint32_t k = float_key(x);
+        mn = min(mn, k);
+        mx = max(mx, k);
+    });
+    mn = wave_min_last(mn);
+    mx = wave_max_last(mx);
+    if (threadIdx.x == 0) {
+        S.key_min = S.above = 0xffffffffu;
+        S.key_max = 0u;
+        S.n_cand = 0;
+    }
+    reinterpret_cast<int2*>(S.bins)[threadIdx.x] = make_int2(0, 0);
+    for (int i = threadIdx.x; i < SEL_CAND; i += WALK_THREADS) S.cand[i] = 0xffffffffu;
+    __syncthreads();
+    if (lane == 63) {
+        atomicMin(&S.key_min, mn);
+        atomicMax(&S.key_max, mx);
+    }
+    __syncthreads();
+    const uint32_t kmin = S.key_min, span = S.key_max - kmin;
+    const int shift = max(0, 32 - __builtin_clz(span | 1u) - 11);  // parts of 2^shift keys
+    for_elements(v, N, [&](float x, int) { atomicAdd(&S.bins[(float_key(x) - kmin) >> shift], 1); });
+    __syncthreads();
+    const int2 b = reinterpret_cast<const int2*>(S.bins)[threadIdx.x];  // thread t owns parts 2t and 2t + 1
+    const int own = b.x + b.y;
+    const int incl = (int)dpp_scan((uint32_t)own, 0u, [](uint32_t p, uint32_t q) { return p + q; });
+    if (lane == 63) S.wave[wave] = incl;
+    __syncthreads();
+    int before = incl - own;
+    for (int w = 0; w < WALK_THREADS / 64; ++w) before += w < wave ? S.wave[w] : 0;
+    if (before <= rank && rank < before + own) {
+        const bool second = before + b.x <= rank;
+        S.part = 2 * threadIdx.x + second;
+        S.rank = rank - (second ? before + b.x : before);
+        S.cnt = second ? b.y : b.x;
+    }
+    __syncthreads();
+    const int part = S.part, r = S.rank, cnt = S.cnt;
+    if (cnt > SEL_CAND && shift > 0) {
+        const uint32_t key = block_select(v, N, rank, S.hist, S.sh);
+        if (threadIdx.x == 0) S.cnt = 0;
+        __syncthreads();
+        int c = 0;
+        mn = 0xffffffffu;
+        for_elements(v, N, [&](float x, int) {
+            const uint32_t k = float_key(x);
+            if (k <= key) ++c;
+            else mn = min(mn, k);
+        });
+        c = (int)dpp_scan((uint32_t)c, 0u, [](uint32_t p, uint32_t q) { return p + q; });
+        mn = wave_min_last(mn);
+        if (lane == 63) {
+            atomicAdd(&S.cnt, c);
+            atomicMin(&S.above, mn);
+        }
+        __syncthreads();
+        return Ranked{key, rank + 1 < S.cnt ? key : S.above};
+    }
+    mn = 0xffffffffu;  // smallest key of the parts above
+    for_elements(v, N, [&](float x, int) {
+        const uint32_t k = float_key(x) - kmin;
+        const int p = (int)(k >> shift);
+        if (p == part && shift > 0) S.cand[atomicAdd(&S.n_cand, 1)] = k;
+        if (p > part) mn = min(mn, k);
+    });
+    mn = wave_min_last(mn);
+    if (lane == 63) atomicMin(&S.above, mn);
+    __syncthreads();
+    const uint32_t above = kmin + S.above;
+    if (shift == 0) {  // a part is one key
+        const uint32_t key = kmin + (uint32_t)part;
+        return Ranked{key, r + 1 < cnt ? key : above};
+    }
+    for (int i = threadIdx.x; i < cnt; i += WALK_THREADS) {
+        const uint32_t k = S.cand[i];
+        uint32_t more = 0xffffffffu;
+        int less = 0, same = 0;
+#pragma unroll 4
+        for (int j = 0; j < cnt; j += 4) {  // the rest of the last four is the largest key
+            const uint4 o = *reinterpret_cast<const uint4*>(S.cand + j);
+            const uint32_t e[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                less += e[q] < k;
+                same += e[q] == k;
+                more = min(more, e[q] > k ? e[q] : 0xffffffffu);
+            }
+        }
+        if (less <= r && r < less + same) {  // several equal candidates write the same
+            S.key = kmin + k;
+            S.next = r + 1 < less + same ? kmin + k : more != 0xffffffffu ? kmin + more : above;
+        }
+    }
+    __syncthreads();
+    return Ranked{S.key, S.next};
+}
+
+// The move of the greedy walk at cell (x, y) (main_conv_ff.py:35-62), on the map with a row and a column of zeros
+// beyond its end.
+__device__ __forceinline__ void walk_move(const float* __restrict__ pooled, int nb, int& x, int& y) {
+    auto at = [&](int xx, int yy) -> float { return (xx < nb && yy < nb) ? pooled[xx * nb + yy] : 0.f; };
+    const float Dn = at(x + 1, y), Rt = at(x, y + 1), Dg = at(x + 1, y + 1);
+    const bool down = Dn > Rt && Dn > Dg, right = !(Dn > Rt) && Rt > Dg;
+    if (!right) ++x;
+    if (!down) ++y;
+}
+
+// torch.quantile's rank arithmetic and lerp, every step rounded to fp32 (no fused multiply-add).
+__device__ __forceinline__ float quantile_rank(float q, int N, int& lo, int& hi) {
+#pragma clang fp contract(off)
+    const float r = q * (float)(N - 1);
+    lo = (int)floorf(r);
+    hi = (int)ceilf(r);
+    return r - (float)lo;
+}
+__device__ __forceinline__ float lerp_as_torch(float a, float b, float w) {
+#pragma clang fp contract(off)
+    const float diff = b - a;
+    return w < 0.5f ? a + w * diff : b - diff * (1.0f - w);
+}
+
+// One work-group per map.  Block grids up to JUMP_NB x JUMP_NB: what a walker does at a cell depends on the cell alone,
+// so every cell's move goes into a table in LDS, the table is squared twice, and four threads take a walker's path
+// between them, each every fourth cell of it -- a quarter of up to 2 nb dependent look-ups of one word instead of that
+// many of three, with their comparisons.  (Squaring until the whole path is covered was measured: every squaring is a
+// pass over all cells, seven of them took longer than the walk they saved.)  Larger grids walk the map itself.
+// Four maps, 64 x 64 blocks: 40.5 -> 12.1 us.
+constexpr int JUMP_NB = 128;  // LDS at the limit: pooled 64 KB, two move tables 64 KB, marks 16 KB, selection 11 KB
+constexpr int MOVE_MARKS = 0x8000;  // flag of a table entry: the cell's value passes the threshold (cells need 15 bits)
 __global__ __launch_bounds__(WALK_THREADS) void threshold_walk_kernel(const float* __restrict__ pooled_all,
                                                                       float* __restrict__ mat_all,
                                                                       float* __restrict__ thresh_out, int nb, int mode,
-                                                                      float q, int topk) {
-    __shared__ int hist[256];
-    __shared__ int sh[2];
+                                                                      float q, int topk, int replicas,
+                                                                      size_t replica_stride) {
     __shared__ int s_cnt;
     __shared__ uint32_t s_min;
-    extern __shared__ float s_pooled[];  // N floats when N <= POOLED_LDS (sized by the launch)
+    __shared__ __attribute__((aligned(16))) SelectSpace sel;
+    extern __shared__ __attribute__((aligned(16))) float s_pooled[];  // N floats (N <= POOLED_LDS), then tables and marks
     const int map = blockIdx.x, N = nb * nb;
     const float* pooled = pooled_all + (size_t)map * N;
     float* mat = mat_all + (size_t)map * N;
+    const bool jump = mode == SPION_PATTERN_FLOOD && nb <= JUMP_NB;
+    unsigned short* move = reinterpret_cast<unsigned short*>(s_pooled + N);
+    unsigned short* move2 = move + N + 1;
+    unsigned char* marks = reinterpret_cast<unsigned char*>(move2 + N + 1);
 
-    for (int i = threadIdx.x; i < N; i += blockDim.x) mat[i] = 0.f;
+    if (!jump)
+        for (int i = threadIdx.x; i < N; i += blockDim.x) mat[i] = 0.f;
     if (N <= POOLED_LDS) {
         // the select passes and the walkers' dependent neighbour reads then stay in LDS
-        for (int i = threadIdx.x; i < N; i += blockDim.x) s_pooled[i] = pooled[i];
+        for_elements(pooled, N, [&](float x, int i) { s_pooled[i] = x; });
         __syncthreads();
         pooled = s_pooled;
     }
 
     if (mode == SPION_PATTERN_FLOOD) {
         // torch.quantile, linear interpolation, every step in fp32 (main_conv_ff.py:268)
-        const float r = q * (float)(N - 1);
-        const int lo = (int)floorf(r), hi = (int)ceilf(r);
-        const float wgt = r - (float)lo;
-        const uint32_t klo = block_select(pooled, N, lo, hist, sh);
-        if (threadIdx.x == 0) {
-            s_cnt = 0;
-            s_min = 0xffffffffu;
-        }
-        __syncthreads();
-        int c = 0;
-        uint32_t mn = 0xffffffffu;
-        for (int i = threadIdx.x; i < N; i += blockDim.x) {
-            uint32_t k = float_key(pooled[i]);
-            if (k <= klo) ++c;
-            else mn = min(mn, k);
-        }
-        atomicAdd(&s_cnt, c);
-        atomicMin(&s_min, mn);
-        __syncthreads();
-        const float a = key_float(klo);
-        const float b = (hi < s_cnt) ? a : key_float(s_min);  // sorted[hi]
-        const float diff = b - a;
-        float thresh;
-        if (wgt < 0.5f) thresh = a + __fmul_rn(wgt, diff);
-        else thresh = b - __fmul_rn(diff, 1.0f - wgt);
+        int lo, hi;
+        const float wgt = quantile_rank(q, N, lo, hi);
+        const Ranked k = range_select(pooled, N, lo, sel);
+        const float a = key_float(k.key);
+        const float b = hi == lo ? a : key_float(k.next);  // sorted[hi]
+        const float thresh = lerp_as_torch(a, b, wgt);
         if (threadIdx.x == 0 && thresh_out) thresh_out[map] = thresh;
-        __syncthreads();  // mat is zeroed for everyone
 
-        // greedy walks: walker k < nb starts at (0, k), walker nb + k at (k, 0)  (main_conv_ff.py:271-274)
+        // walker k < nb starts at (0, k), walker nb + k at (k, 0)  (main_conv_ff.py:271-274); the cell moved to is
+        // marked when its value exceeds the threshold, and binarised with ff_mat > 0
+        if (jump) {
+            const int dx = WALK_THREADS / nb, dy = WALK_THREADS % nb;
+            int x = threadIdx.x / nb, y = threadIdx.x % nb;
+            for (int i = threadIdx.x; i <= N; i += WALK_THREADS) {
+                int nx = x, ny = y, e = N;  // N: beyond the grid, where a walker stays
+                if (i < N) {
+                    walk_move(pooled, nb, nx, ny);
+                    if (nx < nb && ny < nb) e = nx * nb + ny;
+                    if (pooled[i] > thresh && pooled[i] > 0.f) e |= MOVE_MARKS;
+                }
+                move[i] = (unsigned short)e;
+                marks[i] = 0;
+                x += dx;
+                y += dy;
+                if (y >= nb) {
+                    y -= nb;
+                    ++x;
+                }
+            }
+            __syncthreads();
+            auto square = [&](const unsigned short* from, unsigned short* to) {
+                for (int i0 = threadIdx.x; i0 <= N; i0 += 4 * WALK_THREADS) {
+                    int e[4], m[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) e[c] = from[min(i0 + c * WALK_THREADS, N)];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) m[c] = from[e[c] & ~MOVE_MARKS];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)  // past the end: the last entry once more
+                        to[min(i0 + c * WALK_THREADS, N)] = (unsigned short)((e[c] & MOVE_MARKS) | (m[c] & ~MOVE_MARKS));
+                }
+                __syncthreads();
+            };
+            square(move, move2);
+            // threads 4w .. 4w + 3 share walker w: cells after 0, 1, 2 and 3 moves, then four moves at a time
+            const int walker = threadIdx.x >> 2, phase = threadIdx.x & 3;  // 2 nb <= WALK_THREADS / 4
+            const bool walks = walker < 2 * nb;
+            int at = walker < nb ? walker : (walker - nb) * nb, arrived = phase != 0;
+            if (!walks) at = N;
+            if (phase & 1) at = move[at] & ~MOVE_MARKS;
+            if (phase & 2) at = move2[at] & ~MOVE_MARKS;
+            __syncthreads();  // the table of single moves makes room for that of four
+            square(move2, move);
+            while (at != N) {
+                const int e = move[at];
+                if (arrived && (e & MOVE_MARKS)) marks[at] = 1;
+                arrived = 1;
+                at = e & ~MOVE_MARKS;
+            }
+            __syncthreads();
+            const bool fours = N % 4 == 0 && reinterpret_cast<size_t>(mat_all) % 16 == 0;
+            for (int i0 = 4 * threadIdx.x; i0 < N; i0 += 4 * WALK_THREADS) {
+                float o[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const int i = min(i0 + c, N);
+                    o[c] = (marks[i] || i % (nb + 1) == 0) ? 1.f : 0.f;  // the diagonal too (main_conv_ff.py:277-278)
+                }
+                for (int rep = 0; rep < replicas; ++rep) {
+                    float* m = mat + rep * replica_stride + i0;
+                    if (fours) {
+                        *reinterpret_cast<float4*>(m) = make_float4(o[0], o[1], o[2], o[3]);
+                    } else {
+                        for (int c = 0; c < 4 && i0 + c < N; ++c) m[c] = o[c];
+                    }
+                }
+            }
+            return;
+        }
+        __syncthreads();  // mat is zeroed for everyone
         for (int wk = threadIdx.x; wk < 2 * nb; wk += blockDim.x) {
             int x = wk < nb ? 0 : wk - nb, y = wk < nb ? wk : 0;
-            auto at = [&](int xx, int yy) -> float { return (xx < nb && yy < nb) ? pooled[xx * nb + yy] : 0.f; };
-            while (x < nb && y < nb) {  // x+1 != nb+1 and y+1 != nb+1 on the sentinel-padded map
-                const float Dn = at(x + 1, y), Rt = at(x, y + 1), Dg = at(x + 1, y + 1);
-                int nx, ny;
-                float val;
-                if (Dn > Rt) {
-                    if (Dn > Dg) { nx = x + 1; ny = y; val = Dn; }
-                    else { nx = x + 1; ny = y + 1; val = Dg; }
-                } else {
-                    if (Rt > Dg) { nx = x; ny = y + 1; val = Rt; }
-                    else { nx = x + 1; ny = y + 1; val = Dg; }
-                }
-                // ff_mat[nx][ny] = val, later binarised with ff_mat > 0
-                if (val > thresh && val > 0.f && nx < nb && ny < nb) mat[nx * nb + ny] = 1.f;
-                x = nx;
-                y = ny;
+            for (walk_move(pooled, nb, x, y); x < nb && y < nb; walk_move(pooled, nb, x, y)) {
+                const float val = pooled[x * nb + y];
+                if (val > thresh && val > 0.f) mat[x * nb + y] = 1.f;
             }
         }
     } else {
@@ -233,7 +483,7 @@ __global__ __launch_bounds__(WALK_THREADS) void threshold_walk_kernel(const floa
         if (threadIdx.x == 0 && thresh_out) thresh_out[map] = 0.f;
         if (topk > 0) {
             const int k = min(topk, N);
-            const uint32_t kk = block_select(pooled, N, N - k, hist, sh);  // k-th largest
+            const uint32_t kk = range_select(pooled, N, N - k, sel).key;  // k-th largest
             if (threadIdx.x == 0) s_cnt = 0;
             __syncthreads();
             if (threadIdx.x == 0) s_min = 0u;  // number of blocks equal to the k-th largest
@@ -268,6 +518,9 @@ __global__ __launch_bounds__(WALK_THREADS) void threshold_walk_kernel(const floa
     }
     __syncthreads();
     for (int i = threadIdx.x; i < nb; i += blockDim.x) mat[i * nb + i] = 1.f;  // main_conv_ff.py:277-278
+    __syncthreads();
+    for (int r = 1; r < replicas; ++r)
+        for (int i = threadIdx.x; i < N; i += blockDim.x) mat[r * replica_stride + i] = mat[i];
 }
 
 static std::mutex g_ws_mutex;
@@ -429,17 +682,22 @@ int transition_update(const float* Cur, float* Prev, int layers, long long n, fl
     return SPION_HIP_OK(hipGetLastError()) ? 0 : 1;
 }
 
-int pattern_generate(const float* Score, int n_maps, int L, int bs, int ksize, int mode, double param, float* Mat,
-                     float* Pooled, float* Thresh, hipStream_t stream) {
+int pattern_generate_maps(const float* const* Score, int n_maps, int L, int bs, int ksize, int mode, double param,
+                          float* Mat, int replicas, float* Pooled, float* Thresh, hipStream_t stream) {
     if (!Score || !Mat) {
         set_error("spion_pattern_generate: null Score or Mat");
         return 1;
     }
-    if (n_maps <= 0 || L <= 0 || bs <= 0 || L % bs) {
-        set_error("spion_pattern_generate: need n_maps > 0 and seq_len a positive multiple of block_size (got %d, %d, %d)",
-                  n_maps, L, bs);
+    if (n_maps <= 0 || L <= 0 || bs <= 0 || L % bs || replicas <= 0) {
+        set_error("spion_pattern_generate: need n_maps > 0, replicas > 0 and seq_len a positive multiple of block_size "
+                  "(got %d, %d, %d, %d)", n_maps, replicas, L, bs);
         return 1;
     }
+    for (int m = 0; m < n_maps; ++m)
+        if (!Score[m]) {
+            set_error("spion_pattern_generate: null Score or Mat");
+            return 1;
+        }
     if (ksize < 0 || (ksize && ksize % 2 == 0)) {
         set_error("spion_pattern_generate: conv_ksize must be 0 or odd (got %d)", ksize);
         return 1;
@@ -477,29 +735,49 @@ int pattern_generate(const float* Score, int n_maps, int L, int bs, int ksize, i
     const int hk = ksize / 2;
     // blocks per work-group of the streaming kernel (0: block size too small for it, or too wide)
     const int gb = bs >= 2 * hk && bs + 2 * hk <= CP_COLS ? std::min((CP_COLS - 2 * hk) / bs, CP_COLS * CP_RG / 64) : 0;
-    if (gb > 0)
-        hipLaunchKernelGGL(conv_pool_cols_kernel, dim3((nb + gb - 1) / gb, nb, n_maps), dim3(CP_COLS * CP_RG), 0, stream,
-                           Score, pooled, L, bs, nb, hk, gb);
-    else
-        hipLaunchKernelGGL(conv_pool_kernel, dim3(nb, nb, n_maps), dim3(POOL_THREADS), 0, stream, Score, pooled, L, bs,
-                           nb, hk);
+    for (int m0 = 0; m0 < n_maps; m0 += MAPS_PER_LAUNCH) {
+        const int n = std::min(MAPS_PER_LAUNCH, n_maps - m0);
+        ScoreMaps maps{};
+        for (int m = 0; m < n; ++m) maps.p[m] = Score[m0 + m];
+        float* out = pooled + (size_t)m0 * nb * nb;
+        if (gb > 0)
+            hipLaunchKernelGGL(conv_pool_cols_kernel, dim3((nb + gb - 1) / gb * nb * n), dim3(CP_COLS * CP_RG), 0, stream,
+                               maps, out, L, bs, nb, hk, gb);
+        else
+            hipLaunchKernelGGL(conv_pool_kernel, dim3(nb, nb, n), dim3(POOL_THREADS), 0, stream, maps, out, L, bs, nb,
+                               hk);
+    }
     if (!check_launch("conv_pool_kernel")) return 1;
     int topk = 0;
     if (mode == SPION_PATTERN_TOPK) topk = (int)((double)(nb * nb) * param - (double)nb);  // main_conv.py:247
-    const size_t walk_lds = (size_t)nb * nb <= (size_t)POOLED_LDS ? sizeof(float) * nb * nb : 0;
+    const size_t cells = (size_t)nb * nb;
+    size_t walk_lds = cells <= (size_t)POOLED_LDS ? sizeof(float) * cells : 0;
+    if (mode == SPION_PATTERN_FLOOD && nb <= JUMP_NB) walk_lds += 5 * (cells + 1);  // two 16-bit tables and the flags
     if (walk_lds > 32 * 1024) {  // beyond what a launch may ask for without saying so first
         static std::once_flag once;
         static hipError_t attr_err = hipSuccess;
         std::call_once(once, [] {
+            constexpr size_t jump = sizeof(float) * JUMP_NB * JUMP_NB + 5 * (JUMP_NB * JUMP_NB + 1);
             attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(threshold_walk_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(float) * POOLED_LDS);
+                                           hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)std::max(sizeof(float) * POOLED_LDS, jump));
         });
         if (!SPION_HIP_OK(attr_err)) return 1;
     }
     hipLaunchKernelGGL(threshold_walk_kernel, dim3(n_maps), dim3(WALK_THREADS), walk_lds, stream, pooled, Mat, Thresh, nb,
-                       mode, (float)param, topk);
+                       mode, (float)param, topk, replicas, (size_t)n_maps * cells);
     if (!check_launch("threshold_walk_kernel")) return 1;
     return 0;
+}
+
+// The same for maps that follow one another in memory.
+int pattern_generate(const float* Score, int n_maps, int L, int bs, int ksize, int mode, double param, float* Mat,
+                     float* Pooled, float* Thresh, hipStream_t stream) {
+    if (!Score || n_maps <= 0 || L <= 0)
+        return pattern_generate_maps(nullptr, n_maps, L, bs, ksize, mode, param, Mat, 1, Pooled, Thresh, stream);
+    std::vector<const float*> maps(n_maps);
+    for (int m = 0; m < n_maps; ++m) maps[m] = Score + (size_t)m * L * L;
+    return pattern_generate_maps(maps.data(), n_maps, L, bs, ksize, mode, param, Mat, 1, Pooled, Thresh, stream);
 }
 
 }  // namespace spion

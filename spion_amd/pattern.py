@@ -9,12 +9,29 @@ per-layer score maps and the model config dict) and give the same ``mat_lst`` te
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
 
 PATTERN_FLOOD = 0
 PATTERN_TOPK = 1
+
+
+def _mode(mode: str, ksize: int, threshold=None, density=None):
+    """(filter size, library mode, parameter) of a generator."""
+    if mode == "conv_ff":
+        k, kind, param = ksize, PATTERN_FLOOD, threshold
+    elif mode == "ff":
+        k, kind, param = 0, PATTERN_FLOOD, threshold
+    elif mode == "conv":
+        k, kind, param = ksize, PATTERN_TOPK, density
+    else:
+        raise ValueError(f"unknown mode {mode!r}")
+    if param is None:
+        raise ValueError("threshold (conv_ff / ff) or density (conv) is required")
+    return k, kind, float(param)
 
 
 def discover_block_masks(score_maps: torch.Tensor, block_size: int, *, mode: str = "conv_ff",
@@ -36,21 +53,12 @@ def discover_block_masks(score_maps: torch.Tensor, block_size: int, *, mode: str
     if L != L2 or L % block_size:
         raise ValueError(f"score maps must be square with L a multiple of block_size, got {tuple(x.shape)}")
     nb = L // block_size
-    if mode == "conv_ff":
-        k, kind, param = ksize, PATTERN_FLOOD, threshold
-    elif mode == "ff":
-        k, kind, param = 0, PATTERN_FLOOD, threshold
-    elif mode == "conv":
-        k, kind, param = ksize, PATTERN_TOPK, density
-    else:
-        raise ValueError(f"unknown mode {mode!r}")
-    if param is None:
-        raise ValueError("threshold (conv_ff / ff) or density (conv) is required")
+    k, kind, param = _mode(mode, ksize, threshold=threshold, density=density)
     mat = torch.empty((n, nb, nb), dtype=torch.float32, device=x.device)
     pooled = torch.empty((n, nb, nb), dtype=torch.float32, device=x.device)
     thresh = torch.empty((n,), dtype=torch.float32, device=x.device)
     stream = torch.cuda.current_stream(x.device).cuda_stream
-    rc = _lib.core().spion_pattern_generate(x.data_ptr(), n, L, block_size, k, kind, float(param),
+    rc = _lib.core().spion_pattern_generate(x.data_ptr(), n, L, block_size, k, kind, param,
                                             mat.data_ptr(), pooled.data_ptr(), thresh.data_ptr(), stream)
     if rc != 0:
         _lib.check_error("spion_pattern_generate")
@@ -81,33 +89,41 @@ def mean_score_map(attn: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def _stack_layers(attn_lst, model_config):
-    L = model_config["max_seq_len"]
-    # the reference keeps the first L rows of each gathered map (main_conv_ff.py:255)
-    return torch.stack([a[:L].detach() for a in attn_lst[: model_config["num_layers"]]], 0)
-
-
-def _as_mat_lst(mats: torch.Tensor) -> torch.Tensor:
-    # [layers, nb, nb] -> [4, layers, nb, nb]: one copy per data-parallel replica (main_conv_ff.py:298-299)
-    return torch.stack([mats, mats, mats, mats], 0)
+def _mat_lst(attn_lst, model_config, mode: str, **param) -> torch.Tensor:
+    """[4, layers, nb, nb] masks of the first ``num_layers`` maps: one copy per data-parallel replica
+    (main_conv_ff.py:298-299).  The reference keeps the first L rows of each gathered map (main_conv_ff.py:255).  Maps
+    that lie on the GPU as contiguous fp32 are read where they are; anything else is converted first, as before."""
+    L, bs = model_config["max_seq_len"], model_config["block_size"]
+    maps = [a[:L].detach() for a in attn_lst[: model_config["num_layers"]]]
+    if not maps or any(not x.is_cuda or x.dim() != 2 or x.shape != (L, L) or x.device != maps[0].device for x in maps) \
+            or L % bs:
+        mats = discover_block_masks(torch.stack(maps, 0), bs, mode=mode, **param)  # converts, or says what is wrong
+        return torch.stack([mats] * 4, 0)
+    maps = [x.to(torch.float32).contiguous() for x in maps]
+    ksize, kind, value = _mode(mode, 31, **param)
+    n, nb, dev = len(maps), L // bs, maps[0].device
+    out = torch.empty((4, n, nb, nb), dtype=torch.float32, device=dev)
+    pooled = torch.empty((n, nb, nb), dtype=torch.float32, device=dev)
+    ptrs = (ctypes.c_void_p * n)(*[x.data_ptr() for x in maps])
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    rc = _lib.core().spion_pattern_generate_maps(ptrs, n, L, bs, ksize, kind, value, out.data_ptr(), 4,
+                                                 pooled.data_ptr(), None, stream)
+    if rc != 0:
+        _lib.check_error("spion_pattern_generate_maps")
+        raise _lib.SpionLibraryError("spion_pattern_generate_maps failed")
+    return out
 
 
 def generate_pattern_conv_ff(attn_lst, model_config) -> torch.Tensor:
     """SPION-CF masks for every layer; reads block_size, max_seq_len, num_layers, threshold."""
-    mats = discover_block_masks(_stack_layers(attn_lst, model_config), model_config["block_size"],
-                                mode="conv_ff", threshold=model_config["threshold"])
-    return _as_mat_lst(mats)
+    return _mat_lst(attn_lst, model_config, "conv_ff", threshold=model_config["threshold"])
 
 
 def generate_pattern_ff(attn_lst, model_config) -> torch.Tensor:
     """SPION-F masks (no filter)."""
-    mats = discover_block_masks(_stack_layers(attn_lst, model_config), model_config["block_size"],
-                                mode="ff", threshold=model_config["threshold"])
-    return _as_mat_lst(mats)
+    return _mat_lst(attn_lst, model_config, "ff", threshold=model_config["threshold"])
 
 
 def generate_pattern_conv(attn_lst, model_config) -> torch.Tensor:
     """SPION-C masks (top-k of the pooled filtered map); reads density instead of threshold."""
-    mats = discover_block_masks(_stack_layers(attn_lst, model_config), model_config["block_size"],
-                                mode="conv", density=model_config["density"])
-    return _as_mat_lst(mats)
+    return _mat_lst(attn_lst, model_config, "conv", density=model_config["density"])

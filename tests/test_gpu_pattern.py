@@ -62,6 +62,43 @@ def test_pattern_large_block_grids(L, bs):
     _check_maps(maps, bs, 0.95, 31)
 
 
+@pytest.mark.parametrize("levels", [0, 1, 4])
+@pytest.mark.parametrize("nb", [1, 2, 3, 64, 127, 128, 129, 192, 193])
+def test_walk_and_quantile_on_block_grids_of_every_size(nb, levels):
+    """Quantile and walk alone (no filter, block size 1: the map is its own pooled map) on both sides of the grids whose
+    walk is taken by squaring the move table (128) and whose map stays in LDS (192), on distinct values (levels 0) and
+    on values with so many ties that the selection falls back to its plain form."""
+    g = torch.Generator().manual_seed(nb)
+    maps = torch.rand(3, nb, nb, generator=g)
+    if levels:
+        maps = torch.floor(maps * levels) + 1.0
+    for q in (0.0, 0.5, 0.9, 1.0):
+        mat, pooled, thresh = discover_block_masks(maps.cuda(), 1, mode="ff", threshold=q, return_aux=True)
+        assert torch.equal(pooled.cpu(), maps)
+        for i in range(3):
+            t = op.quantile_linear(maps[i].numpy(), q)[0]
+            assert float(thresh[i]) == float(t)
+            assert np.array_equal(mat[i].cpu().numpy().astype(np.int8), op.mask_from_pooled(maps[i].numpy(), t)), (q, i)
+
+
+@pytest.mark.parametrize("L,bs", [(96, 32), (1056, 32), (2048, 64)])
+def test_generators_read_the_layers_maps_in_place(L, bs):
+    """The generators on separate maps (more of them than one launch takes, one with rows to drop, one that has to be
+    made contiguous) against the masks of the stacked maps, in all four copies."""
+    g = torch.Generator().manual_seed(L)
+    maps = [torch.softmax(torch.randn(L, L, generator=g) * 2, -1).cuda() for _ in range(18)]
+    lst = list(maps)
+    lst[1] = torch.cat([maps[1], torch.ones(32, L, device="cuda")])
+    lst[2] = maps[2].t().contiguous().t()
+    for gen, mode, cfg in ((generate_pattern_conv_ff, "conv_ff", {"threshold": 0.9}), (generate_pattern_ff, "ff", {"threshold": 0.8}),
+                           (generate_pattern_conv, "conv", {"density": 0.3})):
+        out = gen(lst, {"max_seq_len": L, "block_size": bs, "num_layers": 18, **cfg})
+        ref = discover_block_masks(torch.stack(maps), bs, mode=mode, **cfg)
+        assert out.shape == (4, 18, L // bs, L // bs)
+        for r in range(4):
+            assert torch.equal(out[r], ref)
+
+
 def test_pattern_config2_bit_exact_against_both_routes():
     """Config 2: two 1024x1024 maps, 31x31 diagonal filter, 32x32 pooling, q = 0.90.
     The seed is one whose decision margin exceeds the float32-route error (tests/golden/config2.json),
