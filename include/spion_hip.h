@@ -380,6 +380,27 @@ void spion_dense_forward_strided_mean(void* handle, const float* Q, const float*
  * attention entry points take.  Returns 0 on success. */
 int spion_transpose_last2(const float* in, float* out, int batch, int rows, int cols, void* stream);
 
+/* The projections around the attention core (models/attention.py:84-103: three nn.Linear into the heads, one out of
+ * them), fp32, all matrices row-major and 16-byte aligned, rows, n and dim multiples of 32.
+ *   spion_project_forward:         Y [rows][segs*n] = X [rows][dim] . W^T + b.  W, b: HOST arrays of segs (1 to 3) device
+ *                                  pointers, W[s] [n][dim], b[s] [n]; outputs of segment s are columns s*n .. s*n + n-1.
+ *   spion_project_backward_input:  dX [rows][dim] = dY [rows][segs*n] . W
+ *   spion_project_backward_weight: dW [outputs][dim] = dY^T . X and db [outputs] = column sums of dY [rows][outputs];
+ *                                  workspace: spion_project_workspace(rows, outputs, dim) floats, contents unspecified.
+ *                                  The sum over the rows has a fixed order: the same inputs give the same bits.
+ * Each returns 0 on success. */
+int spion_project_forward(const float* X, const float* const* W, const float* const* b, float* Y, long long rows, int n,
+                          int segs, int dim, void* stream);
+int spion_project_backward_input(const float* dY, const float* const* W, float* dX, long long rows, int n, int segs,
+                                 int dim, void* stream);
+long long spion_project_workspace(long long rows, int outputs, int dim);
+int spion_project_backward_weight(const float* dY, const float* X, float* dW, float* db, float* workspace, long long rows,
+                                  int outputs, int dim, void* stream);
+
+/* mask [batch][seq_len] (1 = key, 0 = padding) -> penalty [batch*heads][seq_len] = 1e6 * (1 - mask), the Mask operand
+ * of the key-mask entry points (models/attention_blockcuda_mask.py:42-43).  Returns 0 on success. */
+int spion_key_penalty(const float* mask, float* penalty, int batch, int heads, int seq_len, void* stream);
+
 const char* spion_version(void);
 
 #ifdef __cplusplus

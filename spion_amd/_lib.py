@@ -127,6 +127,16 @@ def core() -> ctypes.CDLL:
     lib.spion_pattern_generate.restype = c_int
     lib.spion_pattern_generate_maps.argtypes = [_P, c_int, c_int, c_int, c_int, c_int, c_double, _P, c_int, _P, _P, _P]
     lib.spion_pattern_generate_maps.restype = c_int
+    lib.spion_project_forward.argtypes = [_P] * 4 + [ctypes.c_longlong, c_int, c_int, c_int, _P]
+    lib.spion_project_forward.restype = c_int
+    lib.spion_project_backward_input.argtypes = [_P] * 3 + [ctypes.c_longlong, c_int, c_int, c_int, _P]
+    lib.spion_project_backward_input.restype = c_int
+    lib.spion_project_workspace.argtypes = [ctypes.c_longlong, c_int, c_int]
+    lib.spion_project_workspace.restype = ctypes.c_longlong
+    lib.spion_project_backward_weight.argtypes = [_P] * 5 + [ctypes.c_longlong, c_int, c_int, _P]
+    lib.spion_project_backward_weight.restype = c_int
+    lib.spion_key_penalty.argtypes = [_P, _P, c_int, c_int, c_int, _P]
+    lib.spion_key_penalty.restype = c_int
     lib.spion_score_map_mean.argtypes = [_P, c_int, c_int, c_int, c_int, _P, _P]
     lib.spion_score_map_mean.restype = c_int
     for fam, extra in (("block", 0), ("blockmask", 1)):

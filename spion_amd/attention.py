@@ -74,6 +74,19 @@ class _FusedQKV(torch.autograd.Function):
         return (dX, dW[:n], dW[n:2 * n], dW[2 * n:], db[:n], db[n:2 * n], db[2 * n:], None, None)
 
 
+_CORES: list = []
+
+
+def _core_types():
+    """The sparse modules whose forward the compiled node restates (a subclass may have changed it)."""
+    if not _CORES:
+        from .attention_blockcuda import CUDABlockAttention
+        from .attention_blockcuda_mask import CUDABlockMaskAttention
+
+        _CORES.extend((CUDABlockAttention, CUDABlockMaskAttention))
+    return _CORES
+
+
 class Attention(nn.Module):
     def __init__(self, config, inference=False):
         super().__init__()
@@ -116,7 +129,15 @@ class Attention(nn.Module):
         torch's usual rule for capturing a backward: warm up on a side stream and keep no autograd graph of a step
         that ran on the default stream alive (its AccumulateGrad nodes belong to the legacy stream, which a capture
         must not touch; breaking this rule ends in a crash inside capture_end on ROCm, not in an error message)."""
-        if self.fused_qkv and X.dtype == torch.float32 and not torch.is_autocast_enabled():
+        node = self._compiled_node(X, mask)
+        if node is not None and mat is not None:
+            done = self._sparse_layer(node, X, mask, mat)
+            if done is not None:
+                return done
+        if node is not None:
+            Q, K, V = self._in_node(node.project_heads, X, self.W_q.weight, self.W_k.weight, self.W_v.weight,
+                                    self.W_q.bias, self.W_k.bias, self.W_v.bias, self.num_head, self.head_dim)
+        elif self.fused_qkv and X.dtype == torch.float32 and not torch.is_autocast_enabled():
             Q, K, V = _FusedQKV.apply(X, self.W_q.weight, self.W_k.weight, self.W_v.weight, self.W_q.bias,
                                       self.W_k.bias, self.W_v.bias, self.num_head, self.head_dim)
         else:
@@ -129,8 +150,51 @@ class Attention(nn.Module):
                 attn_out, attn = self.attn(Q.float(), K.float(), V.float(), mask.float())
             else:
                 attn_out, attn = self.block_attn(Q.float(), K.float(), V.float(), mask.float(), mat)
+        if node is not None and attn_out.dtype == torch.float32:
+            return self._in_node(node.merge_heads, attn_out, self.ff.weight, self.ff.bias), attn
         attn_out = self.combine_heads(attn_out)
         return self.ff(attn_out), attn
+
+    def _compiled_node(self, X, mask):
+        """The compiled node when it covers the projections of this call (csrc/project.hip: fp32 on the GPU, features in
+        multiples of 32, plain linear layers without hooks, no autocast), else None."""
+        if not (self.fused_qkv and X.is_cuda and X.dtype == torch.float32 and X.dim() == 3 and X.shape[2] == self.dim
+                and isinstance(mask, torch.Tensor) and X.shape[0] * X.shape[1] % 32 == 0 and X.numel() > 0
+                and self.num_head * self.head_dim % 32 == 0 and self.dim % 32 == 0
+                and not torch.is_autocast_enabled()):
+            return None
+        for m in (self.W_q, self.W_k, self.W_v, self.ff):
+            if (type(m) is not nn.Linear or m.bias is None or m.weight.dtype != torch.float32
+                    or m.weight.device != X.device or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                    or m._backward_pre_hooks):
+                return None
+        return _lib.autograd_node()
+
+    def _in_node(self, call, *args):
+        """A call of the node on X's stream; errors of the library come out as the modules raise them."""
+        index = args[0].device.index
+        try:
+            return call(*args, _lib._raw_stream(torch.cuda.current_device() if index is None else index))
+        except RuntimeError as e:
+            if str(e).startswith(("attn_forward:", "projection:")):
+                raise _lib.SpionLibraryError(str(e)) from None
+            raise
+
+    def _sparse_layer(self, node, X, mask, mat):
+        """The whole layer in one call -- projections, core, output projection, and no torch operation in between --
+        or None when the core is not one of this package's modules as they are, or has hooks."""
+        core = self.block_attn
+        if (type(core) not in _core_types() or not core.reads_views
+                or X.shape[0] != core.batch_size or X.shape[1] != core.seq_len or core._forward_hooks
+                or core._forward_pre_hooks or core._backward_hooks or core._backward_pre_hooks):
+            return None
+        idx = core.csr_cache.get(mat, core.block_size)
+        key_mask, is_mask = core.key_operand(mask if mask.dtype == torch.float32 else mask.float())
+        y, p_flat = self._in_node(
+            node.sparse_layer, X, self.W_q.weight, self.W_k.weight, self.W_v.weight, self.W_q.bias, self.W_k.bias,
+            self.W_v.bias, self.ff.weight, self.ff.bias, key_mask, is_mask, idx.offsets, idx.columns, idx.sum_mat,
+            core.attn_handle, idx.nnz, self.num_head, self.head_dim)
+        return y, 0 if core.with_mask else p_flat
 
     def reconstruct_for_blocksparse(self, config):
         """Switch the layer to the sparse path: load the block library, create its handle and the

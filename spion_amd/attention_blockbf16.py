@@ -19,6 +19,17 @@ from . import _lib
 from .csr import CsrCache
 
 
+def _penalty(mask, m, dev):
+    """1e6 * (1 - mask) per head, [B*H, L], in one launch where the mask is what the kernel takes."""
+    if mask.dtype == torch.float32 and mask.is_cuda and mask.is_contiguous() and mask.shape == (m.batch_size, m.seq_len):
+        pen = torch.empty((m.num_batches, m.seq_len), dtype=torch.float32, device=dev)
+        index = dev.index if dev.index is not None else torch.cuda.current_device()
+        m.lib.spion_key_penalty(mask.data_ptr(), pen.data_ptr(), m.batch_size, m.num_heads, m.seq_len,
+                                _lib._raw_stream(index))
+        return pen
+    return (1e6 * (1.0 - mask.to(torch.float32))).repeat_interleave(m.num_heads, 0).contiguous()
+
+
 class _BlockBF16Function(torch.autograd.Function):
     @staticmethod
     def forward(ctx, query, key, value, mask, mat, module):
@@ -31,7 +42,7 @@ class _BlockBF16Function(torch.autograd.Function):
         dev = query.device
         pen = None
         if m.key_mask:
-            pen = (1e6 * (1.0 - mask.to(torch.float32))).repeat_interleave(m.num_heads, 0).contiguous()  # [B*H, L]
+            pen = _penalty(mask, m, dev)
         pen_ptr = pen.data_ptr() if pen is not None else None
         lse = torch.empty((m.num_batches, m.seq_len), dtype=torch.float32, device=dev)
         # bf16 heads that are views of [B, L, H*d] projections (models/attention.py:136-139) are read in place and

@@ -159,6 +159,17 @@ class _BlockAttentionBase(nn.Module):
         self.reads_views = self.emb_dim in (16, 32, 64, 128)
 
 
+    def key_operand(self, mask):
+        """What the compiled node takes for the key mask: (mask, True) when the library makes the penalties from it
+        (spion_key_penalty: one launch where the expression below is three or four), (penalties [B, H*L], False) for a
+        mask of another type or layout, (None, False) without one."""
+        if not self.with_mask:
+            return None, False
+        if mask.dtype == torch.float32 and mask.is_cuda and mask.is_contiguous() and not mask.requires_grad \
+                and mask.shape == (self.batch_size, self.seq_len):
+            return mask, True
+        return (1e6 * (1.0 - mask.repeat(1, self.num_heads))).to(torch.float32).contiguous(), False
+
     def run(self, query, key, value, mask, mat):
         """(out, p_flat) through the compiled autograd node (csrc/autograd_node.cpp) -- the same steps as
         ``_BlockAttnFunction`` with the node, the saved tensors and the allocations on the C++ side of PyTorch, which
@@ -170,13 +181,11 @@ class _BlockAttentionBase(nn.Module):
         if query.shape != self.head_shape:
             raise ValueError(f"query shape {tuple(query.shape)} does not match the handle {self.head_shape}")
         idx = self.csr_cache.get(mat, self.block_size)
-        pen = None
-        if self.with_mask:
-            pen = (1e6 * (1.0 - mask.repeat(1, self.num_heads))).to(torch.float32).contiguous()  # [B, H*L]
+        key_mask, is_mask = self.key_operand(mask)
         index = query.device.index
         try:
-            out, p_flat = node.sparse_attention(query, key, value, pen, idx.offsets, idx.columns, idx.sum_mat,
-                                                self.attn_handle, idx.nnz, self.num_heads, self.reads_views,
+            out, p_flat = node.sparse_attention(query, key, value, key_mask, is_mask, idx.offsets, idx.columns,
+                                                idx.sum_mat, self.attn_handle, idx.nnz, self.num_heads, self.reads_views,
                                                 _lib._raw_stream(torch.cuda.current_device() if index is None else index))
         except RuntimeError as e:
             if str(e).startswith(("attn_forward:", "attn_backward:")):

@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "lib")
 OBJ = os.path.join(LIB, "obj")
 
-HIP_SOURCES = ["capi.hip", "sparse_attn.hip", "dense_attn.hip", "pattern.hip"]
+HIP_SOURCES = ["sparse_attn.hip", "dense_attn.hip", "capi.hip", "pattern.hip", "project.hip"]
 DROPINS = {1: "attn.so", 2: "attn_mask.so", 3: "block_attn.so", 4: "block_attn_mask.so"}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -64,54 +64,69 @@ const float* fp(const Tensor& t) { return t.defined() ? static_cast<const float*
 float* fpm(Tensor& t) { return static_cast<float*>(t.data_ptr()); }
 const int* ip(const Tensor& t) { return static_cast<const int*>(t.data_ptr()); }
 
+// What a forward of the attention core leaves for its backward.
+struct CoreResult {
+    Tensor q, k, v, out, p_flat;
+    bool strided = false, tiled = false;
+};
+
+CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& pen,
+                        const Tensor& offsets, const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz,
+                        int64_t num_heads, bool reads_views, int64_t stream) {
+    void* h = reinterpret_cast<void*>(handle);
+    spion_set_stream(h, reinterpret_cast<void*>(stream));
+    TORCH_CHECK(query.dim() == 4 && key.sizes() == query.sizes() && value.sizes() == query.sizes(),
+                "query, key and value must be [B, H, L, d] tensors of one shape");
+    TORCH_CHECK(query.scalar_type() == torch::kFloat32 && query.is_cuda(), "fp32 tensors on the GPU expected");
+    const int64_t B = query.size(0), H = query.size(1);
+    const auto opt = query.options();
+    CoreResult r;
+    r.p_flat = torch::empty({B * H * nnz}, opt);
+    spion_head_layout lin{}, lout{}, lk{}, lv{};
+    r.strided = reads_views && !(query.is_contiguous() && key.is_contiguous() && value.is_contiguous()) &&
+                head_layout(query, lin) && head_layout(key, lk) && head_layout(value, lv) && same_strides(key, query) &&
+                same_strides(value, query);
+    if (r.strided) {
+        r.q = query;
+        r.k = key;
+        r.v = value;
+        r.out = empty_heads(query.sizes(), query.stride(1) < query.stride(2), opt);
+        head_layout(r.out, lout);
+        spion_attn_forward_strided(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.p_flat), fpm(r.out), ip(offsets),
+                                   ip(columns), ip(sum_mat), (int)nnz, (int)num_heads, &lin, &lout);
+    } else {
+        r.q = query.contiguous();
+        r.k = key.contiguous();
+        r.v = value.contiguous();
+        r.out = torch::empty(query.sizes(), opt);
+        spion_attn_forward_rowmajor(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.p_flat), fpm(r.out), ip(offsets),
+                                    ip(columns), ip(sum_mat), (int)nnz);
+    }
+    check_library("attn_forward");
+    r.tiled = spion_last_path(h) == 1;
+    return r;
+}
+
 struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
     // pen_opt: [B, H*L] key penalties of the key-mask modules, or nothing.  stream: torch's current raw
     // stream at the call; autograd runs the backward of a node on the stream its forward ran on.
     static variable_list forward(AutogradContext* ctx, Tensor query, Tensor key, Tensor value,
                                  c10::optional<Tensor> pen_opt, Tensor offsets, Tensor columns, Tensor sum_mat, int64_t handle, int64_t nnz,
                                  int64_t num_heads, bool reads_views, int64_t stream) {
-        void* h = reinterpret_cast<void*>(handle);
         const Tensor pen = pen_opt.has_value() ? *pen_opt : Tensor();
-        spion_set_stream(h, reinterpret_cast<void*>(stream));
-        TORCH_CHECK(query.dim() == 4 && key.sizes() == query.sizes() && value.sizes() == query.sizes(),
-                    "query, key and value must be [B, H, L, d] tensors of one shape");
-        TORCH_CHECK(query.scalar_type() == torch::kFloat32 && query.is_cuda(), "fp32 tensors on the GPU expected");
-        const int64_t B = query.size(0), H = query.size(1);
-        const auto opt = query.options();
-        Tensor p_flat = torch::empty({B * H * nnz}, opt);
-        spion_head_layout lin{}, lout{}, lk{}, lv{};
-        bool strided = reads_views && !(query.is_contiguous() && key.is_contiguous() && value.is_contiguous()) &&
-                       head_layout(query, lin) && head_layout(key, lk) && head_layout(value, lv) &&
-                       same_strides(key, query) && same_strides(value, query);
-        Tensor q, k, v, out;
-        if (strided) {
-            q = query;
-            k = key;
-            v = value;
-            out = empty_heads(query.sizes(), query.stride(1) < query.stride(2), opt);
-            head_layout(out, lout);
-            spion_attn_forward_strided(h, fp(q), fp(k), fp(v), fp(pen), fpm(p_flat), fpm(out), ip(offsets), ip(columns),
-                                       ip(sum_mat), (int)nnz, (int)num_heads, &lin, &lout);
-        } else {
-            q = query.contiguous();
-            k = key.contiguous();
-            v = value.contiguous();
-            out = torch::empty(query.sizes(), opt);
-            spion_attn_forward_rowmajor(h, fp(q), fp(k), fp(v), fp(pen), fpm(p_flat), fpm(out), ip(offsets), ip(columns),
-                                        ip(sum_mat), (int)nnz);
-        }
-        check_library("attn_forward");
+        CoreResult r = core_forward(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, num_heads, reads_views,
+                                    stream);
         // which kernel family serves THIS pattern (the handle may run other patterns before the backward)
-        ctx->saved_data["tiled"] = spion_last_path(h) == 1;
+        ctx->saved_data["tiled"] = r.tiled;
         ctx->saved_data["handle"] = handle;
         ctx->saved_data["nnz"] = nnz;
         ctx->saved_data["heads"] = num_heads;
-        ctx->saved_data["strided"] = strided;
+        ctx->saved_data["strided"] = r.strided;
         ctx->saved_data["stream"] = stream;
-        ctx->save_for_backward({q, k, v, p_flat, offsets, columns, sum_mat, out});
+        ctx->save_for_backward({r.q, r.k, r.v, r.p_flat, offsets, columns, sum_mat, r.out});
         ctx->set_materialize_grads(false);  // the gradient of the returned probabilities is ignored anyway
-        if (pen.defined()) ctx->mark_non_differentiable({p_flat});
-        return {out, p_flat};
+        if (pen.defined()) ctx->mark_non_differentiable({r.p_flat});
+        return {r.out, r.p_flat};
     }
 
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -164,10 +179,170 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
     }
 };
 
+// 1e6 * (1 - mask) per head, [B, H*L], from a [B, L] fp32 key mask (models/attention_blockcuda_mask.py:42-43).
+Tensor key_penalty(const Tensor& mask, int64_t heads, int64_t stream) {
+    Tensor pen = torch::empty({mask.size(0), heads * mask.size(1)}, mask.options());
+    spion_key_penalty(fp(mask), fpm(pen), (int)mask.size(0), (int)heads, (int)mask.size(1), reinterpret_cast<void*>(stream));
+    check_library("attn_forward");
+    return pen;
+}
+// The modules hand over a key mask, or penalties made from one the kernel does not take (is_mask = false).
+c10::optional<Tensor> penalty_of(const c10::optional<Tensor>& mask_or_pen, bool is_mask, int64_t heads, int64_t stream) {
+    if (!is_mask || !mask_or_pen.has_value()) return mask_or_pen;
+    return key_penalty(*mask_or_pen, heads, stream);
+}
+
+// ---- the projections of models/attention.py:84-103 on the library's own kernels ------------------
+Tensor aligned(const Tensor& t) {  // contiguous, 16-byte aligned
+    Tensor c = t.contiguous();
+    return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 ? c.clone() : c;
+}
+
+Tensor project_weight_grads(const float* dy, const Tensor& x, int64_t rows, int64_t outputs, int64_t dim, int64_t stream,
+                            Tensor& db) {
+    const auto opt = x.options();
+    Tensor dw = torch::empty({outputs, dim}, opt), ws = torch::empty({spion_project_workspace(rows, (int)outputs, (int)dim)}, opt);
+    db = torch::empty({outputs}, opt);
+    spion_project_backward_weight(dy, fp(x), fpm(dw), fpm(db), fpm(ws), rows, (int)outputs, (int)dim,
+                                  reinterpret_cast<void*>(stream));
+    return dw;
+}
+
+// X [B, L, dim] -> the [B, H, L, d] heads of the three projections, slices of one [B, L, 3, H, d] buffer.
+std::vector<Tensor> qkv_forward(const Tensor& x, const Tensor (&w)[3], const Tensor (&b)[3], int64_t H, int64_t d,
+                                int64_t stream) {
+    const int64_t B = x.size(0), L = x.size(1), dim = x.size(2);
+    Tensor buf = torch::empty({B, L, 3, H, d}, x.options());
+    const float* wp[3] = {fp(w[0]), fp(w[1]), fp(w[2])};
+    const float* bp[3] = {fp(b[0]), fp(b[1]), fp(b[2])};
+    spion_project_forward(fp(x), wp, bp, fpm(buf), B * L, (int)(H * d), 3, (int)dim, reinterpret_cast<void*>(stream));
+    check_library("projection");
+    std::vector<Tensor> out;
+    for (int i = 0; i < 3; ++i)  // the slice [:, :, i].transpose(1, 2)
+        out.push_back(buf.as_strided({B, H, L, d}, {L * 3 * H * d, d, 3 * H * d, 1}, i * H * d));
+    return out;
+}
+
+struct QkvNode : public torch::autograd::Function<QkvNode> {
+    static variable_list forward(AutogradContext* ctx, Tensor x, Tensor wq, Tensor wk, Tensor wv, Tensor bq, Tensor bk,
+                                 Tensor bv, int64_t H, int64_t d, int64_t stream) {
+        const Tensor xc = aligned(x);
+        const Tensor w[3] = {aligned(wq), aligned(wk), aligned(wv)}, b[3] = {aligned(bq), aligned(bk), aligned(bv)};
+        ctx->save_for_backward({xc, w[0], w[1], w[2]});
+        ctx->saved_data["H"] = H;
+        ctx->saved_data["stream"] = stream;
+        return qkv_forward(xc, w, b, H, d, stream);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor& x = saved[0];
+        const int64_t H = ctx->saved_data["H"].toInt(), stream = ctx->saved_data["stream"].toInt();
+        const int64_t B = x.size(0), L = x.size(1), dim = x.size(2), n = saved[1].size(0), d = n / H, rows = B * L;
+        for (auto& t : g)
+            if (!t.defined()) t = torch::zeros({B, H, L, d}, x.options());
+        Tensor keep;  // [B, L, 3, H, d]
+        const float* dy = fp(g[0]);
+        if (!adjacent_head_views(g[0], g[1], g[2]) || reinterpret_cast<uintptr_t>(dy) % 16) {
+            keep = torch::stack({g[0].transpose(1, 2), g[1].transpose(1, 2), g[2].transpose(1, 2)}, 2).contiguous();
+            dy = fp(keep);
+        }
+        variable_list r(10);
+        if (ctx->needs_input_grad(0)) {
+            r[0] = torch::empty_like(x);
+            const float* wp[3] = {fp(saved[1]), fp(saved[2]), fp(saved[3])};
+            spion_project_backward_input(dy, wp, fpm(r[0]), rows, (int)n, 3, (int)dim, reinterpret_cast<void*>(stream));
+        }
+        bool any = false;
+        for (int i = 1; i < 7; ++i) any = any || ctx->needs_input_grad(i);
+        if (any) {
+            Tensor db, dw = project_weight_grads(dy, x, rows, 3 * n, dim, stream, db);
+            for (int i = 0; i < 3; ++i) {
+                r[1 + i] = dw.narrow(0, i * n, n);
+                r[4 + i] = db.narrow(0, i * n, n);
+            }
+        }
+        check_library("projection");
+        return r;
+    }
+};
+
+// The output projection on heads [B, H, L, d] that lie interleaved ([B, L, H*d] in memory: what the core's forward makes
+// for the slices above), y [B, L, dim].
+Tensor merge_forward(const Tensor& merged, const Tensor& w, const Tensor& b, int64_t stream) {
+    const int64_t B = merged.size(0), L = merged.size(1), n = merged.size(2) * merged.size(3);
+    Tensor y = torch::empty({B, L, w.size(0)}, merged.options());
+    const float* wp[1] = {fp(w)};
+    const float* bp[1] = {fp(b)};
+    spion_project_forward(fp(merged), wp, bp, fpm(y), B * L, (int)w.size(0), 1, (int)n, reinterpret_cast<void*>(stream));
+    check_library("projection");
+    return y;
+}
+struct MergeNode : public torch::autograd::Function<MergeNode> {
+    static Tensor forward(AutogradContext* ctx, Tensor heads, Tensor w, Tensor b, int64_t stream) {
+        const Tensor a = aligned(heads.transpose(1, 2)), wc = aligned(w), bc = aligned(b);
+        ctx->save_for_backward({a, wc});
+        ctx->saved_data["stream"] = stream;
+        return merge_forward(a, wc, bc, stream);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &a = saved[0], &w = saved[1];
+        const int64_t stream = ctx->saved_data["stream"].toInt();
+        const int64_t rows = a.size(0) * a.size(1), n = a.size(2) * a.size(3), dim = w.size(0);
+        const Tensor dy = aligned(g[0]);
+        variable_list r(4);
+        if (ctx->needs_input_grad(0)) {
+            Tensor da = torch::empty_like(a);
+            const float* wp[1] = {fp(w)};
+            spion_project_backward_input(fp(dy), wp, fpm(da), rows, (int)dim, 1, (int)n, reinterpret_cast<void*>(stream));
+            r[0] = da.transpose(1, 2);
+        }
+        if (ctx->needs_input_grad(1) || ctx->needs_input_grad(2)) r[1] = project_weight_grads(fp(dy), a, rows, dim, n, stream, r[2]);
+        check_library("projection");
+        return r;
+    }
+};
+
+// The attention layer in its sparse phase (models/attention.py:84-103): projections, sparse core, output projection in
+// one call from Python.  Returns [y, p_flat].
+std::vector<Tensor> sparse_layer(const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& bq,
+                                 const Tensor& bk, const Tensor& bv, const Tensor& wf, const Tensor& bf,
+                                 const c10::optional<Tensor>& mask_or_pen, bool is_mask, const Tensor& offsets,
+                                 const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t num_heads, int64_t head_dim,
+                                 int64_t stream) {
+    const auto pen = penalty_of(mask_or_pen, is_mask, num_heads, stream);
+    if (!torch::GradMode::is_enabled()) {  // nothing to record: no nodes
+        const Tensor w[3] = {aligned(wq), aligned(wk), aligned(wv)}, b[3] = {aligned(bq), aligned(bk), aligned(bv)};
+        const auto qkv = qkv_forward(aligned(x), w, b, num_heads, head_dim, stream);
+        const CoreResult r = core_forward(qkv[0], qkv[1], qkv[2], pen.has_value() ? *pen : Tensor(), offsets, columns, sum_mat,
+                                          handle, nnz, num_heads, true, stream);
+        return {merge_forward(aligned(r.out.transpose(1, 2)), aligned(wf), aligned(bf), stream), r.p_flat};
+    }
+    const auto qkv = QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream);
+    const auto core = SparseAttnNode::apply(qkv[0], qkv[1], qkv[2], pen, offsets, columns, sum_mat, handle, nnz, num_heads,
+                                            true, stream);
+    return {MergeNode::apply(core[0], wf, bf, stream), core[1]};
+}
+
+// The two projections by themselves, around a core of the caller's (the dense phase).
+std::vector<Tensor> project_heads(const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& bq,
+                                  const Tensor& bk, const Tensor& bv, int64_t num_heads, int64_t head_dim, int64_t stream) {
+    return QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream);
+}
+Tensor merge_heads(const Tensor& heads, const Tensor& w, const Tensor& b, int64_t stream) {
+    return MergeNode::apply(heads, w, b, stream);
+}
+
 std::vector<Tensor> sparse_attention(const Tensor& query, const Tensor& key, const Tensor& value,
-                                     const c10::optional<Tensor>& pen, const Tensor& offsets, const Tensor& columns,
-                                     const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t num_heads,
+                                     const c10::optional<Tensor>& mask_or_pen, bool is_mask, const Tensor& offsets,
+                                     const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t num_heads,
                                      bool reads_views, int64_t stream) {
+    const auto pen = penalty_of(mask_or_pen, is_mask, num_heads, stream);
+    if (!torch::GradMode::is_enabled()) {
+        const CoreResult r = core_forward(query, key, value, pen.has_value() ? *pen : Tensor(), offsets, columns, sum_mat,
+                                          handle, nnz, num_heads, reads_views, stream);
+        return {r.out, r.p_flat};
+    }
     return SparseAttnNode::apply(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, num_heads, reads_views,
                                  stream);
 }
@@ -175,9 +350,12 @@ std::vector<Tensor> sparse_attention(const Tensor& query, const Tensor& key, con
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-    m.doc() = "C++ autograd node of the sparse attention modules";
+    m.doc() = "C++ autograd nodes of the sparse attention modules";
     m.def("sparse_attention", &sparse_attention, "forward of the sparse attention modules; returns [out, p_flat]",
-          py::arg("query"), py::arg("key"), py::arg("value"), py::arg("pen"), py::arg("offsets"), py::arg("columns"),
-          py::arg("sum_mat"), py::arg("handle"), py::arg("nnz"), py::arg("num_heads"), py::arg("reads_views"),
-          py::arg("stream"));
+          py::arg("query"), py::arg("key"), py::arg("value"), py::arg("mask_or_pen"), py::arg("is_mask"), py::arg("offsets"),
+          py::arg("columns"), py::arg("sum_mat"), py::arg("handle"), py::arg("nnz"), py::arg("num_heads"),
+          py::arg("reads_views"), py::arg("stream"));
+    m.def("sparse_layer", &sparse_layer, "forward of the attention layer in its sparse phase; returns [y, p_flat]");
+    m.def("project_heads", &project_heads, "the three input projections; returns the [B, H, L, d] heads");
+    m.def("merge_heads", &merge_heads, "the output projection of [B, H, L, d] heads");
 }

@@ -90,6 +90,11 @@ void dense_forward(void*, const float*, const float*, const float*, const float*
 void dense_backward(void*, const float*, const float*, const float*, const float*, const float*, float*, float*,
                     float*);
 int pattern_generate(const float*, int, int, int, int, int, double, float*, float*, float*, hipStream_t);
+int project_forward(const float*, const float* const*, const float* const*, float*, long long, int, int, int, hipStream_t);
+int project_backward_input(const float*, const float* const*, float*, long long, int, int, int, hipStream_t);
+long long project_workspace(long long, int, int);
+int project_backward_weight(const float*, const float*, float*, float*, float*, long long, int, int, hipStream_t);
+int key_penalty(const float*, float*, int, int, int, hipStream_t);
 int pattern_generate_maps(const float* const*, int, int, int, int, int, double, float*, int, float*, float*, hipStream_t);
 int score_map_mean(const float*, int, int, int, int, float*, hipStream_t, float post = 1.0f);
 void dense_forward_strided_mean(void*, const float*, const float*, const float*, const float*, float*, float*, float*, int,
@@ -216,6 +221,28 @@ void spion_densemask_attn_backward(void* h, const float* Qt, const float* Kt, co
     dense_backward(h, Qt, Kt, V, P, dOt, dQ, dK, dV);
 }
 void spion_densemask_destroy(void* h) { dense_destroy(h); }
+
+// ---- projections around the attention core -------------------------------------------------------
+int spion_project_forward(const float* X, const float* const* W, const float* const* b, float* Y, long long rows, int n,
+                          int segs, int dim, void* stream) {
+    note_current_handle(nullptr);
+    return project_forward(X, W, b, Y, rows, n, segs, dim, static_cast<hipStream_t>(stream));
+}
+int spion_project_backward_input(const float* dY, const float* const* W, float* dX, long long rows, int n, int segs, int dim,
+                                 void* stream) {
+    note_current_handle(nullptr);
+    return project_backward_input(dY, W, dX, rows, n, segs, dim, static_cast<hipStream_t>(stream));
+}
+long long spion_project_workspace(long long rows, int outputs, int dim) { return project_workspace(rows, outputs, dim); }
+int spion_project_backward_weight(const float* dY, const float* X, float* dW, float* db, float* workspace, long long rows,
+                                  int outputs, int dim, void* stream) {
+    note_current_handle(nullptr);
+    return project_backward_weight(dY, X, dW, db, workspace, rows, outputs, dim, static_cast<hipStream_t>(stream));
+}
+int spion_key_penalty(const float* mask, float* penalty, int batch, int heads, int seq_len, void* stream) {
+    note_current_handle(nullptr);
+    return key_penalty(mask, penalty, batch, heads, seq_len, static_cast<hipStream_t>(stream));
+}
 
 // ---- pattern discovery ---------------------------------------------------------------------------
 int spion_pattern_generate_maps(const float* const* Score, int n_maps, int seq_len, int block_size, int conv_ksize,

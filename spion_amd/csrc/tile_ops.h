@@ -10,6 +10,8 @@ namespace spion {
 // =================================================================================================
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
@@ -46,6 +48,84 @@ __device__ __forceinline__ int xcd_remap(int pid, int total) {
 // A contraction over the 32 keys/queries of a tile is a chain of 16 instructions in which slot (s, h)
 // stands for tile row acc_row(s, h): the accumulator of the first product is then already the A
 // operand of the second one, register for register, and nothing goes through LDS.
+
+// =================================================================================================
+// fp32 products on the bf16 matrix pipe
+// =================================================================================================
+// A float is the exact sum of three bf16 numbers -- hi = bf16(x), mid = bf16(x - hi), lo = x - hi - mid, all rounded
+// to nearest: 8 + 8 + 8 significant bits, the signs of mid and lo taking up what rounding up borrows -- and a product
+// of two bf16 numbers is exact in fp32.  Of the nine partial products of a . b the six with hi.hi, hi.mid, mid.hi,
+// mid.mid, hi.lo and lo.hi are formed; the other three are below 2^-25 of |a||b|, less than the rounding of one fp32
+// product.  Sums are accumulated in fp32 by the MFMA as before.  Measured against float64 on MI355X (32x32x32
+// products of normal, positive, wide-range and one-signed operands, 1 to 128 of them accumulated): relative error
+// 3.8e-8 against 1.0e-7 of the v_mfma_f32_32x32x2_f32 chain for one product, 1.02e-6 against 1.15e-6 for 128; all
+// nine partial products give the same figures as six.
+// Why: v_mfma_f32_32x32x16_bf16 does sixteen times the work of v_mfma_f32_32x32x2_f32 in half its time, so six of
+// them per 16 terms take 384 cycles for a 32x32x32 product instead of 1024; they overlap with vector-ALU work, which
+// the fp32 MFMA does not, so that the splitting (88 instructions per 16 floats and lane) is mostly hidden; and they
+// draw less power: under sustained load the fp32 chain takes 435 to 755 ns per product and SIMD (the clock drops), the
+// six-product chain 217 ns, 280 ns with one operand split on the way.
+// Range: an infinite operand gives NaN; |x| >= 2^128 - 2^119 rounds to an infinite hi (fp32 overflow is 2^128); below 2^-110 the lo part is
+// subnormal or lost, an absolute error under 2^-133.
+template <int N>
+struct Split3 {
+    bf16x8 p[3][N / 8];  // hi, mid, lo of elements 8t .. 8t+7
+};
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+    bf16x2 v;
+    v[0] = (__bf16)a;
+    v[1] = (__bf16)b;
+    unsigned u = __builtin_bit_cast(unsigned, v);
+    asm("" : "+v"(u));  // the compiler would otherwise convert a and b once more, one at a time, to widen them again
+    return u;
+}
+__device__ __forceinline__ float bf16_lo(unsigned u) { return __builtin_bit_cast(float, u << 16); }
+__device__ __forceinline__ float bf16_hi(unsigned u) { return __builtin_bit_cast(float, u & 0xffff0000u); }
+template <int N>
+__device__ __forceinline__ Split3<N> split3(const float (&x)[N]) {
+    typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+    Split3<N> s;
+#pragma unroll
+    for (int t = 0; t < N / 8; ++t) {
+        u32x4_t hi, mid, lo;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float a = x[8 * t + 2 * j], b = x[8 * t + 2 * j + 1];
+            hi[j] = pack_bf16(a, b);
+            a -= bf16_lo(hi[j]);
+            b -= bf16_hi(hi[j]);
+            mid[j] = pack_bf16(a, b);
+            a -= bf16_lo(mid[j]);
+            b -= bf16_hi(mid[j]);
+            lo[j] = pack_bf16(a, b);
+        }
+        s.p[0][t] = __builtin_bit_cast(bf16x8, hi);
+        s.p[1][t] = __builtin_bit_cast(bf16x8, mid);
+        s.p[2][t] = __builtin_bit_cast(bf16x8, lo);
+    }
+    return s;
+}
+__device__ __forceinline__ f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+// acc += A.B over the N slots of each half-wave (small partial products first)
+template <int N>
+__device__ __forceinline__ f32x16 mma_split(const Split3<N>& a, const Split3<N>& b, f32x16 acc) {
+#pragma unroll
+    for (int t = 0; t < N / 8; ++t) {
+        acc = mfma_bf16(a.p[2][t], b.p[0][t], acc);
+        acc = mfma_bf16(a.p[0][t], b.p[2][t], acc);
+        acc = mfma_bf16(a.p[1][t], b.p[1][t], acc);
+    }
+#pragma unroll
+    for (int t = 0; t < N / 8; ++t) {
+        acc = mfma_bf16(a.p[1][t], b.p[0][t], acc);
+        acc = mfma_bf16(a.p[0][t], b.p[1][t], acc);
+    }
+#pragma unroll
+    for (int t = 0; t < N / 8; ++t) acc = mfma_bf16(a.p[0][t], b.p[0][t], acc);
+    return acc;
+}
 
 template <int D>
 __device__ __forceinline__ void load_rows(const float* __restrict__ X, int row0, int li, int h, float (&x)[D / 2]) {

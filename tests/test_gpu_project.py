@@ -1,0 +1,128 @@
+"""Projection kernels (spion_project_*) and the layer that runs on them, against float64 (GPU box only)."""
+import ctypes
+
+import pytest
+import torch
+
+import spion_amd
+from spion_amd import _lib, workloads
+
+pytestmark = pytest.mark.gpu
+
+
+def _ptrs(ts):
+    return (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+
+
+def _check(got, a, b, extra=None, pieces=1):
+    """got = a @ b (+ extra): every fp32 accumulation step rounds by at most 2^-24 of the running sum of magnitudes; a
+    reduction index takes 12/32 matrix instructions, each of which adds once to the accumulator, the six dropped or
+    rounded partial products of an element pair stay below 2^-24 of it, and pieces are added once more each."""
+    a, b = a.double(), b.double()
+    ref, mag = a @ b, a.abs() @ b.abs()
+    if extra is not None:
+        ref, mag = ref + extra.double(), mag + extra.double().abs()
+    steps = 12 * a.shape[-1] / 32 + pieces + 2
+    assert bool(((got.double() - ref).abs() <= steps * 2.0 ** -24 * mag).all()), float(((got.double() - ref).abs() / mag).max())
+
+
+# tile edges (64 and 128), odd numbers of 32-blocks, one segment and three, many pieces, the 128 x 128 tiles
+@pytest.mark.parametrize("rows,dim,n,segs", [(32, 32, 32, 1), (64, 32, 32, 3), (96, 64, 32, 2), (1056, 96, 96, 3), (4000, 64, 64, 3),
+                                             (65536, 64, 64, 1), (160, 160, 352, 1), (8192, 512, 512, 3), (65536, 256, 128, 3)])
+def test_projection_kernels_match_float64(rows, dim, n, segs):
+    g = torch.Generator().manual_seed(rows + dim)
+    x = torch.randn(rows, dim, generator=g).cuda()
+    w = [torch.randn(n, dim, generator=g).cuda() for _ in range(segs)]
+    b = [torch.randn(n, generator=g).cuda() for _ in range(segs)]
+    dy = (torch.randn(rows, segs * n, generator=g) + 0.5).cuda()  # a mean: the column sums grow
+    core, stream = _lib.core(), torch.cuda.current_stream().cuda_stream
+    y = torch.full((rows + 1, segs * n), 7.0, device="cuda")
+    assert core.spion_project_forward(x.data_ptr(), _ptrs(w), _ptrs(b), y.data_ptr(), rows, n, segs, dim, stream) == 0
+    assert bool((y[rows] == 7.0).all())  # nothing past the end
+    W, bias = torch.cat(w), torch.cat(b)
+    _check(y[:rows], x, W.t(), bias)
+    dx = torch.full((rows + 1, dim), 7.0, device="cuda")
+    assert core.spion_project_backward_input(dy.data_ptr(), _ptrs(w), dx.data_ptr(), rows, n, segs, dim, stream) == 0
+    assert bool((dx[rows] == 7.0).all())
+    _check(dx[:rows], dy, W)
+    N = segs * n
+    got = []
+    for _ in range(2):
+        dw = torch.full((N * dim + 4,), 7.0, device="cuda")
+        db = torch.full((N + 4,), 7.0, device="cuda")
+        ws = torch.empty(core.spion_project_workspace(rows, N, dim), device="cuda")
+        assert core.spion_project_backward_weight(dy.data_ptr(), x.data_ptr(), dw.data_ptr(), db.data_ptr(), ws.data_ptr(), rows,
+                                                  N, dim, stream) == 0
+        assert bool((dw[N * dim:] == 7.0).all()) and bool((db[N:] == 7.0).all())
+        got.append((dw[: N * dim].view(N, dim), db[:N]))
+    _check(got[0][0], dy.t(), x, pieces=256)
+    _check(got[0][1][:, None], dy.t(), torch.ones(rows, 1, device="cuda"), pieces=256 + rows)
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+def test_weight_gradient_of_one_signed_data_keeps_fp32_accuracy():
+    """All operands just above a bf16 number, summed over many rows: the small partial products then share a sign and must
+    not be lost against the large sum."""
+    rows = 131072
+    dy = torch.full((rows, 32), 1.0 + 3 * 2.0 ** -16, device="cuda")
+    x = torch.full((rows, 32), 1.0 + 3 * 2.0 ** -16, device="cuda")
+    core, stream = _lib.core(), torch.cuda.current_stream().cuda_stream
+    dw, db = torch.empty(32, 32, device="cuda"), torch.empty(32, device="cuda")
+    ws = torch.empty(core.spion_project_workspace(rows, 32, 32), device="cuda")
+    assert core.spion_project_backward_weight(dy.data_ptr(), x.data_ptr(), dw.data_ptr(), db.data_ptr(), ws.data_ptr(), rows, 32, 32,
+                                              stream) == 0
+    ref = rows * (1.0 + 3 * 2.0 ** -16) ** 2
+    assert float((dw.double() - ref).abs().max()) / ref < 2e-6  # 512 rows a piece and 256 pieces: about 30 roundings of 2^-24
+
+
+@pytest.mark.parametrize("heads", [1, 2, 5])
+def test_key_penalty_is_the_modules_expression(heads):
+    mask = workloads.valid_length_mask(3, 96, 10, 96, seed=1).cuda()
+    mask[0, 0] = 0.25
+    pen = torch.empty(3, heads * 96, device="cuda")
+    assert _lib.core().spion_key_penalty(mask.data_ptr(), pen.data_ptr(), 3, heads, 96, torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(pen, 1e6 * (1.0 - mask.repeat(1, heads)))
+
+
+@pytest.mark.parametrize("heads,d,L,masked", [(2, 32, 256, False), (1, 32, 288, True), (4, 64, 128, True), (3, 32, 160, False)])
+def test_layer_in_one_call_matches_its_steps(heads, d, L, masked):
+    """The compiled whole-layer path against the same layer run step by step (torch projections), with and without
+    gradients; a frozen weight gets none; a hook on a submodule switches to the steps."""
+    if _lib.autograd_node() is None:
+        pytest.skip("SPION_PY_NODE=1")
+    B, bs = 3, 32
+    cfg = dict(head_dim=d, num_head=heads, max_seq_len=L, batch_size=B, block_size=bs, transformer_dim=96, attention_dropout=0.0,
+               task="lra-text" if masked else "lra-image")
+    torch.manual_seed(heads)
+    layer = spion_amd.Attention(cfg, inference=True).cuda()
+    layer.reconstruct_for_blocksparse(cfg)
+    mat = torch.from_numpy(workloads.band_random_block_mask(L // bs, 1, extra_frac=0.2, seed=3)).cuda()
+    mask = workloads.valid_length_mask(B, L, L // 2, L, seed=5).cuda()
+    x, dy = torch.randn(B, L, 96, device="cuda", requires_grad=True), torch.randn(B, L, 96, device="cuda")
+
+    def run():
+        x.grad = None
+        layer.zero_grad(set_to_none=True)
+        y, p = layer(x, mask, mat)
+        y.backward(dy)
+        return [y.detach(), p] + [x.grad] + [t.grad for t in layer.parameters()]
+
+    fused = [t.detach() if isinstance(t, torch.Tensor) else t for t in run()]
+    with torch.no_grad():
+        y0, p0 = layer(x, mask, mat)
+    assert torch.equal(y0, fused[0]) and (masked or torch.equal(p0, fused[1]))
+    calls = []
+    hook = layer.ff.register_forward_hook(lambda *a: calls.append(1))
+    steps = [t.detach() if isinstance(t, torch.Tensor) else t for t in run()]
+    assert calls
+    hook.remove()
+    for a, b in zip(fused, steps):
+        if isinstance(a, int):
+            assert a == b == 0
+            continue
+        assert a.shape == b.shape
+        assert float((a - b).norm() / b.norm()) < 2e-6  # both fp32 throughout
+    layer.W_k.weight.requires_grad_(False)
+    again = run()
+    assert layer.W_k.weight.grad is None
+    assert torch.equal(again[2], fused[2])
