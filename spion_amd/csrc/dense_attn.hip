@@ -5,7 +5,8 @@
 // models/attention_cuda.py:18-74): Qt/Vt/dOt and all gradients are feature-major [NB][d][L], K (forward) and
 // V (backward) are row-major [NB][L][d], and the map is stored key-major: Attn[h][j][i] = P[i][j].
 // One work-group owns 32 queries (forward, row pass) or 32 keys (column pass) of one head and walks all
-// L/32 tiles of the other dimension with v_mfma_f32_32x32x2_f32; see tile_ops.h for the register layout.
+// L/32 tiles of the other dimension; see tile_ops.h for the register layout, tile_kernels.h (mma_feat_init) for which
+// products run on the fp32 and which, with split operands, on the bf16 matrix pipe.
 #include "common.h"
 #include "tile_kernels.h"
 #include "../../include/spion_hip.h"
@@ -159,6 +160,7 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg_kernel(
     else ldr_cols<D>(rQ, L, (h * KH * L + li) * 4, I * 128, q);
 #pragma unroll
     for (int s = 0; s < KH; ++s) q[s] *= c2;
+    const Split3<KH> qs = split3(q);
 
     float m = -10.f * LOG2E, z = 0.f;  // models/attn.cu:17
     f32x16 S[MAXT];
@@ -198,7 +200,7 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg_kernel(
                 }
                 wait_lgkm0();  // the tile's space is requested again one iteration on
                 __builtin_amdgcn_sched_barrier(0);
-                S[u] = mma_feat_init<D>(kf, q, init);  // S^T: register = key, lane = query
+                S[u] = mma_feat_init<D>(kf, qs, init);  // S^T: register = key, lane = query
                 m = max16(S[u], m);
             }
         }
@@ -342,7 +344,8 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
     ldr_rows<D>(make_rsrc(Q + ib, hbytes), (li * ild + h * KH) * 4, I * 32 * ild * 4, q);
 #pragma unroll
     for (int s = 0; s < KH; ++s) q[s] *= c2;
-    settle(q);
+    const Split3<KH> qs = split3(q);
+    settle(qs);
 
     float m = -10.f * LOG2E, z = 0.f;  // models/attn.cu:17
     f32x16 S[MAXT];
@@ -375,7 +378,7 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
                 wait_lgkm0();
                 if (u + 1 < MAXT && u + 1 < nu) issue_k(u + 1);
                 __builtin_amdgcn_sched_barrier(0);
-                S[u] = mma_feat_init<D>(kf, q, init);  // S^T: register = key, lane = query
+                S[u] = mma_feat_init<D>(kf, qs, init);  // S^T: register = key, lane = query
                 m = max16(S[u], m);
             }
         }
@@ -433,11 +436,9 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
                 wait_lgkm0();
                 if (u + 1 < MAXT && u + 1 < nu) issue(wV, w + (u + 1) * WAVES);
                 __builtin_amdgcn_sched_barrier(0);
+                const Split3<16> ps = split3(p);
 #pragma unroll
-                for (int c = 0; c < 2; ++c)
-#pragma unroll
-                    for (int s = 0; s < 16; ++s)
-                        o[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[c][s], p[s], o[c], 0, 0, 0);
+                for (int c = 0; c < 2; ++c) o[c] = mma_split(split3(vb[c]), ps, o[c]);
                 str_tile_lin(rA, alin, (J * 32 * L + I * 32) * 4, L, pl);
             }
         }
@@ -496,6 +497,7 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
     else ldr_cols<D>(rQ, L, (h * KH * L + li) * 4, I * 128, q);
 #pragma unroll
     for (int s = 0; s < KH; ++s) q[s] *= c2;
+    const Split3<KH> qs = split3(q);
 
     struct Pre1 {
         f32x4 k[4];
@@ -535,7 +537,7 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
 #pragma unroll
                     for (int r = 0; r < 16; ++r) init[r] = -LOG2E * c.pj[r];
                 }
-                const f32x16 S = mma_feat_init<D>(kf, q, init);  // register = key, lane = query
+                const f32x16 S = mma_feat_init<D>(kf, qs, init);  // register = key, lane = query
                 const float mn = max16(S, m);
                 z *= __builtin_amdgcn_exp2f(m - mn);
                 m = mn;
@@ -595,7 +597,7 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
 #pragma unroll
                     for (int r = 0; r < 16; ++r) init[r] -= LOG2E * c.pj[r];
                 }
-                const f32x16 S = mma_feat_init<D>(kf, q, init);  // logits minus the row maximum
+                const f32x16 S = mma_feat_init<D>(kf, qs, init);  // logits minus the row maximum
                 float p[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(S[r]) * rinv;
@@ -751,13 +753,13 @@ __global__ __launch_bounds__(64 * DENSE_WAVES) void dense_bwd_col_kernel(
 // the initial accumulator of the dP chain; the 1/sqrt(d) is applied to the 32 x d results.
 // RM: K, dO, Out (OutCopy) and dQ are row-major head slices located by `ly`, V as well.
 template <int WAVES, bool RM = false>
-SPION_TILE_KERNEL(WAVES) void dense_bwd_row32_kernel(
+SPION_TILE_KERNEL_D(WAVES, 32) void dense_bwd_row32_kernel(
     const float* __restrict__ Kt, const float* __restrict__ V, const float* __restrict__ Attn,
     const float* __restrict__ dOt, const float* __restrict__ OutCopy, float* __restrict__ G,
     float* __restrict__ dQ, int L, int nbr, int NB, float scale, Layouts ly) {
     constexpr int D = 32, KH = 16;
-    __shared__ float lds[WAVES * 16 * 64];
     __shared__ __attribute__((aligned(16))) float lds_t[WAVES][3 * 1024];
+    float* lds = &lds_t[0][0];  // the final reduction, a barrier after the last tile
     // last head first: the tail of the map is what the memory-side cache still holds after the forward
     const int item = xcd_remap(blockIdx.x, nbr * NB);
     const int bh = NB - 1 - item / nbr, I = item % nbr;
@@ -788,6 +790,7 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_row32_kernel(
     g += __shfl_xor(g, 32, 64);
     if (w == 0 && h == 0) G[(size_t)bh * L + I * 32 + li] = -g;
     const f32x16 gneg = splat16(-g);
+    const Split3<KH> gos = split3(go);
 
     f32x16 acc = splat16(0.f);  // dQ^T: register = feature, lane = query
     // The V, map and K tiles go straight into wave-private LDS; the operands of tile i are read out into registers,
@@ -820,27 +823,27 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_row32_kernel(
             wait_lgkm0();
             if (i + 1 < nu) issue(w + (i + 1) * WAVES);
             __builtin_amdgcn_sched_barrier(0);
-            f32x16 dp = mma_feat_init<D>(vt, go, gneg);  // register = key, lane = query: dO_i . v_j - g_i
+            f32x16 dp = mma_feat_init<D>(vt, gos, gneg);  // register = key, lane = query: dO_i . v_j - g_i
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
-#pragma unroll
-            for (int s = 0; s < 16; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kb[s], ds[s], acc, 0, 0, 0);
+            acc = mma_split(split3(kb), split3(ds), acc);
         }
     }
+    if (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
     f32x16 out[1] = {acc * scale};
     if constexpr (RM) reduce_store_rows<WAVES>(out[0], dQ + gb, I * 32, w, li, h, lds, gld);
     else reduce_store<D, WAVES, true>(out, dQ + hb, I * 32, w, li, h, lds, L);
 }
 
 template <int WAVES, bool RM = false>
-SPION_TILE_KERNEL(WAVES) void dense_bwd_col32_kernel(
+SPION_TILE_KERNEL_D(WAVES, 32) void dense_bwd_col32_kernel(
     const float* __restrict__ Qt, const float* __restrict__ V, const float* __restrict__ Attn,
     const float* __restrict__ dOt, const float* __restrict__ G, float* __restrict__ dK, float* __restrict__ dV,
     int L, int nbr, int NB, float scale, Layouts ly) {
     constexpr int D = 32, KH = 16;
-    __shared__ float lds[WAVES * 16 * 64];
     __shared__ __attribute__((aligned(16))) float lds_t[WAVES][3 * 1024 + 64];
+    float* lds = &lds_t[0][0];  // the final reductions, a barrier after the last tile
     const int item = xcd_remap(blockIdx.x, nbr * NB);
     const int bh = item / nbr, J = item % nbr;
     const int w = wave_index(), l = threadIdx.x & 63, h = l >> 5, li = l & 31;
@@ -891,7 +894,8 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_col32_kernel(
         DmaTileF32::load(wQ, lq, ql, I * QSTEP, qx);
         dma_b32(wG, lg, l * 4, I * 128);
     };
-    settle(v);
+    const Split3<KH> vs = split3(v);
+    settle(vs);
     if (nu > 0) {
         issue(w);
         for (int i = 0; i < nu; ++i) {
@@ -913,7 +917,7 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_col32_kernel(
             wait_lgkm0();
             if (i + 1 < nu) issue(w + (i + 1) * WAVES);
             __builtin_amdgcn_sched_barrier(0);
-            f32x16 dp = mma_feat_init<D>(go, v, init);  // register = query, lane = key
+            f32x16 dp = mma_feat_init<D>(go, vs, init);  // register = query, lane = key
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * p[r];
@@ -923,6 +927,7 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_col32_kernel(
             for (int s = 0; s < 16; ++s) av = __builtin_amdgcn_mfma_f32_32x32x2f32(ob[s], p[s], av, 0, 0, 0);
         }
     }
+    if (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
     f32x16 out[1] = {ak * scale};
     if constexpr (RM) {
         reduce_store_rows<WAVES>(out[0], dK + gb, J * 32, w, li, h, lds, gld);
@@ -968,6 +973,7 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_row64_kernel(
     g += __shfl_xor(g, 32, 64);
     if (w == 0 && h == 0) G[(size_t)bh * L + I * 32 + li] = -g;
     const f32x16 gneg = splat16(-g);
+    const Split3<KH> gos = split3(go);
 
     f32x16 acc[2] = {splat16(0.f), splat16(0.f)};  // dQ: register = query, lane = feature
     const char* Tv = smem + w * WB;
@@ -1000,11 +1006,11 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_row64_kernel(
             wait_lgkm0();
             if (i + 1 < nu) issue(w + (i + 1) * WAVES);
             __builtin_amdgcn_sched_barrier(0);
-            f32x16 dp = mma_feat_init<D>(vt, go, gneg);  // register = key, lane = query: dO_i . v_j - g_i
+            f32x16 dp = mma_feat_init<D>(vt, gos, gneg);  // register = key, lane = query: dO_i . v_j - g_i
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
-            mma_b<D>(ds, kb, acc);
+            mma_b_split<D>(ds, kb, acc);
         }
     }
     if (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
@@ -1058,7 +1064,8 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_col64_kernel(
         DmaTileF32::load(wO, lo, ol, I * 32 * old_ * 4, ox);
         DmaTileF32::load(wO, lo + DmaTileF32::TILE, ol, I * 32 * old_ * 4 + 128, ox);
     };
-    settle(vt);
+    const Split3<KH> vts = split3(vt);
+    settle(vts);
     if (nu > 0) {
         issue(w);
         float gl = ld1(rG, li * 4, w * 128);
@@ -1080,12 +1087,12 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_col64_kernel(
             }
             __builtin_amdgcn_sched_barrier(0);
             const f32x16 init = __builtin_amdgcn_mfma_f32_32x32x2f32(ga, 1.0f, splat16(0.f), 0, 0, 0);  // -g_i in every column
-            f32x16 dp = mma_feat_init<D>(go, vt, init);  // register = query, lane = key
+            f32x16 dp = mma_feat_init<D>(go, vts, init);  // register = query, lane = key
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pc[r];
-            mma_b<D>(ds, qb, ak);
-            mma_b<D>(pc, ob, av);
+            mma_b_split<D>(ds, qb, ak);
+            mma_b_split<D>(pc, ob, av);
         }
     }
     if (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles

@@ -278,6 +278,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
     ldr_rows<D>(rQ, (li * ild + h * KH) * 4, I * tile_bytes, q);
 #pragma unroll
     for (int s = 0; s < KH; ++s) q[s] *= c2;
+    const Split3<KH> qs = split3(q);
     const float2 rem = Stats[(size_t)bh * L + I * 32 + li];  // the remainder of row li
 
     // ---- index of this wavefront's tiles (positions past the end repeat the last one: valid, redundant) -----
@@ -318,7 +319,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
             lds_put_lin(Tx, l, raw[u & 1]);
             float kf[KH];
             lds_get_feat32(Tx, li, h, kf);
-            S[u] = mma_feat_init<D>(kf, q, init);  // register = key acc_row(r, h), lane = query li
+            S[u] = mma_feat_init<D>(kf, qs, init);  // register = key acc_row(r, h), lane = query li
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 if (!((bits_l[u] >> acc_row(r, h)) & 1u)) S[u][r] = HYB_ABSENT;
@@ -479,6 +480,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_row_kernel(const float* __restrict__ K
     g += __shfl_xor(g, 32, 64);
     if (w == 0 && h == 0) G[(size_t)bh * L + I * 32 + li] = -g;
     const f32x16 gneg = splat16(-g);
+    const Split3<KH> gos = split3(go);
 
     const int t0 = ix.t_rp[I], cnt = ix.t_rp[I + 1] - t0;
     const int n = cnt > w ? (cnt - w + WAVES - 1) / WAVES : 0;
@@ -505,7 +507,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_row_kernel(const float* __restrict__ K
             lds_get_feat32(Tx, li, h, vt);
             lds_put_cols(T, li, h, x.p);
             lds_get_rows(T, li, h, pr);                        // pr[r] = P[query li][key acc_row(r, h)]
-            const f32x16 dp = mma_feat_init<D>(vt, go, gneg);  // dp[r] = dO_i . v_j - g_i
+            const f32x16 dp = mma_feat_init<D>(vt, gos, gneg);  // dp[r] = dO_i . v_j - g_i
             lds_put_lin(Tx, l, x.b);
             lds_get_cols(Tx, li, h, kb[0]);
             float ds[16];
@@ -601,6 +603,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_col_kernel(const float* __restrict__ Q
 
     float vt[KH];
     ldr_rows<D>(rV, (li * ild + h * KH) * 4, J * 32 * ild * 4, vt);
+    const Split3<KH> vts = split3(vt);
 
     f32x16 ak[1] = {splat16(0.f)}, av[1] = {splat16(0.f)};
     const int e0 = ix.t_cp[J], ecnt = ix.t_cp[J + 1] - e0;
@@ -634,7 +637,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_col_kernel(const float* __restrict__ Q
             f32x16 init;
 #pragma unroll
             for (int r = 0; r < 16; ++r) init[r] = __builtin_bit_cast(float, gn[r]);
-            const f32x16 dp = mma_feat_init<D>(go, vt, init);  // dO_i . v_j - g_i, i = acc_row(r, h), j = li
+            const f32x16 dp = mma_feat_init<D>(go, vts, init);  // dO_i . v_j - g_i, i = acc_row(r, h), j = li
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * x.p[r];

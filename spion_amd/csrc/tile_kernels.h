@@ -2,7 +2,9 @@
 //
 // What shapes these kernels (measured on MI355X): an fp32 MFMA and ordinary vector-ALU instructions
 // do not overlap on a SIMD -- every VALU instruction adds its ~4-5 cycles (v_exp_f32 ~13) to the 64 cycles
-// of each v_mfma_f32_32x32x2_f32 -- while memory instructions issue for free.  So the kernels
+// of each v_mfma_f32_32x32x2_f32 -- while memory instructions issue for free; on the bf16 pipe they do overlap, but
+// an fp32 operand has to be split for it (88 VALU instructions).  Which product runs where: see mma_feat_init.  VALU
+// instructions being what both are short of, the kernels
 //   * do all addressing in scalar registers: buffer loads/stores with a per-head resource, one lane
 //     offset computed once per kernel and a scalar byte offset per tile;
 //   * fold constants into the MFMA chain instead of touching every element afterwards: the row maximum
@@ -28,6 +30,9 @@
 namespace spion {
 
 #define SPION_TILE_KERNEL(W) __global__ __launch_bounds__(64 * (W)) __attribute__((amdgpu_waves_per_eu(2, 2)))
+// three wavefronts per SIMD (d = 32), two (d = 64)
+#define SPION_TILE_KERNEL_D(W, D) \
+    __global__ __launch_bounds__(64 * (W)) __attribute__((amdgpu_waves_per_eu((D) == 32 ? 3 : 2, (D) == 32 ? 3 : 2)))
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
@@ -266,6 +271,13 @@ __device__ __forceinline__ void settle(const float (&x)[N]) {
 #pragma unroll
     for (int t = 0; t < N; ++t) asm volatile("" ::"v"(x[t]));
 }
+template <int N>
+__device__ __forceinline__ void settle(const Split3<N>& x) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int t = 0; t < N / 8; ++t) asm volatile("" ::"v"(x.p[k][t]));
+}
 // 64 floats (lane l: 4 bytes at voff) to 256 bytes of LDS
 __device__ __forceinline__ void dma_b32(u32x4 r, unsigned lds, int voff, int soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r),
@@ -377,20 +389,75 @@ struct DmaTileF32 {
     }
 };
 
-// acc = init + A.B over the head dimension (chain of D/2 MFMA).
+// Which pipe a product runs on.  On the bf16 pipe (mma_split, tile_ops.h: the accuracy of the fp32 chain) a 32 x 32 x 32
+// product takes 384 cycles instead of 1024 and overlaps with vector-ALU work, but each operand that is not kept costs
+// 88 vector-ALU instructions to split, some 370 cycles, and these draw enough power to lower the clock (measured: 2.4
+// GHz under fp32 chains, 1.98 to 2.2 GHz with every product split).  So
+//   * products over the head dimension, whose other operand a wavefront keeps for all its tiles, are split: one
+//     operand per tile;
+//   * products over a tile's rows, which need two operands split, run on the bf16 pipe at d = 64 (one of the two
+//     serves two products) and in the column pass (two of its three products; three wavefronts per SIMD hide the
+//     splitting), on the fp32 pipe in the forward and the row pass at d = 32.
+// Measured in us per launch, all fp32 / all split / as chosen: 32 x 2 heads of 4096 tokens, d = 32, 32 x 32 blocks, a
+// tenth kept: forward 162 / 176 / 150, row pass 141 / 134 / 130, column pass 185 / 168 / 168; 256 x 2 heads of 1024:
+// 143 / 140 / 134, 122 / 118 / 117, 147 / 133 / 133; 3 x 8 heads of 4000, d = 64, all fp32 / split: 98 / 75, 99 / 82,
+// 119 / 116.  The dense kernels (dense_attn.hip, 64 x 2 heads of 1024): forward 181 / 172 / 171, row pass (split)
+// 178 / 155, column pass 236 / 260 / 211 (its three splits do not fit the registers of three wavefronts per SIMD).
+// Against float64 the outputs and gradients of both are as close as the fp32 chains' or closer (2-norms, 1024 to 4096
+// tokens: 1.0e-7 to 5.8e-7 where those gave 2.2e-7 to 6.1e-7).
+// acc = init + A.B over the head dimension; B is an operand the kernel keeps.
 template <int D>
-__device__ __forceinline__ f32x16 mma_feat_init(const float (&a)[D / 2], const float (&b)[D / 2], f32x16 init) {
-    f32x16 acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[0], b[0], init, 0, 0, 0);
+__device__ __forceinline__ f32x16 mma_feat_init(const float (&a)[D / 2], const Split3<D / 2>& b, f32x16 init) {
+    if constexpr (D == 64) {  // sixteen slots after the other: the parts of all 32 would be 48 registers
+        f32x16 acc = init;
 #pragma unroll
-    for (int s = 1; s < D / 2; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
+        for (int t = 0; t < 2; ++t) {
+            float x[16];
+            Split3<16> bt;
+#pragma unroll
+            for (int s = 0; s < 16; ++s) x[s] = a[16 * t + s];
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) bt.p[k][j] = b.p[k][2 * t + j];
+            acc = mma_split(split3(x), bt, acc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        return acc;
+    } else {
+        return mma_split(split3(a), b, init);
+    }
+}
+// both on the fp32 pipe
+template <int D>
+__device__ __forceinline__ f32x16 mma_feat_f32(const float (&a)[D / 2], const float (&b)[D / 2], f32x16 init) {
+    f32x16 acc = init;
+#pragma unroll
+    for (int s = 0; s < D / 2; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
     return acc;
 }
 template <int D>
-__device__ __forceinline__ void mma_b(const float (&w)[16], const float (&x)[D / 32][16], f32x16 (&out)[D / 32]) {
+__device__ __forceinline__ void mma_b_f32(const float (&w)[16], const float (&x)[D / 32][16], f32x16 (&out)[D / 32]) {
 #pragma unroll
     for (int c = 0; c < D / 32; ++c)
 #pragma unroll
         for (int s = 0; s < 16; ++s) out[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[s], x[c][s], out[c], 0, 0, 0);
+}
+// out[c] += W.X over the 32 rows of a tile, on the bf16 pipe
+template <int D>
+__device__ __forceinline__ void mma_b_split(const float (&w)[16], const float (&x)[D / 32][16], f32x16 (&out)[D / 32]) {
+    const Split3<16> ws = split3(w);
+#pragma unroll
+    for (int c = 0; c < D / 32; ++c) {
+        if (c) __builtin_amdgcn_sched_barrier(0);
+        out[c] = mma_split(ws, split3(x[c]), out[c]);
+    }
+}
+// the same on the pipe the forward and the row pass use
+template <int D>
+__device__ __forceinline__ void mma_b(const float (&w)[16], const float (&x)[D / 32][16], f32x16 (&out)[D / 32]) {
+    if constexpr (D == 32) mma_b_f32<D>(w, x, out);
+    else mma_b_split<D>(w, x, out);
 }
 __device__ __forceinline__ f32x16 splat16(float v) {
     return (f32x16){v, v, v, v, v, v, v, v, v, v, v, v, v, v, v, v};
@@ -506,9 +573,9 @@ __device__ __forceinline__ void tile_pipeline(int n, Pre& a, Pre& b, Fetch fetch
 // recomputing the logits (any row length).  Ocache (optional): second copy of O for the backward.
 // -------------------------------------------------------------------------------------------------
 // KROW: the K operand is row-major [NB][L][D] (what a caller has before it makes the transposed copy the
-// reference's ABI asks for) instead of feature-major [NB][D][L].  For d = 64 every lane then reads 128 bytes of
-// its own row (one cache line per lane), which is slower than the feature-major form: the row-major entry points
-// for contiguous heads therefore still transpose once; only the strided entry points use it.
+// reference's ABI asks for) instead of feature-major [NB][D][L].  Tiles that go through LDS cost the same either way;
+// in the two sweeps of d = 64 every lane reads 128 bytes of its own row (one cache line per lane), which is slower
+// than the feature-major form.
 // MAXT <= 6 at d = 32 (at most six logit tiles per wavefront) fits three wavefronts per SIMD: the buffer of the
 // final reduction then shares the space of the wave-private tiles (a barrier in between).
 // LONG (with MAXT > 0): a strip too long for the registers of its wavefronts takes the two sweeps inside the same
@@ -568,6 +635,7 @@ void tile_fwd_kernel(
     ldr_rows<D>(rQ, (li * ild + h * KH) * 4, I * 32 * ild * 4, q);
 #pragma unroll
     for (int s = 0; s < KH; ++s) q[s] *= c2;
+    const Split3<KH> qs = split3(q);
     // operand over the head dimension of key tile J (lane = key, features h*D/2 ..)
     auto load_kf = [&](int J, float (&x)[KH]) {
         if constexpr (KROW) ldr_rows<D>(rK, (li * ild + h * KH) * 4, J * 32 * ild * 4, x);
@@ -591,6 +659,17 @@ void tile_fwd_kernel(
     for (int c = 0; c < D / 32; ++c) o[c] = splat16(0.f);
 
     auto two_sweeps = [&]() {
+        // d = 64: two register sets of a K and a V tile leave no room for split operands; fp32 chains there
+        float qf[D == 64 ? KH : 1];
+        if constexpr (D == 64) {
+            ldr_rows<D>(rQ, (li * ild + h * KH) * 4, I * 32 * ild * 4, qf);
+#pragma unroll
+            for (int s = 0; s < KH; ++s) qf[s] *= c2;
+        }
+        auto logits = [&](const float (&k)[KH], f32x16 init) -> f32x16 {
+            if constexpr (D == 64) return mma_feat_f32<D>(k, qf, init);
+            else return mma_feat_init<D>(k, qs, init);
+        };
         // ---- sweep 1: online row maximum and denominator -------------------------------------------
         const int nu = cnt > w ? (cnt - w + WAVES - 1) / WAVES : 0;  // tiles of this wavefront
         struct PreK {
@@ -614,7 +693,7 @@ void tile_fwd_kernel(
         {
             PreK ka, kb;
             tile_pipeline(nu, ka, kb, fetch_k, [&](PreK& c, int) {
-                f32x16 s = mma_feat_init<D>(c.k, q, init_of(c, 0.f));
+                f32x16 s = logits(c.k, init_of(c, 0.f));
                 const float tm = max16(s, m);
                 float zz = 0.f;
 #pragma unroll
@@ -640,12 +719,12 @@ void tile_fwd_kernel(
                     ldr_tile_b<D>(rV, b_voff, tcol[t0 + w + min(i, nu - 1) * WAVES] * 32 * ild * 4, x.vb, ild);
                 },
                 [&](PreKV& c, int i) {
-                    f32x16 s = mma_feat_init<D>(c.k.k, q, init_of(c.k, m));
+                    f32x16 s = logits(c.k.k, init_of(c.k, m));
                     float p[16];
 #pragma unroll
                     for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(s[r]) * rinv;
                     store_p(p, w + i * WAVES);
-                    mma_b<D>(p, c.vb, o);
+                    mma_b_f32<D>(p, c.vb, o);
                 });
         }
     };
@@ -709,7 +788,7 @@ void tile_fwd_kernel(
                     }
                     wait_lgkm0();  // the tile's space is requested again one iteration on
                     __builtin_amdgcn_sched_barrier(0);
-                    S[u] = mma_feat_init<D>(kf, q, init);
+                    S[u] = mma_feat_init<D>(kf, qs, init);
                     m = max16(S[u], m);
                 }
             }
@@ -753,7 +832,7 @@ void tile_fwd_kernel(
                     wait_lgkm0();
                     if (u + 1 < MAXT && u + 1 < nu) issue_k(u + 1 < MAXT ? u + 1 : u);
                     __builtin_amdgcn_sched_barrier(0);
-                    S[u] = mma_feat_init<D>(kf, q, init);
+                    S[u] = mma_feat_init<D>(kf, qs, init);
                     m = max16(S[u], m);
                 }
             }
@@ -883,18 +962,16 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
     int L, int nbr, int NB, int nnz, float scale, int hc, Layouts ly, int s0, int ns) {
     static_assert(!ST || (VROW && HAVE_O), "strided heads: row-major operands, Out given");
     constexpr int KH = D / 2;
-    // LDS of a wavefront: the V, P and K tiles of one pattern tile, 4 KB per 32 features.  d = 64 needs 20 KB, which
-    // eight wavefronts per CU fill to the last byte: the buffer of the final reduction and the partial row sums
-    // of the first sweep then lie inside that space (CARVE), each separated from the tiles by a barrier.
-    constexpr bool CARVE = D == 64;
+    // LDS of a wavefront: the V, P and K tiles of one pattern tile, 4 KB per 32 features: 12 KB (d = 32, twelve
+    // wavefronts per CU) or 20 KB (d = 64, eight, which fill the LDS to the last byte).  The buffer of the final
+    // reduction and the partial row sums of the first sweep lie inside that space, each separated from the tiles by
+    // a barrier.
     constexpr int WB = (1 + 2 * (D / 32)) * DmaTileF32::TILE;
     constexpr int RED = WAVES > 1 ? WAVES * (D / 32) * 16 * 64 * 4 : 0;
-    static_assert(!CARVE || RED <= WAVES * WB, "the reduction fits in the tile space");
-    __shared__ __attribute__((aligned(16))) char smem[CARVE ? WAVES * WB : WAVES * WB + RED + WAVES * 128];
-    float* lds = reinterpret_cast<float*>(CARVE ? smem : smem + WAVES * WB);
-    auto lds_g = [&](int ww) {
-        return reinterpret_cast<float*>(CARVE ? smem + ww * WB + WB - 128 : smem + WAVES * WB + RED + ww * 128);
-    };
+    static_assert(RED <= WAVES * WB, "the reduction fits in the tile space");
+    __shared__ __attribute__((aligned(16))) char smem[WAVES * WB];
+    float* lds = reinterpret_cast<float*>(smem);
+    auto lds_g = [&](int ww) { return reinterpret_cast<float*>(smem + ww * WB + WB - 128); };
     // Last head first: the forward wrote P front to back, so its tail is what the memory-side cache still holds.
     // This launch covers strips s0 .. s0+ns-1 of every head's strip order.
     const int item = xcd_remap(blockIdx.x, ns * NB);
@@ -927,6 +1004,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
 
     float go[KH];
     ldr_rows<D>(rdO, ro_voff, I * 32 * old_ * 4, go);
+    const Split3<KH> gos = split3(go);
 
     float g = 0.f;
     if (HAVE_O) {
@@ -952,7 +1030,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
             [&](PreG& c, int) {
                 float pr[16];
                 p_rows(c.pv, pr);
-                f32x16 dp = mma_feat_init<D>(c.vt, go, splat16(0.f));
+                f32x16 dp = mma_feat_init<D>(c.vt, gos, splat16(0.f));
 #pragma unroll
                 for (int r = 0; r < 16; ++r) g = fmaf(dp[r], pr[r], g);
             });
@@ -963,7 +1041,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
             g = 0.f;
 #pragma unroll
             for (int ww = 0; ww < WAVES; ++ww) g += lds_g(ww)[li];
-            if constexpr (CARVE) __syncthreads();  // the partial sums lie where tiles are about to land
+            __syncthreads();  // the partial sums lie where tiles are about to land
         }
     }
     if (w == 0 && h == 0) G[(size_t)bh * L + I * 32 + li] = -g;
@@ -1011,7 +1089,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
                 if (i + 1 < nu) issue(w + (i + 1) * WAVES, Jn);
                 Jn = Jnn;
                 __builtin_amdgcn_sched_barrier(0);
-                f32x16 dp = mma_feat_init<D>(vt, go, gneg);  // dp[r] = dO_i . v_j - g_i
+                f32x16 dp = mma_feat_init<D>(vt, gos, gneg);  // dp[r] = dO_i . v_j - g_i
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
@@ -1062,7 +1140,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
                 if (i + 1 < nu) issue(w + (i + 1) * WAVES, Jn);
                 Jn = Jnn;
                 __builtin_amdgcn_sched_barrier(0);
-                f32x16 dp = mma_feat_init<D>(vt, go, gneg);  // dp[r] = dO_i . v_j - g_i
+                f32x16 dp = mma_feat_init<D>(vt, gos, gneg);  // dp[r] = dO_i . v_j - g_i
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
@@ -1070,7 +1148,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
             }
         }
     }
-    if constexpr (CARVE && WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
+    if constexpr (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
 #pragma unroll
     for (int c = 0; c < D / 32; ++c) acc[c] *= scale;
     reduce_store<D, WAVES>(acc, dQ + gb, I * 32, w, li, h, lds, gld);
@@ -1083,7 +1161,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
 // -------------------------------------------------------------------------------------------------
 // VROW: as in the row pass.
 template <int D, int WAVES, bool VROW = false, bool ST = false>
-SPION_TILE_KERNEL(WAVES) void tile_bwd_col_kernel(
+SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
     const float* __restrict__ Q, const float* __restrict__ Vt, const float* __restrict__ P,
     const float* __restrict__ dO, const float* __restrict__ G, float* __restrict__ dK, float* __restrict__ dV,
     const int* __restrict__ cdesc, const int* __restrict__ tcdesc, int L, int nbr, int NB, int nnz, float scale,
@@ -1091,14 +1169,13 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_col_kernel(
     static_assert(!ST || VROW, "strided heads: row-major operands");
     constexpr int KH = D / 2;
     // LDS of a wavefront: d = 32, the P, Q and dO tiles and 64 floats of -g; d = 64, the P tile and two tiles each for
-    // Q and dO, 20 KB, which eight wavefronts per CU fill to the last byte: -g then travels in a register, and the
-    // buffer of the final reductions lies inside the tile space (CARVE), a barrier in between.
-    constexpr bool CARVE = D == 64;
+    // Q and dO, 20 KB, which eight wavefronts per CU fill to the last byte: -g then travels in a register.  The
+    // buffer of the final reductions lies inside the tile space, a barrier in between.
     constexpr int WB = D == 32 ? 3 * DmaTileF32::TILE + 256 : 5 * DmaTileF32::TILE;
     constexpr int RED = WAVES > 1 ? WAVES * (D / 32) * 16 * 64 * 4 : 0;
-    static_assert(!CARVE || RED <= WAVES * WB, "the reduction fits in the tile space");
-    __shared__ __attribute__((aligned(16))) char smem[CARVE ? WAVES * WB : WAVES * WB + (RED ? RED : 4)];
-    float* lds = reinterpret_cast<float*>(CARVE ? smem : smem + WAVES * WB);
+    static_assert(RED <= WAVES * WB, "the reduction fits in the tile space");
+    __shared__ __attribute__((aligned(16))) char smem[WAVES * WB];
+    float* lds = reinterpret_cast<float*>(smem);
     const int item = xcd_remap(blockIdx.x, ns * NB);  // strips s0 .. s0+ns-1 of every head's strip order
     int bh, pos;
     item_to_head_strip(item, ns, hc, bh, pos);
@@ -1157,7 +1234,8 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_col_kernel(
             DmaTileF32::load(wO, lo, ol, I * 32 * old_ * 4, ox);
             dma_b32(wG, lg, l * 4, I * 128);
         };
-        settle(vt);
+        const Split3<KH> vts = split3(vt);
+        settle(vts);
         if (nu > 0) {
             issue(desc[w]);
             int4 dn = desc[w + (nu > 1 ? WAVES : 0)];
@@ -1182,12 +1260,12 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_col_kernel(
                 if (i + 1 < nu) issue(dn);
                 dn = dnn;
                 __builtin_amdgcn_sched_barrier(0);
-                f32x16 dp = mma_feat_init<D>(go, vt, init);  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
+                f32x16 dp = mma_feat_init<D>(go, vts, init);  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pc[r];
-                mma_b<D>(ds, qb, ak);
-                mma_b<D>(pc, ob, av);
+                mma_b_split<D>(ds, qb, ak);
+                mma_b_split<D>(pc, ob, av);
             }
         }
     } else {
@@ -1217,7 +1295,8 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_col_kernel(
             DmaTileF32::load(wO, lo, ol, I * 32 * old_ * 4, ox);
             DmaTileF32::load(wO, lo + DmaTileF32::TILE, ol, I * 32 * old_ * 4 + 128, ox);
         };
-        settle(vt);
+        const Split3<KH> vts = split3(vt);
+        settle(vts);
         if (nu > 0) {
             int4 dn = desc[w];
             issue(dn);
@@ -1243,16 +1322,16 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_col_kernel(
                 dn = dnn;
                 __builtin_amdgcn_sched_barrier(0);
                 const f32x16 init = __builtin_amdgcn_mfma_f32_32x32x2f32(ga, 1.0f, splat16(0.f), 0, 0, 0);  // -g_i in every column
-                f32x16 dp = mma_feat_init<D>(go, vt, init);  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
+                f32x16 dp = mma_feat_init<D>(go, vts, init);  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pc[r];
-                mma_b<D>(ds, qb, ak);
-                mma_b<D>(pc, ob, av);
+                mma_b_split<D>(ds, qb, ak);
+                mma_b_split<D>(pc, ob, av);
             }
         }
     }
-    if constexpr (CARVE && WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
+    if constexpr (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
 #pragma unroll
     for (int c = 0; c < D / 32; ++c) ak[c] *= scale;
     reduce_store<D, WAVES>(ak, dK + gb, J * 32, w, li, h, lds, gld);
