@@ -2,10 +2,10 @@
 //
 // Two kernel families serve the same C ABI:
 //   * tile path    -- the pattern is a union of aligned 32x32 tiles (what a block mask of block size
-//                     32, 64, ... expands to).  Every contraction is a dense 32x32xd product done with
-//                     v_mfma_f32_32x32x2_f32; operands go straight from global memory into the MFMA
-//                     register layout (every access is a coalesced 128-byte row segment), the tile
-//                     list of a block row / block column is walked per wavefront.
+//                     32, 64, ... expands to).  Every contraction is a dense 32x32xd product on the matrix
+//                     cores, in fp32 or with operands split into three bf16 parts (tile_kernels.h); tiles go
+//                     from global memory into LDS or the MFMA register layout in whole 128-byte rows, the
+//                     tile list of a block row / block column is walked per wavefront.
 //   * element path -- any other CSR (element-sparse patterns, odd head sizes): one wavefront per
 //                     row gathers K/V rows; a transposed (CSC) index built on the host once per
 //                     pattern makes dK/dV deterministic without atomics.
@@ -1610,13 +1610,24 @@ void sparse_forward(void* h, const float* Q, const float* Kt, const float* V, co
                 else launch_tile_fwd<32, false, false>(a, Q, Kt, V, nullptr, Attn, Out, Offsets, nnz);
             }
         } else {
-            if (krow) {  // the d = 64 kernels read the transposed operand only: make it
+            // Where logits stay in registers, tiles of a row-major K go through LDS and cost what those of the transposed
+            // copy cost, without the launch that makes it (11 of 98 us at 3 x 8 heads of 4000 tokens).  In the two
+            // sweeps every lane loads its own 128-byte row instead, so a pattern whose strips mostly take them is
+            // given the copy.
+            const bool sweeps = a->pat.max_row_tiles > 16 && a->pat.n_fwd_long24 * 4 >= a->L / 32;
+            if (krow && sweeps) {
                 if (!ensure_ws(&a->ws_trans, (size_t)a->NB * a->L * a->d)) return;
                 if (transpose_last2(Kt, a->ws_trans, a->NB, a->L, a->d, a->hdr.stream) != 0) return;
                 Kt = a->ws_trans;
+                krow = false;
             }
-            if (a->has_mask) launch_tile_fwd<64, true, false>(a, Q, Kt, V, Mask, Attn, Out, Offsets, nnz);
-            else launch_tile_fwd<64, false, false>(a, Q, Kt, V, nullptr, Attn, Out, Offsets, nnz);
+            if (krow) {
+                if (a->has_mask) launch_tile_fwd<64, true, true>(a, Q, Kt, V, Mask, Attn, Out, Offsets, nnz);
+                else launch_tile_fwd<64, false, true>(a, Q, Kt, V, nullptr, Attn, Out, Offsets, nnz);
+            } else {
+                if (a->has_mask) launch_tile_fwd<64, true, false>(a, Q, Kt, V, Mask, Attn, Out, Offsets, nnz);
+                else launch_tile_fwd<64, false, false>(a, Q, Kt, V, nullptr, Attn, Out, Offsets, nnz);
+            }
         }
         check_launch("tile_fwd_kernel");
         return;
@@ -1667,12 +1678,9 @@ void sparse_backward(void* h, const float* Q, const float* K, const float* Vt, c
             if (vrow) launch_tile_bwd<32, true>(a, Q, K, Vt, P, dO, dQ, dK, dV, Offsets, nnz, Out);
             else launch_tile_bwd<32, false>(a, Q, K, Vt, P, dO, dQ, dK, dV, Offsets, nnz, Out);
         } else {
-            if (vrow) {
-                if (!ensure_ws(&a->ws_trans, (size_t)a->NB * a->L * a->d)) return;
-                if (transpose_last2(Vt, a->ws_trans, a->NB, a->L, a->d, a->hdr.stream) != 0) return;
-                Vt = a->ws_trans;
-            }
-            launch_tile_bwd<64, false>(a, Q, K, Vt, P, dO, dQ, dK, dV, Offsets, nnz, Out);
+            // V tiles reach the kernels through LDS in either layout: no transposed copy (11 us of either pass's 90)
+            if (vrow) launch_tile_bwd<64, true>(a, Q, K, Vt, P, dO, dQ, dK, dV, Offsets, nnz, Out);
+            else launch_tile_bwd<64, false>(a, Q, K, Vt, P, dO, dQ, dK, dV, Offsets, nnz, Out);
         }
         check_launch("tile_bwd kernels");
         return;
