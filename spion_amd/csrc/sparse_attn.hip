@@ -590,10 +590,16 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
     for (int i = 0; i < nstrips; ++i) ntiles += ptr[i + 1] - ptr[i];
     const int groups = NB % 8 == 0 ? 8 : 1;  // dies
     const int lanes = std::max(groups, lanes_wanted / groups * groups);
-    // no item much longer than a lane's share of the launch, nor shorter than a few tiles
+    // No item much longer than a lane's share of the launch, nor shorter than an average strip or a few tiles: in a small
+    // launch a lane's share is a strip or less, and cutting every strip in two for it costs more in partial results and
+    // their merging than it balances.  Forward + backward kernels without / with the average as a limit: 8 heads of 8192
+    // tokens (13 tiles a strip) 158 / 86 us, 16 of 2048 97 / 62, 4 of 16384 203 / 114, 9 of 3072 (d = 32) 57 / 47; where
+    // the share is larger (64 heads of 2048, 32 of 16384) nothing changes; half as much again as the average: 90, 63,
+    // 109, 51.
     const long long share = (ntiles * NB + lanes - 1) / lanes;
     const int avg = nstrips ? (int)((ntiles + nstrips - 1) / nstrips) : 0;
-    const int long_len = (int)std::max<long long>(std::min<long long>(std::max(4 * avg + 8, 32), std::max<long long>(share / 2, 8)), 8);
+    const int long_len = (int)std::max<long long>(
+        std::min<long long>(std::max(4 * avg + 8, 32), std::max<long long>(share / 2, avg)), 8);
     struct It {
         int strip, t0, n, kind;
     };

@@ -106,3 +106,17 @@ def test_schedule_rejects_bad_arguments():
     assert core.spion_debug_bf16_plan(None, 2, 0, 4, 8, None, 0, None, 0, None, 0, None, 0, None) == -1
     assert core.spion_debug_bf16_plan(ptr, 2, 0, 0, 8, None, 0, None, 0, None, 0, None, 0, None) == -1
     assert core.spion_debug_bf16_plan(ptr, 2, 0, 4, 0, None, 0, None, 0, None, 0, None, 0, None) == -1
+
+
+@pytest.mark.parametrize("pairs", [False, True])
+@pytest.mark.parametrize("NB,nstrips", [(1, 64), (8, 256), (3, 96)])
+def test_small_launches_cut_no_strip_of_average_length(NB, nstrips, pairs):
+    """With more lanes than strips a lane's share is less than a strip: only strips longer than the average (and never
+    shorter than nine tiles) are cut, however many lanes there are."""
+    rng = np.random.default_rng(NB * nstrips)
+    cnt = rng.integers(4, 20, nstrips)
+    cnt[0] = nstrips
+    cnt = np.repeat(cnt[::2], 2)
+    plan = _plan(np.concatenate([[0], np.cumsum(cnt)]), pairs, NB, 1 << 14)
+    limit = max(-(-int(cnt.sum()) // nstrips), 8)
+    assert sorted(s for s, *_ in plan["longs"]) == [i for i in range(nstrips) if cnt[i] > limit]
