@@ -726,7 +726,7 @@ __global__ __launch_bounds__(HYB_CL_THREADS) void hyb_rem_bwd_col_lds_kernel(
     Layouts ly) {
     __shared__ f32x4 sq[HYB_CL_ROWS * 8], so[HYB_CL_ROWS * 8];
     constexpr int HYB_CL_COLS = NC * (HYB_CL_THREADS / 8);
-    const int ncg = L / HYB_CL_COLS;
+    const int ncg = (L + HYB_CL_COLS - 1) / HYB_CL_COLS;  // the last one's columns past the end have no entries
     const int item = xcd_remap((int)blockIdx.x, (int)gridDim.x);  // the work-groups of a head share an XCD's L2
     const int bh = item / ncg, cg = item % ncg;
     const int t = threadIdx.x, grp = t >> 3, sub = t & 7, lane = t & 63;
@@ -746,14 +746,14 @@ __global__ __launch_bounds__(HYB_CL_THREADS) void hyb_rem_bwd_col_lds_kernel(
         const int col = cg * HYB_CL_COLS + c * (HYB_CL_THREADS / 8) + grp;
         ak[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
         av[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        e[c] = c_ptr[col];
-        eend[c] = c_ptr[col + 1];
+        e[c] = col < L ? c_ptr[col] : 0;
+        eend[c] = col < L ? c_ptr[col + 1] : 0;
     }
     for (int r0 = 0; r0 < L; r0 += HYB_CL_ROWS) {
         __syncthreads();  // everybody has finished with the previous range
 #pragma unroll
         for (int k = 0; k < HYB_CL_ROWS * 8 / HYB_CL_THREADS; ++k) {
-            const int idx = t + k * HYB_CL_THREADS, row = r0 + (idx >> 3), piece = idx & 7;
+            const int idx = t + k * HYB_CL_THREADS, row = min(r0 + (idx >> 3), L - 1), piece = idx & 7;
             sq[idx] = reinterpret_cast<const f32x4*>(Q + ib + (size_t)row * ild)[piece];
             so[idx] = reinterpret_cast<const f32x4*>(dO + ob + (size_t)row * old_)[piece];
         }
@@ -805,6 +805,7 @@ __global__ __launch_bounds__(HYB_CL_THREADS) void hyb_rem_bwd_col_lds_kernel(
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         const int col = cg * HYB_CL_COLS + c * (HYB_CL_THREADS / 8) + grp;
+        if (col >= L) continue;
         f32x4* kr = reinterpret_cast<f32x4*>(dK + gb + (size_t)col * gld) + sub;
         f32x4* vr = reinterpret_cast<f32x4*>(dV + gb + (size_t)col * gld) + sub;
         if constexpr (PAIRS) {
@@ -836,7 +837,7 @@ __global__ __launch_bounds__(HYB_LL_THREADS) void hyb_rem_logits_lds_kernel(
     __shared__ f32x4 sk[HYB_LL_KEYS * 8];
     __shared__ float spen[MASK ? HYB_LL_KEYS : 1];
     constexpr int ROWS = NR * (HYB_LL_THREADS / 8);
-    const int nrg = L / ROWS;
+    const int nrg = (L + ROWS - 1) / ROWS;  // the last one's rows past the end have no entries
     const int item = xcd_remap((int)blockIdx.x, (int)gridDim.x);  // the work-groups of a head share an XCD's L2
     const int bh = item / nrg, rg = item % nrg;
     const int t = threadIdx.x, grp = t >> 3, sub = t & 7, qi = t & 3, lane = t & 63;
@@ -851,13 +852,13 @@ __global__ __launch_bounds__(HYB_LL_THREADS) void hyb_rem_logits_lds_kernel(
 #pragma unroll
     for (int c = 0; c < NR; ++c) {
         const int row = rg * ROWS + c * (HYB_LL_THREADS / 8) + grp;
-        const f32x4* qr = reinterpret_cast<const f32x4*>(Q + ib + (size_t)row * ild);
+        const f32x4* qr = reinterpret_cast<const f32x4*>(Q + ib + (size_t)min(row, L - 1) * ild);
         q0[c] = qr[qi] * c2;
         q1[c] = qr[4 + qi] * c2;
         m[c] = HYB_ABSENT;
         z[c] = 0.f;
-        e[c] = ix.r_off[row];
-        eend[c] = ix.r_off[row + 1];
+        e[c] = row < L ? ix.r_off[row] : 0;
+        eend[c] = row < L ? ix.r_off[row + 1] : 0;
     }
     auto fdpp = [](auto ctrl, float x) {
         return __int_as_float(hyb_dpp<decltype(ctrl)::value>(__float_as_int(x)));
@@ -867,9 +868,9 @@ __global__ __launch_bounds__(HYB_LL_THREADS) void hyb_rem_logits_lds_kernel(
 #pragma unroll
         for (int k = 0; k < HYB_LL_KEYS * 8 / HYB_LL_THREADS; ++k) {
             const int idx = t + k * HYB_LL_THREADS;
-            sk[idx] = reinterpret_cast<const f32x4*>(K + ib + (size_t)(k0 + (idx >> 3)) * ild)[idx & 7];
+            sk[idx] = reinterpret_cast<const f32x4*>(K + ib + (size_t)min(k0 + (idx >> 3), L - 1) * ild)[idx & 7];
         }
-        if constexpr (MASK) spen[t] = pen[(size_t)bh * L + k0 + t] * LOG2E;
+        if constexpr (MASK) spen[t] = pen[(size_t)bh * L + min(k0 + t, L - 1)] * LOG2E;
         __syncthreads();
         const int kend = k0 + HYB_LL_KEYS;
 #pragma unroll
@@ -926,7 +927,7 @@ __global__ __launch_bounds__(HYB_LL_THREADS) void hyb_rem_logits_lds_kernel(
 #pragma unroll
     for (int c = 0; c < NR; ++c) {
         const int row = rg * ROWS + c * (HYB_LL_THREADS / 8) + grp;
-        if (sub == 0) Stats[(size_t)bh * L + row] = make_float2(m[c], z[c]);
+        if (sub == 0 && row < L) Stats[(size_t)bh * L + row] = make_float2(m[c], z[c]);
     }
 }
 
@@ -944,7 +945,7 @@ __global__ __launch_bounds__(HYB_RL_THREADS) void hyb_rem_pv_lds_kernel(
     const float* __restrict__ V, const float* __restrict__ Raw, float* __restrict__ P, float* __restrict__ O,
     float* __restrict__ Ocache, const float2* __restrict__ Stats, HybIndex ix, int L, int NB, int nnz, Layouts ly) {
     __shared__ f32x4 sv[HYB_RL_KEYS * 8];
-    const int nrg = L / HYB_RL_ROWS;
+    const int nrg = (L + HYB_RL_ROWS - 1) / HYB_RL_ROWS;  // the last one's rows past the end have no entries
     const int item = xcd_remap((int)blockIdx.x, (int)gridDim.x);  // the work-groups of a head share an XCD's L2
     const int bh = item / nrg, rg = item % nrg;
     const int t = threadIdx.x, grp = t >> 3, sub = t & 7, lane = t & 63;
@@ -962,16 +963,16 @@ __global__ __launch_bounds__(HYB_RL_THREADS) void hyb_rem_pv_lds_kernel(
     for (int c = 0; c < NR; ++c) {
         const int row = rg * HYB_RL_ROWS + c * (HYB_RL_THREADS / 8) + grp;
         acc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        st[c] = Stats[(size_t)bh * L + row];
-        e[c] = ix.r_off[row];
-        eend[c] = ix.r_off[row + 1];
+        st[c] = Stats[(size_t)bh * L + min(row, L - 1)];
+        e[c] = row < L ? ix.r_off[row] : 0;
+        eend[c] = row < L ? ix.r_off[row + 1] : 0;
     }
     for (int k0 = 0; k0 < L; k0 += HYB_RL_KEYS) {
         __syncthreads();  // everybody has finished with the previous range
 #pragma unroll
         for (int k = 0; k < HYB_RL_KEYS * 8 / HYB_RL_THREADS; ++k) {
             const int idx = t + k * HYB_RL_THREADS;
-            sv[idx] = reinterpret_cast<const f32x4*>(V + ib + (size_t)(k0 + (idx >> 3)) * ild)[idx & 7];
+            sv[idx] = reinterpret_cast<const f32x4*>(V + ib + (size_t)min(k0 + (idx >> 3), L - 1) * ild)[idx & 7];
         }
         __syncthreads();
         const int kend = k0 + HYB_RL_KEYS;
@@ -1011,7 +1012,7 @@ __global__ __launch_bounds__(HYB_RL_THREADS) void hyb_rem_pv_lds_kernel(
 #pragma unroll
     for (int c = 0; c < NR; ++c) {
         const int row = rg * HYB_RL_ROWS + c * (HYB_RL_THREADS / 8) + grp;
-        if (eend[c] == ix.r_off[row]) continue;  // a row without remainder entries
+        if (row >= L || eend[c] == ix.r_off[row]) continue;  // a row without remainder entries
         f32x4* orow = reinterpret_cast<f32x4*>(O + ob + (size_t)row * old_) + sub;
         const f32x4 sum = *orow + acc[c];
         *orow = sum;

@@ -1415,25 +1415,40 @@ static void launch_tile_bwd(SparseAttn* a, const float* Q, const float* K, const
 #undef SPION_BY_WAVES
 }
 
-// The remainder's column pass with its gathered operands in LDS: columns per lane group (work-groups of 1024, 512 or
-// 256 columns of a head), the most that still gives every CU a work-group -- with half of them idle the kernel that
-// gathers from L2 is as fast (configuration 4 at half its batch: 0.248 against 0.244 ms) -- or 0 for that kernel
-// (also with SPION_HYB_GATHER=1).
+// The remainder's kernels with their gathered operands in LDS take one work-group of sixteen wavefronts per CU.  How full
+// a launch over work-groups of `per` rows or columns of a head keeps the machine: the rows over those its rounds of 256
+// work-groups could take.
+static int hyb_groups(int L, int per) { return (L + per - 1) / per; }
+static double hyb_filling(const SparseAttn* a, int per) {
+    const long long rounds = ((long long)a->NB * hyb_groups(a->L, per) + 255) / 256;
+    return (double)a->NB * a->L / (256.0 * per * rounds);
+}
+static bool hyb_lds_off(const SparseAttn* a) {
+    static const bool gather = getenv("SPION_HYB_GATHER") != nullptr;
+    return gather || a->L < 1024;
+}
+// Columns per lane group of the column pass (work-groups of 1024, 512 or 256 columns): the one that leaves the machine
+// fullest, a quarter of a column counted for the ranges every work-group loads; 0, the kernel that gathers from L2, below
+// 0.6 -- full against full the LDS form takes 0.54 of its time.
 static int hyb_lds_columns(const SparseAttn* a) {
-    static const bool gather = getenv("SPION_HYB_GATHER") != nullptr;
-    if (gather || a->L % 1024) return 0;
-    for (int nc = 8; nc >= 2; nc >>= 1)
-        if ((long long)a->NB * (a->L / (128 * nc)) >= 256) return nc;
-    return 0;
+    if (hyb_lds_off(a)) return 0;
+    int best = 0;
+    double most = 0.6;
+    for (int nc = 8; nc >= 2; nc >>= 1) {
+        const double f = hyb_filling(a, 128 * nc) * nc / (nc + 0.25);
+        if (f > most) {
+            most = f;
+            best = nc;
+        }
+    }
+    return best;
 }
-// The same for the forward's logits of the remainder: work-groups of 512 rows (four per lane group; eight need more
-// registers than a wavefront of sixteen has and are no faster), when every CU gets one.
-static bool hyb_lds_rows(const SparseAttn* a) {
-    static const bool gather = getenv("SPION_HYB_GATHER") != nullptr;
-    return !gather && a->L % 1024 == 0 && (long long)a->NB * (a->L / 512) >= 256;
-}
+// The forward's logits: work-groups of 512 rows (four per lane group; eight need more registers than a wavefront of
+// sixteen has and are no faster); 0.77 of the gather kernel's time on a full machine.  Its P.V: 1024 rows, 0.95.
+static bool hyb_lds_rows(const SparseAttn* a) { return !hyb_lds_off(a) && hyb_filling(a, 512) >= 0.78; }
+static bool hyb_lds_pv(const SparseAttn* a) { return !hyb_lds_off(a) && hyb_filling(a, HYB_RL_ROWS) >= 0.95; }
 #define SPION_HYB_COL_LDS(ST_, PAIRS_, NC_, ...)                                                          \
-    hipLaunchKernelGGL((hyb_rem_bwd_col_lds_kernel<ST_, PAIRS_, NC_>), dim3(a->NB * (a->L / (128 * NC_))), \
+    hipLaunchKernelGGL((hyb_rem_bwd_col_lds_kernel<ST_, PAIRS_, NC_>), dim3(a->NB * hyb_groups(a->L, 128 * NC_)), \
                        dim3(HYB_CL_THREADS), 0, a->hdr.stream, __VA_ARGS__)
 
 // Hybrid patterns (dense tiles + remainder, d = 32).  Every operand row-major; ST: heads located by `ly`.
@@ -1458,7 +1473,7 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
     float2* stats = reinterpret_cast<float2*>(a->ws_stats);
     const bool lds_logits = hyb_lds_rows(a);
 #define SPION_HYB_LOGITS_LDS(MASKED, NR_)                                                                            \
-    hipLaunchKernelGGL((hyb_rem_logits_lds_kernel<MASKED, ST, NR_>), dim3(a->NB * (a->L / (128 * NR_))),             \
+    hipLaunchKernelGGL((hyb_rem_logits_lds_kernel<MASKED, ST, NR_>), dim3(a->NB * hyb_groups(a->L, 128 * NR_)),             \
                        dim3(HYB_LL_THREADS), 0, a->hdr.stream, Q, K, Mask, a->ws_raw, stats, a->pat.hyb, a->L, a->NB, \
                        a->scale, ly)
 #define SPION_HYB_FWD(MASKED)                                                                                        \
@@ -1482,8 +1497,8 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
         SPION_HYB_FWD(false);
 #undef SPION_HYB_FWD
 #undef SPION_HYB_LOGITS_LDS
-    if (hyb_lds_columns(a) == 8)  // a full machine of work-groups of 1024 rows: the V rows in LDS
-        hipLaunchKernelGGL(hyb_rem_pv_lds_kernel<ST>, dim3(a->NB * (a->L / HYB_RL_ROWS)), dim3(HYB_RL_THREADS), 0,
+    if (hyb_lds_pv(a))
+        hipLaunchKernelGGL(hyb_rem_pv_lds_kernel<ST>, dim3(a->NB * hyb_groups(a->L, HYB_RL_ROWS)), dim3(HYB_RL_THREADS), 0,
                            a->hdr.stream, V, (const float*)a->ws_raw, Attn, Out, ocopy, (const float2*)stats, a->pat.hyb,
                            a->L, a->NB, nnz, ly);
     else
