@@ -64,14 +64,16 @@ __global__ __launch_bounds__(POOL_THREADS) void conv_pool_kernel(ScoreMaps maps,
 // of them in [dp - bs + 1, dp], a trapezoid in dp: min(dp + 1 - lo, hi - lo + 1, hi + bs - dp), not below zero.  Small
 // whole numbers, so it is formed in fp32 (four instructions, the integer form took eight comparisons per element), and
 // for one of the two sums only: the shifts of a column's own block and of its neighbour make up all of them, so the
-// neighbour's sum is that over the full trapezoid, the same for every column and looked up per row, less the own one.
+// neighbour's weight is that of the full trapezoid, the same for every column and looked up per row, less the own one.
+// The weights are subtracted, which is exact; the difference of the two sums would be rounding noise wherever a
+// column's own sum is many orders above its neighbour's, as on maps that decay steeply away from the diagonal.
 // A batch of loads is issued before any of them is used, with the row clamped instead of a remainder loop whose loads
-// would each wait alone.  Four maps of 2048 x 2048, block 32: 52.7 -> 25.2 us.
+// would each wait alone.  Four maps of 2048 x 2048, block 32: 52.7 -> 25.6 us (25.1 with the sums subtracted).
 constexpr int CP_COLS = 256, CP_RG = 2, CP_BATCH = 16;
 __global__ __launch_bounds__(CP_COLS* CP_RG) void conv_pool_cols_kernel(ScoreMaps maps, float* __restrict__ pooled, int L,
                                                                          int bs, int nb, int hk, int gb) {
     __shared__ double part[CP_RG][2][CP_COLS];
-    __shared__ double full[CP_COLS];  // full trapezoid of row dp at [dp + hk]
+    __shared__ float full[CP_COLS];  // full trapezoid of row dp at [dp + hk]
     // consecutive items -- the groups of a block row, then the next block row of the same map, whose rows overlap --
     // run on one die, whose L2 then serves the bs + 2 hk rows' overlap
     const int groups = (nb + gb - 1) / gb;
@@ -88,10 +90,10 @@ __global__ __launch_bounds__(CP_COLS* CP_RG) void conv_pool_cols_kernel(ScoreMap
         return fmaxf(0.f, fminf(fminf(dp + lo1, n), top - dp));
     };
     if ((int)threadIdx.x < bs + 2 * hk)
-        full[threadIdx.x] = (double)trapezoid((float)((int)threadIdx.x - hk), (float)(1 + hk),
-                                              (float)min(2 * hk + 1, bs), (float)(hk + bs));
+        full[threadIdx.x] = trapezoid((float)((int)threadIdx.x - hk), (float)(1 + hk), (float)min(2 * hk + 1, bs),
+                                      (float)(hk + bs));
     __syncthreads();
-    double a0 = 0.0, all = 0.0;
+    double a0 = 0.0, a1 = 0.0;
     if (cc < ncols && q >= 0 && q < L) {
         const int c = q % bs;
         const int lo = max(-hk, c - bs + 1), hi = min(hk, c);
@@ -107,14 +109,15 @@ __global__ __launch_bounds__(CP_COLS* CP_RG) void conv_pool_cols_kernel(ScoreMap
                 if (p < p1) {
                     const int dp = p - I * bs;
                     const double x = (double)v[k];
-                    a0 += x * (double)trapezoid((float)dp, lo1, n, top);
-                    all += x * full[dp + hk];
+                    const float own = trapezoid((float)dp, lo1, n, top);
+                    a0 += x * (double)own;
+                    a1 += x * (double)(full[dp + hk] - own);
                 }
             }
         }
     }
     part[rg][0][cc] = a0;
-    part[rg][1][cc] = all - a0;
+    part[rg][1][cc] = a1;
     __syncthreads();
     // wavefront b adds up block b: entries e = 0 .. CP_RG (bs + 2 hk) - 1, lane-strided, then a butterfly
     const int b = threadIdx.x >> 6, lane = threadIdx.x & 63;

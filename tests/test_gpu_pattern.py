@@ -62,6 +62,28 @@ def test_pattern_large_block_grids(L, bs):
     _check_maps(maps, bs, 0.95, 31)
 
 
+@pytest.mark.parametrize("L,bs", [(512, 32), (512, 64), (544, 32)])
+@pytest.mark.parametrize("decay", [0.25, 1.0, 1.5, 2.0])
+def test_steep_local_maps(L, bs, decay):
+    """Softmax maps that fall by e^-decay per token away from the diagonal: a column's sum for its own block then lies up to
+    forty orders above the one for the neighbour it reaches into, and both have to be right by themselves.  Every
+    pooled value is a sum of positive terms, exact but for fp64 rounding, rounded once to fp32: 2^-24 of its own size
+    (with 1 % for the fp64 part), and not of the map's largest value."""
+    g = torch.Generator().manual_seed(L + bs)
+    i = torch.arange(L)
+    slope = -decay * (i[:, None] - i[None, :]).abs().float()
+    maps = torch.softmax(slope + 0.5 * torch.randn(4, L, L, generator=g), -1)
+    for q in (0.5, 0.7, 0.8, 0.95):
+        mat, pooled, thresh = discover_block_masks(maps.cuda(), bs, threshold=q, return_aux=True)
+        for n in range(4):
+            C = op.block_pool_closed_form(op.conv_diag_closed_form(maps[n].numpy(), 31), bs)
+            normal = C >= 2.0 ** -126
+            err = np.abs(pooled[n].cpu().numpy().astype(np.float64) - C)[normal] / C[normal]
+            assert err.max() <= 1.01 * 2.0 ** -24, (q, n, err.max())
+            ref = op.generate_mask_conv_ff(maps[n].numpy(), bs, q, ksize=31, route="fp64")[0]
+            assert np.array_equal(mat[n].cpu().numpy().astype(np.int8), ref), (q, n)
+
+
 @pytest.mark.parametrize("levels", [0, 1, 4])
 @pytest.mark.parametrize("nb", [1, 2, 3, 64, 127, 128, 129, 192, 193])
 def test_walk_and_quantile_on_block_grids_of_every_size(nb, levels):
