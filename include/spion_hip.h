@@ -242,6 +242,11 @@ int spion_register_pattern(void* handle, const int* Offsets, const int* Columns,
  * needs the dS scratch.  It describes the most recent call on the handle, not a particular pattern. */
 int spion_last_path(void* handle);
 
+/* The sizes a sparse handle was created with: what a caller compares its tensors with, since every entry point works on
+ * the handle's num_batches x seq_len x emb_dim and not on sizes of the call's.  0 on success, 1 for a handle that is none
+ * of a sparse family (recorded as an error). */
+int spion_block_sizes(void* handle, int* emb_dim, int* seq_len, int* num_batches);
+
 /* Most recent failure recorded by a call on THIS handle ("" if none), besides the process-wide slot of
  * spion_last_error, which any thread or handle can overwrite.  Every failure is also written to stderr unless
  * the environment has SPION_QUIET=1; SPION_ABORT_ON_ERROR=1 makes a failure abort the process (for callers of the

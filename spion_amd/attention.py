@@ -182,10 +182,11 @@ class Attention(nn.Module):
 
     def _sparse_layer(self, node, X, mask, mat):
         """The whole layer in one call -- projections, core, output projection, and no torch operation in between --
-        or None when the core is not one of this package's modules as they are, or has hooks."""
+        or None when the core is not one of this package's modules as they are, was built for heads of another shape
+        (reconstruct_for_blocksparse takes a config of its own; the module then says so), or has hooks."""
         core = self.block_attn
         if (type(core) not in _core_types() or not core.reads_views
-                or X.shape[0] != core.batch_size or X.shape[1] != core.seq_len or core._forward_hooks
+                or core.head_shape != (X.shape[0], self.num_head, X.shape[1], self.head_dim) or core._forward_hooks
                 or core._forward_pre_hooks or core._backward_hooks or core._backward_pre_hooks):
             return None
         idx = core.csr_cache.get(mat, core.block_size)

@@ -77,8 +77,17 @@ CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& va
     spion_set_stream(h, reinterpret_cast<void*>(stream));
     TORCH_CHECK(query.dim() == 4 && key.sizes() == query.sizes() && value.sizes() == query.sizes(),
                 "query, key and value must be [B, H, L, d] tensors of one shape");
-    TORCH_CHECK(query.scalar_type() == torch::kFloat32 && query.is_cuda(), "fp32 tensors on the GPU expected");
     const int64_t B = query.size(0), H = query.size(1);
+    // the kernels take every size from the handle: tensors of other sizes would be read and written past their ends
+    int hd = 0, hl = 0, hnb = 0;
+    if (spion_block_sizes(h, &hd, &hl, &hnb)) check_library("attn_forward");
+    TORCH_CHECK_VALUE(B * H == hnb && H == num_heads && query.size(2) == hl && query.size(3) == hd, "query shape ",
+                      query.sizes(), " does not match the handle (", hnb, " heads in all, ", num_heads, " a sample, ", hl,
+                      " rows of ", hd, ")");
+    TORCH_CHECK_VALUE(!pen.defined() || pen.numel() >= B * H * query.size(2), "key mask smaller than [B, L]");
+    for (const Tensor* t : {&query, &key, &value, &pen})
+        TORCH_CHECK(!t->defined() || (t->scalar_type() == torch::kFloat32 && t->device() == query.device() && t->is_cuda()),
+                    "fp32 tensors on one GPU expected");
     const auto opt = query.options();
     CoreResult r;
     r.p_flat = torch::empty({B * H * nnz}, opt);

@@ -67,6 +67,7 @@ void sparse_backward_noalloc(void*, const float*, const float*, const float*, co
                              float*, float*, float*, const int*, const int*, int);
 size_t sparse_noalloc_max_rows();
 int sparse_last_path(void*);
+int sparse_sizes(void*, int*, int*, int*);
 void sparse_force_element(void*, int);
 void sparse_set_bwd_passes(void*, int);
 int sparse_debug_counter(void*, int);
@@ -312,6 +313,7 @@ int spion_register_pattern(void* h, const int* Offsets, const int* Columns, int 
 }
 void spion_forget_pattern(void* h, const int* Offsets, const int* Columns) { sparse_forget_pattern(h, Offsets, Columns); }
 int spion_last_path(void* h) { return sparse_last_path(h); }
+int spion_block_sizes(void* h, int* d, int* L, int* NB) { return sparse_sizes(h, d, L, NB); }
 void spion_force_element_path(void* h, int on) { sparse_force_element(h, on); }
 void spion_set_backward_passes(void* h, int mask) { sparse_set_bwd_passes(h, mask); }
 int spion_debug_counter(void* h, int which) { return sparse_debug_counter(h, which); }

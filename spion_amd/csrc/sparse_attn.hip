@@ -2294,6 +2294,14 @@ int sparse_last_path(void* h) {
     SparseAttn* a = as_sparse(h, "spion_last_path");
     return a ? a->last_path : 0;
 }
+int sparse_sizes(void* h, int* d, int* L, int* NB) {
+    SparseAttn* a = as_sparse(h, "spion_block_sizes");
+    if (!a) return 1;
+    *d = a->d;
+    *L = a->L;
+    *NB = a->NB;
+    return 0;
+}
 // The schedule build_bf16_plan makes for a tile list, copied out for inspection (host only: nothing is launched or
 // allocated on a device).  Returns the number of lanes; counts = {ints in items, ints in lane_ent, ints in longs,
 // workspace slots}.  Arrays that are null or too small (cap_* in ints) are left alone.
