@@ -156,19 +156,20 @@ class Attention(nn.Module):
         return self.ff(attn_out), attn
 
     def _compiled_node(self, X, mask):
-        """The compiled node when it covers the projections of this call (csrc/project.hip: fp32 on the GPU, features in
-        multiples of 32, plain linear layers without hooks, no autocast), else None."""
-        if not (self.fused_qkv and X.is_cuda and X.dtype == torch.float32 and X.dim() == 3 and X.shape[2] == self.dim
-                and isinstance(mask, torch.Tensor) and X.shape[0] * X.shape[1] % 32 == 0 and X.numel() > 0
-                and self.num_head * self.head_dim % 32 == 0 and self.dim % 32 == 0
-                and not torch.is_autocast_enabled()):
+        """The compiled node when it covers the projections of this call (csrc/project.hip: fp32 on the GPU, rows and
+        features in multiples of 32, plain linear layers of the layer's sizes without hooks, no autocast), else None."""
+        if not (self.fused_qkv and X.is_cuda and isinstance(mask, torch.Tensor) and not torch.is_autocast_enabled()):
             return None
         for m in (self.W_q, self.W_k, self.W_v, self.ff):
-            if (type(m) is not nn.Linear or m.bias is None or m.weight.dtype != torch.float32
-                    or m.weight.device != X.device or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                    or m._backward_pre_hooks):
+            if (type(m) is not nn.Linear or m.bias is None or m._forward_hooks or m._forward_pre_hooks
+                    or m._backward_hooks or m._backward_pre_hooks):
                 return None
-        return _lib.autograd_node()
+        node = _lib.autograd_node()
+        if node is None or not node.projections_fit(
+                X, self.W_q.weight, self.W_k.weight, self.W_v.weight, self.W_q.bias, self.W_k.bias, self.W_v.bias,
+                self.ff.weight, self.ff.bias, self.num_head, self.head_dim):
+            return None
+        return node
 
     def _in_node(self, call, *args):
         """A call of the node on X's stream; errors of the library come out as the modules raise them."""

@@ -207,6 +207,30 @@ Tensor aligned(const Tensor& t) {  // contiguous, 16-byte aligned
     return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 ? c.clone() : c;
 }
 
+// y = x.w^T + b: w [outputs, features], b [outputs], fp32 tensors with memory of their own on x's device.  The kernels
+// take the sizes of all of them from x and the heads, so anything else would be read past its end.
+bool projection_fits(const Tensor& x, const Tensor& w, const Tensor& b, int64_t outputs, int64_t features) {
+    for (const Tensor* t : {&x, &w, &b})
+        if (!t->defined() || t->scalar_type() != torch::kFloat32 || t->device() != x.device() ||
+            t->layout() != torch::kStrided || t->unsafeGetTensorImpl()->is_python_dispatch())
+            return false;
+    return w.dim() == 2 && w.size(0) == outputs && w.size(1) == features && b.dim() == 1 && b.size(0) == outputs;
+}
+void check_projection(const Tensor& x, const Tensor& w, const Tensor& b, int64_t outputs, int64_t features) {
+    TORCH_CHECK_VALUE(projection_fits(x, w, b, outputs, features), "projection: weight [", outputs, ", ", features,
+                      "] and bias [", outputs, "], fp32 on the input's device, expected");
+}
+// Whether the projection kernels take this layer's four linear layers as they are; the layer uses torch's otherwise.
+bool projections_fit(const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& bq, const Tensor& bk,
+                     const Tensor& bv, const Tensor& wf, const Tensor& bf, int64_t H, int64_t d) {
+    if (x.dim() != 3 || !wf.defined() || wf.dim() != 2) return false;
+    const int64_t n = H * d, dim = x.size(2), outputs = wf.size(0), rows = x.size(0) * x.size(1);
+    for (const int64_t size : {n, dim, outputs, rows})
+        if (size <= 0 || size % 32) return false;
+    return projection_fits(x, wq, bq, n, dim) && projection_fits(x, wk, bk, n, dim) && projection_fits(x, wv, bv, n, dim) &&
+           projection_fits(x, wf, bf, outputs, n);
+}
+
 Tensor project_weight_grads(const float* dy, const Tensor& x, int64_t rows, int64_t outputs, int64_t dim, int64_t stream,
                             Tensor& db) {
     const auto opt = x.options();
@@ -220,7 +244,10 @@ Tensor project_weight_grads(const float* dy, const Tensor& x, int64_t rows, int6
 // X [B, L, dim] -> the [B, H, L, d] heads of the three projections, slices of one [B, L, 3, H, d] buffer.
 std::vector<Tensor> qkv_forward(const Tensor& x, const Tensor (&w)[3], const Tensor (&b)[3], int64_t H, int64_t d,
                                 int64_t stream) {
+    TORCH_CHECK_VALUE(x.dim() == 3, "projection: input [B, L, features] expected");
     const int64_t B = x.size(0), L = x.size(1), dim = x.size(2);
+    for (int i = 0; i < 3; ++i) check_projection(x, w[i], b[i], H * d, dim);
+    TORCH_CHECK(x.is_cuda(), "fp32 tensors on the GPU expected");
     Tensor buf = torch::empty({B, L, 3, H, d}, x.options());
     const float* wp[3] = {fp(w[0]), fp(w[1]), fp(w[2])};
     const float* bp[3] = {fp(b[0]), fp(b[1]), fp(b[2])};
@@ -278,7 +305,10 @@ struct QkvNode : public torch::autograd::Function<QkvNode> {
 // The output projection on heads [B, H, L, d] that lie interleaved ([B, L, H*d] in memory: what the core's forward makes
 // for the slices above), y [B, L, dim].
 Tensor merge_forward(const Tensor& merged, const Tensor& w, const Tensor& b, int64_t stream) {
+    TORCH_CHECK_VALUE(merged.dim() == 4 && w.dim() == 2, "projection: heads [B, L, H, d] and a weight matrix expected");
     const int64_t B = merged.size(0), L = merged.size(1), n = merged.size(2) * merged.size(3);
+    check_projection(merged, w, b, w.size(0), n);
+    TORCH_CHECK(merged.is_cuda(), "fp32 tensors on the GPU expected");
     Tensor y = torch::empty({B, L, w.size(0)}, merged.options());
     const float* wp[1] = {fp(w)};
     const float* bp[1] = {fp(b)};
@@ -365,6 +395,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("columns"), py::arg("sum_mat"), py::arg("handle"), py::arg("nnz"), py::arg("num_heads"),
           py::arg("reads_views"), py::arg("stream"));
     m.def("sparse_layer", &sparse_layer, "forward of the attention layer in its sparse phase; returns [y, p_flat]");
+    m.def("projections_fit", &projections_fit, "whether the projection kernels take this layer's linear layers");
     m.def("project_heads", &project_heads, "the three input projections; returns the [B, H, L, d] heads");
     m.def("merge_heads", &merge_heads, "the output projection of [B, H, L, d] heads");
 }

@@ -126,3 +126,50 @@ def test_layer_in_one_call_matches_its_steps(heads, d, L, masked):
     again = run()
     assert layer.W_k.weight.grad is None
     assert torch.equal(again[2], fused[2])
+
+
+@pytest.mark.parametrize("outputs", [48, 64, 160])
+def test_layer_with_a_replaced_output_projection(outputs):
+    """Another width of the output projection: on the kernels where it is a multiple of 32, torch's steps where not."""
+    B, L = 2, 64
+    cfg = dict(head_dim=32, num_head=2, max_seq_len=L, batch_size=B, block_size=32, transformer_dim=96, attention_dropout=0.0,
+               task="lra-image")
+    layer = spion_amd.Attention(cfg, inference=True)
+    layer.ff = torch.nn.Linear(64, outputs)
+    layer = layer.cuda()
+    layer.reconstruct_for_blocksparse(cfg)
+    x, mat = torch.randn(B, L, 96, device="cuda", requires_grad=True), torch.eye(2, device="cuda")
+    seen = []
+    ones = torch.ones(B, L, device="cuda")
+    y, _ = layer(x, ones, mat)
+    layer.block_attn.register_forward_hook(lambda m, i, o: seen.append(o[0].detach()))
+    y2, _ = layer(x, ones, mat)
+    ref = torch.nn.functional.linear(layer.combine_heads(seen[0]).double(), layer.ff.weight.double(), layer.ff.bias.double())
+    assert y.shape == (B, L, outputs)
+    for t in (y, y2):
+        assert float((t.detach().double() - ref.detach()).norm() / ref.detach().norm()) < 2e-6
+    y.sum().backward()
+    assert layer.ff.weight.grad.shape == (outputs, 64)
+
+
+@pytest.mark.parametrize("which", ["W_q", "W_v", "ff"])
+def test_layer_with_a_replaced_projection_that_does_not_fit_raises(which):
+    B, L = 2, 64
+    cfg = dict(head_dim=32, num_head=2, max_seq_len=L, batch_size=B, block_size=32, transformer_dim=96, attention_dropout=0.0,
+               task="lra-image")
+    layer = spion_amd.Attention(cfg, inference=True)
+    setattr(layer, which, torch.nn.Linear(32, 96) if which == "ff" else torch.nn.Linear(96, 32))
+    layer = layer.cuda()
+    layer.reconstruct_for_blocksparse(cfg)
+    with pytest.raises(RuntimeError):
+        layer(torch.randn(B, L, 96, device="cuda"), torch.ones(B, L, device="cuda"), torch.eye(2, device="cuda"))
+
+
+def test_layer_with_a_core_of_other_heads_raises():
+    B, L = 2, 64
+    cfg = dict(head_dim=32, num_head=2, max_seq_len=L, batch_size=B, block_size=32, transformer_dim=96, attention_dropout=0.0,
+               task="lra-image")
+    layer = spion_amd.Attention(cfg, inference=True).cuda()
+    layer.reconstruct_for_blocksparse(dict(cfg, num_head=4))
+    with pytest.raises(ValueError, match="does not match the handle"):
+        layer(torch.randn(B, L, 96, device="cuda"), torch.ones(B, L, device="cuda"), torch.eye(2, device="cuda"))

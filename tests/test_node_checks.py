@@ -53,3 +53,50 @@ def test_layer_with_a_core_of_other_heads_is_not_taken_in_one_call(heads, d):
     layer.reconstruct_for_blocksparse(_config(heads, d))
     x = torch.zeros(2, 64, 64)
     assert layer._sparse_layer(_Unused(), x, torch.ones(2, 64), torch.ones(2, 2)) is None
+
+
+def _linears(n, dim, out):
+    w = [torch.zeros(n, dim) for _ in range(3)] + [torch.zeros(out, n)]
+    return w, [torch.zeros(t.shape[0]) for t in w]
+
+
+def _fits(x, w, b, heads=2, d=32):
+    return _lib.autograd_node().projections_fit(x, w[0], w[1], w[2], b[0], b[1], b[2], w[3], b[3], heads, d)
+
+
+@needs_node
+def test_projections_fit_only_weights_of_the_layers_sizes():
+    x = torch.zeros(2, 64, 96)
+    assert _fits(x, *_linears(64, 96, 96))
+    assert _fits(x, *_linears(64, 96, 128))  # an output projection to another width
+    assert not _fits(x, *_linears(64, 96, 48))  # which is no multiple of 32
+    assert not _fits(torch.zeros(2, 48, 96)[:1], *_linears(64, 96, 96))  # rows
+    assert not _fits(torch.zeros(2, 64, 80), *_linears(64, 80, 96))  # features
+    assert not _fits(torch.zeros(0, 64, 96), *_linears(64, 96, 96))
+    assert not _fits(torch.zeros(64, 96), *_linears(64, 96, 96))
+    for i in range(4):
+        for bad in ((32, 96), (64, 64), (96, 64), (64, 160)):
+            w, b = _linears(64, 96, 96)
+            if tuple(w[i].shape) == bad or (i == 3 and bad[1] == 64):
+                continue
+            w[i] = torch.zeros(bad)
+            assert not _fits(x, w, b), (i, bad)
+        for bad in (torch.zeros(32), torch.zeros(64, 1), torch.zeros(64).double(), torch.zeros(64, device="meta")):
+            w, b = _linears(64, 96, 96)
+            b[i] = bad
+            assert not _fits(x, w, b), (i, bad.shape, bad.dtype, bad.device)
+        w, b = _linears(64, 96, 96)
+        w[i] = w[i].half()
+        assert not _fits(x, w, b)
+
+
+@needs_node
+@pytest.mark.parametrize("which", ["rows", "columns", "bias", "type"])
+def test_node_refuses_projections_of_other_sizes(which):
+    w, b = _linears(64, 96, 96)
+    w[1] = {"rows": torch.zeros(32, 96), "columns": torch.zeros(64, 64), "type": torch.zeros(64, 96).double()}.get(which, w[1])
+    b[1] = torch.zeros(32) if which == "bias" else b[1]
+    with pytest.raises(ValueError, match="projection"):
+        _lib.autograd_node().project_heads(torch.zeros(2, 64, 96), w[0], w[1], w[2], b[0], b[1], b[2], 2, 32, 0)
+    with pytest.raises(ValueError, match="projection"):
+        _lib.autograd_node().merge_heads(torch.zeros(2, 2, 64, 32 if which == "rows" else 48), torch.zeros(64, 96), torch.zeros(32), 0)
