@@ -7,6 +7,7 @@
 // time between autograd's engine, ctypes and tensor bookkeeping.  The arithmetic is the library's: the row-major
 // and strided entry points declared in include/spion_hip.h.  The Python function stays the statement of the
 // behaviour; tests run both and compare.
+#include <ATen/FuncTorchTLS.h>
 #include <torch/extension.h>
 
 #include <stdexcept>
@@ -63,6 +64,16 @@ bool adjacent_head_views(const Tensor& q, const Tensor& k, const Tensor& v) {
 const float* fp(const Tensor& t) { return t.defined() ? static_cast<const float*>(t.data_ptr()) : nullptr; }
 float* fpm(Tensor& t) { return static_cast<float*>(t.data_ptr()); }
 const int* ip(const Tensor& t) { return static_cast<const int*>(t.data_ptr()); }
+
+// Whether a call needs no node: nothing is recorded for a backward, no input carries a forward-mode tangent (which does
+// not depend on grad mode, and which a node refuses instead of dropping it) and no functorch transform is at work.
+bool has_tangent(const Tensor& t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
+bool without_node(std::initializer_list<const Tensor*> inputs) {
+    if (torch::GradMode::is_enabled() || at::functorch::functorchTLSAccessor()) return false;
+    for (const Tensor* t : inputs)
+        if (has_tangent(*t)) return false;
+    return true;
+}
 
 // What a forward of the attention core leaves for its backward.
 struct CoreResult {
@@ -198,6 +209,7 @@ Tensor key_penalty(const Tensor& mask, int64_t heads, int64_t stream) {
 // The modules hand over a key mask, or penalties made from one the kernel does not take (is_mask = false).
 c10::optional<Tensor> penalty_of(const c10::optional<Tensor>& mask_or_pen, bool is_mask, int64_t heads, int64_t stream) {
     if (!is_mask || !mask_or_pen.has_value()) return mask_or_pen;
+    if (has_tangent(*mask_or_pen)) return (1e6 * (1.0 - mask_or_pen->repeat({1, heads}))).contiguous();
     return key_penalty(*mask_or_pen, heads, stream);
 }
 
@@ -350,11 +362,12 @@ std::vector<Tensor> sparse_layer(const Tensor& x, const Tensor& wq, const Tensor
                                  const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t num_heads, int64_t head_dim,
                                  int64_t stream) {
     const auto pen = penalty_of(mask_or_pen, is_mask, num_heads, stream);
-    if (!torch::GradMode::is_enabled()) {  // nothing to record: no nodes
+    const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
+    if (without_node({&x, &wq, &wk, &wv, &bq, &bk, &bv, &wf, &bf, &pen_or_none})) {
         const Tensor w[3] = {aligned(wq), aligned(wk), aligned(wv)}, b[3] = {aligned(bq), aligned(bk), aligned(bv)};
         const auto qkv = qkv_forward(aligned(x), w, b, num_heads, head_dim, stream);
-        const CoreResult r = core_forward(qkv[0], qkv[1], qkv[2], pen.has_value() ? *pen : Tensor(), offsets, columns, sum_mat,
-                                          handle, nnz, num_heads, true, stream);
+        const CoreResult r = core_forward(qkv[0], qkv[1], qkv[2], pen_or_none, offsets, columns, sum_mat, handle,
+                                          nnz, num_heads, true, stream);
         return {merge_forward(aligned(r.out.transpose(1, 2)), aligned(wf), aligned(bf), stream), r.p_flat};
     }
     const auto qkv = QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream);
@@ -377,9 +390,10 @@ std::vector<Tensor> sparse_attention(const Tensor& query, const Tensor& key, con
                                      const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t num_heads,
                                      bool reads_views, int64_t stream) {
     const auto pen = penalty_of(mask_or_pen, is_mask, num_heads, stream);
-    if (!torch::GradMode::is_enabled()) {
-        const CoreResult r = core_forward(query, key, value, pen.has_value() ? *pen : Tensor(), offsets, columns, sum_mat,
-                                          handle, nnz, num_heads, reads_views, stream);
+    const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
+    if (without_node({&query, &key, &value, &pen_or_none})) {
+        const CoreResult r = core_forward(query, key, value, pen_or_none, offsets, columns, sum_mat, handle, nnz,
+                                          num_heads, reads_views, stream);
         return {r.out, r.p_flat};
     }
     return SparseAttnNode::apply(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, num_heads, reads_views,

@@ -94,3 +94,49 @@ def test_node_ignores_the_gradient_of_the_probabilities_and_reports_errors():
     with pytest.raises(ValueError):
         mod(q[:, :1], k[:, :1], v[:, :1], ones, mat)
     cpp.destroy(mod.attn_handle)
+
+
+@pytest.mark.parametrize("which", ["query", "key", "value", "mask"])
+def test_forward_mode_is_refused_also_without_gradients(which):
+    """Forward-mode AD does not depend on grad mode: a tangent must not be dropped because the node is passed by."""
+    import torch.autograd.forward_ad as fwd
+
+    if _lib.autograd_node() is None:
+        pytest.skip("SPION_PY_NODE=1")
+    B, H, L, d, bs = 1, 2, 64, 32, 32
+    mat = torch.eye(L // bs, device="cuda")
+    mod, cpp = _module(B, H, L, d, bs, True)
+    q, k, v, _ = _inputs(B, H, L, d, "contiguous", seed=2)
+    ones = torch.ones(B, L, device="cuda")
+    args = dict(query=q, key=k, value=v, mask=ones)
+    for guard in (torch.no_grad(), torch.enable_grad()):
+        with guard, fwd.dual_level():
+            dual = dict(args, **{which: fwd.make_dual(args[which], torch.ones_like(args[which]))})
+            with pytest.raises(RuntimeError, match="jvp"):
+                mod(dual["query"], dual["key"], dual["value"], dual["mask"], mat)
+    with torch.no_grad(), fwd.dual_level():  # no tangent among the inputs
+        mod(q, k, v, ones, mat)
+    cpp.destroy(mod.attn_handle)
+
+
+@pytest.mark.parametrize("which", ["input", "weight", "bias"])
+def test_forward_mode_is_refused_by_the_whole_layer_without_gradients(which):
+    import torch.autograd.forward_ad as fwd
+
+    if _lib.autograd_node() is None:
+        pytest.skip("SPION_PY_NODE=1")
+    B, L = 2, 64
+    cfg = dict(head_dim=32, num_head=2, max_seq_len=L, batch_size=B, block_size=32, transformer_dim=64, attention_dropout=0.0,
+               task="lra-image")
+    layer = Attention(cfg, inference=True).cuda()
+    layer.reconstruct_for_blocksparse(cfg)
+    x, mat = torch.randn(B, L, 64, device="cuda"), torch.eye(2, device="cuda")
+    with torch.no_grad(), fwd.dual_level():
+        if which == "input":
+            x = fwd.make_dual(x, torch.ones_like(x))
+        else:
+            t = getattr(layer.ff, which).detach()
+            delattr(layer.ff, which)
+            setattr(layer.ff, which, fwd.make_dual(t, torch.ones_like(t)))
+        with pytest.raises(RuntimeError, match="jvp"):
+            layer(x, torch.ones(B, L, device="cuda"), mat)
