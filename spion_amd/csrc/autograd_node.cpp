@@ -271,23 +271,37 @@ std::vector<Tensor> qkv_forward(const Tensor& x, const Tensor (&w)[3], const Ten
     return out;
 }
 
+// The backward of both projections runs torch's own operations on the saved inputs when it is itself recorded
+// (create_graph): the kernels would leave no graph, and second-order terms would be lost without a word.
 struct QkvNode : public torch::autograd::Function<QkvNode> {
     static variable_list forward(AutogradContext* ctx, Tensor x, Tensor wq, Tensor wk, Tensor wv, Tensor bq, Tensor bk,
                                  Tensor bv, int64_t H, int64_t d, int64_t stream) {
-        const Tensor xc = aligned(x);
         const Tensor w[3] = {aligned(wq), aligned(wk), aligned(wv)}, b[3] = {aligned(bq), aligned(bk), aligned(bv)};
-        ctx->save_for_backward({xc, w[0], w[1], w[2]});
+        ctx->save_for_backward({x, wq, wk, wv});
         ctx->saved_data["H"] = H;
         ctx->saved_data["stream"] = stream;
-        return qkv_forward(xc, w, b, H, d, stream);
+        return qkv_forward(aligned(x), w, b, H, d, stream);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
-        const Tensor& x = saved[0];
         const int64_t H = ctx->saved_data["H"].toInt(), stream = ctx->saved_data["stream"].toInt();
-        const int64_t B = x.size(0), L = x.size(1), dim = x.size(2), n = saved[1].size(0), d = n / H, rows = B * L;
+        const int64_t B = saved[0].size(0), L = saved[0].size(1), dim = saved[0].size(2), n = saved[1].size(0), d = n / H,
+                      rows = B * L;
         for (auto& t : g)
-            if (!t.defined()) t = torch::zeros({B, H, L, d}, x.options());
+            if (!t.defined()) t = torch::zeros({B, H, L, d}, saved[0].options());
+        if (torch::GradMode::is_enabled()) {
+            const Tensor dy = torch::stack({g[0].transpose(1, 2), g[1].transpose(1, 2), g[2].transpose(1, 2)}, 2)
+                                  .reshape({rows, 3 * n});
+            const Tensor dw = dy.t().matmul(saved[0].reshape({rows, dim})), db = dy.sum(0);
+            variable_list r(10);
+            r[0] = dy.matmul(torch::cat({saved[1], saved[2], saved[3]}, 0)).view({B, L, dim});
+            for (int i = 0; i < 3; ++i) {
+                r[1 + i] = dw.narrow(0, i * n, n);
+                r[4 + i] = db.narrow(0, i * n, n);
+            }
+            return r;
+        }
+        const Tensor x = aligned(saved[0]);
         Tensor keep;  // [B, L, 3, H, d]
         const float* dy = fp(g[0]);
         if (!adjacent_head_views(g[0], g[1], g[2]) || reinterpret_cast<uintptr_t>(dy) % 16) {
@@ -297,7 +311,8 @@ struct QkvNode : public torch::autograd::Function<QkvNode> {
         variable_list r(10);
         if (ctx->needs_input_grad(0)) {
             r[0] = torch::empty_like(x);
-            const float* wp[3] = {fp(saved[1]), fp(saved[2]), fp(saved[3])};
+            const Tensor w[3] = {aligned(saved[1]), aligned(saved[2]), aligned(saved[3])};
+            const float* wp[3] = {fp(w[0]), fp(w[1]), fp(w[2])};
             spion_project_backward_input(dy, wp, fpm(r[0]), rows, (int)n, 3, (int)dim, reinterpret_cast<void*>(stream));
         }
         bool any = false;
@@ -330,18 +345,24 @@ Tensor merge_forward(const Tensor& merged, const Tensor& w, const Tensor& b, int
 }
 struct MergeNode : public torch::autograd::Function<MergeNode> {
     static Tensor forward(AutogradContext* ctx, Tensor heads, Tensor w, Tensor b, int64_t stream) {
-        const Tensor a = aligned(heads.transpose(1, 2)), wc = aligned(w), bc = aligned(b);
-        ctx->save_for_backward({a, wc});
+        ctx->save_for_backward({heads, w});
         ctx->saved_data["stream"] = stream;
-        return merge_forward(a, wc, bc, stream);
+        return merge_forward(aligned(heads.transpose(1, 2)), aligned(w), aligned(b), stream);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &a = saved[0], &w = saved[1];
         const int64_t stream = ctx->saved_data["stream"].toInt();
-        const int64_t rows = a.size(0) * a.size(1), n = a.size(2) * a.size(3), dim = w.size(0);
-        const Tensor dy = aligned(g[0]);
+        const int64_t B = saved[0].size(0), H = saved[0].size(1), L = saved[0].size(2), d = saved[0].size(3);
+        const int64_t rows = B * L, n = H * d, dim = saved[1].size(0);
         variable_list r(4);
+        if (torch::GradMode::is_enabled()) {
+            const Tensor dy = g[0].reshape({rows, dim});
+            r[0] = dy.matmul(saved[1]).view({B, L, H, d}).transpose(1, 2);
+            r[1] = dy.t().matmul(saved[0].transpose(1, 2).reshape({rows, n}));
+            r[2] = dy.sum(0);
+            return r;
+        }
+        const Tensor a = aligned(saved[0].transpose(1, 2)), w = aligned(saved[1]), dy = aligned(g[0]);
         if (ctx->needs_input_grad(0)) {
             Tensor da = torch::empty_like(a);
             const float* wp[1] = {fp(w)};

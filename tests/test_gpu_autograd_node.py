@@ -140,3 +140,39 @@ def test_forward_mode_is_refused_by_the_whole_layer_without_gradients(which):
             setattr(layer.ff, which, fwd.make_dual(t, torch.ones_like(t)))
         with pytest.raises(RuntimeError, match="jvp"):
             layer(x, torch.ones(B, L, device="cuda"), mat)
+
+
+def test_projections_around_a_differentiable_core_are_twice_differentiable():
+    """The layer with the plain PyTorch core: gradients of a function of the first gradients, against the same layer written
+    out in float64.  Both routes are chains of fp32 products of at most 64 terms with values of order one: 2^-24 a step,
+    some hundred steps in all."""
+    B, H, L, d, dim = 2, 2, 32, 32, 64
+    cfg = dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=B, block_size=32, transformer_dim=dim, attention_dropout=0.0,
+               task="lra-pathfinder32-curv_contour_length_14")
+    torch.manual_seed(3)
+    layer = Attention(cfg).cuda()
+    mask = torch.ones(B, L, device="cuda")
+    x, dy = torch.randn(B, L, dim, device="cuda", requires_grad=True), torch.randn(B, L, dim, device="cuda", requires_grad=True)
+    params = list(layer.parameters())
+    r = [torch.randn_like(t) for t in [x] + params]
+
+    def written_out(x, dy, params):
+        (wq, bq, wk, bk, wv, bv, wf, bf), lin = params, torch.nn.functional.linear
+        q, k, v = (layer.split_heads(lin(x, w, b)) for w, b in ((wq, bq), (wk, bk), (wv, bv)))
+        p = torch.softmax(q @ k.transpose(-1, -2) / d ** 0.5, -1)
+        return lin(layer.combine_heads(p @ v), wf, bf)
+
+    def second(forward, x, dy, params, r):
+        first = torch.autograd.grad(forward(x, dy, params), [x] + params, dy, create_graph=True)
+        return torch.autograd.grad(sum((a * b).sum() for a, b in zip(first, r)), [x, dy] + params, allow_unused=True)
+
+    assert [n for n, _ in layer.named_parameters()] == [f"{m}.{t}" for m in ("W_q", "W_k", "W_v", "ff") for t in ("weight", "bias")]
+    got = second(lambda x, dy, p: layer(x, mask)[0], x, dy, params, r)
+    up = lambda t: t.detach().cpu().double().requires_grad_()
+    ref = second(written_out, up(x), up(dy), [up(t) for t in params], [t.cpu().double() for t in r])
+    assert len(got) == len(ref) == 10
+    for a, b in zip(got, ref):
+        if b is None or float(b.norm()) < 1e-9:  # (exactly zero: what a bias's shift leaves unchanged)
+            assert a is None or float(a.norm()) < 1e-3
+            continue
+        assert float((a.cpu().double() - b).norm() / b.norm()) < 1e-5
