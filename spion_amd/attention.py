@@ -11,6 +11,7 @@ import math
 
 import torch
 import torch.nn as nn
+from torch.nn.modules import module as _nn_module
 
 from . import _lib
 
@@ -87,6 +88,12 @@ def _core_types():
     return _CORES
 
 
+def _observed(m):
+    """Whether somebody watches or replaced this module's call: hooks of its own, or a forward set on the instance."""
+    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                or "forward" in m.__dict__)
+
+
 class Attention(nn.Module):
     def __init__(self, config, inference=False):
         super().__init__()
@@ -157,12 +164,13 @@ class Attention(nn.Module):
 
     def _compiled_node(self, X, mask):
         """The compiled node when it covers the projections of this call (csrc/project.hip: fp32 on the GPU, rows and
-        features in multiples of 32, plain linear layers of the layer's sizes without hooks, no autocast), else None."""
-        if not (self.fused_qkv and X.is_cuda and isinstance(mask, torch.Tensor) and not torch.is_autocast_enabled()):
+        features in multiples of 32, plain linear layers of the layer's sizes, no hooks on them or on all modules, no
+        autocast), else None."""
+        if not (self.fused_qkv and X.is_cuda and isinstance(mask, torch.Tensor) and not torch.is_autocast_enabled()) \
+                or _nn_module._has_any_global_hook():
             return None
         for m in (self.W_q, self.W_k, self.W_v, self.ff):
-            if (type(m) is not nn.Linear or m.bias is None or m._forward_hooks or m._forward_pre_hooks
-                    or m._backward_hooks or m._backward_pre_hooks):
+            if type(m) is not nn.Linear or m.bias is None or _observed(m):
                 return None
         node = _lib.autograd_node()
         if node is None or not node.projections_fit(
@@ -187,8 +195,7 @@ class Attention(nn.Module):
         (reconstruct_for_blocksparse takes a config of its own; the module then says so), or has hooks."""
         core = self.block_attn
         if (type(core) not in _core_types() or not core.reads_views
-                or core.head_shape != (X.shape[0], self.num_head, X.shape[1], self.head_dim) or core._forward_hooks
-                or core._forward_pre_hooks or core._backward_hooks or core._backward_pre_hooks):
+                or core.head_shape != (X.shape[0], self.num_head, X.shape[1], self.head_dim) or _observed(core)):
             return None
         idx = core.csr_cache.get(mat, core.block_size)
         key_mask, is_mask = core.key_operand(mask if mask.dtype == torch.float32 else mask.float())

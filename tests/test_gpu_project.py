@@ -128,6 +128,36 @@ def test_layer_in_one_call_matches_its_steps(heads, d, L, masked):
     assert torch.equal(again[2], fused[2])
 
 
+@pytest.mark.parametrize("how", ["global hook", "global pre-hook", "own forward"])
+def test_layer_runs_its_modules_when_they_are_watched(how):
+    """Hooks on all modules see the core and the output projection, and a forward set on an instance runs."""
+    B, L = 2, 64
+    cfg = dict(head_dim=32, num_head=2, max_seq_len=L, batch_size=B, block_size=32, transformer_dim=96, attention_dropout=0.0,
+               task="lra-image")
+    layer = spion_amd.Attention(cfg, inference=True).cuda()
+    layer.reconstruct_for_blocksparse(cfg)
+    args = (torch.randn(B, L, 96, device="cuda"), torch.ones(B, L, device="cuda"), torch.eye(2, device="cuda"))
+    plain = layer(*args)[0]
+    seen, handle = [], None
+    if how == "own forward":
+        for m in (layer.ff, layer.block_attn):
+            m.forward = lambda *a, m=m: (seen.append(m), type(m).forward(m, *a))[1]
+    elif how == "global hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda m, i, o: seen.append(m) and None)
+    else:
+        handle = torch.nn.modules.module.register_module_forward_pre_hook(lambda m, i: seen.append(m) and None)
+    try:
+        watched = layer(*args)[0]
+    finally:
+        if handle:
+            handle.remove()
+    assert layer.ff in seen and layer.block_attn in seen
+    assert float((watched - plain).detach().norm() / plain.detach().norm()) < 2e-6
+    if handle:
+        seen.clear()
+        assert torch.equal(layer(*args)[0], plain) and not seen
+
+
 @pytest.mark.parametrize("outputs", [48, 64, 160])
 def test_layer_with_a_replaced_output_projection(outputs):
     """Another width of the output projection: on the kernels where it is a multiple of 32, torch's steps where not."""
