@@ -239,6 +239,7 @@ bool projections_fit(const Tensor& x, const Tensor& wq, const Tensor& wk, const 
     const int64_t n = H * d, dim = x.size(2), outputs = wf.size(0), rows = x.size(0) * x.size(1);
     for (const int64_t size : {n, dim, outputs, rows})
         if (size <= 0 || size % 32) return false;
+    if (rows >= 1 << 30 || std::max(3 * n, outputs) > 1 << 20 || std::max(3 * n * dim, outputs * n) > 1 << 30) return false;
     return projection_fits(x, wq, bq, n, dim) && projection_fits(x, wk, bk, n, dim) && projection_fits(x, wv, bv, n, dim) &&
            projection_fits(x, wf, bf, outputs, n);
 }

@@ -22,6 +22,11 @@
 
 namespace spion {
 
+// Most rows a call may have, and what a matrix stored in one piece has for `seg`: no row index reaches it, and twice as
+// much is still an int.
+constexpr int MAX_ROWS = INT_MAX / 2, ONE_PIECE = INT_MAX / 2;
+static_assert(MAX_ROWS - 1 < ONE_PIECE && ONE_PIECE <= INT_MAX - ONE_PIECE, "every row lies in the first piece");
+
 // Rows of a matrix that is stored as up to three matrices of `seg` rows each.
 struct SegRows {
     const float* p[3];
@@ -312,15 +317,15 @@ static bool wide_tiles(long long M, long long N) {
 
 static bool project_args(const char* who, long long M, int n, int segs, int K, std::initializer_list<const void*> ptrs) {
     bool ok = M > 0 && M % 32 == 0 && n > 0 && n % 32 == 0 && K > 0 && K % 32 == 0 && segs >= 1 && segs <= 3 &&
-              M <= INT_MAX / 2 && (long long)segs * n <= 1 << 20;
+              M <= MAX_ROWS && (long long)segs * n <= 1 << 20 && (long long)segs * n * K <= 1 << 30;
     for (const void* p : ptrs) ok = ok && p && reinterpret_cast<uintptr_t>(p) % 16 == 0;
-    if (!ok) set_error("%s: rows, features and outputs must be positive multiples of 32, pointers 16-byte aligned (got %lld, %d, %d x %d)",
+    if (!ok) set_error("%s: rows, features and outputs must be positive multiples of 32 (at most 2^30 rows, 2^20 outputs, 2^30 weights), pointers 16-byte aligned (got %lld, %d, %d x %d)",
                        who, M, K, segs, n);
     return ok;
 }
-static SegRows plain_rows(const float* p, int ld) { return SegRows{{p, p, p}, INT_MAX / 4, ld}; }
+static SegRows plain_rows(const float* p, int ld) { return SegRows{{p, p, p}, ONE_PIECE, ld}; }
 static SegRows weight_rows(const float* const* W, int segs, int n, int K) {
-    return SegRows{{W[0], W[segs > 1 ? 1 : 0], W[segs > 2 ? 2 : 0]}, segs > 1 ? n : INT_MAX / 4, K};
+    return SegRows{{W[0], W[segs > 1 ? 1 : 0], W[segs > 2 ? 2 : 0]}, segs > 1 ? n : ONE_PIECE, K};
 }
 
 int project_forward(const float* X, const float* const* W, const float* const* b, float* Y, long long M, int n, int segs,
@@ -331,7 +336,7 @@ int project_forward(const float* X, const float* const* W, const float* const* b
     }
     for (int s = 0; s < segs; ++s)
         if (!project_args("spion_project_forward", M, n, segs, K, {W[s], b[s]})) return 1;
-    const SegBias bias{{b[0], b[segs > 1 ? 1 : 0], b[segs > 2 ? 2 : 0]}, segs > 1 ? n : INT_MAX / 4};
+    const SegBias bias{{b[0], b[segs > 1 ? 1 : 0], b[segs > 2 ? 2 : 0]}, segs > 1 ? n : ONE_PIECE};
     const int N = segs * n;
     const bool ok = wide_tiles(M, N)
         ? launch_project<false, false, 2, 2, false>(plain_rows(X, K), weight_rows(W, segs, n, K), bias, Y, N, nullptr, (int)M, N, K, 1, K / 32, stream)
@@ -348,7 +353,7 @@ int project_backward_input(const float* dY, const float* const* W, float* dX, lo
     for (int s = 0; s < segs; ++s)
         if (!project_args("spion_project_backward_input", M, n, segs, K, {W[s]})) return 1;
     const int N = segs * n;
-    const SegBias none{{nullptr, nullptr, nullptr}, INT_MAX / 4};
+    const SegBias none{{nullptr, nullptr, nullptr}, ONE_PIECE};
     const bool ok = wide_tiles(M, K)
         ? launch_project<false, true, 2, 2, false>(plain_rows(dY, N), weight_rows(W, segs, n, K), none, dX, K, nullptr, (int)M, K, N, 1, N / 32, stream)
         : launch_project<false, true, 1, 1, false>(plain_rows(dY, N), weight_rows(W, segs, n, K), none, dX, K, nullptr, (int)M, K, N, 1, N / 32, stream);
@@ -372,7 +377,7 @@ int project_backward_weight(const float* dY, const float* X, float* dW, float* d
     const int want = weight_pieces(M, N, K), rows = (int)(M / 32);
     const int chunks = (rows + want - 1) / want, pieces = (rows + chunks - 1) / chunks;
     float* sums = ws + (size_t)pieces * N * K;
-    const SegBias none{{nullptr, nullptr, nullptr}, INT_MAX / 4};
+    const SegBias none{{nullptr, nullptr, nullptr}, ONE_PIECE};
     if (!launch_project<true, true, 1, 1, true>(plain_rows(dY, N), plain_rows(X, K), none, ws, K, sums, N, K, (int)M, pieces,
                                                 chunks, stream))
         return 1;

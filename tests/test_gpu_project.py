@@ -60,6 +60,25 @@ def test_projection_kernels_match_float64(rows, dim, n, segs):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
+def test_rows_past_a_quarter_of_the_int_range():
+    """Row indices from 2^29 on are rows of the matrix like any other: the last 64 of 2^29 + 32 rows."""
+    rows = 2 ** 29 + 32
+    if torch.cuda.mem_get_info()[0] < 160 * 2 ** 30:
+        pytest.skip("needs 140 GB of device memory")
+    x = torch.zeros(rows, 32, device="cuda")
+    tail = torch.randn(64, 32, generator=torch.Generator().manual_seed(1)).cuda()
+    x[-64:] = tail
+    w, b = torch.randn(32, 32, device="cuda"), torch.randn(32, device="cuda")
+    y = torch.empty(rows, 32, device="cuda")
+    core, stream = _lib.core(), torch.cuda.current_stream().cuda_stream
+    assert core.spion_project_forward(x.data_ptr(), _ptrs([w]), _ptrs([b]), y.data_ptr(), rows, 32, 1, 32, stream) == 0
+    _check(y[-64:], tail, w.t(), b)
+    assert core.spion_project_backward_input(x.data_ptr(), _ptrs([w]), y.data_ptr(), rows, 32, 1, 32, stream) == 0
+    _check(y[-64:], tail, w)
+    del x, y
+    torch.cuda.empty_cache()
+
+
 def test_weight_gradient_of_one_signed_data_keeps_fp32_accuracy():
     """All operands just above a bf16 number, summed over many rows: the small partial products then share a sign and must
     not be lost against the large sum."""
