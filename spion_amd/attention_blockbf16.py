@@ -24,8 +24,10 @@ def _penalty(mask, m, dev):
     if mask.dtype == torch.float32 and mask.is_cuda and mask.is_contiguous() and mask.shape == (m.batch_size, m.seq_len):
         pen = torch.empty((m.num_batches, m.seq_len), dtype=torch.float32, device=dev)
         index = dev.index if dev.index is not None else torch.cuda.current_device()
-        m.lib.spion_key_penalty(mask.data_ptr(), pen.data_ptr(), m.batch_size, m.num_heads, m.seq_len,
-                                _lib._raw_stream(index))
+        if m.lib.spion_key_penalty(mask.data_ptr(), pen.data_ptr(), m.batch_size, m.num_heads, m.seq_len,
+                                   _lib._raw_stream(index)) != 0:
+            _lib.check_error("spion_key_penalty")
+            raise _lib.SpionLibraryError("spion_key_penalty failed")
         return pen
     return (1e6 * (1.0 - mask.to(torch.float32))).repeat_interleave(m.num_heads, 0).contiguous()
 

@@ -100,3 +100,21 @@ def test_node_refuses_projections_of_other_sizes(which):
         _lib.autograd_node().project_heads(torch.zeros(2, 64, 96), w[0], w[1], w[2], b[0], b[1], b[2], 2, 32, 0)
     with pytest.raises(ValueError, match="projection"):
         _lib.autograd_node().merge_heads(torch.zeros(2, 2, 64, 32 if which == "rows" else 48), torch.zeros(64, 96), torch.zeros(32), 0)
+
+
+def test_bf16_module_reports_a_failed_key_penalty(monkeypatch):
+    """The penalties' buffer is uninitialised where the launch failed: the call must not go on with it."""
+    from types import SimpleNamespace
+
+    from spion_amd import attention_blockbf16 as bf16
+
+    monkeypatch.setattr(_lib, "_raw_stream", lambda index: 0)
+    mask = SimpleNamespace(dtype=torch.float32, is_cuda=True, is_contiguous=lambda: True, shape=(2, 64), data_ptr=lambda: 0)
+    m = SimpleNamespace(batch_size=2, seq_len=64, num_heads=2, num_batches=4, lib=_lib.core())
+    dev = SimpleNamespace(index=0)
+    monkeypatch.setattr(bf16.torch, "empty", lambda *a, **k: SimpleNamespace(data_ptr=lambda: 0))
+    with pytest.raises(_lib.SpionLibraryError, match="spion_key_penalty"):
+        bf16._penalty(mask, m, dev)
+    monkeypatch.setattr(m, "lib", SimpleNamespace(spion_key_penalty=lambda *a: 1))
+    with pytest.raises(_lib.SpionLibraryError, match="spion_key_penalty"):
+        bf16._penalty(mask, m, dev)
