@@ -383,6 +383,7 @@ std::vector<Tensor> sparse_layer(const Tensor& x, const Tensor& wq, const Tensor
                                  const c10::optional<Tensor>& mask_or_pen, bool is_mask, const Tensor& offsets,
                                  const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t num_heads, int64_t head_dim,
                                  int64_t stream) {
+    const c10::DeviceGuard on(x.device());  // `stream` is one of x's device, which need not be the current one
     const auto pen = penalty_of(mask_or_pen, is_mask, num_heads, stream);
     const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
     if (without_node({&x, &wq, &wk, &wv, &bq, &bk, &bv, &wf, &bf, &pen_or_none})) {
@@ -401,9 +402,11 @@ std::vector<Tensor> sparse_layer(const Tensor& x, const Tensor& wq, const Tensor
 // The two projections by themselves, around a core of the caller's (the dense phase).
 std::vector<Tensor> project_heads(const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& bq,
                                   const Tensor& bk, const Tensor& bv, int64_t num_heads, int64_t head_dim, int64_t stream) {
+    const c10::DeviceGuard on(x.device());
     return QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream);
 }
 Tensor merge_heads(const Tensor& heads, const Tensor& w, const Tensor& b, int64_t stream) {
+    const c10::DeviceGuard on(heads.device());
     return MergeNode::apply(heads, w, b, stream);
 }
 
@@ -411,6 +414,7 @@ std::vector<Tensor> sparse_attention(const Tensor& query, const Tensor& key, con
                                      const c10::optional<Tensor>& mask_or_pen, bool is_mask, const Tensor& offsets,
                                      const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t num_heads,
                                      bool reads_views, int64_t stream) {
+    const c10::DeviceGuard on(query.device());
     const auto pen = penalty_of(mask_or_pen, is_mask, num_heads, stream);
     const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
     if (without_node({&query, &key, &value, &pen_or_none})) {

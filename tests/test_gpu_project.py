@@ -222,3 +222,20 @@ def test_layer_with_a_core_of_other_heads_raises():
     layer.reconstruct_for_blocksparse(dict(cfg, num_head=4))
     with pytest.raises(ValueError, match="does not match the handle"):
         layer(torch.randn(B, L, 96, device="cuda"), torch.ones(B, L, device="cuda"), torch.eye(2, device="cuda"))
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs two GPUs")
+def test_layer_runs_on_its_inputs_device():
+    """A layer on another GPU than the current one, as torch's linear layers allow."""
+    B, L = 2, 64
+    cfg = dict(head_dim=32, num_head=2, max_seq_len=L, batch_size=B, block_size=32, transformer_dim=96, attention_dropout=0.0,
+               task="lra-text")
+    args = (torch.randn(B, L, 96, device="cuda:1"), torch.ones(B, L, device="cuda:1"), torch.eye(2, device="cuda:1"))
+    with torch.cuda.device(1):
+        layer = spion_amd.Attention(cfg, inference=True).cuda()
+        layer.reconstruct_for_blocksparse(cfg)
+        there = layer(*args)[0]
+    with torch.cuda.device(0):
+        here = layer(*args)[0]
+        here.sum().backward()
+    assert here.device == there.device and torch.equal(here, there)
