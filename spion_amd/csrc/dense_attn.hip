@@ -1064,8 +1064,7 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_col64_kernel(
         DmaTileF32::load(wO, lo, ol, I * 32 * old_ * 4, ox);
         DmaTileF32::load(wO, lo + DmaTileF32::TILE, ol, I * 32 * old_ * 4 + 128, ox);
     };
-    const Split3<KH> vts = split3(vt);
-    settle(vts);
+    settle(vt);
     if (nu > 0) {
         issue(w);
         float gl = ld1(rG, li * 4, w * 128);
@@ -1087,12 +1086,12 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_col64_kernel(
             }
             __builtin_amdgcn_sched_barrier(0);
             const f32x16 init = __builtin_amdgcn_mfma_f32_32x32x2f32(ga, 1.0f, splat16(0.f), 0, 0, 0);  // -g_i in every column
-            f32x16 dp = mma_feat_init<D>(go, vts, init);  // register = query, lane = key
+            f32x16 dp = mma_feat_f32<D>(go, vt, init);  // register = query, lane = key
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pc[r];
-            mma_b_split<D>(ds, qb, ak);
-            mma_b_split<D>(pc, ob, av);
+            mma_b_f32<D>(ds, qb, ak);
+            mma_b_f32<D>(pc, ob, av);
         }
     }
     if (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles

@@ -480,7 +480,6 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_row_kernel(const float* __restrict__ K
     g += __shfl_xor(g, 32, 64);
     if (w == 0 && h == 0) G[(size_t)bh * L + I * 32 + li] = -g;
     const f32x16 gneg = splat16(-g);
-    const Split3<KH> gos = split3(go);
 
     const int t0 = ix.t_rp[I], cnt = ix.t_rp[I + 1] - t0;
     const int n = cnt > w ? (cnt - w + WAVES - 1) / WAVES : 0;
@@ -507,7 +506,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_row_kernel(const float* __restrict__ K
             lds_get_feat32(Tx, li, h, vt);
             lds_put_cols(T, li, h, x.p);
             lds_get_rows(T, li, h, pr);                        // pr[r] = P[query li][key acc_row(r, h)]
-            const f32x16 dp = mma_feat_init<D>(vt, gos, gneg);  // dp[r] = dO_i . v_j - g_i
+            const f32x16 dp = mma_feat_f32<D>(vt, go, gneg);  // dp[r] = dO_i . v_j - g_i
             lds_put_lin(Tx, l, x.b);
             lds_get_cols(Tx, li, h, kb[0]);
             float ds[16];

@@ -395,14 +395,20 @@ struct DmaTileF32 {
 // GHz under fp32 chains, 1.98 to 2.2 GHz with every product split).  So
 //   * products over the head dimension, whose other operand a wavefront keeps for all its tiles, are split: one
 //     operand per tile;
-//   * products over a tile's rows, which need two operands split, run on the bf16 pipe at d = 64 (one of the two
-//     serves two products) and in the column pass (two of its three products; three wavefronts per SIMD hide the
-//     splitting), on the fp32 pipe in the forward and the row pass at d = 32.
-// Measured in us per launch, all fp32 / all split / as chosen: 32 x 2 heads of 4096 tokens, d = 32, 32 x 32 blocks, a
-// tenth kept: forward 162 / 176 / 150, row pass 141 / 134 / 130, column pass 185 / 168 / 168; 256 x 2 heads of 1024:
-// 143 / 140 / 134, 122 / 118 / 117, 147 / 133 / 133; 3 x 8 heads of 4000, d = 64, all fp32 / split: 98 / 75, 99 / 82,
-// 119 / 116.  The dense kernels (dense_attn.hip, 64 x 2 heads of 1024): forward 181 / 172 / 171, row pass (split)
-// 178 / 155, column pass 236 / 260 / 211 (its three splits do not fit the registers of three wavefronts per SIMD).
+//   * products over a tile's rows, which need two operands split, run on the bf16 pipe in the forward and the row pass at
+//     d = 64 (one of the two serves two products) and in the column pass at d = 32 (two of its three products; three
+//     wavefronts per SIMD hide the splitting), on the fp32 pipe in the forward and the row pass at d = 32;
+//   * the column pass at d = 64 uses fp32 chains alone: split operands for its five products spill registers, and whole
+//     steps are 0 to 4 % faster without (split / fp32 chains, same box: 64 x 2 heads of 1024, 14 % kept, 194 / 187 us; 16 x 4
+//     of 2048, 10 %, 262 / 255; 3 x 8 of 4000, 8 %, 278 / 274).
+// Measured in us per launch in a training loop, all kernels on fp32 chains / as now, same box.  32 x 2 heads of 4096 tokens,
+// d = 32, 32 x 32 blocks, a tenth kept: forward 162 / 155, row pass 141 / 134, column pass 184 / 161; 256 x 2 heads of 1024:
+// 139 / 139, 122 / 121, 148 / 132; 2 x 2 of 8192, a fifth kept (two sweeps): 104 / 97, 76 / 71, 98 / 91; 3 x 8 heads of 4000,
+// d = 64: 98 / 76, 99 / 80.  The dense kernels (dense_attn.hip), 64 x 2 heads of 1024, d = 32: forward 180 / 177, row pass 177
+// / 156, column pass 235 / 209 (of its products the first; three splits do not fit the registers of three wavefronts per
+// SIMD: 260); 4 x 2 of 3072: 163 / 136, 108 / 86, 148 / 118; 4 x 8 of 2048, d = 64: 319 / 276, 276 / 240.  The dense
+// tiles of element patterns (hybrid_kernels.h, 32 x 2 heads of 4096): forward 97 / 91, column pass 99 / 96; the row pass (84 / 84)
+// stays on fp32 chains.
 // Against float64 the outputs and gradients of both are as close as the fp32 chains' or closer (2-norms, 1024 to 4096
 // tokens: 1.0e-7 to 5.8e-7 where those gave 2.2e-7 to 6.1e-7).
 // acc = init + A.B over the head dimension; B is an operand the kernel keeps.
@@ -1295,8 +1301,7 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
             DmaTileF32::load(wO, lo, ol, I * 32 * old_ * 4, ox);
             DmaTileF32::load(wO, lo + DmaTileF32::TILE, ol, I * 32 * old_ * 4 + 128, ox);
         };
-        const Split3<KH> vts = split3(vt);
-        settle(vts);
+        settle(vt);
         if (nu > 0) {
             int4 dn = desc[w];
             issue(dn);
@@ -1322,12 +1327,12 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
                 dn = dnn;
                 __builtin_amdgcn_sched_barrier(0);
                 const f32x16 init = __builtin_amdgcn_mfma_f32_32x32x2f32(ga, 1.0f, splat16(0.f), 0, 0, 0);  // -g_i in every column
-                f32x16 dp = mma_feat_init<D>(go, vts, init);  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
+                f32x16 dp = mma_feat_f32<D>(go, vt, init);  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pc[r];
-                mma_b_split<D>(ds, qb, ak);
-                mma_b_split<D>(pc, ob, av);
+                mma_b_f32<D>(ds, qb, ak);
+                mma_b_f32<D>(pc, ob, av);
             }
         }
     }
