@@ -151,19 +151,27 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg_kernel(
     const u32x4 wM = rsrc_words(MASK ? pen + (size_t)bh * L : pen, MASK ? (size_t)L * 4 : 0);
     const int alin = lin_voff(l, L);
     const int vld = RM ? ild : L, VSTEP = RM ? 32 * ild * 4 : 128;
-    const int kl = DmaTileF32::voff(l, ild), kx = DmaTileF32::extra_step(ild);
+    const int kx = DmaTileF32::extra_step(ild);
     const int vl = DmaTileF32::voff(l, vld), vx = DmaTileF32::extra_step(vld);
     const float c2 = scale * LOG2E;
 
-    float q[KH];
-    if constexpr (RM) ldr_rows<D>(rQ, (li * ild + h * KH) * 4, I * 32 * ild * 4, q);
-    else ldr_cols<D>(rQ, L, (h * KH * L + li) * 4, I * 128, q);
+    auto load_q = [&](float (&q)[KH], int l) {
+        if constexpr (RM) ldr_rows<D>(rQ, ((l & 31) * ild + (l >> 5) * KH) * 4, I * 32 * ild * 4, q);
+        else ldr_cols<D>(rQ, L, ((l >> 5) * KH * L + (l & 31)) * 4, I * 128, q);
 #pragma unroll
-    for (int s = 0; s < KH; ++s) q[s] *= c2;
-    const Split3<KH> qs = split3(q);
+        for (int s = 0; s < KH; ++s) q[s] *= c2;
+    };
+    float q[KH];
+    load_q(q, l);
 
-    float m = -10.f * LOG2E, z = 0.f;  // models/attn.cu:17
+    float m, z;
     f32x16 S[MAXT];
+    // as in tile_fwd_kernel (tile_kernels.h); qk: the query operand, split or whole
+    auto own_softmax = [&](const auto& qk, int l) {
+    const int h = l >> 5, li = l & 31;
+    const int kl = DmaTileF32::voff(l, ild);
+    m = -10.f * LOG2E;  // models/attn.cu:17
+    z = 0.f;
     {
         // K tile u + 1 (and its key penalties) is requested before the chain of tile u starts; loads into LDS and
         // the map's stores share one in-order counter (wait_vm)
@@ -200,7 +208,7 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg_kernel(
                 }
                 wait_lgkm0();  // the tile's space is requested again one iteration on
                 __builtin_amdgcn_sched_barrier(0);
-                S[u] = mma_feat_init<D>(kf, qs, init);  // S^T: register = key, lane = query
+                S[u] = mma_feat_init<D>(kf, qk, init);  // S^T: register = key, lane = query
                 m = max16(S[u], m);
             }
         }
@@ -216,6 +224,13 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg_kernel(
                 z += e;
             }
         }
+    }
+    };
+    own_softmax(split3(q), l);
+    if (split_failed(z)) {
+        const int l2 = second_walk(l);
+        load_q(q, l2);
+        own_softmax(whole(q), l2);
     }
     const float m_own = m;
     z += __shfl_xor(z, 32, 64);
@@ -332,29 +347,36 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
     const rsrc_t rA = make_rsrc(Attn + (size_t)bh * L * L, (size_t)L * L * 4);
     const u32x4 wK = rsrc_words(K + ib, hbytes), wV = rsrc_words(V + ib, hbytes);
     const u32x4 wM = rsrc_words(MASK ? pen + (size_t)bh * L : pen, MASK ? (size_t)L * 4 : 0);
-    const int alin = lin_voff(l, L);
-    const int kl = DmaTileF32::voff(l, ild), kx = DmaTileF32::extra_step(ild);
+    const int kx = DmaTileF32::extra_step(ild);
     const float c2 = scale * LOG2E;
-    auto issue = [&](const u32x4& r, int J) {
+    auto issue = [&](const u32x4& r, int J, int kl) {
         DmaTileF32::load(r, lb, kl, J * 32 * ild * 4, kx);
         DmaTileF32::load(r, lb + DmaTileF32::TILE, kl, J * 32 * ild * 4 + 128, kx);
     };
 
-    float q[KH];
-    ldr_rows<D>(make_rsrc(Q + ib, hbytes), (li * ild + h * KH) * 4, I * 32 * ild * 4, q);
+    auto load_q = [&](float (&q)[KH], int l) {
+        ldr_rows<D>(make_rsrc(Q + ib, hbytes), ((l & 31) * ild + (l >> 5) * KH) * 4, I * 32 * ild * 4, q);
 #pragma unroll
-    for (int s = 0; s < KH; ++s) q[s] *= c2;
-    const Split3<KH> qs = split3(q);
-    settle(qs);
+        for (int s = 0; s < KH; ++s) q[s] *= c2;
+    };
+    float q[KH];
+    load_q(q, l);
 
-    float m = -10.f * LOG2E, z = 0.f;  // models/attn.cu:17
+    float m, z;
     f32x16 S[MAXT];
+    // as in tile_fwd_kernel (tile_kernels.h); qk: the query operand, split or whole
+    auto own_softmax = [&](const auto& qk, int l) {
+    const int h = l >> 5, li = l & 31;
+    const int kl = DmaTileF32::voff(l, ild);
+    settle(qk);
+    m = -10.f * LOG2E;  // models/attn.cu:17
+    z = 0.f;
     {
         const auto a_k = DmaTileF32::own8_addr(Tb + h * DmaTileF32::TILE, li);  // K[key li][feature 32h + s]
         const char* Tm = Tb + 2 * DmaTileF32::TILE + 16 * h;
         auto issue_k = [&](int u) {
             const int J = w + u * WAVES;
-            issue(wK, J);
+            issue(wK, J, kl);
             if constexpr (MASK) dma_b32(wM, lb + 2 * DmaTileF32::TILE, l * 4, J * 128);
         };
         if (nu > 0) issue_k(0);
@@ -378,7 +400,7 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
                 wait_lgkm0();
                 if (u + 1 < MAXT && u + 1 < nu) issue_k(u + 1);
                 __builtin_amdgcn_sched_barrier(0);
-                S[u] = mma_feat_init<D>(kf, qs, init);  // S^T: register = key, lane = query
+                S[u] = mma_feat_init<D>(kf, qk, init);  // S^T: register = key, lane = query
                 m = max16(S[u], m);
             }
         }
@@ -394,6 +416,13 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
                 z += e;
             }
         }
+    }
+    };
+    own_softmax(split3(q), l);
+    if (split_failed(z)) {
+        const int l2 = second_walk(l);
+        load_q(q, l2);
+        own_softmax(whole(q), l2);
     }
     const float m_own = m;
     z += __shfl_xor(z, 32, 64);
@@ -416,8 +445,9 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
 
     f32x16 o[2] = {splat16(0.f), splat16(0.f)};  // O^T: register = feature (+32), lane = query
     {
+        const int kl = DmaTileF32::voff(l, ild), alin = lin_voff(l, L);
         const auto a_v = DmaTileF32::cols_addr(Tb, li, h);  // vb[c][s] = V[key acc_row(s, h)][feature 32c + li]
-        if (nu > 0) issue(wV, w);
+        if (nu > 0) issue(wV, w, kl);
 #pragma unroll
         for (int u = 0; u < MAXT; ++u) {
             if (u < nu) {
@@ -434,13 +464,35 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
                 f32x4 pl[4];
                 lds_get_lin(T, l, pl);
                 wait_lgkm0();
-                if (u + 1 < MAXT && u + 1 < nu) issue(wV, w + (u + 1) * WAVES);
+                if (u + 1 < MAXT && u + 1 < nu) issue(wV, w + (u + 1) * WAVES, kl);
                 __builtin_amdgcn_sched_barrier(0);
                 const Split3<16> ps = split3(p);
 #pragma unroll
                 for (int c = 0; c < 2; ++c) o[c] = mma_split(split3(vb[c]), ps, o[c]);
                 str_tile_lin(rA, alin, (J * 32 * L + I * 32) * 4, L, pl);
             }
+        }
+    }
+    if (split_failed(o)) {  // once more, from the map tiles just stored (the registers they came from are long reused)
+        const int l2 = second_walk(l), kl = DmaTileF32::voff(l2, ild), alin = lin_voff(l2, L);
+        const auto a_v = DmaTileF32::cols_addr(Tb, l2 & 31, l2 >> 5);
+        o[0] = splat16(0.f);
+        o[1] = splat16(0.f);
+        wait_vm<0>();
+#pragma unroll 1
+        for (int J = w; J < nbr; J += WAVES) {
+            issue(wV, J, kl);
+            f32x4 pl[4];
+            ldr_tile_lin_l2(rA, alin, (J * 32 * L + I * 32) * 4, L, pl);
+            wait_vm<0>();
+            float p[16], vb[2][16];
+            lds_put_lin(T, l2, pl);
+            lds_get_cols(T, l2 & 31, l2 >> 5, p);
+            DmaTileF32::get(a_v, vb[0]);
+            DmaTileF32::get(a_v, vb[1], DmaTileF32::TILE);
+            wait_lgkm0();
+#pragma unroll
+            for (int c = 0; c < 2; ++c) o[c] = mma_chain(vb[c], p, o[c]);
         }
     }
     reduce_store_rows<WAVES>(o[0], Out + ob, I * 32, w, li, h, lds, old_);
@@ -488,16 +540,17 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
     float* T = lds_t[w];          // map tile on its way to memory
     float* Tk = T + 32 * TS;
     float* Tv = T + 64 * TS;
-    const int klin = lin_voff(l, ild), alin = lin_voff(l, L);
-    const int vld = RM ? ild : L, vlin = lin_voff(l, vld), VSTEP = RM ? 32 * ild * 4 : 128;
+    const int vld = RM ? ild : L, VSTEP = RM ? 32 * ild * 4 : 128;
     const float c2 = scale * LOG2E;
 
-    float q[KH];
-    if constexpr (RM) ldr_rows<D>(rQ, (li * ild + h * KH) * 4, I * 32 * ild * 4, q);
-    else ldr_cols<D>(rQ, L, (h * KH * L + li) * 4, I * 128, q);
+    auto load_q = [&](float (&q)[KH], int l) {
+        if constexpr (RM) ldr_rows<D>(rQ, ((l & 31) * ild + (l >> 5) * KH) * 4, I * 32 * ild * 4, q);
+        else ldr_cols<D>(rQ, L, ((l >> 5) * KH * L + (l & 31)) * 4, I * 128, q);
 #pragma unroll
-    for (int s = 0; s < KH; ++s) q[s] *= c2;
-    const Split3<KH> qs = split3(q);
+        for (int s = 0; s < KH; ++s) q[s] *= c2;
+    };
+    float q[KH];
+    load_q(q, l);
 
     struct Pre1 {
         f32x4 k[4];
@@ -507,25 +560,29 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
         f32x4 k[4], v[4];
         float pj[MASK ? 16 : 1];
     };
-    auto penalties = [&](float (&pj)[MASK ? 16 : 1], int J) {
+    auto penalties = [&](float (&pj)[MASK ? 16 : 1], int J, int l) {
         if constexpr (MASK) {
             float t[16];
-            ldr_4x4(rM, 16 * h, J * 128, t);
+            ldr_4x4(rM, 16 * (l >> 5), J * 128, t);
 #pragma unroll
             for (int r = 0; r < 16; ++r) pj[r] = t[r];
         }
     };
 
     // ---- sweep 1: running maximum and sum over this wavefront's tiles (log2 domain) ----------------
-    float m = -10.f * LOG2E, z = 0.f;  // models/attn.cu:17
-    {
+    float m, z;
+    auto sweep1 = [&](const auto& qk, int l) {  // qk: the query operand, split or whole
+        const int h = l >> 5, li = l & 31;
+        const int klin = lin_voff(l, ild);
+        m = -10.f * LOG2E;  // models/attn.cu:17
+        z = 0.f;
         Pre1 xa, xb;
         tile_pipeline(
             nu, xa, xb,
             [&](Pre1& x, int i) {
                 const int J = w + min(i, nu - 1) * WAVES;
                 ldr_tile_lin(rK, klin, J * 32 * ild * 4, ild, x.k);
-                penalties(x.pj, J);
+                penalties(x.pj, J, l);
             },
             [&](Pre1& c, int) {
                 lds_put_lin(Tk, l, c.k);
@@ -537,13 +594,20 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
 #pragma unroll
                     for (int r = 0; r < 16; ++r) init[r] = -LOG2E * c.pj[r];
                 }
-                const f32x16 S = mma_feat_init<D>(kf, qs, init);  // register = key, lane = query
+                const f32x16 S = mma_feat_init<D>(kf, qk, init);  // register = key, lane = query
                 const float mn = max16(S, m);
                 z *= __builtin_amdgcn_exp2f(m - mn);
                 m = mn;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) z += __builtin_amdgcn_exp2f(S[r] - m);
             });
+    };
+    sweep1(split3(q), l);
+    const bool exact = split_failed(z);
+    if (exact) {
+        const int l2 = second_walk(l);
+        load_q(q, l2);
+        sweep1(whole(q), l2);
     }
     {   // the two half-waves, then the four wavefronts
         const float mo = __shfl_xor(m, 32, 64), zo = __shfl_xor(z, 32, 64);
@@ -569,7 +633,9 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
 
     // ---- sweep 2: probabilities, map tiles and O^T --------------------------------------------------
     f32x16 o[1] = {splat16(0.f)};  // O^T: register = feature, lane = query
-    {
+    auto sweep2 = [&](const auto& qk, int l) {
+        const int h = l >> 5, li = l & 31;
+        const int klin = lin_voff(l, ild), vlin = lin_voff(l, vld), alin = lin_voff(l, L);
         Pre2 xa, xb;
         tile_pipeline(
             nu, xa, xb,
@@ -577,7 +643,7 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
                 const int J = w + min(i, nu - 1) * WAVES;
                 ldr_tile_lin(rK, klin, J * 32 * ild * 4, ild, x.k);
                 ldr_tile_lin(rV, vlin, J * VSTEP, vld, x.v);
-                penalties(x.pj, J);
+                penalties(x.pj, J, l);
             },
             [&](Pre2& c, int i) {
                 const int J = w + i * WAVES;
@@ -597,7 +663,7 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
 #pragma unroll
                     for (int r = 0; r < 16; ++r) init[r] -= LOG2E * c.pj[r];
                 }
-                const f32x16 S = mma_feat_init<D>(kf, qs, init);  // logits minus the row maximum
+                const f32x16 S = mma_feat_init<D>(kf, qk, init);  // logits minus the row maximum
                 float p[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(S[r]) * rinv;
@@ -615,6 +681,13 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
                     str_tile_lin_cached(rS, alin, (J * 32 * L + I * 32) * 4, L, pl);
                 }
             });
+    };
+    if (exact) {
+        const int l2 = second_walk(l);
+        load_q(q, l2);
+        sweep2(whole(q), l2);
+    } else {
+        sweep2(split3(q), l);
     }
     if constexpr (RM) {
         reduce_store_rows<WAVES>(o[0], Out + ob, I * 32, w, li, h, lds, old_);
@@ -776,12 +849,15 @@ SPION_TILE_KERNEL_D(WAVES, 32) void dense_bwd_row32_kernel(
     const char* Tp = Tv + DmaTileF32::TILE;
     const char* Tk = Tv + 2 * DmaTileF32::TILE;
 
+    auto load_go = [&](float (&go)[KH], int l) {
+        if constexpr (RM) ldr_rows<D>(rdO, ((l & 31) * old_ + (l >> 5) * KH) * 4, I * 32 * old_ * 4, go);
+        else ldr_cols<D>(rdO, L, ((l >> 5) * KH * L + (l & 31)) * 4, I * 128, go);
+    };
     float go[KH], oo[KH];
+    load_go(go, l);
     if constexpr (RM) {
-        ldr_rows<D>(rdO, (li * old_ + h * KH) * 4, I * 32 * old_ * 4, go);
         ldr_rows<D>(make_rsrc(OutCopy + ob, obytes), (li * old_ + h * KH) * 4, I * 32 * old_ * 4, oo);
     } else {
-        ldr_cols<D>(rdO, L, (h * KH * L + li) * 4, I * 128, go);
         ldr_cols<D>(make_rsrc(OutCopy + hb, hbytes), L, (h * KH * L + li) * 4, I * 128, oo);
     }
     float g = 0.f;
@@ -790,15 +866,17 @@ SPION_TILE_KERNEL_D(WAVES, 32) void dense_bwd_row32_kernel(
     g += __shfl_xor(g, 32, 64);
     if (w == 0 && h == 0) G[(size_t)bh * L + I * 32 + li] = -g;
     const f32x16 gneg = splat16(-g);
-    const Split3<KH> gos = split3(go);
 
-    f32x16 acc = splat16(0.f);  // dQ^T: register = feature, lane = query
+    f32x16 acc[1];  // dQ^T: register = feature, lane = query
     // The V, map and K tiles go straight into wave-private LDS; the operands of tile i are read out into registers,
     // then the same space is requested for tile i + 1, whose loads have the two chains of tile i to arrive.
     const unsigned lv = lds_address(Tv), lp = lv + DmaTileF32::TILE, lk = lv + 2 * DmaTileF32::TILE;
     const u32x4 wV = rsrc_words(V + ib, hbytes), wK = rsrc_words(Kt + ib, hbytes);
     const u32x4 wP = rsrc_words(Attn + (size_t)bh * L * L, (size_t)L * L * 4);
     const int kld = RM ? ild : L, KSTEP = RM ? 32 * ild * 4 : 128;
+    auto walk = [&](const auto& gk, int l) {  // gk: the dO operand, split or whole
+    const int h = l >> 5, li = l & 31;
+    acc[0] = splat16(0.f);
     const int vl = DmaTileF32::voff(l, ild), pl = DmaTileF32::voff(l, L), kl = DmaTileF32::voff(l, kld);
     const int vx = DmaTileF32::extra_step(ild), px = DmaTileF32::extra_step(L), kx = DmaTileF32::extra_step(kld);
     const auto a_v = DmaTileF32::own_addr(Tv, li, 4 * h, 1);  // V[key li][feature 16h + s]
@@ -823,15 +901,23 @@ SPION_TILE_KERNEL_D(WAVES, 32) void dense_bwd_row32_kernel(
             wait_lgkm0();
             if (i + 1 < nu) issue(w + (i + 1) * WAVES);
             __builtin_amdgcn_sched_barrier(0);
-            f32x16 dp = mma_feat_init<D>(vt, gos, gneg);  // register = key, lane = query: dO_i . v_j - g_i
+            f32x16 dp = mma_feat_init<D>(vt, gk, gneg);  // register = key, lane = query: dO_i . v_j - g_i
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
-            acc = mma_split(split3(kb), split3(ds), acc);
+            if constexpr (is_whole<std::decay_t<decltype(gk)>>) acc[0] = mma_chain(kb, ds, acc[0]);
+            else acc[0] = mma_split(split3(kb), split3(ds), acc[0]);
         }
     }
+    };
+    walk(split3(go), l);
+    if (split_failed(acc)) {
+        const int l2 = second_walk(l);
+        load_go(go, l2);
+        walk(whole(go), l2);
+    }
     if (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
-    f32x16 out[1] = {acc * scale};
+    f32x16 out[1] = {acc[0] * scale};
     if constexpr (RM) reduce_store_rows<WAVES>(out[0], dQ + gb, I * 32, w, li, h, lds, gld);
     else reduce_store<D, WAVES, true>(out, dQ + hb, I * 32, w, li, h, lds, L);
 }
@@ -860,10 +946,13 @@ SPION_TILE_KERNEL_D(WAVES, 32) void dense_bwd_col32_kernel(
     const char* Tq = To + 2 * DmaTileF32::TILE;
     const char* Tg = To + 3 * DmaTileF32::TILE;
 
+    auto load_v = [&](float (&v)[KH], int l) {
+        ldr_rows<D>(rV, ((l & 31) * ild + (l >> 5) * KH) * 4, J * 32 * ild * 4, v);
+    };
     float v[KH];
-    ldr_rows<D>(rV, (li * ild + h * KH) * 4, J * 32 * ild * 4, v);
+    load_v(v, l);
 
-    f32x16 ak = splat16(0.f), av = splat16(0.f);  // dK^T, dV^T: register = feature, lane = key
+    f32x16 ak[1], av;  // dK^T, dV^T: register = feature, lane = key
     // The dO, map and Q tiles and the 32 values of -g go straight into wave-private LDS; the operands of tile i are
     // read out into registers (the dO tile in both of its roles), then the same space is requested for tile i + 1.
     const unsigned lo = lds_address(To), lp = lo + DmaTileF32::TILE, lq = lo + 2 * DmaTileF32::TILE,
@@ -872,6 +961,10 @@ SPION_TILE_KERNEL_D(WAVES, 32) void dense_bwd_col32_kernel(
     const u32x4 wP = rsrc_words(Attn + (size_t)bh * L * L, (size_t)L * L * 4), wG = rsrc_words(G + (size_t)bh * L, (size_t)L * 4);
     const int qld = RM ? ild : L, QSTEP = RM ? 32 * ild * 4 : 128;
     const int dld = RM ? old_ : L, DSTEP = RM ? 32 * old_ * 4 : 128;
+    auto walk = [&](const auto& vk, int l) {  // vk: the V operand, split or whole
+    const int h = l >> 5, li = l & 31;
+    ak[0] = splat16(0.f);
+    av = splat16(0.f);
     const int dl = DmaTileF32::voff(l, dld), pl = DmaTileF32::voff(l, L), ql = DmaTileF32::voff(l, qld);
     const int dx = DmaTileF32::extra_step(dld), px = DmaTileF32::extra_step(L), qx = DmaTileF32::extra_step(qld);
     const auto a_p = DmaTileF32::own_addr(Tp, li, h, 2);  // P[query acc_row(r, h)][key li]
@@ -894,8 +987,7 @@ SPION_TILE_KERNEL_D(WAVES, 32) void dense_bwd_col32_kernel(
         DmaTileF32::load(wQ, lq, ql, I * QSTEP, qx);
         dma_b32(wG, lg, l * 4, I * 128);
     };
-    const Split3<KH> vs = split3(v);
-    settle(vs);
+    settle(vk);
     if (nu > 0) {
         issue(w);
         for (int i = 0; i < nu; ++i) {
@@ -917,18 +1009,23 @@ SPION_TILE_KERNEL_D(WAVES, 32) void dense_bwd_col32_kernel(
             wait_lgkm0();
             if (i + 1 < nu) issue(w + (i + 1) * WAVES);
             __builtin_amdgcn_sched_barrier(0);
-            f32x16 dp = mma_feat_init<D>(go, vs, init);  // register = query, lane = key
+            f32x16 dp = mma_feat_init<D>(go, vk, init);  // register = query, lane = key
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * p[r];
-#pragma unroll
-            for (int s = 0; s < 16; ++s) ak = __builtin_amdgcn_mfma_f32_32x32x2f32(qb[s], ds[s], ak, 0, 0, 0);
-#pragma unroll
-            for (int s = 0; s < 16; ++s) av = __builtin_amdgcn_mfma_f32_32x32x2f32(ob[s], p[s], av, 0, 0, 0);
+            ak[0] = mma_chain(qb, ds, ak[0]);
+            av = mma_chain(ob, p, av);
         }
     }
+    };
+    walk(split3(v), l);
+    if (split_failed(ak)) {  // (dV comes from fp32 chains in any case)
+        const int l2 = second_walk(l);
+        load_v(v, l2);
+        walk(whole(v), l2);
+    }
     if (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
-    f32x16 out[1] = {ak * scale};
+    f32x16 out[1] = {ak[0] * scale};
     if constexpr (RM) {
         reduce_store_rows<WAVES>(out[0], dK + gb, J * 32, w, li, h, lds, gld);
         __syncthreads();
@@ -964,8 +1061,11 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_row64_kernel(
     head_slice<true, D>(ly.out, ly.H, bh, L, ob, old_, obytes);
     head_slice<true, D>(ly.grad, ly.H, bh, L, gb, gld, gbytes);
 
+    auto load_go = [&](float (&go)[KH], int l) {
+        ldr_rows<D>(make_rsrc(dO + ob, obytes), ((l & 31) * old_ + (l >> 5) * KH) * 4, I * 32 * old_ * 4, go);
+    };
     float go[KH], oo[KH];
-    ldr_rows<D>(make_rsrc(dO + ob, obytes), (li * old_ + h * KH) * 4, I * 32 * old_ * 4, go);
+    load_go(go, l);
     ldr_rows<D>(make_rsrc(Out + ob, obytes), (li * old_ + h * KH) * 4, I * 32 * old_ * 4, oo);
     float g = 0.f;
 #pragma unroll
@@ -973,15 +1073,18 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_row64_kernel(
     g += __shfl_xor(g, 32, 64);
     if (w == 0 && h == 0) G[(size_t)bh * L + I * 32 + li] = -g;
     const f32x16 gneg = splat16(-g);
-    const Split3<KH> gos = split3(go);
 
-    f32x16 acc[2] = {splat16(0.f), splat16(0.f)};  // dQ: register = query, lane = feature
+    f32x16 acc[2];  // dQ: register = query, lane = feature
     const char* Tv = smem + w * WB;
     const char* Tk = Tv + 2 * DmaTileF32::TILE;
     const char* Tp = Tv + 4 * DmaTileF32::TILE;
     const unsigned lv = lds_address(Tv), lk = lv + 2 * DmaTileF32::TILE, lp = lv + 4 * DmaTileF32::TILE;
     const u32x4 wV = rsrc_words(V + ib, hbytes), wK = rsrc_words(K + ib, hbytes);
     const u32x4 wP = rsrc_words(Attn + (size_t)bh * L * L, (size_t)L * L * 4);
+    auto walk = [&](const auto& gk, int l) {  // gk: the dO operand, split or whole
+    const int h = l >> 5, li = l & 31;
+    acc[0] = splat16(0.f);
+    acc[1] = splat16(0.f);
     const int vl = DmaTileF32::voff(l, ild), pl = DmaTileF32::voff(l, L);
     const int vx = DmaTileF32::extra_step(ild), px = DmaTileF32::extra_step(L);
     const auto a_v = DmaTileF32::own8_addr(Tv + h * DmaTileF32::TILE, li);  // V[key li][feature 32h + s]
@@ -1006,12 +1109,19 @@ SPION_TILE_KERNEL(WAVES) void dense_bwd_row64_kernel(
             wait_lgkm0();
             if (i + 1 < nu) issue(w + (i + 1) * WAVES);
             __builtin_amdgcn_sched_barrier(0);
-            f32x16 dp = mma_feat_init<D>(vt, gos, gneg);  // register = key, lane = query: dO_i . v_j - g_i
+            f32x16 dp = mma_feat_init<D>(vt, gk, gneg);  // register = key, lane = query: dO_i . v_j - g_i
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
-            mma_b_split<D>(ds, kb, acc);
+            mma_b_split<D, is_whole<std::decay_t<decltype(gk)>>>(ds, kb, acc);
         }
+    }
+    };
+    walk(split3(go), l);
+    if (split_failed(acc)) {
+        const int l2 = second_walk(l);
+        load_go(go, l2);
+        walk(whole(go), l2);
     }
     if (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
     acc[0] *= scale;

@@ -274,11 +274,13 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
     const float c2 = scale * LOG2E;
     const int lin = lin_voff(l, ild), tile_bytes = 32 * ild * 4;
 
-    float q[KH];
-    ldr_rows<D>(rQ, (li * ild + h * KH) * 4, I * tile_bytes, q);
+    auto load_q = [&](float (&q)[KH], int l) {
+        ldr_rows<D>(rQ, ((l & 31) * ild + (l >> 5) * KH) * 4, I * tile_bytes, q);
 #pragma unroll
-    for (int s = 0; s < KH; ++s) q[s] *= c2;
-    const Split3<KH> qs = split3(q);
+        for (int s = 0; s < KH; ++s) q[s] *= c2;
+    };
+    float q[KH];
+    load_q(q, l);
     const float2 rem = Stats[(size_t)bh * L + I * 32 + li];  // the remainder of row li
 
     // ---- index of this wavefront's tiles (positions past the end repeat the last one: valid, redundant) -----
@@ -295,9 +297,14 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
     }
 
     // ---- logits of the tiles, own maximum; the next tile of K is in flight while one is worked on --------
-    float m = MASK ? 0.f : -100.f * LOG2E, z = 0.f;
+    float m, z;
     f32x16 S[MAXT];
     f32x4 raw[2][4];
+    auto own_softmax = [&](const auto& qk, int l) {  // qk: the query operand, split or whole
+    const int h = l >> 5, li = l & 31;
+    const int lin = lin_voff(l, ild);
+    m = MASK ? 0.f : -100.f * LOG2E;
+    z = 0.f;
     float pj[2][16];
     ldr_tile_lin(rK, lin, Js[0] * tile_bytes, ild, raw[0]);
     if constexpr (MASK) ldr_4x4(rM, 16 * h, Js[0] * 128, pj[0]);
@@ -319,7 +326,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
             lds_put_lin(Tx, l, raw[u & 1]);
             float kf[KH];
             lds_get_feat32(Tx, li, h, kf);
-            S[u] = mma_feat_init<D>(kf, qs, init);  // register = key acc_row(r, h), lane = query li
+            S[u] = mma_feat_init<D>(kf, qk, init);  // register = key acc_row(r, h), lane = query li
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 if (!((bits_l[u] >> acc_row(r, h)) & 1u)) S[u][r] = HYB_ABSENT;
@@ -338,6 +345,13 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
                 z += e;
             }
         }
+    }
+    };
+    own_softmax(split3(q), l);
+    if (split_failed(z)) {
+        const int l2 = second_walk(l);
+        load_q(q, l2);
+        own_softmax(whole(q), l2);
     }
     const float m_own = m;
     z += __shfl_xor(z, 32, 64);
@@ -598,15 +612,21 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_col_kernel(const float* __restrict__ Q
     float* Tq = lds_t[w];
     float* To = Tq + 32 * TS;
     int* X = lds_x[w];
-    const int lin_i = lin_voff(l, ild), lin_o = lin_voff(l, old_);
 
+    auto load_vt = [&](float (&vt)[KH], int l) {
+        ldr_rows<D>(rV, ((l & 31) * ild + (l >> 5) * KH) * 4, J * 32 * ild * 4, vt);
+    };
     float vt[KH];
-    ldr_rows<D>(rV, (li * ild + h * KH) * 4, J * 32 * ild * 4, vt);
-    const Split3<KH> vts = split3(vt);
+    load_vt(vt, l);
 
-    f32x16 ak[1] = {splat16(0.f)}, av[1] = {splat16(0.f)};
+    f32x16 ak[1], av[1];
     const int e0 = ix.t_cp[J], ecnt = ix.t_cp[J + 1] - e0;
     const int n = ecnt > w ? (ecnt - w + WAVES - 1) / WAVES : 0;
+    auto walk = [&](const auto& vk, int l) {  // vk: the V operand, split or whole
+    const int h = l >> 5, li = l & 31;
+    const int lin_i = lin_voff(l, ild), lin_o = lin_voff(l, old_);
+    ak[0] = splat16(0.f);
+    av[0] = splat16(0.f);
     HybPre xa, xb;
     hyb_pipeline(
         n, xa, xb,
@@ -636,13 +656,20 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_col_kernel(const float* __restrict__ Q
             f32x16 init;
 #pragma unroll
             for (int r = 0; r < 16; ++r) init[r] = __builtin_bit_cast(float, gn[r]);
-            const f32x16 dp = mma_feat_init<D>(go, vts, init);  // dO_i . v_j - g_i, i = acc_row(r, h), j = li
+            const f32x16 dp = mma_feat_init<D>(go, vk, init);  // dO_i . v_j - g_i, i = acc_row(r, h), j = li
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * x.p[r];
             mma_b<D>(ds, qb, ak);
             mma_b<D>(x.p, ob, av);
         });
+    };
+    walk(split3(vt), l);
+    if (split_failed(ak)) {  // (dV comes from fp32 chains in any case)
+        const int l2 = second_walk(l);
+        load_vt(vt, l2);
+        walk(whole(vt), l2);
+    }
     if constexpr (WAVES > 1) __syncthreads();
     hyb_reduce_store<WAVES>(ak[0], scale, dK + gb, gld, J * 32, w, li, h, lds);
     if constexpr (WAVES > 1) __syncthreads();

@@ -278,6 +278,10 @@ __device__ __forceinline__ void settle(const Split3<N>& x) {
 #pragma unroll
         for (int t = 0; t < N / 8; ++t) asm volatile("" ::"v"(x.p[k][t]));
 }
+template <int N>
+__device__ __forceinline__ void settle(const Whole<N>& x) {
+    settle(x.x);
+}
 // 64 floats (lane l: 4 bytes at voff) to 256 bytes of LDS
 __device__ __forceinline__ void dma_b32(u32x4 r, unsigned lds, int voff, int soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r),
@@ -411,7 +415,7 @@ struct DmaTileF32 {
 // stays on fp32 chains.
 // Against float64 the outputs and gradients of both are as close as the fp32 chains' or closer (2-norms, 1024 to 4096
 // tokens: 1.0e-7 to 5.8e-7 where those gave 2.2e-7 to 6.1e-7).
-// acc = init + A.B over the head dimension; B is an operand the kernel keeps.
+// acc = init + A.B over the head dimension; B is an operand the kernel keeps, split or whole.
 template <int D>
 __device__ __forceinline__ f32x16 mma_feat_init(const float (&a)[D / 2], const Split3<D / 2>& b, f32x16 init) {
     if constexpr (D == 64) {  // sixteen slots after the other: the parts of all 32 would be 48 registers
@@ -434,7 +438,7 @@ __device__ __forceinline__ f32x16 mma_feat_init(const float (&a)[D / 2], const S
         return mma_split(split3(a), b, init);
     }
 }
-// both on the fp32 pipe
+// fp32 chain
 template <int D>
 __device__ __forceinline__ f32x16 mma_feat_f32(const float (&a)[D / 2], const float (&b)[D / 2], f32x16 init) {
     f32x16 acc = init;
@@ -443,27 +447,35 @@ __device__ __forceinline__ f32x16 mma_feat_f32(const float (&a)[D / 2], const fl
     return acc;
 }
 template <int D>
+__device__ __forceinline__ f32x16 mma_feat_init(const float (&a)[D / 2], const Whole<D / 2>& b, f32x16 init) {
+    return mma_feat_f32<D>(a, b.x, init);
+}
+template <int D>
 __device__ __forceinline__ void mma_b_f32(const float (&w)[16], const float (&x)[D / 32][16], f32x16 (&out)[D / 32]) {
 #pragma unroll
     for (int c = 0; c < D / 32; ++c)
 #pragma unroll
         for (int s = 0; s < 16; ++s) out[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[s], x[c][s], out[c], 0, 0, 0);
 }
-// out[c] += W.X over the 32 rows of a tile, on the bf16 pipe
-template <int D>
+// out[c] += W.X over the 32 rows of a tile, on the bf16 pipe, or (EXACT) by fp32 chains
+template <int D, bool EXACT>
 __device__ __forceinline__ void mma_b_split(const float (&w)[16], const float (&x)[D / 32][16], f32x16 (&out)[D / 32]) {
-    const Split3<16> ws = split3(w);
+    if constexpr (EXACT) {
+        mma_b_f32<D>(w, x, out);
+    } else {
+        const Split3<16> ws = split3(w);
 #pragma unroll
-    for (int c = 0; c < D / 32; ++c) {
-        if (c) __builtin_amdgcn_sched_barrier(0);
-        out[c] = mma_split(ws, split3(x[c]), out[c]);
+        for (int c = 0; c < D / 32; ++c) {
+            if (c) __builtin_amdgcn_sched_barrier(0);
+            out[c] = mma_split(ws, split3(x[c]), out[c]);
+        }
     }
 }
 // the same on the pipe the forward and the row pass use
-template <int D>
+template <int D, bool EXACT = false>
 __device__ __forceinline__ void mma_b(const float (&w)[16], const float (&x)[D / 32][16], f32x16 (&out)[D / 32]) {
     if constexpr (D == 32) mma_b_f32<D>(w, x, out);
-    else mma_b_split<D>(w, x, out);
+    else mma_b_split<D, EXACT>(w, x, out);
 }
 __device__ __forceinline__ f32x16 splat16(float v) {
     return (f32x16){v, v, v, v, v, v, v, v, v, v, v, v, v, v, v, v};
@@ -623,69 +635,47 @@ void tile_fwd_kernel(
     const rsrc_t rP = make_rsrc(P + (size_t)bh * nnz, (size_t)nnz * 4);
     const rsrc_t rM = make_rsrc(MASK ? pen + (size_t)bh * L : pen, MASK ? (size_t)L * 4 : 0);
     const int p_base = sd.w * 4;
-    const int pc_voff = (4 * h * rn + li) * 4;  // col-owner access to a P tile
-    const int col_voff = (h * KH * L + li) * 4;
-    const int b_voff = (4 * h * ild + li) * 4;
-    const int m_voff = 16 * h;
     float* T = lds_t[w];
     // P tile t of this block row: transpose to the col-owner layout and store full rows
-    auto store_p = [&](const float (&p)[16], int t) {
+    auto store_p = [&](const float (&p)[16], int t, int l) {
+        const int h = l >> 5, li = l & 31;
         float pc[16];
         lds_put_rows(T, li, h, p);
         lds_get_cols(T, li, h, pc);
-        str_tile_cols(rP, pc_voff, p_base + t * 128, rn, pc);
+        str_tile_cols(rP, (4 * h * rn + li) * 4, p_base + t * 128, rn, pc);
     };
     const float c2 = scale * LOG2E;
 
+    auto load_q = [&](float (&q)[KH], int l) {
+        ldr_rows<D>(rQ, ((l & 31) * ild + (l >> 5) * KH) * 4, I * 32 * ild * 4, q);
+#pragma unroll
+        for (int s = 0; s < KH; ++s) q[s] *= c2;
+    };
     float q[KH];
-    ldr_rows<D>(rQ, (li * ild + h * KH) * 4, I * 32 * ild * 4, q);
-#pragma unroll
-    for (int s = 0; s < KH; ++s) q[s] *= c2;
-    const Split3<KH> qs = split3(q);
+    load_q(q, l);
     // operand over the head dimension of key tile J (lane = key, features h*D/2 ..)
-    auto load_kf = [&](int J, float (&x)[KH]) {
-        if constexpr (KROW) ldr_rows<D>(rK, (li * ild + h * KH) * 4, J * 32 * ild * 4, x);
-        else ldr_cols<D>(rK, L, col_voff, J * 128, x);
+    auto load_kf = [&](int J, float (&x)[KH], int l) {
+        if constexpr (KROW) ldr_rows<D>(rK, ((l & 31) * ild + (l >> 5) * KH) * 4, J * 32 * ild * 4, x);
+        else ldr_cols<D>(rK, L, ((l >> 5) * KH * L + (l & 31)) * 4, J * 128, x);
     };
 
-    // initial accumulator of a logit chain: minus the key penalties of the tile, in the log2 domain
-    auto chain_init = [&](int J) -> f32x16 {
-        if (!MASK) return splat16(0.f);
-        float pj[16];
-        ldr_4x4(rM, m_voff, J * 128, pj);
-        f32x16 v;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = -LOG2E * pj[r];
-        return v;
-    };
-
-    float m = MASK ? 0.f : -100.f * LOG2E, z = 0.f;
+    constexpr float M0 = MASK ? 0.f : -100.f * LOG2E;
+    float m = M0, z = 0.f;
     f32x16 o[D / 32];
 #pragma unroll
     for (int c = 0; c < D / 32; ++c) o[c] = splat16(0.f);
 
     auto two_sweeps = [&]() {
-        // d = 64: two register sets of a K and a V tile leave no room for split operands; fp32 chains there
-        float qf[D == 64 ? KH : 1];
-        if constexpr (D == 64) {
-            ldr_rows<D>(rQ, (li * ild + h * KH) * 4, I * 32 * ild * 4, qf);
-#pragma unroll
-            for (int s = 0; s < KH; ++s) qf[s] *= c2;
-        }
-        auto logits = [&](const float (&k)[KH], f32x16 init) -> f32x16 {
-            if constexpr (D == 64) return mma_feat_f32<D>(k, qf, init);
-            else return mma_feat_init<D>(k, qs, init);
-        };
         // ---- sweep 1: online row maximum and denominator -------------------------------------------
         const int nu = cnt > w ? (cnt - w + WAVES - 1) / WAVES : 0;  // tiles of this wavefront
         struct PreK {
             float k[KH];
             float pj[16];  // key penalties of the tile (MASK only)
         };
-        auto fetch_k = [&](PreK& x, int i) {
+        auto fetch_k = [&](PreK& x, int i, int l) {
             const int J = tcol[t0 + w + min(i, nu - 1) * WAVES];
-            load_kf(J, x.k);
-            if constexpr (MASK) ldr_4x4(rM, m_voff, J * 128, x.pj);
+            load_kf(J, x.k, l);
+            if constexpr (MASK) ldr_4x4(rM, 16 * (l >> 5), J * 128, x.pj);
         };
         auto init_of = [&](const PreK& x, float shift) -> f32x16 {
             f32x16 v;
@@ -696,10 +686,12 @@ void tile_fwd_kernel(
             }
             return v;
         };
-        {
+        auto sweep1 = [&](const auto& qk, int l) {  // qk: the query operand, split or whole
+            m = M0;
+            z = 0.f;
             PreK ka, kb;
-            tile_pipeline(nu, ka, kb, fetch_k, [&](PreK& c, int) {
-                f32x16 s = logits(c.k, init_of(c, 0.f));
+            tile_pipeline(nu, ka, kb, [&](PreK& x, int i) { fetch_k(x, i, l); }, [&](PreK& c, int) {
+                f32x16 s = mma_feat_init<D>(c.k, qk, init_of(c, 0.f));
                 const float tm = max16(s, m);
                 float zz = 0.f;
 #pragma unroll
@@ -707,31 +699,56 @@ void tile_fwd_kernel(
                 z = z * __builtin_amdgcn_exp2f(m - tm) + zz;
                 m = tm;
             });
+        };
+        // d = 64: two register sets of a K and a V tile leave no room for split operands; fp32 chains there
+        bool exact = D == 64;
+        if constexpr (D == 64) {
+            sweep1(whole(q), l);
+        } else {
+            sweep1(split3(q), l);
+            exact = split_failed(z);
+            if (exact) {
+                const int l2 = second_walk(l);
+                load_q(q, l2);
+                sweep1(whole(q), l2);
+            }
         }
         merge_max_sum<WAVES>(m, z, w, h, li, lds_m, lds_z);
         z += (float)(L - rn) * __builtin_amdgcn_exp2f(-m);
         const float rinv = 1.0f / z;
         // ---- sweep 2: logits again (minus the row maximum, folded into the chain), P, O ------------
-        {
+        auto sweep2 = [&](const auto& qk, int l) {
             struct PreKV {
                 PreK k;
                 float vb[D / 32][16];
             };
+            const int h = l >> 5, li = l & 31;
             PreKV xa, xb;
             tile_pipeline(
                 nu, xa, xb,
                 [&](PreKV& x, int i) {
-                    fetch_k(x.k, i);
-                    ldr_tile_b<D>(rV, b_voff, tcol[t0 + w + min(i, nu - 1) * WAVES] * 32 * ild * 4, x.vb, ild);
+                    fetch_k(x.k, i, l);
+                    ldr_tile_b<D>(rV, (4 * h * ild + li) * 4, tcol[t0 + w + min(i, nu - 1) * WAVES] * 32 * ild * 4, x.vb, ild);
                 },
                 [&](PreKV& c, int i) {
-                    f32x16 s = logits(c.k.k, init_of(c.k, m));
+                    f32x16 s = mma_feat_init<D>(c.k.k, qk, init_of(c.k, m));
                     float p[16];
 #pragma unroll
                     for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(s[r]) * rinv;
-                    store_p(p, w + i * WAVES);
+                    store_p(p, w + i * WAVES, l);
                     mma_b_f32<D>(p, c.vb, o);
                 });
+        };
+        if constexpr (D == 64) {
+            sweep2(whole(q), l);
+        } else {
+            if (exact) {
+                const int l2 = second_walk(l);
+                load_q(q, l2);
+                sweep2(whole(q), l2);
+            } else {
+                sweep2(split3(q), l);
+            }
         }
     };
     constexpr bool FALLBACK = LONG && MAXT > 0;
@@ -753,7 +770,12 @@ void tile_fwd_kernel(
         // a K tile is 32 features x 32 keys with rows L floats apart, or (KROW) 32 keys x 32 features, contiguous
         const int KSTEP = KROW ? 32 * ild * 4 : 128;
         const int kld = KROW ? ild : L;
-        const int plin = lin_voff(l, rn);
+        // The logits of this wavefront's tiles, their exponentials relative to its own maximum (left in S) and the sum of
+        // these over its half of the keys; qk: the query operand, split or whole.
+        auto own_softmax = [&](const auto& qk, int l) {
+        const int h = l >> 5, li = l & 31;
+        m = M0;
+        z = 0.f;
         if constexpr (LIN) {
             const u32x4 wK = rsrc_words(Kt + ib, hbytes);
             const u32x4 wM = rsrc_words(MASK ? pen + (size_t)bh * L : pen, MASK ? (size_t)L * 4 : 0);
@@ -794,7 +816,7 @@ void tile_fwd_kernel(
                     }
                     wait_lgkm0();  // the tile's space is requested again one iteration on
                     __builtin_amdgcn_sched_barrier(0);
-                    S[u] = mma_feat_init<D>(kf, qs, init);
+                    S[u] = mma_feat_init<D>(kf, qk, init);
                     m = max16(S[u], m);
                 }
             }
@@ -838,7 +860,7 @@ void tile_fwd_kernel(
                     wait_lgkm0();
                     if (u + 1 < MAXT && u + 1 < nu) issue_k(u + 1 < MAXT ? u + 1 : u);
                     __builtin_amdgcn_sched_barrier(0);
-                    S[u] = mma_feat_init<D>(kf, qs, init);
+                    S[u] = mma_feat_init<D>(kf, qk, init);
                     m = max16(S[u], m);
                 }
             }
@@ -857,6 +879,13 @@ void tile_fwd_kernel(
                     z += e;
                 }
             }
+        }
+        };
+        own_softmax(split3(q), l);
+        if (split_failed(z)) {
+            const int l2 = second_walk(l);
+            load_q(q, l2);
+            own_softmax(whole(q), l2);
         }
         const float m_own = m;
         z += __shfl_xor(z, 32, 64);
@@ -879,6 +908,7 @@ void tile_fwd_kernel(
         // +inf denominator -> 0 -> P = 0, as in the reference
         const float rinv = __builtin_amdgcn_exp2f(m_own - m) * (1.0f / z);
 
+        const int plin = lin_voff(l, rn);
         if constexpr (LIN) {
             // V tiles the same way: request u + 2 goes out when tile u has been read.  What was issued after the
             // loads of tile u when its turn comes: the loads of tile u + 1 (if any), and the P stores of the one
@@ -943,6 +973,29 @@ void tile_fwd_kernel(
                     str_tile_lin(rP, plin, p_base + t * 128, rn, pl);
                 }
             }
+            if (split_failed(o)) {  // once more, from the probabilities just stored (their registers are long reused)
+                const int l2 = second_walk(l), vl2 = DmaTileF32::voff(l2, ild), plin2 = lin_voff(l2, rn);
+                const auto a_v2 = DmaTileF32::cols_addr(Tb, l2 & 31, l2 >> 5);
+#pragma unroll
+                for (int c = 0; c < D / 32; ++c) o[c] = splat16(0.f);
+                wait_vm<0>();
+#pragma unroll 1
+                for (int t = w; t < cnt; t += WAVES) {
+                    const int J = tcol[t0 + t];
+                    DmaTileF32::load(wV, lb64, vl2, J * 32 * ild * 4, vx);
+                    DmaTileF32::load(wV, lb64 + DmaTileF32::TILE, vl2, J * 32 * ild * 4 + 128, vx);
+                    f32x4 pl[4];
+                    ldr_tile_lin_l2(rP, plin2, p_base + t * 128, rn, pl);
+                    wait_vm<0>();
+                    float p[16], vb[2][16];
+                    lds_put_lin(T, l2, pl);
+                    lds_get_rows(T, l2 & 31, l2 >> 5, p);
+                    DmaTileF32::get(a_v2, vb[0]);
+                    DmaTileF32::get(a_v2, vb[1], DmaTileF32::TILE);
+                    wait_lgkm0();
+                    mma_b_f32<D>(p, vb, o);
+                }
+            }
         }
       }
     } else {
@@ -1001,6 +1054,9 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
     const int col_voff = (h * KH * L + li) * 4;
     const int b_voff = (4 * h * ild + li) * 4;
     const int r_voff = (li * ild + h * KH) * 4, ro_voff = (li * old_ + h * KH) * 4;
+    auto load_go = [&](float (&go)[KH], int l) {
+        ldr_rows<D>(rdO, ((l & 31) * old_ + (l >> 5) * KH) * 4, I * 32 * old_ * 4, go);
+    };
     float* T = reinterpret_cast<float*>(smem + w * WB);
     // P tile as loaded (col owner) -> row-owner layout, the one dP^T comes in
     auto p_rows = [&](const float (&pc)[16], float (&pr)[16]) {
@@ -1009,8 +1065,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
     };
 
     float go[KH];
-    ldr_rows<D>(rdO, ro_voff, I * 32 * old_ * 4, go);
-    const Split3<KH> gos = split3(go);
+    load_go(go, l);
 
     float g = 0.f;
     if (HAVE_O) {
@@ -1019,7 +1074,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
 #pragma unroll
         for (int s = 0; s < KH; ++s) g = fmaf(go[s], oo[s], g);
         g += __shfl_xor(g, 32, 64);
-    } else {
+    } else {  // fp32 chains
         struct PreG {
             float vt[KH];
             float pv[16];
@@ -1036,7 +1091,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
             [&](PreG& c, int) {
                 float pr[16];
                 p_rows(c.pv, pr);
-                f32x16 dp = mma_feat_init<D>(c.vt, gos, splat16(0.f));
+                f32x16 dp = mma_feat_f32<D>(c.vt, go, splat16(0.f));
 #pragma unroll
                 for (int r = 0; r < 16; ++r) g = fmaf(dp[r], pr[r], g);
             });
@@ -1054,6 +1109,9 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
     const f32x16 gneg = splat16(-g);
 
     f32x16 acc[D / 32];
+    auto walk = [&](const auto& gk, int l) {  // gk: the dO operand, split or whole
+    const int h = l >> 5, li = l & 31;
+    constexpr bool EXACT = is_whole<std::decay_t<decltype(gk)>>;
 #pragma unroll
     for (int c = 0; c < D / 32; ++c) acc[c] = splat16(0.f);
     if constexpr (D == 32) {
@@ -1095,11 +1153,11 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
                 if (i + 1 < nu) issue(w + (i + 1) * WAVES, Jn);
                 Jn = Jnn;
                 __builtin_amdgcn_sched_barrier(0);
-                f32x16 dp = mma_feat_init<D>(vt, gos, gneg);  // dp[r] = dO_i . v_j - g_i
+                f32x16 dp = mma_feat_init<D>(vt, gk, gneg);  // dp[r] = dO_i . v_j - g_i
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
-                mma_b<D>(ds, kb, acc);
+                mma_b<D, EXACT>(ds, kb, acc);
             }
         }
     } else {
@@ -1146,13 +1204,20 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
                 if (i + 1 < nu) issue(w + (i + 1) * WAVES, Jn);
                 Jn = Jnn;
                 __builtin_amdgcn_sched_barrier(0);
-                f32x16 dp = mma_feat_init<D>(vt, gos, gneg);  // dp[r] = dO_i . v_j - g_i
+                f32x16 dp = mma_feat_init<D>(vt, gk, gneg);  // dp[r] = dO_i . v_j - g_i
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
-                mma_b<D>(ds, kb, acc);
+                mma_b<D, EXACT>(ds, kb, acc);
             }
         }
+    }
+    };
+    walk(split3(go), l);
+    if (split_failed(acc)) {
+        const int l2 = second_walk(l);
+        load_go(go, l2);
+        walk(whole(go), l2);
     }
     if constexpr (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
 #pragma unroll
@@ -1196,23 +1261,28 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
     const rsrc_t rQ = make_rsrc(Q + ib, hbytes), rV = make_rsrc(Vt + ib, hbytes), rdO = make_rsrc(dO + ob, obytes);
     const rsrc_t rP = make_rsrc(P + (size_t)bh * nnz, (size_t)nnz * 4);
     const rsrc_t rG = make_rsrc(G + (size_t)bh * L, (size_t)L * 4);
-    const int b_voff = (4 * h * ild + li) * 4, bo_voff = (4 * h * old_ + li) * 4;
-    const int r_voff = (li * ild + h * KH) * 4, ro_voff = (li * old_ + h * KH) * 4;
 
+    auto load_vt = [&](float (&vt)[KH], int l) {
+        if constexpr (VROW) ldr_rows<D>(rV, ((l & 31) * ild + (l >> 5) * KH) * 4, J * 32 * ild * 4, vt);
+        else ldr_cols<D>(rV, L, ((l >> 5) * KH * L + (l & 31)) * 4, J * 128, vt);
+    };
     float vt[KH];
-    if constexpr (VROW) ldr_rows<D>(rV, r_voff, J * 32 * ild * 4, vt);
-    else ldr_cols<D>(rV, L, (h * KH * L + li) * 4, J * 128, vt);
+    load_vt(vt, l);
 
     f32x16 ak[D / 32], av[D / 32];
+    // Per tile of the transposed index: {block row I, offset of the tile in this head's P, row stride}.
+    const int4* __restrict__ desc = reinterpret_cast<const int4*>(tcdesc) + e0;
+    const int nu = cnt > w ? (cnt - w + WAVES - 1) / WAVES : 0;  // tiles of this wavefront
+    float* T = reinterpret_cast<float*>(smem + w * WB);
+    auto walk = [&](const auto& vk, int l) {  // vk: the V operand, split or whole
+    const int h = l >> 5, li = l & 31;
+    constexpr bool EXACT = is_whole<std::decay_t<decltype(vk)>>;
+    settle(vk);
 #pragma unroll
     for (int c = 0; c < D / 32; ++c) {
         ak[c] = splat16(0.f);
         av[c] = splat16(0.f);
     }
-    // Per tile of the transposed index: {block row I, offset of the tile in this head's P, row stride}.
-    const int4* __restrict__ desc = reinterpret_cast<const int4*>(tcdesc) + e0;
-    const int nu = cnt > w ? (cnt - w + WAVES - 1) / WAVES : 0;  // tiles of this wavefront
-    float* T = reinterpret_cast<float*>(smem + w * WB);
     if constexpr (D == 32) {
         // The P, Q and dO tiles and the 32 values of -g go straight into wave-private LDS (thirteen instructions, no
         // registers in flight); the operands of tile i are read out of LDS into registers -- the dO tile in both
@@ -1240,8 +1310,6 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
             DmaTileF32::load(wO, lo, ol, I * 32 * old_ * 4, ox);
             dma_b32(wG, lg, l * 4, I * 128);
         };
-        const Split3<KH> vts = split3(vt);
-        settle(vts);
         if (nu > 0) {
             issue(desc[w]);
             int4 dn = desc[w + (nu > 1 ? WAVES : 0)];
@@ -1266,12 +1334,12 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
                 if (i + 1 < nu) issue(dn);
                 dn = dnn;
                 __builtin_amdgcn_sched_barrier(0);
-                f32x16 dp = mma_feat_init<D>(go, vts, init);  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
+                f32x16 dp = mma_feat_init<D>(go, vk, init);  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pc[r];
-                mma_b_split<D>(ds, qb, ak);
-                mma_b_split<D>(pc, ob, av);
+                mma_b_split<D, EXACT>(ds, qb, ak);
+                mma_b_split<D, EXACT>(pc, ob, av);
             }
         }
     } else {
@@ -1301,7 +1369,6 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
             DmaTileF32::load(wO, lo, ol, I * 32 * old_ * 4, ox);
             DmaTileF32::load(wO, lo + DmaTileF32::TILE, ol, I * 32 * old_ * 4 + 128, ox);
         };
-        settle(vt);
         if (nu > 0) {
             int4 dn = desc[w];
             issue(dn);
@@ -1327,13 +1394,24 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
                 dn = dnn;
                 __builtin_amdgcn_sched_barrier(0);
                 const f32x16 init = __builtin_amdgcn_mfma_f32_32x32x2f32(ga, 1.0f, splat16(0.f), 0, 0, 0);  // -g_i in every column
-                f32x16 dp = mma_feat_f32<D>(go, vt, init);  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
+                f32x16 dp = mma_feat_init<D>(go, vk, init);  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pc[r];
-                mma_b_f32<D>(ds, qb, ak);
-                mma_b_f32<D>(pc, ob, av);
+                mma_b_split<D, EXACT>(ds, qb, ak);
+                mma_b_split<D, EXACT>(pc, ob, av);
             }
+        }
+    }
+    };
+    if constexpr (D == 64) {
+        walk(whole(vt), l);
+    } else {
+        walk(split3(vt), l);
+        if (split_failed(ak) || split_failed(av)) {
+            const int l2 = second_walk(l);
+            load_vt(vt, l2);
+            walk(whole(vt), l2);
         }
     }
     if constexpr (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles

@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace spion {
 
 // =================================================================================================
@@ -55,18 +57,23 @@ __device__ __forceinline__ int xcd_remap(int pid, int total) {
 // A float is the exact sum of three bf16 numbers -- hi = bf16(x), mid = bf16(x - hi), lo = x - hi - mid, all rounded
 // to nearest: 8 + 8 + 8 significant bits, the signs of mid and lo taking up what rounding up borrows -- and a product
 // of two bf16 numbers is exact in fp32.  Of the nine partial products of a . b the six with hi.hi, hi.mid, mid.hi,
-// mid.mid, hi.lo and lo.hi are formed; the other three are below 2^-25 of |a||b|, less than the rounding of one fp32
-// product.  Sums are accumulated in fp32 by the MFMA as before.  Measured against float64 on MI355X (32x32x32
-// products of normal, positive, wide-range and one-signed operands, 1 to 128 of them accumulated): relative error
-// 3.8e-8 against 1.0e-7 of the v_mfma_f32_32x32x2_f32 chain for one product, 1.02e-6 against 1.15e-6 for 128; all
-// nine partial products give the same figures as six.
+// mid.mid, hi.lo and lo.hi are formed; of the other three mid.lo and lo.mid reach 2^-25 of |a||b| each, so that all
+// three together are at most 2^-24 (1 + 2^-9) of it, what one rounding of an fp32 product can be.  Sums are accumulated
+// in fp32 by the MFMA as before.  Measured against float64 on MI355X (32x32x32 products of normal, positive, wide-range
+// and one-signed operands, 1 to 128 of them accumulated): relative error 3.8e-8 against 1.0e-7 of the
+// v_mfma_f32_32x32x2_f32 chain for one product, 1.02e-6 against 1.15e-6 for 128; all nine partial products give the same
+// figures as six.
 // Why: v_mfma_f32_32x32x16_bf16 does sixteen times the work of v_mfma_f32_32x32x2_f32 in half its time, so six of
 // them per 16 terms take 384 cycles for a 32x32x32 product instead of 1024; they overlap with vector-ALU work, which
 // the fp32 MFMA does not, so that the splitting (88 instructions per 16 floats and lane) is mostly hidden; and they
 // draw less power: under sustained load the fp32 chain takes 435 to 755 ns per product and SIMD (the clock drops), the
 // six-product chain 217 ns, 280 ns with one operand split on the way.
-// Range: an infinite operand gives NaN; |x| >= 2^128 - 2^119 rounds to an infinite hi (fp32 overflow is 2^128); below 2^-110 the lo part is
-// subnormal or lost, an absolute error under 2^-133.
+// Range: an infinite operand, or a finite one of 2^128 - 2^119 and more, whose hi rounds to infinity, gives parts that are
+// not numbers and so a NaN in every sum it enters; below 2^-110 the lo part is subnormal or lost, an absolute error under
+// 2^-133.  So a wavefront looks once a strip at what came out of its products (split_failed) and, where that is not
+// finite, or all of it so small that its operands may lie down there, walks its tiles again with fp32 chains:
+// infinities, NaN and the ends of the range come out as those give them.  What is left are operands below 2^-110 whose
+// products partners above 2^20 lift above 2^-90; there the absolute error of 2^-133 of the operand remains.
 template <int N>
 struct Split3 {
     bf16x8 p[3][N / 8];  // hi, mid, lo of elements 8t .. 8t+7
@@ -124,6 +131,55 @@ __device__ __forceinline__ f32x16 mma_split(const Split3<N>& a, const Split3<N>&
     }
 #pragma unroll
     for (int t = 0; t < N / 8; ++t) acc = mfma_bf16(a.p[0][t], b.p[0][t], acc);
+    return acc;
+}
+
+// The same operand for fp32 chains.
+template <int N>
+struct Whole {
+    float x[N];
+};
+template <int N>
+__device__ __forceinline__ Whole<N> whole(const float (&x)[N]) {
+    Whole<N> w;
+#pragma unroll
+    for (int s = 0; s < N; ++s) w.x[s] = x[s];
+    return w;
+}
+template <class X>
+constexpr bool is_whole = false;
+template <int N>
+constexpr bool is_whole<Whole<N>> = true;
+
+// Whether sums of split products have to be formed again by fp32 chains (the same answer in every lane): one of them is not
+// finite, or none of the wavefront's reaches 2^-90 although not all are zero.  (Sums whose magnitudes overflow
+// only together cost time and nothing else.)
+__device__ __forceinline__ bool split_failed_sum(float s) {  // s: the sum of a lane's magnitudes
+    const bool finite = s < __builtin_inff();                 // false for NaN
+    return __builtin_expect(__any(!finite) || (!__any(s >= 0x1p-90f) && __any(s != 0.f)), 0);
+}
+template <int N>
+__device__ __forceinline__ bool split_failed(const f32x16 (&acc)[N]) {
+    float s = 0.f;
+#pragma unroll
+    for (int c = 0; c < N; ++c)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s += fabsf(acc[c][r]);
+    return split_failed_sum(s);
+}
+// The same for the exponentials of logits: a NaN among them.  (Logits may be as small as they like.)
+__device__ __forceinline__ bool split_failed(float z) { return __builtin_expect(__any(z != z), 0); }
+// The lane for such a second walk, hidden from the compiler: addresses made from it are not shared with the first walk
+// and so take no registers there.
+__device__ __forceinline__ int second_walk(int l) {
+    asm volatile("" : "+v"(l));
+    return l;
+}
+
+// acc += A.B over the 16 slots of each half-wave, an fp32 chain
+__device__ __forceinline__ f32x16 mma_chain(const float (&a)[16], const float (&b)[16], f32x16 acc) {
+#pragma unroll
+    for (int s = 0; s < 16; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
     return acc;
 }
 
