@@ -139,6 +139,8 @@ struct OperandLds {
 // COLSUM (the sums over many rows): the hi.hi products and the small ones have accumulators of their own -- adding the
 // small ones one by one to a sum that has grown a hundredfold would lose their last bits when they share a sign -- and
 // the work-groups of the first column of tiles also leave sum_r A[r][m] in Csum[z][m].
+// A wavefront whose sums are not finite, or all too small for split operands (Split3, tile_ops.h), forms them again from
+// the operands in memory, one fp32 term after the other: some 30 us at 256 terms, and rare.
 template <bool A_ACROSS, bool B_ACROSS, int WM, int WN, bool COLSUM>
 __global__ __launch_bounds__(256, 2) void project_kernel(SegRows A, SegRows B, SegBias bias, float* __restrict__ C, int ldc,
                                                       float* __restrict__ Csum, int M, int N, int R, int chunks,
@@ -228,6 +230,43 @@ __global__ __launch_bounds__(256, 2) void project_kernel(SegRows A, SegRows B, S
 #pragma unroll
                 for (int k = 0; k < 2; ++k) hi[i][j] = mfma_bf16(a[0][k], b[j][0][k], hi[i][j]);
             }
+        }
+    }
+    float mag = 0.f;
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                mag += fabsf(hi[i][j][q]);
+                if constexpr (COLSUM) mag += fabsf(lo[i][j][q]);
+            }
+    if (split_failed_sum(mag)) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                hi[i][j] = splat16(0.f);
+                if constexpr (COLSUM) lo[i][j] = splat16(0.f);
+            }
+#pragma unroll 1
+        for (int r = r0; r < r0 + nchunks * 32; ++r) {
+            float b[WN];
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                const int n = min(n0 + wn + 32 * j + li, N - 1);
+                b[j] = B_ACROSS ? B.row(r)[n] : B.row(n)[r];
+            }
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    const int m = min(m0 + wm + 32 * i + acc_row(q, h), M - 1);
+                    const float a = A_ACROSS ? A.row(r)[m] : A.row(m)[r];
+#pragma unroll
+                    for (int j = 0; j < WN; ++j) hi[i][j][q] = fmaf(a, b[j], hi[i][j][q]);
+                }
         }
     }
     float* Cz = C + (size_t)z * M * N;

@@ -60,6 +60,56 @@ def test_projection_kernels_match_float64(rows, dim, n, segs):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
+def _kinds(x):
+    return torch.isposinf(x) + 2 * torch.isneginf(x) + 3 * torch.isnan(x)
+
+
+# narrow and wide tiles; many pieces of the weight gradient's sum
+@pytest.mark.parametrize("rows,dim,n", [(96, 64, 32), (16384, 64, 64), (8192, 512, 512)])
+@pytest.mark.parametrize("which", ["x", "w", "dy"])
+def test_infinities_nan_and_the_largest_floats(rows, dim, n, which):
+    """One special element: the same results infinite and NaN as torch's fp32 products give, finite ones to the accuracy that
+    they have without it.  Beside a finite one everything is a sixteenth, so that no product with it overflows."""
+    g = torch.Generator().manual_seed(rows)
+    core, stream = _lib.core(), torch.cuda.current_stream().cuda_stream
+    for value in (float("inf"), -float("inf"), float("nan"), 2.0 ** 128 - 2.0 ** 104, -(2.0 ** 128 - 2.0 ** 119)):
+        t = {k: torch.randn(*s, generator=g).cuda() for k, s in dict(x=(rows, dim), w=(n, dim), dy=(rows, n)).items()}
+        if 1.0 < abs(value) < float("inf"):
+            t = {k: v / 16 for k, v in t.items()}
+        t[which][5, 7] = value
+        x, w, dy, b = t["x"], t["w"], t["dy"], torch.randn(n, device="cuda")
+        y, dx, dw, db = (torch.empty_like(v) for v in (dy, x, w, b))
+        ws = torch.empty(core.spion_project_workspace(rows, n, dim), device="cuda")
+        assert core.spion_project_forward(x.data_ptr(), _ptrs([w]), _ptrs([b]), y.data_ptr(), rows, n, 1, dim, stream) == 0
+        assert core.spion_project_backward_input(dy.data_ptr(), _ptrs([w]), dx.data_ptr(), rows, n, 1, dim, stream) == 0
+        assert core.spion_project_backward_weight(dy.data_ptr(), x.data_ptr(), dw.data_ptr(), db.data_ptr(), ws.data_ptr(), rows,
+                                                  n, dim, stream) == 0
+        for name, got, a, c, extra in (("y", y, x, w.t(), b), ("dx", dx, dy, w, None), ("dw", dw, dy.t(), x, None)):
+            ref = a @ c if extra is None else a @ c + extra
+            assert torch.equal(_kinds(got), _kinds(ref)), (name, value)
+            ok = torch.isfinite(ref)
+            mag = a.abs().double() @ c.abs().double()
+            err = (got.double() - ref.double()).abs()
+            terms = min(a.shape[1], 1024) + 256  # a piece's terms one by one on both sides, and the pieces
+            assert bool((err[ok] <= 2 * terms * 2.0 ** -24 * mag[ok] + 2.0 ** -20).all()), (name, value)
+
+
+def test_products_near_the_smallest_floats():
+    """Operands of 2^-117: their third parts are subnormal or lost, up to 2^-16 of an element."""
+    rows, dim, n = 2048, 64, 64
+    g = torch.Generator().manual_seed(1)
+    core, stream = _lib.core(), torch.cuda.current_stream().cuda_stream
+    x, w = torch.randn(rows, dim, generator=g).cuda(), torch.randn(n, dim, generator=g).cuda()
+    dy = (torch.randn(rows, n, generator=g) * 2.0 ** -117).cuda()
+    dx, dw, db = torch.empty_like(x), torch.empty_like(w), torch.empty(n, device="cuda")
+    ws = torch.empty(core.spion_project_workspace(rows, n, dim), device="cuda")
+    assert core.spion_project_backward_input(dy.data_ptr(), _ptrs([w]), dx.data_ptr(), rows, n, 1, dim, stream) == 0
+    assert core.spion_project_backward_weight(dy.data_ptr(), x.data_ptr(), dw.data_ptr(), db.data_ptr(), ws.data_ptr(), rows, n,
+                                              dim, stream) == 0
+    for got, ref in ((dx, dy.double() @ w.double()), (dw, dy.double().t() @ x.double())):
+        assert float((got.double() - ref).norm() / ref.norm()) < 1e-6  # some tens of roundings of 2^-24
+
+
 def test_rows_past_a_quarter_of_the_int_range():
     """Row indices from 2^29 on are rows of the matrix like any other: the last 64 of 2^29 + 32 rows."""
     rows = 2 ** 29 + 32
