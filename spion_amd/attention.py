@@ -88,10 +88,11 @@ def _core_types():
     return _CORES
 
 
-def _observed(m):
-    """Whether somebody watches or replaced this module's call: hooks of its own, or a forward set on the instance."""
-    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                or "forward" in m.__dict__)
+def _observed(d):
+    """Whether somebody watches or replaced a module's call (d: the module's __dict__): hooks of its own, or a forward set
+    on the instance."""
+    return d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] \
+        or "forward" in d
 
 
 class Attention(nn.Module):
@@ -136,14 +137,13 @@ class Attention(nn.Module):
         torch's usual rule for capturing a backward: warm up on a side stream and keep no autograd graph of a step
         that ran on the default stream alive (its AccumulateGrad nodes belong to the legacy stream, which a capture
         must not touch; breaking this rule ends in a crash inside capture_end on ROCm, not in an error message)."""
-        node = self._compiled_node(X, mask)
+        node, weights = self._compiled_node(X, mask)
         if node is not None and mat is not None:
-            done = self._sparse_layer(node, X, mask, mat)
+            done = self._sparse_layer(node, weights, X, mask, mat)
             if done is not None:
                 return done
         if node is not None:
-            Q, K, V = self._in_node(node.project_heads, X, self.W_q.weight, self.W_k.weight, self.W_v.weight,
-                                    self.W_q.bias, self.W_k.bias, self.W_v.bias, self.num_head, self.head_dim)
+            Q, K, V = self._in_node(node.project_heads, X, *weights[:6], self.num_head, self.head_dim)
         elif self.fused_qkv and X.dtype == torch.float32 and not torch.is_autocast_enabled():
             Q, K, V = _FusedQKV.apply(X, self.W_q.weight, self.W_k.weight, self.W_v.weight, self.W_q.bias,
                                       self.W_k.bias, self.W_v.bias, self.num_head, self.head_dim)
@@ -158,26 +158,32 @@ class Attention(nn.Module):
             else:
                 attn_out, attn = self.block_attn(Q.float(), K.float(), V.float(), mask.float(), mat)
         if node is not None and attn_out.dtype == torch.float32:
-            return self._in_node(node.merge_heads, attn_out, self.ff.weight, self.ff.bias), attn
+            return self._in_node(node.merge_heads, attn_out, *weights[6:]), attn
         attn_out = self.combine_heads(attn_out)
         return self.ff(attn_out), attn
 
     def _compiled_node(self, X, mask):
-        """The compiled node when it covers the projections of this call (csrc/project.hip: fp32 on the GPU, rows and
-        features in multiples of 32, plain linear layers of the layer's sizes, no hooks on them or on all modules, no
-        autocast), else None."""
-        if not (self.fused_qkv and X.is_cuda and isinstance(mask, torch.Tensor) and not torch.is_autocast_enabled()) \
+        """(node, weights) when the compiled node covers the projections of this call (csrc/project.hip: fp32 on the GPU, rows
+        and features in multiples of 32, plain linear layers of the layer's sizes, no hooks on them or on all modules, no
+        autocast), else (None, None).  weights: those of W_q, W_k and W_v, their biases, weight and bias of ff."""
+        if not (self.fused_qkv and X.is_cuda and isinstance(mask, torch.Tensor)) or torch.is_autocast_enabled() \
                 or _nn_module._has_any_global_hook():
-            return None
-        for m in (self.W_q, self.W_k, self.W_v, self.ff):
-            if type(m) is not nn.Linear or m.bias is None or _observed(m):
-                return None
+            return None, None
+        w = []
+        for name in ("W_q", "W_k", "W_v", "ff"):  # (through the modules' dictionaries: their attributes are slow)
+            m = self._modules.get(name)
+            if type(m) is not nn.Linear or _observed(m.__dict__):
+                return None, None
+            p = m._parameters
+            weight, bias = p["weight"] if "weight" in p else m.weight, p["bias"] if "bias" in p else m.bias
+            if weight is None or bias is None:
+                return None, None
+            w += weight, bias
+        weights = (*w[0:6:2], *w[1:6:2], *w[6:])
         node = _lib.autograd_node()
-        if node is None or not node.projections_fit(
-                X, self.W_q.weight, self.W_k.weight, self.W_v.weight, self.W_q.bias, self.W_k.bias, self.W_v.bias,
-                self.ff.weight, self.ff.bias, self.num_head, self.head_dim):
-            return None
-        return node
+        if node is None or not node.projections_fit(X, *weights, self.num_head, self.head_dim):
+            return None, None
+        return node, weights
 
     def _in_node(self, call, *args):
         """A call of the node on X's stream; errors of the library come out as the modules raise them."""
@@ -189,20 +195,19 @@ class Attention(nn.Module):
                 raise _lib.SpionLibraryError(str(e)) from None
             raise
 
-    def _sparse_layer(self, node, X, mask, mat):
+    def _sparse_layer(self, node, weights, X, mask, mat):
         """The whole layer in one call -- projections, core, output projection, and no torch operation in between --
         or None when the core is not one of this package's modules as they are, was built for heads of another shape
         (reconstruct_for_blocksparse takes a config of its own; the module then says so), or has hooks."""
         core = self.block_attn
         if (type(core) not in _core_types() or not core.reads_views
-                or core.head_shape != (X.shape[0], self.num_head, X.shape[1], self.head_dim) or _observed(core)):
+                or core.head_shape != (X.shape[0], self.num_head, X.shape[1], self.head_dim) or _observed(core.__dict__)):
             return None
         idx = core.csr_cache.get(mat, core.block_size)
         key_mask, is_mask = core.key_operand(mask if mask.dtype == torch.float32 else mask.float())
         y, p_flat = self._in_node(
-            node.sparse_layer, X, self.W_q.weight, self.W_k.weight, self.W_v.weight, self.W_q.bias, self.W_k.bias,
-            self.W_v.bias, self.ff.weight, self.ff.bias, key_mask, is_mask, idx.offsets, idx.columns, idx.sum_mat,
-            core.attn_handle, idx.nnz, self.num_head, self.head_dim)
+            node.sparse_layer, X, *weights, key_mask, is_mask, idx.offsets, idx.columns, idx.sum_mat, core.attn_handle,
+            idx.nnz, self.num_head, self.head_dim)
         return y, 0 if core.with_mask else p_flat
 
     def reconstruct_for_blocksparse(self, config):

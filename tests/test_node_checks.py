@@ -52,7 +52,7 @@ def test_layer_with_a_core_of_other_heads_is_not_taken_in_one_call(heads, d):
     layer = Attention(_config(2, 32), inference=True)
     layer.reconstruct_for_blocksparse(_config(heads, d))
     x = torch.zeros(2, 64, 64)
-    assert layer._sparse_layer(_Unused(), x, torch.ones(2, 64), torch.ones(2, 2)) is None
+    assert layer._sparse_layer(_Unused(), (None,) * 8, x, torch.ones(2, 64), torch.ones(2, 2)) is None
 
 
 def _linears(n, dim, out):
