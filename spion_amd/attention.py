@@ -163,9 +163,9 @@ class Attention(nn.Module):
         return self.ff(attn_out), attn
 
     def _compiled_node(self, X, mask):
-        """(node, weights) when the compiled node covers the projections of this call (csrc/project.hip: fp32 on the GPU, rows
-        and features in multiples of 32, plain linear layers of the layer's sizes, no hooks on them or on all modules, no
-        autocast), else (None, None).  weights: those of W_q, W_k and W_v, their biases, weight and bias of ff."""
+        """(node, weights) when the compiled node covers the projections of this call (csrc/project.hip: fp32 on the GPU,
+        rows and features in multiples of 32, plain linear layers of the layer's sizes, no hooks on them or on all modules,
+        no autocast), else (None, None).  weights: those of W_q, W_k and W_v, their biases, weight and bias of ff."""
         if not (self.fused_qkv and X.is_cuda and isinstance(mask, torch.Tensor)) or torch.is_autocast_enabled() \
                 or _nn_module._has_any_global_hook():
             return None, None

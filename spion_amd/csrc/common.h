@@ -53,6 +53,21 @@ inline bool check_launch(const char* what) {
     return true;
 }
 
+// Compute units of the device current at the first call (256 on MI355X, fewer on a partition of it): what rules that fill
+// the machine count with.
+inline int device_cus() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
+            (void)hipGetLastError();
+            n = 256;
+        }
+        return n;
+    }();
+    return cus;
+}
+
 // Named ranges around the phases of a call (the reference brackets its cuSPARSE steps with nvtxRangePush / Pop,
 // models/block_attn.cu:163-223): with SPION_ROCTX=1 in the environment the ROCm tools library is loaded on first use
 // and every PhaseRange pushes / pops a roctx range, so that a marker trace of a training step attributes host time

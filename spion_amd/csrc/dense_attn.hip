@@ -1459,15 +1459,7 @@ static void dense_forward_strided_impl(void* h, const float* Q, const float* K, 
         // C partial maps: the smallest divisor of NB that fills the device -- one eight-wavefront work-group per CU
         // for the register-resident form (measured at B=256, H=2, L=1024: 0.95 ms with 256 work-groups, 1.05 with
         // 512, 1.22 with 1024: fewer, longer work-groups store fewer partial maps), two four-wavefront ones otherwise
-        static int cus = 0;
-        if (!cus) {
-            int dev = 0;
-            if (hipGetDevice(&dev) != hipSuccess ||
-                hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
-                (void)hipGetLastError();
-                cus = 256;
-            }
-        }
+        const int cus = device_cus();
         const long long want = nbr <= 32 ? cus : 2LL * cus;
         int C = a->NB;
         for (int c = 1; c <= a->NB; ++c)

@@ -351,7 +351,7 @@ static bool launch_project(const SegRows& A, const SegRows& B, const SegBias& bi
 // little of their width; else 64 x 64.  Forward at 32768 x 256 -> 768: 93.5 us wide, 129 narrow; at 65536 x 64 -> 192, where
 // a third of the second tile would be empty: 25.6 and 21.2; at 4096 x 512 -> 1536, 384 wide tiles: 57.4 and 56.1.
 static bool wide_tiles(long long M, long long N) {
-    return (M / 128) * (N / 128) >= 512 && (N + 127) / 128 * 128 * 5 <= N * 6;
+    return (M / 128) * (N / 128) >= 2 * device_cus() && (N + 127) / 128 * 128 * 5 <= N * 6;
 }
 
 static bool project_args(const char* who, long long M, int n, int segs, int K, std::initializer_list<const void*> ptrs) {
@@ -403,7 +403,7 @@ int project_backward_input(const float* dY, const float* const* W, float* dX, lo
 // no more than 256 of them (what a piece leaves is written and read back once).
 static int weight_pieces(long long M, int N, int K) {
     const long long tiles = (long long)((N + 63) / 64) * ((K + 63) / 64);
-    long long p = (768 + tiles - 1) / tiles;
+    long long p = (3 * device_cus() + tiles - 1) / tiles;
     p = std::min<long long>(std::min<long long>(p, 256), M / 128);
     return (int)std::max<long long>(p, 1);
 }

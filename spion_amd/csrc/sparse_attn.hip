@@ -662,18 +662,8 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
 // SPION_BF16_LANES (tests; read whenever a pattern is indexed) overrides the number: with a handful of lanes every
 // lane walks many items of several heads even on a small problem.
 static int bf16_lanes() {
-    static int device_lanes = 0;
-    if (!device_lanes) {
-        int dev = 0, cus = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            cus <= 0) {
-            (void)hipGetLastError();
-            cus = 256;
-        }
-        device_lanes = cus * 8;
-    }
     if (const char* env = getenv("SPION_BF16_LANES")) return std::min(std::max(1, atoi(env)), 1 << 16);
-    return device_lanes;
+    return device_cus() * 8;
 }
 
 // Copy the index to the host once (unless the caller hands over host copies), validate it, detect the tile
@@ -1416,12 +1406,12 @@ static void launch_tile_bwd(SparseAttn* a, const float* Q, const float* K, const
 }
 
 // The remainder's kernels with their gathered operands in LDS take one work-group of sixteen wavefronts per CU.  How full
-// a launch over work-groups of `per` rows or columns of a head keeps the machine: the rows over those its rounds of 256
-// work-groups could take.
+// a launch over work-groups of `per` rows or columns of a head keeps the machine: the rows over those its rounds of one
+// work-group per CU could take.
 static int hyb_groups(int L, int per) { return (L + per - 1) / per; }
 static double hyb_filling(const SparseAttn* a, int per) {
-    const long long rounds = ((long long)a->NB * hyb_groups(a->L, per) + 255) / 256;
-    return (double)a->NB * a->L / (256.0 * per * rounds);
+    const long long cus = device_cus(), rounds = ((long long)a->NB * hyb_groups(a->L, per) + cus - 1) / cus;
+    return (double)a->NB * a->L / ((double)cus * per * rounds);
 }
 static bool hyb_lds_off(const SparseAttn* a) {
     static const bool gather = getenv("SPION_HYB_GATHER") != nullptr;
