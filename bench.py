@@ -37,6 +37,47 @@ PEAK_HBM_GBS = 8000.0
 PEAK_BF16_MFMA_TFLOPS = 2500.0
 
 
+def _matrix_ceiling(split, chains, algorithmic=2):
+    """What the matrix pipes allow a kernel, in algorithmic TFLOP/s: per 32 x 32 x 32 product twelve bf16 MFMAs (384 cycles of a
+    SIMD) where its operands are split into bf16 parts, sixteen fp32 MFMAs (1024 cycles, the rate PEAK_FP32_MFMA_TFLOPS
+    stands for) where they are not.  ``algorithmic``: the products the FLOPs count (a column pass forms dP again)."""
+    return PEAK_FP32_MFMA_TFLOPS * algorithmic * 1024.0 / (384.0 * split + 1024.0 * chains)
+
+
+# (split, fp32) products per tile of forward, row pass and column pass (spion_amd/csrc/tile_kernels.h, mma_feat_init, says why);
+# the forward in its register-resident form
+_TILE_PRODUCTS = {32: ((1, 1), (1, 1), (3, 0)), 64: ((2, 0), (2, 0), (0, 3))}
+_DENSE_PRODUCTS = {32: ((1, 1), (2, 0), (1, 2)), 64: ((2, 0), (2, 0), (0, 3))}
+
+
+def _floors_ms(flops, ceiling, nbytes):
+    """Shortest times the matrix pipes (at ``ceiling`` TFLOP/s) and HBM allow a kernel."""
+    return {"mfma": flops / ceiling / 1e9, "hbm": nbytes / PEAK_HBM_GBS / 1e6}
+
+
+def _roof_of(kernel, ms, flops, ceiling, nbytes):
+    """Roofline of one kernel against the longer of its floors."""
+    floors = _floors_ms(flops, ceiling, nbytes)
+    bound = max(floors, key=floors.get)
+    work, peak, unit = (flops / ms / 1e9, ceiling, "TFLOP/s") if bound == "mfma" else (nbytes / ms / 1e6, PEAK_HBM_GBS, "GB/s")
+    return dict(bound=bound, kernel=kernel, achieved=work, peak=peak, unit=unit, traffic=None)
+
+
+def _hybrid_lds_kernels(L, NB):
+    """Which of the remainder's kernels take their operands from LDS (the library's rule: how full the work-groups, one per CU
+    and round, leave the machine): logits, P.V, column pass."""
+    if L < 1024 or "SPION_HYB_GATHER" in os.environ:
+        return False, False, False
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+
+    def filling(per):
+        rounds = -(-NB * -(-L // per) // cus)
+        return NB * L / (cus * per * rounds)
+
+    return (filling(512) >= 0.78, filling(1024) >= 0.95,
+            max(filling(128 * n) * n / (n + 0.25) for n in (8, 4, 2)) > 0.6)
+
+
 def _event_ms(fn, iters, warm=3):
     """Average duration of fn() in ms from HIP events on the current (= the library's) stream."""
     for _ in range(warm):
@@ -490,11 +531,13 @@ def bench_dense_phase(args, dev, d=32):
     alg_flops = 12.0 * L * L * d * NB
     k_fwd = "dense_fwd_reg_kernel" if d == 32 else "dense_fwd_reg64_kernel"
     k_bwd = f"dense_bwd_row{d}_kernel + dense_bwd_col{d}_kernel"
-    roof = dict(bound="mfma", kernel=k_fwd, achieved=alg_flops / 3.0 / t_fwd_rm / 1e9,
-                peak=PEAK_FP32_MFMA_TFLOPS, unit="TFLOP/s", traffic=None)
+    ceil_fwd, ceil_row, ceil_col = (_matrix_ceiling(*p) for p in _DENSE_PRODUCTS[d])
+    map_bytes, third = 4.0 * NB * L * L, alg_flops / 3.0  # each kernel writes or reads the map once
+    roof = _roof_of(k_fwd, t_fwd_rm, third, ceil_fwd, map_bytes + 16.0 * NB * L * d)
     roof["frac"] = roof["achieved"] / roof["peak"]
     roof["kernel_ms"] = {k_fwd: round(t_fwd_rm, 4), k_bwd: round(t_bwd_rm, 4)}
-    roof["backward_frac"] = alg_flops * 2.0 / 3.0 / t_bwd_rm / 1e9 / PEAK_FP32_MFMA_TFLOPS
+    roof["backward_frac"] = (max(_floors_ms(third, ceil_row, map_bytes + 20.0 * NB * L * d).values())
+                             + max(_floors_ms(third, ceil_col, map_bytes + 20.0 * NB * L * d).values())) / t_bwd_rm
     if t_fwd_mean is not None:
         roof["forward_with_mean_ms"] = round(t_fwd_mean, 4)  # spion_dense_forward_strided_mean: maps + their mean
     # the feature-major ABI: the same kernels at d = 32, the two-sweep kernels with operand-layout loads at d = 64
@@ -756,21 +799,24 @@ def bench_sparse_layer(args, dev, workload, full=True):
     alg_flops = workloads.sparse_flops(nnz, d, NB)
     alg_bytes = workloads.sparse_bytes(nnz, L, d, NB)
     third = alg_flops / 3.0  # forward, row pass and column pass carry 4*n*d*NB each
+    lds = ["_lds" if x else "" for x in _hybrid_lds_kernels(L, NB)]
     names = {1: ("tile_fwd_kernel", "tile_bwd_row_kernel", "tile_bwd_col_kernel"),
              2: ("elem_fwd_kernel", "elem_bwd_row_kernel", "elem_bwd_col_kernel"),
              # hybrid: dense window tiles on the MFMA units + gathered remainder; each phase is two or three launches
-             3: ("hyb_rem_logits_lds_kernel + hyb_tile_fwd_kernel + hyb_rem_pv_lds_kernel"
-                 if L % 1024 == 0 and NB * (L // 1024) >= 256 and "SPION_HYB_GATHER" not in os.environ
-                 else "hyb_rem_logits_kernel + hyb_tile_fwd_kernel + hyb_rem_pv_kernel",
+             3: (f"hyb_rem_logits{lds[0]}_kernel + hyb_tile_fwd_kernel + hyb_rem_pv{lds[1]}_kernel",
                  "hyb_tile_bwd_row_kernel + hyb_rem_bwd_row_kernel",
-                 "hyb_tile_bwd_col_kernel + " + ("hyb_rem_bwd_col_lds_kernel" if L % 1024 == 0 and NB * (L // 256) >= 256
-                                                  and "SPION_HYB_GATHER" not in os.environ else "hyb_rem_bwd_col_kernel"))}[path]
+                 f"hyb_tile_bwd_col_kernel + hyb_rem_bwd_col{lds[2]}_kernel")}[path]
     kernels = dict(zip(names, (t_fwd, t_row, t_col)))
     dom = max(kernels, key=kernels.get)
     dom_ms = kernels[dom]
+    floors = {}
     if path == 1:
-        roof = dict(bound="mfma", kernel=dom, achieved=third / dom_ms / 1e9, peak=PEAK_FP32_MFMA_TFLOPS,
-                    unit="TFLOP/s", traffic=None)
+        # the matrix pipes a kernel's products run on against the bytes it cannot do without: P once, and Q, K, V, O / K, V,
+        # dO, O, dQ / Q, V, dO, dK, dV
+        ceiling = {k_: _matrix_ceiling(*p) for k_, p in zip(names, _TILE_PRODUCTS[d])}
+        nbytes = {k_: 4.0 * (t_ * L * d + nnz) * NB for k_, t_ in zip(names, (4, 5, 5))}
+        floors = {k_: _floors_ms(third, ceiling[k_], nbytes[k_]) for k_ in names}
+        roof = _roof_of(dom, dom_ms, third, ceiling[dom], nbytes[dom])
     else:
         # element path: HBM-bound by design; the slowest kernel's share of the algorithmic bytes
         share = {names[0]: 4.0 * (4 * L * d + nnz) * NB, names[1]: 4.0 * (4 * L * d + nnz) * NB,
@@ -791,12 +837,8 @@ def bench_sparse_layer(args, dev, workload, full=True):
             "what": "bytes of gathered operand rows per kernel over its time; for scale, 256 CUs x 64 B per clock "
                     "at 2.4 GHz of vector L1 bandwidth would be 39 TB/s"}
     if path == 1:
-        # MFMA work a tile costs each kernel against its algorithmic share: the column pass recomputes dP (1.5x);
-        # the forward is taken in its register-resident form (1x; its two-sweep form for very long rows is 1.5x)
-        executed = {"tile_fwd_kernel": 1.0, "tile_bwd_row_kernel": 1.0, "tile_bwd_col_kernel": 1.5}
-        roof["frac_per_kernel"] = {k_: round(third / v_ / 1e9 / PEAK_FP32_MFMA_TFLOPS, 4) for k_, v_ in kernels.items()}
-        roof["frac_on_executed_mfma"] = {k_: round(executed[k_] * third / v_ / 1e9 / PEAK_FP32_MFMA_TFLOPS, 4)
-                                         for k_, v_ in kernels.items()}
+        roof["floor_ms_per_kernel"] = {k_: {b: round(t_, 4) for b, t_ in v_.items()} for k_, v_ in floors.items()}
+        roof["frac_per_kernel"] = {k_: round(max(floors[k_].values()) / v_, 4) for k_, v_ in kernels.items()}
 
     result = {
         "metric": "sparse-attn fwd+bwd effective TFLOP/s (12*n*d*NB algorithmic FLOPs / step time), 1 GPU",
@@ -825,10 +867,9 @@ def bench_sparse_layer(args, dev, workload, full=True):
                    "fwd_plus_bwd": round(t_fwd_abi + t_bwd_abi, 4), "fwd_then_bwd_sequence": round(t_seq_abi, 4),
                    "what": "the reference's ABI: transposed K / V operands, kept copies of Out"},
         "kernels_effective_tflops": alg_flops / (t_fwd + t_bwd) / 1e9,
-        "kernels_fraction_of_fp32_mfma_peak": alg_flops / (t_fwd + t_bwd) / 1e9 / PEAK_FP32_MFMA_TFLOPS,
+        "kernels_fraction_of_floor": sum(max(v_.values()) for v_ in floors.values()) / (t_fwd + t_bwd) if floors else None,
         "kernels_effective_hbm_gbs": alg_bytes / (t_fwd + t_bwd) / 1e6,
         "abi_effective_tflops": alg_flops / (t_fwd_abi + t_bwd_abi) / 1e9,
-        "abi_fraction_of_fp32_mfma_peak": alg_flops / (t_fwd_abi + t_bwd_abi) / 1e9 / PEAK_FP32_MFMA_TFLOPS,
         "algorithmic": {"gflop": alg_flops / 1e9, "mbytes": alg_bytes / 1e6},
         "roofline": roof,
     }
