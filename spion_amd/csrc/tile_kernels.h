@@ -403,10 +403,10 @@ struct DmaTileF32 {
 //     d = 64 (one of the two serves two products) and in the column pass at d = 32 (two of its three products; three
 //     wavefronts per SIMD hide the splitting), on the fp32 pipe in the forward and the row pass at d = 32;
 //   * the column pass at d = 64 uses fp32 chains alone: split operands for its five products spill registers, and whole
-//     steps are 1 % slower to 4 % faster without (split / fp32 chains in us, same box, four boxes: 64 x 2 heads of 1024,
+//     steps are 1 % slower to 4 % faster without (split / fp32 chains in us, on four machines: 64 x 2 heads of 1024,
 //     14 % kept, 194 to 202 / 187 to 194; 16 x 4 of 2048, 10 %, 262 to 274 / 255 to 265; 3 x 8 of 4000, 8 %, 278 to 291 / 274
 //     to 291).
-// Measured in us per launch in a training loop, all kernels on fp32 chains / as now, same box.  32 x 2 heads of 4096 tokens,
+// Measured in us per launch in a training loop, all kernels on fp32 chains / as now.  32 x 2 heads of 4096 tokens,
 // d = 32, 32 x 32 blocks, a tenth kept: forward 162 / 155, row pass 141 / 134, column pass 184 / 161; 256 x 2 heads of 1024:
 // 139 / 139, 122 / 121, 148 / 132; 2 x 2 of 8192, a fifth kept (two sweeps): 104 / 97, 76 / 71, 98 / 91; 3 x 8 heads of 4000,
 // d = 64: 98 / 76, 99 / 80.  The dense kernels (dense_attn.hip), 64 x 2 heads of 1024, d = 32: forward 180 / 177, row pass 177
