@@ -8,7 +8,7 @@
 // L/32 tiles of the other dimension; see tile_ops.h for the register layout, tile_kernels.h (mma_feat_init) for which
 // products run on the fp32 and which, with split operands, on the bf16 matrix pipe.
 #include "common.h"
-#include "tile_kernels.h"
+#include "dense_group_kernels.h"
 #include "../../include/spion_hip.h"
 
 #include <cmath>
@@ -1542,6 +1542,19 @@ void dense_forward_strided_mean(void* h, const float* Q, const float* K, const f
     dense_forward_strided_impl(h, Q, K, V, Mask, Attn, Out, Mean, heads, in, out, "dense attn_forward_strided_mean");
 }
 
+// Whether the backward of row-major heads runs as work-groups that share their tiles (dense_group_kernels.h).  A step of such
+// a work-group is long and cannot be divided, so it depends on how full they leave the machine: the share of wavefront places
+// with a strip of their own, counting one work-group to a CU and whole rounds.  us of both passes, four wavefronts to a strip /
+// groups.  d = 32: 20 heads of 1024 (0.62) 74 / 75, 26 (0.81) 89 / 78, 34 (0.53) 113 / 118, 40 of 1056 (0.64) 134 / 125, 18 of 1984
+// (0.54) 201 / 210, 32 of 1024 (1.0) 104 / 87.  d = 64: 20 heads of 1024 (0.31) 152 / 167, 28 (0.44) 173 / 169, 32 (0.50) 195 / 174,
+// 40 (0.63) 242 / 187, 128 of 544 (0.53) 267 / 241, 6 of 2048 (0.19) 155 / 311.
+static bool dense_groups_fill(const DenseAttn* a) {
+    const int nbr = a->L / 32, G = a->d / 8;
+    const long long cus = device_cus(), groups = (long long)((nbr + G - 1) / G) * a->NB;
+    const double filling = (double)nbr * a->NB / ((groups + cus - 1) / cus * cus * G);
+    return filling >= (a->d == 32 ? 0.64 : 0.44);
+}
+
 void dense_backward_strided(void* h, const float* Q, const float* K, const float* V, const float* P, const float* Out,
                             const float* dO, float* dQ, float* dK, float* dV, int heads, const HeadLayout& in,
                             const HeadLayout& out, const HeadLayout& grad) {
@@ -1570,7 +1583,20 @@ void dense_backward_strided(void* h, const float* Q, const float* K, const float
     ly.H = heads;
     const int nbr = a->L / 32;
     const dim3 grid(nbr * a->NB), block4(64 * 4);
-    if (a->d == 64) {
+    if (dense_groups_fill(a)) {
+        const int G = a->d / 8;
+        const dim3 groups((nbr + G - 1) / G * a->NB), block(64 * G);
+#define SPION_LAUNCH(DD)                                                                                             \
+    do {                                                                                                             \
+        hipLaunchKernelGGL(dense_group_row_kernel<DD>, groups, block, 0, a->hdr.stream, K, V, P, dO, Out, a->ws_rowsum, dQ, \
+                           a->L, nbr, a->NB, a->scale, ly);                                                          \
+        hipLaunchKernelGGL(dense_group_col_kernel<DD>, groups, block, 0, a->hdr.stream, Q, V, P, dO, a->ws_rowsum, dK, dV, \
+                           a->L, nbr, a->NB, a->scale, ly);                                                          \
+    } while (0)
+        if (a->d == 64) SPION_LAUNCH(64);
+        else SPION_LAUNCH(32);
+#undef SPION_LAUNCH
+    } else if (a->d == 64) {
         hipLaunchKernelGGL(dense_bwd_row64_kernel<4>, grid, block4, 0, a->hdr.stream, K, V, P, dO, Out, a->ws_rowsum,
                            dQ, a->L, nbr, a->NB, a->scale, ly);
         hipLaunchKernelGGL(dense_bwd_col64_kernel<4>, grid, block4, 0, a->hdr.stream, Q, V, P, dO, a->ws_rowsum, dK, dV,
