@@ -68,12 +68,25 @@ __global__ __launch_bounds__(POOL_THREADS) void conv_pool_kernel(ScoreMaps maps,
 // The weights are subtracted, which is exact; the difference of the two sums would be rounding noise wherever a
 // column's own sum is many orders above its neighbour's, as on maps that decay steeply away from the diagonal.
 // A batch of loads is issued before any of them is used, with the row clamped instead of a remainder loop whose loads
-// would each wait alone.  Four maps of 2048 x 2048, block 32: 52.7 -> 25.6 us (25.1 with the sums subtracted).
-constexpr int CP_COLS = 256, CP_RG = 2, CP_BATCH = 16;
+// would each wait alone, and the next batch before one is used.
+// The weights were half of the inner loop's instructions, so for the block sizes in use they come from a table, two LDS
+// reads and four fp64 instructions an element; a thread per column instead of two halves what a work-group spends on its
+// table and reduction, once there are enough work-groups (2048: 8 per CU) for the machine not to run dry.  us, weights
+// formed / table, block 32: four maps of 2048^2 25.4 / 22.0, six of 4096^2 121 / 95 (two threads a column 106), two of 2048^2
+// 14.6 / 13.7, one of 1024^2 6.2 / 6.1 (one thread 7.8); block 64: 21.5 / 20.5, 96.6 / 92.2 (fp64 table: 24).
+// Left: without any load 18, without any sum 20 of the 22 us, i.e. latency of waves that live for 31 to 62 rows.  Several
+// block rows per work-group, the next one's loads in flight during a reduction, need 94 registers and are slower (30.5).
+constexpr int CP_COLS = 256, CP_BATCH = 16;
+// BS: 32 or 64 (filters of up to 33 taps), the own sum's weights in a table (fp64 for 32; for 64 that would leave room for two
+// work-groups to a CU, so fp32, converted); 0, any block size, formed per element.  CP_RG: threads to a column, each every CP_RG-th row.
+template <int BS, int CP_RG>
 __global__ __launch_bounds__(CP_COLS* CP_RG) void conv_pool_cols_kernel(ScoreMaps maps, float* __restrict__ pooled, int L,
-                                                                         int bs, int nb, int hk, int gb) {
+                                                                         int bs_, int nb, int hk, int gb) {
     __shared__ double part[CP_RG][2][CP_COLS];
-    __shared__ float full[CP_COLS];  // full trapezoid of row dp at [dp + hk]
+    typedef typename std::conditional<BS == 32, double, float>::type weight_t;
+    __shared__ weight_t full[BS ? 2 * BS : CP_COLS];  // full trapezoid of row dp at [dp + hk]
+    __shared__ weight_t table[BS ? (BS + 32) * BS : 1];  // own weight of (row dp, column c of a block) at [(dp + hk) * BS + c]
+    const int bs = BS ? BS : bs_;
     // consecutive items -- the groups of a block row, then the next block row of the same map, whose rows overlap --
     // run on one die, whose L2 then serves the bs + 2 hk rows' overlap
     const int groups = (nb + gb - 1) / gb;
@@ -86,46 +99,58 @@ __global__ __launch_bounds__(CP_COLS* CP_RG) void conv_pool_cols_kernel(ScoreMap
     const int ncols = gb * bs + 2 * hk;
     const int q = Jg * bs - hk + cc;
     const int p0 = max(0, I * bs - hk), p1 = min(L, I * bs + bs + hk);
+    const bool works = cc < ncols && q >= 0 && q < L;
+    const float* col = Am + (works ? q : 0);
+    const auto request = [&](int pb, float (&v)[CP_BATCH]) {
+#pragma unroll
+        for (int k = 0; k < CP_BATCH; ++k) v[k] = col[(size_t)min(pb + k * CP_RG, p1 - 1) * L];
+    };
+    float v[CP_BATCH];
+    request(p0 + rg, v);
     const auto trapezoid = [&](float dp, float lo1, float n, float top) {
         return fmaxf(0.f, fminf(fminf(dp + lo1, n), top - dp));
+    };
+    const auto own_weight = [&](float dp, int c) {
+        const int lo = max(-hk, c - bs + 1), hi = min(hk, c);
+        return trapezoid(dp, (float)(1 - lo), (float)min(hi - lo + 1, bs), (float)(hi + bs));
     };
     if ((int)threadIdx.x < bs + 2 * hk)
         full[threadIdx.x] = trapezoid((float)((int)threadIdx.x - hk), (float)(1 + hk), (float)min(2 * hk + 1, bs),
                                       (float)(hk + bs));
+    if constexpr (BS > 0)
+        for (int e = threadIdx.x; e < (BS + 2 * hk) * BS; e += CP_COLS * CP_RG)
+            table[e] = (weight_t)own_weight((float)(e / BS - hk), e % BS);
     __syncthreads();
     double a0 = 0.0, a1 = 0.0;
-    if (cc < ncols && q >= 0 && q < L) {
-        const int c = q % bs;
-        const int lo = max(-hk, c - bs + 1), hi = min(hk, c);
-        const float lo1 = (float)(1 - lo), n = (float)min(hi - lo + 1, bs), top = (float)(hi + bs);
-        const float* col = Am + q;
-        for (int pb = p0 + rg; pb < p1; pb += CP_RG * CP_BATCH) {
-            float v[CP_BATCH];
+    const int c = (works ? q : 0) % bs;
+    for (int pb = p0 + rg; pb < p1; pb += CP_RG * CP_BATCH) {
+        float next[CP_BATCH];
+        if (pb + CP_RG * CP_BATCH < p1) request(pb + CP_RG * CP_BATCH, next);
 #pragma unroll
-            for (int k = 0; k < CP_BATCH; ++k) v[k] = col[(size_t)min(pb + k * CP_RG, p1 - 1) * L];
-#pragma unroll
-            for (int k = 0; k < CP_BATCH; ++k) {
-                const int p = pb + k * CP_RG;
-                if (p < p1) {
-                    const int dp = p - I * bs;
-                    const double x = (double)v[k];
-                    const float own = trapezoid((float)dp, lo1, n, top);
-                    a0 += x * (double)own;
-                    a1 += x * (double)(full[dp + hk] - own);
-                }
+        for (int k = 0; k < CP_BATCH; ++k) {
+            const int p = pb + k * CP_RG;
+            if (p < p1) {
+                const int dp = p - I * bs;
+                const double x = (double)v[k];
+                const weight_t own = BS ? table[(dp + hk) * BS + c] : (weight_t)own_weight((float)dp, c);
+                a0 += x * (double)own;
+                a1 += x * (double)(full[dp + hk] - own);
             }
         }
+#pragma unroll
+        for (int k = 0; k < CP_BATCH; ++k) v[k] = next[k];
     }
+    if (!works) a0 = a1 = 0.0;
     part[rg][0][cc] = a0;
     part[rg][1][cc] = a1;
     __syncthreads();
-    // wavefront b adds up block b: entries e = 0 .. CP_RG (bs + 2 hk) - 1, lane-strided, then a butterfly
-    const int b = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (b < gb && Jg + b < nb) {
+    // a wavefront adds up a block: entries e = 0 .. CP_RG (bs + 2 hk) - 1, lane-strided, then a butterfly
+    const int lane = threadIdx.x & 63;
+    for (int b = threadIdx.x >> 6; b < gb && Jg + b < nb; b += CP_COLS * CP_RG / 64) {
         const int base = hk + b * bs, span = bs + 2 * hk;
         double s = 0.0;
         for (int e = lane; e < CP_RG * span; e += 64) {
-            const int r = e / span, k = e - r * span - hk;  // column base + k, k = -hk .. bs + hk - 1
+            const int r = e >= span, k = e - r * span - hk;  // column base + k, k = -hk .. bs + hk - 1
             s += part[r][(k < 0 || k >= bs) ? 1 : 0][base + k];
         }
         for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
@@ -737,16 +762,22 @@ int pattern_generate_maps(const float* const* Score, int n_maps, int L, int bs, 
     }
     const int hk = ksize / 2;
     // blocks per work-group of the streaming kernel (0: block size too small for it, or too wide)
-    const int gb = bs >= 2 * hk && bs + 2 * hk <= CP_COLS ? std::min((CP_COLS - 2 * hk) / bs, CP_COLS * CP_RG / 64) : 0;
+    const int gb = bs >= 2 * hk && bs + 2 * hk <= CP_COLS ? (CP_COLS - 2 * hk) / bs : 0;
     for (int m0 = 0; m0 < n_maps; m0 += MAPS_PER_LAUNCH) {
         const int n = std::min(MAPS_PER_LAUNCH, n_maps - m0);
         ScoreMaps maps{};
         for (int m = 0; m < n; ++m) maps.p[m] = Score[m0 + m];
         float* out = pooled + (size_t)m0 * nb * nb;
-        if (gb > 0)
-            hipLaunchKernelGGL(conv_pool_cols_kernel, dim3((nb + gb - 1) / gb * nb * n), dim3(CP_COLS * CP_RG), 0, stream,
-                               maps, out, L, bs, nb, hk, gb);
-        else
+        if (gb > 0) {
+#define SPION_LAUNCH(BS, RG)                                                                                         \
+    hipLaunchKernelGGL((conv_pool_cols_kernel<BS, RG>), dim3(groups), dim3(CP_COLS * RG), 0, stream, maps, out, L, bs, nb, hk, gb)
+            const int groups = (nb + gb - 1) / gb * nb * n;
+            if (bs == 32 && hk <= 16 && groups >= 8 * device_cus()) SPION_LAUNCH(32, 1);
+            else if (bs == 32 && hk <= 16) SPION_LAUNCH(32, 2);
+            else if (bs == 64 && hk <= 16) SPION_LAUNCH(64, 2);
+            else SPION_LAUNCH(0, 2);
+#undef SPION_LAUNCH
+        } else
             hipLaunchKernelGGL(conv_pool_kernel, dim3(nb, nb, n), dim3(POOL_THREADS), 0, stream, maps, out, L, bs, nb,
                                hk);
     }

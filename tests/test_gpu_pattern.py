@@ -84,6 +84,24 @@ def test_steep_local_maps(L, bs, decay):
             assert np.array_equal(mat[n].cpu().numpy().astype(np.int8), ref), (q, n)
 
 
+# block sizes whose weights come from a table (filters of up to 33 taps) and are formed per element, one thread and two to a
+# column (from 2048 work-groups on), no filter, the widest for the block size, block rows cut by the map's edge
+@pytest.mark.parametrize("L,bs,ksize,n", [(256, 32, 33, 2), (256, 32, 0, 2), (256, 32, 3, 2), (256, 64, 33, 2), (256, 64, 35, 2),
+                                          (512, 64, 65, 1), (64, 64, 31, 1), (32, 32, 31, 1), (1024, 32, 31, 13)])
+def test_filter_weights_of_every_kind(L, bs, ksize, n):
+    """As above: every pooled value to one rounding of its own size."""
+    g = torch.Generator().manual_seed(L + bs + ksize)
+    i = torch.arange(L)
+    maps = torch.softmax(-0.7 * (i[:, None] - i[None, :]).abs().float() + torch.randn(n, L, L, generator=g), -1)
+    _, pooled, _ = discover_block_masks(maps.cuda(), bs, mode="conv_ff" if ksize else "ff", threshold=0.9, ksize=ksize or 31,
+                                        return_aux=True)
+    for m in range(n):
+        a = maps[m].numpy()
+        C = op.block_pool_closed_form(op.conv_diag_closed_form(a, ksize) if ksize else a.astype(np.float64), bs)
+        err = np.abs(pooled[m].cpu().numpy().astype(np.float64) - C) / C
+        assert err[C >= 2.0 ** -126].max() <= 1.01 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("levels", [0, 1, 4])
 @pytest.mark.parametrize("nb", [1, 2, 3, 64, 127, 128, 129, 192, 193])
 def test_walk_and_quantile_on_block_grids_of_every_size(nb, levels):
