@@ -396,6 +396,10 @@ int spion_transpose_last2(const float* in, float* out, int batch, int rows, int 
  * Each returns 0 on success. */
 int spion_project_forward(const float* X, const float* const* W, const float* const* b, float* Y, long long rows, int n,
                           int segs, int dim, void* stream);
+/* The same, and in the same launch what spion_key_penalty makes of a key mask. */
+int spion_project_forward_keys(const float* X, const float* const* W, const float* const* b, float* Y, long long rows, int n,
+                               int segs, int dim, const float* mask, float* penalty, int batch, int heads, int seq_len,
+                               void* stream);
 int spion_project_backward_input(const float* dY, const float* const* W, float* dX, long long rows, int n, int segs,
                                  int dim, void* stream);
 long long spion_project_workspace(long long rows, int outputs, int dim);

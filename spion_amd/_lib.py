@@ -129,6 +129,9 @@ def core() -> ctypes.CDLL:
     lib.spion_pattern_generate_maps.restype = c_int
     lib.spion_project_forward.argtypes = [_P] * 4 + [ctypes.c_longlong, c_int, c_int, c_int, _P]
     lib.spion_project_forward.restype = c_int
+    lib.spion_project_forward_keys.argtypes = ([_P] * 4 + [ctypes.c_longlong, c_int, c_int, c_int] + [_P] * 2 +
+                                               [c_int, c_int, c_int, _P])
+    lib.spion_project_forward_keys.restype = c_int
     lib.spion_project_backward_input.argtypes = [_P] * 3 + [ctypes.c_longlong, c_int, c_int, c_int, _P]
     lib.spion_project_backward_input.restype = c_int
     lib.spion_project_workspace.argtypes = [ctypes.c_longlong, c_int, c_int]

@@ -254,9 +254,15 @@ Tensor project_weight_grads(const float* dy, const Tensor& x, int64_t rows, int6
     return dw;
 }
 
+// A [B, L] key mask whose penalties the launch of the input projections is to make as well (null: none).
+struct KeyMask {
+    const float* mask = nullptr;
+    float* pen = nullptr;
+    int batch = 0, heads = 0, length = 0;
+};
 // X [B, L, dim] -> the [B, H, L, d] heads of the three projections, slices of one [B, L, 3, H, d] buffer.
 std::vector<Tensor> qkv_forward(const Tensor& x, const Tensor (&w)[3], const Tensor (&b)[3], int64_t H, int64_t d,
-                                int64_t stream) {
+                                int64_t stream, const KeyMask* keys = nullptr) {
     TORCH_CHECK_VALUE(x.dim() == 3, "projection: input [B, L, features] expected");
     const int64_t B = x.size(0), L = x.size(1), dim = x.size(2);
     for (int i = 0; i < 3; ++i) check_projection(x, w[i], b[i], H * d, dim);
@@ -264,7 +270,11 @@ std::vector<Tensor> qkv_forward(const Tensor& x, const Tensor (&w)[3], const Ten
     Tensor buf = torch::empty({B, L, 3, H, d}, x.options());
     const float* wp[3] = {fp(w[0]), fp(w[1]), fp(w[2])};
     const float* bp[3] = {fp(b[0]), fp(b[1]), fp(b[2])};
-    spion_project_forward(fp(x), wp, bp, fpm(buf), B * L, (int)(H * d), 3, (int)dim, reinterpret_cast<void*>(stream));
+    if (keys && keys->mask)
+        spion_project_forward_keys(fp(x), wp, bp, fpm(buf), B * L, (int)(H * d), 3, (int)dim, keys->mask, keys->pen, keys->batch,
+                                   keys->heads, keys->length, reinterpret_cast<void*>(stream));
+    else
+        spion_project_forward(fp(x), wp, bp, fpm(buf), B * L, (int)(H * d), 3, (int)dim, reinterpret_cast<void*>(stream));
     check_library("projection");
     std::vector<Tensor> out;
     for (int i = 0; i < 3; ++i)  // the slice [:, :, i].transpose(1, 2)
@@ -276,12 +286,12 @@ std::vector<Tensor> qkv_forward(const Tensor& x, const Tensor (&w)[3], const Ten
 // (create_graph): the kernels would leave no graph, and second-order terms would be lost without a word.
 struct QkvNode : public torch::autograd::Function<QkvNode> {
     static variable_list forward(AutogradContext* ctx, Tensor x, Tensor wq, Tensor wk, Tensor wv, Tensor bq, Tensor bk,
-                                 Tensor bv, int64_t H, int64_t d, int64_t stream) {
+                                 Tensor bv, int64_t H, int64_t d, int64_t stream, const KeyMask* keys) {
         const Tensor w[3] = {aligned(wq), aligned(wk), aligned(wv)}, b[3] = {aligned(bq), aligned(bk), aligned(bv)};
         ctx->save_for_backward({x, wq, wk, wv});
         ctx->saved_data["H"] = H;
         ctx->saved_data["stream"] = stream;
-        return qkv_forward(aligned(x), w, b, H, d, stream);
+        return qkv_forward(aligned(x), w, b, H, d, stream, keys);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
@@ -294,7 +304,7 @@ struct QkvNode : public torch::autograd::Function<QkvNode> {
             const Tensor dy = torch::stack({g[0].transpose(1, 2), g[1].transpose(1, 2), g[2].transpose(1, 2)}, 2)
                                   .reshape({rows, 3 * n});
             const Tensor dw = dy.t().matmul(saved[0].reshape({rows, dim})), db = dy.sum(0);
-            variable_list r(10);
+            variable_list r(11);
             r[0] = dy.matmul(torch::cat({saved[1], saved[2], saved[3]}, 0)).view({B, L, dim});
             for (int i = 0; i < 3; ++i) {
                 r[1 + i] = dw.narrow(0, i * n, n);
@@ -309,7 +319,7 @@ struct QkvNode : public torch::autograd::Function<QkvNode> {
             keep = torch::stack({g[0].transpose(1, 2), g[1].transpose(1, 2), g[2].transpose(1, 2)}, 2).contiguous();
             dy = fp(keep);
         }
-        variable_list r(10);
+        variable_list r(11);
         if (ctx->needs_input_grad(0)) {
             r[0] = torch::empty_like(x);
             const Tensor w[3] = {aligned(saved[1]), aligned(saved[2]), aligned(saved[3])};
@@ -384,16 +394,25 @@ std::vector<Tensor> sparse_layer(const Tensor& x, const Tensor& wq, const Tensor
                                  const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t num_heads, int64_t head_dim,
                                  int64_t stream) {
     const c10::DeviceGuard on(x.device());  // `stream` is one of x's device, which need not be the current one
-    const auto pen = penalty_of(mask_or_pen, is_mask, num_heads, stream);
+    // the penalties of a plain key mask come out of the projections' launch
+    KeyMask keys;
+    c10::optional<Tensor> pen;
+    if (is_mask && mask_or_pen.has_value() && !has_tangent(*mask_or_pen)) {
+        const Tensor& mask = *mask_or_pen;
+        pen = torch::empty({mask.size(0), num_heads * mask.size(1)}, mask.options());
+        keys = {fp(mask), fpm(*pen), (int)mask.size(0), (int)num_heads, (int)mask.size(1)};
+    } else {
+        pen = penalty_of(mask_or_pen, is_mask, num_heads, stream);
+    }
     const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
     if (without_node({&x, &wq, &wk, &wv, &bq, &bk, &bv, &wf, &bf, &pen_or_none})) {
         const Tensor w[3] = {aligned(wq), aligned(wk), aligned(wv)}, b[3] = {aligned(bq), aligned(bk), aligned(bv)};
-        const auto qkv = qkv_forward(aligned(x), w, b, num_heads, head_dim, stream);
+        const auto qkv = qkv_forward(aligned(x), w, b, num_heads, head_dim, stream, &keys);
         const CoreResult r = core_forward(qkv[0], qkv[1], qkv[2], pen_or_none, offsets, columns, sum_mat, handle,
                                           nnz, num_heads, true, stream);
         return {merge_forward(aligned(r.out.transpose(1, 2)), aligned(wf), aligned(bf), stream), r.p_flat};
     }
-    const auto qkv = QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream);
+    const auto qkv = QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream, (const KeyMask*)&keys);
     const auto core = SparseAttnNode::apply(qkv[0], qkv[1], qkv[2], pen, offsets, columns, sum_mat, handle, nnz, num_heads,
                                             true, stream);
     return {MergeNode::apply(core[0], wf, bf, stream), core[1]};
@@ -403,7 +422,7 @@ std::vector<Tensor> sparse_layer(const Tensor& x, const Tensor& wq, const Tensor
 std::vector<Tensor> project_heads(const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& bq,
                                   const Tensor& bk, const Tensor& bv, int64_t num_heads, int64_t head_dim, int64_t stream) {
     const c10::DeviceGuard on(x.device());
-    return QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream);
+    return QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream, (const KeyMask*)nullptr);
 }
 Tensor merge_heads(const Tensor& heads, const Tensor& w, const Tensor& b, int64_t stream) {
     const c10::DeviceGuard on(heads.device());

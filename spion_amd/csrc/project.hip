@@ -141,16 +141,40 @@ struct OperandLds {
 // the work-groups of the first column of tiles also leave sum_r A[r][m] in Csum[z][m].
 // A wavefront whose sums are not finite, or all too small for split operands (Split3, tile_ops.h), forms them again from
 // the operands in memory, one fp32 term after the other: some 30 us at 256 terms, and rare.
+// Forward: work-groups past the last item turn a key mask into penalties, which an attention layer needs right after its
+// projections and which take 2.5 us as a launch of their own, whatever their number (KeyMask::total 0: none).
+struct KeyMask {
+    const float* mask;
+    float* pen;
+    long long L, total;
+    int H, groups;
+};
+// [B][L] key mask (1 valid, 0 padded) -> [B*H][L] additive penalties 1e6 (1 - mask), one copy per head
+// (models/attention_blockcuda_mask.py:42-43): the elements of work-group g of `groups`.
+__device__ __forceinline__ void key_penalties(const KeyMask& k, int g) {
+    for (long long i = (long long)g * 256 + threadIdx.x; i < k.total; i += (long long)k.groups * 256) {
+        const long long bh = i / k.L;
+        k.pen[i] = 1e6f * (1.0f - k.mask[bh / k.H * k.L + (i - bh * k.L)]);
+    }
+}
 template <bool A_ACROSS, bool B_ACROSS, int WM, int WN, bool COLSUM>
 __global__ __launch_bounds__(256, 2) void project_kernel(SegRows A, SegRows B, SegBias bias, float* __restrict__ C, int ldc,
                                                       float* __restrict__ Csum, int M, int N, int R, int chunks,
-                                                      int mtiles, int ntiles) {
+                                                      int mtiles, int ntiles, KeyMask keys) {
+    int items = gridDim.x;
+    if constexpr (!A_ACROSS && !B_ACROSS) {
+        items -= keys.groups;
+        if ((int)blockIdx.x >= items) {
+            key_penalties(keys, blockIdx.x - items);
+            return;
+        }
+    }
     typedef OperandLds<A_ACROSS, WM> LA;
     typedef OperandLds<B_ACROSS, WN> LB;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int t = threadIdx.x, w = t >> 6, l = t & 63, h = l >> 5, li = l & 31;
     // consecutive items share the rows of A (the larger operand) and run on one die
-    const int item = xcd_remap(blockIdx.x, gridDim.x);
+    const int item = xcd_remap(blockIdx.x, items);
     const int nt = item % ntiles, mt = item / ntiles % mtiles, z = item / ntiles / mtiles;
     const int m0 = mt * 64 * WM, n0 = nt * 64 * WN;
     const int r0 = z * chunks * 32, nchunks = min(chunks, R / 32 - z * chunks);
@@ -334,7 +358,7 @@ __global__ __launch_bounds__(256) void project_reduce_kernel(const float* __rest
 
 template <bool AA, bool BA, int WM, int WN, bool CS>
 static bool launch_project(const SegRows& A, const SegRows& B, const SegBias& bias, float* C, int ldc, float* Csum, int M,
-                           int N, int R, int pieces, int chunks, hipStream_t stream) {
+                           int N, int R, int pieces, int chunks, hipStream_t stream, const KeyMask& keys = KeyMask{}) {
     constexpr int lds = OperandLds<AA, WM>::BYTES + OperandLds<BA, WN>::BYTES;
     if (lds > 64 * 1024) {  // beyond what a launch may ask for without saying so first
         static const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(project_kernel<AA, BA, WM, WN, CS>),
@@ -342,8 +366,8 @@ static bool launch_project(const SegRows& A, const SegRows& B, const SegBias& bi
         if (!SPION_HIP_OK(err)) return false;
     }
     const int mt = (M + 64 * WM - 1) / (64 * WM), nt = (N + 64 * WN - 1) / (64 * WN);
-    hipLaunchKernelGGL((project_kernel<AA, BA, WM, WN, CS>), dim3((unsigned)mt * nt * pieces), dim3(256), lds, stream, A, B,
-                       bias, C, ldc, Csum, M, N, R, chunks, mt, nt);
+    hipLaunchKernelGGL((project_kernel<AA, BA, WM, WN, CS>), dim3((unsigned)mt * nt * pieces + keys.groups), dim3(256), lds,
+                       stream, A, B, bias, C, ldc, Csum, M, N, R, chunks, mt, nt, keys);
     return check_launch("project_kernel");
 }
 
@@ -367,8 +391,24 @@ static SegRows weight_rows(const float* const* W, int segs, int n, int K) {
     return SegRows{{W[0], W[segs > 1 ? 1 : 0], W[segs > 2 ? 2 : 0]}, segs > 1 ? n : ONE_PIECE, K};
 }
 
+static bool key_mask(const char* who, const float* mask, float* pen, int B, int H, int L, KeyMask& keys) {
+    if (!mask || !pen || B <= 0 || H <= 0 || L <= 0) {
+        set_error("%s: bad arguments", who);
+        return false;
+    }
+    keys.mask = mask;
+    keys.pen = pen;
+    keys.L = L;
+    keys.total = (long long)B * H * L;
+    keys.H = H;
+    keys.groups = (int)std::min<long long>((keys.total + 255) / 256, 2048);
+    return true;
+}
+
 int project_forward(const float* X, const float* const* W, const float* const* b, float* Y, long long M, int n, int segs,
-                    int K, hipStream_t stream) {
+                    int K, const float* mask, float* pen, int B, int H, int L, hipStream_t stream) {
+    KeyMask keys{};
+    if (mask && !key_mask("spion_project_forward_keys", mask, pen, B, H, L, keys)) return 1;
     if (!W || !b || !project_args("spion_project_forward", M, n, segs, K, {X, Y})) {
         if (!W || !b) set_error("spion_project_forward: null weights");
         return 1;
@@ -378,8 +418,8 @@ int project_forward(const float* X, const float* const* W, const float* const* b
     const SegBias bias{{b[0], b[segs > 1 ? 1 : 0], b[segs > 2 ? 2 : 0]}, segs > 1 ? n : ONE_PIECE};
     const int N = segs * n;
     const bool ok = wide_tiles(M, N)
-        ? launch_project<false, false, 2, 2, false>(plain_rows(X, K), weight_rows(W, segs, n, K), bias, Y, N, nullptr, (int)M, N, K, 1, K / 32, stream)
-        : launch_project<false, false, 1, 1, false>(plain_rows(X, K), weight_rows(W, segs, n, K), bias, Y, N, nullptr, (int)M, N, K, 1, K / 32, stream);
+        ? launch_project<false, false, 2, 2, false>(plain_rows(X, K), weight_rows(W, segs, n, K), bias, Y, N, nullptr, (int)M, N, K, 1, K / 32, stream, keys)
+        : launch_project<false, false, 1, 1, false>(plain_rows(X, K), weight_rows(W, segs, n, K), bias, Y, N, nullptr, (int)M, N, K, 1, K / 32, stream, keys);
     return ok ? 0 : 1;
 }
 
@@ -426,23 +466,11 @@ int project_backward_weight(const float* dY, const float* X, float* dW, float* d
     return check_launch("project_reduce_kernel") ? 0 : 1;
 }
 
-// [B][L] key mask (1 valid, 0 padded) -> [B*H][L] additive penalties 1e6 (1 - mask), one copy per head
-// (models/attention_blockcuda_mask.py:42-43).
-__global__ __launch_bounds__(256) void key_penalty_kernel(const float* __restrict__ mask, float* __restrict__ pen, int H,
-                                                          long long L, long long total) {
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {
-        const long long bh = i / L;
-        pen[i] = 1e6f * (1.0f - mask[bh / H * L + (i - bh * L)]);
-    }
-}
+__global__ __launch_bounds__(256) void key_penalty_kernel(KeyMask keys) { key_penalties(keys, blockIdx.x); }
 int key_penalty(const float* mask, float* pen, int B, int H, int L, hipStream_t stream) {
-    if (!mask || !pen || B <= 0 || H <= 0 || L <= 0) {
-        set_error("spion_key_penalty: bad arguments");
-        return 1;
-    }
-    const long long total = (long long)B * H * L;
-    const int blocks = (int)std::min<long long>((total + 255) / 256, 2048);
-    hipLaunchKernelGGL(key_penalty_kernel, dim3(blocks), dim3(256), 0, stream, mask, pen, H, (long long)L, total);
+    KeyMask keys;
+    if (!key_mask("spion_key_penalty", mask, pen, B, H, L, keys)) return 1;
+    hipLaunchKernelGGL(key_penalty_kernel, dim3(keys.groups), dim3(256), 0, stream, keys);
     return check_launch("key_penalty_kernel") ? 0 : 1;
 }
 

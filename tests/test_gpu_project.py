@@ -289,3 +289,28 @@ def test_layer_runs_on_its_inputs_device():
         here = layer(*args)[0]
         here.sum().backward()
     assert here.device == there.device and torch.equal(here, there)
+
+
+# narrow and wide tiles; fewer and more penalties than a work-group's 256 threads, several rounds of the most work-groups
+@pytest.mark.parametrize("rows,dim,B,H,L", [(32, 32, 1, 1, 32), (96, 64, 3, 2, 32), (4096, 64, 2, 8, 2048), (32768, 256, 16, 4, 2048),
+                                            (65536, 32, 64, 16, 1024)])
+def test_penalties_made_beside_the_projections(rows, dim, B, H, L):
+    """Both outputs bit for bit as from launches of their own."""
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, dim, generator=g, device="cuda")
+    w = [torch.randn(64, dim, generator=g, device="cuda") for _ in range(3)]
+    b = [torch.randn(64, generator=g, device="cuda") for _ in range(3)]
+    mask = torch.rand(B, L, generator=g, device="cuda").round()
+    mask[0, 0] = 0.25
+    core, stream = _lib.core(), torch.cuda.current_stream().cuda_stream
+    y, y2 = (torch.full((rows, 192), float("nan"), device="cuda") for _ in range(2))
+    pen, pen2 = (torch.full((B * H, L), float("nan"), device="cuda") for _ in range(2))
+    assert core.spion_project_forward(x.data_ptr(), _ptrs(w), _ptrs(b), y.data_ptr(), rows, 64, 3, dim, stream) == 0
+    assert core.spion_key_penalty(mask.data_ptr(), pen.data_ptr(), B, H, L, stream) == 0
+    assert core.spion_project_forward_keys(x.data_ptr(), _ptrs(w), _ptrs(b), y2.data_ptr(), rows, 64, 3, dim, mask.data_ptr(),
+                                           pen2.data_ptr(), B, H, L, stream) == 0
+    assert torch.equal(y, y2) and torch.equal(pen, pen2)
+    assert core.spion_project_forward_keys(x.data_ptr(), _ptrs(w), _ptrs(b), y2.data_ptr(), rows, 64, 3, dim, None, None, B, H, L,
+                                           stream) != 0
+    with pytest.raises(_lib.SpionLibraryError, match="null mask"):
+        _lib.check_error("projection")
