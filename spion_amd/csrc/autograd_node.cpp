@@ -1,4 +1,4 @@
-// Autograd node of the sparse attention modules, compiled against libtorch (host code only).
+// Autograd nodes of the attention modules, compiled against libtorch (host code only).
 //
 // It does what _BlockAttnFunction in attention_blockcuda.py does -- the reference's function is
 // models/attention_blockcuda.py:20-112 (key-mask variant: models/attention_blockcuda_mask.py) -- with the node, the
@@ -28,13 +28,14 @@ void check_library(const char* where) {
     throw std::runtime_error(std::string(where) + ": " + text);
 }
 
-// Layout of a [B, H, L, d] fp32 view for the strided entry points; false when they cannot take it (last dimension
-// not unit-stride, strides not multiples of 16 bytes, storage not 16-byte aligned).
+// Layout of a [B, H, L, d] view for the strided entry points; false when they cannot take it (last dimension not
+// unit-stride, strides not multiples of 16 bytes, storage not 16-byte aligned).
 bool head_layout(const Tensor& t, spion_head_layout& lay) {
     if (t.dim() != 4) return false;
     const int64_t sb = t.stride(0), sh = t.stride(1), sl = t.stride(2), sf = t.stride(3);
     if (sf != 1 || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16) return false;
-    if (sb % 4 || sh % 4 || sl % 4 || sl < t.size(3) || sb < 0 || sh < 0) return false;
+    const int64_t unit = 16 / t.element_size();
+    if (sb % unit || sh % unit || sl % unit || sl < t.size(3) || sb < 0 || sh < 0) return false;
     if (t.size(2) * sl >= (int64_t(1) << 29)) return false;
     lay.batch_stride = sb;
     lay.head_stride = (int)sh;
@@ -212,6 +213,172 @@ c10::optional<Tensor> penalty_of(const c10::optional<Tensor>& mask_or_pen, bool 
     if (has_tangent(*mask_or_pen)) return (1e6 * (1.0 - mask_or_pen->repeat({1, heads}))).contiguous();
     return key_penalty(*mask_or_pen, heads, stream);
 }
+
+// The gradient of a core's output in that output's strides, as the strided entry points take it.
+Tensor grad_like(const Tensor& go, const Tensor& out) {
+    spion_head_layout lay{};
+    if (go.scalar_type() == out.scalar_type() && same_strides(go, out) && head_layout(go, lay)) return go;
+    return torch::empty_like(out).copy_(go);
+}
+
+// ---- the dense phase: what _DenseAttnFunction in attention_cuda.py does through the strided entry points ----------
+struct DenseResult {
+    Tensor q, k, v, attn, out, mean;  // attn: memory [key][query]
+};
+DenseResult dense_forward(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& pen, int64_t handle,
+                          bool emit_mean, int64_t stream) {
+    void* h = reinterpret_cast<void*>(handle);
+    spion_set_stream(h, reinterpret_cast<void*>(stream));
+    const auto opt = query.options();
+    const int64_t B = query.size(0), H = query.size(1), L = query.size(2);
+    DenseResult r;
+    spion_head_layout lin{}, lk{}, lv{}, lout{};
+    const bool views = head_layout(query, lin) && head_layout(key, lk) && head_layout(value, lv) && same_strides(key, query) &&
+                       same_strides(value, query);
+    r.q = views ? query : query.contiguous();
+    r.k = views ? key : key.contiguous();
+    r.v = views ? value : value.contiguous();
+    head_layout(r.q, lin);
+    r.attn = torch::empty({B, H, L, L}, opt);
+    r.out = empty_heads(query.sizes(), r.q.stride(1) < r.q.stride(2), opt);
+    head_layout(r.out, lout);
+    if (emit_mean) {
+        r.mean = torch::empty({L, L}, opt);
+        spion_dense_forward_strided_mean(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.attn), fpm(r.out), fpm(r.mean), (int)H,
+                                         &lin, &lout);
+    } else {
+        spion_dense_forward_strided(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.attn), fpm(r.out), (int)H, &lin, &lout);
+    }
+    check_library("attn_forward");
+    return r;
+}
+struct DenseAttnNode : public torch::autograd::Function<DenseAttnNode> {
+    static variable_list forward(AutogradContext* ctx, Tensor query, Tensor key, Tensor value, c10::optional<Tensor> pen,
+                                 int64_t handle, bool emit_mean, int64_t stream) {
+        DenseResult r = dense_forward(query, key, value, pen.has_value() ? *pen : Tensor(), handle, emit_mean, stream);
+        ctx->saved_data["handle"] = handle;
+        ctx->saved_data["stream"] = stream;
+        ctx->save_for_backward({r.q, r.k, r.v, r.attn, r.out});
+        ctx->set_materialize_grads(false);  // the gradient of the returned map is ignored (as in the reference)
+        if (!emit_mean) return {r.out, r.attn.transpose(2, 3)};
+        ctx->mark_non_differentiable({r.mean});
+        return {r.out, r.attn.transpose(2, 3), r.mean};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &attn = saved[3], &out = saved[4];
+        void* h = reinterpret_cast<void*>(ctx->saved_data["handle"].toInt());
+        spion_set_stream(h, reinterpret_cast<void*>(ctx->saved_data["stream"].toInt()));
+        const auto opt = q.options();
+        const Tensor go = grads[0].defined() ? grad_like(grads[0], out) : torch::zeros_like(out);
+        Tensor dq, dk, dv;
+        if (adjacent_head_views(q, k, v)) {  // slices of one fused projection: the gradients likewise
+            Tensor buf = torch::empty({q.size(0), q.size(2), 3, q.size(1), q.size(3)}, opt);
+            dq = buf.select(2, 0).transpose(1, 2);
+            dk = buf.select(2, 1).transpose(1, 2);
+            dv = buf.select(2, 2).transpose(1, 2);
+        } else {
+            const bool inter = q.stride(1) < q.stride(2);
+            dq = empty_heads(q.sizes(), inter, opt);
+            dk = empty_heads(q.sizes(), inter, opt);
+            dv = empty_heads(q.sizes(), inter, opt);
+        }
+        spion_head_layout lin{}, lout{}, lgrad{};
+        head_layout(q, lin);
+        head_layout(out, lout);
+        head_layout(dq, lgrad);
+        spion_dense_backward_strided(h, fp(q), fp(k), fp(v), fp(attn), fp(out), fp(go), fpm(dq), fpm(dk), fpm(dv), (int)q.size(1),
+                                     &lin, &lout, &lgrad);
+        check_library("attn_backward");
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// ---- bf16: what _BlockBF16Function in attention_blockbf16.py does -----------------------------------------------
+struct BF16Result {
+    Tensor q, k, v, out, lse;
+    bool strided = false;
+};
+const void* vp(const Tensor& t) { return t.data_ptr(); }
+BF16Result bf16_forward(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& pen, const Tensor& offsets,
+                        const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t stream) {
+    void* h = reinterpret_cast<void*>(handle);
+    spion_set_stream(h, reinterpret_cast<void*>(stream));
+    const auto opt = query.options().dtype(torch::kBFloat16);
+    const int64_t B = query.size(0), H = query.size(1), L = query.size(2);
+    BF16Result r;
+    r.lse = torch::empty({B * H, L}, query.options().dtype(torch::kFloat32));
+    // bf16 heads that are views of projections are read in place and the output is interleaved the same way; anything
+    // else is converted and made contiguous first
+    spion_head_layout lin{}, lk{}, lv{}, lout{};
+    bool all = true;
+    for (const Tensor* t : {&query, &key, &value}) all = all && t->scalar_type() == torch::kBFloat16;
+    r.strided = all && !(query.is_contiguous() && key.is_contiguous() && value.is_contiguous()) && head_layout(query, lin) &&
+                head_layout(key, lk) && head_layout(value, lv) && same_strides(key, query) && same_strides(value, query);
+    if (r.strided) {
+        r.q = query;
+        r.k = key;
+        r.v = value;
+        r.out = empty_heads(query.sizes(), query.stride(1) < query.stride(2), opt);
+        head_layout(r.out, lout);
+        spion_block_bf16_attn_forward_strided(h, vp(r.q), vp(r.k), vp(r.v), fp(pen), r.out.data_ptr(), fpm(r.lse), ip(offsets),
+                                              ip(columns), ip(sum_mat), (int)nnz, (int)H, &lin, &lout);
+    } else {
+        r.q = query.to(torch::kBFloat16).contiguous();
+        r.k = key.to(torch::kBFloat16).contiguous();
+        r.v = value.to(torch::kBFloat16).contiguous();
+        r.out = torch::empty(query.sizes(), opt);
+        spion_block_bf16_attn_forward(h, vp(r.q), vp(r.k), vp(r.v), fp(pen), r.out.data_ptr(), fpm(r.lse), ip(offsets),
+                                      ip(columns), ip(sum_mat), (int)nnz);
+    }
+    check_library("spion_block_bf16_attn_forward");
+    return r;
+}
+struct BF16AttnNode : public torch::autograd::Function<BF16AttnNode> {
+    static Tensor forward(AutogradContext* ctx, Tensor query, Tensor key, Tensor value, c10::optional<Tensor> pen_opt,
+                          Tensor offsets, Tensor columns, Tensor sum_mat, int64_t handle, int64_t nnz, int64_t stream) {
+        const Tensor pen = pen_opt.has_value() ? *pen_opt : Tensor();
+        const BF16Result r = bf16_forward(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, stream);
+        ctx->saved_data["handle"] = handle;
+        ctx->saved_data["nnz"] = nnz;
+        ctx->saved_data["stream"] = stream;
+        ctx->saved_data["strided"] = r.strided;
+        ctx->save_for_backward({r.q, r.k, r.v, r.out, r.lse, offsets, columns, sum_mat, pen});
+        return r.out;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &offsets = saved[5],
+                     &columns = saved[6], &sum_mat = saved[7], &pen = saved[8];
+        void* h = reinterpret_cast<void*>(ctx->saved_data["handle"].toInt());
+        const int nnz = (int)ctx->saved_data["nnz"].toInt();
+        spion_set_stream(h, reinterpret_cast<void*>(ctx->saved_data["stream"].toInt()));
+        Tensor dq, dk, dv;
+        if (ctx->saved_data["strided"].toBool()) {
+            const Tensor go = grad_like(grads[0], out);
+            const bool inter = q.stride(1) < q.stride(2);
+            dq = empty_heads(q.sizes(), inter, q.options());
+            dk = empty_heads(q.sizes(), inter, q.options());
+            dv = empty_heads(q.sizes(), inter, q.options());
+            spion_head_layout lin{}, lout{}, lgrad{};
+            head_layout(q, lin);
+            head_layout(out, lout);
+            head_layout(dq, lgrad);
+            spion_block_bf16_attn_backward_strided(h, vp(q), vp(k), vp(v), fp(pen), vp(out), fp(lse), vp(go), dq.data_ptr(),
+                                                   dk.data_ptr(), dv.data_ptr(), ip(offsets), ip(columns), ip(sum_mat), nnz,
+                                                   (int)q.size(1), &lin, &lout, &lgrad);
+        } else {
+            const Tensor go = grads[0].to(torch::kBFloat16).contiguous();
+            dq = torch::empty_like(q);
+            dk = torch::empty_like(q);
+            dv = torch::empty_like(q);
+            spion_block_bf16_attn_backward(h, vp(q), vp(k), vp(v), fp(pen), vp(out), fp(lse), vp(go), dq.data_ptr(),
+                                           dk.data_ptr(), dv.data_ptr(), ip(offsets), ip(columns), ip(sum_mat), nnz);
+        }
+        check_library("spion_block_bf16_attn_backward");
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
 
 // ---- the projections of models/attention.py:84-103 on the library's own kernels ------------------
 Tensor aligned(const Tensor& t) {  // contiguous, 16-byte aligned
@@ -445,6 +612,35 @@ std::vector<Tensor> sparse_attention(const Tensor& query, const Tensor& key, con
                                  stream);
 }
 
+// fp32 heads of the handle's sizes on one GPU (the module's test); mask_or_pen as for sparse_attention.  [out, map, mean or
+// nothing]
+std::vector<Tensor> dense_attention(const Tensor& query, const Tensor& key, const Tensor& value,
+                                    const c10::optional<Tensor>& mask_or_pen, bool is_mask, int64_t handle, bool emit_mean,
+                                    int64_t stream) {
+    const c10::DeviceGuard on(query.device());
+    const auto pen = penalty_of(mask_or_pen, is_mask, query.size(1), stream);
+    const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
+    if (without_node({&query, &key, &value, &pen_or_none})) {
+        DenseResult r = dense_forward(query, key, value, pen_or_none, handle, emit_mean, stream);
+        return {r.out, r.attn.transpose(2, 3), r.mean};
+    }
+    auto r = DenseAttnNode::apply(query, key, value, pen, handle, emit_mean, stream);
+    r.resize(3);
+    return r;
+}
+
+// The same for the bf16 module: heads of any floating type.
+Tensor bf16_attention(const Tensor& query, const Tensor& key, const Tensor& value, const c10::optional<Tensor>& mask_or_pen,
+                      bool is_mask, const Tensor& offsets, const Tensor& columns, const Tensor& sum_mat, int64_t handle,
+                      int64_t nnz, int64_t stream) {
+    const c10::DeviceGuard on(query.device());
+    const auto pen = penalty_of(mask_or_pen, is_mask, query.size(1), stream);
+    const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
+    if (without_node({&query, &key, &value, &pen_or_none}))
+        return bf16_forward(query, key, value, pen_or_none, offsets, columns, sum_mat, handle, nnz, stream).out;
+    return BF16AttnNode::apply(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, stream);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -453,6 +649,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("query"), py::arg("key"), py::arg("value"), py::arg("mask_or_pen"), py::arg("is_mask"), py::arg("offsets"),
           py::arg("columns"), py::arg("sum_mat"), py::arg("handle"), py::arg("nnz"), py::arg("num_heads"),
           py::arg("reads_views"), py::arg("stream"));
+    m.def("dense_attention", &dense_attention, "forward of the dense-phase modules; returns [out, map, mean map or None]");
+    m.def("bf16_attention", &bf16_attention, "forward of the bf16 module");
     m.def("sparse_layer", &sparse_layer, "forward of the attention layer in its sparse phase; returns [y, p_flat]");
     m.def("projections_fit", &projections_fit, "whether the projection kernels take this layer's linear layers");
     m.def("project_heads", &project_heads, "the three input projections; returns the [B, H, L, d] heads");

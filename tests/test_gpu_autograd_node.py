@@ -176,3 +176,109 @@ def test_projections_around_a_differentiable_core_are_twice_differentiable():
             assert a is None or float(a.norm()) < 1e-3
             continue
         assert float((a.cpu().double() - b).norm() / b.norm()) < 1e-5
+
+
+# ---- the dense-phase modules and the bf16 module ---------------------------------------------------
+def _python_only(mod, fn):
+    mod._node_takes = lambda *a: False
+    try:
+        return fn()
+    finally:
+        del mod._node_takes
+
+
+@pytest.mark.parametrize("layout", ["contiguous", "proj", "fused", "mixed"])
+@pytest.mark.parametrize("mask_kind", [None, "float", "double"])
+@pytest.mark.parametrize("d", [32, 64])
+def test_dense_node_equals_python_function(layout, mask_kind, d):
+    if _lib.autograd_node() is None:
+        pytest.skip("SPION_PY_NODE=1")
+    B, H, L = 2, 2, 160
+    cfg = dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=B)
+    cpp = getattr(Attention, "_cuda_mask_compile_module" if mask_kind else "_cuda_compile_module")()
+    mod = (spion_amd.CUDAMaskAttention if mask_kind else spion_amd.CUDAAttention)(cfg, cpp, cpp.init(d, L, B * H))
+    mask = workloads.valid_length_mask(B, L, L // 2, L, seed=5).cuda()
+    if mask_kind == "double":  # the penalties are then made by torch
+        mask = mask.double()
+
+    def step(grad):
+        leaves = [t.requires_grad_(grad) for t in _inputs(B, H, L, d, layout if layout != "mixed" else "contiguous", seed=11)[:3]]
+        do = _inputs(B, H, L, d, "contiguous", seed=12)[3]
+        if layout == "mixed":  # no common strides: copies
+            leaves[1] = leaves[1].detach().transpose(1, 2).contiguous().transpose(1, 2).requires_grad_(grad)
+        mod.score_map = None
+        with torch.set_grad_enabled(grad):
+            out, attn = mod(*leaves, mask)
+        grads = torch.autograd.grad(out, leaves, do) if grad else ()
+        if grad and layout == "fused":
+            assert _lib.adjacent_head_views(*grads)
+        return [out.detach(), attn.detach(), *grads] + ([mod.score_map] if mod.emit_score_map else [])
+
+    for emit in (False, True):
+        mod.emit_score_map = emit
+        for grad in (True, False):
+            a, b = step(grad), _python_only(mod, lambda: step(grad))
+            assert len(a) == len(b) and all(x.stride() == y.stride() and torch.equal(x, y) for x, y in zip(a, b))
+    cpp.destroy(mod.attn_handle)
+
+
+@pytest.mark.parametrize("layout", ["contiguous", "proj", "mixed"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("mask_kind", [None, "float", "double"])
+def test_bf16_node_equals_python_function(layout, dtype, mask_kind):
+    if _lib.autograd_node() is None:
+        pytest.skip("SPION_PY_NODE=1")
+    B, H, L, d, bs = 2, 2, 256, 64, 32
+    mod = spion_amd.BlockAttentionBF16(dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=B, block_size=bs), mask_kind is not None)
+    mat = torch.from_numpy(workloads.band_random_block_mask(L // bs, 1, extra_frac=0.1, seed=3).astype(np.float32)).cuda()
+    mask = workloads.valid_length_mask(B, L, L // 2, L, seed=5).cuda()
+    if mask_kind == "double":
+        mask = mask.double()
+
+    def step(grad):
+        leaves = [t.to(dtype).requires_grad_(grad) for t in _inputs(B, H, L, d, "contiguous" if layout == "mixed" else layout, seed=11)[:3]]
+        if layout == "mixed":
+            leaves[1] = leaves[1].detach().transpose(1, 2).contiguous().transpose(1, 2).requires_grad_(grad)
+        with torch.set_grad_enabled(grad):
+            out, zero = mod(*leaves, mask, mat)
+        assert zero == 0
+        do = _inputs(B, H, L, d, "contiguous", seed=12)[3].to(torch.bfloat16)
+        return [out.detach()] + (list(torch.autograd.grad(out, leaves, do)) if grad else [])
+
+    for grad in (True, False):
+        a, b = step(grad), _python_only(mod, lambda: step(grad))
+        assert len(a) == len(b) and all(x.dtype == y.dtype and x.stride() == y.stride() and torch.equal(x, y) for x, y in zip(a, b))
+    mod.lib.spion_block_bf16_destroy(mod.attn_handle)
+
+
+def test_dense_and_bf16_nodes_leave_other_calls_to_the_python_functions():
+    """Wrong sizes and types keep their errors, forward mode stays refused, the map's gradient is ignored."""
+    import torch.autograd.forward_ad as fwd
+
+    if _lib.autograd_node() is None:
+        pytest.skip("SPION_PY_NODE=1")
+    B, H, L, d = 1, 2, 64, 32
+    cfg = dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=B, block_size=32)
+    cpp = Attention._cuda_compile_module()
+    dense = spion_amd.CUDAAttention(cfg, cpp, cpp.init(d, L, B * H))
+    bf16 = spion_amd.BlockAttentionBF16(cfg)
+    q, k, v, _ = _inputs(B, H, L, d, "contiguous", seed=2)
+    ones, mat = torch.ones(B, L, device="cuda"), torch.ones(2, 2, device="cuda")
+    half = [t.bfloat16() for t in (q, k, v)]
+    with pytest.raises(ValueError):
+        dense(q[:, :1], k[:, :1], v[:, :1], ones)
+    with pytest.raises(ValueError):
+        bf16(half[0], half[1][:, :, :32], half[2], ones, mat)
+    for guard in (torch.no_grad(), torch.enable_grad()):
+        with guard, fwd.dual_level():
+            with pytest.raises(RuntimeError, match="jvp"):
+                dense(q, fwd.make_dual(k, torch.ones_like(k)), v, ones)
+            with pytest.raises(RuntimeError, match="jvp"):
+                bf16(fwd.make_dual(half[0], torch.ones_like(half[0])), half[1], half[2], ones, mat)
+    leaves = [t.clone().requires_grad_() for t in (q, k, v)]
+    out, attn = dense(*leaves, ones)
+    (attn.sum() + 0.0 * out.sum()).backward()
+    assert all(torch.count_nonzero(t.grad) == 0 for t in leaves)
+    cpp.destroy(dense.attn_handle)
+    bf16.lib.spion_block_bf16_destroy(bf16.attn_handle)
+
