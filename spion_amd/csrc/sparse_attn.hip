@@ -578,8 +578,8 @@ static int long_strip_threshold(int nstrips, int ntiles) {
 //   lane_ptr / lane_ent  CSR-like: lane s works on entries lane_ptr[s] .. lane_ptr[s+1]-1, each {head, item};
 //   longs    {strip, first slot, chunks, tiles} per long strip, for the merge kernels.
 // Lanes are dealt to the dies in turn (lane s runs on die s % 8, as work-groups are), and a die's lanes share the
-// heads of that die one head after the other (the K/V of a head then stay in the die's L2); within a head the items
-// go longest first to the lane with the least work so far.
+// heads of that die: the chunks first, then the strips one head after the other (the K/V of a head then stay in the die's
+// L2); items go longest first to the lane with the least work so far.
 struct Bf16PlanHost {
     std::vector<int> items, lane_ptr, lane_ent, longs;
     int slots = 0, lanes = 0;
@@ -628,29 +628,45 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return weight(its[x]) > weight(its[y]); });
     for (const It& x : its) out.items.insert(out.items.end(), {x.strip, x.t0, x.n, x.kind});
     if (out.items.empty()) out.items.assign(4, 0);
-    // deal: per die, head after head, every item to the lane of that die with the least work so far
+    // deal: per die, every item to the lane of that die with the least work so far; the chunks of all heads first, then the
+    // strips head after head.  (With a head's chunks among its strips the last head's came last, onto lanes that were full:
+    // up to 1.3 of the average work.  A lane still takes its items head after head.)  Kernels of a step in us, head after
+    // head / chunks first: 32 heads of 16384 554 / 520, 32 of 4096, forward alone, 42.2 / 38.5, 83 of 5600 428 / 420, 30 of 9952, d
+    // = 32, 363 / 318, 10 of 6144 160 / 142; half as long chunks: 2 % less to 20 % more.  Launches of up to two items a lane
+    // whose heads are not dealt to dies: all items longest first, 131 for the 10 of 6144, 36 of 3072, d = 32, 96 / 85; with more
+    // items, or a die's own heads, the lanes drift apart in heads and lose the K and V in L2 (562, 40.2, 425, 337).
     const int per_group = lanes / groups, heads_per_group = NB / groups;
-    std::vector<std::vector<int>> lane_list(lanes);
+    const bool mixed = groups == 1 && (long long)its.size() * NB <= 2LL * lanes;
+    std::vector<std::vector<std::pair<int, int>>> lane_list(lanes);  // {head, item}
     for (int g = 0; g < groups; ++g) {
         typedef std::pair<long long, int> Load;  // (work so far, lane of this die)
         std::priority_queue<Load, std::vector<Load>, std::greater<Load>> heap;
         for (int j = 0; j < per_group; ++j) heap.push({0, j});
-        for (int hh = 0; hh < heads_per_group; ++hh) {
-            const int bh = g * heads_per_group + hh;
-            for (int o : order) {
-                Load top = heap.top();
-                heap.pop();
-                const int lane = top.second * groups + g;
-                lane_list[lane].push_back(bh);
-                lane_list[lane].push_back(o);
-                top.first += weight(its[o]);
-                heap.push(top);
-            }
+        auto deal = [&](int hh, int o) {
+            Load top = heap.top();
+            heap.pop();
+            const int lane = top.second * groups + g;
+            lane_list[lane].push_back({g * heads_per_group + hh, o});
+            top.first += weight(its[o]);
+            heap.push(top);
+        };
+        if (mixed) {
+            for (int o : order)
+                for (int hh = 0; hh < heads_per_group; ++hh) deal(hh, o);
+            continue;
         }
+        for (int o : order)
+            if (its[o].kind >= 0)
+                for (int hh = 0; hh < heads_per_group; ++hh) deal(hh, o);
+        for (int hh = 0; hh < heads_per_group; ++hh)
+            for (int o : order)
+                if (its[o].kind < 0) deal(hh, o);
     }
     out.lane_ptr.assign(1, 0);
     for (int sidx = 0; sidx < lanes; ++sidx) {
-        out.lane_ent.insert(out.lane_ent.end(), lane_list[sidx].begin(), lane_list[sidx].end());
+        // a lane takes its items head after head, in the order they were dealt
+        std::stable_sort(lane_list[sidx].begin(), lane_list[sidx].end(), [](auto x, auto y) { return x.first < y.first; });
+        for (const auto& e : lane_list[sidx]) out.lane_ent.insert(out.lane_ent.end(), {e.first, e.second});
         out.lane_ptr.push_back((int)out.lane_ent.size() / 2);
     }
     if (out.lane_ent.empty()) out.lane_ent.assign(2, 0);
