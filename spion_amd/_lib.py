@@ -234,6 +234,13 @@ def plain_autograd() -> bool:
     return forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
 
 
+def keep_for_backward(out, module) -> None:
+    """Let the node of ``out`` hold the module: the backward works on its handle, which a program may tie to the module's
+    life."""
+    if out.grad_fn is not None:
+        out.grad_fn.metadata["module"] = module
+
+
 def use_current_stream(module, device) -> None:
     """Point the module's handle at torch's current stream on ``device`` (the reference runs on the legacy
     default stream only): what makes the modules usable on side streams and under HIP graph capture.  One

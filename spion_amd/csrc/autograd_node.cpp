@@ -214,6 +214,12 @@ c10::optional<Tensor> penalty_of(const c10::optional<Tensor>& mask_or_pen, bool 
     return key_penalty(*mask_or_pen, heads, stream);
 }
 
+// The layout of heads the strided entry points have to take: contiguous ones may start off 16 bytes, and saved-tensor hooks
+// may have put saved ones somewhere else.
+void taken_layout(const Tensor& t, spion_head_layout& lay) {
+    TORCH_CHECK_TYPE(t.is_cuda() && head_layout(t, lay), "heads on the GPU, 16-byte aligned, expected");
+}
+
 // The gradient of a core's output in that output's strides, as the strided entry points take it.
 Tensor grad_like(const Tensor& go, const Tensor& out) {
     spion_head_layout lay{};
@@ -238,7 +244,7 @@ DenseResult dense_forward(const Tensor& query, const Tensor& key, const Tensor& 
     r.q = views ? query : query.contiguous();
     r.k = views ? key : key.contiguous();
     r.v = views ? value : value.contiguous();
-    head_layout(r.q, lin);
+    taken_layout(r.q, lin);
     r.attn = torch::empty({B, H, L, L}, opt);
     r.out = empty_heads(query.sizes(), r.q.stride(1) < r.q.stride(2), opt);
     head_layout(r.out, lout);
@@ -284,8 +290,8 @@ struct DenseAttnNode : public torch::autograd::Function<DenseAttnNode> {
             dv = empty_heads(q.sizes(), inter, opt);
         }
         spion_head_layout lin{}, lout{}, lgrad{};
-        head_layout(q, lin);
-        head_layout(out, lout);
+        taken_layout(q, lin);
+        taken_layout(out, lout);
         head_layout(dq, lgrad);
         spion_dense_backward_strided(h, fp(q), fp(k), fp(v), fp(attn), fp(out), fp(go), fpm(dq), fpm(dk), fpm(dv), (int)q.size(1),
                                      &lin, &lout, &lgrad);
@@ -361,8 +367,8 @@ struct BF16AttnNode : public torch::autograd::Function<BF16AttnNode> {
             dk = empty_heads(q.sizes(), inter, q.options());
             dv = empty_heads(q.sizes(), inter, q.options());
             spion_head_layout lin{}, lout{}, lgrad{};
-            head_layout(q, lin);
-            head_layout(out, lout);
+            taken_layout(q, lin);
+            taken_layout(out, lout);
             head_layout(dq, lgrad);
             spion_block_bf16_attn_backward_strided(h, vp(q), vp(k), vp(v), fp(pen), vp(out), fp(lse), vp(go), dq.data_ptr(),
                                                    dk.data_ptr(), dv.data_ptr(), ip(offsets), ip(columns), ip(sum_mat), nnz,
@@ -612,6 +618,13 @@ std::vector<Tensor> sparse_attention(const Tensor& query, const Tensor& key, con
                                  stream);
 }
 
+// The kernels read a penalty for every key of every head: fewer, or a tensor elsewhere, would be read past its end.
+void check_penalties(const Tensor& pen, const Tensor& query) {
+    if (!pen.defined()) return;
+    TORCH_CHECK(pen.scalar_type() == torch::kFloat32 && pen.device() == query.device(), "fp32 tensors on one GPU expected");
+    TORCH_CHECK_VALUE(pen.numel() >= query.size(0) * query.size(1) * query.size(2), "key mask smaller than [B, L]");
+}
+
 // fp32 heads of the handle's sizes on one GPU (the module's test); mask_or_pen as for sparse_attention.  [out, map, mean or
 // nothing]
 std::vector<Tensor> dense_attention(const Tensor& query, const Tensor& key, const Tensor& value,
@@ -620,6 +633,7 @@ std::vector<Tensor> dense_attention(const Tensor& query, const Tensor& key, cons
     const c10::DeviceGuard on(query.device());
     const auto pen = penalty_of(mask_or_pen, is_mask, query.size(1), stream);
     const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
+    check_penalties(pen_or_none, query);
     if (without_node({&query, &key, &value, &pen_or_none})) {
         DenseResult r = dense_forward(query, key, value, pen_or_none, handle, emit_mean, stream);
         return {r.out, r.attn.transpose(2, 3), r.mean};
@@ -636,6 +650,7 @@ Tensor bf16_attention(const Tensor& query, const Tensor& key, const Tensor& valu
     const c10::DeviceGuard on(query.device());
     const auto pen = penalty_of(mask_or_pen, is_mask, query.size(1), stream);
     const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
+    check_penalties(pen_or_none, query);
     if (without_node({&query, &key, &value, &pen_or_none}))
         return bf16_forward(query, key, value, pen_or_none, offsets, columns, sum_mat, handle, nnz, stream).out;
     return BF16AttnNode::apply(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, stream);

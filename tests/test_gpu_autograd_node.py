@@ -282,3 +282,76 @@ def test_dense_and_bf16_nodes_leave_other_calls_to_the_python_functions():
     cpp.destroy(dense.attn_handle)
     bf16.lib.spion_block_bf16_destroy(bf16.attn_handle)
 
+
+
+@pytest.mark.parametrize("kind", ["dense", "bf16"])
+def test_nodes_hold_their_module_and_refuse_short_masks(kind):
+    """The backward works on the module's handle: a graph that outlives its caller's module holds it, and lets it go.  A
+    mask with fewer entries than [B, L], or on the host, is refused before a kernel reads past its end."""
+    import gc
+    import weakref
+
+    if _lib.autograd_node() is None:
+        pytest.skip("SPION_PY_NODE=1")
+    B, H, L, d = 2, 2, 64, 32
+    cfg = dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=B, block_size=32)
+    q, k, v, do = _inputs(B, H, L, d, "contiguous", seed=2)
+    if kind == "dense":
+        cpp = Attention._cuda_mask_compile_module()
+        mod = spion_amd.CUDAMaskAttention(cfg, cpp, cpp.init(d, L, B * H))
+        destroy, rest = cpp.destroy, ()
+    else:
+        mod = spion_amd.BlockAttentionBF16(cfg, True)
+        destroy, rest = mod.lib.spion_block_bf16_destroy, (torch.ones(2, 2, device="cuda"),)
+        q, k, v, do = (t.bfloat16() for t in (q, k, v, do))
+    handle, held = mod.attn_handle, weakref.ref(mod)
+    with pytest.raises(ValueError):
+        mod(q, k, v, torch.ones(1, L, device="cuda"), *rest)
+    with pytest.raises(RuntimeError):
+        mod(q, k, v, torch.ones(B, L), *rest)
+    leaves = [t.clone().requires_grad_() for t in (q, k, v)]
+    out = mod(*leaves, torch.ones(B, L, device="cuda"), *rest)[0]
+    del mod
+    gc.collect()
+    assert held() is not None
+    grads = torch.autograd.grad(out, leaves, do)
+    assert all(torch.isfinite(g).all() for g in grads)
+    del out, grads
+    gc.collect()
+    assert held() is None
+    destroy(handle)
+
+
+def test_nodes_refuse_heads_the_strided_entries_cannot_take():
+    """Contiguous heads off 16 bytes, and saved heads that hooks bring back so: refused as by the Python functions.  Hooks
+    that bring them back contiguous change nothing."""
+    if _lib.autograd_node() is None:
+        pytest.skip("SPION_PY_NODE=1")
+    B, H, L, d = 2, 2, 64, 32
+    cfg = dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=B, block_size=32)
+    cpp = Attention._cuda_compile_module()
+    dense = spion_amd.CUDAAttention(cfg, cpp, cpp.init(d, L, B * H))
+    bf16 = spion_amd.BlockAttentionBF16(cfg)
+    ones, mat = torch.ones(B, L, device="cuda"), torch.ones(2, 2, device="cuda")
+
+    def off(t):
+        return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+
+    q, k, v, do = _inputs(B, H, L, d, "proj", seed=4)
+    for call in (lambda: dense(off(q), k, v, ones), lambda: _python_only(dense, lambda: dense(off(q), k, v, ones))):
+        with pytest.raises(TypeError):
+            call()
+    for mod, rest, t in ((dense, (ones,), (q, k, v)), (bf16, (ones, mat), tuple(x.bfloat16() for x in (q, k, v)))):
+        leaves = [x.clone(memory_format=torch.preserve_format).requires_grad_() for x in t]
+
+        def step(unpack):
+            with torch.autograd.graph.saved_tensors_hooks(lambda x: x, unpack):
+                out = mod(*leaves, *rest)[0]
+            return torch.autograd.grad(out, leaves, do.to(out.dtype))
+
+        for a, b in zip(step(lambda x: x), step(lambda x: x.contiguous())):
+            assert torch.equal(a, b)
+        with pytest.raises(TypeError):
+            step(off)
+    cpp.destroy(dense.attn_handle)
+    bf16.lib.spion_block_bf16_destroy(bf16.attn_handle)
