@@ -45,9 +45,9 @@ def _matrix_ceiling(split, chains, algorithmic=2):
 
 
 # (split, fp32) products per tile of forward, row pass and column pass (spion_amd/csrc/tile_kernels.h, mma_feat_init, says why);
-# the forward in its register-resident form
+# the dense forward in its register-resident form, the dense backward with shared tiles (dense_group_kernels.h)
 _TILE_PRODUCTS = {32: ((1, 1), (1, 1), (3, 0)), 64: ((2, 0), (2, 0), (0, 3))}
-_DENSE_PRODUCTS = {32: ((1, 1), (2, 0), (1, 2)), 64: ((2, 0), (2, 0), (0, 3))}
+_DENSE_PRODUCTS = {32: ((1, 1), (2, 0), (3, 0)), 64: ((2, 0), (2, 0), (3, 0))}
 
 
 def _floors_ms(flops, ceiling, nbytes):
@@ -530,7 +530,7 @@ def bench_dense_phase(args, dev, d=32):
     _lib.check_error("dense backward")
     alg_flops = 12.0 * L * L * d * NB
     k_fwd = "dense_fwd_reg_kernel" if d == 32 else "dense_fwd_reg64_kernel"
-    k_bwd = f"dense_bwd_row{d}_kernel + dense_bwd_col{d}_kernel"
+    k_bwd = "dense_group_row_kernel + dense_group_col_kernel"
     ceil_fwd, ceil_row, ceil_col = (_matrix_ceiling(*p) for p in _DENSE_PRODUCTS[d])
     map_bytes, third = 4.0 * NB * L * L, alg_flops / 3.0  # each kernel writes or reads the map once
     roof = _roof_of(k_fwd, t_fwd_rm, third, ceil_fwd, map_bytes + 16.0 * NB * L * d)
@@ -540,10 +540,12 @@ def bench_dense_phase(args, dev, d=32):
                              + max(_floors_ms(third, ceil_col, map_bytes + 20.0 * NB * L * d).values())) / t_bwd_rm
     if t_fwd_mean is not None:
         roof["forward_with_mean_ms"] = round(t_fwd_mean, 4)  # spion_dense_forward_strided_mean: maps + their mean
-    # the feature-major ABI: the same kernels at d = 32, the two-sweep kernels with operand-layout loads at d = 64
+    # the feature-major ABI: at d = 32 the same forward and a backward whose wavefronts have tiles of their own, at d = 64 the
+    # two-sweep kernels with operand-layout loads
     roof["reference_abi_kernel_ms"] = {
         k_fwd if d == 32 else "dense_fwd_kernel": round(t_fwd, 4),
-        k_bwd if d == 32 else "dense_bwd_row_kernel + dense_bwd_col_kernel": round(t_bwd, 4)}
+        "dense_bwd_row32_kernel + dense_bwd_col32_kernel" if d == 32 else "dense_bwd_row_kernel + dense_bwd_col_kernel":
+            round(t_bwd, 4)}
     result = {
         "metric": "dense-phase attn fwd+bwd effective TFLOP/s (12*L*L*d*NB FLOPs / step time), 1 GPU",
         "value": alg_flops / ms_step / 1e9, "unit": "TFLOP/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
