@@ -75,7 +75,9 @@ __global__ __launch_bounds__(POOL_THREADS) void conv_pool_kernel(ScoreMaps maps,
 // formed / table, block 32: four maps of 2048^2 25.4 / 22.0, six of 4096^2 121 / 95 (two threads a column 106), two of 2048^2
 // 14.6 / 13.7, one of 1024^2 6.2 / 6.1 (one thread 7.8); block 64: 21.5 / 20.5, 96.6 / 92.2 (fp64 table: 24).
 // Left: without any load 18, without any sum 20 of the 22 us, i.e. latency of waves that live for 31 to 62 rows.  Several
-// block rows per work-group, the next one's loads in flight during a reduction, need 94 registers and are slower (30.5).
+// block rows per work-group, the next one's loads in flight during a reduction, need 94 registers and are slower (30.5); two
+// one after the other with one table are slower too (calls of four maps of 2048^2 32.4 / 35.1, six of 4096^2 124 / 156), and
+// the partial sums in the table's place, eight work-groups to a CU instead of seven, change nothing (1 % either way).
 constexpr int CP_COLS = 256, CP_BATCH = 16;
 // BS: 32 or 64 (filters of up to 33 taps), the own sum's weights in a table (fp64 for 32; for 64 that would leave room for two
 // work-groups to a CU, so fp32, converted); 0, any block size, formed per element.  CP_RG: threads to a column, each every CP_RG-th row.
