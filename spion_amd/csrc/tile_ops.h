@@ -70,10 +70,13 @@ __device__ __forceinline__ int xcd_remap(int pid, int total) {
 // six-product chain 217 ns, 280 ns with one operand split on the way.
 // Range: an infinite operand, or a finite one of 2^128 - 2^119 and more, whose hi rounds to infinity, gives parts that are
 // not numbers and so a NaN in every sum it enters; below 2^-110 the lo part is subnormal or lost, an absolute error under
-// 2^-133.  So a wavefront looks once a strip at what came out of its products (split_failed) and, where that is not
-// finite, or all of it so small that its operands may lie down there, walks its tiles again with fp32 chains:
-// infinities, NaN and the ends of the range come out as those give them.  What is left are operands below 2^-110 whose
-// products partners above 2^20 lift above 2^-90; there the absolute error of 2^-133 of the operand remains.
+// 2^-133.  So a wavefront looks once a strip at what came out of its products (split_failed) and, where one of its sums is
+// not finite, or so small that its operands may lie down there, walks its tiles again with fp32 chains: infinities, NaN and
+// the ends of the range come out as those give them.  What is left: operands below 2^-110 whose products partners above 2^20
+// lift above 2^-90, where the absolute error of 2^-133 of the operand remains; and sums that are zero because one operand of
+// every product is below 2^-134, which the bf16 format does not hold (fp32 chains give up to 2^-134 times the partners).
+// (The projections, project.hip, ask whether all sums of a wavefront are that small: they make 32 x 32 outputs and more of
+// it, and an output of 2^-90 that a dying weight leaves among them would cost every call the second walk.)
 template <int N>
 struct Split3 {
     bf16x8 p[3][N / 8];  // hi, mid, lo of elements 8t .. 8t+7
@@ -152,20 +155,28 @@ template <int N>
 constexpr bool is_whole<Whole<N>> = true;
 
 // Whether sums of split products have to be formed again by fp32 chains (the same answer in every lane): one of them is not
-// finite, or none of the wavefront's reaches 2^-90 although not all are zero.  (Sums whose magnitudes overflow
-// only together cost time and nothing else.)
-__device__ __forceinline__ bool split_failed_sum(float s) {  // s: the sum of a lane's magnitudes
-    const bool finite = s < __builtin_inff();                 // false for NaN
-    return __builtin_expect(__any(!finite) || (!__any(s >= 0x1p-90f) && __any(s != 0.f)), 0);
-}
+// finite, or is not zero and below 2^-90.  Every sum by itself: a key or a query whose gradients are that small may lie among
+// 31 ordinary ones (a key of probability 2^-118: relative error of its row of dV 1e-5, of 2^-124 1e-3, from split products).
+// (Sums whose magnitudes overflow only together cost time and nothing else.)
 template <int N>
 __device__ __forceinline__ bool split_failed(const f32x16 (&acc)[N]) {
     float s = 0.f;
+    unsigned least = ~0u;  // of twice the bits without the sign, less one: a zero is the largest
 #pragma unroll
     for (int c = 0; c < N; ++c)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s += fabsf(acc[c][r]);
-    return split_failed_sum(s);
+        for (int r = 0; r < 16; ++r) {
+            s += fabsf(acc[c][r]);
+            least = min(least, 2u * __float_as_uint(acc[c][r]) - 1u);
+        }
+    const bool finite = s < __builtin_inff();  // false for NaN
+    return __builtin_expect(__any(!finite || least < 2u * __builtin_bit_cast(unsigned, 0x1p-90f) - 1u), 0);
+}
+// One of a wavefront's sums is not finite, or none of them reaches 2^-90 although not all are zero; s: the sum of a lane's
+// magnitudes.
+__device__ __forceinline__ bool split_failed_sum(float s) {
+    const bool finite = s < __builtin_inff();
+    return __builtin_expect(__any(!finite) || (!__any(s >= 0x1p-90f) && __any(s != 0.f)), 0);
 }
 // The same for the exponentials of logits: a NaN among them.  (Logits may be as small as they like.)
 __device__ __forceinline__ bool split_failed(float z) { return __builtin_expect(__any(z != z), 0); }

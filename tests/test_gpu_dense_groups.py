@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import spion_amd
-from tests.test_gpu_split_products import EPS, LIMITS, LOG2E, _bounds, _compare, _special
+from tests.test_gpu_split_products import EPS, LIMITS, LOG2E, _bounds, _compare, _special, compare_by_element, improbable
 
 pytestmark = pytest.mark.gpu
 
@@ -115,3 +115,19 @@ def test_shared_tiles_near_the_smallest_floats(d, L, B):
     (p @ ref[2]).backward(do[3].double())
     for x, y in zip(got[1:], ref):
         assert float((x[3].double() - y.grad).norm() / y.grad.norm()) < 2 * L ** 0.5 * EPS
+
+
+# (and the kernels whose wavefronts have tiles of their own, row-major and feature-major)
+@pytest.mark.parametrize("d,L,B,views", [(32, 96, 128, True), (32, 1056, 20, True), (64, 160, 128, True), (32, 96, 2, True),
+                                         (32, 96, 2, False), (64, 160, 2, True)])
+def test_a_small_row_among_ordinary_ones(d, L, B, views):
+    H = 2
+    one = improbable(H, L, d, L + d)
+    t = {n: torch.cat([x, torch.randn(B - 1, H, L, d, generator=torch.Generator().manual_seed(1))]).cuda() for n, x in one.items()}
+    mod, cpp = _module(B, H, L, d, False)
+    mod.reads_views = views
+    leaves = [t[n].requires_grad_() for n in "qkv"]
+    out, p = mod(*leaves, torch.ones(B, L, device="cuda"))
+    out.backward(t["do"])
+    cpp.destroy(mod.attn_handle)
+    compare_by_element(one, p.detach()[0], out.detach()[0], [x.grad[0] for x in leaves], d)

@@ -212,3 +212,65 @@ def test_gradients_near_the_smallest_floats(d, power):
     for name, x, y in zip(NAMES[1:], got[1:], ref):
         err = float((x.double() - y.grad).norm() / y.grad.norm())
         assert err < 2 * L ** 0.5 * EPS, (name, err)
+
+
+def improbable(H, L, d, seed):
+    """Normal operands [1, H, L, d] in which one key, L/2 + 1, has a logit of -80 in every row (a probability of about 2^-122),
+    and the gradients of one query, L/2 - 5, are 2^-118 of the others'."""
+    g = torch.Generator().manual_seed(seed)
+    t = dict(zip(("q", "k", "v", "do"), (torch.randn(1, H, L, d, generator=g) for _ in range(4))))
+    t["q"][..., 0] = 4.0
+    t["k"][..., 0] = 0.0
+    t["k"][:, :, L // 2 + 1] = 0.0
+    t["k"][:, :, L // 2 + 1, 0] = -80.0 * d ** 0.5 / 4.0
+    t["do"][:, :, L // 2 - 5] *= 2.0 ** -118
+    return t
+
+
+def compare_by_element(t, p, out, grads, d):
+    """Gradients [H, L, d] against float64 steps from the probabilities [H, L, L] and the output the kernels left, each element
+    within the roundings of its own terms: `n + 8` of the magnitudes of a sum of n, as in `_bounds`, two for the product
+    with a probability, and 2^-149 a term where a product is subnormal."""
+    L = p.shape[-1]
+    rnd, tr = lambda n: (n + 8) * EPS, lambda x: x.transpose(-1, -2)
+    q, k, v, do = (t[n][0].double() for n in ("q", "k", "v", "do"))
+    p, out = p.double().cpu(), out.double().cpu()
+    assert 2.0 ** -126 < float(p[..., L // 2 + 1].max()) < 2.0 ** -120
+    mag = do.abs() @ tr(v).abs() + (do * out).abs().sum(-1, keepdim=True)
+    ds = p * (do @ tr(v) - (do * out).sum(-1, keepdim=True))
+    eds = (rnd(d) + 2 * EPS) * p * mag + 2.0 ** -149
+    want = [ds @ k * d ** -0.5, tr(ds) @ q * d ** -0.5, tr(p) @ do]
+    bound = [d ** -0.5 * (eds @ k.abs() + rnd(L) * ds.abs() @ k.abs()), d ** -0.5 * (tr(eds) @ q.abs() + rnd(L) * tr(ds).abs() @ q.abs()),
+             rnd(L) * tr(p) @ do.abs()]
+    for name, x, y, e in zip(NAMES[1:], grads, want, bound):
+        worst = float(((x.double().cpu() - y).abs() / (e + L * 2.0 ** -149)).max())
+        assert worst <= 1.0, f"{name}: {worst} of the bound"
+
+
+# a wavefront to a strip and four
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("L,route", [(96, "module"), (640, "module"), (640, "strided"), (640, "abi")])
+def test_a_small_row_among_ordinary_ones(L, route, d):
+    H, bs = 2, 32
+    t = improbable(H, L, d, L + d)
+    mat = np.ones((L // bs, L // bs), dtype=np.float32)
+    if route == "abi":
+        abi = SparseABI(d, L, H, bs, with_mask=True)
+        abi.set_pattern(*_csr(mat, bs))
+        q, k, v, do = (t[n][0].cuda() for n in ("q", "k", "v", "do"))
+        out, p = abi.forward(q, k, v, torch.zeros(H, L, device="cuda"))
+        grads, path = abi.backward(q, k, v, p, do), abi.last_path()
+        abi.close()
+    else:
+        cpp = spion_amd.Attention._blockcuda_compile_module()
+        handle = cpp.init(d, L, H, bs)
+        mod = spion_amd.CUDABlockAttention(dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=1, block_size=bs), cpp, handle)
+        place = lambda x: x.cuda().transpose(1, 2).contiguous().transpose(1, 2) if route == "strided" else x.cuda()
+        leaves = [place(t[n]).requires_grad_() for n in "qkv"]
+        out, p = mod(*leaves, torch.ones(1, L, device="cuda"), torch.from_numpy(mat).cuda())
+        out.backward(t["do"].cuda())
+        grads, path = [x.grad[0] for x in leaves], _lib.core().spion_last_path(handle)
+        out, p = out.detach()[0], p.detach()
+        cpp.destroy(handle)
+    assert path == 1
+    compare_by_element(t, p.reshape(H, L, L), out, grads, d)
