@@ -47,7 +47,11 @@ def _cdll(name: str) -> ctypes.CDLL:
 def autograd_node():
     """The compiled autograd node (lib/_spion_node.so, csrc/autograd_node.cpp), or None when SPION_PY_NODE=1 asks for
     the Python function instead (A/B timing, tests of the Python statement).  Both run the same kernels through the
-    same entry points; a missing build is an error like any other missing library."""
+    same entry points; a missing build is an error like any other missing library.  None also while torch.jit.trace
+    records: it records a Python function as one operation, but of the node only the allocations, without the kernels
+    that fill them."""
+    if torch._C._get_tracing_state() is not None:
+        return None
     if "node" in _cache:
         return _cache["node"]
     mod = None

@@ -355,3 +355,50 @@ def test_nodes_refuse_heads_the_strided_entries_cannot_take():
             step(off)
     cpp.destroy(dense.attn_handle)
     bf16.lib.spion_block_bf16_destroy(bf16.attn_handle)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("kind", ["sparse", "sparse_mask", "dense", "dense_mask", "bf16", "layer"])
+def test_traced_modules_compute(kind, grad):
+    """torch.jit.trace records the modules' Python functions: a traced module gives on other inputs what the module gives,
+    with gradients.  (The layer's projections are torch's products then: 1e-5 of the 2-norm.)"""
+    B, H, L, d = 2, 2, 64, 32
+    cfg = dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=B, block_size=32, transformer_dim=H * d, attention_dropout=0.0,
+               task="lra-image")
+    mask, mat = torch.ones(B, L, device="cuda"), torch.ones(2, 2, device="cuda")
+    mask[0, L // 2:] = 0
+    rest = (mask,) if kind.startswith("dense") else (mask, mat)
+    if kind == "layer":
+        mod = Attention(cfg, inference=True).cuda().requires_grad_(grad)
+        mod.reconstruct_for_blocksparse(cfg)
+    elif kind.startswith("dense"):
+        cpp = getattr(Attention, "_cuda_mask_compile_module" if kind == "dense_mask" else "_cuda_compile_module")()
+        cls = spion_amd.CUDAMaskAttention if kind == "dense_mask" else spion_amd.CUDAAttention
+        mod = cls(cfg, cpp, cpp.init(d, L, B * H))
+    elif kind == "bf16":
+        mod = spion_amd.BlockAttentionBF16(cfg, True)
+    else:
+        mod, cpp = _module(B, H, L, d, 32, kind == "sparse_mask")
+
+    class Caller(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.mod = mod
+
+        def forward(self, *x):
+            return 2 * self.mod(*x, *rest)[0]
+
+    def inputs(seed):
+        x = [torch.randn(B, L, H * d, generator=torch.Generator().manual_seed(seed)).cuda()] if kind == "layer" else \
+            list(_inputs(B, H, L, d, "contiguous", seed)[:3])
+        return [t.to(torch.bfloat16 if kind == "bf16" else t.dtype).requires_grad_(grad) for t in x]
+
+    caller, x = Caller(), inputs(2)
+    with torch.set_grad_enabled(grad):
+        traced = torch.jit.trace(caller, tuple(inputs(1)), check_trace=False)
+        got, want = [traced(*x)], [caller(*x)]
+    if grad:
+        go = torch.randn(want[0].shape, generator=torch.Generator().manual_seed(3)).to("cuda", want[0].dtype)
+        got, want = (y + list(torch.autograd.grad(y[0], x, go)) for y in (got, want))
+    for a, b in zip(got, want):
+        assert float((a - b).norm()) <= 1e-5 * float(b.norm()) if kind == "layer" else torch.equal(a, b)
