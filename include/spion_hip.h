@@ -247,6 +247,12 @@ int spion_last_path(void* handle);
  * of a sparse family (recorded as an error). */
 int spion_block_sizes(void* handle, int* emb_dim, int* seq_len, int* num_batches);
 
+/* Work that will come back to a handle -- a recorded backward -- may outlive the object a program ties the handle to.
+ * Between spion_hold (0 on success, 1 for what is no handle: recorded as an error) and spion_release a destroy of any family
+ * leaves the handle usable; the release of the last hold then frees it.  From any thread. */
+int spion_hold(void* handle);
+void spion_release(void* handle);
+
 /* Most recent failure recorded by a call on THIS handle ("" if none), besides the process-wide slot of
  * spion_last_error, which any thread or handle can overwrite.  Every failure is also written to stderr unless
  * the environment has SPION_QUIET=1; SPION_ABORT_ON_ERROR=1 makes a failure abort the process (for callers of the

@@ -24,6 +24,9 @@ void spion_set_backward_passes(void* handle, int mask);
  * graph recorded before the growth still points at them).  -1 otherwise. */
 int spion_debug_counter(void* handle, int which);
 
+/* Handles of all families that have not been freed (destroyed ones that are still held, spion_hold, are among them). */
+int spion_debug_handles(void);
+
 /* The schedule the bf16 kernels would walk for a tile list (host only: needs no device).  tile_ptr[nstrips + 1]: first
  * tile of every 32-row (or 32-column) strip; pairs != 0: strips 2p and 2p+1 hold the same tiles and are walked
  * together; lanes: persistent wavefronts asked for.  Returns the number of lanes the schedule uses (-1 on bad

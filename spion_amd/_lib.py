@@ -88,6 +88,12 @@ def core() -> ctypes.CDLL:
     lib.spion_forget_pattern.restype = None
     lib.spion_register_pattern.argtypes = [_P, _P, _P, c_int, _P, _P]
     lib.spion_register_pattern.restype = c_int
+    lib.spion_hold.argtypes = [_P]
+    lib.spion_hold.restype = c_int
+    lib.spion_release.argtypes = [_P]
+    lib.spion_release.restype = None
+    lib.spion_debug_handles.argtypes = []
+    lib.spion_debug_handles.restype = c_int
     lib.spion_handle_error.argtypes = [_P]
     lib.spion_handle_error.restype = c_char_p
     lib.spion_clear_handle_error.argtypes = [_P]
@@ -236,13 +242,6 @@ def plain_autograd() -> bool:
     """Neither a forward-mode level nor a functorch transform is at work: those meet the Python functions, which refuse
     them."""
     return forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
-
-
-def keep_for_backward(out, module) -> None:
-    """Let the node of ``out`` hold the module: the backward works on its handle, which a program may tie to the module's
-    life."""
-    if out.grad_fn is not None:
-        out.grad_fn.metadata["module"] = module
 
 
 def use_current_stream(module, device) -> None:

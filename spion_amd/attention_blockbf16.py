@@ -149,7 +149,6 @@ class BlockAttentionBF16(nn.Module):
             if str(e).startswith(("attn_forward:", "spion_block_bf16_attn_")):
                 raise _lib.SpionLibraryError(str(e)) from None
             raise
-        _lib.keep_for_backward(out, self)
         return out, 0
 
     def _node_takes(self, query, key, value):

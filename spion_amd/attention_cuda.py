@@ -188,7 +188,6 @@ class _DenseAttentionBase(nn.Module):
             if str(e).startswith(("attn_forward:", "attn_backward:")):
                 raise _lib.SpionLibraryError(str(e)) from None
             raise
-        _lib.keep_for_backward(out, self)
         if fused_mean:
             self.score_map = mean
         elif self.emit_score_map:  # head dimension 64: one pass over the maps just written

@@ -76,6 +76,19 @@ bool without_node(std::initializer_list<const Tensor*> inputs) {
     return true;
 }
 
+// What a node keeps of the handle its backward works on, which a program may destroy before, for instance with the module
+// it is tied to.  (The module itself is not held: Python's collector does not see what a compiled node refers to, and a
+// module that keeps its own output would never be freed.)
+// It is a tensor without elements whose storage lets go: compiled autograd takes no other object along with a node.
+void keep_handle(AutogradContext* ctx, int64_t handle) {
+    void* h = reinterpret_cast<void*>(handle);
+    ctx->saved_data["handle"] = handle;
+    if (spion_hold(h)) check_library("attn_forward");
+    c10::Storage hold(c10::Storage::use_byte_size_t(), 0, c10::DataPtr(h, h, &spion_release, c10::Device(c10::kCPU)));
+    ctx->saved_data["hold"] = at::detail::make_tensor<c10::TensorImpl>(
+        std::move(hold), c10::DispatchKeySet(c10::DispatchKey::CPU), caffe2::TypeMeta::Make<uint8_t>());
+}
+
 // What a forward of the attention core leaves for its backward.
 struct CoreResult {
     Tensor q, k, v, out, p_flat;
@@ -139,7 +152,7 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
                                     stream);
         // which kernel family serves THIS pattern (the handle may run other patterns before the backward)
         ctx->saved_data["tiled"] = r.tiled;
-        ctx->saved_data["handle"] = handle;
+        keep_handle(ctx, handle);
         ctx->saved_data["nnz"] = nnz;
         ctx->saved_data["heads"] = num_heads;
         ctx->saved_data["strided"] = r.strided;
@@ -262,7 +275,7 @@ struct DenseAttnNode : public torch::autograd::Function<DenseAttnNode> {
     static variable_list forward(AutogradContext* ctx, Tensor query, Tensor key, Tensor value, c10::optional<Tensor> pen,
                                  int64_t handle, bool emit_mean, int64_t stream) {
         DenseResult r = dense_forward(query, key, value, pen.has_value() ? *pen : Tensor(), handle, emit_mean, stream);
-        ctx->saved_data["handle"] = handle;
+        keep_handle(ctx, handle);
         ctx->saved_data["stream"] = stream;
         ctx->save_for_backward({r.q, r.k, r.v, r.attn, r.out});
         ctx->set_materialize_grads(false);  // the gradient of the returned map is ignored (as in the reference)
@@ -345,7 +358,7 @@ struct BF16AttnNode : public torch::autograd::Function<BF16AttnNode> {
                           Tensor offsets, Tensor columns, Tensor sum_mat, int64_t handle, int64_t nnz, int64_t stream) {
         const Tensor pen = pen_opt.has_value() ? *pen_opt : Tensor();
         const BF16Result r = bf16_forward(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, stream);
-        ctx->saved_data["handle"] = handle;
+        keep_handle(ctx, handle);
         ctx->saved_data["nnz"] = nnz;
         ctx->saved_data["stream"] = stream;
         ctx->saved_data["strided"] = r.strided;

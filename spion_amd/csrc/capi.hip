@@ -2,7 +2,9 @@
 #include "common.h"
 
 #include <cstdlib>
+#include <set>
 #include "../../include/spion_hip.h"
+#include "../../include/spion_hip_debug.h"
 
 namespace spion {
 
@@ -11,6 +13,22 @@ static std::string g_err;
 static thread_local HandleHeader* t_handle = nullptr;
 
 void note_current_handle(HandleHeader* h) { t_handle = h; }
+
+// Every handle that has not been freed; also what its holds are counted under.  (Never destroyed itself: a handle may be
+// let go as late as the end of the process.)
+static std::mutex g_handle_mutex;
+static std::set<HandleHeader*>& live_handles() {
+    static auto* s = new std::set<HandleHeader*>;
+    return *s;
+}
+HandleHeader::HandleHeader() {
+    std::lock_guard<std::mutex> lock(g_handle_mutex);
+    live_handles().insert(this);
+}
+HandleHeader::~HandleHeader() {
+    std::lock_guard<std::mutex> lock(g_handle_mutex);
+    live_handles().erase(this);
+}
 
 // The entry points return void like the reference's, and the reference's Python never asks for an error: so a
 // failure is also written to stderr (SPION_QUIET=1 silences it) and SPION_ABORT_ON_ERROR=1 turns it into an abort,
@@ -24,7 +42,10 @@ void set_error(const char* fmt, ...) {
     {
         std::lock_guard<std::mutex> lock(g_err_mutex);
         g_err = buf;
-        if (t_handle) {
+    }
+    {
+        std::lock_guard<std::mutex> lock(g_handle_mutex);
+        if (t_handle && live_handles().count(t_handle)) {  // (another thread may have freed it)
             strncpy(t_handle->err, buf, sizeof(t_handle->err) - 1);
             t_handle->err[sizeof(t_handle->err) - 1] = 0;
         }
@@ -102,6 +123,19 @@ int score_map_mean(const float*, int, int, int, int, float*, hipStream_t, float 
 void dense_forward_strided_mean(void*, const float*, const float*, const float*, const float*, float*, float*, float*, int,
                                 const HeadLayout&, const HeadLayout&);
 
+// A handle that is held is freed by the release of its last hold.
+static void destroy_handle(void* h, uint32_t kind) {
+    {
+        std::lock_guard<std::mutex> lock(g_handle_mutex);
+        HandleHeader* hd = static_cast<HandleHeader*>(h);
+        if (hd && hd->magic == kind && hd->holds > 0) {
+            hd->destroyed = true;
+            return;
+        }
+    }
+    kind == KIND_DENSE ? dense_destroy(h) : sparse_destroy(h);
+}
+
 }  // namespace spion
 
 using namespace spion;
@@ -124,7 +158,7 @@ void spion_block_bf16_attn_backward(void* h, const void* Q, const void* K, const
     (void)SumMat;
     sparse_bf16_backward(h, Q, K, V, Mask, Out, Lse, dO, dQ, dK, dV, Offsets, Columns, nnz);
 }
-void spion_block_bf16_destroy(void* h) { sparse_destroy(h); }
+void spion_block_bf16_destroy(void* h) { destroy_handle(h, KIND_SPARSE); }
 static spion::HeadLayout to_layout(const spion_head_layout* y);
 void spion_block_bf16_attn_forward_strided(void* h, const void* Q, const void* K, const void* V, const float* Mask,
                                            void* Out, float* Lse, const int* Offsets, const int* Columns,
@@ -167,7 +201,7 @@ void spion_block_attn_backward(void* h, const float* Q, const float* K, const fl
     (void)SumMat;
     sparse_backward(h, Q, K, Vt, P, dO, dP, dS, dQ, dK, dV, Offsets, Columns, nnz, nullptr, false);
 }
-void spion_block_destroy(void* h) { sparse_destroy(h); }
+void spion_block_destroy(void* h) { destroy_handle(h, KIND_SPARSE); }
 
 // ---- sparse, key mask --------------------------------------------------------------------------
 void* spion_blockmask_init(int emb_dim, int seq_len, int num_batches, int block_size) {
@@ -186,7 +220,7 @@ void spion_blockmask_attn_backward(void* h, const float* Q, const float* K, cons
     (void)SumMat;
     sparse_backward(h, Q, K, Vt, P, dO, dP, dS, dQ, dK, dV, Offsets, Columns, nnz, nullptr, false);
 }
-void spion_blockmask_destroy(void* h) { sparse_destroy(h); }
+void spion_blockmask_destroy(void* h) { destroy_handle(h, KIND_SPARSE); }
 
 // ---- dense phase ---------------------------------------------------------------------------------
 void* spion_dense_init(int emb_dim, int seq_len, int num_batches) {
@@ -204,7 +238,7 @@ void spion_dense_attn_backward(void* h, const float* Qt, const float* Kt, const 
     (void)dS;
     dense_backward(h, Qt, Kt, V, P, dOt, dQ, dK, dV);
 }
-void spion_dense_destroy(void* h) { dense_destroy(h); }
+void spion_dense_destroy(void* h) { destroy_handle(h, KIND_DENSE); }
 
 void* spion_densemask_init(int emb_dim, int seq_len, int num_batches) {
     note_current_handle(nullptr);
@@ -222,7 +256,7 @@ void spion_densemask_attn_backward(void* h, const float* Qt, const float* Kt, co
     (void)dS;
     dense_backward(h, Qt, Kt, V, P, dOt, dQ, dK, dV);
 }
-void spion_densemask_destroy(void* h) { dense_destroy(h); }
+void spion_densemask_destroy(void* h) { destroy_handle(h, KIND_DENSE); }
 
 // ---- projections around the attention core -------------------------------------------------------
 int spion_project_forward(const float* X, const float* const* W, const float* const* b, float* Y, long long rows, int n,
@@ -316,6 +350,30 @@ void spion_set_stream(void* h, void* stream) {
         return;
     }
     hd->stream = static_cast<hipStream_t>(stream);
+}
+int spion_hold(void* h) {
+    HandleHeader* hd = static_cast<HandleHeader*>(h);
+    if (!hd || (hd->magic != KIND_SPARSE && hd->magic != KIND_DENSE)) {
+        set_error("spion_hold: not a spion handle");
+        return 1;
+    }
+    std::lock_guard<std::mutex> lock(g_handle_mutex);
+    ++hd->holds;
+    return 0;
+}
+void spion_release(void* h) {
+    HandleHeader* hd = static_cast<HandleHeader*>(h);
+    uint32_t kind;
+    {
+        std::lock_guard<std::mutex> lock(g_handle_mutex);
+        if (!hd || hd->holds <= 0 || --hd->holds > 0 || !hd->destroyed) return;
+        kind = hd->magic;
+    }
+    destroy_handle(h, kind);
+}
+int spion_debug_handles(void) {
+    std::lock_guard<std::mutex> lock(g_handle_mutex);
+    return (int)live_handles().size();
 }
 void spion_invalidate_pattern(void* h) { sparse_invalidate(h); }
 int spion_register_pattern(void* h, const int* Offsets, const int* Columns, int nnz, const int* host_Offsets,

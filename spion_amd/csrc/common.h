@@ -38,6 +38,10 @@ struct HandleHeader {
     uint32_t magic;
     hipStream_t stream;
     char err[256];  // most recent failure of a call on this handle ("" if none), besides the process-wide slot
+    int holds = 0;           // spion_hold calls without their spion_release
+    bool destroyed = false;  // destroyed while held: the last release frees it
+    HandleHeader();          // enters and leaves the list of the process's handles (capi.hip)
+    ~HandleHeader();
 };
 
 // The handle the calling thread is working on (set by the handle checks of every entry point, cleared by

@@ -105,3 +105,26 @@ def test_autograd_node_library_loads_without_a_gpu():
     if node is None:
         pytest.skip("SPION_PY_NODE=1")
     assert callable(node.sparse_attention)
+
+
+@pytest.mark.parametrize("family", ["block", "dense"])
+def test_a_held_handle_outlives_its_destruction(family):
+    core = _lib.core()
+    alive = core.spion_debug_handles()
+    h = core.spion_block_init(32, 64, 4, 32) if family == "block" else core.spion_dense_init(32, 64, 4)
+    assert core.spion_hold(h) == 0 and core.spion_hold(h) == 0
+    getattr(core, f"spion_{family}_destroy")(h)
+    core.spion_release(h)
+    core.spion_set_stream(h, None)  # still a handle
+    _lib.check_error()
+    assert core.spion_debug_handles() == alive + 1
+    core.spion_release(h)
+    assert core.spion_debug_handles() == alive
+    h = core.spion_block_init(32, 64, 4, 32)
+    assert core.spion_hold(h) == 0
+    core.spion_release(h)  # not destroyed: stays
+    assert core.spion_debug_handles() == alive + 1
+    core.spion_block_destroy(h)
+    assert core.spion_debug_handles() == alive and core.spion_hold(None) == 1
+    with pytest.raises(_lib.SpionLibraryError, match="spion_hold"):
+        _lib.check_error()

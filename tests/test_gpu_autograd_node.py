@@ -284,42 +284,73 @@ def test_dense_and_bf16_nodes_leave_other_calls_to_the_python_functions():
 
 
 
-@pytest.mark.parametrize("kind", ["dense", "bf16"])
-def test_nodes_hold_their_module_and_refuse_short_masks(kind):
-    """The backward works on the module's handle: a graph that outlives its caller's module holds it, and lets it go.  A
-    mask with fewer entries than [B, L], or on the host, is refused before a kernel reads past its end."""
+def _of_kind(kind, B, H, L, d):
+    """(module, what its forward takes after the heads, destroy)"""
+    cfg = dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=B, block_size=32)
+    ones, mat = torch.ones(B, L, device="cuda"), torch.ones(L // 32, L // 32, device="cuda")
+    if kind == "dense":
+        cpp = Attention._cuda_mask_compile_module()
+        return spion_amd.CUDAMaskAttention(cfg, cpp, cpp.init(d, L, B * H)), (ones,), cpp.destroy
+    if kind == "bf16":
+        mod = spion_amd.BlockAttentionBF16(cfg, True)
+        return mod, (ones, mat), mod.lib.spion_block_bf16_destroy
+    mod, cpp = _module(B, H, L, d, 32, True)
+    return mod, (ones, mat), cpp.destroy
+
+
+@pytest.mark.parametrize("kind", ["sparse", "dense", "bf16"])
+def test_nodes_hold_their_handle_and_refuse_short_masks(kind):
+    """The backward works on the module's handle: a graph that outlives its caller's module holds it, also where it is destroyed
+    with the module, and lets it go.  A mask with fewer entries than [B, L], or on the host, is refused before a kernel reads
+    past its end."""
     import gc
     import weakref
 
     if _lib.autograd_node() is None:
         pytest.skip("SPION_PY_NODE=1")
     B, H, L, d = 2, 2, 64, 32
-    cfg = dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=B, block_size=32)
-    q, k, v, do = _inputs(B, H, L, d, "contiguous", seed=2)
-    if kind == "dense":
-        cpp = Attention._cuda_mask_compile_module()
-        mod = spion_amd.CUDAMaskAttention(cfg, cpp, cpp.init(d, L, B * H))
-        destroy, rest = cpp.destroy, ()
-    else:
-        mod = spion_amd.BlockAttentionBF16(cfg, True)
-        destroy, rest = mod.lib.spion_block_bf16_destroy, (torch.ones(2, 2, device="cuda"),)
-        q, k, v, do = (t.bfloat16() for t in (q, k, v, do))
-    handle, held = mod.attn_handle, weakref.ref(mod)
+    dtype = torch.bfloat16 if kind == "bf16" else torch.float32
+    q, k, v, do = (t.to(dtype) for t in _inputs(B, H, L, d, "contiguous", seed=2))
+    alive = _lib.core().spion_debug_handles()
+    mod, (mask, *rest), destroy = _of_kind(kind, B, H, L, d)
     with pytest.raises(ValueError):
         mod(q, k, v, torch.ones(1, L, device="cuda"), *rest)
     with pytest.raises(RuntimeError):
         mod(q, k, v, torch.ones(B, L), *rest)
     leaves = [t.clone().requires_grad_() for t in (q, k, v)]
-    out = mod(*leaves, torch.ones(B, L, device="cuda"), *rest)[0]
+    want = torch.autograd.grad(mod(*leaves, mask, *rest)[0], leaves, do)
+    gc.collect()
+    weakref.finalize(mod, destroy, mod.attn_handle)
+    held = weakref.ref(mod)
+    out = mod(*leaves, mask, *rest)[0]
     del mod
     gc.collect()
-    assert held() is not None
+    assert held() is None and _lib.core().spion_debug_handles() == alive + 1
     grads = torch.autograd.grad(out, leaves, do)
-    assert all(torch.isfinite(g).all() for g in grads)
+    assert all(torch.equal(a, b) for a, b in zip(grads, want))
     del out, grads
     gc.collect()
-    assert held() is None
-    destroy(handle)
+    assert _lib.core().spion_debug_handles() == alive
+
+
+@pytest.mark.parametrize("kind", ["sparse", "dense", "bf16"])
+def test_modules_that_keep_their_outputs_are_collected(kind):
+    import gc
+    import weakref
+
+    B, H, L, d = 2, 2, 64, 32
+    q, k, v, do = (t.to(torch.bfloat16 if kind == "bf16" else torch.float32) for t in _inputs(B, H, L, d, "contiguous", seed=2))
+    alive = _lib.core().spion_debug_handles()
+    for backward in (False, True):
+        mod, rest, destroy = _of_kind(kind, B, H, L, d)
+        weakref.finalize(mod, destroy, mod.attn_handle)
+        freed = weakref.ref(mod)
+        mod.kept = mod(*(t.clone().requires_grad_() for t in (q, k, v)), *rest)[0]
+        if backward:
+            mod.kept.backward(do)
+        del mod
+        gc.collect()
+        assert freed() is None and _lib.core().spion_debug_handles() == alive
 
 
 def test_nodes_refuse_heads_the_strided_entries_cannot_take():
