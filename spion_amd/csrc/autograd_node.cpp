@@ -143,10 +143,12 @@ CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& va
 
 struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
     // pen_opt: [B, H*L] key penalties of the key-mask modules, or nothing.  stream: torch's current raw
-    // stream at the call; autograd runs the backward of a node on the stream its forward ran on.
+    // stream at the call; autograd runs the backward of a node on the stream its forward ran on.  fixed: takes what
+    // carries no gradient, the probabilities of the key-mask modules (compiled autograd refuses nodes with outputs that
+    // are marked so).
     static variable_list forward(AutogradContext* ctx, Tensor query, Tensor key, Tensor value,
                                  c10::optional<Tensor> pen_opt, Tensor offsets, Tensor columns, Tensor sum_mat, int64_t handle, int64_t nnz,
-                                 int64_t num_heads, bool reads_views, int64_t stream) {
+                                 int64_t num_heads, bool reads_views, int64_t stream, Tensor* fixed) {
         const Tensor pen = pen_opt.has_value() ? *pen_opt : Tensor();
         CoreResult r = core_forward(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, num_heads, reads_views,
                                     stream);
@@ -159,8 +161,9 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
         ctx->saved_data["stream"] = stream;
         ctx->save_for_backward({r.q, r.k, r.v, r.p_flat, offsets, columns, sum_mat, r.out});
         ctx->set_materialize_grads(false);  // the gradient of the returned probabilities is ignored anyway
-        if (pen.defined()) ctx->mark_non_differentiable({r.p_flat});
-        return {r.out, r.p_flat};
+        if (!pen.defined()) return {r.out, r.p_flat};
+        *fixed = r.p_flat;
+        return {r.out};
     }
 
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -209,7 +212,7 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
                                          ip(offsets), ip(columns), ip(sum_mat), (int)nnz);
         }
         check_library("attn_backward");
-        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -273,15 +276,14 @@ DenseResult dense_forward(const Tensor& query, const Tensor& key, const Tensor& 
 }
 struct DenseAttnNode : public torch::autograd::Function<DenseAttnNode> {
     static variable_list forward(AutogradContext* ctx, Tensor query, Tensor key, Tensor value, c10::optional<Tensor> pen,
-                                 int64_t handle, bool emit_mean, int64_t stream) {
+                                 int64_t handle, bool emit_mean, int64_t stream, Tensor* mean) {
         DenseResult r = dense_forward(query, key, value, pen.has_value() ? *pen : Tensor(), handle, emit_mean, stream);
         keep_handle(ctx, handle);
         ctx->saved_data["stream"] = stream;
         ctx->save_for_backward({r.q, r.k, r.v, r.attn, r.out});
         ctx->set_materialize_grads(false);  // the gradient of the returned map is ignored (as in the reference)
-        if (!emit_mean) return {r.out, r.attn.transpose(2, 3)};
-        ctx->mark_non_differentiable({r.mean});
-        return {r.out, r.attn.transpose(2, 3), r.mean};
+        *mean = r.mean;  // (no output of the node: it carries no gradient, see SparseAttnNode)
+        return {r.out, r.attn.transpose(2, 3)};
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const auto saved = ctx->get_saved_variables();
@@ -309,7 +311,7 @@ struct DenseAttnNode : public torch::autograd::Function<DenseAttnNode> {
         spion_dense_backward_strided(h, fp(q), fp(k), fp(v), fp(attn), fp(out), fp(go), fpm(dq), fpm(dk), fpm(dv), (int)q.size(1),
                                      &lin, &lout, &lgrad);
         check_library("attn_backward");
-        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor()};
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -599,9 +601,10 @@ std::vector<Tensor> sparse_layer(const Tensor& x, const Tensor& wq, const Tensor
         return {merge_forward(aligned(r.out.transpose(1, 2)), aligned(wf), aligned(bf), stream), r.p_flat};
     }
     const auto qkv = QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream, (const KeyMask*)&keys);
+    Tensor fixed;
     const auto core = SparseAttnNode::apply(qkv[0], qkv[1], qkv[2], pen, offsets, columns, sum_mat, handle, nnz, num_heads,
-                                            true, stream);
-    return {MergeNode::apply(core[0], wf, bf, stream), core[1]};
+                                            true, stream, &fixed);
+    return {MergeNode::apply(core[0], wf, bf, stream), core.size() > 1 ? core[1] : fixed};
 }
 
 // The two projections by themselves, around a core of the caller's (the dense phase).
@@ -627,8 +630,11 @@ std::vector<Tensor> sparse_attention(const Tensor& query, const Tensor& key, con
                                           num_heads, reads_views, stream);
         return {r.out, r.p_flat};
     }
-    return SparseAttnNode::apply(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, num_heads, reads_views,
-                                 stream);
+    Tensor fixed;
+    auto r = SparseAttnNode::apply(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, num_heads, reads_views,
+                                   stream, &fixed);
+    if (r.size() == 1) r.push_back(fixed);
+    return r;
 }
 
 // The kernels read a penalty for every key of every head: fewer, or a tensor elsewhere, would be read past its end.
@@ -651,9 +657,9 @@ std::vector<Tensor> dense_attention(const Tensor& query, const Tensor& key, cons
         DenseResult r = dense_forward(query, key, value, pen_or_none, handle, emit_mean, stream);
         return {r.out, r.attn.transpose(2, 3), r.mean};
     }
-    auto r = DenseAttnNode::apply(query, key, value, pen, handle, emit_mean, stream);
-    r.resize(3);
-    return r;
+    Tensor mean;
+    const auto r = DenseAttnNode::apply(query, key, value, pen, handle, emit_mean, stream, &mean);
+    return {r[0], r[1], mean};
 }
 
 // The same for the bf16 module: heads of any floating type.

@@ -333,6 +333,42 @@ def test_nodes_hold_their_handle_and_refuse_short_masks(kind):
     assert _lib.core().spion_debug_handles() == alive
 
 
+@pytest.mark.parametrize("kind", ["sparse", "sparse_plain", "dense", "dense_mean", "bf16", "layer"])
+def test_compiled_autograd_takes_the_nodes(kind):
+    from torch._dynamo import compiled_autograd
+
+    """A recorded graph's backward through torch's compiled autograd: the gradients of the plain one, bit for bit."""
+    B, H, L, d = 2, 2, 64, 32
+    dtype = torch.bfloat16 if kind == "bf16" else torch.float32
+    *leaves, do = (t.to(dtype) for t in _inputs(B, H, L, d, "contiguous", seed=2))
+    ones, mat = torch.ones(B, L, device="cuda"), torch.ones(2, 2, device="cuda")
+    destroy = None
+    if kind == "layer":
+        cfg = dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=B, block_size=32, transformer_dim=H * d, attention_dropout=0.0,
+                   task="lra-text")
+        mod, rest = Attention(cfg, inference=True).cuda(), (ones, mat)
+        mod.reconstruct_for_blocksparse(cfg)
+        leaves, do = [leaves[0].transpose(1, 2).reshape(B, L, H * d)], do.transpose(1, 2).reshape(B, L, H * d)
+    elif kind == "sparse_plain":
+        (mod, cpp), rest = _module(B, H, L, d, 32, False), (ones, mat)
+        destroy = cpp.destroy
+    else:
+        mod, rest, destroy = _of_kind(kind.removesuffix("_mean"), B, H, L, d)
+        mod.emit_score_map = kind == "dense_mean"
+    leaves = [t.requires_grad_() for t in leaves]
+    want = torch.autograd.grad(mod(*leaves, *rest)[0], leaves, do)
+    out, second = mod(*leaves, *rest)
+    if isinstance(second, torch.Tensor) and kind == "sparse":
+        assert not second.requires_grad
+    with compiled_autograd._enable(torch.compile(backend="eager")):
+        out.backward(do)
+    assert all(torch.equal(a, t.grad) for a, t in zip(want, leaves))
+    if kind == "dense_mean":
+        assert not mod.score_map.requires_grad
+    if destroy:
+        destroy(mod.attn_handle)
+
+
 @pytest.mark.parametrize("kind", ["sparse", "dense", "bf16"])
 def test_modules_that_keep_their_outputs_are_collected(kind):
     import gc
