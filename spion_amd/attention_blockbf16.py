@@ -73,10 +73,10 @@ class _BlockBF16Function(torch.autograd.Function):
             m.lib.spion_block_bf16_attn_forward(m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), pen_ptr,
                                                 out.data_ptr(), lse.data_ptr(), *idx.tail)
         _lib.check_error("spion_block_bf16_attn_forward")
-        ctx.save_for_backward(q, k, v, out, lse, idx.offsets, idx.columns, idx.sum_mat)
+        ctx.save_for_backward(q, k, v, out, lse)
         ctx.pen = pen
         ctx.module = m
-        ctx.tail = idx.tail
+        ctx.index = idx  # not among the saved tensors: the library knows it by its address
         ctx.strided = lay is not None
         return out
 
@@ -84,7 +84,7 @@ class _BlockBF16Function(torch.autograd.Function):
     def backward(ctx, grad_output):
         m = ctx.module
         _lib.use_current_stream(m, ctx.saved_tensors[0].device)
-        q, k, v, out, lse, offsets, columns, sum_mat = ctx.saved_tensors
+        q, k, v, out, lse = ctx.saved_tensors
         pen = ctx.pen
         pen_ptr = pen.data_ptr() if pen is not None else None
         if ctx.strided:
@@ -100,7 +100,7 @@ class _BlockBF16Function(torch.autograd.Function):
             lin, lout, lgrad = _lib.head_layout(q), _lib.head_layout(out), _lib.head_layout(dq)
             m.lib.spion_block_bf16_attn_backward_strided(
                 m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), pen_ptr, out.data_ptr(), lse.data_ptr(),
-                go.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), *ctx.tail, m.num_heads,
+                go.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), *ctx.index.tail, m.num_heads,
                 ctypes.addressof(lin), ctypes.addressof(lout), ctypes.addressof(lgrad))
             _lib.check_error("spion_block_bf16_attn_backward_strided")
             return dq, dk, dv, None, None, None
@@ -108,7 +108,7 @@ class _BlockBF16Function(torch.autograd.Function):
         dq, dk, dv = torch.empty_like(q), torch.empty_like(q), torch.empty_like(q)
         m.lib.spion_block_bf16_attn_backward(m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), pen_ptr,
                                              out.data_ptr(), lse.data_ptr(), go.data_ptr(), dq.data_ptr(),
-                                             dk.data_ptr(), dv.data_ptr(), *ctx.tail)
+                                             dk.data_ptr(), dv.data_ptr(), *ctx.index.tail)
         _lib.check_error("spion_block_bf16_attn_backward")
         return dq, dk, dv, None, None, None
 

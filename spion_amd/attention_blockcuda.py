@@ -69,11 +69,10 @@ class _BlockAttnFunction(torch.autograd.Function):
         _lib.check_error("attn_forward")
         # which kernel family serves THIS pattern (the handle may run other patterns before the backward)
         ctx.tiled = _lib.core().spion_last_path(m.attn_handle) == 1
-        ctx.save_for_backward(q, k, v, p_flat, idx.offsets, idx.columns, idx.sum_mat, out)
+        ctx.save_for_backward(q, k, v, p_flat, out)
         ctx.set_materialize_grads(False)  # the gradient of the returned probabilities is ignored anyway
         ctx.module = m
-        ctx.nnz = idx.nnz
-        ctx.tail = idx.tail  # the index tensors themselves are among the saved tensors
+        ctx.index = idx  # not among the saved tensors: the library knows it by its address
         ctx.strided = lay is not None
         if m.with_mask:
             ctx.mark_non_differentiable(p_flat)
@@ -83,9 +82,9 @@ class _BlockAttnFunction(torch.autograd.Function):
     def backward(ctx, grad_output, grad_weight):
         m = ctx.module
         _lib.use_current_stream(m, ctx.saved_tensors[0].device)
-        q, k, v, p_flat, offsets, columns, sum_mat, out = ctx.saved_tensors
+        q, k, v, p_flat, out = ctx.saved_tensors
         dev = q.device
-        n_total = m.num_batches * ctx.nnz
+        n_total = m.num_batches * ctx.index.nnz
         if grad_output is None:  # only the probabilities were used downstream: their gradient is ignored
             grad_output = torch.zeros(m.batch_size, m.num_heads, m.seq_len, m.emb_dim, dtype=torch.float32, device=dev)
         core = _lib.core()
@@ -102,7 +101,7 @@ class _BlockAttnFunction(torch.autograd.Function):
             lin, lout, lgrad = _lib.head_layout(q), _lib.head_layout(out), _lib.head_layout(dq)
             core.spion_attn_backward_strided(
                 m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), p_flat.data_ptr(), out.data_ptr(),
-                go.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), *ctx.tail, m.num_heads,
+                go.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), *ctx.index.tail, m.num_heads,
                 ctypes.addressof(lin), ctypes.addressof(lout), ctypes.addressof(lgrad))
             _lib.check_error("attn_backward")
             return dq, dk, dv, None, None, None
@@ -119,7 +118,7 @@ class _BlockAttnFunction(torch.autograd.Function):
         core.spion_attn_backward_rowmajor(
             m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), p_flat.data_ptr(), out.data_ptr(), go.data_ptr(),
             scratch_ds.data_ptr() if scratch_ds is not None else None, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-            *ctx.tail)
+            *ctx.index.tail)
         _lib.check_error("attn_backward")
         return dq, dk, dv, None, None, None
 

@@ -89,6 +89,15 @@ void keep_handle(AutogradContext* ctx, int64_t handle) {
         std::move(hold), c10::DispatchKeySet(c10::DispatchKey::CPU), caffe2::TypeMeta::Make<uint8_t>());
 }
 
+// The index tensors are kept beside the saved tensors, out of the reach of saved-tensor hooks: the library knows an index by
+// its address, and one that a hook brings back somewhere else would be analysed anew (a wait for the stream, and an error
+// under capture) and stay on file for whatever index lies there next.
+void keep_index(AutogradContext* ctx, const Tensor& offsets, const Tensor& columns, const Tensor& sum_mat) {
+    ctx->saved_data["offsets"] = offsets;
+    ctx->saved_data["columns"] = columns;
+    ctx->saved_data["sum_mat"] = sum_mat;
+}
+
 // What a forward of the attention core leaves for its backward.
 struct CoreResult {
     Tensor q, k, v, out, p_flat;
@@ -159,7 +168,8 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
         ctx->saved_data["heads"] = num_heads;
         ctx->saved_data["strided"] = r.strided;
         ctx->saved_data["stream"] = stream;
-        ctx->save_for_backward({r.q, r.k, r.v, r.p_flat, offsets, columns, sum_mat, r.out});
+        keep_index(ctx, offsets, columns, sum_mat);
+        ctx->save_for_backward({r.q, r.k, r.v, r.p_flat, r.out});
         ctx->set_materialize_grads(false);  // the gradient of the returned probabilities is ignored anyway
         if (!pen.defined()) return {r.out, r.p_flat};
         *fixed = r.p_flat;
@@ -168,8 +178,9 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
 
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &p_flat = saved[3], &offsets = saved[4],
-                     &columns = saved[5], &sum_mat = saved[6], &out = saved[7];
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &p_flat = saved[3], &out = saved[4],
+                     &offsets = ctx->saved_data["offsets"].toTensor(), &columns = ctx->saved_data["columns"].toTensor(),
+                     &sum_mat = ctx->saved_data["sum_mat"].toTensor();
         void* h = reinterpret_cast<void*>(ctx->saved_data["handle"].toInt());
         const int64_t nnz = ctx->saved_data["nnz"].toInt();
         const int heads = (int)ctx->saved_data["heads"].toInt();
@@ -364,13 +375,15 @@ struct BF16AttnNode : public torch::autograd::Function<BF16AttnNode> {
         ctx->saved_data["nnz"] = nnz;
         ctx->saved_data["stream"] = stream;
         ctx->saved_data["strided"] = r.strided;
-        ctx->save_for_backward({r.q, r.k, r.v, r.out, r.lse, offsets, columns, sum_mat, pen});
+        keep_index(ctx, offsets, columns, sum_mat);
+        ctx->save_for_backward({r.q, r.k, r.v, r.out, r.lse, pen});
         return r.out;
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &offsets = saved[5],
-                     &columns = saved[6], &sum_mat = saved[7], &pen = saved[8];
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &pen = saved[5],
+                     &offsets = ctx->saved_data["offsets"].toTensor(), &columns = ctx->saved_data["columns"].toTensor(),
+                     &sum_mat = ctx->saved_data["sum_mat"].toTensor();
         void* h = reinterpret_cast<void*>(ctx->saved_data["handle"].toInt());
         const int nnz = (int)ctx->saved_data["nnz"].toInt();
         spion_set_stream(h, reinterpret_cast<void*>(ctx->saved_data["stream"].toInt()));

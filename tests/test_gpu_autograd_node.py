@@ -10,6 +10,7 @@ import torch
 import spion_amd
 from spion_amd import _lib, workloads
 from spion_amd.attention import Attention
+from spion_amd.attention_blockbf16 import _BlockBF16Function
 
 pytestmark = pytest.mark.gpu
 
@@ -283,7 +284,6 @@ def test_dense_and_bf16_nodes_leave_other_calls_to_the_python_functions():
     bf16.lib.spion_block_bf16_destroy(bf16.attn_handle)
 
 
-
 def _of_kind(kind, B, H, L, d):
     """(module, what its forward takes after the heads, destroy)"""
     cfg = dict(head_dim=d, num_head=H, max_seq_len=L, batch_size=B, block_size=32)
@@ -335,9 +335,9 @@ def test_nodes_hold_their_handle_and_refuse_short_masks(kind):
 
 @pytest.mark.parametrize("kind", ["sparse", "sparse_plain", "dense", "dense_mean", "bf16", "layer"])
 def test_compiled_autograd_takes_the_nodes(kind):
+    """A recorded graph's backward through torch's compiled autograd: the gradients of the plain one, bit for bit."""
     from torch._dynamo import compiled_autograd
 
-    """A recorded graph's backward through torch's compiled autograd: the gradients of the plain one, bit for bit."""
     B, H, L, d = 2, 2, 64, 32
     dtype = torch.bfloat16 if kind == "bf16" else torch.float32
     *leaves, do = (t.to(dtype) for t in _inputs(B, H, L, d, "contiguous", seed=2))
@@ -387,6 +387,41 @@ def test_modules_that_keep_their_outputs_are_collected(kind):
         del mod
         gc.collect()
         assert freed() is None and _lib.core().spion_debug_handles() == alive
+
+
+@pytest.mark.parametrize("python", [False, True])
+@pytest.mark.parametrize("kind", ["sparse", "bf16"])
+def test_saved_tensor_hooks_do_not_meet_the_index(kind, python):
+    """The library knows an index by its address: one that a hook brings back somewhere else would be analysed again, and
+    stay on file for whatever index comes to lie there next.  Masks of as many entries taken in turn, everything saved moved
+    to the host: the gradients as without, bit for bit, and the hooks see floating tensors alone."""
+    B, H, L, d = 2, 2, 128, 32
+    mod, (ones, _), destroy = _of_kind(kind, B, H, L, d)
+    dtype = torch.bfloat16 if kind == "bf16" else torch.float32
+    *leaves, do = (t.to(dtype) for t in _inputs(B, H, L, d, "contiguous", seed=6))
+    leaves = [t.requires_grad_() for t in leaves]
+    mats = [torch.eye(4, device="cuda").roll(k, 0).contiguous() for k in range(3)]
+    seen = set()
+
+    def pack(t):
+        seen.add(t.dtype)
+        return t.cpu()
+
+    def forward(m):
+        if not python:
+            return mod(*leaves, ones, m)[0]
+        if kind == "bf16":
+            return _BlockBF16Function.apply(*leaves, ones, m, mod)
+        return mod.attn_func.apply(*leaves, ones, m, mod)[0]
+
+    want = [torch.autograd.grad(forward(m), leaves, do) for m in mats]
+    for m, w in list(zip(mats, want)) * 2:
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+            out = forward(m)
+        got = torch.autograd.grad(out, leaves, do)
+        assert all(torch.equal(a, b) for a, b in zip(got, w))
+    assert all(t.is_floating_point for t in seen)
+    destroy(mod.attn_handle)
 
 
 def test_nodes_refuse_heads_the_strided_entries_cannot_take():
