@@ -223,6 +223,36 @@ def head_layout(t: "torch.Tensor") -> HeadLayout | None:
     return HeadLayout(sb, sh, sl)
 
 
+def taken_layout(t: "torch.Tensor") -> HeadLayout:
+    """The layout of heads the strided entry points have to take."""
+    lay = head_layout(t)
+    if lay is None:
+        raise TypeError("heads on the GPU, 16-byte aligned, expected")
+    return lay
+
+
+def save_for_backward(ctx, *tensors) -> None:
+    ctx.save_for_backward(*tensors)
+    ctx.saved_as = [(tuple(int(n) for n in t.shape), t.dtype, t.device) for t in tensors]
+
+
+def saved_tensors(ctx):
+    """The saved tensors, which hooks may have brought back as something else, while the kernels take types and sizes as they
+    were saved: other strides are the caller's to put right (``one_layout``), anything else is refused."""
+    saved = ctx.saved_tensors
+    for t, as_saved in zip(saved, ctx.saved_as):
+        if (tuple(t.shape), t.dtype, t.device) != as_saved:
+            raise TypeError("saved tensors of the device, type and size they were saved with expected")
+    return saved
+
+
+def one_layout(*heads):
+    """The heads as they are if the strided entry points take them and they share their strides, contiguous otherwise."""
+    if all(head_layout(t) is not None and t.stride() == heads[0].stride() for t in heads):
+        return heads
+    return tuple(t.contiguous() for t in heads)
+
+
 def adjacent_head_views(q, k, v):
     """True when q, k, v ([B,H,L,d] views) are the three slices of one [B, L, 3, H, d] buffer, in this order."""
     B, H, L, d = q.shape

@@ -73,7 +73,7 @@ class _BlockBF16Function(torch.autograd.Function):
             m.lib.spion_block_bf16_attn_forward(m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), pen_ptr,
                                                 out.data_ptr(), lse.data_ptr(), *idx.tail)
         _lib.check_error("spion_block_bf16_attn_forward")
-        ctx.save_for_backward(q, k, v, out, lse)
+        _lib.save_for_backward(ctx, q, k, v, out, lse)
         ctx.pen = pen
         ctx.module = m
         ctx.index = idx  # not among the saved tensors: the library knows it by its address
@@ -83,11 +83,13 @@ class _BlockBF16Function(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         m = ctx.module
-        _lib.use_current_stream(m, ctx.saved_tensors[0].device)
-        q, k, v, out, lse = ctx.saved_tensors
+        q, k, v, out, lse = _lib.saved_tensors(ctx)
+        _lib.use_current_stream(m, q.device)
+        lse = lse.contiguous()
         pen = ctx.pen
         pen_ptr = pen.data_ptr() if pen is not None else None
         if ctx.strided:
+            (q, k, v), (out,) = _lib.one_layout(q, k, v), _lib.one_layout(out)
             go = grad_output
             if go.dtype != torch.bfloat16 or go.stride() != out.stride() or _lib.head_layout(go) is None:
                 go = torch.empty_like(out).copy_(grad_output)  # preserves out's strides
@@ -97,14 +99,14 @@ class _BlockBF16Function(torch.autograd.Function):
                               for _ in range(3))
             else:
                 dq, dk, dv = (torch.empty((B, H, L, d), dtype=torch.bfloat16, device=q.device) for _ in range(3))
-            lin, lout, lgrad = _lib.head_layout(q), _lib.head_layout(out), _lib.head_layout(dq)
+            lin, lout, lgrad = _lib.taken_layout(q), _lib.taken_layout(out), _lib.head_layout(dq)
             m.lib.spion_block_bf16_attn_backward_strided(
                 m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), pen_ptr, out.data_ptr(), lse.data_ptr(),
                 go.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), *ctx.index.tail, m.num_heads,
                 ctypes.addressof(lin), ctypes.addressof(lout), ctypes.addressof(lgrad))
             _lib.check_error("spion_block_bf16_attn_backward_strided")
             return dq, dk, dv, None, None, None
-        go = grad_output.to(torch.bfloat16).contiguous()
+        q, k, v, out, go = (t.contiguous() for t in (q, k, v, out, grad_output.to(torch.bfloat16)))
         dq, dk, dv = torch.empty_like(q), torch.empty_like(q), torch.empty_like(q)
         m.lib.spion_block_bf16_attn_backward(m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), pen_ptr,
                                              out.data_ptr(), lse.data_ptr(), go.data_ptr(), dq.data_ptr(),

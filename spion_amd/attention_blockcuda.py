@@ -69,7 +69,7 @@ class _BlockAttnFunction(torch.autograd.Function):
         _lib.check_error("attn_forward")
         # which kernel family serves THIS pattern (the handle may run other patterns before the backward)
         ctx.tiled = _lib.core().spion_last_path(m.attn_handle) == 1
-        ctx.save_for_backward(q, k, v, p_flat, out)
+        _lib.save_for_backward(ctx, q, k, v, p_flat, out)
         ctx.set_materialize_grads(False)  # the gradient of the returned probabilities is ignored anyway
         ctx.module = m
         ctx.index = idx  # not among the saved tensors: the library knows it by its address
@@ -81,14 +81,15 @@ class _BlockAttnFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output, grad_weight):
         m = ctx.module
-        _lib.use_current_stream(m, ctx.saved_tensors[0].device)
-        q, k, v, p_flat, out = ctx.saved_tensors
-        dev = q.device
+        q, k, v, p_flat, out = _lib.saved_tensors(ctx)
+        p_flat, dev = p_flat.contiguous(), q.device
+        _lib.use_current_stream(m, dev)
         n_total = m.num_batches * ctx.index.nnz
         if grad_output is None:  # only the probabilities were used downstream: their gradient is ignored
             grad_output = torch.zeros(m.batch_size, m.num_heads, m.seq_len, m.emb_dim, dtype=torch.float32, device=dev)
         core = _lib.core()
         if ctx.strided:
+            (q, k, v), (out,) = _lib.one_layout(q, k, v), _lib.one_layout(out)
             go = grad_output
             if go.stride() != out.stride() or _lib.head_layout(go) is None:
                 go = torch.empty_like(out).copy_(grad_output)  # preserves out's strides
@@ -98,14 +99,14 @@ class _BlockAttnFunction(torch.autograd.Function):
                 dq, dk, dv = _lib.empty_adjacent_heads(*shape, dev)
             else:
                 dq, dk, dv = (_empty_heads(shape, interleaved, dev) for _ in range(3))
-            lin, lout, lgrad = _lib.head_layout(q), _lib.head_layout(out), _lib.head_layout(dq)
+            lin, lout, lgrad = _lib.taken_layout(q), _lib.taken_layout(out), _lib.head_layout(dq)
             core.spion_attn_backward_strided(
                 m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), p_flat.data_ptr(), out.data_ptr(),
                 go.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), *ctx.index.tail, m.num_heads,
                 ctypes.addressof(lin), ctypes.addressof(lout), ctypes.addressof(lgrad))
             _lib.check_error("attn_backward")
             return dq, dk, dv, None, None, None
-        go = grad_output.contiguous()
+        q, k, v, out, go = (t.contiguous() for t in (q, k, v, out, grad_output))
         # Of the ABI's two [NB*nnz] scratch arguments (models/attention_blockcuda.py:83-84) the tile kernels use
         # neither and the element kernels only dS: nothing that size is allocated unless it is needed.
         scratch_ds = None

@@ -75,7 +75,7 @@ class _DenseAttnFunction(torch.autograd.Function):
             if m.emit_score_map and d != 32:  # head dimension 64: one pass over the maps just written
                 from .pattern import mean_score_map
                 m.score_map = mean_score_map(attn.permute(0, 1, 3, 2))
-            ctx.save_for_backward(query, key, value, attn, out)
+            _lib.save_for_backward(ctx, query, key, value, attn, out)
             ctx.set_materialize_grads(False)
             ctx.module = m
             ctx.strided = True
@@ -96,7 +96,7 @@ class _DenseAttnFunction(torch.autograd.Function):
         if m.emit_score_map:  # shapes the fused kernel does not serve: one pass over the maps just written
             from .pattern import mean_score_map
             m.score_map = mean_score_map(attn.permute(0, 1, 3, 2))
-        ctx.save_for_backward(qt, key, value, attn)
+        _lib.save_for_backward(ctx, qt, key, value, attn)
         ctx.set_materialize_grads(False)  # the gradient of the returned map is ignored (as in the reference)
         ctx.module = m
         return out_t.permute(0, 1, 3, 2), attn.permute(0, 1, 3, 2)
@@ -104,10 +104,12 @@ class _DenseAttnFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output, grad_weights):
         m = ctx.module
-        _lib.use_current_stream(m, ctx.saved_tensors[0].device)
+        saved = _lib.saved_tensors(ctx)
+        _lib.use_current_stream(m, saved[0].device)
         B, H, L, d = m.batch_size, m.num_heads, m.seq_len, m.emb_dim
         if ctx.strided:
-            q, k, v, attn, out = ctx.saved_tensors
+            q, k, v, attn, out = saved
+            (q, k, v), attn, (out,) = _lib.one_layout(q, k, v), attn.contiguous(), _lib.one_layout(out)
             dev = q.device
             if grad_output is None:  # only the returned map was used downstream: its gradient is ignored
                 grad_output = torch.zeros(B, H, L, d, dtype=torch.float32, device=dev)
@@ -118,15 +120,15 @@ class _DenseAttnFunction(torch.autograd.Function):
                 dq, dk, dv = _lib.empty_adjacent_heads(B, H, L, d, dev)
             else:
                 dq, dk, dv = (_empty_heads((B, H, L, d), q.stride(1) < q.stride(2), dev) for _ in range(3))
-            lin, lout, lgrad = _lib.head_layout(q), _lib.head_layout(out), _lib.head_layout(dq)
+            lin, lout, lgrad = _lib.taken_layout(q), _lib.taken_layout(out), _lib.head_layout(dq)
             _lib.core().spion_dense_backward_strided(
                 m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), attn.data_ptr(), out.data_ptr(),
                 go.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), H, ctypes.addressof(lin),
                 ctypes.addressof(lout), ctypes.addressof(lgrad))
             _lib.check_error("attn_backward")
             return dq, dk, dv, None, None
-        qt, key, value, attn = ctx.saved_tensors
-        dev = qt.device
+        qt, key, value, attn = saved
+        qt, attn, dev = qt.contiguous(), attn.contiguous(), qt.device
         kt = _lib.transpose_last2(key)
         v = value.contiguous()
         if grad_output is None:  # only the returned map was used downstream: its gradient is ignored

@@ -98,6 +98,54 @@ void keep_index(AutogradContext* ctx, const Tensor& offsets, const Tensor& colum
     ctx->saved_data["sum_mat"] = sum_mat;
 }
 
+// The layout of heads the strided entry points have to take: contiguous ones may start off 16 bytes, and saved-tensor hooks
+// may have put saved ones somewhere else.
+void taken_layout(const Tensor& t, spion_head_layout& lay) {
+    TORCH_CHECK_TYPE(t.is_cuda() && head_layout(t, lay), "heads on the GPU, 16-byte aligned, expected");
+}
+
+// Saved tensors as the backward finds them: hooks may bring any of them back as something else, while the kernels take types
+// and sizes as they were saved and one layout for q, k and v.  Other strides are put right; another device or type, or fewer
+// values, are refused.
+void keep_sizes(AutogradContext* ctx, const Tensor& q) {
+    ctx->saved_data["sizes"] =
+        std::vector<int64_t>{q.size(0), q.size(1), q.size(2), q.size(3), static_cast<int64_t>(q.device().index())};
+}
+struct SavedTensors {
+    const std::vector<int64_t> sizes;
+    const variable_list saved;
+    explicit SavedTensors(AutogradContext* ctx)
+        : sizes(ctx->saved_data["sizes"].toIntVector()), saved(ctx->get_saved_variables()) {}
+    const Tensor& checked(size_t i, at::ScalarType type) const {
+        const Tensor& t = saved.at(i);
+        TORCH_CHECK_TYPE(t.defined() && t.is_cuda() && t.device().index() == sizes[4] && t.scalar_type() == type,
+                         "saved tensors of the device and type they were saved with expected");
+        return t;
+    }
+    Tensor heads(size_t i, at::ScalarType type) const {
+        const Tensor& t = checked(i, type);
+        TORCH_CHECK_TYPE(t.sizes() == c10::IntArrayRef(sizes.data(), 4), "saved heads of the size they were saved with expected");
+        spion_head_layout lay{};
+        return head_layout(t, lay) ? t : t.contiguous();
+    }
+    // the saved tensors 0 to 2, in one layout
+    void inputs(at::ScalarType type, Tensor& q, Tensor& k, Tensor& v) const {
+        q = heads(0, type);
+        k = heads(1, type);
+        v = heads(2, type);
+        if (same_strides(k, q) && same_strides(v, q)) return;
+        q = q.contiguous();
+        k = k.contiguous();
+        v = v.contiguous();
+    }
+    // fp32 values, `per_head` for each of the heads
+    Tensor values(size_t i, int64_t per_head) const {
+        const Tensor& t = checked(i, torch::kFloat32);
+        TORCH_CHECK_TYPE(t.numel() >= sizes[0] * sizes[1] * per_head, "saved values as many as were saved expected");
+        return t.contiguous();
+    }
+};
+
 // What a forward of the attention core leaves for its backward.
 struct CoreResult {
     Tensor q, k, v, out, p_flat;
@@ -169,6 +217,7 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
         ctx->saved_data["strided"] = r.strided;
         ctx->saved_data["stream"] = stream;
         keep_index(ctx, offsets, columns, sum_mat);
+        keep_sizes(ctx, r.q);
         ctx->save_for_backward({r.q, r.k, r.v, r.p_flat, r.out});
         ctx->set_materialize_grads(false);  // the gradient of the returned probabilities is ignored anyway
         if (!pen.defined()) return {r.out, r.p_flat};
@@ -177,12 +226,14 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
     }
 
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
-        const auto saved = ctx->get_saved_variables();
-        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &p_flat = saved[3], &out = saved[4],
-                     &offsets = ctx->saved_data["offsets"].toTensor(), &columns = ctx->saved_data["columns"].toTensor(),
+        const Tensor &offsets = ctx->saved_data["offsets"].toTensor(), &columns = ctx->saved_data["columns"].toTensor(),
                      &sum_mat = ctx->saved_data["sum_mat"].toTensor();
         void* h = reinterpret_cast<void*>(ctx->saved_data["handle"].toInt());
         const int64_t nnz = ctx->saved_data["nnz"].toInt();
+        const SavedTensors saved(ctx);
+        Tensor q, k, v, out = saved.heads(4, torch::kFloat32);
+        saved.inputs(torch::kFloat32, q, k, v);
+        const Tensor p_flat = saved.values(3, nnz);
         const int heads = (int)ctx->saved_data["heads"].toInt();
         spion_set_stream(h, reinterpret_cast<void*>(ctx->saved_data["stream"].toInt()));
         const auto opt = q.options();
@@ -203,12 +254,16 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
                 dk = empty_heads(q.sizes(), inter, opt);
                 dv = empty_heads(q.sizes(), inter, opt);
             }
-            head_layout(q, lin);
-            head_layout(out, lout);
+            taken_layout(q, lin);
+            taken_layout(out, lout);
             head_layout(dq, lgrad);
             spion_attn_backward_strided(h, fp(q), fp(k), fp(v), fp(p_flat), fp(out), fp(go), fpm(dq), fpm(dk), fpm(dv),
                                         ip(offsets), ip(columns), ip(sum_mat), (int)nnz, heads, &lin, &lout, &lgrad);
         } else {
+            q = q.contiguous();
+            k = k.contiguous();
+            v = v.contiguous();
+            out = out.contiguous();
             go = go.contiguous();
             // of the ABI's two [NB*nnz] scratch arguments (models/attention_blockcuda.py:83-84) the tile kernels use
             // neither and the element kernels only dS
@@ -239,12 +294,6 @@ c10::optional<Tensor> penalty_of(const c10::optional<Tensor>& mask_or_pen, bool 
     if (!is_mask || !mask_or_pen.has_value()) return mask_or_pen;
     if (has_tangent(*mask_or_pen)) return (1e6 * (1.0 - mask_or_pen->repeat({1, heads}))).contiguous();
     return key_penalty(*mask_or_pen, heads, stream);
-}
-
-// The layout of heads the strided entry points have to take: contiguous ones may start off 16 bytes, and saved-tensor hooks
-// may have put saved ones somewhere else.
-void taken_layout(const Tensor& t, spion_head_layout& lay) {
-    TORCH_CHECK_TYPE(t.is_cuda() && head_layout(t, lay), "heads on the GPU, 16-byte aligned, expected");
 }
 
 // The gradient of a core's output in that output's strides, as the strided entry points take it.
@@ -291,14 +340,17 @@ struct DenseAttnNode : public torch::autograd::Function<DenseAttnNode> {
         DenseResult r = dense_forward(query, key, value, pen.has_value() ? *pen : Tensor(), handle, emit_mean, stream);
         keep_handle(ctx, handle);
         ctx->saved_data["stream"] = stream;
+        keep_sizes(ctx, r.q);
         ctx->save_for_backward({r.q, r.k, r.v, r.attn, r.out});
         ctx->set_materialize_grads(false);  // the gradient of the returned map is ignored (as in the reference)
         *mean = r.mean;  // (no output of the node: it carries no gradient, see SparseAttnNode)
         return {r.out, r.attn.transpose(2, 3)};
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
-        const auto saved = ctx->get_saved_variables();
-        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &attn = saved[3], &out = saved[4];
+        const SavedTensors saved(ctx);
+        Tensor q, k, v;
+        saved.inputs(torch::kFloat32, q, k, v);
+        const Tensor attn = saved.values(3, q.size(2) * q.size(2)), out = saved.heads(4, torch::kFloat32);
         void* h = reinterpret_cast<void*>(ctx->saved_data["handle"].toInt());
         spion_set_stream(h, reinterpret_cast<void*>(ctx->saved_data["stream"].toInt()));
         const auto opt = q.options();
@@ -376,14 +428,17 @@ struct BF16AttnNode : public torch::autograd::Function<BF16AttnNode> {
         ctx->saved_data["stream"] = stream;
         ctx->saved_data["strided"] = r.strided;
         keep_index(ctx, offsets, columns, sum_mat);
+        keep_sizes(ctx, r.q);
         ctx->save_for_backward({r.q, r.k, r.v, r.out, r.lse, pen});
         return r.out;
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
-        const auto saved = ctx->get_saved_variables();
-        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &pen = saved[5],
-                     &offsets = ctx->saved_data["offsets"].toTensor(), &columns = ctx->saved_data["columns"].toTensor(),
+        const Tensor &offsets = ctx->saved_data["offsets"].toTensor(), &columns = ctx->saved_data["columns"].toTensor(),
                      &sum_mat = ctx->saved_data["sum_mat"].toTensor();
+        const SavedTensors saved(ctx);
+        Tensor q, k, v, out = saved.heads(3, torch::kBFloat16);
+        saved.inputs(torch::kBFloat16, q, k, v);
+        const Tensor lse = saved.values(4, q.size(2)), pen = saved.saved[5].defined() ? saved.values(5, q.size(2)) : Tensor();
         void* h = reinterpret_cast<void*>(ctx->saved_data["handle"].toInt());
         const int nnz = (int)ctx->saved_data["nnz"].toInt();
         spion_set_stream(h, reinterpret_cast<void*>(ctx->saved_data["stream"].toInt()));
@@ -402,6 +457,10 @@ struct BF16AttnNode : public torch::autograd::Function<BF16AttnNode> {
                                                    dk.data_ptr(), dv.data_ptr(), ip(offsets), ip(columns), ip(sum_mat), nnz,
                                                    (int)q.size(1), &lin, &lout, &lgrad);
         } else {
+            q = q.contiguous();
+            k = k.contiguous();
+            v = v.contiguous();
+            out = out.contiguous();
             const Tensor go = grads[0].to(torch::kBFloat16).contiguous();
             dq = torch::empty_like(q);
             dk = torch::empty_like(q);
@@ -455,6 +514,14 @@ Tensor project_weight_grads(const float* dy, const Tensor& x, int64_t rows, int6
     return dw;
 }
 
+// What the nodes below saved, as hooks bring it back: the kernels take sizes from what was saved.
+const Tensor& saved_as(const Tensor& t, c10::IntArrayRef sizes, int64_t device) {
+    TORCH_CHECK_TYPE(t.defined() && t.is_cuda() && t.device().index() == device && t.scalar_type() == torch::kFloat32 &&
+                         t.sizes() == sizes,
+                     "saved tensors of the device, type and size they were saved with expected");
+    return t;
+}
+
 // A [B, L] key mask whose penalties the launch of the input projections is to make as well (null: none).
 struct KeyMask {
     const float* mask = nullptr;
@@ -491,14 +558,20 @@ struct QkvNode : public torch::autograd::Function<QkvNode> {
         const Tensor w[3] = {aligned(wq), aligned(wk), aligned(wv)}, b[3] = {aligned(bq), aligned(bk), aligned(bv)};
         ctx->save_for_backward({x, wq, wk, wv});
         ctx->saved_data["H"] = H;
+        ctx->saved_data["d"] = d;
+        ctx->saved_data["x_sizes"] = x.sizes().vec();
+        ctx->saved_data["device"] = static_cast<int64_t>(x.device().index());
         ctx->saved_data["stream"] = stream;
         return qkv_forward(aligned(x), w, b, H, d, stream, keys);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
-        const int64_t H = ctx->saved_data["H"].toInt(), stream = ctx->saved_data["stream"].toInt();
-        const int64_t B = saved[0].size(0), L = saved[0].size(1), dim = saved[0].size(2), n = saved[1].size(0), d = n / H,
-                      rows = B * L;
+        const int64_t H = ctx->saved_data["H"].toInt(), d = ctx->saved_data["d"].toInt(), n = H * d,
+                      stream = ctx->saved_data["stream"].toInt(), device = ctx->saved_data["device"].toInt();
+        const auto sizes = ctx->saved_data["x_sizes"].toIntVector();
+        const int64_t B = sizes[0], L = sizes[1], dim = sizes[2], rows = B * L;
+        saved_as(saved[0], sizes, device);
+        for (int i = 1; i < 4; ++i) saved_as(saved[i], {n, dim}, device);
         for (auto& t : g)
             if (!t.defined()) t = torch::zeros({B, H, L, d}, saved[0].options());
         if (torch::GradMode::is_enabled()) {
@@ -558,14 +631,20 @@ Tensor merge_forward(const Tensor& merged, const Tensor& w, const Tensor& b, int
 struct MergeNode : public torch::autograd::Function<MergeNode> {
     static Tensor forward(AutogradContext* ctx, Tensor heads, Tensor w, Tensor b, int64_t stream) {
         ctx->save_for_backward({heads, w});
+        ctx->saved_data["heads_sizes"] = heads.sizes().vec();
+        ctx->saved_data["outputs"] = w.size(0);
+        ctx->saved_data["device"] = static_cast<int64_t>(heads.device().index());
         ctx->saved_data["stream"] = stream;
         return merge_forward(aligned(heads.transpose(1, 2)), aligned(w), aligned(b), stream);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
-        const int64_t stream = ctx->saved_data["stream"].toInt();
-        const int64_t B = saved[0].size(0), H = saved[0].size(1), L = saved[0].size(2), d = saved[0].size(3);
-        const int64_t rows = B * L, n = H * d, dim = saved[1].size(0);
+        const int64_t stream = ctx->saved_data["stream"].toInt(), device = ctx->saved_data["device"].toInt();
+        const auto sizes = ctx->saved_data["heads_sizes"].toIntVector();
+        const int64_t B = sizes[0], H = sizes[1], L = sizes[2], d = sizes[3];
+        const int64_t rows = B * L, n = H * d, dim = ctx->saved_data["outputs"].toInt();
+        saved_as(saved[0], sizes, device);
+        saved_as(saved[1], {dim, n}, device);
         variable_list r(4);
         if (torch::GradMode::is_enabled()) {
             const Tensor dy = g[0].reshape({rows, dim});
