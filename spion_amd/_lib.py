@@ -223,6 +223,24 @@ def head_layout(t: "torch.Tensor") -> HeadLayout | None:
     return HeadLayout(sb, sh, sl)
 
 
+def check_heads(shape, query, key, value, dtype=None) -> None:
+    """The kernels take sizes, types and devices of the heads from the handle: anything else would be read past its end."""
+    for name, t in (("query", query), ("key", key), ("value", value)):
+        if tuple(t.shape) != tuple(shape):
+            raise ValueError(f"{name} shape {tuple(t.shape)} does not match the handle {tuple(shape)}")
+    for t in (query, key, value):
+        if not t.is_cuda or t.device != query.device or (dtype is not None and t.dtype != dtype):
+            raise RuntimeError(("fp32 " if dtype == torch.float32 else "") + "tensors on one GPU expected")
+
+
+def check_penalties(pen, shape, device) -> None:
+    """A penalty for every key of every head, where the kernels read it."""
+    if pen.device != device:
+        raise RuntimeError("fp32 tensors on one GPU expected")
+    if pen.numel() < shape[0] * shape[1] * shape[2]:
+        raise ValueError("key mask smaller than [B, L]")
+
+
 def taken_layout(t: "torch.Tensor") -> HeadLayout:
     """The layout of heads the strided entry points have to take."""
     lay = head_layout(t)

@@ -36,15 +36,15 @@ class _BlockBF16Function(torch.autograd.Function):
     @staticmethod
     def forward(ctx, query, key, value, mask, mat, module):
         m = module
+        shape = (m.batch_size, m.num_heads, m.seq_len, m.emb_dim)
+        _lib.check_heads(shape, query, key, value)
         _lib.use_current_stream(m, query.device)
         idx = m.csr_cache.get(mat, m.block_size)
-        shape = (m.batch_size, m.num_heads, m.seq_len, m.emb_dim)
-        if tuple(query.shape) != shape or tuple(key.shape) != shape or tuple(value.shape) != shape:
-            raise ValueError(f"query/key/value shapes {tuple(query.shape)} do not match the handle {shape}")
         dev = query.device
         pen = None
         if m.key_mask:
             pen = _penalty(mask, m, dev)
+            _lib.check_penalties(pen, shape, dev)
         pen_ptr = pen.data_ptr() if pen is not None else None
         lse = torch.empty((m.num_batches, m.seq_len), dtype=torch.float32, device=dev)
         # bf16 heads that are views of [B, L, H*d] projections (models/attention.py:136-139) are read in place and

@@ -36,17 +36,17 @@ class _BlockAttnFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, query, key, value, mask, mat, module):
         m = module
+        shape = m.head_shape
+        _lib.check_heads(shape, query, key, value, torch.float32)
         _lib.use_current_stream(m, query.device)
         idx = m.csr_cache.get(mat, m.block_size)
         nb_ = m.num_batches
-        shape = m.head_shape
-        if query.shape != shape:
-            raise ValueError(f"query shape {tuple(query.shape)} does not match the handle {shape}")
         dev = query.device
         p_flat = torch.empty(nb_ * idx.nnz, dtype=torch.float32, device=dev)
         pen_ptr = None
         if m.with_mask:
             pen = (1e6 * (1.0 - mask.repeat(1, m.num_heads))).to(torch.float32).contiguous()  # [B, H*L]
+            _lib.check_penalties(pen, shape, dev)
             pen_ptr = pen.data_ptr()
         lay = None
         if m.reads_views and not (query.is_contiguous() and key.is_contiguous() and value.is_contiguous()):

@@ -41,10 +41,9 @@ class _DenseAttnFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, query, key, value, mask, module):
         m = module
-        _lib.use_current_stream(m, query.device)
         B, H, L, d = m.batch_size, m.num_heads, m.seq_len, m.emb_dim
-        if tuple(query.shape) != (B, H, L, d):
-            raise ValueError(f"query shape {tuple(query.shape)} does not match the handle ({B}, {H}, {L}, {d})")
+        _lib.check_heads((B, H, L, d), query, key, value, torch.float32)
+        _lib.use_current_stream(m, query.device)
         dev = query.device
         ctx.strided = False
         if m.reads_views:
@@ -58,6 +57,7 @@ class _DenseAttnFunction(torch.autograd.Function):
             pen_ptr = None
             if m.with_mask:
                 pen = (1e6 * (1.0 - mask.repeat(1, H))).to(torch.float32).contiguous()
+                _lib.check_penalties(pen, (B, H, L), dev)
                 pen_ptr = pen.data_ptr()
             if m.emit_score_map and d == 32:
                 # models/model_transformer.py:136-137 averages the returned maps over batch and heads; the kernel
@@ -87,6 +87,7 @@ class _DenseAttnFunction(torch.autograd.Function):
         out_t = torch.empty((B, H, d, L), dtype=torch.float32, device=dev)
         if m.with_mask:
             pen = (1e6 * (1.0 - mask.repeat(1, H))).to(torch.float32).contiguous()
+            _lib.check_penalties(pen, (B, H, L), dev)
             m.attn_cpp.attn_forward(m.attn_handle, qt.data_ptr(), k.data_ptr(), vt.data_ptr(), pen.data_ptr(),
                                     attn.data_ptr(), out_t.data_ptr())
         else:

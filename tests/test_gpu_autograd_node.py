@@ -394,6 +394,30 @@ def test_modules_that_keep_their_outputs_are_collected(kind):
         assert freed() is None and _lib.core().spion_debug_handles() == alive
 
 
+@pytest.mark.parametrize("kind", ["sparse", "dense", "bf16"])
+def test_python_functions_refuse_other_types_and_masks(kind):
+    """Heads in another type (those of bf16 are converted), and masks short or on the host, which kernels would read past
+    their end."""
+    B, H, L, d = 2, 2, 64, 32
+    mod, (ones, *rest), destroy = _of_kind(kind, B, H, L, d)
+    function = _BlockBF16Function if kind == "bf16" else mod.attn_func
+    q, k, v, _ = _inputs(B, H, L, d, "contiguous", seed=2)
+    with torch.no_grad():
+        function.apply(q, k, v, ones, *rest, mod)
+        for heads in ((q.half(), k, v), (q, k, v.half())) if kind != "bf16" else ():
+            with pytest.raises(RuntimeError, match="fp32"):
+                function.apply(*heads, ones, *rest, mod)
+            with pytest.raises(RuntimeError, match="fp32"):
+                mod(*heads, ones, *rest)
+        with pytest.raises(ValueError, match="key mask"):
+            function.apply(q, k, v, ones[:1], *rest, mod)
+        with pytest.raises(RuntimeError, match="one GPU"):
+            function.apply(q, k, v, ones.cpu(), *rest, mod)
+        with pytest.raises(RuntimeError, match="one GPU"):
+            function.apply(q, k.cpu(), v, ones, *rest, mod)
+    destroy(mod.attn_handle)
+
+
 @pytest.mark.parametrize("python", [False, True])
 @pytest.mark.parametrize("kind", ["sparse", "bf16"])
 def test_saved_tensor_hooks_do_not_meet_the_index(kind, python):

@@ -6,6 +6,7 @@ import torch
 import spion_amd
 from spion_amd import _lib
 from spion_amd.attention import Attention
+from spion_amd.attention_blockbf16 import _BlockBF16Function
 
 needs_node = pytest.mark.skipif(_lib.autograd_node() is None, reason="SPION_PY_NODE=1")
 
@@ -39,6 +40,34 @@ def test_node_refuses_a_key_mask_that_is_too_small():
     with pytest.raises(ValueError, match="key mask"):
         _lib.autograd_node().sparse_attention(q, q, q, torch.zeros(2, 64), False, index, index, index, handle, 1, 2, True, 0)
     cpp.destroy(handle)
+
+
+@pytest.mark.parametrize("family", ["sparse", "dense", "dense_feature_major", "bf16"])
+@pytest.mark.parametrize("which", range(3))
+def test_python_functions_refuse_what_the_handle_does_not_fit(family, which):
+    """The Python functions, which take the calls that the compiled node leaves them and those under torch.jit.trace, check
+    query, key and value: a key or value of fewer rows, a host tensor."""
+    d, L = (64, 2080) if family == "dense_feature_major" else (32, 64)
+    cfg = _config(2, d, L)
+    mat, mask = torch.ones(2, 2), torch.ones(2, L)
+    if family == "bf16":
+        mod = spion_amd.BlockAttentionBF16(cfg)
+        call = lambda *heads: _BlockBF16Function.apply(*heads, mask, mat, mod)
+    elif family == "sparse":
+        cpp = Attention._blockcuda_compile_module()
+        mod = spion_amd.CUDABlockAttention(cfg, cpp, cpp.init(d, L, 4, 32))
+        call = lambda *heads: mod.attn_func.apply(*heads, mask, mat, mod)
+    else:
+        cpp = Attention._cuda_compile_module()
+        mod = spion_amd.CUDAAttention(cfg, cpp, cpp.init(d, L, 4))
+        assert mod.reads_views == (family == "dense")
+        call = lambda *heads: mod(*heads, mask)
+    heads = [torch.zeros(2, 2, L, d) for _ in range(3)]
+    with pytest.raises(RuntimeError, match="GPU expected"):
+        call(*heads)
+    heads[which] = heads[which][:, :, :32]
+    with pytest.raises(ValueError, match="does not match the handle"):
+        call(*heads)
 
 
 class _Unused:
