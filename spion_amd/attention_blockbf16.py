@@ -43,6 +43,8 @@ class _BlockBF16Function(torch.autograd.Function):
         dev = query.device
         pen = None
         if m.key_mask:
+            if mask.device != dev:
+                raise RuntimeError("fp32 tensors on one GPU expected")
             pen = _penalty(mask, m, dev)
             _lib.check_penalties(pen, shape, dev)
         pen_ptr = pen.data_ptr() if pen is not None else None
@@ -141,6 +143,8 @@ class BlockAttentionBF16(nn.Module):
         idx = self.csr_cache.get(mat, self.block_size)
         key_mask, is_mask = None, False
         if self.key_mask:
+            if mask.device != query.device:
+                raise RuntimeError("fp32 tensors on one GPU expected")
             is_mask = mask.dtype == torch.float32 and mask.is_cuda and mask.is_contiguous() and not mask.requires_grad \
                 and mask.shape == (self.batch_size, self.seq_len)
             key_mask = mask if is_mask else _penalty(mask, self, query.device)

@@ -289,8 +289,11 @@ Tensor key_penalty(const Tensor& mask, int64_t heads, int64_t stream) {
     check_library("attn_forward");
     return pen;
 }
-// The modules hand over a key mask, or penalties made from one the kernel does not take (is_mask = false).
-c10::optional<Tensor> penalty_of(const c10::optional<Tensor>& mask_or_pen, bool is_mask, int64_t heads, int64_t stream) {
+// The modules hand over a key mask, or penalties made from one the kernel does not take (is_mask = false); either has to lie
+// on the device of the heads.
+c10::optional<Tensor> penalty_of(const c10::optional<Tensor>& mask_or_pen, bool is_mask, int64_t heads, c10::Device device,
+                                 int64_t stream) {
+    TORCH_CHECK(!mask_or_pen.has_value() || mask_or_pen->device() == device, "fp32 tensors on one GPU expected");
     if (!is_mask || !mask_or_pen.has_value()) return mask_or_pen;
     if (has_tangent(*mask_or_pen)) return (1e6 * (1.0 - mask_or_pen->repeat({1, heads}))).contiguous();
     return key_penalty(*mask_or_pen, heads, stream);
@@ -677,12 +680,12 @@ std::vector<Tensor> sparse_layer(const Tensor& x, const Tensor& wq, const Tensor
     // the penalties of a plain key mask come out of the projections' launch
     KeyMask keys;
     c10::optional<Tensor> pen;
-    if (is_mask && mask_or_pen.has_value() && !has_tangent(*mask_or_pen)) {
+    if (is_mask && mask_or_pen.has_value() && mask_or_pen->device() == x.device() && !has_tangent(*mask_or_pen)) {
         const Tensor& mask = *mask_or_pen;
         pen = torch::empty({mask.size(0), num_heads * mask.size(1)}, mask.options());
         keys = {fp(mask), fpm(*pen), (int)mask.size(0), (int)num_heads, (int)mask.size(1)};
     } else {
-        pen = penalty_of(mask_or_pen, is_mask, num_heads, stream);
+        pen = penalty_of(mask_or_pen, is_mask, num_heads, x.device(), stream);
     }
     const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
     if (without_node({&x, &wq, &wk, &wv, &bq, &bk, &bv, &wf, &bf, &pen_or_none})) {
@@ -715,7 +718,7 @@ std::vector<Tensor> sparse_attention(const Tensor& query, const Tensor& key, con
                                      const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t num_heads,
                                      bool reads_views, int64_t stream) {
     const c10::DeviceGuard on(query.device());
-    const auto pen = penalty_of(mask_or_pen, is_mask, num_heads, stream);
+    const auto pen = penalty_of(mask_or_pen, is_mask, num_heads, query.device(), stream);
     const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
     if (without_node({&query, &key, &value, &pen_or_none})) {
         const CoreResult r = core_forward(query, key, value, pen_or_none, offsets, columns, sum_mat, handle, nnz,
@@ -742,7 +745,7 @@ std::vector<Tensor> dense_attention(const Tensor& query, const Tensor& key, cons
                                     const c10::optional<Tensor>& mask_or_pen, bool is_mask, int64_t handle, bool emit_mean,
                                     int64_t stream) {
     const c10::DeviceGuard on(query.device());
-    const auto pen = penalty_of(mask_or_pen, is_mask, query.size(1), stream);
+    const auto pen = penalty_of(mask_or_pen, is_mask, query.size(1), query.device(), stream);
     const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
     check_penalties(pen_or_none, query);
     if (without_node({&query, &key, &value, &pen_or_none})) {
@@ -759,7 +762,7 @@ Tensor bf16_attention(const Tensor& query, const Tensor& key, const Tensor& valu
                       bool is_mask, const Tensor& offsets, const Tensor& columns, const Tensor& sum_mat, int64_t handle,
                       int64_t nnz, int64_t stream) {
     const c10::DeviceGuard on(query.device());
-    const auto pen = penalty_of(mask_or_pen, is_mask, query.size(1), stream);
+    const auto pen = penalty_of(mask_or_pen, is_mask, query.size(1), query.device(), stream);
     const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
     check_penalties(pen_or_none, query);
     if (without_node({&query, &key, &value, &pen_or_none}))

@@ -42,6 +42,21 @@ def test_node_refuses_a_key_mask_that_is_too_small():
     cpp.destroy(handle)
 
 
+@needs_node
+@pytest.mark.parametrize("is_mask", [True, False])
+def test_node_refuses_a_key_mask_on_another_device(is_mask):
+    """(No handle is looked at before.)"""
+    node, q, index = _lib.autograd_node(), torch.zeros(2, 2, 64, 32), torch.zeros(4, dtype=torch.int32)
+    mask = torch.zeros(2, 64, device="meta")
+    weights = [torch.zeros(64, 64)] * 3 + [torch.zeros(64)] * 3 + [torch.zeros(64, 64), torch.zeros(64)]
+    for call in (lambda: node.sparse_attention(q, q, q, mask, is_mask, index, index, index, 0, 1, 2, True, 0),
+                 lambda: node.dense_attention(q, q, q, mask, is_mask, 0, False, 0),
+                 lambda: node.bf16_attention(q, q, q, mask, is_mask, index, index, index, 0, 1, 0),
+                 lambda: node.sparse_layer(torch.zeros(2, 64, 64), *weights, mask, is_mask, index, index, index, 0, 1, 2, 32, 0)):
+        with pytest.raises(RuntimeError, match="one GPU"):
+            call()
+
+
 @pytest.mark.parametrize("family", ["sparse", "dense", "dense_feature_major", "bf16"])
 @pytest.mark.parametrize("which", range(3))
 def test_python_functions_refuse_what_the_handle_does_not_fit(family, which):
