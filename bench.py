@@ -45,9 +45,10 @@ def _matrix_ceiling(split, chains, algorithmic=2):
 
 
 # (split, fp32) products per tile of forward, row pass and column pass (spion_amd/csrc/tile_kernels.h, mma_feat_init, says why);
-# the dense forward in its register-resident form, the dense backward with shared tiles (dense_group_kernels.h)
+# the dense forward in its register-resident form, the dense backward with shared tiles (dense_group_kernels.h) and without
 _TILE_PRODUCTS = {32: ((1, 1), (1, 1), (3, 0)), 64: ((2, 0), (2, 0), (0, 3))}
-_DENSE_PRODUCTS = {32: ((1, 1), (2, 0), (3, 0)), 64: ((2, 0), (2, 0), (3, 0))}
+_DENSE_PRODUCTS = {(32, True): ((1, 1), (2, 0), (3, 0)), (64, True): ((2, 0), (2, 0), (3, 0)),
+                   (32, False): ((1, 1), (2, 0), (1, 2)), (64, False): ((2, 0), (2, 0), (0, 3))}
 
 
 def _floors_ms(flops, ceiling, nbytes):
@@ -530,8 +531,9 @@ def bench_dense_phase(args, dev, d=32):
     _lib.check_error("dense backward")
     alg_flops = 12.0 * L * L * d * NB
     k_fwd = "dense_fwd_reg_kernel" if d == 32 else "dense_fwd_reg64_kernel"
-    k_bwd = "dense_group_row_kernel + dense_group_col_kernel"
-    ceil_fwd, ceil_row, ceil_col = (_matrix_ceiling(*p) for p in _DENSE_PRODUCTS[d])
+    shared = core.spion_debug_dense_groups(handle) == 1
+    k_bwd = "dense_group_row_kernel + dense_group_col_kernel" if shared else f"dense_bwd_row{d}_kernel + dense_bwd_col{d}_kernel"
+    ceil_fwd, ceil_row, ceil_col = (_matrix_ceiling(*p) for p in _DENSE_PRODUCTS[d, shared])
     map_bytes, third = 4.0 * NB * L * L, alg_flops / 3.0  # each kernel writes or reads the map once
     roof = _roof_of(k_fwd, t_fwd_rm, third, ceil_fwd, map_bytes + 16.0 * NB * L * d)
     roof["frac"] = roof["achieved"] / roof["peak"]

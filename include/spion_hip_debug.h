@@ -24,6 +24,10 @@ void spion_set_backward_passes(void* handle, int mask);
  * graph recorded before the growth still points at them).  -1 otherwise. */
 int spion_debug_counter(void* handle, int which);
 
+/* Whether the backward of row-major heads of a dense handle runs as work-groups that share their tiles on the current
+ * device (1), or with four wavefronts to a strip (0); -1 for other handles. */
+int spion_debug_dense_groups(void* handle);
+
 /* Handles of all families that have not been freed (destroyed ones that are still held, spion_hold, are among them). */
 int spion_debug_handles(void);
 

@@ -111,6 +111,7 @@ void dense_destroy(void*);
 void dense_forward(void*, const float*, const float*, const float*, const float*, float*, float*, bool);
 void dense_backward(void*, const float*, const float*, const float*, const float*, const float*, float*, float*,
                     float*);
+int dense_groups(void*);
 int pattern_generate(const float*, int, int, int, int, int, double, float*, float*, float*, hipStream_t);
 int project_forward(const float*, const float* const*, const float* const*, float*, long long, int, int, int, const float*, float*, int,
                     int, int, hipStream_t);
@@ -385,6 +386,7 @@ int spion_last_path(void* h) { return sparse_last_path(h); }
 int spion_block_sizes(void* h, int* d, int* L, int* NB) { return sparse_sizes(h, d, L, NB); }
 void spion_force_element_path(void* h, int on) { sparse_force_element(h, on); }
 void spion_set_backward_passes(void* h, int mask) { sparse_set_bwd_passes(h, mask); }
+int spion_debug_dense_groups(void* h) { return dense_groups(h); }
 int spion_debug_counter(void* h, int which) { return sparse_debug_counter(h, which); }
 int spion_debug_bf16_plan(const int* tile_ptr, int nstrips, int pairs, int num_batches, int lanes, int* items,
                           int cap_items, int* lane_ptr, int cap_ptr, int* lane_ent, int cap_ent, int* longs,

@@ -1555,6 +1555,11 @@ static bool dense_groups_fill(const DenseAttn* a) {
     return filling >= (a->d == 32 ? 0.64 : 0.44);
 }
 
+int dense_groups(void* h) {
+    const DenseAttn* a = as_dense(h, "spion_debug_dense_groups");
+    return a ? (int)dense_groups_fill(a) : -1;
+}
+
 void dense_backward_strided(void* h, const float* Q, const float* K, const float* V, const float* P, const float* Out,
                             const float* dO, float* dQ, float* dK, float* dV, int heads, const HeadLayout& in,
                             const HeadLayout& out, const HeadLayout& grad) {
