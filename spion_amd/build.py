@@ -40,7 +40,8 @@ def _run(cmd, verbose):
 
 
 def build_autograd_node(verbose: bool = False) -> str:
-    """csrc/autograd_node.cpp -> lib/_spion_node.so: host code against libtorch and libspion_hip.so (g++, no HIP)."""
+    """csrc/autograd_node.cpp -> lib/_spion_node.so: host code against libtorch and libspion_hip.so (g++, no HIP code; the HIP
+    headers are for torch's current stream)."""
     import sysconfig
 
     import torch
@@ -48,13 +49,14 @@ def build_autograd_node(verbose: bool = False) -> str:
 
     out = os.path.join(LIB, "_spion_node.so")
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DTORCH_EXTENSION_NAME=_spion_node",
-           "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
-    for inc in cpp_extension.include_paths() + [sysconfig.get_paths()["include"]]:
+           "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-D__HIP_PLATFORM_AMD__=1"]
+    for inc in cpp_extension.include_paths(device_type="cuda") + [sysconfig.get_paths()["include"]]:
         cmd += ["-isystem", inc]
     cmd += [os.path.join(CSRC, "autograd_node.cpp"), "-o", out, f"-L{LIB}", "-lspion_hip", "-Wl,-rpath,$ORIGIN"]
     for d in cpp_extension.library_paths():
         cmd += [f"-L{d}", f"-Wl,-rpath,{d}"]
-    cmd += ["-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
+    cmd += ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
     _run(cmd, verbose)
     return out
 

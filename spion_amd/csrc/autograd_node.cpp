@@ -8,6 +8,7 @@
 // and strided entry points declared in include/spion_hip.h.  The Python function stays the statement of the
 // behaviour; tests run both and compare.
 #include <ATen/FuncTorchTLS.h>
+#include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
 #include <stdexcept>
@@ -74,6 +75,12 @@ bool without_node(std::initializer_list<const Tensor*> inputs) {
     for (const Tensor* t : inputs)
         if (has_tangent(*t)) return false;
     return true;
+}
+
+// The stream a backward is launched on: the calling thread's, which the tensors it makes belong to as well.  The engine puts
+// a node's backward on the stream of its forward; compiled autograd, and a caller of the node itself, do not.
+int64_t current_stream(int64_t device) {
+    return reinterpret_cast<int64_t>(c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream());
 }
 
 // What a node keeps of the handle its backward works on, which a program may destroy before, for instance with the module
@@ -199,10 +206,9 @@ CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& va
 }
 
 struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
-    // pen_opt: [B, H*L] key penalties of the key-mask modules, or nothing.  stream: torch's current raw
-    // stream at the call; autograd runs the backward of a node on the stream its forward ran on.  fixed: takes what
-    // carries no gradient, the probabilities of the key-mask modules (compiled autograd refuses nodes with outputs that
-    // are marked so).
+    // pen_opt: [B, H*L] key penalties of the key-mask modules, or nothing.  stream: torch's current raw stream at the
+    // call.  fixed: takes what carries no gradient, the probabilities of the key-mask modules (compiled autograd refuses
+    // nodes with outputs that are marked so).
     static variable_list forward(AutogradContext* ctx, Tensor query, Tensor key, Tensor value,
                                  c10::optional<Tensor> pen_opt, Tensor offsets, Tensor columns, Tensor sum_mat, int64_t handle, int64_t nnz,
                                  int64_t num_heads, bool reads_views, int64_t stream, Tensor* fixed) {
@@ -215,7 +221,6 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
         ctx->saved_data["nnz"] = nnz;
         ctx->saved_data["heads"] = num_heads;
         ctx->saved_data["strided"] = r.strided;
-        ctx->saved_data["stream"] = stream;
         keep_index(ctx, offsets, columns, sum_mat);
         keep_sizes(ctx, r.q);
         ctx->save_for_backward({r.q, r.k, r.v, r.p_flat, r.out});
@@ -235,7 +240,7 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
         saved.inputs(torch::kFloat32, q, k, v);
         const Tensor p_flat = saved.values(3, nnz);
         const int heads = (int)ctx->saved_data["heads"].toInt();
-        spion_set_stream(h, reinterpret_cast<void*>(ctx->saved_data["stream"].toInt()));
+        spion_set_stream(h, reinterpret_cast<void*>(current_stream(q.device().index())));
         const auto opt = q.options();
         Tensor go = grads[0];
         if (!go.defined()) go = torch::zeros(q.sizes(), opt);  // only the probabilities were used downstream
@@ -342,7 +347,6 @@ struct DenseAttnNode : public torch::autograd::Function<DenseAttnNode> {
                                  int64_t handle, bool emit_mean, int64_t stream, Tensor* mean) {
         DenseResult r = dense_forward(query, key, value, pen.has_value() ? *pen : Tensor(), handle, emit_mean, stream);
         keep_handle(ctx, handle);
-        ctx->saved_data["stream"] = stream;
         keep_sizes(ctx, r.q);
         ctx->save_for_backward({r.q, r.k, r.v, r.attn, r.out});
         ctx->set_materialize_grads(false);  // the gradient of the returned map is ignored (as in the reference)
@@ -355,7 +359,7 @@ struct DenseAttnNode : public torch::autograd::Function<DenseAttnNode> {
         saved.inputs(torch::kFloat32, q, k, v);
         const Tensor attn = saved.values(3, q.size(2) * q.size(2)), out = saved.heads(4, torch::kFloat32);
         void* h = reinterpret_cast<void*>(ctx->saved_data["handle"].toInt());
-        spion_set_stream(h, reinterpret_cast<void*>(ctx->saved_data["stream"].toInt()));
+        spion_set_stream(h, reinterpret_cast<void*>(current_stream(q.device().index())));
         const auto opt = q.options();
         const Tensor go = grads[0].defined() ? grad_like(grads[0], out) : torch::zeros_like(out);
         Tensor dq, dk, dv;
@@ -428,7 +432,6 @@ struct BF16AttnNode : public torch::autograd::Function<BF16AttnNode> {
         const BF16Result r = bf16_forward(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, stream);
         keep_handle(ctx, handle);
         ctx->saved_data["nnz"] = nnz;
-        ctx->saved_data["stream"] = stream;
         ctx->saved_data["strided"] = r.strided;
         keep_index(ctx, offsets, columns, sum_mat);
         keep_sizes(ctx, r.q);
@@ -444,7 +447,7 @@ struct BF16AttnNode : public torch::autograd::Function<BF16AttnNode> {
         const Tensor lse = saved.values(4, q.size(2)), pen = saved.saved[5].defined() ? saved.values(5, q.size(2)) : Tensor();
         void* h = reinterpret_cast<void*>(ctx->saved_data["handle"].toInt());
         const int nnz = (int)ctx->saved_data["nnz"].toInt();
-        spion_set_stream(h, reinterpret_cast<void*>(ctx->saved_data["stream"].toInt()));
+        spion_set_stream(h, reinterpret_cast<void*>(current_stream(q.device().index())));
         Tensor dq, dk, dv;
         if (ctx->saved_data["strided"].toBool()) {
             const Tensor go = grad_like(grads[0], out);
@@ -564,13 +567,12 @@ struct QkvNode : public torch::autograd::Function<QkvNode> {
         ctx->saved_data["d"] = d;
         ctx->saved_data["x_sizes"] = x.sizes().vec();
         ctx->saved_data["device"] = static_cast<int64_t>(x.device().index());
-        ctx->saved_data["stream"] = stream;
         return qkv_forward(aligned(x), w, b, H, d, stream, keys);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
         const int64_t H = ctx->saved_data["H"].toInt(), d = ctx->saved_data["d"].toInt(), n = H * d,
-                      stream = ctx->saved_data["stream"].toInt(), device = ctx->saved_data["device"].toInt();
+                      device = ctx->saved_data["device"].toInt(), stream = current_stream(device);
         const auto sizes = ctx->saved_data["x_sizes"].toIntVector();
         const int64_t B = sizes[0], L = sizes[1], dim = sizes[2], rows = B * L;
         saved_as(saved[0], sizes, device);
@@ -637,12 +639,11 @@ struct MergeNode : public torch::autograd::Function<MergeNode> {
         ctx->saved_data["heads_sizes"] = heads.sizes().vec();
         ctx->saved_data["outputs"] = w.size(0);
         ctx->saved_data["device"] = static_cast<int64_t>(heads.device().index());
-        ctx->saved_data["stream"] = stream;
         return merge_forward(aligned(heads.transpose(1, 2)), aligned(w), aligned(b), stream);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
-        const int64_t stream = ctx->saved_data["stream"].toInt(), device = ctx->saved_data["device"].toInt();
+        const int64_t device = ctx->saved_data["device"].toInt(), stream = current_stream(device);
         const auto sizes = ctx->saved_data["heads_sizes"].toIntVector();
         const int64_t B = sizes[0], H = sizes[1], L = sizes[2], d = sizes[3];
         const int64_t rows = B * L, n = H * d, dim = ctx->saved_data["outputs"].toInt();

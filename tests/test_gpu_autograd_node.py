@@ -374,6 +374,44 @@ def test_compiled_autograd_takes_the_nodes(kind):
         destroy(mod.attn_handle)
 
 
+@pytest.mark.parametrize("kind", ["sparse", "dense", "bf16", "layer"])
+def test_backward_runs_on_the_callers_stream(kind):
+    """A forward on a side stream, its node called on another, where the gradient is only just being made (by the node itself;
+    for the layer's three nodes by compiled autograd, which does not go back to the forward's stream either)."""
+    from torch._dynamo import compiled_autograd
+
+    if _lib.autograd_node() is None:
+        pytest.skip("SPION_PY_NODE=1")
+    B, H, L, d = 2, 2, 64, 32
+    dtype = torch.bfloat16 if kind == "bf16" else torch.float32
+    *leaves, do = (t.to(dtype) for t in _inputs(B, H, L, d, "contiguous", seed=3))
+    destroy = None
+    if kind == "layer":
+        mod, rest = _layer(B, H, L, d), (torch.ones(B, L, device="cuda"), torch.ones(2, 2, device="cuda"))
+        leaves, do = [leaves[0].transpose(1, 2).reshape(B, L, H * d)], do.transpose(1, 2).reshape(B, L, H * d)
+    else:
+        mod, rest, destroy = _of_kind(kind, B, H, L, d)
+    leaves = [t.requires_grad_() for t in leaves]
+    want = torch.autograd.grad(mod(*leaves, *rest)[0], leaves, do)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        out = mod(*leaves, *rest)[0]
+    torch.cuda.synchronize()
+    late = torch.full_like(do, float("nan"))
+    torch.cuda._sleep(20_000_000)
+    late.copy_(do)
+    if kind == "layer":
+        with compiled_autograd._enable(torch.compile(backend="eager")):
+            out.backward(late)
+        got = [t.grad for t in leaves]
+    else:
+        got = out.grad_fn(late, None) if kind == "dense" else out.grad_fn(late)
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
+    if destroy:
+        destroy(mod.attn_handle)
+
+
 @pytest.mark.parametrize("kind", ["sparse", "dense", "bf16"])
 def test_modules_that_keep_their_outputs_are_collected(kind):
     import gc
