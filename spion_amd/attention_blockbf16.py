@@ -159,8 +159,8 @@ class BlockAttentionBF16(nn.Module):
 
     def _node_takes(self, query, key, value):
         """Whether the compiled node (csrc/autograd_node.cpp) makes this call: the steps of ``_BlockBF16Function``, for heads of
-        the handle's sizes; anything else is that function's, with its errors.  8 heads of 1728 tokens, which the host bounds:
-        training step 121 -> 83 us, forward with key padding 25 -> 16."""
+        the handle's sizes; anything else is that function's, with its errors.  8 heads of 1728 tokens, which the host bounds,
+        with a mask whose index is on file: training step 121 -> 83 us, forward with key padding 25 -> 16; a new mask adds its analysis, 1.1 ms."""
         shape = (self.batch_size, self.num_heads, self.seq_len, self.emb_dim)
         device = query.device
         return device.type == "cuda" and _lib.plain_autograd() and all(

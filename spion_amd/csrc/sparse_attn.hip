@@ -630,11 +630,12 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
     if (out.items.empty()) out.items.assign(4, 0);
     // deal: per die, every item to the lane of that die with the least work so far; the chunks of all heads first, then the
     // strips head after head.  (With a head's chunks among its strips the last head's came last, onto lanes that were full:
-    // up to 1.3 of the average work.  A lane still takes its items head after head.)  Kernels of a step in us, head after
-    // head / chunks first: 32 heads of 16384 554 / 520, 32 of 4096, forward alone, 42.2 / 38.5, 83 of 5600 428 / 420, 30 of 9952, d
-    // = 32, 363 / 318, 10 of 6144 160 / 142; half as long chunks: 2 % less to 20 % more.  Launches of up to two items a lane
-    // whose heads are not dealt to dies: all items longest first, 131 for the 10 of 6144, 36 of 3072, d = 32, 96 / 85; with more
-    // items, or a die's own heads, the lanes drift apart in heads and lose the K and V in L2 (562, 40.2, 425, 337).
+    // up to 1.3 of the average work.  A lane still takes its items head after head.)  Steps in us, one box, head after
+    // head / chunks first / all items longest first: 32 heads of 16384, blocks of 64, 3.7 % kept, 562 / 538 / 564; 32 of 4096, 8 %,
+    // forward alone, 40.3 / 37.5 / 39.3; 83 of 5600, blocks of 32, 5 %, 493 / 482 / 507; 30 of 9952, d = 32, blocks of 32, 5 %, 225 /
+    // 214 / 219.  Longest first, the lanes drift apart in heads and lose the K and V in L2; it is taken where that costs nothing,
+    // in launches of up to two items a lane whose heads are not dealt to dies: 10 of 6144, blocks of 64, 6 %, 103.5 / - / 91.9;
+    // 36 of 3072, d = 32, blocks of 64, 8 %, 95.8 / - / 87.6.  Half as long chunks: 2 % less to 20 % more.
     const int per_group = lanes / groups, heads_per_group = NB / groups;
     const bool mixed = groups == 1 && (long long)its.size() * NB <= 2LL * lanes;
     std::vector<std::vector<std::pair<int, int>>> lane_list(lanes);  // {head, item}
