@@ -22,7 +22,7 @@ DROPINS = {1: "attn.so", 2: "attn_mask.so", 3: "block_attn.so", 4: "block_attn_m
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = [
     "-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC",
-    # packed-fp32 instruction selection is switched off on purpose for this hardware pool
+    # packed-fp32 instruction selection is switched off on purpose for this hardware
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]

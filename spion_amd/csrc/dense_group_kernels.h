@@ -12,7 +12,7 @@
 // Accuracy: a wavefront's sum over all tiles would round twelve times a tile at the size of the whole sum (2-norm errors of
 // dQ, dK, dV against float64 5.0e-7 at 1024 queries), so a tile's product is summed by itself and added: 1.7e-7 to 1.9e-7, where
 // four wavefronts with a quarter of the tiles each gave 2.9e-7 to 3.2e-7.
-// Measured, us per launch in a training loop, without / with sharing, one box: d = 32, 64 x 2 heads of 1024: row pass 157 /
+// Measured, us per launch in a training loop, without / with sharing, one machine: d = 32, 64 x 2 heads of 1024: row pass 157 /
 // 123, column pass 208 / 169; 16 x 2 of 2048: 150 / 123, 204 / 173; d = 64, 64 x 2 of 1024: 260 / 208, 457 / 286.
 // Bound (d = 32, 64 x 2 of 1024, counters): column pass, matrix pipe 59 % and vector ALU 57 % busy (36 and 281 instructions
 // a tile) at 1.81 GHz, which is the power limit (the kernels without sharing run at 2.03); row pass, 4.9 TB/s of the map

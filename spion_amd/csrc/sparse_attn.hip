@@ -630,7 +630,7 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
     if (out.items.empty()) out.items.assign(4, 0);
     // deal: per die, every item to the lane of that die with the least work so far; the chunks of all heads first, then the
     // strips head after head.  (With a head's chunks among its strips the last head's came last, onto lanes that were full:
-    // up to 1.3 of the average work.  A lane still takes its items head after head.)  Steps in us, one box, head after
+    // up to 1.3 of the average work.  A lane still takes its items head after head.)  Steps in us, one machine, head after
     // head / chunks first / all items longest first: 32 heads of 16384, blocks of 64, 3.7 % kept, 562 / 538 / 564; 32 of 4096, 8 %,
     // forward alone, 40.3 / 37.5 / 39.3; 83 of 5600, blocks of 32, 5 %, 493 / 482 / 507; 30 of 9952, d = 32, blocks of 32, 5 %, 225 /
     // 214 / 219.  Longest first, the lanes drift apart in heads and lose the K and V in L2; it is taken where that costs nothing,

@@ -1,4 +1,4 @@
-"""Parity of the bf16 sparse-attention kernels with the float64 oracle, through the C ABI (GPU box only).
+"""Parity of the bf16 sparse-attention kernels with the float64 oracle, through the C ABI (on a GPU only).
 
 The oracle runs on the bf16-rounded inputs in float64.  Tolerance for the bf16 outputs and gradients, 1e-2
 relative, read for tensors whose every element carries the 2^-9 rounding of the bf16 result itself (measured

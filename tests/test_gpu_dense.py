@@ -1,4 +1,4 @@
-"""Parity of the dense-phase HIP kernels with the float64 oracle, through the C ABI (GPU box only)."""
+"""Parity of the dense-phase HIP kernels with the float64 oracle, through the C ABI (on a GPU only)."""
 import numpy as np
 import pytest
 import torch

@@ -1,5 +1,5 @@
 """The dense backward whose work-groups share their tiles (launches that fill the machine) against float64, and where
-elements are infinite, NaN or at the ends of the range (GPU box only)."""
+elements are infinite, NaN or at the ends of the range (on a GPU only)."""
 import pytest
 import torch
 

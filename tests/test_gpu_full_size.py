@@ -1,4 +1,4 @@
-"""Benchmark configurations 3 and 4, and configuration 5's shape in fp32, at their full sizes (GPU box only).
+"""Benchmark configurations 3 and 4, and configuration 5's shape in fp32, at their full sizes (on a GPU only).
 
 The float64 oracle cannot run a whole batch of these sizes in seconds, so each case combines (a) the oracle on a
 bounded part of the very tensors the full-size launch produced (two of the 64 heads; four of the 256 samples) with

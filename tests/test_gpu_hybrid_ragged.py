@@ -1,5 +1,5 @@
 """The remainder kernels that hold their gathered operands in LDS, at lengths that are no multiple of their work-groups or
-ranges (rows, columns and keys past the end), against float64 on some of the heads (GPU box only)."""
+ranges (rows, columns and keys past the end), against float64 on some of the heads (on a GPU only)."""
 import pytest
 import torch
 

@@ -1,4 +1,4 @@
-"""Mask persistence and the inference path (GPU box only): masks written the way the reference writes them
+"""Mask persistence and the inference path (on a GPU only): masks written the way the reference writes them
 (a plain pickle of the [4, layers, nb, nb] tensor as it lies on the GPU, main_conv_ff.py:298-306) are loaded into a
 fresh model, every layer gets its prebuilt index registered with the library, and the timed evaluation loop of
 main_inference.py:49-93 runs over a few batches; losses, accuracy and one backward are compared with the same

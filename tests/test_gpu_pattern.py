@@ -1,4 +1,4 @@
-"""Pattern discovery kernels vs the oracle: pooled maps to 1 ulp-level, masks bit-exact (GPU box only)."""
+"""Pattern discovery kernels vs the oracle: pooled maps to 1 ulp-level, masks bit-exact (on a GPU only)."""
 import json
 import os
 

@@ -1,5 +1,5 @@
 """The library's per-handle cache of analysed patterns and of kept forward outputs, keyed by device addresses:
-eviction, address reuse, registration from host arrays (GPU box only)."""
+eviction, address reuse, registration from host arrays (on a GPU only)."""
 import ctypes
 
 import numpy as np

@@ -1,4 +1,4 @@
-"""Projection kernels (spion_project_*) and the layer that runs on them, against float64 (GPU box only)."""
+"""Projection kernels (spion_project_*) and the layer that runs on them, against float64 (on a GPU only)."""
 import ctypes
 
 import pytest

@@ -1,4 +1,4 @@
-"""Parity of the sparse-attention HIP kernels with the float64 oracle, through the C ABI (GPU box only).
+"""Parity of the sparse-attention HIP kernels with the float64 oracle, through the C ABI (on a GPU only).
 
 Tolerance: fp32 results within 1e-4 relative (see abi_utils.assert_close).
 """

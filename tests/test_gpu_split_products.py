@@ -1,5 +1,5 @@
 """The fp32 tile kernels' products on the bf16 matrix pipe (operands split into three parts), against float64 with
-bounds that scale with the operands (GPU box only)."""
+bounds that scale with the operands (on a GPU only)."""
 import numpy as np
 import pytest
 import torch

@@ -1,5 +1,5 @@
 """spion_attn_backward_noalloc (the entry point that allocates nothing) against spion_attn_backward_rowmajor, bit
-for bit, through the C ABI: two calls in a row, the second on a smaller problem (GPU box only); argument checks
+for bit, through the C ABI: two calls in a row, the second on a smaller problem (on a GPU only); argument checks
 (no GPU needed)."""
 import numpy as np
 import pytest
