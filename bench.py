@@ -64,19 +64,11 @@ def _roof_of(kernel, ms, flops, ceiling, nbytes):
     return dict(bound=bound, kernel=kernel, achieved=work, peak=peak, unit=unit, traffic=None)
 
 
-def _hybrid_lds_kernels(L, NB):
-    """Which of the remainder's kernels take their operands from LDS (the library's rule: how full the work-groups, one per CU
-    and round, leave the machine): logits, P.V, column pass."""
-    if L < 1024 or "SPION_HYB_GATHER" in os.environ:
-        return False, False, False
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-
-    def filling(per):
-        rounds = -(-NB * -(-L // per) // cus)
-        return NB * L / (cus * per * rounds)
-
-    return (filling(512) >= 0.78, filling(1024) >= 0.95,
-            max(filling(128 * n) * n / (n + 0.25) for n in (8, 4, 2)) > 0.6)
+def _remainder_in_lds(L, NB):
+    """Whether the remainder's kernels of the hybrid path take their operands from LDS (the library's rule)."""
+    if L < 512 or L > 1 << 18 or "SPION_HYB_GATHER" in os.environ:
+        return False
+    return NB * -(-L // 256) * 4 >= torch.cuda.get_device_properties(0).multi_processor_count
 
 
 def _event_ms(fn, iters, warm=3):
@@ -803,13 +795,14 @@ def bench_sparse_layer(args, dev, workload, full=True):
     alg_flops = workloads.sparse_flops(nnz, d, NB)
     alg_bytes = workloads.sparse_bytes(nnz, L, d, NB)
     third = alg_flops / 3.0  # forward, row pass and column pass carry 4*n*d*NB each
-    lds = ["_lds" if x else "" for x in _hybrid_lds_kernels(L, NB)]
     names = {1: ("tile_fwd_kernel", "tile_bwd_row_kernel", "tile_bwd_col_kernel"),
              2: ("elem_fwd_kernel", "elem_bwd_row_kernel", "elem_bwd_col_kernel"),
              # hybrid: dense window tiles on the MFMA units + gathered remainder; each phase is two or three launches
-             3: (f"hyb_rem_logits{lds[0]}_kernel + hyb_tile_fwd_kernel + hyb_rem_pv{lds[1]}_kernel",
+             3: ("rem_fwd_kernel + hyb_tile_fwd_kernel", "hyb_tile_bwd_row_kernel + rem_bwd_row_kernel",
+                 "hyb_tile_bwd_col_kernel + rem_bwd_col_kernel") if _remainder_in_lds(L, NB) else
+                ("hyb_rem_logits_kernel + hyb_tile_fwd_kernel + hyb_rem_pv_kernel",
                  "hyb_tile_bwd_row_kernel + hyb_rem_bwd_row_kernel",
-                 f"hyb_tile_bwd_col_kernel + hyb_rem_bwd_col{lds[2]}_kernel")}[path]
+                 "hyb_tile_bwd_col_kernel + hyb_rem_bwd_col_kernel")}[path]
     kernels = dict(zip(names, (t_fwd, t_row, t_col)))
     dom = max(kernels, key=kernels.get)
     dom_ms = kernels[dom]

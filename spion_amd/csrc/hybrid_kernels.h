@@ -19,7 +19,7 @@
 #pragma once
 #include <type_traits>
 #include "gather_ops.h"
-#include "tile_kernels.h"
+#include "remainder_kernels.h"
 
 namespace spion {
 
@@ -56,7 +56,6 @@ constexpr int HYB_MAXT1 = 6;    // dense tiles whose logits a single wavefront k
 constexpr int HYB_MAXT4 = 4;    // the same per wavefront when four share a strip
 constexpr int HYB_MAX_ROW_TILES = 4 * HYB_MAXT4;
 constexpr int HYB_GWAVES = 4;    // wavefronts (rows / columns) per work-group of the gather kernels
-constexpr float HYB_ABSENT = -1.0e30f;  // logit of an entry that is not in the pattern: exp2 gives exactly 0
 // two wavefronts per SIMD, each with the next tile's operands in flight while it works on one
 #define SPION_HYB_KERNEL(W) __global__ __launch_bounds__(64 * (W)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 
@@ -119,9 +118,11 @@ __device__ __forceinline__ void hyb_store_p_cols(float* __restrict__ Ph, const i
 // Sum of the wavefronts' 32 x 32 accumulators (rows acc_row(r, h) of the strip, columns li) times `factor`, in a
 // fixed order, to rows of stride ld.  `lds` (WAVES * 1024 floats, unused for one wavefront) may alias tile space no wavefront uses any
 // more: the caller has a barrier between that use and this call.
-template <int WAVES>
+// ADD: plus add[r] (the same in every wavefront); copy (optional): the result once more, rows of 32.
+template <int WAVES, bool ADD = false>
 __device__ __forceinline__ void hyb_reduce_store(const f32x16& acc, float factor, float* __restrict__ out, int ld,
-                                                 int row0, int w, int li, int h, float* __restrict__ lds) {
+                                                 int row0, int w, int li, int h, float* __restrict__ lds,
+                                                 const float* add = nullptr, float* __restrict__ copy = nullptr) {
     const int l = h * 32 + li;
     if constexpr (WAVES > 1) {
 #pragma unroll
@@ -138,7 +139,10 @@ __device__ __forceinline__ void hyb_reduce_store(const f32x16& acc, float factor
             for (int ww = 0; ww < WAVES; ++ww) s += lds[(ww * 16 + r) * 64 + l];
         }
         s *= factor;
+        if constexpr (ADD) s += add[r];
         out[(size_t)(row0 + acc_row(r, h)) * ld + li] = s;
+        if constexpr (ADD)
+            if (copy) copy[(size_t)(row0 + acc_row(r, h)) * 32 + li] = s;
     }
 }
 
@@ -247,12 +251,14 @@ SPION_HYB_GATHER_KERNEL void hyb_rem_logits_kernel(const float* __restrict__ Q, 
 // maximum, 1 / denominator} for step 3).  Writes the tiles' probabilities to their CSR positions and O = P.V of the
 // tile part (step 3 adds the remainder's share).
 // -------------------------------------------------------------------------------------------------
-template <bool MASK, int WAVES, int MAXT, bool ST>
+// REM: the remainder went through rem_fwd_kernel: O holds its sums relative to its own maximum, which are rescaled and
+// added (Oc, optional: second copy of O, contiguous heads).
+template <bool MASK, int WAVES, int MAXT, bool ST, bool REM>
 SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, const float* __restrict__ K,
                                           const float* __restrict__ V, const float* __restrict__ pen,
-                                          float* __restrict__ P, float* __restrict__ O, float2* __restrict__ Stats,
-                                          const int* __restrict__ offs, HybIndex ix, int L, int nbr, int NB, int nnz,
-                                          float scale, Layouts ly) {
+                                          float* __restrict__ P, float* __restrict__ O, float* __restrict__ Oc,
+                                          float2* __restrict__ Stats, const int* __restrict__ offs, HybIndex ix, int L,
+                                          int nbr, int NB, int nnz, float scale, Layouts ly) {
     constexpr int D = 32, KH = 16;
     __shared__ float lds_m[WAVES][32], lds_z[WAVES][32];
     __shared__ __attribute__((aligned(16))) float lds_t[WAVES][64 * TS];  // two 32-row tiles per wavefront
@@ -404,10 +410,22 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
         }
         __builtin_amdgcn_sched_barrier(0);
     }
+    float add[16];
+    if constexpr (REM) {
+        const float share = __builtin_amdgcn_exp2f(rem.x - Mx) * zinv;  // of the remainder's own sums
+        int sh[16];
+        hyb_rows_from_lanes(X, l, h, __float_as_int(share), sh);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            if (WAVES > 1 && (r % WAVES) != w) continue;  // the registers this wavefront stores
+            add[r] = O[ob + (size_t)(I * 32 + acc_row(r, h)) * old_ + li] * __int_as_float(sh[r]);
+        }
+    }
     if constexpr (WAVES > 1) __syncthreads();
     // every wavefront has consumed the remainder's statistics by now: replace them by the row's final ones
     if (w == 0 && h == 0) Stats[(size_t)bh * L + I * 32 + li] = make_float2(Mx, zinv);
-    hyb_reduce_store<WAVES>(o[0], 1.0f, O + ob, old_, I * 32, w, li, h, lds);
+    hyb_reduce_store<WAVES, REM>(o[0], 1.0f, O + ob, old_, I * 32, w, li, h, lds, add,
+                                 REM && Oc ? Oc + (size_t)bh * L * D : nullptr);
 }
 
 // -------------------------------------------------------------------------------------------------
@@ -728,14 +746,14 @@ __global__ __launch_bounds__(64 * HYB_GWAVES) void hyb_rem_bwd_col_kernel(  // t
 }
 
 // -------------------------------------------------------------------------------------------------
-// The same pass with the gathered operands in LDS instead of L2.  A work-group of sixteen wavefronts owns 128 * NC
-// columns of a head and walks the sequence in ranges of HYB_CL_ROWS rows, whose Q and dO rows (128 KB) it loads
-// once per range.  A group of eight lanes owns NC columns (lane s holds floats 4s .. 4s+3 of their dK and dV rows,
-// 8 * NC accumulator registers that live across the ranges) and walks each column's entries -- rows ascending, so the
-// entries of a range are the next ones of the column's list -- eight at a time: lane s fetches the s-th entry's row
-// and {dS, P} pair with full-width loads, the eight are handed round the group, and every lane adds its 16-byte
-// pieces of the Q and dO rows, read from LDS, to its sums.  Each lane's sums run in a fixed order along the column's
-// list, so the result does not depend on the launch.
+// The element path's column pass (all entries of a pattern, d = 32) with the gathered operands in LDS instead of L2.  A
+// work-group of sixteen wavefronts owns 128 * NC columns of a head and walks the sequence in ranges of HYB_CL_ROWS rows,
+// whose Q and dO rows (128 KB) it loads once per range.  A group of eight lanes owns NC columns (lane s holds floats
+// 4s .. 4s+3 of their dK and dV rows, 8 * NC accumulator registers that live across the ranges) and walks each column's
+// entries -- rows ascending, so the entries of a range are the next ones of the column's list -- eight at a time: lane s
+// fetches the s-th entry's row, dS and P, the eight are handed round the group, and every lane adds its 16-byte pieces of
+// the Q and dO rows, read from LDS, to its sums.  Each lane's sums run in a fixed order along the column's list, so the
+// result does not depend on the launch.
 // -------------------------------------------------------------------------------------------------
 constexpr int HYB_CL_ROWS = 512, HYB_CL_THREADS = 1024;  // a work-group owns NC * 128 columns: 1024 (NC = 8) or 512
 // x of another lane of the same row of sixteen: quad_perm (CTRL = 0x55 * k: lane k of the own quad) or row_half_mirror
@@ -745,12 +763,11 @@ __device__ __forceinline__ int hyb_dpp(int x) {
     return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, false);
 }
 // The list of a column: entries c_ptr[j] .. c_ptr[j+1]-1, their rows c_row (ascending) and c_src, the index of the
-// entry's weights -- PAIRS: in the compact {dS, P} list of a head ([NB][n] float2; the sums are added to what the tile
-// part left in dK and dV); otherwise in the head's dS and P arrays ([NB][n] floats each; the sums are the result).
-template <bool ST, bool PAIRS, int NC>
-__global__ __launch_bounds__(HYB_CL_THREADS) void hyb_rem_bwd_col_lds_kernel(
-    const float* __restrict__ Q, const float* __restrict__ dO, const float2* __restrict__ Pairs,
-    const float* __restrict__ dSa, const float* __restrict__ Pa, float* __restrict__ dK, float* __restrict__ dV,
+// entry's weights in the head's dS and P arrays ([NB][n] floats each).
+template <bool ST, int NC>
+__global__ __launch_bounds__(HYB_CL_THREADS) void elem_bwd_col_lds_kernel(
+    const float* __restrict__ Q, const float* __restrict__ dO, const float* __restrict__ dSa,
+    const float* __restrict__ Pa, float* __restrict__ dK, float* __restrict__ dV,
     const int* __restrict__ c_ptr, const int* __restrict__ c_row, const int* __restrict__ c_src, int n, int L, int NB,
     Layouts ly) {
     __shared__ f32x4 sq[HYB_CL_ROWS * 8], so[HYB_CL_ROWS * 8];
@@ -764,10 +781,8 @@ __global__ __launch_bounds__(HYB_CL_THREADS) void hyb_rem_bwd_col_lds_kernel(
     hyb_head<ST>(ly.in, ly.H, bh, L, ib, ild);
     hyb_head<ST>(ly.out, ly.H, bh, L, ob, old_);
     hyb_head<ST>(ly.grad, ly.H, bh, L, gb, gld);
-    const float2* pairs = PAIRS ? Pairs + (size_t)bh * n : nullptr;
-    const float* dsh = PAIRS ? nullptr : dSa + (size_t)bh * n;
-    const float* ph = PAIRS ? nullptr : Pa + (size_t)bh * n;
-    auto weights = [&](int src) { return PAIRS ? pairs[src] : (float2){dsh[src], ph[src]}; };
+    const float* dsh = dSa + (size_t)bh * n;
+    const float* ph = Pa + (size_t)bh * n;
     f32x4 ak[NC], av[NC];
     int e[NC], eend[NC];
 #pragma unroll
@@ -826,7 +841,7 @@ __global__ __launch_bounds__(HYB_CL_THREADS) void hyb_rem_bwd_col_lds_kernel(
                 const bool in = r1 < rend;
                 nn = __popcll((__ballot(in) >> (lane & 56)) & 0xffull);
                 if (nn == 0) break;
-                add_batch(c, in ? r1 - r0 : 0, in ? weights(s1) : (float2){0.f, 0.f});
+                add_batch(c, in ? r1 - r0 : 0, in ? (float2){dsh[s1], ph[s1]} : (float2){0.f, 0.f});
                 e[c] += nn;
             }
         }
@@ -837,215 +852,8 @@ __global__ __launch_bounds__(HYB_CL_THREADS) void hyb_rem_bwd_col_lds_kernel(
         if (col >= L) continue;
         f32x4* kr = reinterpret_cast<f32x4*>(dK + gb + (size_t)col * gld) + sub;
         f32x4* vr = reinterpret_cast<f32x4*>(dV + gb + (size_t)col * gld) + sub;
-        if constexpr (PAIRS) {
-            if (eend[c] == c_ptr[col]) continue;  // a column without remainder entries
-            *kr = *kr + ak[c];
-            *vr = *vr + av[c];
-        } else {
-            *kr = ak[c];
-            *vr = av[c];
-        }
-    }
-}
-
-// -------------------------------------------------------------------------------------------------
-// Forward, step 1, with the K rows in LDS: a work-group of sixteen wavefronts owns 128 * NR query rows of a head and
-// walks the keys in ranges of HYB_LL_KEYS, whose K rows (128 KB; with a key mask their penalties too) it loads once
-// per range.  A group of eight lanes owns NR rows (their scaled Q rows -- lane i of either quad holds pieces i and
-// i + 4 -- and their running {maximum, sum}) and walks each row's remainder entries eight at a time, lane s fetching
-// the s-th entry's column; then either quad of the group takes the four entries its own lanes hold, one after the
-// other: the column goes round the quad by a DPP move, every lane multiplies its two pieces of the K row, read from
-// LDS, two DPP additions make the dot product, and the lane that holds the entry keeps it.  The eight logits are
-// stored, and the row's statistics follow batch by batch (maximum raised, sum rescaled).
-// -------------------------------------------------------------------------------------------------
-constexpr int HYB_LL_KEYS = 1024, HYB_LL_THREADS = 1024;
-template <bool MASK, bool ST, int NR>
-__global__ __launch_bounds__(HYB_LL_THREADS) void hyb_rem_logits_lds_kernel(
-    const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ pen, float* __restrict__ Raw,
-    float2* __restrict__ Stats, HybIndex ix, int L, int NB, float scale, Layouts ly) {
-    __shared__ f32x4 sk[HYB_LL_KEYS * 8];
-    __shared__ float spen[MASK ? HYB_LL_KEYS : 1];
-    constexpr int ROWS = NR * (HYB_LL_THREADS / 8);
-    const int nrg = (L + ROWS - 1) / ROWS;  // the last one's rows past the end have no entries
-    const int item = xcd_remap((int)blockIdx.x, (int)gridDim.x);  // the work-groups of a head share an XCD's L2
-    const int bh = item / nrg, rg = item % nrg;
-    const int t = threadIdx.x, grp = t >> 3, sub = t & 7, qi = t & 3, lane = t & 63;
-    size_t ib;
-    int ild;
-    hyb_head<ST>(ly.in, ly.H, bh, L, ib, ild);
-    float* raw = Raw + (size_t)bh * ix.nr;
-    const float c2 = scale * LOG2E;
-    f32x4 q0[NR], q1[NR];
-    float m[NR], z[NR];
-    int e[NR], eend[NR];
-#pragma unroll
-    for (int c = 0; c < NR; ++c) {
-        const int row = rg * ROWS + c * (HYB_LL_THREADS / 8) + grp;
-        const f32x4* qr = reinterpret_cast<const f32x4*>(Q + ib + (size_t)min(row, L - 1) * ild);
-        q0[c] = qr[qi] * c2;
-        q1[c] = qr[4 + qi] * c2;
-        m[c] = HYB_ABSENT;
-        z[c] = 0.f;
-        e[c] = row < L ? ix.r_off[row] : 0;
-        eend[c] = row < L ? ix.r_off[row + 1] : 0;
-    }
-    auto fdpp = [](auto ctrl, float x) {
-        return __int_as_float(hyb_dpp<decltype(ctrl)::value>(__float_as_int(x)));
-    };
-    for (int k0 = 0; k0 < L; k0 += HYB_LL_KEYS) {
-        __syncthreads();  // everybody has finished with the previous range
-#pragma unroll
-        for (int k = 0; k < HYB_LL_KEYS * 8 / HYB_LL_THREADS; ++k) {
-            const int idx = t + k * HYB_LL_THREADS;
-            sk[idx] = reinterpret_cast<const f32x4*>(K + ib + (size_t)min(k0 + (idx >> 3), L - 1) * ild)[idx & 7];
-        }
-        if constexpr (MASK) spen[t] = pen[(size_t)bh * L + min(k0 + t, L - 1)] * LOG2E;
-        __syncthreads();
-        const int kend = k0 + HYB_LL_KEYS;
-#pragma unroll
-        for (int c = 0; c < NR; ++c) {
-            int nn = 8;
-            while (nn == 8) {
-                const int my = e[c] + sub;
-                const int col = my < eend[c] ? ix.r_col[my] : 0x7fffffff;
-                const bool in = col < kend;
-                // columns ascend along the list: the entries of this range among the eight are the first nn
-                nn = __popcll((__ballot(in) >> (lane & 56)) & 0xffull);
-                if (nn == 0) break;
-                const int lcol = in ? col - k0 : 0;
-                float v = 0.f;
-#define SPION_HYB_QUAD_STEP(KQ)                                                                       \
-    {                                                                                                 \
-        const int ck = hyb_dpp<0x55 * KQ>(lcol);                                                      \
-        const f32x4 a0 = sk[ck * 8 + qi], a1 = sk[ck * 8 + 4 + qi];                                   \
-        float d = a0.x * q0[c].x;                                                                     \
-        d = fmaf(a0.y, q0[c].y, d);                                                                   \
-        d = fmaf(a0.z, q0[c].z, d);                                                                   \
-        d = fmaf(a0.w, q0[c].w, d);                                                                   \
-        d = fmaf(a1.x, q1[c].x, d);                                                                   \
-        d = fmaf(a1.y, q1[c].y, d);                                                                   \
-        d = fmaf(a1.z, q1[c].z, d);                                                                   \
-        d = fmaf(a1.w, q1[c].w, d);                                                                   \
-        d += fdpp(std::integral_constant<int, 0xB1>{}, d);                                            \
-        d += fdpp(std::integral_constant<int, 0x4E>{}, d);                                            \
-        if constexpr (MASK) d -= spen[ck];                                                            \
-        v = qi == KQ ? d : v;                                                                         \
-    }
-                SPION_HYB_QUAD_STEP(0)
-                SPION_HYB_QUAD_STEP(1)
-                SPION_HYB_QUAD_STEP(2)
-                SPION_HYB_QUAD_STEP(3)
-#undef SPION_HYB_QUAD_STEP
-                if (in) raw[my] = v;
-                else v = HYB_ABSENT;
-                float bm = v;
-                bm = fmaxf(bm, fdpp(std::integral_constant<int, 0xB1>{}, bm));
-                bm = fmaxf(bm, fdpp(std::integral_constant<int, 0x4E>{}, bm));
-                bm = fmaxf(bm, fdpp(std::integral_constant<int, 0x141>{}, bm));
-                const float mnew = fmaxf(m[c], bm);
-                float ex = __builtin_amdgcn_exp2f(v - mnew);  // an absent entry gives exactly 0
-                ex += fdpp(std::integral_constant<int, 0xB1>{}, ex);
-                ex += fdpp(std::integral_constant<int, 0x4E>{}, ex);
-                ex += fdpp(std::integral_constant<int, 0x141>{}, ex);
-                z[c] = z[c] * __builtin_amdgcn_exp2f(m[c] - mnew) + ex;
-                m[c] = mnew;
-                e[c] += nn;
-            }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < NR; ++c) {
-        const int row = rg * ROWS + c * (HYB_LL_THREADS / 8) + grp;
-        if (sub == 0 && row < L) Stats[(size_t)bh * L + row] = make_float2(m[c], z[c]);
-    }
-}
-
-// -------------------------------------------------------------------------------------------------
-// Forward, step 3, with the V rows in LDS: a work-group of sixteen wavefronts owns 1024 query rows of a head and walks
-// the keys in ranges of 1024, whose V rows (128 KB) it loads once per range.  A group of eight lanes owns eight rows
-// (their {maximum, 1 / denominator} and lane s's 16 bytes of their O rows in registers) and walks each row's remainder
-// entries eight at a time: lane s fetches the s-th entry's raw logit, column and position and writes its probability
-// (through the cache: a row's probabilities leave in pieces of at most eight as the ranges go by), the eight
-// {column, probability} go round the group as in the column pass above.
-// -------------------------------------------------------------------------------------------------
-constexpr int HYB_RL_ROWS = 1024, HYB_RL_KEYS = 1024, HYB_RL_THREADS = 1024;
-template <bool ST>
-__global__ __launch_bounds__(HYB_RL_THREADS) void hyb_rem_pv_lds_kernel(
-    const float* __restrict__ V, const float* __restrict__ Raw, float* __restrict__ P, float* __restrict__ O,
-    float* __restrict__ Ocache, const float2* __restrict__ Stats, HybIndex ix, int L, int NB, int nnz, Layouts ly) {
-    __shared__ f32x4 sv[HYB_RL_KEYS * 8];
-    const int nrg = (L + HYB_RL_ROWS - 1) / HYB_RL_ROWS;  // the last one's rows past the end have no entries
-    const int item = xcd_remap((int)blockIdx.x, (int)gridDim.x);  // the work-groups of a head share an XCD's L2
-    const int bh = item / nrg, rg = item % nrg;
-    const int t = threadIdx.x, grp = t >> 3, sub = t & 7, lane = t & 63;
-    size_t ib, ob;
-    int ild, old_;
-    hyb_head<ST>(ly.in, ly.H, bh, L, ib, ild);
-    hyb_head<ST>(ly.out, ly.H, bh, L, ob, old_);
-    float* Ph = P + (size_t)bh * nnz;
-    const float* raw = Raw + (size_t)bh * ix.nr;
-    constexpr int NR = HYB_RL_ROWS / (HYB_RL_THREADS / 8);  // rows per lane group: 8
-    f32x4 acc[NR];
-    float2 st[NR];
-    int e[NR], eend[NR];
-#pragma unroll
-    for (int c = 0; c < NR; ++c) {
-        const int row = rg * HYB_RL_ROWS + c * (HYB_RL_THREADS / 8) + grp;
-        acc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        st[c] = Stats[(size_t)bh * L + min(row, L - 1)];
-        e[c] = row < L ? ix.r_off[row] : 0;
-        eend[c] = row < L ? ix.r_off[row + 1] : 0;
-    }
-    for (int k0 = 0; k0 < L; k0 += HYB_RL_KEYS) {
-        __syncthreads();  // everybody has finished with the previous range
-#pragma unroll
-        for (int k = 0; k < HYB_RL_KEYS * 8 / HYB_RL_THREADS; ++k) {
-            const int idx = t + k * HYB_RL_THREADS;
-            sv[idx] = reinterpret_cast<const f32x4*>(V + ib + (size_t)min(k0 + (idx >> 3), L - 1) * ild)[idx & 7];
-        }
-        __syncthreads();
-        const int kend = k0 + HYB_RL_KEYS;
-#pragma unroll
-        for (int c = 0; c < NR; ++c) {
-            int nn = 8;
-            while (nn == 8) {
-                const int my = e[c] + sub;
-                const int col = my < eend[c] ? ix.r_col[my] : 0x7fffffff;
-                const bool in = col < kend;
-                // columns ascend along the list: the entries of this range among the eight are the first nn
-                nn = __popcll((__ballot(in) >> (lane & 56)) & 0xffull);
-                if (nn == 0) break;
-                float wgt = 0.f;
-                int lcol = 0;
-                if (in) {
-                    wgt = __builtin_amdgcn_exp2f(raw[my] - st[c].x) * st[c].y;
-                    Ph[ix.r_pos[my]] = wgt;
-                    lcol = col - k0;
-                }
-                const int wx = __float_as_int(wgt);
-                const int mcol = hyb_dpp<0x141>(lcol), mx = hyb_dpp<0x141>(wx);
-#define SPION_HYB_ENTRY(CTRL, C, X) acc[c] += sv[hyb_dpp<CTRL>(C) * 8 + sub] * __int_as_float(hyb_dpp<CTRL>(X));
-                SPION_HYB_ENTRY(0x00, lcol, wx)
-                SPION_HYB_ENTRY(0x55, lcol, wx)
-                SPION_HYB_ENTRY(0xaa, lcol, wx)
-                SPION_HYB_ENTRY(0xff, lcol, wx)
-                SPION_HYB_ENTRY(0x00, mcol, mx)
-                SPION_HYB_ENTRY(0x55, mcol, mx)
-                SPION_HYB_ENTRY(0xaa, mcol, mx)
-                SPION_HYB_ENTRY(0xff, mcol, mx)
-#undef SPION_HYB_ENTRY
-                e[c] += nn;
-            }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < NR; ++c) {
-        const int row = rg * HYB_RL_ROWS + c * (HYB_RL_THREADS / 8) + grp;
-        if (row >= L || eend[c] == ix.r_off[row]) continue;  // a row without remainder entries
-        f32x4* orow = reinterpret_cast<f32x4*>(O + ob + (size_t)row * old_) + sub;
-        const f32x4 sum = *orow + acc[c];
-        *orow = sum;
-        if (Ocache) reinterpret_cast<f32x4*>(Ocache + ((size_t)bh * L + row) * 32)[sub] = sum;  // own copy: contiguous
+        *kr = ak[c];
+        *vr = av[c];
     }
 }
 

@@ -424,6 +424,8 @@ struct PatternIndex {
     bool hybrid = false;
     int hyb_tiles = 0, hyb_nr = 0;
     HybIndex hyb{};
+    bool rem_lds = false;  // the remainder's kernels keep its rows in LDS (remainder_kernels.h); `rem` instead of hyb's lists
+    RemIndex rem{};
     void release() {
         if (d_blob) (void)hipFree(d_blob);
         *this = PatternIndex();
@@ -681,6 +683,20 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
 static int bf16_lanes() {
     if (const char* env = getenv("SPION_BF16_LANES")) return std::min(std::max(1, atoi(env)), 1 << 16);
     return device_cus() * 8;
+}
+
+// Whether the remainder of an element pattern keeps its rows in LDS (remainder_kernels.h), lists by ranges instead of by
+// whole rows and columns; SPION_HYB_GATHER: never.  With a quarter of the machine's compute units at work the two are level
+// (16 heads of 1024 with 17 remainder entries a row: forward 12 us against 17 gathered from L2, row pass 12 / 11, column pass
+// 13 / 14), with more the gathers are behind everywhere (32 of 1024 with 27: 18 / 28, 17 / 21, 17 / 26; 16 of 4096 with 80:
+// 53 / 93, 55 / 76, 50 / 93).  A list's word holds the position in a row of the pattern in 18 bits.
+static bool rem_gather_forced() {
+    static const bool gather = getenv("SPION_HYB_GATHER") != nullptr;
+    return gather;
+}
+static bool rem_in_lds(const SparseAttn* a) {
+    return !rem_gather_forced() && a->L >= REM_RANGE && a->L <= (1 << 18) &&
+           (long long)a->NB * ((a->L + REM_QUADS - 1) / REM_QUADS) * 4 >= device_cus();
 }
 
 // Copy the index to the host once (unless the caller hands over host copies), validate it, detect the tile
@@ -946,10 +962,36 @@ static bool analyse_pattern(SparseAttn* a, const int* Offsets, const int* Column
                 }
                 std::vector<int> t_ci(t_ct.size());
                 for (size_t e = 0; e < t_ct.size(); ++e) t_ci[e] = t_row[t_ct[e]];
-                std::vector<int> c_ptr(L + 1, 0), c_row(std::max(nr, 1), 0), c_src(std::max(nr, 1), 0);
-                for (int e = 0; e < nr; ++e) c_ptr[r_col[e] + 1]++;
-                for (int j = 0; j < L; ++j) c_ptr[j + 1] += c_ptr[j];
-                {
+                pi.rem_lds = rem_in_lds(a);
+                if (pi.rem_lds) {
+                    // by ranges of REM_RANGE columns, then rows, columns ascending; and by ranges of rows, then columns
+                    const int nk = (L + REM_RANGE - 1) / REM_RANGE;
+                    std::vector<int> rb_off((size_t)nk * L + 1, 0), cb_off((size_t)nk * L + 1, 0);
+                    std::vector<int> rb_word(nr + REM_BATCH, 0), cb_word(nr + REM_BATCH, 0), fill;
+                    for (int i = 0; i < L; ++i)
+                        for (int e = r_off[i]; e < r_off[i + 1]; ++e) {
+                            rb_off[(size_t)(r_col[e] / REM_RANGE) * L + i + 1]++;
+                            cb_off[(size_t)(i / REM_RANGE) * L + r_col[e] + 1]++;
+                        }
+                    for (size_t x = 1; x < rb_off.size(); ++x) rb_off[x] += rb_off[x - 1];
+                    for (size_t x = 1; x < cb_off.size(); ++x) cb_off[x] += cb_off[x - 1];
+                    std::vector<int> cfill(cb_off.begin(), cb_off.end() - 1);
+                    fill.assign(rb_off.begin(), rb_off.end() - 1);
+                    for (int i = 0; i < L; ++i)
+                        for (int e = r_off[i]; e < r_off[i + 1]; ++e) {
+                            const int J = r_col[e] / REM_RANGE, R = i / REM_RANGE, x = fill[(size_t)J * L + i]++;
+                            rb_word[x] = (r_col[e] % REM_RANGE) | (i % 32) << 9 | (int)((unsigned)(r_pos[e] - off[i]) << 14);
+                            cb_word[cfill[(size_t)R * L + r_col[e]]++] =
+                                (i % REM_RANGE) | (x - rb_off[(size_t)J * L + (size_t)R * REM_RANGE]) << 9;
+                        }
+                    hyb_off[7] = append(rb_off);
+                    hyb_off[8] = append(rb_word);
+                    hyb_off[9] = append(cb_off);
+                    hyb_off[10] = append(cb_word);
+                } else {
+                    std::vector<int> c_ptr(L + 1, 0), c_row(std::max(nr, 1), 0), c_src(std::max(nr, 1), 0);
+                    for (int e = 0; e < nr; ++e) c_ptr[r_col[e] + 1]++;
+                    for (int j = 0; j < L; ++j) c_ptr[j + 1] += c_ptr[j];
                     std::vector<int> fill(c_ptr.begin(), c_ptr.end() - 1);
                     for (int i = 0; i < L; ++i)  // rows ascend: every column's entries end up ordered by row
                         for (int e = r_off[i]; e < r_off[i + 1]; ++e) {
@@ -957,10 +999,16 @@ static bool analyse_pattern(SparseAttn* a, const int* Offsets, const int* Column
                             c_row[x] = i;
                             c_src[x] = e;
                         }
-                }
-                if (r_col.empty()) {
-                    r_col.push_back(0);
-                    r_pos.push_back(0);
+                    if (r_col.empty()) {
+                        r_col.push_back(0);
+                        r_pos.push_back(0);
+                    }
+                    hyb_off[7] = append(r_off);
+                    hyb_off[8] = append(r_col);
+                    hyb_off[9] = append(r_pos);
+                    hyb_off[10] = append(c_ptr);
+                    hyb_off[11] = append(c_row);
+                    hyb_off[12] = append(c_src);
                 }
                 std::vector<int> bits_as_int(t_bits.size());
                 memcpy(bits_as_int.data(), t_bits.data(), t_bits.size() * sizeof(int));
@@ -970,12 +1018,6 @@ static bool analyse_pattern(SparseAttn* a, const int* Offsets, const int* Column
                 hyb_off[4] = append(bits_as_int);
                 hyb_off[5] = append(t_cp);
                 hyb_off[6] = append(t_ct);
-                hyb_off[7] = append(r_off);
-                hyb_off[8] = append(r_col);
-                hyb_off[9] = append(r_pos);
-                hyb_off[10] = append(c_ptr);
-                hyb_off[11] = append(c_row);
-                hyb_off[12] = append(c_src);
                 hyb_off[13] = append(t_ci);
                 pi.hyb_nr = nr;
                 pi.hybrid = true;
@@ -1029,6 +1071,8 @@ static bool analyse_pattern(SparseAttn* a, const int* Offsets, const int* Column
                               reinterpret_cast<const unsigned*>(b + hyb_off[4]), b + hyb_off[5], b + hyb_off[6],
                               b + hyb_off[13], b + hyb_off[7], b + hyb_off[8], b + hyb_off[9], b + hyb_off[10],
                               b + hyb_off[11], b + hyb_off[12], pi.hyb_nr, pi.hyb_tiles};
+            if (pi.rem_lds)
+                pi.rem = RemIndex{b + hyb_off[7], b + hyb_off[8], b + hyb_off[9], b + hyb_off[10], pi.hyb_nr};
         }
     }
     pi.tiled = tiled;
@@ -1422,23 +1466,19 @@ static void launch_tile_bwd(SparseAttn* a, const float* Q, const float* K, const
 #undef SPION_BY_WAVES
 }
 
-// The remainder's kernels with their gathered operands in LDS take one work-group of sixteen wavefronts per CU.  How full
-// a launch over work-groups of `per` rows or columns of a head keeps the machine: the rows over those its rounds of one
+// The element path's column pass with its gathered operands in LDS takes one work-group of sixteen wavefronts per CU.  How
+// full a launch over work-groups of `per` columns of a head keeps the machine: the columns over those its rounds of one
 // work-group per CU could take.
 static int hyb_groups(int L, int per) { return (L + per - 1) / per; }
 static double hyb_filling(const SparseAttn* a, int per) {
     const long long cus = device_cus(), rounds = ((long long)a->NB * hyb_groups(a->L, per) + cus - 1) / cus;
     return (double)a->NB * a->L / ((double)cus * per * rounds);
 }
-static bool hyb_lds_off(const SparseAttn* a) {
-    static const bool gather = getenv("SPION_HYB_GATHER") != nullptr;
-    return gather || a->L < 1024;
-}
-// Columns per lane group of the column pass (work-groups of 1024, 512 or 256 columns): the one that leaves the machine
-// fullest, a quarter of a column counted for the ranges every work-group loads; 0, the kernel that gathers from L2, below
-// 0.6 -- full against full the LDS form takes 0.54 of its time.
-static int hyb_lds_columns(const SparseAttn* a) {
-    if (hyb_lds_off(a)) return 0;
+// Columns per lane group (work-groups of 1024, 512 or 256 columns): the one that leaves the machine fullest, a quarter of a
+// column counted for the ranges every work-group loads; 0, the kernel that gathers from L2, below 0.6 -- full against full
+// the LDS form takes 0.54 of its time.
+static int elem_lds_columns(const SparseAttn* a) {
+    if (rem_gather_forced() || a->L < 1024) return 0;
     int best = 0;
     double most = 0.6;
     for (int nc = 8; nc >= 2; nc >>= 1) {
@@ -1450,13 +1490,19 @@ static int hyb_lds_columns(const SparseAttn* a) {
     }
     return best;
 }
-// The forward's logits: work-groups of 512 rows (four per lane group; eight need more registers than a wavefront of
-// sixteen has and are no faster); 0.77 of the gather kernel's time on a full machine.  Its P.V: 1024 rows, 0.95.
-static bool hyb_lds_rows(const SparseAttn* a) { return !hyb_lds_off(a) && hyb_filling(a, 512) >= 0.78; }
-static bool hyb_lds_pv(const SparseAttn* a) { return !hyb_lds_off(a) && hyb_filling(a, HYB_RL_ROWS) >= 0.95; }
-#define SPION_HYB_COL_LDS(ST_, PAIRS_, NC_, ...)                                                          \
-    hipLaunchKernelGGL((hyb_rem_bwd_col_lds_kernel<ST_, PAIRS_, NC_>), dim3(a->NB * hyb_groups(a->L, 128 * NC_)), \
+#define SPION_ELEM_COL_LDS(ST_, NC_, ...)                                                                       \
+    hipLaunchKernelGGL((elem_bwd_col_lds_kernel<ST_, NC_>), dim3(a->NB * hyb_groups(a->L, 128 * NC_)),          \
                        dim3(HYB_CL_THREADS), 0, a->hdr.stream, __VA_ARGS__)
+// Rows (columns) per quad of the remainder's kernels, work-groups of 256 or 512, one per CU and round: a round of the larger
+// ones takes 1.6 times one of the smaller (64 heads of 4096: two of 87 us against four of 54; 32 of 2048: 56 against 37 in all).
+static int rem_per_quad(const SparseAttn* a) {
+    const long long cus = device_cus();
+    const auto rounds = [&](int per) { return ((long long)a->NB * hyb_groups(a->L, per) + cus - 1) / cus; };
+    return 10 * rounds(REM_QUADS) > 16 * rounds(2 * REM_QUADS) ? 2 : 1;
+}
+#define SPION_REM_LAUNCH(KERNEL_, NO_, ...)                                                                                 \
+    hipLaunchKernelGGL((KERNEL_), dim3(a->NB * hyb_groups(a->L, (NO_) * REM_QUADS)), dim3(REM_THREADS), 0, a->hdr.stream, \
+                       __VA_ARGS__)
 
 // Hybrid patterns (dense tiles + remainder, d = 32).  Every operand row-major; ST: heads located by `ly`.
 // ocopy (contiguous heads only): where a second copy of O goes, or null.
@@ -1478,36 +1524,36 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
     const dim3 grid_t(nbr * a->NB), block_t(one ? 64 : 256);
     const dim3 grid_g((unsigned)((rows + HYB_GWAVES - 1) / HYB_GWAVES)), block_g(64 * HYB_GWAVES);
     float2* stats = reinterpret_cast<float2*>(a->ws_stats);
-    const bool lds_logits = hyb_lds_rows(a);
-#define SPION_HYB_LOGITS_LDS(MASKED, NR_)                                                                            \
-    hipLaunchKernelGGL((hyb_rem_logits_lds_kernel<MASKED, ST, NR_>), dim3(a->NB * hyb_groups(a->L, 128 * NR_)),             \
-                       dim3(HYB_LL_THREADS), 0, a->hdr.stream, Q, K, Mask, a->ws_raw, stats, a->pat.hyb, a->L, a->NB, \
-                       a->scale, ly)
+    const bool lds = a->pat.rem_lds, two = lds && rem_per_quad(a) == 2;
+#define SPION_HYB_TILES(MASKED, WAVES_, MAXT_, REM_)                                                                  \
+    hipLaunchKernelGGL((hyb_tile_fwd_kernel<MASKED, WAVES_, MAXT_, ST, REM_>), grid_t, block_t, 0, a->hdr.stream, Q,  \
+                       K, V, Mask, Attn, Out, REM_ ? ocopy : nullptr, stats, Offsets, a->pat.hyb, a->L, nbr, a->NB,   \
+                       nnz, a->scale, ly)
+#define SPION_REM_FWD(MASKED, NO_)                                                                                     \
+    SPION_REM_LAUNCH((rem_fwd_kernel<MASKED, ST, NO_>), NO_, Q, K, V, Mask, a->ws_raw, stats, Out, a->pat.rem, a->L, \
+                     a->NB, a->scale, ly)
 #define SPION_HYB_FWD(MASKED)                                                                                        \
     do {                                                                                                             \
-        if (lds_logits) SPION_HYB_LOGITS_LDS(MASKED, 4);                                                             \
+        if (two) SPION_REM_FWD(MASKED, 2);                                                                           \
+        else if (lds) SPION_REM_FWD(MASKED, 1);                                                                      \
         else                                                                                                         \
-        hipLaunchKernelGGL((hyb_rem_logits_kernel<MASKED, ST>), grid_g, block_g, 0, a->hdr.stream, Q, K, Mask,       \
-                           a->ws_raw, stats, a->pat.hyb, a->L, a->NB, a->scale, ly);                                 \
-        if (one)                                                                                                     \
-            hipLaunchKernelGGL((hyb_tile_fwd_kernel<MASKED, 1, HYB_MAXT1, ST>), grid_t, block_t, 0, a->hdr.stream,   \
-                               Q, K, V, Mask, Attn, Out, stats, Offsets, a->pat.hyb, a->L, nbr, a->NB, nnz,          \
-                               a->scale, ly);                                                                        \
-        else                                                                                                         \
-            hipLaunchKernelGGL((hyb_tile_fwd_kernel<MASKED, 4, HYB_MAXT4, ST>), grid_t, block_t, 0, a->hdr.stream,   \
-                               Q, K, V, Mask, Attn, Out, stats, Offsets, a->pat.hyb, a->L, nbr, a->NB, nnz,          \
-                               a->scale, ly);                                                                        \
+            hipLaunchKernelGGL((hyb_rem_logits_kernel<MASKED, ST>), grid_g, block_g, 0, a->hdr.stream, Q, K, Mask,   \
+                               a->ws_raw, stats, a->pat.hyb, a->L, a->NB, a->scale, ly);                             \
+        if (one && lds) SPION_HYB_TILES(MASKED, 1, HYB_MAXT1, true);                                                 \
+        else if (one) SPION_HYB_TILES(MASKED, 1, HYB_MAXT1, false);                                                  \
+        else if (lds) SPION_HYB_TILES(MASKED, 4, HYB_MAXT4, true);                                                   \
+        else SPION_HYB_TILES(MASKED, 4, HYB_MAXT4, false);                                                           \
     } while (0)
     if (a->has_mask)
         SPION_HYB_FWD(true);
     else
         SPION_HYB_FWD(false);
 #undef SPION_HYB_FWD
-#undef SPION_HYB_LOGITS_LDS
-    if (hyb_lds_pv(a))
-        hipLaunchKernelGGL(hyb_rem_pv_lds_kernel<ST>, dim3(a->NB * hyb_groups(a->L, HYB_RL_ROWS)), dim3(HYB_RL_THREADS), 0,
-                           a->hdr.stream, V, (const float*)a->ws_raw, Attn, Out, ocopy, (const float2*)stats, a->pat.hyb,
-                           a->L, a->NB, nnz, ly);
+#undef SPION_REM_FWD
+#undef SPION_HYB_TILES
+    if (lds)
+        hipLaunchKernelGGL(rem_prob_kernel, grid_t, dim3(REM_PROB_THREADS), 0, a->hdr.stream, (const float*)a->ws_raw, Attn,
+                           (const float2*)stats, Offsets, a->pat.rem, a->L, nbr, a->NB, nnz);
     else
         hipLaunchKernelGGL(hyb_rem_pv_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, V, (const float*)a->ws_raw, Attn,
                            Out, ocopy, (const float2*)stats, a->pat.hyb, a->L, a->NB, nnz, ly);
@@ -1518,8 +1564,8 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
 // {dS, P} pairs, [NB][nr] (a hybrid pattern keeps at most half of its entries in the remainder).
 template <bool ST>
 static void launch_hyb_bwd(SparseAttn* a, const float* Q, const float* K, const float* V, const float* P,
-                           const float* dO, const float* o, float* dS, float* dQ, float* dK, float* dV, int nnz,
-                           const Layouts& ly) {
+                           const float* dO, const float* o, float* dS, float* dQ, float* dK, float* dV,
+                           const int* Offsets, int nnz, const Layouts& ly) {
     PhaseRange phase("spion backward (hybrid kernels)");
     if (!ensure_ws(&a->ws_rowsum, (size_t)a->NB * a->L)) return;
     a->last_path = 3;
@@ -1529,6 +1575,7 @@ static void launch_hyb_bwd(SparseAttn* a, const float* Q, const float* K, const 
     const dim3 grid_t(nbr * a->NB);
     const dim3 grid_g((unsigned)((rows + HYB_GWAVES - 1) / HYB_GWAVES)), block_g(64 * HYB_GWAVES);
     float2* pairs = reinterpret_cast<float2*>(dS);
+    const bool lds = a->pat.rem_lds, two = lds && rem_per_quad(a) == 2;
     if (a->bwd_passes & 1) {
         if (one_r)
             hipLaunchKernelGGL((hyb_tile_bwd_row_kernel<1, ST>), grid_t, dim3(64), 0, a->hdr.stream, K, V, P, dO, o,
@@ -1536,8 +1583,15 @@ static void launch_hyb_bwd(SparseAttn* a, const float* Q, const float* K, const 
         else
             hipLaunchKernelGGL((hyb_tile_bwd_row_kernel<4, ST>), grid_t, dim3(256), 0, a->hdr.stream, K, V, P, dO, o,
                                a->ws_rowsum, dQ, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
-        hipLaunchKernelGGL(hyb_rem_bwd_row_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, K, V, P, dO,
-                           (const float*)a->ws_rowsum, pairs, dQ, a->pat.hyb, a->L, a->NB, nnz, a->scale, ly);
+#define SPION_REM_ROW(NO_)                                                                                            \
+    SPION_REM_LAUNCH((rem_bwd_row_kernel<ST, NO_>), NO_, K, V, P, dO, (const float*)a->ws_rowsum, pairs, dQ, Offsets, \
+                     a->pat.rem, a->L, a->NB, nnz, a->scale, ly)
+        if (two) SPION_REM_ROW(2);
+        else if (lds) SPION_REM_ROW(1);
+        else
+            hipLaunchKernelGGL(hyb_rem_bwd_row_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, K, V, P, dO,
+                               (const float*)a->ws_rowsum, pairs, dQ, a->pat.hyb, a->L, a->NB, nnz, a->scale, ly);
+#undef SPION_REM_ROW
     }
     if (a->bwd_passes & 2) {
         if (one_c)
@@ -1546,19 +1600,15 @@ static void launch_hyb_bwd(SparseAttn* a, const float* Q, const float* K, const 
         else
             hipLaunchKernelGGL((hyb_tile_bwd_col_kernel<4, ST>), grid_t, dim3(256), 0, a->hdr.stream, Q, V, P, dO,
                                (const float*)a->ws_rowsum, dK, dV, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
-        const int nc = hyb_lds_columns(a);
-        if (nc == 8)
-            SPION_HYB_COL_LDS(ST, true, 8, Q, dO, (const float2*)pairs, nullptr, nullptr, dK, dV, a->pat.hyb.c_ptr,
-                              a->pat.hyb.c_row, a->pat.hyb.c_src, a->pat.hyb.nr, a->L, a->NB, ly);
-        else if (nc == 4)
-            SPION_HYB_COL_LDS(ST, true, 4, Q, dO, (const float2*)pairs, nullptr, nullptr, dK, dV, a->pat.hyb.c_ptr,
-                              a->pat.hyb.c_row, a->pat.hyb.c_src, a->pat.hyb.nr, a->L, a->NB, ly);
-        else if (nc == 2)
-            SPION_HYB_COL_LDS(ST, true, 2, Q, dO, (const float2*)pairs, nullptr, nullptr, dK, dV, a->pat.hyb.c_ptr,
-                              a->pat.hyb.c_row, a->pat.hyb.c_src, a->pat.hyb.nr, a->L, a->NB, ly);
+#define SPION_REM_COL(NO_)                                                                                          \
+    SPION_REM_LAUNCH((rem_bwd_col_kernel<ST, NO_>), NO_, Q, dO, (const float2*)pairs, dK, dV, a->pat.rem, a->L, a->NB, \
+                     ly)
+        if (two) SPION_REM_COL(2);
+        else if (lds) SPION_REM_COL(1);
         else
             hipLaunchKernelGGL(hyb_rem_bwd_col_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, Q, dO,
                                (const float2*)pairs, dK, dV, a->pat.hyb, a->L, a->NB, ly);
+#undef SPION_REM_COL
     }
     check_launch("hyb_bwd kernels");
 }
@@ -1596,15 +1646,15 @@ static void launch_elem_bwd(SparseAttn* a, const float* Q, const float* K, const
                            dS, dQ, offs, cols, a->L, a->NB, nnz, a->scale, ly);
     if (a->bwd_passes & 2) {
         if constexpr (D == 32) {
-            const int nc = hyb_lds_columns(a);  // the Q and dO rows of a range of the sequence in LDS, see hybrid_kernels.h
+            const int nc = elem_lds_columns(a);  // the Q and dO rows of a range of the sequence in LDS, see hybrid_kernels.h
             if (nc == 8)
-                SPION_HYB_COL_LDS(ST, false, 8, Q, dO, nullptr, dS, P, dK, dV, pi.d_ccp, pi.d_crow, pi.d_cpos, nnz, a->L,
+                SPION_ELEM_COL_LDS(ST, 8, Q, dO, dS, P, dK, dV, pi.d_ccp, pi.d_crow, pi.d_cpos, nnz, a->L,
                                   a->NB, ly);
             else if (nc == 4)
-                SPION_HYB_COL_LDS(ST, false, 4, Q, dO, nullptr, dS, P, dK, dV, pi.d_ccp, pi.d_crow, pi.d_cpos, nnz, a->L,
+                SPION_ELEM_COL_LDS(ST, 4, Q, dO, dS, P, dK, dV, pi.d_ccp, pi.d_crow, pi.d_cpos, nnz, a->L,
                                   a->NB, ly);
             else if (nc == 2)
-                SPION_HYB_COL_LDS(ST, false, 2, Q, dO, nullptr, dS, P, dK, dV, pi.d_ccp, pi.d_crow, pi.d_cpos, nnz, a->L,
+                SPION_ELEM_COL_LDS(ST, 2, Q, dO, dS, P, dK, dV, pi.d_ccp, pi.d_crow, pi.d_cpos, nnz, a->L,
                                   a->NB, ly);
             if (nc) return;
         }
@@ -1729,7 +1779,7 @@ void sparse_backward(void* h, const float* Q, const float* K, const float* Vt, c
         // without it the gather kernels below serve the same P
         const float* o = Out ? Out : ocache_for_backward(a, P);
         if (o) {
-            launch_hyb_bwd<false>(a, Q, K, Vrm, P, dO, o, dS, dQ, dK, dV, nnz, Layouts{});
+            launch_hyb_bwd<false>(a, Q, K, Vrm, P, dO, o, dS, dQ, dK, dV, Offsets, nnz, Layouts{});
             return;
         }
     }
@@ -1958,7 +2008,7 @@ void sparse_backward_strided(void* h, const float* Q, const float* K, const floa
         // these entry points have no dS argument: the scratch is the handle's (grown outside graph capture only)
         if (!ensure_ws_grow(a, &a->ws_ds, &a->ws_ds_count, (size_t)a->NB * (size_t)std::max(nnz, 1), who)) return;
         if (a->pat.hybrid) {
-            launch_hyb_bwd<true>(a, Q, K, V, P, dO, Out, a->ws_ds, dQ, dK, dV, nnz, ly);
+            launch_hyb_bwd<true>(a, Q, K, V, P, dO, Out, a->ws_ds, dQ, dK, dV, Offsets, nnz, ly);
             return;
         }
         a->last_path = 2;

@@ -1,0 +1,106 @@
+"""The remainder kernels by ranges (remainder_kernels.h) at the edges of their ranges, batches and work-groups, against float64
+on some of the heads (on a GPU only)."""
+import pytest
+import torch
+
+import spion_amd
+from spion_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _pattern(L, gen):
+    """A window and a few random columns; row 7 and row L - 3 with many entries in one range (more than a batch), a column that
+    every third row has, an empty row, a column of the last range that no row has."""
+    i = torch.arange(L, device="cuda")
+    m = (torch.rand(L, L, generator=gen, device="cuda") < 14 / L).float()
+    m[(i[:, None] - i[None, :]).abs() <= 40] = 1.0
+    m[7, 1:500:3] = 1.0
+    m[L - 3, 100:500:7] = 1.0
+    m[::3, 450] = 1.0
+    m[5] = 0.0
+    m[:, L - 2] = 0.0
+    return m
+
+
+def _reference(q, k, v, do, pattern, valid):
+    q, k, v = (t.double().requires_grad_() for t in (q, k, v))
+    s = q @ k.transpose(-1, -2).contiguous() / q.shape[-1] ** 0.5
+    if valid is not None:
+        s = s - 1e6 * (1.0 - valid.double())[:, None, :]
+    p = torch.softmax(s * pattern, -1) * pattern
+    o = p @ v
+    o.backward(do.double())
+    return p.detach(), o.detach(), q.grad, k.grad, v.grad
+
+
+def _module(B, H, L, masked):
+    cfg = dict(head_dim=32, num_head=H, max_seq_len=L, batch_size=B, block_size=1)
+    load, cls = (("_blockcuda_mask_compile_module", spion_amd.CUDABlockMaskAttention) if masked else
+                 ("_blockcuda_compile_module", spion_amd.CUDABlockAttention))
+    cpp = getattr(spion_amd.Attention, load)()
+    handle = cpp.init(32, L, B * H, 1)
+    return cpp, handle, cls(cfg, cpp, handle)
+
+
+# one range; a second one of 32 rows; work-groups of 256 rows whose last is partial; work-groups of 512, the last partial
+@pytest.mark.parametrize("B,H,L,masked", [(32, 2, 512, False), (16, 2, 544, True), (11, 2, 1056, False), (35, 2, 1056, True),
+                                          (35, 2, 1056, False), (32, 2, 2048, False)])
+@pytest.mark.parametrize("views", [False, True])
+def test_ranges_and_batches(B, H, L, masked, views):
+    gen = torch.Generator(device="cuda").manual_seed(L + B)
+    pattern = _pattern(L, gen)
+    shape = (B, L, H, 32) if views else (B, H, L, 32)
+    make = lambda: torch.randn(*shape, generator=gen, device="cuda")
+    q, k, v, do = (make().transpose(1, 2) if views else make() for _ in range(4))
+    leaves = [t.requires_grad_() for t in (q, k, v)]
+    i = torch.arange(L, device="cuda")
+    valid = (i[None, :] < torch.randint(L // 2, L + 1, (B, 1), generator=gen, device="cuda")).float() if masked else \
+        torch.ones(B, L, device="cuda")
+    cpp, handle, module = _module(B, H, L, masked)
+    out, p = module(*leaves, valid, pattern)
+    out.backward(do)
+    torch.cuda.synchronize()
+    assert _lib.core().spion_last_path(handle) == 3
+    where = pattern.bool()
+    p = None if masked else p.detach().reshape(B, H, -1)  # the masked module does not return it
+    for b, h in ((0, 0), (B // 2, H - 1), (B - 1, H - 1)):
+        at = lambda t: t.detach()[b, h][None]
+        ref = _reference(at(q), at(k), at(v), at(do), pattern.double()[None], valid[b][None] if masked else None)
+        got = (None if masked else p[b, h],) + tuple(at(t) for t in (out, q.grad, k.grad, v.grad))
+        for name, x, y in zip(("P", "out", "dQ", "dK", "dV"), got, (ref[0][0][where],) + ref[1:]):
+            if x is None:
+                continue
+            # a few hundred terms each: 2^-24 of a typical element per rounding, with a wide margin
+            tol = 2e-5 * (y.abs() + y.pow(2).mean().sqrt())
+            worst = float(((x.double() - y).abs() / tol).max())
+            assert worst <= 1.0, f"{name}, head {(b, h)}: {worst}"
+    cpp.destroy(handle)
+
+
+def test_infinities_stay_in_their_rows():
+    """The slots of a batch that hold no entry read a row of zeros: an infinity reaches the rows that have its column (or whose
+    dense tiles do) and no other."""
+    B, H, L, far = 16, 2, 1024, 900
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    pattern = _pattern(L, gen)
+    q, k, v, do = (torch.randn(B, H, L, 32, generator=gen, device="cuda") for _ in range(4))
+    q[..., far, 3] = v[..., far, 3] = do[..., far, 5] = float("inf")
+    q, k, v = (t.requires_grad_() for t in (q, k, v))
+    cpp, handle, module = _module(B, H, L, False)
+    out, p = module(q, k, v, torch.ones(B, L, device="cuda"), pattern)
+    out.backward(do)
+    assert _lib.core().spion_last_path(handle) == 3
+    i = torch.arange(L, device="cuda")
+    near = (i - far).abs() < 128  # the window's tiles
+    reads_v = near | (pattern[:, far] > 0)
+    assert torch.isfinite(out[..., ~reads_v, :]).all() and torch.isfinite(q.grad[..., ~reads_v, :]).all()
+    assert not torch.isfinite(out[..., pattern[:, far] > 0, 3]).any()
+    reads_q = near | (pattern[far] > 0)
+    # dK and dV also take {dS, P} of rows whose own results are not finite
+    bad_rows = (pattern[reads_v] > 0).any(0)
+    clean = ~(reads_q | bad_rows)
+    if clean.any():
+        assert torch.isfinite(k.grad[..., clean, :]).all()
+    assert torch.isfinite(v.grad[..., ~reads_q & ~near, :]).all()
+    cpp.destroy(handle)
