@@ -795,14 +795,16 @@ def bench_sparse_layer(args, dev, workload, full=True):
     alg_flops = workloads.sparse_flops(nnz, d, NB)
     alg_bytes = workloads.sparse_bytes(nnz, L, d, NB)
     third = alg_flops / 3.0  # forward, row pass and column pass carry 4*n*d*NB each
+    # element patterns: dense window tiles on the MFMA units + the remainder by ranges, or gathered; each phase is two or three
+    # launches
+    ranges = ("rem_fwd_kernel + hyb_tile_fwd_kernel + rem_prob_kernel", "hyb_tile_bwd_row_kernel + rem_bwd_row_kernel",
+              "hyb_tile_bwd_col_kernel + rem_bwd_col_kernel")
+    by_ranges = d == 32 and L % 32 == 0 and _remainder_in_lds(L, NB)
     names = {1: ("tile_fwd_kernel", "tile_bwd_row_kernel", "tile_bwd_col_kernel"),
-             2: ("elem_fwd_kernel", "elem_bwd_row_kernel", "elem_bwd_col_kernel"),
-             # hybrid: dense window tiles on the MFMA units + gathered remainder; each phase is two or three launches
-             3: ("rem_fwd_kernel + hyb_tile_fwd_kernel", "hyb_tile_bwd_row_kernel + rem_bwd_row_kernel",
-                 "hyb_tile_bwd_col_kernel + rem_bwd_col_kernel") if _remainder_in_lds(L, NB) else
-                ("hyb_rem_logits_kernel + hyb_tile_fwd_kernel + hyb_rem_pv_kernel",
-                 "hyb_tile_bwd_row_kernel + hyb_rem_bwd_row_kernel",
-                 "hyb_tile_bwd_col_kernel + hyb_rem_bwd_col_kernel")}[path]
+             2: ranges if by_ranges else ("elem_fwd_kernel", "elem_bwd_row_kernel", "elem_bwd_col_kernel"),
+             3: ranges if by_ranges else ("hyb_rem_logits_kernel + hyb_tile_fwd_kernel + hyb_rem_pv_kernel",
+                                          "hyb_tile_bwd_row_kernel + hyb_rem_bwd_row_kernel",
+                                          "hyb_tile_bwd_col_kernel + hyb_rem_bwd_col_kernel")}[path]
     kernels = dict(zip(names, (t_fwd, t_row, t_col)))
     dom = max(kernels, key=kernels.get)
     dom_ms = kernels[dom]

@@ -237,8 +237,9 @@ int spion_register_pattern(void* handle, const int* Offsets, const int* Columns,
                            const int* host_Offsets, const int* host_Columns);
 
 /* Which kernel family the last forward/backward of a sparse handle used:
- * 0 = none yet, 1 = MFMA 32x32 tile path, 2 = element (gather) path, 3 = hybrid path (element-sparse pattern
- * whose well-filled 32x32 tiles run on the MFMA units, the rest on the gather kernels).  For 2 and 3 the backward
+ * 0 = none yet, 1 = MFMA 32x32 tile path, 2 = element path (gathers; with enough rows at emb_dim 32, the hybrid path's
+ * kernels), 3 = hybrid path (element-sparse pattern at least half of whose entries lie in well-filled 32x32 tiles, which
+ * run on the MFMA units, the rest on kernels of their own).  For 2 and 3 the backward
  * needs the dS scratch.  It describes the most recent call on the handle, not a particular pattern. */
 int spion_last_path(void* handle);
 

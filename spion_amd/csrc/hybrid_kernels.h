@@ -146,6 +146,13 @@ __device__ __forceinline__ void hyb_reduce_store(const f32x16& acc, float factor
     }
 }
 
+// acc += W . X of one tile, its 32 terms summed by themselves first: the sums over a strip's tiles are shorter chains.
+__device__ __forceinline__ void hyb_mma_add(const float (&w)[16], const float (&x)[1][16], f32x16 (&acc)[1]) {
+    f32x16 part[1] = {splat16(0.f)};
+    mma_b<32>(w, x, part);
+    acc[0] += part[0];
+}
+
 // Two-deep software pipeline over n tiles with two register sets: while tile i is computed, the operands and P of
 // tile i + 1 are in flight and so is the index of tile i + 2 (requested first, so that waiting for it leaves the
 // younger requests outstanding).  Positions past the end are clamped by the callers (valid, redundant requests).
@@ -402,7 +409,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
             lds_put_rows(T, li, h, p);
             lds_get_cols(Tx, li, h, vb[0]);
             lds_get_cols(T, li, h, pc);
-            mma_b<D>(p, vb, o);
+            hyb_mma_add(p, vb, o);
             int pos[16], bits[16];
             hyb_rows_from_lanes(X, l, h, pos_l[u], pos);
             hyb_rows_from_lanes(X + 64, l, h, (int)bits_l[u], bits);
@@ -544,7 +551,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_row_kernel(const float* __restrict__ K
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
-            mma_b<D>(ds, kb, acc);
+            hyb_mma_add(ds, kb, acc);
         });
     if constexpr (WAVES > 1) __syncthreads();
     hyb_reduce_store<WAVES>(acc[0], scale, dQ + gb, gld, I * 32, w, li, h, lds);
@@ -681,8 +688,8 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_col_kernel(const float* __restrict__ Q
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * x.p[r];
-            mma_b<D>(ds, qb, ak);
-            mma_b<D>(x.p, ob, av);
+            hyb_mma_add(ds, qb, ak);
+            hyb_mma_add(x.p, ob, av);
         });
     };
     walk(split3(vt), l);

@@ -6,9 +6,11 @@
 //                     cores, in fp32 or with operands split into three bf16 parts (tile_kernels.h); tiles go
 //                     from global memory into LDS or the MFMA register layout in whole 128-byte rows, the
 //                     tile list of a block row / block column is walked per wavefront.
-//   * element path -- any other CSR (element-sparse patterns, odd head sizes): one wavefront per
-//                     row gathers K/V rows; a transposed (CSC) index built on the host once per
-//                     pattern makes dK/dV deterministic without atomics.
+//   * element path -- any other CSR (element-sparse patterns, odd head sizes).  d = 32 and enough rows: well-filled
+//                     32x32 tiles of the pattern on the matrix cores (hybrid_kernels.h), the remainder by ranges
+//                     whose rows lie in LDS (remainder_kernels.h); else one wavefront per row gathers K/V rows.
+//                     A transposed index built on the host once per pattern makes dK/dV deterministic without
+//                     atomics.
 //
 // Semantics follow the reference kernels (models/block_attn.cu:33-130, models/block_attn_mask.cu:88-173):
 // the softmax denominator counts every off-pattern key with logit 0.
@@ -19,6 +21,7 @@
 #include "../../include/spion_hip.h"
 
 #include <algorithm>
+#include <initializer_list>
 #include <cmath>
 #include <cstdlib>
 #include <queue>
@@ -422,6 +425,7 @@ struct PatternIndex {
     int *d_ccp = nullptr, *d_crow = nullptr, *d_cpos = nullptr;
     // element-sparse pattern whose well-filled 32x32 tiles run on the MFMA units (hybrid_kernels.h)
     bool hybrid = false;
+    bool hyb_dense = false;  // at least half of the entries lie in dense tiles; otherwise the element kernels take it as well
     int hyb_tiles = 0, hyb_nr = 0;
     HybIndex hyb{};
     bool rem_lds = false;  // the remainder's kernels keep its rows in LDS (remainder_kernels.h); `rem` instead of hyb's lists
@@ -469,6 +473,8 @@ struct SparseAttn {
     float* ws_stats = nullptr;   // [NB][L][2] softmax row statistics handed between the hybrid forward's launches
     float* ws_raw = nullptr;     // [NB][nr] raw logits of a hybrid pattern's remainder, forward only
     size_t ws_raw_count = 0;
+    float* ws_pairs = nullptr;   // [NB][nr] {dS, P} of the remainder where the dS scratch is too small for them
+    size_t ws_pairs_count = 0;
     float* ws_ds = nullptr;      // [NB][nnz] dS scratch of the strided backward on patterns without tile structure
     size_t ws_ds_count = 0;
     float* ws_part = nullptr;    // [NB][slots][slot floats] partial results of the chunks of long strips (bf16 family)
@@ -555,6 +561,7 @@ void sparse_destroy(void* h) {
     if (a->ws_stats) (void)hipFree(a->ws_stats);
     if (a->ws_ds) (void)hipFree(a->ws_ds);
     if (a->ws_raw) (void)hipFree(a->ws_raw);
+    if (a->ws_pairs) (void)hipFree(a->ws_pairs);
     if (a->ws_part) (void)hipFree(a->ws_part);
     for (void* p : a->retired) (void)hipFree(p);
     for (auto& sl : a->oslot)
@@ -901,7 +908,10 @@ static bool analyse_pattern(SparseAttn* a, const int* Offsets, const int* Column
         pi.max_col_tiles = mc;
     } else {
         // ---- hybrid split: aligned 32x32 tiles with at least HYB_MIN_FILL entries become dense tiles (at most
-        // HYB_MAX_ROW_TILES per block row, the fullest first), everything else stays with the gather kernels
+        // HYB_MAX_ROW_TILES per block row, the fullest first), everything else is the remainder.  Where the remainder's rows
+        // lie in LDS every pattern goes this way, whatever part of it the tiles hold (no tiles at all: 32 heads of 4096, 300
+        // random entries a row, forward 542 us gathered from L2 / 213, row pass 548 / 384, column pass 690 / 252); with gathers
+        // only patterns that are mostly tiles.
         if (!a->force_element && a->d == 32 && L % 32 == 0 && nnz > 0) {
             constexpr int HYB_MIN_FILL = 128;
             const int nbr = L / 32;
@@ -928,8 +938,14 @@ static bool analyse_pattern(SparseAttn* a, const int* Offsets, const int* Column
                 dense_of[I] = cand;
                 t_rp[I + 1] = (int)t_col.size();
             }
-            const int nt = (int)t_col.size();
-            if (nt > 0 && dense_entries * 2 >= (long long)nnz) {
+            int nt = (int)t_col.size();
+            pi.hyb_dense = nt > 0 && dense_entries * 2 >= (long long)nnz;
+            if (pi.hyb_dense || rem_in_lds(a)) {
+                if (nt == 0) {  // one that no block row or column lists: what the kernels' clamped look-ups find
+                    t_col.push_back(0);
+                    t_row.push_back(0);
+                    nt = 1;
+                }
                 std::vector<int> t_pos((size_t)nt * 32, 0), r_off(L + 1, 0), r_col, r_pos;
                 std::vector<unsigned> t_bits((size_t)nt * 32, 0u);
                 std::vector<int> slot(nbr);
@@ -953,12 +969,13 @@ static bool analyse_pattern(SparseAttn* a, const int* Offsets, const int* Column
                 }
                 const int nr = (int)r_col.size();
                 // transposed lists: dense tiles by block column, remainder entries column after column
-                std::vector<int> t_cp(nbr + 1, 0), t_ct(std::max(nt, 1));
-                for (int t = 0; t < nt; ++t) t_cp[t_col[t] + 1]++;
+                std::vector<int> t_cp(nbr + 1, 0), t_ct(nt, 0);
+                const int listed = t_rp[nbr];  // tiles that belong to a block row: all, but for that one
+                for (int t = 0; t < listed; ++t) t_cp[t_col[t] + 1]++;
                 for (int J = 0; J < nbr; ++J) t_cp[J + 1] += t_cp[J];
                 {
                     std::vector<int> fill(t_cp.begin(), t_cp.end() - 1);
-                    for (int t = 0; t < nt; ++t) t_ct[fill[t_col[t]]++] = t;
+                    for (int t = 0; t < listed; ++t) t_ct[fill[t_col[t]]++] = t;
                 }
                 std::vector<int> t_ci(t_ct.size());
                 for (size_t e = 0; e < t_ct.size(); ++e) t_ci[e] = t_row[t_ct[e]];
@@ -1141,6 +1158,12 @@ void sparse_forget_pattern(void* h, const int* Offsets, const int* Columns) {
     if (a->pat.valid && a->pat.key_off == Offsets && a->pat.key_col == Columns) a->pat = PatternIndex();
 }
 
+static bool capturing(const SparseAttn* a) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(a->hdr.stream, &cap);
+    return cap != hipStreamCaptureStatusNone;
+}
+
 static bool ensure_ws(float** p, size_t count) {
     if (*p) return true;
     return SPION_HIP_OK(hipMalloc((void**)p, sizeof(float) * count));
@@ -1153,18 +1176,17 @@ static bool ensure_ws(float** p, size_t count) {
 // pattern it was recorded with.
 static bool ensure_ws_grow(SparseAttn* a, float** p, size_t* have, size_t need, const char* who) {
     if (*have >= need) return true;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    (void)hipStreamIsCapturing(a->hdr.stream, &cap);
-    if (cap != hipStreamCaptureStatusNone) {
-        set_error("%s: the workspace for this pattern is not allocated yet; run one step outside the capture", who);
+    if (capturing(a)) {
+        if (who) set_error("%s: the workspace for this pattern is not allocated yet; run one step outside the capture", who);
         return false;
     }
     const size_t want = std::max(need, *have + *have / 2);
     float* fresh = nullptr;
     if (hipMalloc((void**)&fresh, sizeof(float) * want) != hipSuccess) {
         (void)hipGetLastError();
-        if (want == need || !SPION_HIP_OK(hipMalloc((void**)&fresh, sizeof(float) * need))) {
-            if (want == need) set_error("%s: hipMalloc of %zu bytes of workspace failed", who, sizeof(float) * need);
+        if (want == need || hipMalloc((void**)&fresh, sizeof(float) * need) != hipSuccess) {
+            (void)hipGetLastError();
+            if (who) set_error("%s: hipMalloc of %zu bytes of workspace failed", who, sizeof(float) * need);
             return false;
         }
         *have = need;
@@ -1173,6 +1195,44 @@ static bool ensure_ws_grow(SparseAttn* a, float** p, size_t* have, size_t need, 
     }
     if (*p) a->retired.push_back(*p);
     *p = fresh;
+    return true;
+}
+
+static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// Whether a call on a hybrid pattern takes the hybrid kernels.  The remainder's kernels by ranges load 16 bytes a lane; and
+// where the element kernels would do as well (few entries in dense tiles), nothing is refused for want of a workspace.
+static bool take_hybrid(SparseAttn* a, std::initializer_list<const void*> operands) {
+    if (!a->pat.hybrid) return false;
+    if (!a->pat.rem_lds) return true;
+    for (const void* p : operands)
+        if (!aligned16(p)) return false;
+    return true;
+}
+static size_t rem_list(const SparseAttn* a) { return (size_t)a->NB * (size_t)std::max(a->pat.hyb_nr, 1); }
+static bool take_hybrid_forward(SparseAttn* a, std::initializer_list<const void*> operands) {
+    if (!take_hybrid(a, operands)) return false;
+    if (a->pat.hyb_dense) return true;
+    if (!a->ws_stats && (capturing(a) || hipMalloc((void**)&a->ws_stats, sizeof(float) * 2 * a->NB * a->L) != hipSuccess)) {
+        (void)hipGetLastError();
+        a->ws_stats = nullptr;
+        return false;
+    }
+    return ensure_ws_grow(a, &a->ws_raw, &a->ws_raw_count, rem_list(a), nullptr);
+}
+// *pairs: where the row pass leaves {dS, P} for the column pass -- the dS scratch [NB][nnz] if they fit.
+static bool take_hybrid_backward(SparseAttn* a, std::initializer_list<const void*> operands, float* dS, int nnz, float** pairs) {
+    if (!take_hybrid(a, operands)) return false;
+    *pairs = dS;
+    if (a->pat.hyb_dense) return true;
+    if (!a->ws_rowsum && (capturing(a) || hipMalloc((void**)&a->ws_rowsum, sizeof(float) * a->NB * a->L) != hipSuccess)) {
+        (void)hipGetLastError();
+        a->ws_rowsum = nullptr;
+        return false;
+    }
+    if (2LL * a->pat.hyb_nr <= nnz) return true;
+    if (!ensure_ws_grow(a, &a->ws_pairs, &a->ws_pairs_count, 2 * rem_list(a), nullptr)) return false;
+    *pairs = a->ws_pairs;
     return true;
 }
 
@@ -1513,10 +1573,8 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
     if (!ensure_ws(&a->ws_stats, (size_t)a->NB * a->L * 2)) return;
     // the remainder's raw logits between the first and the third launch: a compact list of their own (written and
     // read in full lines) rather than their places inside P, where every four-byte store would pull in a line
-    if (!ensure_ws_grow(a, &a->ws_raw, &a->ws_raw_count, (size_t)a->NB * (size_t)std::max(a->pat.hyb_nr, 1),
-                        "attn_forward"))
-        return;
-    a->last_path = 3;
+    if (!ensure_ws_grow(a, &a->ws_raw, &a->ws_raw_count, rem_list(a), "attn_forward")) return;
+    a->last_path = a->pat.hyb_dense ? 3 : 2;
     const int nbr = a->L / 32;
     const long long rows = (long long)a->NB * a->L;
     // strips of few dense tiles: one wavefront walks the whole strip; else four share it
@@ -1560,15 +1618,14 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
     check_launch("hybrid forward kernels");
 }
 
-// o: the forward's output (same layout as dO).  dS: the caller's [NB][nnz] scratch, which receives the remainder's
-// {dS, P} pairs, [NB][nr] (a hybrid pattern keeps at most half of its entries in the remainder).
+// o: the forward's output (same layout as dO).  dS: scratch for the remainder's {dS, P} pairs, [NB][nr].
 template <bool ST>
 static void launch_hyb_bwd(SparseAttn* a, const float* Q, const float* K, const float* V, const float* P,
                            const float* dO, const float* o, float* dS, float* dQ, float* dK, float* dV,
                            const int* Offsets, int nnz, const Layouts& ly) {
     PhaseRange phase("spion backward (hybrid kernels)");
     if (!ensure_ws(&a->ws_rowsum, (size_t)a->NB * a->L)) return;
-    a->last_path = 3;
+    a->last_path = a->pat.hyb_dense ? 3 : 2;
     const int nbr = a->L / 32;
     const long long rows = (long long)a->NB * a->L;
     const bool one_r = a->pat.max_row_tiles <= 2 * HYB_MAXT1, one_c = a->pat.max_col_tiles <= 2 * HYB_MAXT1;
@@ -1711,7 +1768,8 @@ void sparse_forward(void* h, const float* Q, const float* Kt, const float* V, co
         return;
     }
     a->last_path = 2;
-    float* hyb_ocopy = a->pat.hybrid ? ocache_for_forward(a, Attn) : nullptr;
+    const bool hybrid = take_hybrid_forward(a, {Q, Kt, V, Out});  // (a transposed copy of Kt is aligned as well)
+    float* hyb_ocopy = hybrid ? ocache_for_forward(a, Attn) : nullptr;
     if (!hyb_ocopy) ocache_drop(a, Attn);
     const float* Krm = Kt;  // the element kernels read K row-major
     if (!krow) {
@@ -1719,7 +1777,7 @@ void sparse_forward(void* h, const float* Q, const float* Kt, const float* V, co
         launch_transpose(a, Kt, a->ws_trans);
         Krm = a->ws_trans;
     }
-    if (a->pat.hybrid) {
+    if (hybrid) {
         launch_hyb_fwd<false>(a, Q, Krm, V, Mask, Attn, Out, hyb_ocopy, Offsets, nnz, Layouts{});
         return;
     }
@@ -1778,8 +1836,9 @@ void sparse_backward(void* h, const float* Q, const float* K, const float* Vt, c
         // the hybrid kernels take the row sums from the forward's output (the caller's, or the handle's kept copy);
         // without it the gather kernels below serve the same P
         const float* o = Out ? Out : ocache_for_backward(a, P);
-        if (o) {
-            launch_hyb_bwd<false>(a, Q, K, Vrm, P, dO, o, dS, dQ, dK, dV, Offsets, nnz, Layouts{});
+        float* pairs;
+        if (o && take_hybrid_backward(a, {Q, K, Vrm, dO, o, dQ, dK, dV}, dS, nnz, &pairs)) {
+            launch_hyb_bwd<false>(a, Q, K, Vrm, P, dO, o, pairs, dQ, dK, dV, Offsets, nnz, Layouts{});
             return;
         }
     }
@@ -1896,7 +1955,6 @@ static bool check_layout(const char* who, const char* what, const SparseAttn* a,
     (void)heads;
     return true;
 }
-static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 static SparseAttn* strided_handle(void* h, const char* who, const int* Offsets, const int* Columns, int nnz, int heads) {
     SparseAttn* a = as_sparse(h, who);
@@ -1951,7 +2009,7 @@ void sparse_forward_strided(void* h, const float* Q, const float* K, const float
     ly.H = heads;
     if (!a->pat.tiled) {
         ocache_drop(a, Attn);  // the backward of these entry points is handed Out
-        if (a->pat.hybrid) {
+        if (take_hybrid_forward(a, {Q, K, V, Out})) {
             launch_hyb_fwd<true>(a, Q, K, V, Mask, Attn, Out, nullptr, Offsets, nnz, ly);
             return;
         }
@@ -2007,8 +2065,9 @@ void sparse_backward_strided(void* h, const float* Q, const float* K, const floa
     if (!a->pat.tiled) {
         // these entry points have no dS argument: the scratch is the handle's (grown outside graph capture only)
         if (!ensure_ws_grow(a, &a->ws_ds, &a->ws_ds_count, (size_t)a->NB * (size_t)std::max(nnz, 1), who)) return;
-        if (a->pat.hybrid) {
-            launch_hyb_bwd<true>(a, Q, K, V, P, dO, Out, a->ws_ds, dQ, dK, dV, Offsets, nnz, ly);
+        float* pairs;
+        if (take_hybrid_backward(a, {Q, K, V, dO, Out, dQ, dK, dV}, a->ws_ds, nnz, &pairs)) {
+            launch_hyb_bwd<true>(a, Q, K, V, P, dO, Out, pairs, dQ, dK, dV, Offsets, nnz, ly);
             return;
         }
         a->last_path = 2;

@@ -104,3 +104,70 @@ def test_infinities_stay_in_their_rows():
         assert torch.isfinite(k.grad[..., clean, :]).all()
     assert torch.isfinite(v.grad[..., ~reads_q & ~near, :]).all()
     cpp.destroy(handle)
+
+
+def test_scattered_patterns_and_capture():
+    """A pattern without dense structure: float64 agrees; a graph recorded before the handle has its workspaces holds the
+    element kernels, one recorded after a step the kernels by ranges."""
+    B, H, L = 32, 2, 576
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    pattern = (torch.rand(L, L, generator=gen, device="cuda") < 0.05).float()
+    pattern[17, ::2] = 1.0
+    pattern[9] = 0.0
+    q, k, v, do = (torch.randn(B, H, L, 32, generator=gen, device="cuda") for _ in range(4))
+    where = pattern.bool()
+    off = torch.zeros(L + 1, dtype=torch.int32)
+    off[1:] = where.sum(1).cumsum(0).cpu()
+    col = where.nonzero()[:, 1].to(torch.int32).cpu()
+    d_off, d_col, count = off.cuda(), col.cuda(), where.sum(1).to(torch.int32)
+    nnz = int(off[-1])
+    core = _lib.core()
+    cpp, handle, _ = _module(B, H, L, False)
+    assert core.spion_register_pattern(handle, d_off.data_ptr(), d_col.data_ptr(), nnz, off.data_ptr(), col.data_ptr()) == 0
+    ds = torch.empty(B * H * nnz, device="cuda")
+    out = torch.empty_like(q)
+    p = torch.empty(B * H, nnz, device="cuda")
+    grads = [torch.empty_like(q) for _ in range(3)]
+
+    def step():
+        core.spion_set_stream(handle, torch.cuda.current_stream().cuda_stream)
+        at = (d_off.data_ptr(), d_col.data_ptr(), count.data_ptr(), nnz)
+        core.spion_attn_forward_rowmajor(handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), None, p.data_ptr(), out.data_ptr(), *at)
+        core.spion_attn_backward_rowmajor(handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), p.data_ptr(), out.data_ptr(),
+                                          do.data_ptr(), ds.data_ptr(), *(g.data_ptr() for g in grads), *at)
+
+    def record():
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            step()
+        _lib.check_error("capture")
+        return graph
+
+    def replayed(graph):
+        for t in (out, p, *grads):
+            t.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        return [t.clone() for t in (out, p, *grads)]
+
+    before = record()
+    first = replayed(before)
+    for t in (out, p, *grads):
+        t.fill_(float("nan"))
+    step()
+    torch.cuda.synchronize()
+    assert core.spion_last_path(handle) == 2
+    eager = [t.clone() for t in (out, p, *grads)]
+    after = record()
+    for _ in range(3):
+        assert all(torch.equal(x, y) for x, y in zip(replayed(after), eager))
+        assert all(torch.equal(x, y) for x, y in zip(replayed(before), first))
+    at = lambda t: t[B // 2, 1][None]
+    ref = _reference(at(q), at(k), at(v), at(do), pattern.double()[None], None)
+    for results in (first, eager):
+        got = (results[1][(B // 2) * H + 1],) + tuple(at(results[i]) for i in (0, 2, 3, 4))
+        for name, x, y in zip(("P", "out", "dQ", "dK", "dV"), got, (ref[0][0][where],) + ref[1:]):
+            tol = 2e-5 * (y.abs() + y.pow(2).mean().sqrt())
+            assert float(((x.double() - y).abs() / tol).max()) <= 1.0, name
+    core.spion_set_stream(handle, 0)
+    cpp.destroy(handle)
