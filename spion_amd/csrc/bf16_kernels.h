@@ -27,6 +27,7 @@
 // merge kernel combines the slots of a strip).
 #pragma once
 #include "bf16_tile.h"
+#include "tile_kernels.h"
 
 namespace spion {
 

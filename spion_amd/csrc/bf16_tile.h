@@ -1,6 +1,6 @@
 // 32 x D bf16 tiles in LDS: their layout, the loads that fill them and the two kinds of operand reads.
 #pragma once
-#include "tile_kernels.h"
+#include "tile_ops.h"
 
 namespace spion {
 

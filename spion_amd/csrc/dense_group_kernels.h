@@ -22,6 +22,7 @@
 // the parts written after the last product instead of beside the second, 3 %.
 #pragma once
 #include "bf16_tile.h"
+#include "tile_kernels.h"
 
 namespace spion {
 

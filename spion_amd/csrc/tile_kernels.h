@@ -25,6 +25,7 @@
 //     last tile after it: a prefetch whose only consumer sits in a conditional block would be sunk into
 //     that block by the compiler, next to its use.
 #pragma once
+#include "bf16_tile.h"
 #include "tile_ops.h"
 
 namespace spion {
@@ -232,7 +233,6 @@ __device__ __forceinline__ void lds_get_lin(const float* T, int l, f32x4 (&raw)[
 // instruction -- v_readfirstlane, or v_readlane when the compiler restores a spilled scalar -- needs that distance
 // before a memory instruction reads it, and the compiler, which adds it elsewhere, does not look inside assembly.
 // -------------------------------------------------------------------------------------------------
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ u32x4 rsrc_words(const void* p, size_t bytes) {
     const unsigned long long a = reinterpret_cast<unsigned long long>(p);
     u32x4 r;
@@ -399,9 +399,10 @@ struct DmaTileF32 {
 // GHz under fp32 chains, 1.98 to 2.2 GHz with every product split).  So
 //   * products over the head dimension, whose other operand a wavefront keeps for all its tiles, are split: one
 //     operand per tile;
-//   * products over a tile's rows, which need two operands split, run on the bf16 pipe in the forward and the row pass at
-//     d = 64 (one of the two serves two products) and in the column pass at d = 32 (two of its three products; three
-//     wavefronts per SIMD hide the splitting), on the fp32 pipe in the forward and the row pass at d = 32;
+//   * products over a tile's rows, which need two operands split, run on the bf16 pipe in the forward at d = 64 (one of the
+//     two serves two products), in the row pass and in the column pass at d = 32 (three wavefronts per SIMD hide the
+//     splitting; dO is split once for its two products), on the fp32 pipe in the forward at d = 32 (split there: 32 x 2 heads
+//     of 4096, a tenth kept, whole step 475 -> 488 us; six logit tiles and split operands spill at three wavefronts per SIMD);
 //   * the column pass at d = 64 uses fp32 chains alone: split operands for its five products spill registers, and whole
 //     steps are 1 % slower to 4 % faster without (split / fp32 chains in us, on four machines: 64 x 2 heads of 1024,
 //     14 % kept, 194 to 202 / 187 to 194; 16 x 4 of 2048, 10 %, 262 to 274 / 255 to 265; 3 x 8 of 4000, 8 %, 278 to 291 / 274
@@ -409,7 +410,9 @@ struct DmaTileF32 {
 // Measured in us per launch in a training loop, all kernels on fp32 chains / as now.  32 x 2 heads of 4096 tokens,
 // d = 32, 32 x 32 blocks, a tenth kept: forward 162 / 155, row pass 141 / 134, column pass 184 / 161; 256 x 2 heads of 1024:
 // 139 / 139, 122 / 121, 148 / 132; 2 x 2 of 8192, a fifth kept (two sweeps): 104 / 97, 76 / 71, 98 / 91; 3 x 8 heads of 4000,
-// d = 64: 98 / 76, 99 / 80.  The dense kernels (dense_attn.hip), 64 x 2 heads of 1024, d = 32: forward 180 / 177, row pass 177
+// d = 64: 98 / 76, 99 / 80.  Since then, at the first of these shapes: column pass with dO split once instead of twice (88 of
+// 515 vector-ALU instructions a tile) 156 -> 149, row pass with both products split, whole step 475 -> 468 -> 463 us; the steps
+// of 1024 tokens stay where they are (390: memory), 32 x 2 heads of 2048 in 64 x 64 blocks 133 -> 131.  The dense kernels (dense_attn.hip), 64 x 2 heads of 1024, d = 32: forward 180 / 177, row pass 177
 // / 156, column pass 235 / 209 (of its products the first; three splits do not fit the registers of three wavefronts per
 // SIMD: 260); 4 x 2 of 3072: 163 / 136, 108 / 86, 148 / 118; 4 x 8 of 2048, d = 64: 319 / 276, 276 / 240.  The dense
 // tiles of element patterns (hybrid_kernels.h, 32 x 2 heads of 4096): forward 97 / 91, column pass 99 / 96; the row pass (84 / 84)
@@ -472,11 +475,11 @@ __device__ __forceinline__ void mma_b_split(const float (&w)[16], const float (&
         }
     }
 }
-// the same on the pipe the forward and the row pass use
-template <int D, bool EXACT = false>
+// the same on the pipe the forward uses
+template <int D>
 __device__ __forceinline__ void mma_b(const float (&w)[16], const float (&x)[D / 32][16], f32x16 (&out)[D / 32]) {
     if constexpr (D == 32) mma_b_f32<D>(w, x, out);
-    else mma_b_split<D, EXACT>(w, x, out);
+    else mma_b_split<D, false>(w, x, out);
 }
 __device__ __forceinline__ f32x16 splat16(float v) {
     return (f32x16){v, v, v, v, v, v, v, v, v, v, v, v, v, v, v, v};
@@ -1158,7 +1161,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
-                mma_b<D, EXACT>(ds, kb, acc);
+                mma_b_split<D, EXACT>(ds, kb, acc);
             }
         }
     } else {
@@ -1209,7 +1212,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
-                mma_b<D, EXACT>(ds, kb, acc);
+                mma_b_split<D, EXACT>(ds, kb, acc);
             }
         }
     }
@@ -1286,9 +1289,10 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
     }
     if constexpr (D == 32) {
         // The P, Q and dO tiles and the 32 values of -g go straight into wave-private LDS (thirteen instructions, no
-        // registers in flight); the operands of tile i are read out of LDS into registers -- the dO tile in both
-        // of its roles -- then the same space is requested for tile i + 1, whose loads have the three chains of
-        // tile i to arrive.
+        // registers in flight); P, Q, -g and dO's rows are read out of LDS into registers, and P and -g requested for tile
+        // i + 1.  dO enters two products, by rows and by columns, and is split once for both: its parts are written over the
+        // Q and dO tiles (6 of their 8 KB, planes in the layout of DmaTile<32>) and read back transposed; then Q and dO are
+        // requested, whose loads have the second and third product of tile i to arrive.
         const char* Tp = reinterpret_cast<const char*>(T);
         const char* Tq = Tp + DmaTileF32::TILE;
         const char* To = Tp + 2 * DmaTileF32::TILE;
@@ -1300,26 +1304,27 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
         const int ql = DmaTileF32::voff(l, ild), ol = DmaTileF32::voff(l, old_);
         const int qx = DmaTileF32::extra_step(ild), ox = DmaTileF32::extra_step(old_);
         const int pl0 = 16 * ((l & 7) ^ (l >> 3)), pl1 = (l >> 3) * 4;  // lane offset into a P tile: pl0 + pl1 * row stride
-        const auto a_p = DmaTileF32::cols_addr(Tp, li, h), a_q = DmaTileF32::cols_addr(Tq, li, h),
-                   a_o = DmaTileF32::cols_addr(To, li, h);
+        const auto a_p = DmaTileF32::cols_addr(Tp, li, h);  // the Q tile's are 4 KB on
         const auto a_go = DmaTileF32::own_addr(To, li, 4 * h, 1);
         const char* a_g = Tg + 16 * h;
-        auto issue = [&](const int4 d) {
-            const int I = d.x, rn = d.z;
-            DmaTileF32::load<true>(wP, lp, pl0 + pl1 * rn, d.y * 4, DmaTileF32::extra_step(rn));
-            DmaTileF32::load(wQ, lq, ql, I * 32 * ild * 4, qx);
-            DmaTileF32::load(wO, lo, ol, I * 32 * old_ * 4, ox);
-            dma_b32(wG, lg, l * 4, I * 128);
+        auto issue_pg = [&](const int4 d) {
+            DmaTileF32::load<true>(wP, lp, pl0 + pl1 * d.z, d.y * 4, DmaTileF32::extra_step(d.z));
+            dma_b32(wG, lg, l * 4, d.x * 128);
+        };
+        auto issue_qo = [&](const int4 d) {
+            DmaTileF32::load(wQ, lq, ql, d.x * 32 * ild * 4, qx);
+            DmaTileF32::load(wO, lo, ol, d.x * 32 * old_ * 4, ox);
         };
         if (nu > 0) {
-            issue(desc[w]);
-            int4 dn = desc[w + (nu > 1 ? WAVES : 0)];
+            int4 dn = desc[w];
+            issue_pg(dn);
+            issue_qo(dn);
+            dn = desc[w + (nu > 1 ? WAVES : 0)];
             for (int i = 0; i < nu; ++i) {
                 const int4 dnn = desc[w + min(i + 2, nu - 1) * WAVES];  // descriptor of the tile after the next
                 wait_vm<0>();
-                float pc[16], qb[1][16], ob[1][16], go[KH];
+                float pc[16], qb[1][16], go[KH];
                 f32x16 init;
-                DmaTileF32::get(a_o, ob[0]);
                 DmaTileF32::get(a_go, go);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
@@ -1330,17 +1335,53 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
                     init[4 * g + 3] = v.w;
                 }
                 DmaTileF32::get(a_p, pc);
-                DmaTileF32::get(a_q, qb[0]);
-                wait_lgkm0();
-                if (i + 1 < nu) issue(dn);
-                dn = dnn;
-                __builtin_amdgcn_sched_barrier(0);
-                f32x16 dp = mma_feat_init<D>(go, vk, init);  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
+                DmaTileF32::get(a_p, qb[0], DmaTileF32::TILE);
+                f32x16 dp;  // dO_i . v_j - g_i, i = I*32+acc_row(r,h), j = J*32+li
                 float ds[16];
+                if constexpr (EXACT) {
+                    float ob[1][16];
+                    DmaTileF32::get(a_p, ob[0], 2 * DmaTileF32::TILE);
+                    wait_lgkm0();
+                    if (i + 1 < nu) {
+                        issue_pg(dn);
+                        issue_qo(dn);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    dp = mma_feat_init<D>(go, vk, init);
+                    mma_b_f32<D>(pc, ob, av);
+                } else {
+                    typedef DmaTile<32> Plane;
+                    wait_lgkm0();
+                    if (i + 1 < nu) issue_pg(dn);
+                    __builtin_amdgcn_sched_barrier(0);
+                    const Split3<16> gs = split3(go);
+                    const auto ra = Plane::row_addr(li, h);
+                    const auto ta = Plane::tr_addr(l);
+                    char* planes = const_cast<char*>(Tq);
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) *reinterpret_cast<bf16x8*>(planes + k * Plane::TILE + ra.a[t]) = gs.p[k][t];
+                    dp = mma_split(gs, vk, init);
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("" ::: "memory");  // same-wave LDS accesses complete in order
+                    Split3<16> ot;
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        bf16x8 x[1][2];
+                        Plane::get_tile_t(planes + k * Plane::TILE, ta, x);
+                        ot.p[k][0] = x[0][0];
+                        ot.p[k][1] = x[0][1];
+                    }
+                    wait_lgkm0();
+                    if (i + 1 < nu) issue_qo(dn);
+                    __builtin_amdgcn_sched_barrier(0);
+                    av[0] = mma_split(split3(pc), ot, av[0]);
+                }
+                dn = dnn;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pc[r];
                 mma_b_split<D, EXACT>(ds, qb, ak);
-                mma_b_split<D, EXACT>(pc, ob, av);
             }
         }
     } else {
