@@ -400,6 +400,7 @@ int spion_transpose_last2(const float* in, float* out, int batch, int rows, int 
  *   spion_project_backward_weight: dW [outputs][dim] = dY^T . X and db [outputs] = column sums of dY [rows][outputs];
  *                                  workspace: spion_project_workspace(rows, outputs, dim) floats, contents unspecified.
  *                                  The sum over the rows has a fixed order: the same inputs give the same bits.
+ *   spion_project_backward:        both, with segs * n outputs; the same bits as the two calls, in fewer launches.
  * Each returns 0 on success. */
 int spion_project_forward(const float* X, const float* const* W, const float* const* b, float* Y, long long rows, int n,
                           int segs, int dim, void* stream);
@@ -412,6 +413,8 @@ int spion_project_backward_input(const float* dY, const float* const* W, float* 
 long long spion_project_workspace(long long rows, int outputs, int dim);
 int spion_project_backward_weight(const float* dY, const float* X, float* dW, float* db, float* workspace, long long rows,
                                   int outputs, int dim, void* stream);
+int spion_project_backward(const float* dY, const float* const* W, const float* X, float* dX, float* dW, float* db,
+                           float* workspace, long long rows, int n, int segs, int dim, void* stream);
 
 /* mask [batch][seq_len] (1 = key, 0 = padding) -> penalty [batch*heads][seq_len] = 1e6 * (1 - mask), the Mask operand
  * of the key-mask entry points (models/attention_blockcuda_mask.py:42-43).  Returns 0 on success. */

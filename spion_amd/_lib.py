@@ -151,6 +151,8 @@ def core() -> ctypes.CDLL:
     lib.spion_project_workspace.restype = ctypes.c_longlong
     lib.spion_project_backward_weight.argtypes = [_P] * 5 + [ctypes.c_longlong, c_int, c_int, _P]
     lib.spion_project_backward_weight.restype = c_int
+    lib.spion_project_backward.argtypes = [_P] * 7 + [ctypes.c_longlong, c_int, c_int, c_int, _P]
+    lib.spion_project_backward.restype = c_int
     lib.spion_key_penalty.argtypes = [_P, _P, c_int, c_int, c_int, _P]
     lib.spion_key_penalty.restype = c_int
     lib.spion_score_map_mean.argtypes = [_P, c_int, c_int, c_int, c_int, _P, _P]

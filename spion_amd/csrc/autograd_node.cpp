@@ -510,14 +510,36 @@ bool projections_fit(const Tensor& x, const Tensor& wq, const Tensor& wk, const 
            projection_fits(x, wf, bf, outputs, n);
 }
 
-Tensor project_weight_grads(const float* dy, const Tensor& x, int64_t rows, int64_t outputs, int64_t dim, int64_t stream,
-                            Tensor& db) {
+// What a backward of `segs` projections of x to n outputs each is asked for: the gradients of x, in its memory layout, and of
+// weights and biases together.
+struct ProjectionGrads {
+    Tensor dx, dw, db;
+};
+ProjectionGrads project_backward(const float* dy, const Tensor* w, const Tensor& x, int64_t rows, int64_t n, int segs, int64_t dim,
+                                 int64_t stream, bool input, bool weights) {
     const auto opt = x.options();
-    Tensor dw = torch::empty({outputs, dim}, opt), ws = torch::empty({spion_project_workspace(rows, (int)outputs, (int)dim)}, opt);
-    db = torch::empty({outputs}, opt);
-    spion_project_backward_weight(dy, fp(x), fpm(dw), fpm(db), fpm(ws), rows, (int)outputs, (int)dim,
-                                  reinterpret_cast<void*>(stream));
-    return dw;
+    const int64_t outputs = segs * n;
+    void* s = reinterpret_cast<void*>(stream);
+    ProjectionGrads r;
+    const float* wp[3] = {};
+    if (input) {
+        r.dx = torch::empty_like(x);
+        for (int i = 0; i < segs; ++i) wp[i] = fp(w[i]);
+    }
+    Tensor ws;
+    if (weights) {
+        r.dw = torch::empty({outputs, dim}, opt);
+        ws = torch::empty({spion_project_workspace(rows, (int)outputs, (int)dim)}, opt);
+        r.db = torch::empty({outputs}, opt);
+    }
+    if (input && weights)
+        spion_project_backward(dy, wp, fp(x), fpm(r.dx), fpm(r.dw), fpm(r.db), fpm(ws), rows, (int)n, segs, (int)dim, s);
+    else if (input)
+        spion_project_backward_input(dy, wp, fpm(r.dx), rows, (int)n, segs, (int)dim, s);
+    else if (weights)
+        spion_project_backward_weight(dy, fp(x), fpm(r.dw), fpm(r.db), fpm(ws), rows, (int)outputs, (int)dim, s);
+    check_library("projection");
+    return r;
 }
 
 // What the nodes below saved, as hooks bring it back: the kernels take sizes from what was saved.
@@ -599,22 +621,16 @@ struct QkvNode : public torch::autograd::Function<QkvNode> {
             dy = fp(keep);
         }
         variable_list r(11);
-        if (ctx->needs_input_grad(0)) {
-            r[0] = torch::empty_like(x);
-            const Tensor w[3] = {aligned(saved[1]), aligned(saved[2]), aligned(saved[3])};
-            const float* wp[3] = {fp(w[0]), fp(w[1]), fp(w[2])};
-            spion_project_backward_input(dy, wp, fpm(r[0]), rows, (int)n, 3, (int)dim, reinterpret_cast<void*>(stream));
-        }
         bool any = false;
         for (int i = 1; i < 7; ++i) any = any || ctx->needs_input_grad(i);
-        if (any) {
-            Tensor db, dw = project_weight_grads(dy, x, rows, 3 * n, dim, stream, db);
+        const Tensor w[3] = {aligned(saved[1]), aligned(saved[2]), aligned(saved[3])};
+        const ProjectionGrads grads = project_backward(dy, w, x, rows, n, 3, dim, stream, ctx->needs_input_grad(0), any);
+        r[0] = grads.dx;
+        if (any)
             for (int i = 0; i < 3; ++i) {
-                r[1 + i] = dw.narrow(0, i * n, n);
-                r[4 + i] = db.narrow(0, i * n, n);
+                r[1 + i] = grads.dw.narrow(0, i * n, n);
+                r[4 + i] = grads.db.narrow(0, i * n, n);
             }
-        }
-        check_library("projection");
         return r;
     }
 };
@@ -658,14 +674,11 @@ struct MergeNode : public torch::autograd::Function<MergeNode> {
             return r;
         }
         const Tensor a = aligned(saved[0].transpose(1, 2)), w = aligned(saved[1]), dy = aligned(g[0]);
-        if (ctx->needs_input_grad(0)) {
-            Tensor da = torch::empty_like(a);
-            const float* wp[1] = {fp(w)};
-            spion_project_backward_input(fp(dy), wp, fpm(da), rows, (int)dim, 1, (int)n, reinterpret_cast<void*>(stream));
-            r[0] = da.transpose(1, 2);
-        }
-        if (ctx->needs_input_grad(1) || ctx->needs_input_grad(2)) r[1] = project_weight_grads(fp(dy), a, rows, dim, n, stream, r[2]);
-        check_library("projection");
+        const ProjectionGrads grads = project_backward(fp(dy), &w, a, rows, dim, 1, n, stream, ctx->needs_input_grad(0),
+                                                       ctx->needs_input_grad(1) || ctx->needs_input_grad(2));
+        if (grads.dx.defined()) r[0] = grads.dx.transpose(1, 2);
+        r[1] = grads.dw;
+        r[2] = grads.db;
         return r;
     }
 };

@@ -118,6 +118,7 @@ int project_forward(const float*, const float* const*, const float* const*, floa
 int project_backward_input(const float*, const float* const*, float*, long long, int, int, int, hipStream_t);
 long long project_workspace(long long, int, int);
 int project_backward_weight(const float*, const float*, float*, float*, float*, long long, int, int, hipStream_t);
+int project_backward(const float*, const float* const*, const float*, float*, float*, float*, float*, long long, int, int, int, hipStream_t);
 int key_penalty(const float*, float*, int, int, int, hipStream_t);
 int pattern_generate_maps(const float* const*, int, int, int, int, int, double, float*, int, float*, float*, hipStream_t);
 int score_map_mean(const float*, int, int, int, int, float*, hipStream_t, float post = 1.0f);
@@ -285,6 +286,11 @@ int spion_project_backward_weight(const float* dY, const float* X, float* dW, fl
                                   int outputs, int dim, void* stream) {
     note_current_handle(nullptr);
     return project_backward_weight(dY, X, dW, db, workspace, rows, outputs, dim, static_cast<hipStream_t>(stream));
+}
+int spion_project_backward(const float* dY, const float* const* W, const float* X, float* dX, float* dW, float* db,
+                           float* workspace, long long rows, int n, int segs, int dim, void* stream) {
+    note_current_handle(nullptr);
+    return project_backward(dY, W, X, dX, dW, db, workspace, rows, n, segs, dim, static_cast<hipStream_t>(stream));
 }
 int spion_key_penalty(const float* mask, float* penalty, int batch, int heads, int seq_len, void* stream) {
     note_current_handle(nullptr);

@@ -159,24 +159,22 @@ __device__ __forceinline__ void key_penalties(const KeyMask& k, int g) {
         k.pen[i] = 1e6f * (1.0f - k.mask[bh / k.H * k.L + (i - bh * k.L)]);
     }
 }
+struct Product {
+    SegRows A, B;
+    SegBias bias;
+    float* C;
+    float* Csum;
+    int ldc, M, N, R, chunks, mtiles, ntiles;
+};
 template <bool A_ACROSS, bool B_ACROSS, int WM, int WN, bool COLSUM>
-__global__ __launch_bounds__(256, 2) void project_kernel(SegRows A, SegRows B, SegBias bias, float* __restrict__ C, int ldc,
-                                                      float* __restrict__ Csum, int M, int N, int R, int chunks,
-                                                      int mtiles, int ntiles, KeyMask keys) {
-    int items = gridDim.x;
-    if constexpr (!A_ACROSS && !B_ACROSS) {
-        items -= keys.groups;
-        if ((int)blockIdx.x >= items) {
-            key_penalties(keys, blockIdx.x - items);
-            return;
-        }
-    }
+__device__ __forceinline__ void project_item(const Product& y, int item, char* smem) {
+    const SegRows A = y.A, B = y.B;
+    const SegBias bias = y.bias;
+    float *__restrict__ C = y.C, *__restrict__ Csum = y.Csum;
+    const int ldc = y.ldc, M = y.M, N = y.N, R = y.R, chunks = y.chunks, mtiles = y.mtiles, ntiles = y.ntiles;
     typedef OperandLds<A_ACROSS, WM> LA;
     typedef OperandLds<B_ACROSS, WN> LB;
-    extern __shared__ __attribute__((aligned(16))) char smem[];
     const int t = threadIdx.x, w = t >> 6, l = t & 63, h = l >> 5, li = l & 31;
-    // consecutive items share the rows of A (the larger operand) and run on one die
-    const int item = xcd_remap(blockIdx.x, items);
     const int nt = item % ntiles, mt = item / ntiles % mtiles, z = item / ntiles / mtiles;
     const int m0 = mt * 64 * WM, n0 = nt * 64 * WN;
     const int r0 = z * chunks * 32, nchunks = min(chunks, R / 32 - z * chunks);
@@ -333,6 +331,31 @@ __global__ __launch_bounds__(256, 2) void project_kernel(SegRows A, SegRows B, S
         }
     }
 }
+// consecutive items share the rows of A (the larger operand) and run on one die
+template <bool A_ACROSS, bool B_ACROSS, int WM, int WN, bool COLSUM>
+__global__ __launch_bounds__(256, 2) void project_kernel(Product y, KeyMask keys) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    int items = gridDim.x;
+    if constexpr (!A_ACROSS && !B_ACROSS) {
+        items -= keys.groups;
+        if ((int)blockIdx.x >= items) {
+            key_penalties(keys, blockIdx.x - items);
+            return;
+        }
+    }
+    project_item<A_ACROSS, B_ACROSS, WM, WN, COLSUM>(y, xcd_remap(blockIdx.x, items), smem);
+}
+// Both products of a backward, which read the same dY, in one launch: the pieces of dW (and db) first, whose work-groups live
+// longest, then the tiles of dX, which fill what those leave idle.  By themselves both wait for memory most of their time (3.3
+// TB/s of operands) and, at a few thousand rows, for a launch.  us, dX, then dW and db / in one launch, each with the launch
+// that adds the pieces: 65536 x 64 -> 192 37.1 / 34.3, 65536 x 64 -> 64 22.9 / 16.9, 16384 x 64 -> 192 20.9 / 16.0, 2048 x 64 -> 192 16.5 /
+// 10.7, 8192 x 128 -> 384 31.2 / 22.8, 524288 x 64 -> 192 254 / 243.  (As many registers as the larger of the two needs: with dX in
+// 128 x 128 tiles 242, so that two work-groups to a CU are left where dW had four: 32768 x 256 -> 768 183 / 208.)
+__global__ __launch_bounds__(256, 2) void project_backward_kernel(Product weight, Product input, int pieces) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    if ((int)blockIdx.x < pieces) project_item<true, true, 1, 1, true>(weight, xcd_remap(blockIdx.x, pieces), smem);
+    else project_item<false, true, 1, 1, false>(input, xcd_remap(blockIdx.x - pieces, gridDim.x - pieces), smem);
+}
 
 // out[i] = sum_z part[z][i] for the weight gradient and, behind it, the bias gradient; eight threads share a float4.
 __global__ __launch_bounds__(256) void project_reduce_kernel(const float* __restrict__ part, float* __restrict__ out,
@@ -358,6 +381,11 @@ __global__ __launch_bounds__(256) void project_reduce_kernel(const float* __rest
     }
 }
 
+template <int WM, int WN>
+static Product product(const SegRows& A, const SegRows& B, const SegBias& bias, float* C, int ldc, float* Csum, int M, int N,
+                       int R, int chunks) {
+    return Product{A, B, bias, C, Csum, ldc, M, N, R, chunks, (M + 64 * WM - 1) / (64 * WM), (N + 64 * WN - 1) / (64 * WN)};
+}
 template <bool AA, bool BA, int WM, int WN, bool CS>
 static bool launch_project(const SegRows& A, const SegRows& B, const SegBias& bias, float* C, int ldc, float* Csum, int M,
                            int N, int R, int pieces, int chunks, hipStream_t stream, const KeyMask& keys = KeyMask{}) {
@@ -367,9 +395,9 @@ static bool launch_project(const SegRows& A, const SegRows& B, const SegBias& bi
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (!SPION_HIP_OK(err)) return false;
     }
-    const int mt = (M + 64 * WM - 1) / (64 * WM), nt = (N + 64 * WN - 1) / (64 * WN);
-    hipLaunchKernelGGL((project_kernel<AA, BA, WM, WN, CS>), dim3((unsigned)mt * nt * pieces + keys.groups), dim3(256), lds,
-                       stream, A, B, bias, C, ldc, Csum, M, N, R, chunks, mt, nt, keys);
+    const Product y = product<WM, WN>(A, B, bias, C, ldc, Csum, M, N, R, chunks);
+    hipLaunchKernelGGL((project_kernel<AA, BA, WM, WN, CS>), dim3((unsigned)y.mtiles * y.ntiles * pieces + keys.groups), dim3(256),
+                       lds, stream, y, keys);
     return check_launch("project_kernel");
 }
 
@@ -452,20 +480,56 @@ static int weight_pieces(long long M, int N, int K) {
 long long project_workspace(long long M, int N, int K) {
     return (long long)weight_pieces(M, N, K) * ((long long)N * K + N);
 }
+// The pieces' results, `pieces` of [N][K] and of [N] behind them, to dW and db.
+static bool add_pieces(const float* ws, float* dW, float* db, int N, int K, int pieces, hipStream_t stream) {
+    const int n = N * K;
+    hipLaunchKernelGGL(project_reduce_kernel, dim3((n + N + 127) / 128), dim3(256), 0, stream, ws, dW, n,
+                       ws + (size_t)pieces * n, db, N, pieces);
+    return check_launch("project_reduce_kernel");
+}
+static void weight_split(long long M, int N, int K, int& pieces, int& chunks) {
+    const int want = weight_pieces(M, N, K), rows = (int)(M / 32);
+    chunks = (rows + want - 1) / want;
+    pieces = (rows + chunks - 1) / chunks;
+}
 int project_backward_weight(const float* dY, const float* X, float* dW, float* db, float* ws, long long M, int N, int K,
                             hipStream_t stream) {
     if (!project_args("spion_project_backward_weight", M, N, 1, K, {dY, X, dW, db, ws})) return 1;
-    const int want = weight_pieces(M, N, K), rows = (int)(M / 32);
-    const int chunks = (rows + want - 1) / want, pieces = (rows + chunks - 1) / chunks;
-    float* sums = ws + (size_t)pieces * N * K;
+    int pieces, chunks;
+    weight_split(M, N, K, pieces, chunks);
     const SegBias none{{nullptr, nullptr, nullptr}, ONE_PIECE};
-    if (!launch_project<true, true, 1, 1, true>(plain_rows(dY, N), plain_rows(X, K), none, ws, K, sums, N, K, (int)M, pieces,
-                                                chunks, stream))
+    return launch_project<true, true, 1, 1, true>(plain_rows(dY, N), plain_rows(X, K), none, ws, K, ws + (size_t)pieces * N * K, N,
+                                                  K, (int)M, pieces, chunks, stream) &&
+                   add_pieces(ws, dW, db, N, K, pieces, stream)
+               ? 0
+               : 1;
+}
+
+// dX, dW and db in one launch, and the one that adds the pieces; by the calls above where dX takes 128 x 128 tiles.
+int project_backward(const float* dY, const float* const* W, const float* X, float* dX, float* dW, float* db, float* ws,
+                     long long M, int n, int segs, int K, hipStream_t stream) {
+    if (!W || !project_args("spion_project_backward", M, n, segs, K, {dY, X, dX, dW, db, ws})) {
+        if (!W) set_error("spion_project_backward: null weights");
         return 1;
-    const int n = N * K;
-    hipLaunchKernelGGL(project_reduce_kernel, dim3((n + N + 127) / 128), dim3(256), 0, stream, ws, dW, n, sums, db, N,
-                       pieces);
-    return check_launch("project_reduce_kernel") ? 0 : 1;
+    }
+    for (int s = 0; s < segs; ++s)
+        if (!project_args("spion_project_backward", M, n, segs, K, {W[s]})) return 1;
+    const int N = segs * n;
+    if (wide_tiles(M, K)) {
+        const int err = project_backward_input(dY, W, dX, M, n, segs, K, stream);
+        return err ? err : project_backward_weight(dY, X, dW, db, ws, M, N, K, stream);
+    }
+    int pieces, chunks;
+    weight_split(M, N, K, pieces, chunks);
+    const SegBias none{{nullptr, nullptr, nullptr}, ONE_PIECE};
+    const Product weight = product<1, 1>(plain_rows(dY, N), plain_rows(X, K), none, ws, K, ws + (size_t)pieces * N * K, N, K, (int)M,
+                                         chunks),
+                  input = product<1, 1>(plain_rows(dY, N), weight_rows(W, segs, n, K), none, dX, K, nullptr, (int)M, K, N, N / 32);
+    const int wi = weight.mtiles * weight.ntiles * pieces;
+    constexpr int lds = OperandLds<true, 1>::BYTES + std::max(OperandLds<true, 1>::BYTES, OperandLds<false, 1>::BYTES);
+    hipLaunchKernelGGL(project_backward_kernel, dim3((unsigned)wi + (unsigned)input.mtiles * input.ntiles), dim3(256), lds, stream,
+                       weight, input, wi);
+    return check_launch("project_backward_kernel") && add_pieces(ws, dW, db, N, K, pieces, stream) ? 0 : 1;
 }
 
 __global__ __launch_bounds__(256) void key_penalty_kernel(KeyMask keys) { key_penalties(keys, blockIdx.x); }

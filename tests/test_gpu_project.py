@@ -60,6 +60,30 @@ def test_projection_kernels_match_float64(rows, dim, n, segs):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
+# one launch for dX, dW and db (and its limits: one piece, ragged pieces, tiles past the outputs), 128 x 128 tiles of dX (two calls)
+@pytest.mark.parametrize("rows,dim,n,segs", [(32, 32, 32, 1), (96, 64, 32, 2), (1056, 96, 96, 3), (2080, 64, 64, 3), (65536, 64, 64, 1),
+                                             (160, 160, 352, 1), (65536, 256, 128, 3)])
+def test_joint_backward_has_the_bits_of_the_two_calls(rows, dim, n, segs):
+    g = torch.Generator().manual_seed(rows + dim)
+    x = torch.randn(rows, dim, generator=g).cuda()
+    w = [torch.randn(n, dim, generator=g).cuda() for _ in range(segs)]
+    N = segs * n
+    dy = (torch.randn(rows, N, generator=g) + 0.5).cuda()
+    core, stream = _lib.core(), torch.cuda.current_stream().cuda_stream
+    ws = torch.empty(core.spion_project_workspace(rows, N, dim), device="cuda")
+    outs = [[torch.full((size + 4,), 7.0, device="cuda") for size in (rows * dim, N * dim, N)] for _ in range(2)]
+    dx, dw, db = (t.data_ptr() for t in outs[0])
+    assert core.spion_project_backward(dy.data_ptr(), _ptrs(w), x.data_ptr(), dx, dw, db, ws.data_ptr(), rows, n, segs, dim, stream) == 0
+    dx, dw, db = (t.data_ptr() for t in outs[1])
+    assert core.spion_project_backward_input(dy.data_ptr(), _ptrs(w), dx, rows, n, segs, dim, stream) == 0
+    assert core.spion_project_backward_weight(dy.data_ptr(), x.data_ptr(), dw, db, ws.data_ptr(), rows, N, dim, stream) == 0
+    for a, b in zip(*outs):
+        assert torch.equal(a, b) and bool((a[-4:] == 7.0).all())
+    for args in ((None, x.data_ptr(), dx), (_ptrs(w), None, dx), (_ptrs(w), x.data_ptr(), None)):
+        assert core.spion_project_backward(dy.data_ptr(), *args, dw, db, ws.data_ptr(), rows, n, segs, dim, stream) != 0
+        _lib.core().spion_clear_error()
+
+
 def _kinds(x):
     return torch.isposinf(x) + 2 * torch.isneginf(x) + 3 * torch.isnan(x)
 
