@@ -1150,54 +1150,43 @@ __global__ __launch_bounds__(256) void bf16_merge_fwd_kernel(const float* __rest
     const int4 d = reinterpret_cast<const int4*>(desc)[item % n_long];
     const float* p0 = Part + ((size_t)bh * n_slots + d.y) * PSZ;
     const float* st = p0 + 2 * 32 * D;  // {m[32], z[32]} of chunk 0
-    __shared__ float sm[32], sr[32];
-    const int t = threadIdx.x;
-    if (t < 32) {
-        float M = -3.0e38f;
-        for (int c0 = 0; c0 < d.z; c0 += 8) {
-            float mm[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) mm[k] = st[(size_t)min(c0 + k, d.z - 1) * PSZ + t];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) M = fmaxf(M, mm[k]);
-        }
-        float Z = 0.f;
-        for (int c0 = 0; c0 < d.z; c0 += 8) {
-            float mm[8], zz[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                mm[k] = st[(size_t)min(c0 + k, d.z - 1) * PSZ + t];
-                zz[k] = st[(size_t)min(c0 + k, d.z - 1) * PSZ + 32 + t];
-            }
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (c0 + k < d.z) Z += zz[k] * __builtin_amdgcn_exp2f(mm[k] - M);
-        }
-        const int off_pattern = L - d.w * 32;
-        if (off_pattern > 0) Z += (float)off_pattern * __builtin_amdgcn_exp2f(-M);  // models/block_attn.cu:74
-        sm[t] = M;
-        sr[t] = 1.0f / Z;
-        if (eb == 0) Lse[(size_t)bh * L + d.x * 32 + t] = M + __builtin_amdgcn_logf(Z);
-    }
-    __syncthreads();
-    const int e = eb * 256 + t;
+    const int e = eb * 256 + threadIdx.x;
     const int l = e & 63, r = (e >> 6) & 15, c = e >> 10, row = l & 31;
-    float v = 0.f;
-    for (int c0 = 0; c0 < d.z; c0 += 8) {
-        float x[8], mm[8];
+    // Every thread merges its row's statistics for itself: all it needs of the first eight chunks is requested at once, and
+    // the kernel, which is a chain of look-ups, has one fewer of them and no barrier.  (One thread a row for all, its result
+    // through LDS and the values requested after that: 5.0 us against 3.9, 32 heads of 4096 tokens.)
+    float mm[8], zz[8], x[8];
+    auto request = [&](int c0) {
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            x[k] = p0[(size_t)min(c0 + k, d.z - 1) * PSZ + e];
-            mm[k] = st[(size_t)min(c0 + k, d.z - 1) * PSZ + row];
+            const size_t o = (size_t)min(c0 + k, d.z - 1) * PSZ;
+            mm[k] = st[o + row];
+            zz[k] = st[o + 32 + row];
+            x[k] = p0[o + e];
         }
+    };
+    request(0);
+    float M = -3.0e38f, Z = 0.f, v = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) M = fmaxf(M, mm[k]);
+    for (int k = 8; k < d.z; ++k) M = fmaxf(M, st[(size_t)k * PSZ + row]);
+    for (int c0 = 0; c0 < d.z; c0 += 8) {
+        if (c0) request(c0);
 #pragma unroll
         for (int k = 0; k < 8; ++k)
-            if (c0 + k < d.z) v += x[k] * __builtin_amdgcn_exp2f(mm[k] - sm[row]);
+            if (c0 + k < d.z) {
+                const float f = __builtin_amdgcn_exp2f(mm[k] - M);
+                Z += zz[k] * f;
+                v += x[k] * f;
+            }
     }
+    const int off_pattern = L - d.w * 32;
+    if (off_pattern > 0) Z += (float)off_pattern * __builtin_amdgcn_exp2f(-M);  // models/block_attn.cu:74
+    if (e < 32) Lse[(size_t)bh * L + d.x * 32 + row] = M + __builtin_amdgcn_logf(Z);
     size_t ob, obytes;
     int old_;
     bf16_head<ST, D>(lay, H, bh, L, ob, old_, obytes);
-    O[ob + (size_t)(d.x * 32 + row) * old_ + 32 * c + acc_row(r, l >> 5)] = (__bf16)(v * sr[row]);
+    O[ob + (size_t)(d.x * 32 + row) * old_ + 32 * c + acc_row(r, l >> 5)] = (__bf16)(v * (1.0f / Z));
 }
 
 // Plain sums (backward): out0 from the first 32 x D block of the slots, out1 (column pass: dV; grid twice as
