@@ -392,6 +392,27 @@ void spion_dense_forward_strided_mean(void* handle, const float* Q, const float*
  * attention entry points take.  Returns 0 on success. */
 int spion_transpose_last2(const float* in, float* out, int batch, int rows, int cols, void* stream);
 
+/* The forwards of the key-mask handles on the mask itself -- [num_batches / heads][seq_len], 1 = key, 0 = padding, heads heads
+ * a sample -- in the place of the penalties that spion_key_penalty makes of it: the kernels form them as they read it, and a
+ * call has one launch and one [num_batches][seq_len] array fewer.  mask: 16-byte aligned.  Mean: null, or where the mean map
+ * goes. */
+void spion_attn_forward_rowmajor_keys(void* handle, const float* Q, const float* K, const float* V, const float* mask, int heads,
+                                      float* Attn, float* Out, const int* Offsets, const int* Columns, const int* SumMat,
+                                      int nnz);
+void spion_attn_forward_strided_keys(void* handle, const float* Q, const float* K, const float* V, const float* mask,
+                                     float* Attn, float* Out, const int* Offsets, const int* Columns, const int* SumMat,
+                                     int nnz, int heads, const spion_head_layout* in, const spion_head_layout* out);
+void spion_dense_forward_strided_keys(void* handle, const float* Q, const float* K, const float* V, const float* mask,
+                                      float* Attn, float* Out, float* Mean, int heads, const spion_head_layout* in,
+                                      const spion_head_layout* out);
+void spion_block_bf16_attn_forward_keys(void* handle, const void* Q, const void* K, const void* V, const float* mask, int heads,
+                                        void* Out, float* Lse, const int* Offsets, const int* Columns, const int* SumMat,
+                                        int nnz);
+void spion_block_bf16_attn_forward_strided_keys(void* handle, const void* Q, const void* K, const void* V, const float* mask,
+                                                void* Out, float* Lse, const int* Offsets, const int* Columns,
+                                                const int* SumMat, int nnz, int heads, const spion_head_layout* in,
+                                                const spion_head_layout* out);
+
 /* The projections around the attention core (models/attention.py:84-103: three nn.Linear into the heads, one out of
  * them), fp32, all matrices row-major and 16-byte aligned, rows, n and dim multiples of 32.
  *   spion_project_forward:         Y [rows][segs*n] = X [rows][dim] . W^T + b.  W, b: HOST arrays of segs (1 to 3) device

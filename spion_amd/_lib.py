@@ -128,6 +128,16 @@ def core() -> ctypes.CDLL:
     lib.spion_dense_forward_strided.restype = None
     lib.spion_dense_forward_strided_mean.argtypes = [_P] * 8 + [c_int, _P, _P]
     lib.spion_dense_forward_strided_mean.restype = None
+    lib.spion_attn_forward_rowmajor_keys.argtypes = [_P] * 5 + [c_int] + [_P] * 5 + [c_int]
+    lib.spion_attn_forward_rowmajor_keys.restype = None
+    lib.spion_attn_forward_strided_keys.argtypes = [_P] * 10 + [c_int, c_int, _P, _P]
+    lib.spion_attn_forward_strided_keys.restype = None
+    lib.spion_dense_forward_strided_keys.argtypes = [_P] * 8 + [c_int, _P, _P]
+    lib.spion_dense_forward_strided_keys.restype = None
+    lib.spion_block_bf16_attn_forward_keys.argtypes = [_P] * 5 + [c_int] + [_P] * 5 + [c_int]
+    lib.spion_block_bf16_attn_forward_keys.restype = None
+    lib.spion_block_bf16_attn_forward_strided_keys.argtypes = [_P] * 10 + [c_int, c_int, _P, _P]
+    lib.spion_block_bf16_attn_forward_strided_keys.restype = None
     lib.spion_transition_update.argtypes = [_P, _P, c_int, ctypes.c_longlong, _P, _P, c_int, c_int, _P]
     lib.spion_transition_update.restype = c_int
     lib.spion_dense_backward_strided.argtypes = [_P] * 10 + [c_int, _P, _P, _P]

@@ -160,9 +160,8 @@ class _BlockAttentionBase(nn.Module):
 
 
     def key_operand(self, mask):
-        """What the compiled node takes for the key mask: (mask, True) when the library makes the penalties from it
-        (spion_key_penalty: one launch where the expression below is three or four), (penalties [B, H*L], False) for a
-        mask of another type or layout, (None, False) without one."""
+        """What the compiled node takes for the key mask: (mask, True) when the kernels read it themselves, (penalties
+        [B, H*L], False) for a mask of another type or layout, (None, False) without one."""
         if not self.with_mask:
             return None, False
         if mask.dtype == torch.float32 and mask.is_cuda and mask.is_contiguous() and not mask.requires_grad \

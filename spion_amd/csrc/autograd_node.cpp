@@ -159,7 +159,8 @@ struct CoreResult {
     bool strided = false, tiled = false;
 };
 
-CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& pen,
+// pen: penalties [B, H*L] (mask_heads 0), a key mask [B, L] of mask_heads heads a sample, or nothing.
+CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& pen, int64_t mask_heads,
                         const Tensor& offsets, const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz,
                         int64_t num_heads, bool reads_views, int64_t stream) {
     void* h = reinterpret_cast<void*>(handle);
@@ -173,7 +174,9 @@ CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& va
     TORCH_CHECK_VALUE(B * H == hnb && H == num_heads && query.size(2) == hl && query.size(3) == hd, "query shape ",
                       query.sizes(), " does not match the handle (", hnb, " heads in all, ", num_heads, " a sample, ", hl,
                       " rows of ", hd, ")");
-    TORCH_CHECK_VALUE(!pen.defined() || pen.numel() >= B * H * query.size(2), "key mask smaller than [B, L]");
+    TORCH_CHECK_VALUE(!pen.defined() || (mask_heads ? mask_heads == H && pen.numel() >= B * query.size(2)
+                                                    : pen.numel() >= B * H * query.size(2)),
+                      "key mask smaller than [B, L]");
     for (const Tensor* t : {&query, &key, &value, &pen})
         TORCH_CHECK(!t->defined() || (t->scalar_type() == torch::kFloat32 && t->device() == query.device() && t->is_cuda()),
                     "fp32 tensors on one GPU expected");
@@ -190,15 +193,20 @@ CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& va
         r.v = value;
         r.out = empty_heads(query.sizes(), query.stride(1) < query.stride(2), opt);
         head_layout(r.out, lout);
-        spion_attn_forward_strided(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.p_flat), fpm(r.out), ip(offsets),
-                                   ip(columns), ip(sum_mat), (int)nnz, (int)num_heads, &lin, &lout);
+        (mask_heads ? spion_attn_forward_strided_keys : spion_attn_forward_strided)(
+            h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.p_flat), fpm(r.out), ip(offsets), ip(columns), ip(sum_mat), (int)nnz,
+            (int)num_heads, &lin, &lout);
     } else {
         r.q = query.contiguous();
         r.k = key.contiguous();
         r.v = value.contiguous();
         r.out = torch::empty(query.sizes(), opt);
-        spion_attn_forward_rowmajor(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.p_flat), fpm(r.out), ip(offsets),
-                                    ip(columns), ip(sum_mat), (int)nnz);
+        if (mask_heads)
+            spion_attn_forward_rowmajor_keys(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), (int)mask_heads, fpm(r.p_flat), fpm(r.out),
+                                             ip(offsets), ip(columns), ip(sum_mat), (int)nnz);
+        else
+            spion_attn_forward_rowmajor(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.p_flat), fpm(r.out), ip(offsets),
+                                        ip(columns), ip(sum_mat), (int)nnz);
     }
     check_library("attn_forward");
     r.tiled = spion_last_path(h) == 1;
@@ -206,15 +214,15 @@ CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& va
 }
 
 struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
-    // pen_opt: [B, H*L] key penalties of the key-mask modules, or nothing.  stream: torch's current raw stream at the
+    // pen_opt, mask_heads: key penalties or the key mask of the key-mask modules, or nothing (core_forward).  stream: torch's current raw stream at the
     // call.  fixed: takes what carries no gradient, the probabilities of the key-mask modules (compiled autograd refuses
     // nodes with outputs that are marked so).
     static variable_list forward(AutogradContext* ctx, Tensor query, Tensor key, Tensor value,
-                                 c10::optional<Tensor> pen_opt, Tensor offsets, Tensor columns, Tensor sum_mat, int64_t handle, int64_t nnz,
-                                 int64_t num_heads, bool reads_views, int64_t stream, Tensor* fixed) {
+                                 c10::optional<Tensor> pen_opt, int64_t mask_heads, Tensor offsets, Tensor columns,
+                                 Tensor sum_mat, int64_t handle, int64_t nnz, int64_t num_heads, bool reads_views, int64_t stream, Tensor* fixed) {
         const Tensor pen = pen_opt.has_value() ? *pen_opt : Tensor();
-        CoreResult r = core_forward(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, num_heads, reads_views,
-                                    stream);
+        CoreResult r = core_forward(query, key, value, pen, mask_heads, offsets, columns, sum_mat, handle, nnz, num_heads,
+                                    reads_views, stream);
         // which kernel family serves THIS pattern (the handle may run other patterns before the backward)
         ctx->saved_data["tiled"] = r.tiled;
         keep_handle(ctx, handle);
@@ -283,7 +291,11 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
                                          ip(offsets), ip(columns), ip(sum_mat), (int)nnz);
         }
         check_library("attn_backward");
-        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        variable_list r(14);
+        r[0] = dq;
+        r[1] = dk;
+        r[2] = dv;
+        return r;
     }
 };
 
@@ -294,14 +306,30 @@ Tensor key_penalty(const Tensor& mask, int64_t heads, int64_t stream) {
     check_library("attn_forward");
     return pen;
 }
-// The modules hand over a key mask, or penalties made from one the kernel does not take (is_mask = false); either has to lie
-// on the device of the heads.
+// The modules hand over a key mask, or penalties made from one the kernels do not take (is_mask = false); either has to lie on
+// the device of the heads.  Where the forward's kernels alone need it, they read a mask of the heads' sizes themselves.
+struct KeyOperand {
+    c10::optional<Tensor> t;
+    int64_t mask_heads = 0;  // 0: penalties
+    Tensor or_none() const { return t.has_value() ? *t : Tensor(); }
+};
 c10::optional<Tensor> penalty_of(const c10::optional<Tensor>& mask_or_pen, bool is_mask, int64_t heads, c10::Device device,
                                  int64_t stream) {
     TORCH_CHECK(!mask_or_pen.has_value() || mask_or_pen->device() == device, "fp32 tensors on one GPU expected");
     if (!is_mask || !mask_or_pen.has_value()) return mask_or_pen;
     if (has_tangent(*mask_or_pen)) return (1e6 * (1.0 - mask_or_pen->repeat({1, heads}))).contiguous();
     return key_penalty(*mask_or_pen, heads, stream);
+}
+
+KeyOperand key_operand(const c10::optional<Tensor>& mask_or_pen, bool is_mask, int64_t batch, int64_t heads, int64_t length,
+                       c10::Device device, int64_t stream) {
+    if (is_mask && mask_or_pen.has_value() && !has_tangent(*mask_or_pen)) {
+        const Tensor& m = *mask_or_pen;
+        if (m.device() == device && m.is_cuda() && m.scalar_type() == torch::kFloat32 && m.dim() == 2 && m.size(0) == batch &&
+            m.size(1) == length && m.is_contiguous() && !m.requires_grad() && reinterpret_cast<uintptr_t>(m.data_ptr()) % 16 == 0)
+            return {mask_or_pen, heads};
+    }
+    return {penalty_of(mask_or_pen, is_mask, heads, device, stream), 0};
 }
 
 // The gradient of a core's output in that output's strides, as the strided entry points take it.
@@ -315,8 +343,8 @@ Tensor grad_like(const Tensor& go, const Tensor& out) {
 struct DenseResult {
     Tensor q, k, v, attn, out, mean;  // attn: memory [key][query]
 };
-DenseResult dense_forward(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& pen, int64_t handle,
-                          bool emit_mean, int64_t stream) {
+DenseResult dense_forward(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& pen, int64_t mask_heads,
+                          int64_t handle, bool emit_mean, int64_t stream) {
     void* h = reinterpret_cast<void*>(handle);
     spion_set_stream(h, reinterpret_cast<void*>(stream));
     const auto opt = query.options();
@@ -332,8 +360,11 @@ DenseResult dense_forward(const Tensor& query, const Tensor& key, const Tensor& 
     r.attn = torch::empty({B, H, L, L}, opt);
     r.out = empty_heads(query.sizes(), r.q.stride(1) < r.q.stride(2), opt);
     head_layout(r.out, lout);
-    if (emit_mean) {
-        r.mean = torch::empty({L, L}, opt);
+    if (emit_mean) r.mean = torch::empty({L, L}, opt);
+    if (mask_heads) {
+        spion_dense_forward_strided_keys(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.attn), fpm(r.out),
+                                         emit_mean ? fpm(r.mean) : nullptr, (int)H, &lin, &lout);
+    } else if (emit_mean) {
         spion_dense_forward_strided_mean(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.attn), fpm(r.out), fpm(r.mean), (int)H,
                                          &lin, &lout);
     } else {
@@ -344,8 +375,8 @@ DenseResult dense_forward(const Tensor& query, const Tensor& key, const Tensor& 
 }
 struct DenseAttnNode : public torch::autograd::Function<DenseAttnNode> {
     static variable_list forward(AutogradContext* ctx, Tensor query, Tensor key, Tensor value, c10::optional<Tensor> pen,
-                                 int64_t handle, bool emit_mean, int64_t stream, Tensor* mean) {
-        DenseResult r = dense_forward(query, key, value, pen.has_value() ? *pen : Tensor(), handle, emit_mean, stream);
+                                 int64_t mask_heads, int64_t handle, bool emit_mean, int64_t stream, Tensor* mean) {
+        DenseResult r = dense_forward(query, key, value, pen.has_value() ? *pen : Tensor(), mask_heads, handle, emit_mean, stream);
         keep_handle(ctx, handle);
         keep_sizes(ctx, r.q);
         ctx->save_for_backward({r.q, r.k, r.v, r.attn, r.out});
@@ -381,7 +412,7 @@ struct DenseAttnNode : public torch::autograd::Function<DenseAttnNode> {
         spion_dense_backward_strided(h, fp(q), fp(k), fp(v), fp(attn), fp(out), fp(go), fpm(dq), fpm(dk), fpm(dv), (int)q.size(1),
                                      &lin, &lout, &lgrad);
         check_library("attn_backward");
-        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -391,8 +422,8 @@ struct BF16Result {
     bool strided = false;
 };
 const void* vp(const Tensor& t) { return t.data_ptr(); }
-BF16Result bf16_forward(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& pen, const Tensor& offsets,
-                        const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t stream) {
+BF16Result bf16_forward(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& pen, int64_t mask_heads,
+                        const Tensor& offsets, const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t stream) {
     void* h = reinterpret_cast<void*>(handle);
     spion_set_stream(h, reinterpret_cast<void*>(stream));
     const auto opt = query.options().dtype(torch::kBFloat16);
@@ -412,15 +443,20 @@ BF16Result bf16_forward(const Tensor& query, const Tensor& key, const Tensor& va
         r.v = value;
         r.out = empty_heads(query.sizes(), query.stride(1) < query.stride(2), opt);
         head_layout(r.out, lout);
-        spion_block_bf16_attn_forward_strided(h, vp(r.q), vp(r.k), vp(r.v), fp(pen), r.out.data_ptr(), fpm(r.lse), ip(offsets),
-                                              ip(columns), ip(sum_mat), (int)nnz, (int)H, &lin, &lout);
+        (mask_heads ? spion_block_bf16_attn_forward_strided_keys : spion_block_bf16_attn_forward_strided)(
+            h, vp(r.q), vp(r.k), vp(r.v), fp(pen), r.out.data_ptr(), fpm(r.lse), ip(offsets), ip(columns), ip(sum_mat), (int)nnz,
+            (int)H, &lin, &lout);
     } else {
         r.q = query.to(torch::kBFloat16).contiguous();
         r.k = key.to(torch::kBFloat16).contiguous();
         r.v = value.to(torch::kBFloat16).contiguous();
         r.out = torch::empty(query.sizes(), opt);
-        spion_block_bf16_attn_forward(h, vp(r.q), vp(r.k), vp(r.v), fp(pen), r.out.data_ptr(), fpm(r.lse), ip(offsets),
-                                      ip(columns), ip(sum_mat), (int)nnz);
+        if (mask_heads)
+            spion_block_bf16_attn_forward_keys(h, vp(r.q), vp(r.k), vp(r.v), fp(pen), (int)mask_heads, r.out.data_ptr(), fpm(r.lse),
+                                               ip(offsets), ip(columns), ip(sum_mat), (int)nnz);
+        else
+            spion_block_bf16_attn_forward(h, vp(r.q), vp(r.k), vp(r.v), fp(pen), r.out.data_ptr(), fpm(r.lse), ip(offsets),
+                                          ip(columns), ip(sum_mat), (int)nnz);
     }
     check_library("spion_block_bf16_attn_forward");
     return r;
@@ -429,7 +465,7 @@ struct BF16AttnNode : public torch::autograd::Function<BF16AttnNode> {
     static Tensor forward(AutogradContext* ctx, Tensor query, Tensor key, Tensor value, c10::optional<Tensor> pen_opt,
                           Tensor offsets, Tensor columns, Tensor sum_mat, int64_t handle, int64_t nnz, int64_t stream) {
         const Tensor pen = pen_opt.has_value() ? *pen_opt : Tensor();
-        const BF16Result r = bf16_forward(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, stream);
+        const BF16Result r = bf16_forward(query, key, value, pen, 0, offsets, columns, sum_mat, handle, nnz, stream);
         keep_handle(ctx, handle);
         ctx->saved_data["nnz"] = nnz;
         ctx->saved_data["strided"] = r.strided;
@@ -550,15 +586,9 @@ const Tensor& saved_as(const Tensor& t, c10::IntArrayRef sizes, int64_t device) 
     return t;
 }
 
-// A [B, L] key mask whose penalties the launch of the input projections is to make as well (null: none).
-struct KeyMask {
-    const float* mask = nullptr;
-    float* pen = nullptr;
-    int batch = 0, heads = 0, length = 0;
-};
 // X [B, L, dim] -> the [B, H, L, d] heads of the three projections, slices of one [B, L, 3, H, d] buffer.
 std::vector<Tensor> qkv_forward(const Tensor& x, const Tensor (&w)[3], const Tensor (&b)[3], int64_t H, int64_t d,
-                                int64_t stream, const KeyMask* keys = nullptr) {
+                                int64_t stream) {
     TORCH_CHECK_VALUE(x.dim() == 3, "projection: input [B, L, features] expected");
     const int64_t B = x.size(0), L = x.size(1), dim = x.size(2);
     for (int i = 0; i < 3; ++i) check_projection(x, w[i], b[i], H * d, dim);
@@ -566,11 +596,7 @@ std::vector<Tensor> qkv_forward(const Tensor& x, const Tensor (&w)[3], const Ten
     Tensor buf = torch::empty({B, L, 3, H, d}, x.options());
     const float* wp[3] = {fp(w[0]), fp(w[1]), fp(w[2])};
     const float* bp[3] = {fp(b[0]), fp(b[1]), fp(b[2])};
-    if (keys && keys->mask)
-        spion_project_forward_keys(fp(x), wp, bp, fpm(buf), B * L, (int)(H * d), 3, (int)dim, keys->mask, keys->pen, keys->batch,
-                                   keys->heads, keys->length, reinterpret_cast<void*>(stream));
-    else
-        spion_project_forward(fp(x), wp, bp, fpm(buf), B * L, (int)(H * d), 3, (int)dim, reinterpret_cast<void*>(stream));
+    spion_project_forward(fp(x), wp, bp, fpm(buf), B * L, (int)(H * d), 3, (int)dim, reinterpret_cast<void*>(stream));
     check_library("projection");
     std::vector<Tensor> out;
     for (int i = 0; i < 3; ++i)  // the slice [:, :, i].transpose(1, 2)
@@ -582,14 +608,14 @@ std::vector<Tensor> qkv_forward(const Tensor& x, const Tensor (&w)[3], const Ten
 // (create_graph): the kernels would leave no graph, and second-order terms would be lost without a word.
 struct QkvNode : public torch::autograd::Function<QkvNode> {
     static variable_list forward(AutogradContext* ctx, Tensor x, Tensor wq, Tensor wk, Tensor wv, Tensor bq, Tensor bk,
-                                 Tensor bv, int64_t H, int64_t d, int64_t stream, const KeyMask* keys) {
+                                 Tensor bv, int64_t H, int64_t d, int64_t stream) {
         const Tensor w[3] = {aligned(wq), aligned(wk), aligned(wv)}, b[3] = {aligned(bq), aligned(bk), aligned(bv)};
         ctx->save_for_backward({x, wq, wk, wv});
         ctx->saved_data["H"] = H;
         ctx->saved_data["d"] = d;
         ctx->saved_data["x_sizes"] = x.sizes().vec();
         ctx->saved_data["device"] = static_cast<int64_t>(x.device().index());
-        return qkv_forward(aligned(x), w, b, H, d, stream, keys);
+        return qkv_forward(aligned(x), w, b, H, d, stream);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
@@ -605,7 +631,7 @@ struct QkvNode : public torch::autograd::Function<QkvNode> {
             const Tensor dy = torch::stack({g[0].transpose(1, 2), g[1].transpose(1, 2), g[2].transpose(1, 2)}, 2)
                                   .reshape({rows, 3 * n});
             const Tensor dw = dy.t().matmul(saved[0].reshape({rows, dim})), db = dy.sum(0);
-            variable_list r(11);
+            variable_list r(10);
             r[0] = dy.matmul(torch::cat({saved[1], saved[2], saved[3]}, 0)).view({B, L, dim});
             for (int i = 0; i < 3; ++i) {
                 r[1 + i] = dw.narrow(0, i * n, n);
@@ -620,7 +646,7 @@ struct QkvNode : public torch::autograd::Function<QkvNode> {
             keep = torch::stack({g[0].transpose(1, 2), g[1].transpose(1, 2), g[2].transpose(1, 2)}, 2).contiguous();
             dy = fp(keep);
         }
-        variable_list r(11);
+        variable_list r(10);
         bool any = false;
         for (int i = 1; i < 7; ++i) any = any || ctx->needs_input_grad(i);
         const Tensor w[3] = {aligned(saved[1]), aligned(saved[2]), aligned(saved[3])};
@@ -691,27 +717,19 @@ std::vector<Tensor> sparse_layer(const Tensor& x, const Tensor& wq, const Tensor
                                  const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t num_heads, int64_t head_dim,
                                  int64_t stream) {
     const c10::DeviceGuard on(x.device());  // `stream` is one of x's device, which need not be the current one
-    // the penalties of a plain key mask come out of the projections' launch
-    KeyMask keys;
-    c10::optional<Tensor> pen;
-    if (is_mask && mask_or_pen.has_value() && mask_or_pen->device() == x.device() && !has_tangent(*mask_or_pen)) {
-        const Tensor& mask = *mask_or_pen;
-        pen = torch::empty({mask.size(0), num_heads * mask.size(1)}, mask.options());
-        keys = {fp(mask), fpm(*pen), (int)mask.size(0), (int)num_heads, (int)mask.size(1)};
-    } else {
-        pen = penalty_of(mask_or_pen, is_mask, num_heads, x.device(), stream);
-    }
-    const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
+    TORCH_CHECK_VALUE(x.dim() == 3, "projection: input [B, L, features] expected");
+    const KeyOperand keys = key_operand(mask_or_pen, is_mask, x.size(0), num_heads, x.size(1), x.device(), stream);
+    const Tensor pen_or_none = keys.or_none();
     if (without_node({&x, &wq, &wk, &wv, &bq, &bk, &bv, &wf, &bf, &pen_or_none})) {
         const Tensor w[3] = {aligned(wq), aligned(wk), aligned(wv)}, b[3] = {aligned(bq), aligned(bk), aligned(bv)};
-        const auto qkv = qkv_forward(aligned(x), w, b, num_heads, head_dim, stream, &keys);
-        const CoreResult r = core_forward(qkv[0], qkv[1], qkv[2], pen_or_none, offsets, columns, sum_mat, handle,
+        const auto qkv = qkv_forward(aligned(x), w, b, num_heads, head_dim, stream);
+        const CoreResult r = core_forward(qkv[0], qkv[1], qkv[2], pen_or_none, keys.mask_heads, offsets, columns, sum_mat, handle,
                                           nnz, num_heads, true, stream);
         return {merge_forward(aligned(r.out.transpose(1, 2)), aligned(wf), aligned(bf), stream), r.p_flat};
     }
-    const auto qkv = QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream, (const KeyMask*)&keys);
+    const auto qkv = QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream);
     Tensor fixed;
-    const auto core = SparseAttnNode::apply(qkv[0], qkv[1], qkv[2], pen, offsets, columns, sum_mat, handle, nnz, num_heads,
+    const auto core = SparseAttnNode::apply(qkv[0], qkv[1], qkv[2], keys.t, keys.mask_heads, offsets, columns, sum_mat, handle, nnz, num_heads,
                                             true, stream, &fixed);
     return {MergeNode::apply(core[0], wf, bf, stream), core.size() > 1 ? core[1] : fixed};
 }
@@ -720,7 +738,7 @@ std::vector<Tensor> sparse_layer(const Tensor& x, const Tensor& wq, const Tensor
 std::vector<Tensor> project_heads(const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& bq,
                                   const Tensor& bk, const Tensor& bv, int64_t num_heads, int64_t head_dim, int64_t stream) {
     const c10::DeviceGuard on(x.device());
-    return QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream, (const KeyMask*)nullptr);
+    return QkvNode::apply(x, wq, wk, wv, bq, bk, bv, num_heads, head_dim, stream);
 }
 Tensor merge_heads(const Tensor& heads, const Tensor& w, const Tensor& b, int64_t stream) {
     const c10::DeviceGuard on(heads.device());
@@ -732,25 +750,28 @@ std::vector<Tensor> sparse_attention(const Tensor& query, const Tensor& key, con
                                      const Tensor& columns, const Tensor& sum_mat, int64_t handle, int64_t nnz, int64_t num_heads,
                                      bool reads_views, int64_t stream) {
     const c10::DeviceGuard on(query.device());
-    const auto pen = penalty_of(mask_or_pen, is_mask, num_heads, query.device(), stream);
-    const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
+    const bool heads = query.dim() == 4;  // (core_forward asks for them)
+    const KeyOperand keys = key_operand(mask_or_pen, is_mask, heads ? query.size(0) : -1, num_heads, heads ? query.size(2) : -1,
+                                        query.device(), stream);
+    const Tensor pen_or_none = keys.or_none();
     if (without_node({&query, &key, &value, &pen_or_none})) {
-        const CoreResult r = core_forward(query, key, value, pen_or_none, offsets, columns, sum_mat, handle, nnz,
+        const CoreResult r = core_forward(query, key, value, pen_or_none, keys.mask_heads, offsets, columns, sum_mat, handle, nnz,
                                           num_heads, reads_views, stream);
         return {r.out, r.p_flat};
     }
     Tensor fixed;
-    auto r = SparseAttnNode::apply(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, num_heads, reads_views,
+    auto r = SparseAttnNode::apply(query, key, value, keys.t, keys.mask_heads, offsets, columns, sum_mat, handle, nnz, num_heads, reads_views,
                                    stream, &fixed);
     if (r.size() == 1) r.push_back(fixed);
     return r;
 }
 
 // The kernels read a penalty for every key of every head: fewer, or a tensor elsewhere, would be read past its end.
-void check_penalties(const Tensor& pen, const Tensor& query) {
+void check_penalties(const Tensor& pen, int64_t mask_heads, const Tensor& query) {
     if (!pen.defined()) return;
     TORCH_CHECK(pen.scalar_type() == torch::kFloat32 && pen.device() == query.device(), "fp32 tensors on one GPU expected");
-    TORCH_CHECK_VALUE(pen.numel() >= query.size(0) * query.size(1) * query.size(2), "key mask smaller than [B, L]");
+    TORCH_CHECK_VALUE(pen.numel() >= query.size(0) * (mask_heads ? 1 : query.size(1)) * query.size(2),
+                      "key mask smaller than [B, L]");
 }
 
 // fp32 heads of the handle's sizes on one GPU (the module's test); mask_or_pen as for sparse_attention.  [out, map, mean or
@@ -759,15 +780,15 @@ std::vector<Tensor> dense_attention(const Tensor& query, const Tensor& key, cons
                                     const c10::optional<Tensor>& mask_or_pen, bool is_mask, int64_t handle, bool emit_mean,
                                     int64_t stream) {
     const c10::DeviceGuard on(query.device());
-    const auto pen = penalty_of(mask_or_pen, is_mask, query.size(1), query.device(), stream);
-    const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
-    check_penalties(pen_or_none, query);
+    const KeyOperand keys = key_operand(mask_or_pen, is_mask, query.size(0), query.size(1), query.size(2), query.device(), stream);
+    const Tensor pen_or_none = keys.or_none();
+    check_penalties(pen_or_none, keys.mask_heads, query);
     if (without_node({&query, &key, &value, &pen_or_none})) {
-        DenseResult r = dense_forward(query, key, value, pen_or_none, handle, emit_mean, stream);
+        DenseResult r = dense_forward(query, key, value, pen_or_none, keys.mask_heads, handle, emit_mean, stream);
         return {r.out, r.attn.transpose(2, 3), r.mean};
     }
     Tensor mean;
-    const auto r = DenseAttnNode::apply(query, key, value, pen, handle, emit_mean, stream, &mean);
+    const auto r = DenseAttnNode::apply(query, key, value, keys.t, keys.mask_heads, handle, emit_mean, stream, &mean);
     return {r[0], r[1], mean};
 }
 
@@ -776,12 +797,15 @@ Tensor bf16_attention(const Tensor& query, const Tensor& key, const Tensor& valu
                       bool is_mask, const Tensor& offsets, const Tensor& columns, const Tensor& sum_mat, int64_t handle,
                       int64_t nnz, int64_t stream) {
     const c10::DeviceGuard on(query.device());
-    const auto pen = penalty_of(mask_or_pen, is_mask, query.size(1), query.device(), stream);
-    const Tensor pen_or_none = pen.has_value() ? *pen : Tensor();
-    check_penalties(pen_or_none, query);
-    if (without_node({&query, &key, &value, &pen_or_none}))
-        return bf16_forward(query, key, value, pen_or_none, offsets, columns, sum_mat, handle, nnz, stream).out;
-    return BF16AttnNode::apply(query, key, value, pen, offsets, columns, sum_mat, handle, nnz, stream);
+    // a backward needs the penalties too, whatever has become of the mask by then
+    const bool plain = without_node({&query, &key, &value});
+    const KeyOperand keys = plain ? key_operand(mask_or_pen, is_mask, query.size(0), query.size(1), query.size(2), query.device(), stream)
+                                  : KeyOperand{penalty_of(mask_or_pen, is_mask, query.size(1), query.device(), stream), 0};
+    const Tensor pen_or_none = keys.or_none();
+    check_penalties(pen_or_none, keys.mask_heads, query);
+    if (plain && without_node({&pen_or_none}))
+        return bf16_forward(query, key, value, pen_or_none, keys.mask_heads, offsets, columns, sum_mat, handle, nnz, stream).out;
+    return BF16AttnNode::apply(query, key, value, keys.t, offsets, columns, sum_mat, handle, nnz, stream);
 }
 
 }  // namespace

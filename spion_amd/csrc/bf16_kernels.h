@@ -202,7 +202,7 @@ enum { EL_TILE = 0, EL_A = 1, EL_B = 2 };
 template <int D, bool MASK, bool ST, bool PAIRS>
 SPION_BF16_LANE(2) void bf16_fwd_kernel(
     const __bf16* __restrict__ Q, const __bf16* __restrict__ K, const __bf16* __restrict__ V,
-    const float* __restrict__ pen, __bf16* __restrict__ O, float* __restrict__ Lse, const int* __restrict__ tcol,
+    KeyTerms keys, __bf16* __restrict__ O, float* __restrict__ Lse, const int* __restrict__ tcol,
     const int* __restrict__ plan_items, const int* __restrict__ lane_ptr, const int* __restrict__ lane_ent, int L,
     int NB, float scale, float* __restrict__ Part, int n_slots, Layouts ly, unsigned in_bytes, unsigned out_bytes) {
     typedef DmaTile<D> DT;
@@ -213,14 +213,14 @@ SPION_BF16_LANE(2) void bf16_fwd_kernel(
     const const_ints ents = as_constant(lane_ent), items = as_constant(plan_items), tiles = as_constant(tcol);
     const int ild = ST ? ly.in.ld : D, old_ = ST ? ly.out.ld : D;
     const u32x4 wQ = rsrc_words(Q, in_bytes), wK = rsrc_words(K, in_bytes), wV = rsrc_words(V, in_bytes);
-    const u32x4 wM = rsrc_words(MASK ? (const void*)pen : (const void*)K, MASK ? (size_t)NB * L * 4 : in_bytes);
+    const u32x4 wM = rsrc_words(MASK ? (const void*)keys.p : (const void*)K, MASK ? (size_t)(NB / keys.heads) * L * 4 : in_bytes);
     const rsrc_t rO = make_rsrc(O, out_bytes);
     const int t_bytes = 32 * ild * 2;
     const int vin = DT::voff(l, ild), xin = DT::extra_step(ild), vout = DT::voff(l, old_);
     const unsigned lds_w = lds_address(Tw);
     const typename DT::RowAddr ra = DT::row_addr(li, h);
     const typename DT::TrAddr ta = DT::tr_addr(l);
-    const float c2 = scale * LOG2E, pen_mul = -1.0f / scale;
+    const float c2 = scale * LOG2E, kmul = keys.mul * (1.0f / scale), kadd = keys.add * (1.0f / scale);
     constexpr int E = 1, OPS = 2 * DT::NI + 1;
 
     LaneEntry en = lane_entry(ents, e0);
@@ -236,6 +236,7 @@ SPION_BF16_LANE(2) void bf16_fwd_kernel(
             itn = plan_item(items, en.y);
         }
         const int bhn = en.x;
+        const int mh = MASK ? bh / keys.heads : 0, mhn = MASK ? bhn / keys.heads : 0;  // whose row of key terms
         const int I = it.x, t0 = it.y, n = it.z;
         const bool pair = PAIRS && it.w == -2;
         const int In = itn.x, t0n = itn.y;
@@ -245,7 +246,7 @@ SPION_BF16_LANE(2) void bf16_fwd_kernel(
         const unsigned hb = bf16_head_bytes<ST, D>(ly.in, ly.H, bh, L), hbn = bf16_head_bytes<ST, D>(ly.in, ly.H, bhn, L);
         // element k of an item (given by value: selecting between variables captured by reference would pin them to
         // memory)
-        auto locate_in = [&](int k, int bhX, int IX, int t0X, unsigned hbX, bool pairX) __attribute__((always_inline)) {
+        auto locate_in = [&](int k, int mhX, int IX, int t0X, unsigned hbX, bool pairX) __attribute__((always_inline)) {
             if (k == 0) {
                 sk = EL_A;
                 sa = uniform((int)(hbX + (unsigned)(IX * t_bytes)));
@@ -256,13 +257,13 @@ SPION_BF16_LANE(2) void bf16_fwd_kernel(
                 sk = EL_TILE;
                 sa = uniform((int)(hbX + (unsigned)(J * t_bytes)));
                 sb = sa;
-                sc = MASK ? uniform((bhX * L + J * 32) * 4) : sa;
+                sc = MASK ? uniform((mhX * L + J * 32) * 4) : sa;
             }
         };
-        auto locate = [&, bh, bhn, I, In, t0, t0n, hb, hbn, pair, pairn, len, g0](int gg) __attribute__((always_inline)) {
+        auto locate = [&, mh, mhn, I, In, t0, t0n, hb, hbn, pair, pairn, len, g0](int gg) __attribute__((always_inline)) {
             const int k = gg - g0;
-            if (k < len) locate_in(k, bh, I, t0, hb, pair);
-            else locate_in(k - len, bhn, In, t0n, hbn, pairn);
+            if (k < len) locate_in(k, mh, I, t0, hb, pair);
+            else locate_in(k - len, mhn, In, t0n, hbn, pairn);
             sq_g = gg;
         };
         auto issue = [&]() __attribute__((always_inline)) {  // element gi -> buffer gi % 2, then look the following one up
@@ -325,9 +326,9 @@ SPION_BF16_LANE(2) void bf16_fwd_kernel(
             f32x16 init = splat16(0.f);
             if constexpr (MASK) {
                 float pj[16];
-                lds_get_rows(reinterpret_cast<const float*>(Tk + 2 * DT::TILE), 0, h, pj);  // pj[r] = pen[acc_row(r, h)]
+                lds_get_rows(reinterpret_cast<const float*>(Tk + 2 * DT::TILE), 0, h, pj);  // pj[r]: of key acc_row(r, h)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) init[r] = pj[r] * pen_mul;
+                for (int r = 0; r < 16; ++r) init[r] = fmaf(pj[r], kmul, kadd);
             }
             if (quick) {
                 wait_lgkm0();
@@ -335,7 +336,7 @@ SPION_BF16_LANE(2) void bf16_fwd_kernel(
                 const int s2 = uniform((int)(hb + (unsigned)(J2 * t_bytes)));
                 DT::load(wK, a, vin, s2, xin);
                 DT::load(wV, a + DT::TILE, vin, s2, xin);
-                dma_b32(wM, a + 2 * DT::TILE, l * 4, MASK ? uniform((bh * L + J2 * 32) * 4) : s2);
+                dma_b32(wM, a + 2 * DT::TILE, l * 4, MASK ? uniform((mh * L + J2 * 32) * 4) : s2);
                 ++gi;
             } else if (!last) {
                 release();

@@ -63,7 +63,7 @@ bool error_pending() {
 // implemented in sparse_attn.hip / dense_attn.hip / pattern.hip
 void* sparse_init(int, int, int, int, bool);
 void sparse_destroy(void*);
-void sparse_forward(void*, const float*, const float*, const float*, const float*, float*, float*, const int*,
+void sparse_forward(void*, const float*, const float*, const float*, const KeyTerms&, float*, float*, const int*,
                     const int*, int, bool, bool);
 void sparse_backward(void*, const float*, const float*, const float*, const float*, const float*, float*, float*,
                      float*, float*, float*, const int*, const int*, int, const float*, bool);
@@ -72,12 +72,12 @@ struct HeadLayout {  // as in tile_kernels.h
     int hstride;
     int ld;
 };
-void sparse_forward_strided(void*, const float*, const float*, const float*, const float*, float*, float*, const int*,
+void sparse_forward_strided(void*, const float*, const float*, const float*, const KeyTerms&, float*, float*, const int*,
                             const int*, int, int, const HeadLayout&, const HeadLayout&);
 void sparse_backward_strided(void*, const float*, const float*, const float*, const float*, const float*, const float*,
                              float*, float*, float*, const int*, const int*, int, int, const HeadLayout&,
                              const HeadLayout&, const HeadLayout&);
-void dense_forward_strided(void*, const float*, const float*, const float*, const float*, float*, float*, int,
+void dense_forward_strided(void*, const float*, const float*, const float*, const KeyTerms&, float*, float*, int,
                            const HeadLayout&, const HeadLayout&);
 void dense_backward_strided(void*, const float*, const float*, const float*, const float*, const float*, const float*,
                             float*, float*, float*, int, const HeadLayout&, const HeadLayout&, const HeadLayout&);
@@ -95,11 +95,11 @@ int sparse_debug_counter(void*, int);
 int sparse_debug_bf16_plan(const int*, int, int, int, int, int*, int, int*, int, int*, int, int*, int, int*);
 void sparse_use_ocache(void*, int);
 void* sparse_bf16_init(int, int, int, int);
-void sparse_bf16_forward(void*, const void*, const void*, const void*, const float*, void*, float*, const int*,
+void sparse_bf16_forward(void*, const void*, const void*, const void*, const KeyTerms&, void*, float*, const int*,
                          const int*, int);
 void sparse_bf16_backward(void*, const void*, const void*, const void*, const float*, const void*, const float*,
                           const void*, void*, void*, void*, const int*, const int*, int);
-void sparse_bf16_forward_strided(void*, const void*, const void*, const void*, const float*, void*, float*, const int*,
+void sparse_bf16_forward_strided(void*, const void*, const void*, const void*, const KeyTerms&, void*, float*, const int*,
                                  const int*, int, int, const HeadLayout&, const HeadLayout&);
 void sparse_bf16_backward_strided(void*, const void*, const void*, const void*, const float*, const void*, const float*,
                                   const void*, void*, void*, void*, const int*, const int*, int, int, const HeadLayout&,
@@ -108,7 +108,7 @@ int transpose_last2(const float*, float*, int, int, int, hipStream_t);
 int transition_update(const float*, float*, int, long long, float*, double*, int, int, hipStream_t);
 void* dense_init(int, int, int, bool);
 void dense_destroy(void*);
-void dense_forward(void*, const float*, const float*, const float*, const float*, float*, float*, bool);
+void dense_forward(void*, const float*, const float*, const float*, const KeyTerms&, float*, float*, bool);
 void dense_backward(void*, const float*, const float*, const float*, const float*, const float*, float*, float*,
                     float*);
 int dense_groups(void*);
@@ -122,7 +122,7 @@ int project_backward(const float*, const float* const*, const float*, float*, fl
 int key_penalty(const float*, float*, int, int, int, hipStream_t);
 int pattern_generate_maps(const float* const*, int, int, int, int, int, double, float*, int, float*, float*, hipStream_t);
 int score_map_mean(const float*, int, int, int, int, float*, hipStream_t, float post = 1.0f);
-void dense_forward_strided_mean(void*, const float*, const float*, const float*, const float*, float*, float*, float*, int,
+void dense_forward_strided_mean(void*, const float*, const float*, const float*, const KeyTerms&, float*, float*, float*, int,
                                 const HeadLayout&, const HeadLayout&);
 
 // A handle that is held is freed by the release of its last hold.
@@ -478,6 +478,63 @@ void spion_dense_backward_strided(void* h, const float* Q, const float* K, const
         return;
     }
     dense_backward_strided(h, Q, K, V, P, Out, dO, dQ, dK, dV, heads, to_layout(in), to_layout(out), to_layout(grad));
+}
+// The forwards above on a key mask itself.
+static bool key_mask_given(const char* who, const float* mask, int heads) {
+    if (mask && heads > 0 && reinterpret_cast<uintptr_t>(mask) % 16 == 0) return true;
+    note_current_handle(nullptr);
+    set_error("%s: a key mask, 16-byte aligned, and the heads of a sample expected", who);
+    return false;
+}
+void spion_attn_forward_rowmajor_keys(void* h, const float* Q, const float* K, const float* V, const float* mask, int heads,
+                                      float* Attn, float* Out, const int* Offsets, const int* Columns, const int* SumMat,
+                                      int nnz) {
+    (void)SumMat;
+    if (!key_mask_given("attn_forward_rowmajor_keys", mask, heads)) return;
+    sparse_forward(h, Q, K, V, KeyTerms(mask, heads), Attn, Out, Offsets, Columns, nnz, true, true);
+}
+void spion_attn_forward_strided_keys(void* h, const float* Q, const float* K, const float* V, const float* mask, float* Attn,
+                                     float* Out, const int* Offsets, const int* Columns, const int* SumMat, int nnz,
+                                     int heads, const spion_head_layout* in, const spion_head_layout* out) {
+    (void)SumMat;
+    if (!key_mask_given("attn_forward_strided_keys", mask, heads)) return;
+    if (!in || !out) {
+        set_error("attn_forward_strided_keys: null layout argument");
+        return;
+    }
+    sparse_forward_strided(h, Q, K, V, KeyTerms(mask, heads), Attn, Out, Offsets, Columns, nnz, heads, to_layout(in),
+                           to_layout(out));
+}
+void spion_dense_forward_strided_keys(void* h, const float* Q, const float* K, const float* V, const float* mask, float* Attn,
+                                      float* Out, float* Mean, int heads, const spion_head_layout* in,
+                                      const spion_head_layout* out) {
+    if (!key_mask_given("dense attn_forward_strided_keys", mask, heads)) return;
+    if (!in || !out) {
+        set_error("dense attn_forward_strided_keys: null layout argument");
+        return;
+    }
+    if (Mean) dense_forward_strided_mean(h, Q, K, V, KeyTerms(mask, heads), Attn, Out, Mean, heads, to_layout(in), to_layout(out));
+    else dense_forward_strided(h, Q, K, V, KeyTerms(mask, heads), Attn, Out, heads, to_layout(in), to_layout(out));
+}
+void spion_block_bf16_attn_forward_keys(void* h, const void* Q, const void* K, const void* V, const float* mask, int heads,
+                                        void* Out, float* Lse, const int* Offsets, const int* Columns, const int* SumMat,
+                                        int nnz) {
+    (void)SumMat;
+    if (!key_mask_given("bf16 attn_forward_keys", mask, heads)) return;
+    sparse_bf16_forward(h, Q, K, V, KeyTerms(mask, heads), Out, Lse, Offsets, Columns, nnz);
+}
+void spion_block_bf16_attn_forward_strided_keys(void* h, const void* Q, const void* K, const void* V, const float* mask,
+                                                void* Out, float* Lse, const int* Offsets, const int* Columns,
+                                                const int* SumMat, int nnz, int heads, const spion_head_layout* in,
+                                                const spion_head_layout* out) {
+    (void)SumMat;
+    if (!key_mask_given("bf16 attn_forward_strided_keys", mask, heads)) return;
+    if (!in || !out) {
+        set_error("bf16 attn_forward_strided_keys: null layout argument");
+        return;
+    }
+    sparse_bf16_forward_strided(h, Q, K, V, KeyTerms(mask, heads), Out, Lse, Offsets, Columns, nnz, heads, to_layout(in),
+                                to_layout(out));
 }
 int spion_transpose_last2(const float* in, float* out, int batch, int rows, int cols, void* stream) {
     note_current_handle(nullptr);

@@ -44,6 +44,19 @@ struct HandleHeader {
     ~HandleHeader();
 };
 
+// What keys add to the logits: p[(head / heads) * L + key] * mul + add.  Penalties [NB][L], as the ABI hands them over, are
+// subtracted; a [B][L] key mask of `heads` heads a sample (1 valid, 0 padded) adds 1e6 (mask - 1)
+// (models/attention_blockcuda_mask.py:42-43).
+struct KeyTerms {
+    const float* p;
+    int heads;
+    float mul, add;
+    KeyTerms(const float* penalties) : p(penalties), heads(1), mul(-1.f), add(0.f) {}
+    KeyTerms(const float* mask, int heads_) : p(mask), heads(heads_), mul(1e6f), add(-1e6f) {}
+    explicit operator bool() const { return p != nullptr; }
+    __host__ __device__ const float* row(int bh, int L) const { return p + (size_t)(bh / heads) * L; }
+};
+
 // The handle the calling thread is working on (set by the handle checks of every entry point, cleared by
 // entry points without a handle): set_error files the message there as well.
 void note_current_handle(HandleHeader* h);

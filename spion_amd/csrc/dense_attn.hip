@@ -21,7 +21,7 @@ constexpr int DENSE_WAVES = 4;
 template <int D, bool MASK>
 __global__ __launch_bounds__(64 * DENSE_WAVES) void dense_fwd_kernel(
     const float* __restrict__ Qt, const float* __restrict__ K, const float* __restrict__ Vt,
-    const float* __restrict__ pen, float* __restrict__ Attn, float* __restrict__ Out, float* __restrict__ OutCopy,
+    KeyTerms keys, float* __restrict__ Attn, float* __restrict__ Out, float* __restrict__ OutCopy,
     int L, int nbr, int NB, float scale) {
     constexpr int WAVES = DENSE_WAVES;
     __shared__ float lds[WAVES * (D / 32) * 16 * 64];
@@ -30,7 +30,7 @@ __global__ __launch_bounds__(64 * DENSE_WAVES) void dense_fwd_kernel(
     const int bh = item / nbr, I = item % nbr;
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, h = l >> 5, li = l & 31;
     const size_t hb = (size_t)bh * L * D;
-    const float* penh = MASK ? pen + (size_t)bh * L : nullptr;
+    const float* krow = MASK ? keys.row(bh, L) : nullptr;
     float* Ah = Attn + (size_t)bh * L * L + I * 32 + li;
 
     float q[D / 2];
@@ -45,7 +45,7 @@ __global__ __launch_bounds__(64 * DENSE_WAVES) void dense_fwd_kernel(
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             v[r] = s[r] * scale;
-            if (MASK) v[r] -= penh[J * 32 + acc_row(r, h)];
+            if (MASK) v[r] += fmaf(krow[J * 32 + acc_row(r, h)], keys.mul, keys.add);
             tm = fmaxf(tm, v[r]);
         }
         float zz = 0.f;
@@ -86,7 +86,7 @@ __global__ __launch_bounds__(64 * DENSE_WAVES) void dense_fwd_kernel(
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             float v = s[r] * scale;
-            if (MASK) v -= penh[J * 32 + acc_row(r, h)];
+            if (MASK) v += fmaf(krow[J * 32 + acc_row(r, h)], keys.mul, keys.add);
             p[r] = __expf(v - m) * rinv;
             // the map is written once and is far larger than the caches: non-temporal
             __builtin_nontemporal_store(p[r], &Ah[(size_t)(J * 32 + acc_row(r, h)) * L]);
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(64 * DENSE_WAVES) void dense_fwd_kernel(
 template <bool MASK, bool RM = false, int WAVES = 4, bool MEAN = false, int MAXT = 32 / WAVES>
 SPION_TILE_KERNEL(WAVES) void dense_fwd_reg_kernel(
     const float* __restrict__ Qt, const float* __restrict__ K, const float* __restrict__ Vt,
-    const float* __restrict__ pen, float* __restrict__ Attn, float* __restrict__ Out, float* __restrict__ OutCopy,
+    KeyTerms keys, float* __restrict__ Attn, float* __restrict__ Out, float* __restrict__ OutCopy,
     int L, int nbr, int NB, float scale, Layouts ly, float* __restrict__ Part = nullptr, int C = 0) {
     static_assert(!MEAN || RM, "the mean-emitting forward takes row-major operands");
     constexpr int D = 32, KH = 16;
@@ -148,7 +148,8 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg_kernel(
     const rsrc_t rQ = make_rsrc(Qt + ib, hbytes);
     const rsrc_t rA = make_rsrc(Attn + (size_t)bh * L * L, (size_t)L * L * 4);
     const u32x4 wK = rsrc_words(K + ib, hbytes), wV = rsrc_words(Vt + ib, hbytes);
-    const u32x4 wM = rsrc_words(MASK ? pen + (size_t)bh * L : pen, MASK ? (size_t)L * 4 : 0);
+    const u32x4 wM = rsrc_words(MASK ? keys.row(bh, L) : nullptr, MASK ? (size_t)L * 4 : 0);
+    const float kmul = keys.mul * LOG2E, kadd = keys.add * LOG2E;  // key terms, log2 domain
     const int alin = lin_voff(l, L);
     const int vld = RM ? ild : L, VSTEP = RM ? 32 * ild * 4 : 128;
     const int kx = DmaTileF32::extra_step(ild);
@@ -200,10 +201,10 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg_kernel(
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         const f32x4 x = *reinterpret_cast<const f32x4*>(Tm + (u & 1) * 256 + 32 * g);
-                        init[4 * g + 0] = -LOG2E * x.x;
-                        init[4 * g + 1] = -LOG2E * x.y;
-                        init[4 * g + 2] = -LOG2E * x.z;
-                        init[4 * g + 3] = -LOG2E * x.w;
+                        init[4 * g + 0] = fmaf(x.x, kmul, kadd);
+                        init[4 * g + 1] = fmaf(x.y, kmul, kadd);
+                        init[4 * g + 2] = fmaf(x.z, kmul, kadd);
+                        init[4 * g + 3] = fmaf(x.w, kmul, kadd);
                     }
                 }
                 wait_lgkm0();  // the tile's space is requested again one iteration on
@@ -327,7 +328,7 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg_kernel(
 template <bool MASK, int WAVES = 4>
 SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
     const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
-    const float* __restrict__ pen, float* __restrict__ Attn, float* __restrict__ Out,
+    KeyTerms keys, float* __restrict__ Attn, float* __restrict__ Out,
     int L, int nbr, int NB, float scale, Layouts ly) {
     constexpr int D = 64, KH = 32, MAXT = 8;
     __shared__ float lds[WAVES * 16 * 64];
@@ -346,7 +347,8 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
     head_slice<true, D>(ly.out, ly.H, bh, L, ob, old_, obytes);
     const rsrc_t rA = make_rsrc(Attn + (size_t)bh * L * L, (size_t)L * L * 4);
     const u32x4 wK = rsrc_words(K + ib, hbytes), wV = rsrc_words(V + ib, hbytes);
-    const u32x4 wM = rsrc_words(MASK ? pen + (size_t)bh * L : pen, MASK ? (size_t)L * 4 : 0);
+    const u32x4 wM = rsrc_words(MASK ? keys.row(bh, L) : nullptr, MASK ? (size_t)L * 4 : 0);
+    const float kmul = keys.mul * LOG2E, kadd = keys.add * LOG2E;  // key terms, log2 domain
     const int kx = DmaTileF32::extra_step(ild);
     const float c2 = scale * LOG2E;
     auto issue = [&](const u32x4& r, int J, int kl) {
@@ -391,10 +393,10 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         const f32x4 x = *reinterpret_cast<const f32x4*>(Tm + 32 * g);
-                        init[4 * g + 0] = -LOG2E * x.x;
-                        init[4 * g + 1] = -LOG2E * x.y;
-                        init[4 * g + 2] = -LOG2E * x.z;
-                        init[4 * g + 3] = -LOG2E * x.w;
+                        init[4 * g + 0] = fmaf(x.x, kmul, kadd);
+                        init[4 * g + 1] = fmaf(x.y, kmul, kadd);
+                        init[4 * g + 2] = fmaf(x.z, kmul, kadd);
+                        init[4 * g + 3] = fmaf(x.w, kmul, kadd);
                     }
                 }
                 wait_lgkm0();
@@ -514,7 +516,7 @@ SPION_TILE_KERNEL(WAVES) void dense_fwd_reg64_kernel(
 template <bool MASK, bool RM = false, bool MEAN = false>
 SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
     const float* __restrict__ Qt, const float* __restrict__ K, const float* __restrict__ Vt,
-    const float* __restrict__ pen, float* __restrict__ Attn, float* __restrict__ Out, float* __restrict__ OutCopy,
+    KeyTerms keys, float* __restrict__ Attn, float* __restrict__ Out, float* __restrict__ OutCopy,
     int L, int nbr, int NB, float scale, Layouts ly, float* __restrict__ Part = nullptr, int C = 0) {
     static_assert(!MEAN || RM, "the mean-emitting forward takes row-major operands");
     constexpr int D = 32, KH = 16, WAVES = 4;
@@ -536,7 +538,8 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
     const rsrc_t rQ = make_rsrc(Qt + ib, hbytes), rK = make_rsrc(K + ib, hbytes), rV = make_rsrc(Vt + ib, hbytes);
     const rsrc_t rA = make_rsrc(Attn + (size_t)bh * L * L, (size_t)L * L * 4);
     const rsrc_t rS = make_rsrc(MEAN ? Part + (size_t)bh0 * L * L : Part, MEAN ? (size_t)L * L * 4 : 0);
-    const rsrc_t rM = make_rsrc(MASK ? pen + (size_t)bh * L : pen, MASK ? (size_t)L * 4 : 0);
+    const rsrc_t rM = make_rsrc(MASK ? keys.row(bh, L) : nullptr, MASK ? (size_t)L * 4 : 0);
+    const float kmul = keys.mul * LOG2E, kadd = keys.add * LOG2E;  // key terms, log2 domain
     float* T = lds_t[w];          // map tile on its way to memory
     float* Tk = T + 32 * TS;
     float* Tv = T + 64 * TS;
@@ -592,7 +595,7 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
                 f32x16 init = splat16(0.f);
                 if constexpr (MASK) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) init[r] = -LOG2E * c.pj[r];
+                    for (int r = 0; r < 16; ++r) init[r] = fmaf(c.pj[r], kmul, kadd);
                 }
                 const f32x16 S = mma_feat_init<D>(kf, qk, init);  // register = key, lane = query
                 const float mn = max16(S, m);
@@ -661,7 +664,7 @@ SPION_TILE_KERNEL(4) void dense_fwd_sweep32_kernel(
                 f32x16 init = minus_m;
                 if constexpr (MASK) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) init[r] -= LOG2E * c.pj[r];
+                    for (int r = 0; r < 16; ++r) init[r] += fmaf(c.pj[r], kmul, kadd);
                 }
                 const f32x16 S = mma_feat_init<D>(kf, qk, init);  // logits minus the row maximum
                 float p[16];
@@ -1271,7 +1274,7 @@ void dense_destroy(void* h) {
 }
 
 template <int D>
-static void dense_fwd_launch(DenseAttn* a, const float* Qt, const float* K, const float* Vt, const float* Mask,
+static void dense_fwd_launch(DenseAttn* a, const float* Qt, const float* K, const float* Vt, const KeyTerms& Mask,
                              float* Attn, float* Out) {
     const int nbr = a->L / 32;
     dim3 grid(nbr * a->NB), block(64 * DENSE_WAVES);
@@ -1342,7 +1345,7 @@ static void dense_bwd_launch(DenseAttn* a, const float* Qt, const float* Kt, con
                        a->L, nbr, a->NB, a->scale);
 }
 
-void dense_forward(void* h, const float* Qt, const float* K, const float* Vt, const float* Mask, float* Attn,
+void dense_forward(void* h, const float* Qt, const float* K, const float* Vt, const KeyTerms& Mask, float* Attn,
                    float* Out, bool mask_entry) {
     DenseAttn* a = as_dense(h, "attn_forward");
     if (!a) return;
@@ -1405,13 +1408,13 @@ int score_map_mean(const float* Attn, int batch, int heads, int L, int key_major
 
 // Mean != nullptr: the launch also leaves the mean of all NB maps (queries x keys) in Mean, accumulated while the
 // maps are written (see dense_fwd_reg_kernel) and finished by one reduction over the partial maps.
-static void dense_forward_strided_impl(void* h, const float* Q, const float* K, const float* V, const float* Mask,
+static void dense_forward_strided_impl(void* h, const float* Q, const float* K, const float* V, const KeyTerms& Mask,
                                        float* Attn, float* Out, float* Mean, int heads, const HeadLayout& in,
                                        const HeadLayout& out, const char* who) {
     const HeadLayout* lays[2] = {&in, &out};
     DenseAttn* a = dense_strided_handle(h, who, heads, lays, 2);
     if (!a) return;
-    if (a->has_mask != (Mask != nullptr)) {
+    if (a->has_mask != (bool)Mask) {
         set_error("%s: handle was created by the %s init", who, a->has_mask ? "mask" : "no-mask");
         return;
     }
@@ -1528,11 +1531,11 @@ static void dense_forward_strided_impl(void* h, const float* Q, const float* K, 
     check_launch("dense_fwd kernels");
 }
 
-void dense_forward_strided(void* h, const float* Q, const float* K, const float* V, const float* Mask, float* Attn,
+void dense_forward_strided(void* h, const float* Q, const float* K, const float* V, const KeyTerms& Mask, float* Attn,
                            float* Out, int heads, const HeadLayout& in, const HeadLayout& out) {
     dense_forward_strided_impl(h, Q, K, V, Mask, Attn, Out, nullptr, heads, in, out, "dense attn_forward_strided");
 }
-void dense_forward_strided_mean(void* h, const float* Q, const float* K, const float* V, const float* Mask, float* Attn,
+void dense_forward_strided_mean(void* h, const float* Q, const float* K, const float* V, const KeyTerms& Mask, float* Attn,
                                 float* Out, float* Mean, int heads, const HeadLayout& in, const HeadLayout& out) {
     if (!Mean) {
         as_dense(h, "dense attn_forward_strided_mean");

@@ -208,7 +208,7 @@ typedef GatherRowAcc<8> HybRowAcc;
 // -------------------------------------------------------------------------------------------------
 template <bool MASK, bool ST>
 SPION_HYB_GATHER_KERNEL void hyb_rem_logits_kernel(const float* __restrict__ Q, const float* __restrict__ K,
-                                                   const float* __restrict__ pen, float* __restrict__ Raw,
+                                                   KeyTerms keys, float* __restrict__ Raw,
                                                    float2* __restrict__ Stats, HybIndex ix, int L, int NB,
                                                    float scale, Layouts ly) {
     const int lane = threadIdx.x & 63, ent = hyb_entry_of_lane(lane);
@@ -232,7 +232,7 @@ SPION_HYB_GATHER_KERNEL void hyb_rem_logits_kernel(const float* __restrict__ Q, 
         const int col = k < rc ? ix.r_col[r0 + k] : 0;
         float v = hyb_gather_dot(q4, K + ib, ild, col, min(64, rc - c0), lane);
         if (k < rc) {
-            if (MASK) v -= pen[(size_t)bh * L + col] * LOG2E;
+            if (MASK) v += fmaf(keys.row(bh, L)[col], keys.mul * LOG2E, keys.add * LOG2E);
             raw[k] = v;
             mx = fmaxf(mx, v);
         } else {
@@ -262,7 +262,7 @@ SPION_HYB_GATHER_KERNEL void hyb_rem_logits_kernel(const float* __restrict__ Q, 
 // added (Oc, optional: second copy of O, contiguous heads).
 template <bool MASK, int WAVES, int MAXT, bool ST, bool REM>
 SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, const float* __restrict__ K,
-                                          const float* __restrict__ V, const float* __restrict__ pen,
+                                          const float* __restrict__ V, KeyTerms keys,
                                           float* __restrict__ P, float* __restrict__ O, float* __restrict__ Oc,
                                           float2* __restrict__ Stats, const int* __restrict__ offs, HybIndex ix, int L,
                                           int nbr, int NB, int nnz, float scale, Layouts ly) {
@@ -279,7 +279,8 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
     head_slice<ST, D>(ly.in, ly.H, bh, L, ib, ild, ibytes);
     head_slice<ST, D>(ly.out, ly.H, bh, L, ob, old_, obytes);
     const rsrc_t rQ = make_rsrc(Q + ib, ibytes), rK = make_rsrc(K + ib, ibytes), rV = make_rsrc(V + ib, ibytes);
-    const rsrc_t rM = make_rsrc(MASK ? pen + (size_t)bh * L : pen, MASK ? (size_t)L * 4 : 0);
+    const rsrc_t rM = make_rsrc(MASK ? keys.row(bh, L) : nullptr, MASK ? (size_t)L * 4 : 0);
+    const float kmul = keys.mul * LOG2E, kadd = keys.add * LOG2E;
     float* Ph = P + (size_t)bh * nnz;
     float* T = lds_t[w];
     float* Tx = T + 32 * TS;
@@ -334,7 +335,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
             f32x16 init = splat16(0.f);
             if constexpr (MASK) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) init[r] = -LOG2E * pj[u & 1][r];
+                for (int r = 0; r < 16; ++r) init[r] = fmaf(pj[u & 1][r], kmul, kadd);
             }
             lds_put_lin(Tx, l, raw[u & 1]);
             float kf[KH];

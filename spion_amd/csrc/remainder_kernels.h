@@ -115,7 +115,7 @@ __device__ __forceinline__ rsrc_t rem_word_rsrc(const int* w, int nr) { return m
 // -------------------------------------------------------------------------------------------------
 template <bool MASK, bool ST, int NO>
 __global__ __launch_bounds__(REM_THREADS) void rem_fwd_kernel(const float* __restrict__ Q, const float* __restrict__ K,
-                                                              const float* __restrict__ V, const float* __restrict__ pen,
+                                                              const float* __restrict__ V, KeyTerms keys,
                                                               float* __restrict__ Raw, float2* __restrict__ Stats,
                                                               float* __restrict__ O, RemIndex ix, int L, int NB, float scale,
                                                               Layouts ly) {
@@ -234,7 +234,8 @@ __global__ __launch_bounds__(REM_THREADS) void rem_fwd_kernel(const float* __res
     for (int k = 0; k * REM_RANGE < L; ++k) {
         __syncthreads();  // everybody has finished with the previous range
         if constexpr (MASK)
-            if (threadIdx.x < REM_RANGE) spen[threadIdx.x] = pen[(size_t)bh * L + min(k * REM_RANGE + (int)threadIdx.x, L - 1)] * LOG2E;
+            if (threadIdx.x < REM_RANGE) spen[threadIdx.x] = fmaf(keys.row(bh, L)[min(k * REM_RANGE + (int)threadIdx.x, L - 1)], -keys.mul * LOG2E,
+                                         -keys.add * LOG2E);
         rem_load_range<true>(K + ib, ild, V + ib, ild, k * REM_RANGE, L, tile);
         __syncthreads();
 #pragma unroll

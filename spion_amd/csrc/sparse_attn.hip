@@ -122,7 +122,7 @@ struct RowAcc {
 template <int D, bool MASK, bool ST>
 __global__ __launch_bounds__(64 * ELEM_WAVES) __attribute__((amdgpu_waves_per_eu(D <= 32 ? 6 : D == 64 ? 3 : 2, 8))) void elem_fwd_kernel(
     const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
-    const float* __restrict__ pen, float* __restrict__ P, float* __restrict__ O,
+    KeyTerms keys, float* __restrict__ P, float* __restrict__ O,
     const int* __restrict__ offs, const int* __restrict__ cols, int L, int NB, int nnz, float scale, Layouts ly) {
     const int lane = threadIdx.x & 63;
     // consecutive rows (which gather overlapping K/V rows and share lines of P) on the same XCD
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(64 * ELEM_WAVES) __attribute__((amdgpu_waves_per_eu
             const int col = k < cnt ? cj[k] : 0;
             float v = gather_dot<LPR>(q4, K + ib, ild, col, min(64, cnt - c0), lane) * scale;
             if (k < cnt) {
-                if (MASK) v -= pen[(size_t)bh * L + col];
+                if (MASK) v += fmaf(keys.row(bh, L)[col], keys.mul, keys.add);
                 p[k] = v;
                 m = fmaxf(m, v);
             }
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(64 * ELEM_WAVES) __attribute__((amdgpu_waves_per_eu
         for (int k = lane; k < cnt; k += 64) {
             int col = cj[k];
             float v = row_dot<D>(q, K + ib + (size_t)col * ild) * scale;
-            if (MASK) v -= pen[(size_t)bh * L + col];
+            if (MASK) v += fmaf(keys.row(bh, L)[col], keys.mul, keys.add);
             p[k] = v;
             m = fmaxf(m, v);
         }
@@ -1319,7 +1319,7 @@ static int heads_per_group(const SparseAttn* a) {
 }
 
 template <int D, bool MASK, bool KROW, bool ST = false>
-static void launch_tile_fwd(SparseAttn* a, const float* Q, const float* Kt, const float* V, const float* pen, float* P,
+static void launch_tile_fwd(SparseAttn* a, const float* Q, const float* Kt, const float* V, const KeyTerms& pen, float* P,
                             float* O, const int* offs, int nnz, const Layouts& ly = Layouts{}) {
     PhaseRange phase("spion forward (tile kernels)");
     const PatternIndex& pi = a->pat;
@@ -1567,7 +1567,7 @@ static int rem_per_quad(const SparseAttn* a) {
 // Hybrid patterns (dense tiles + remainder, d = 32).  Every operand row-major; ST: heads located by `ly`.
 // ocopy (contiguous heads only): where a second copy of O goes, or null.
 template <bool ST>
-static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const float* V, const float* Mask,
+static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const float* V, const KeyTerms& Mask,
                            float* Attn, float* Out, float* ocopy, const int* Offsets, int nnz, const Layouts& ly) {
     PhaseRange phase("spion forward (hybrid kernels)");
     if (!ensure_ws(&a->ws_stats, (size_t)a->NB * a->L * 2)) return;
@@ -1676,7 +1676,7 @@ static void launch_transpose(SparseAttn* a, const float* Xt, float* X) {
 }
 
 template <int D, bool ST = false>
-static void launch_elem_fwd(SparseAttn* a, const float* Q, const float* Krm, const float* V, const float* pen,
+static void launch_elem_fwd(SparseAttn* a, const float* Q, const float* Krm, const float* V, const KeyTerms& pen,
                             float* P, float* O, const int* offs, const int* cols, int nnz,
                             const Layouts& ly = Layouts{}) {
     PhaseRange phase("spion forward (element kernels)");
@@ -1721,7 +1721,7 @@ static void launch_elem_bwd(SparseAttn* a, const float* Q, const float* K, const
 }
 
 // krow: Kt is K itself, row-major [NB][L][d], not the transposed copy of the reference's ABI.
-void sparse_forward(void* h, const float* Q, const float* Kt, const float* V, const float* Mask, float* Attn,
+void sparse_forward(void* h, const float* Q, const float* Kt, const float* V, const KeyTerms& Mask, float* Attn,
                     float* Out, const int* Offsets, const int* Columns, int nnz, bool mask_entry, bool krow) {
     SparseAttn* a = as_sparse(h, "attn_forward");
     if (!a) return;
@@ -1731,6 +1731,10 @@ void sparse_forward(void* h, const float* Q, const float* Kt, const float* V, co
     }
     if (!Q || !Kt || !V || !Attn || !Out || !Offsets || (nnz > 0 && !Columns) || (mask_entry && !Mask)) {
         set_error("attn_forward: null pointer argument");
+        return;
+    }
+    if (a->NB % Mask.heads) {
+        set_error("attn_forward: %d heads a sample do not divide the handle's %d", Mask.heads, a->NB);
         return;
     }
     if (!ensure_pattern(a, Offsets, Columns, nnz)) return;
@@ -1979,13 +1983,13 @@ static SparseAttn* strided_handle(void* h, const char* who, const int* Offsets, 
     return a;
 }
 
-void sparse_forward_strided(void* h, const float* Q, const float* K, const float* V, const float* Mask, float* Attn,
+void sparse_forward_strided(void* h, const float* Q, const float* K, const float* V, const KeyTerms& Mask, float* Attn,
                             float* Out, const int* Offsets, const int* Columns, int nnz, int heads,
                             const HeadLayout& in, const HeadLayout& out) {
     const char* who = "attn_forward_strided";
     SparseAttn* a = strided_handle(h, who, Offsets, Columns, nnz, heads);
     if (!a) return;
-    if (a->has_mask != (Mask != nullptr)) {
+    if (a->has_mask != (bool)Mask) {
         set_error("%s: handle was created by the %s init", who, a->has_mask ? "mask" : "no-mask");
         return;
     }
@@ -2140,7 +2144,7 @@ static unsigned bf16_extent(const SparseAttn* a, bool strided, const HeadLayout&
 }
 
 template <bool ST>
-static void bf16_forward_impl(SparseAttn* a, const void* Q, const void* K, const void* V, const float* Mask, void* Out,
+static void bf16_forward_impl(SparseAttn* a, const void* Q, const void* K, const void* V, const KeyTerms& Mask, void* Out,
                               float* Lse, const Layouts& ly) {
     PhaseRange phase("spion forward (bf16 kernels)");
     const PatternIndex& pi = a->pat;
@@ -2244,7 +2248,7 @@ static void bf16_backward_impl(SparseAttn* a, const void* Q, const void* K, cons
     check_launch("bf16_bwd kernels");
 }
 
-void sparse_bf16_forward(void* h, const void* Q, const void* K, const void* V, const float* Mask, void* Out, float* Lse,
+void sparse_bf16_forward(void* h, const void* Q, const void* K, const void* V, const KeyTerms& Mask, void* Out, float* Lse,
                          const int* Offsets, const int* Columns, int nnz) {
     if (!Q || !K || !V || !Out || !Lse || !Offsets || (nnz > 0 && !Columns)) {
         set_error("bf16 attn_forward: null pointer argument");
@@ -2252,6 +2256,10 @@ void sparse_bf16_forward(void* h, const void* Q, const void* K, const void* V, c
     }
     SparseAttn* a = as_bf16(h, "bf16 attn_forward", Offsets, Columns, nnz);
     if (!a) return;
+    if (a->NB % Mask.heads) {
+        set_error("bf16 attn_forward: %d heads a sample do not divide the handle's %d", Mask.heads, a->NB);
+        return;
+    }
     bf16_forward_impl<false>(a, Q, K, V, Mask, Out, Lse, Layouts{});
 }
 
@@ -2281,7 +2289,7 @@ static bool check_layout_bf16(const char* who, const char* what, const SparseAtt
     return true;
 }
 
-void sparse_bf16_forward_strided(void* h, const void* Q, const void* K, const void* V, const float* Mask, void* Out,
+void sparse_bf16_forward_strided(void* h, const void* Q, const void* K, const void* V, const KeyTerms& Mask, void* Out,
                                  float* Lse, const int* Offsets, const int* Columns, int nnz, int heads,
                                  const HeadLayout& in, const HeadLayout& out) {
     const char* who = "bf16 attn_forward_strided";

@@ -26,6 +26,7 @@
 //     that block by the compiler, next to its use.
 #pragma once
 #include "bf16_tile.h"
+#include "common.h"
 #include "tile_ops.h"
 
 namespace spion {
@@ -607,7 +608,7 @@ template <int D, int WAVES, bool MASK, int MAXT, bool KROW = false, bool ST = fa
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D == 32 && MAXT > 0 && MAXT <= 6 && !LONG ? 3 : 2, D == 32 && MAXT > 0 && MAXT <= 6 && !LONG ? 3 : 2)))
 void tile_fwd_kernel(
     const float* __restrict__ Q, const float* __restrict__ Kt, const float* __restrict__ V,
-    const float* __restrict__ pen, float* __restrict__ P, float* __restrict__ O, float* __restrict__ Ocache,
+    KeyTerms keys, float* __restrict__ P, float* __restrict__ O, float* __restrict__ Ocache,
     const int* __restrict__ rdesc, const int* __restrict__ tcol, int L, int nbr,
     int NB, int nnz, float scale, int s0, int ns, int hc, Layouts ly) {
     static_assert(!ST || KROW, "strided heads: row-major operands");
@@ -637,7 +638,9 @@ void tile_fwd_kernel(
     head_slice<ST, D>(ly.out, ly.H, bh, L, ob, old_, obytes);
     const rsrc_t rQ = make_rsrc(Q + ib, hbytes), rK = make_rsrc(Kt + ib, hbytes), rV = make_rsrc(V + ib, hbytes);
     const rsrc_t rP = make_rsrc(P + (size_t)bh * nnz, (size_t)nnz * 4);
-    const rsrc_t rM = make_rsrc(MASK ? pen + (size_t)bh * L : pen, MASK ? (size_t)L * 4 : 0);
+    const float* krow = MASK ? keys.row(bh, L) : nullptr;  // key terms, log2 domain: fmaf(krow[j], kmul, kadd)
+    const float kmul = keys.mul * LOG2E, kadd = keys.add * LOG2E;
+    const rsrc_t rM = make_rsrc(krow, MASK ? (size_t)L * 4 : 0);
     const int p_base = sd.w * 4;
     float* T = lds_t[w];
     // P tile t of this block row: transpose to the col-owner layout and store full rows
@@ -685,7 +688,7 @@ void tile_fwd_kernel(
             f32x16 v;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                if constexpr (MASK) v[r] = -LOG2E * x.pj[r] - shift;
+                if constexpr (MASK) v[r] = fmaf(x.pj[r], kmul, kadd) - shift;
                 else v[r] = -shift;
             }
             return v;
@@ -782,7 +785,7 @@ void tile_fwd_kernel(
         z = 0.f;
         if constexpr (LIN) {
             const u32x4 wK = rsrc_words(Kt + ib, hbytes);
-            const u32x4 wM = rsrc_words(MASK ? pen + (size_t)bh * L : pen, MASK ? (size_t)L * 4 : 0);
+            const u32x4 wM = rsrc_words(krow, MASK ? (size_t)L * 4 : 0);
             const int kl = DmaTileF32::voff(l, kld), kx = DmaTileF32::extra_step(kld);
             const auto a_k0 = [&] {
                 if constexpr (KROW) return DmaTileF32::own_addr(Tb, li, 4 * h, 1);
@@ -812,10 +815,10 @@ void tile_fwd_kernel(
 #pragma unroll
                         for (int g = 0; g < 4; ++g) {
                             const f32x4 v = *reinterpret_cast<const f32x4*>(Tm + (u & 1) * 256 + 32 * g);
-                            init[4 * g + 0] = -LOG2E * v.x;
-                            init[4 * g + 1] = -LOG2E * v.y;
-                            init[4 * g + 2] = -LOG2E * v.z;
-                            init[4 * g + 3] = -LOG2E * v.w;
+                            init[4 * g + 0] = fmaf(v.x, kmul, kadd);
+                            init[4 * g + 1] = fmaf(v.y, kmul, kadd);
+                            init[4 * g + 2] = fmaf(v.z, kmul, kadd);
+                            init[4 * g + 3] = fmaf(v.w, kmul, kadd);
                         }
                     }
                     wait_lgkm0();  // the tile's space is requested again one iteration on
@@ -829,7 +832,7 @@ void tile_fwd_kernel(
             // read out into registers, then the place is requested for tile u + 1, which has the chain to arrive.
             static_assert(D == 64, "head dimension 32 or 64");
             const u32x4 wK = rsrc_words(Kt + ib, hbytes);
-            const u32x4 wM = rsrc_words(MASK ? pen + (size_t)bh * L : pen, MASK ? (size_t)L * 4 : 0);
+            const u32x4 wM = rsrc_words(krow, MASK ? (size_t)L * 4 : 0);
             const int kl = DmaTileF32::voff(l, kld), kx = DmaTileF32::extra_step(kld);
             const int KHALF = KROW ? 128 : 32 * L * 4;
             const unsigned lb64 = lds_address(Tb);
@@ -855,10 +858,10 @@ void tile_fwd_kernel(
 #pragma unroll
                         for (int g = 0; g < 4; ++g) {
                             const f32x4 v = *reinterpret_cast<const f32x4*>(Tm + 32 * g);
-                            init[4 * g + 0] = -LOG2E * v.x;
-                            init[4 * g + 1] = -LOG2E * v.y;
-                            init[4 * g + 2] = -LOG2E * v.z;
-                            init[4 * g + 3] = -LOG2E * v.w;
+                            init[4 * g + 0] = fmaf(v.x, kmul, kadd);
+                            init[4 * g + 1] = fmaf(v.y, kmul, kadd);
+                            init[4 * g + 2] = fmaf(v.z, kmul, kadd);
+                            init[4 * g + 3] = fmaf(v.w, kmul, kadd);
                         }
                     }
                     wait_lgkm0();
