@@ -32,12 +32,6 @@ __device__ __forceinline__ void dma_b128(u32x4 r, unsigned lds, int voff, int so
                  "s"(soff)
                  : "memory");
 }
-// LDS accesses of all wavefronts before are complete after; loads from global memory may be in flight across it.
-__device__ __forceinline__ void group_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
 
 // The two operand tiles (32 rows x D floats each) of a step.  Wavefront w of the G = D/8 loads 1 KB of each (rows RPW*w ..)
 // into a place of its own, takes it back out, a lane 16 bytes, and writes the three parts into planes in the layout of
