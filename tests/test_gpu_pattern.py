@@ -361,3 +361,27 @@ def test_device_transition_detector_matches_host_detector():
         if a and decided is None:
             decided = step
     assert decided is not None and decided >= 2
+
+
+# batches and heads around the eight maps requested together; the smallest and a ragged number of 32 x 32 tiles
+@pytest.mark.parametrize("key_major", [0, 1])
+@pytest.mark.parametrize("batch,heads,L", [(1, 1, 32), (7, 1, 96), (8, 1, 64), (9, 1, 32), (3, 5, 96), (1, 17, 64), (16, 2, 160)])
+def test_mean_map_of_aligned_and_other_maps(batch, heads, L, key_major):
+    """Both kernels add in the same order: the same bits, and the mean of float64 to the roundings of its sums."""
+    g = torch.Generator().manual_seed(batch + L)
+    n = batch * heads * L * L
+    flat = torch.empty(n + 1, device="cuda")
+    flat[1:] = (torch.rand(n, generator=g) + 0.125).cuda()
+    maps = flat[1:].clone()
+    from spion_amd import _lib
+
+    core, stream, got = _lib.core(), torch.cuda.current_stream().cuda_stream, []
+    for a in (flat[1:], maps):
+        out = torch.full((L * L + 4,), 7.0, device="cuda")
+        assert core.spion_score_map_mean(a.data_ptr(), batch, heads, L, key_major, out.data_ptr(), stream) == 0
+        assert bool((out[L * L:] == 7.0).all())
+        got.append(out[: L * L].view(L, L))
+    assert torch.equal(got[0], got[1])
+    ref = maps.view(batch, heads, L, L).double().mean((0, 1))
+    ref = ref.t() if key_major else ref
+    assert float(((got[1].double() - ref).abs() / ref).max()) <= (batch + heads + 4) * 2.0 ** -24
