@@ -32,11 +32,13 @@ __device__ __forceinline__ float wave_sum(float v) {
 __device__ __forceinline__ int acc_row(int r, int h) { return 8 * (r >> 2) + 4 * h + (r & 3); }
 
 // Work-group id -> work item, so that consecutive work items (same head) run on the same XCD and
-// share its L2: the hardware deals work-groups round-robin over the 8 XCDs.
+// share its L2: the hardware deals work-groups round-robin over the 8 XCDs.  (Numbers of items that eight does not divide were
+// once left as they are, so that every XCD's L2 saw all heads at a time.  us, before / now: steps of 45 heads of 3296 231 / 209, of 202
+// of 1056 161 / 142, with key mask of 75 of 1632 (d = 64) 259 / 243; discovery of two maps of 2720^2 49.4 / 41.6.)
 __device__ __forceinline__ int xcd_remap(int pid, int total) {
     constexpr int XCDS = 8;
-    if (total % XCDS) return pid;
-    return (pid % XCDS) * (total / XCDS) + pid / XCDS;
+    const int xcd = pid % XCDS, share = total / XCDS, rest = total % XCDS;  // the first `rest` XCDs have one more
+    return xcd * share + min(xcd, rest) + pid / XCDS;
 }
 
 // =================================================================================================
