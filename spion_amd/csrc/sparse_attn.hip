@@ -597,8 +597,8 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
     Bf16PlanHost out;
     long long ntiles = 0;
     for (int i = 0; i < nstrips; ++i) ntiles += ptr[i + 1] - ptr[i];
-    const int groups = NB % 8 == 0 ? 8 : 1;  // dies
-    const int lanes = std::max(groups, lanes_wanted / groups * groups);
+    const int even = NB % 8 == 0 ? 8 : 1;
+    const int lanes = std::max(even, lanes_wanted / even * even);
     // No item much longer than a lane's share of the launch, nor shorter than an average strip or a few tiles: in a small
     // launch a lane's share is a strip or less, and cutting every strip in two for it costs more in partial results and
     // their merging than it balances.  Forward + backward kernels without / with the average as a limit: 8 heads of 8192
@@ -645,32 +645,55 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
     // 214 / 219.  Longest first, the lanes drift apart in heads and lose the K and V in L2; it is taken where that costs nothing,
     // in launches of up to two items a lane whose heads are not dealt to dies: 10 of 6144, blocks of 64, 6 %, 103.5 / - / 91.9;
     // 36 of 3072, d = 32, blocks of 64, 8 %, 95.8 / - / 87.6.  Half as long chunks: 2 % less to 20 % more.
-    const int per_group = lanes / groups, heads_per_group = NB / groups;
-    const bool mixed = groups == 1 && (long long)its.size() * NB <= 2LL * lanes;
+    //
+    // Heads that eight does not divide: each die has NB / 8 heads to itself and an eighth of the work of the others, in the order of
+    // the strips, so that it sees two of them at most.  (All of them dealt among all lanes, every die's L2 saw every head.  Steps in us,
+    // so / now: 83 of 5600, blocks of 32, 5 %, 480 / 329; 12 of 16384 266 / 226; 30 of 9952, d = 32, 220 / 184; 61 of 14080, d = 32, 697 / 615.)
+    const bool mixed = even == 1 && (long long)its.size() * NB <= 2LL * lanes;
+    const int groups = even == 1 && !mixed && lanes % 8 == 0 && lanes >= 64 ? 8 : even;  // dies
+    const int per_group = lanes / groups, heads_per_group = NB / groups, whole_heads = heads_per_group * groups;
     std::vector<std::vector<std::pair<int, int>>> lane_list(lanes);  // {head, item}
+    std::vector<unsigned char> die_of((size_t)(NB - whole_heads) * its.size());  // of the items of the heads left over
+    {
+        long long one = 0, done = 0;
+        for (const It& x : its) one += weight(x);
+        const long long all = std::max<long long>(one * (NB - whole_heads), 1);
+        for (size_t i = 0; i < die_of.size(); ++i) {
+            const int w = weight(its[i % its.size()]);
+            die_of[i] = (unsigned char)std::min<long long>(groups - 1, (2 * done + w) * groups / (2 * all));
+            done += w;
+        }
+    }
     for (int g = 0; g < groups; ++g) {
         typedef std::pair<long long, int> Load;  // (work so far, lane of this die)
         std::priority_queue<Load, std::vector<Load>, std::greater<Load>> heap;
         for (int j = 0; j < per_group; ++j) heap.push({0, j});
-        auto deal = [&](int hh, int o) {
+        std::vector<int> heads;  // this die's: its own, then those it has a part of
+        for (int hh = 0; hh < heads_per_group; ++hh) heads.push_back(g * heads_per_group + hh);
+        for (int i = 0; i < NB - whole_heads; ++i) {
+            const auto first = die_of.begin() + i * its.size(), last = first + its.size();
+            if (std::find(first, last, (unsigned char)g) != last) heads.push_back(whole_heads + i);
+        }
+        auto deal = [&](int head, int o) {
+            if (head >= whole_heads && die_of[(size_t)(head - whole_heads) * its.size() + o] != g) return;
             Load top = heap.top();
             heap.pop();
             const int lane = top.second * groups + g;
-            lane_list[lane].push_back({g * heads_per_group + hh, o});
+            lane_list[lane].push_back({head, o});
             top.first += weight(its[o]);
             heap.push(top);
         };
         if (mixed) {
             for (int o : order)
-                for (int hh = 0; hh < heads_per_group; ++hh) deal(hh, o);
+                for (int head : heads) deal(head, o);
             continue;
         }
         for (int o : order)
             if (its[o].kind >= 0)
-                for (int hh = 0; hh < heads_per_group; ++hh) deal(hh, o);
-        for (int hh = 0; hh < heads_per_group; ++hh)
+                for (int head : heads) deal(head, o);
+        for (int head : heads)
             for (int o : order)
-                if (its[o].kind < 0) deal(hh, o);
+                if (its[o].kind < 0) deal(head, o);
     }
     out.lane_ptr.assign(1, 0);
     for (int sidx = 0; sidx < lanes; ++sidx) {

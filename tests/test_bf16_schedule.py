@@ -51,7 +51,7 @@ def _tile_ptr(rng, nstrips, kind, pairs):
 
 @pytest.mark.parametrize("kind", ["band", "global", "empty", "random"])
 @pytest.mark.parametrize("pairs", [False, True])
-@pytest.mark.parametrize("NB,lanes", [(32, 2048), (5, 2048), (8, 24), (3, 3), (16, 1)])
+@pytest.mark.parametrize("NB,lanes", [(32, 2048), (5, 2048), (8, 24), (3, 3), (16, 1), (13, 64), (3, 64), (1, 64)])
 def test_schedule_walks_every_tile_once(kind, pairs, NB, lanes):
     rng = np.random.default_rng(zlib.crc32(repr((kind, pairs, NB, lanes)).encode()))
     nstrips = int(rng.choice([2, 8, 64, 512]))
@@ -91,6 +91,13 @@ def test_schedule_walks_every_tile_once(kind, pairs, NB, lanes):
         heads = ents[lane_ptr[lane]: lane_ptr[lane + 1], 0]
         assert np.all(heads // per_die == lane % groups) if groups == 8 else True
         assert np.all(np.diff(heads) >= 0)
+    # heads that eight does not divide, more than two items a lane: a die has NB / 8 to itself and parts of two others at most
+    if groups == 1 and lanes == 64 and len(items) * NB > 2 * lanes:
+        for die in range(8):
+            on_die = np.unique(np.concatenate([ents[lane_ptr[l]: lane_ptr[l + 1], 0] for l in range(die, lanes, 8)]))
+            own = np.arange(die * (NB // 8), (die + 1) * (NB // 8))
+            shared = on_die[on_die >= NB // 8 * 8]
+            assert set(on_die) == set(own) | set(shared) and len(shared) <= 2
     # balance: no lane carries more than its die's average plus one longest item
     w = np.where(items[:, 3] == -2, 2, 1) * items[:, 2] + 2
     load = np.array([w[ents[lane_ptr[l]: lane_ptr[l + 1], 1]].sum() for l in range(plan["lanes"])])
