@@ -642,15 +642,14 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
     // up to 1.3 of the average work.  A lane still takes its items head after head.)  Steps in us, one machine, head after
     // head / chunks first / all items longest first: 32 heads of 16384, blocks of 64, 3.7 % kept, 562 / 538 / 564; 32 of 4096, 8 %,
     // forward alone, 40.3 / 37.5 / 39.3; 83 of 5600, blocks of 32, 5 %, 493 / 482 / 507; 30 of 9952, d = 32, blocks of 32, 5 %, 225 /
-    // 214 / 219.  Longest first, the lanes drift apart in heads and lose the K and V in L2; it is taken where that costs nothing,
-    // in launches of up to two items a lane whose heads are not dealt to dies: 10 of 6144, blocks of 64, 6 %, 103.5 / - / 91.9;
-    // 36 of 3072, d = 32, blocks of 64, 8 %, 95.8 / - / 87.6.  Half as long chunks: 2 % less to 20 % more.
+    // 214 / 219.  Longest first, the lanes drift apart in heads and lose the K and V in L2.  Half as long chunks: 2 % less to 20 % more.
     //
     // Heads that eight does not divide: each die has NB / 8 heads to itself and an eighth of the work of the others, in the order of
     // the strips, so that it sees two of them at most.  (All of them dealt among all lanes, every die's L2 saw every head.  Steps in us,
-    // so / now: 83 of 5600, blocks of 32, 5 %, 480 / 329; 12 of 16384 266 / 226; 30 of 9952, d = 32, 220 / 184; 61 of 14080, d = 32, 697 / 615.)
-    const bool mixed = even == 1 && (long long)its.size() * NB <= 2LL * lanes;
-    const int groups = even == 1 && !mixed && lanes % 8 == 0 && lanes >= 64 ? 8 : even;  // dies
+    // so / now: 83 of 5600, blocks of 32, 5 %, 480 / 329; 12 of 16384 266 / 226; 30 of 9952, d = 32, 220 / 184; 61 of 14080, d = 32, 697 / 615; 10 of
+    // 6144, up to two items a lane, 88 / 83, which dealt among all lanes longest first; so did forwards of 9 of 8192, 44.0 / 31.7, and of
+    // 20 of 4096, 28.6 / 25.0.)
+    const int groups = lanes % 8 == 0 && lanes >= 64 ? 8 : even;  // dies
     const int per_group = lanes / groups, heads_per_group = NB / groups, whole_heads = heads_per_group * groups;
     std::vector<std::vector<std::pair<int, int>>> lane_list(lanes);  // {head, item}
     std::vector<unsigned char> die_of((size_t)(NB - whole_heads) * its.size());  // of the items of the heads left over
@@ -683,11 +682,6 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
             top.first += weight(its[o]);
             heap.push(top);
         };
-        if (mixed) {
-            for (int o : order)
-                for (int head : heads) deal(head, o);
-            continue;
-        }
         for (int o : order)
             if (its[o].kind >= 0)
                 for (int head : heads) deal(head, o);

@@ -91,8 +91,8 @@ def test_schedule_walks_every_tile_once(kind, pairs, NB, lanes):
         heads = ents[lane_ptr[lane]: lane_ptr[lane + 1], 0]
         assert np.all(heads // per_die == lane % groups) if groups == 8 else True
         assert np.all(np.diff(heads) >= 0)
-    # heads that eight does not divide, more than two items a lane: a die has NB / 8 to itself and parts of two others at most
-    if groups == 1 and lanes == 64 and len(items) * NB > 2 * lanes:
+    # heads that eight does not divide: a die has NB / 8 to itself and parts of two others at most
+    if groups == 1 and lanes >= 64:
         for die in range(8):
             on_die = np.unique(np.concatenate([ents[lane_ptr[l]: lane_ptr[l + 1], 0] for l in range(die, lanes, 8)]))
             own = np.arange(die * (NB // 8), (die + 1) * (NB // 8))
