@@ -237,8 +237,8 @@ int spion_register_pattern(void* handle, const int* Offsets, const int* Columns,
                            const int* host_Offsets, const int* host_Columns);
 
 /* Which kernel family the last forward/backward of a sparse handle used:
- * 0 = none yet, 1 = MFMA 32x32 tile path, 2 = element path (gathers; with enough rows at emb_dim 32, the hybrid path's
- * kernels), 3 = hybrid path (element-sparse pattern at least half of whose entries lie in well-filled 32x32 tiles, which
+ * 0 = none yet, 1 = MFMA 32x32 tile path, 2 = element path (gathers; at emb_dim 32 and in the caller's scratch,
+ * spion_attn_forward_scratch, the hybrid path's kernels where those are faster), 3 = hybrid path (element-sparse pattern at least half of whose entries lie in well-filled 32x32 tiles, which
  * run on the MFMA units, the rest on kernels of their own).  For 2 and 3 the backward
  * needs the dS scratch.  It describes the most recent call on the handle, not a particular pattern. */
 int spion_last_path(void* handle);
@@ -325,7 +325,7 @@ long long spion_noalloc_max_rows(void);
  * the results equal those of the row-major entry points bit for bit.  Attn / P stay [NB][nnz] as everywhere.
  * The kept copies of Out are not used: the backward takes Out (required).  On patterns without tile structure
  * the backward's dS scratch ([NB][nnz] floats) belongs to the handle and is allocated by the first such call
- * (not under HIP graph capture).  Workspaces that follow the pattern's size grow when a larger pattern arrives; the
+ * (not under HIP graph capture); spion_attn_backward_scratch takes it from the caller.  Workspaces that follow the pattern's size grow when a larger pattern arrives; the
  * buffer a larger one replaces stays allocated until the handle is destroyed, so a HIP graph recorded earlier on
  * the handle can still be replayed. */
 typedef struct spion_head_layout {
@@ -343,6 +343,26 @@ void spion_attn_backward_strided(void* handle, const float* Q, const float* K, c
                                  const int* Offsets, const int* Columns, const int* SumMat, int nnz,
                                  int heads, const spion_head_layout* in, const spion_head_layout* out,
                                  const spion_head_layout* grad);
+
+/* The row-major (in, out, grad null: contiguous heads) and the strided calls above in scratch of the caller's: what the launches
+ * of a call on an element or hybrid pattern leave for each other then lies there and nothing of it in the handle, so that calls
+ * which share nothing else -- forwards on two streams -- may overlap.  (The passes over patterns of aligned tiles hand
+ * their row sums through the handle: backwards of one handle run one after the other.)  Patterns with less than half of their
+ * entries in well-filled tiles take the hybrid path's kernels, where those are the faster ones, in such scratch only; a call
+ * without one takes the element kernels for them, which work in the caller's buffers alone.
+ *   spion_attn_scratch   floats a call needs (0: none; -1: an error), after an analysis of the pattern if it is new;
+ *   scratch              16-byte aligned, contents unspecified, the caller's again when the call's work on the handle's
+ *                        stream has ended; one that is too small counts as none;
+ *   Mask, mask_heads     penalties [num_batches][seq_len] (0 heads), or a key mask as for the _keys entry points; null for
+ *                        handles without a mask. */
+long long spion_attn_scratch(void* handle, const int* Offsets, const int* Columns, int nnz, int backward);
+void spion_attn_forward_scratch(void* handle, const float* Q, const float* K, const float* V, const float* Mask, int mask_heads,
+                                float* Attn, float* Out, const int* Offsets, const int* Columns, int nnz, int heads,
+                                const spion_head_layout* in, const spion_head_layout* out, float* scratch, long long floats);
+void spion_attn_backward_scratch(void* handle, const float* Q, const float* K, const float* V, const float* P, const float* Out,
+                                 const float* dO, float* dQ, float* dK, float* dV, const int* Offsets, const int* Columns,
+                                 int nnz, int heads, const spion_head_layout* in, const spion_head_layout* out,
+                                 const spion_head_layout* grad, float* scratch, long long floats);
 
 /* The bf16 family on the same kind of views (no counterpart in the reference; models/attention.py:136-139 is where
  * its fp32 layer makes them): Q, K, V / Out, dO / dQ, dK, dV as [B][H][L][d] views located by one layout per group,

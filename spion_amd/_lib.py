@@ -124,6 +124,12 @@ def core() -> ctypes.CDLL:
     lib.spion_attn_forward_strided.restype = None
     lib.spion_attn_backward_strided.argtypes = [_P] * 13 + [c_int, c_int, _P, _P, _P]
     lib.spion_attn_backward_strided.restype = None
+    lib.spion_attn_scratch.argtypes = [_P, _P, _P, c_int, c_int]
+    lib.spion_attn_scratch.restype = ctypes.c_longlong
+    lib.spion_attn_forward_scratch.argtypes = ([_P] * 5 + [c_int] + [_P] * 4 + [c_int, c_int] + [_P] * 3 + [ctypes.c_longlong])
+    lib.spion_attn_forward_scratch.restype = None
+    lib.spion_attn_backward_scratch.argtypes = [_P] * 12 + [c_int, c_int] + [_P] * 4 + [ctypes.c_longlong]
+    lib.spion_attn_backward_scratch.restype = None
     lib.spion_dense_forward_strided.argtypes = [_P] * 7 + [c_int, _P, _P]
     lib.spion_dense_forward_strided.restype = None
     lib.spion_dense_forward_strided_mean.argtypes = [_P] * 8 + [c_int, _P, _P]

@@ -22,7 +22,7 @@ class _BlockAttnFunction(torch.autograd.Function):
     """The reference's function (models/attention_blockcuda.py:20-112) makes a transposed copy of K for the forward
     and of V for the backward because its ABI takes them that way, and its backward is not handed the forward's
     output.  Here every tensor stays row-major and autograd's saved ``out`` goes to the backward: the library's
-    row-major entry points (spion_attn_forward_rowmajor / spion_attn_backward_rowmajor) take them as they are.
+    row-major calls (spion_attn_forward_scratch / spion_attn_backward_scratch) take them as they are.
     ``attn_cpp`` (the drop-in with the reference's four symbols) is still what created the handle.
 
     The reference also starts with ``.contiguous()`` copies of query, key and value (models/attention_blockcuda.py:
@@ -57,18 +57,15 @@ class _BlockAttnFunction(torch.autograd.Function):
         if lay is not None:
             q, k, v = query, key, value
             out = _empty_heads(shape, interleaved=query.stride(1) < query.stride(2), device=dev)
-            lout = _lib.head_layout(out)
-            _lib.core().spion_attn_forward_strided(
-                m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), pen_ptr, p_flat.data_ptr(), out.data_ptr(),
-                *idx.tail, m.num_heads, ctypes.addressof(lay), ctypes.addressof(lout))
         else:
             q, k, v = query.contiguous(), key.contiguous(), value.contiguous()
             out = torch.empty(shape, dtype=torch.float32, device=dev)
-            _lib.core().spion_attn_forward_rowmajor(m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), pen_ptr,
-                                                    p_flat.data_ptr(), out.data_ptr(), *idx.tail)
+        lout = _lib.head_layout(out) if lay is not None else None
+        scratch = _scratch(m, idx, False, dev)
+        _lib.core().spion_attn_forward_scratch(
+            m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), pen_ptr, 0, p_flat.data_ptr(), out.data_ptr(),
+            *idx.tail[:2], idx.nnz, m.num_heads, _address(lay), _address(lout), *scratch[1:])
         _lib.check_error("attn_forward")
-        # which kernel family serves THIS pattern (the handle may run other patterns before the backward)
-        ctx.tiled = _lib.core().spion_last_path(m.attn_handle) == 1
         _lib.save_for_backward(ctx, q, k, v, p_flat, out)
         ctx.set_materialize_grads(False)  # the gradient of the returned probabilities is ignored anyway
         ctx.module = m
@@ -84,10 +81,9 @@ class _BlockAttnFunction(torch.autograd.Function):
         q, k, v, p_flat, out = _lib.saved_tensors(ctx)
         p_flat, dev = p_flat.contiguous(), q.device
         _lib.use_current_stream(m, dev)
-        n_total = m.num_batches * ctx.index.nnz
         if grad_output is None:  # only the probabilities were used downstream: their gradient is ignored
             grad_output = torch.zeros(m.batch_size, m.num_heads, m.seq_len, m.emb_dim, dtype=torch.float32, device=dev)
-        core = _lib.core()
+        lin = lout = lgrad = None
         if ctx.strided:
             (q, k, v), (out,) = _lib.one_layout(q, k, v), _lib.one_layout(out)
             go = grad_output
@@ -100,28 +96,32 @@ class _BlockAttnFunction(torch.autograd.Function):
             else:
                 dq, dk, dv = (_empty_heads(shape, interleaved, dev) for _ in range(3))
             lin, lout, lgrad = _lib.taken_layout(q), _lib.taken_layout(out), _lib.head_layout(dq)
-            core.spion_attn_backward_strided(
-                m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), p_flat.data_ptr(), out.data_ptr(),
-                go.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), *ctx.index.tail, m.num_heads,
-                ctypes.addressof(lin), ctypes.addressof(lout), ctypes.addressof(lgrad))
-            _lib.check_error("attn_backward")
-            return dq, dk, dv, None, None, None
-        q, k, v, out, go = (t.contiguous() for t in (q, k, v, out, grad_output))
-        # Of the ABI's two [NB*nnz] scratch arguments (models/attention_blockcuda.py:83-84) the tile kernels use
-        # neither and the element kernels only dS: nothing that size is allocated unless it is needed.
-        scratch_ds = None
-        if not ctx.tiled:
-            scratch_ds = torch.empty(max(n_total, 1), dtype=torch.float32, device=dev)
-        shape = m.head_shape
-        dq = torch.empty(shape, dtype=torch.float32, device=dev)
-        dk = torch.empty(shape, dtype=torch.float32, device=dev)
-        dv = torch.empty(shape, dtype=torch.float32, device=dev)
-        core.spion_attn_backward_rowmajor(
+        else:
+            q, k, v, out, go = (t.contiguous() for t in (q, k, v, out, grad_output))
+            dq, dk, dv = (torch.empty(m.head_shape, dtype=torch.float32, device=dev) for _ in range(3))
+        # in place of the ABI's two [NB*nnz] scratch arguments (models/attention_blockcuda.py:83-84)
+        scratch = _scratch(m, ctx.index, True, dev)
+        _lib.core().spion_attn_backward_scratch(
             m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), p_flat.data_ptr(), out.data_ptr(), go.data_ptr(),
-            scratch_ds.data_ptr() if scratch_ds is not None else None, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-            *ctx.index.tail)
+            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), *ctx.index.tail[:2], ctx.index.nnz, m.num_heads,
+            _address(lin), _address(lout), _address(lgrad), *scratch[1:])
         _lib.check_error("attn_backward")
         return dq, dk, dv, None, None, None
+
+
+def _address(layout):
+    return None if layout is None else ctypes.addressof(layout)
+
+
+def _scratch(m, index, backward, device):
+    """Scratch of a call of the core: (tensor, pointer, floats)."""
+    floats = _lib.core().spion_attn_scratch(m.attn_handle, *index.tail[:2], index.nnz, int(backward))
+    if floats < 0:
+        _lib.check_error("attn_backward" if backward else "attn_forward")
+    if floats <= 0:
+        return None, None, 0
+    t = torch.empty(floats, dtype=torch.float32, device=device)
+    return t, t.data_ptr(), floats
 
 
 def _empty_heads(shape, interleaved, device):

@@ -156,8 +156,17 @@ struct SavedTensors {
 // What a forward of the attention core leaves for its backward.
 struct CoreResult {
     Tensor q, k, v, out, p_flat;
-    bool strided = false, tiled = false;
+    bool strided = false;
 };
+
+// Scratch of a call of the core, of its stream as every tensor made here is.
+Tensor core_scratch(void* h, const Tensor& offsets, const Tensor& columns, int64_t nnz, bool backward, const torch::TensorOptions& opt) {
+    const int64_t floats = spion_attn_scratch(h, ip(offsets), ip(columns), (int)nnz, backward);
+    if (floats < 0) check_library(backward ? "attn_backward" : "attn_forward");
+    return floats > 0 ? torch::empty({floats}, opt) : Tensor();
+}
+float* fps(Tensor& t) { return t.defined() ? fpm(t) : nullptr; }
+int64_t count(const Tensor& t) { return t.defined() ? t.numel() : 0; }
 
 // pen: penalties [B, H*L] (mask_heads 0), a key mask [B, L] of mask_heads heads a sample, or nothing.
 CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& pen, int64_t mask_heads,
@@ -183,33 +192,24 @@ CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& va
     const auto opt = query.options();
     CoreResult r;
     r.p_flat = torch::empty({B * H * nnz}, opt);
+    Tensor scratch = core_scratch(h, offsets, columns, nnz, false, opt);
     spion_head_layout lin{}, lout{}, lk{}, lv{};
     r.strided = reads_views && !(query.is_contiguous() && key.is_contiguous() && value.is_contiguous()) &&
                 head_layout(query, lin) && head_layout(key, lk) && head_layout(value, lv) && same_strides(key, query) &&
                 same_strides(value, query);
+    r.q = r.strided ? query : query.contiguous();
+    r.k = r.strided ? key : key.contiguous();
+    r.v = r.strided ? value : value.contiguous();
     if (r.strided) {
-        r.q = query;
-        r.k = key;
-        r.v = value;
         r.out = empty_heads(query.sizes(), query.stride(1) < query.stride(2), opt);
         head_layout(r.out, lout);
-        (mask_heads ? spion_attn_forward_strided_keys : spion_attn_forward_strided)(
-            h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.p_flat), fpm(r.out), ip(offsets), ip(columns), ip(sum_mat), (int)nnz,
-            (int)num_heads, &lin, &lout);
     } else {
-        r.q = query.contiguous();
-        r.k = key.contiguous();
-        r.v = value.contiguous();
         r.out = torch::empty(query.sizes(), opt);
-        if (mask_heads)
-            spion_attn_forward_rowmajor_keys(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), (int)mask_heads, fpm(r.p_flat), fpm(r.out),
-                                             ip(offsets), ip(columns), ip(sum_mat), (int)nnz);
-        else
-            spion_attn_forward_rowmajor(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), fpm(r.p_flat), fpm(r.out), ip(offsets),
-                                        ip(columns), ip(sum_mat), (int)nnz);
     }
+    spion_attn_forward_scratch(h, fp(r.q), fp(r.k), fp(r.v), fp(pen), (int)mask_heads, fpm(r.p_flat), fpm(r.out), ip(offsets),
+                               ip(columns), (int)nnz, (int)num_heads, r.strided ? &lin : nullptr, r.strided ? &lout : nullptr,
+                               fps(scratch), count(scratch));
     check_library("attn_forward");
-    r.tiled = spion_last_path(h) == 1;
     return r;
 }
 
@@ -223,8 +223,6 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
         const Tensor pen = pen_opt.has_value() ? *pen_opt : Tensor();
         CoreResult r = core_forward(query, key, value, pen, mask_heads, offsets, columns, sum_mat, handle, nnz, num_heads,
                                     reads_views, stream);
-        // which kernel family serves THIS pattern (the handle may run other patterns before the backward)
-        ctx->saved_data["tiled"] = r.tiled;
         keep_handle(ctx, handle);
         ctx->saved_data["nnz"] = nnz;
         ctx->saved_data["heads"] = num_heads;
@@ -253,8 +251,10 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
         Tensor go = grads[0];
         if (!go.defined()) go = torch::zeros(q.sizes(), opt);  // only the probabilities were used downstream
         Tensor dq, dk, dv;
-        if (ctx->saved_data["strided"].toBool()) {
-            spion_head_layout lin{}, lout{}, lgrad{}, lgo{};
+        const bool strided = ctx->saved_data["strided"].toBool();
+        spion_head_layout lin{}, lout{}, lgrad{};
+        if (strided) {
+            spion_head_layout lgo{};
             if (!same_strides(go, out) || !head_layout(go, lgo)) go = torch::empty_like(out).copy_(go);  // out's strides
             if (adjacent_head_views(q, k, v)) {  // slices of one fused projection: the gradients likewise
                 Tensor buf = torch::empty({q.size(0), q.size(2), 3, q.size(1), q.size(3)}, opt);
@@ -270,26 +270,21 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
             taken_layout(q, lin);
             taken_layout(out, lout);
             head_layout(dq, lgrad);
-            spion_attn_backward_strided(h, fp(q), fp(k), fp(v), fp(p_flat), fp(out), fp(go), fpm(dq), fpm(dk), fpm(dv),
-                                        ip(offsets), ip(columns), ip(sum_mat), (int)nnz, heads, &lin, &lout, &lgrad);
         } else {
             q = q.contiguous();
             k = k.contiguous();
             v = v.contiguous();
             out = out.contiguous();
             go = go.contiguous();
-            // of the ABI's two [NB*nnz] scratch arguments (models/attention_blockcuda.py:83-84) the tile kernels use
-            // neither and the element kernels only dS
-            Tensor scratch;
-            if (!ctx->saved_data["tiled"].toBool())
-                scratch = torch::empty({std::max<int64_t>(q.size(0) * q.size(1) * nnz, 1)}, opt);
             dq = torch::empty(q.sizes(), opt);
             dk = torch::empty(q.sizes(), opt);
             dv = torch::empty(q.sizes(), opt);
-            spion_attn_backward_rowmajor(h, fp(q), fp(k), fp(v), fp(p_flat), fp(out), fp(go),
-                                         scratch.defined() ? fpm(scratch) : nullptr, fpm(dq), fpm(dk), fpm(dv),
-                                         ip(offsets), ip(columns), ip(sum_mat), (int)nnz);
         }
+        // (in place of the ABI's two [NB*nnz] scratch arguments, models/attention_blockcuda.py:83-84)
+        Tensor scratch = core_scratch(h, offsets, columns, nnz, true, opt);
+        spion_attn_backward_scratch(h, fp(q), fp(k), fp(v), fp(p_flat), fp(out), fp(go), fpm(dq), fpm(dk), fpm(dv), ip(offsets),
+                                    ip(columns), (int)nnz, heads, strided ? &lin : nullptr, strided ? &lout : nullptr,
+                                    strided ? &lgrad : nullptr, fps(scratch), count(scratch));
         check_library("attn_backward");
         variable_list r(14);
         r[0] = dq;

@@ -64,19 +64,21 @@ bool error_pending() {
 void* sparse_init(int, int, int, int, bool);
 void sparse_destroy(void*);
 void sparse_forward(void*, const float*, const float*, const float*, const KeyTerms&, float*, float*, const int*,
-                    const int*, int, bool, bool);
+                    const int*, int, bool, bool, const CallScratch& = CallScratch{});
 void sparse_backward(void*, const float*, const float*, const float*, const float*, const float*, float*, float*,
-                     float*, float*, float*, const int*, const int*, int, const float*, bool);
+                     float*, float*, float*, const int*, const int*, int, const float*, bool,
+                     const CallScratch& = CallScratch{});
+long long sparse_scratch_floats(void*, const int*, const int*, int, bool);
 struct HeadLayout {  // as in tile_kernels.h
     long long bstride;
     int hstride;
     int ld;
 };
 void sparse_forward_strided(void*, const float*, const float*, const float*, const KeyTerms&, float*, float*, const int*,
-                            const int*, int, int, const HeadLayout&, const HeadLayout&);
+                            const int*, int, int, const HeadLayout&, const HeadLayout&, const CallScratch& = CallScratch{});
 void sparse_backward_strided(void*, const float*, const float*, const float*, const float*, const float*, const float*,
                              float*, float*, float*, const int*, const int*, int, int, const HeadLayout&,
-                             const HeadLayout&, const HeadLayout&);
+                             const HeadLayout&, const HeadLayout&, const CallScratch& = CallScratch{});
 void dense_forward_strided(void*, const float*, const float*, const float*, const KeyTerms&, float*, float*, int,
                            const HeadLayout&, const HeadLayout&);
 void dense_backward_strided(void*, const float*, const float*, const float*, const float*, const float*, const float*,
@@ -438,6 +440,37 @@ void spion_attn_forward_strided(void* h, const float* Q, const float* K, const f
         return;
     }
     sparse_forward_strided(h, Q, K, V, Mask, Attn, Out, Offsets, Columns, nnz, heads, to_layout(in), to_layout(out));
+}
+// Calls that bring their scratch along.
+long long spion_attn_scratch(void* h, const int* Offsets, const int* Columns, int nnz, int backward) {
+    return sparse_scratch_floats(h, Offsets, Columns, nnz, backward != 0);
+}
+static CallScratch call_scratch(float* p, long long floats) {
+    const bool given = p && floats > 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+    return given ? CallScratch{p, (size_t)floats} : CallScratch{};
+}
+static bool key_mask_given(const char* who, const float* mask, int heads);
+void spion_attn_forward_scratch(void* h, const float* Q, const float* K, const float* V, const float* Mask, int mask_heads,
+                                float* Attn, float* Out, const int* Offsets, const int* Columns, int nnz, int heads,
+                                const spion_head_layout* in, const spion_head_layout* out, float* scratch, long long floats) {
+    if (mask_heads && !key_mask_given("attn_forward_scratch", Mask, mask_heads)) return;
+    const KeyTerms keys = mask_heads ? KeyTerms(Mask, mask_heads) : KeyTerms(Mask);
+    const CallScratch s = call_scratch(scratch, floats);
+    if (!in && !out) sparse_forward(h, Q, K, V, keys, Attn, Out, Offsets, Columns, nnz, Mask != nullptr, true, s);
+    else if (in && out) sparse_forward_strided(h, Q, K, V, keys, Attn, Out, Offsets, Columns, nnz, heads, to_layout(in), to_layout(out), s);
+    else set_error("attn_forward_scratch: one of the layouts is null");
+}
+void spion_attn_backward_scratch(void* h, const float* Q, const float* K, const float* V, const float* P, const float* Out,
+                                 const float* dO, float* dQ, float* dK, float* dV, const int* Offsets, const int* Columns,
+                                 int nnz, int heads, const spion_head_layout* in, const spion_head_layout* out,
+                                 const spion_head_layout* grad, float* scratch, long long floats) {
+    const CallScratch s = call_scratch(scratch, floats);
+    if (!in && !out && !grad)
+        sparse_backward(h, Q, K, V, P, dO, nullptr, nullptr, dQ, dK, dV, Offsets, Columns, nnz, Out, true, s);
+    else if (in && out && grad)
+        sparse_backward_strided(h, Q, K, V, P, Out, dO, dQ, dK, dV, Offsets, Columns, nnz, heads, to_layout(in), to_layout(out),
+                                to_layout(grad), s);
+    else set_error("attn_backward_scratch: some of the layouts are null");
 }
 void spion_attn_backward_strided(void* h, const float* Q, const float* K, const float* V, const float* P,
                                  const float* Out, const float* dO, float* dQ, float* dK, float* dV,

@@ -57,6 +57,12 @@ struct KeyTerms {
     __host__ __device__ const float* row(int bh, int L) const { return p + (size_t)(bh / heads) * L; }
 };
 
+// Memory that a caller hands over for one call: what the call's launches leave for each other lies there and not in the handle.
+struct CallScratch {
+    float* p = nullptr;
+    size_t floats = 0;
+};
+
 // The handle the calling thread is working on (set by the handle checks of every entry point, cleared by
 // entry points without a handle): set_error files the message there as well.
 void note_current_handle(HandleHeader* h);

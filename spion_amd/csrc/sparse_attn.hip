@@ -473,8 +473,6 @@ struct SparseAttn {
     float* ws_stats = nullptr;   // [NB][L][2] softmax row statistics handed between the hybrid forward's launches
     float* ws_raw = nullptr;     // [NB][nr] raw logits of a hybrid pattern's remainder, forward only
     size_t ws_raw_count = 0;
-    float* ws_pairs = nullptr;   // [NB][nr] {dS, P} of the remainder where the dS scratch is too small for them
-    size_t ws_pairs_count = 0;
     float* ws_ds = nullptr;      // [NB][nnz] dS scratch of the strided backward on patterns without tile structure
     size_t ws_ds_count = 0;
     float* ws_part = nullptr;    // [NB][slots][slot floats] partial results of the chunks of long strips (bf16 family)
@@ -561,7 +559,6 @@ void sparse_destroy(void* h) {
     if (a->ws_stats) (void)hipFree(a->ws_stats);
     if (a->ws_ds) (void)hipFree(a->ws_ds);
     if (a->ws_raw) (void)hipFree(a->ws_raw);
-    if (a->ws_pairs) (void)hipFree(a->ws_pairs);
     if (a->ws_part) (void)hipFree(a->ws_part);
     for (void* p : a->retired) (void)hipFree(p);
     for (auto& sl : a->oslot)
@@ -1194,7 +1191,7 @@ static bool ensure_ws(float** p, size_t count) {
 static bool ensure_ws_grow(SparseAttn* a, float** p, size_t* have, size_t need, const char* who) {
     if (*have >= need) return true;
     if (capturing(a)) {
-        if (who) set_error("%s: the workspace for this pattern is not allocated yet; run one step outside the capture", who);
+        set_error("%s: the workspace for this pattern is not allocated yet; run one step outside the capture", who);
         return false;
     }
     const size_t want = std::max(need, *have + *have / 2);
@@ -1203,7 +1200,7 @@ static bool ensure_ws_grow(SparseAttn* a, float** p, size_t* have, size_t need, 
         (void)hipGetLastError();
         if (want == need || hipMalloc((void**)&fresh, sizeof(float) * need) != hipSuccess) {
             (void)hipGetLastError();
-            if (who) set_error("%s: hipMalloc of %zu bytes of workspace failed", who, sizeof(float) * need);
+            set_error("%s: hipMalloc of %zu bytes of workspace failed", who, sizeof(float) * need);
             return false;
         }
         *have = need;
@@ -1217,40 +1214,63 @@ static bool ensure_ws_grow(SparseAttn* a, float** p, size_t* have, size_t need, 
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-// Whether a call on a hybrid pattern takes the hybrid kernels.  The remainder's kernels by ranges load 16 bytes a lane; and
-// where the element kernels would do as well (few entries in dense tiles), nothing is refused for want of a workspace.
-static bool take_hybrid(SparseAttn* a, std::initializer_list<const void*> operands) {
+// Whether a call on a hybrid pattern takes the hybrid kernels, and what their launches leave for each other (null: in the
+// handle).  The remainder's kernels by ranges load 16 bytes a lane.  Where the element kernels would do as well (few entries in
+// dense tiles) the hybrid ones are taken in the caller's scratch only: the element kernels work in the caller's buffers alone,
+// and calls on a handle that were independent of each other -- forwards on two streams, from two threads -- stay so.
+struct HybForwardWork {
+    float2* stats = nullptr;  // [NB][L] softmax row statistics
+    float* raw = nullptr;     // [NB][nr] raw logits of the remainder
+};
+struct HybBackwardWork {
+    float* rowsum = nullptr;  // [NB][L] row sums
+    float2* pairs = nullptr;  // [NB][nr] {dS, P} of the remainder
+};
+static size_t rem_list(const SparseAttn* a) { return (size_t)a->NB * (size_t)std::max(a->pat.hyb_nr, 1); }
+static size_t hyb_forward_floats(const SparseAttn* a) { return 2 * (size_t)a->NB * a->L + rem_list(a); }
+static size_t hyb_backward_floats(const SparseAttn* a) { return (size_t)a->NB * a->L + 2 * rem_list(a); }
+static bool take_hybrid(const SparseAttn* a, std::initializer_list<const void*> operands) {
     if (!a->pat.hybrid) return false;
     if (!a->pat.rem_lds) return true;
     for (const void* p : operands)
         if (!aligned16(p)) return false;
     return true;
 }
-static size_t rem_list(const SparseAttn* a) { return (size_t)a->NB * (size_t)std::max(a->pat.hyb_nr, 1); }
-static bool take_hybrid_forward(SparseAttn* a, std::initializer_list<const void*> operands) {
+static bool take_hybrid_forward(const SparseAttn* a, std::initializer_list<const void*> operands, const CallScratch& scratch,
+                                HybForwardWork* work) {
     if (!take_hybrid(a, operands)) return false;
-    if (a->pat.hyb_dense) return true;
-    if (!a->ws_stats && (capturing(a) || hipMalloc((void**)&a->ws_stats, sizeof(float) * 2 * a->NB * a->L) != hipSuccess)) {
-        (void)hipGetLastError();
-        a->ws_stats = nullptr;
-        return false;
-    }
-    return ensure_ws_grow(a, &a->ws_raw, &a->ws_raw_count, rem_list(a), nullptr);
-}
-// *pairs: where the row pass leaves {dS, P} for the column pass -- the dS scratch [NB][nnz] if they fit.
-static bool take_hybrid_backward(SparseAttn* a, std::initializer_list<const void*> operands, float* dS, int nnz, float** pairs) {
-    if (!take_hybrid(a, operands)) return false;
-    *pairs = dS;
-    if (a->pat.hyb_dense) return true;
-    if (!a->ws_rowsum && (capturing(a) || hipMalloc((void**)&a->ws_rowsum, sizeof(float) * a->NB * a->L) != hipSuccess)) {
-        (void)hipGetLastError();
-        a->ws_rowsum = nullptr;
-        return false;
-    }
-    if (2LL * a->pat.hyb_nr <= nnz) return true;
-    if (!ensure_ws_grow(a, &a->ws_pairs, &a->ws_pairs_count, 2 * rem_list(a), nullptr)) return false;
-    *pairs = a->ws_pairs;
+    if (scratch.floats < hyb_forward_floats(a)) return a->pat.hyb_dense;
+    work->stats = reinterpret_cast<float2*>(scratch.p);
+    work->raw = scratch.p + 2 * (size_t)a->NB * a->L;
     return true;
+}
+// dS: [NB][nnz] floats, which hold the pairs of a pattern at least half of which lies in dense tiles; or null.
+static bool take_hybrid_backward(const SparseAttn* a, std::initializer_list<const void*> operands, float* dS,
+                                 const CallScratch& scratch, HybBackwardWork* work) {
+    if (!take_hybrid(a, operands)) return false;
+    if (scratch.floats < hyb_backward_floats(a)) {
+        work->pairs = reinterpret_cast<float2*>(dS);
+        return a->pat.hyb_dense && dS;
+    }
+    work->rowsum = scratch.p;
+    work->pairs = reinterpret_cast<float2*>(scratch.p + (size_t)a->NB * a->L);
+    return true;
+}
+
+// Floats of scratch with which a call on this pattern leaves nothing in the handle (the fp32 element and hybrid patterns; the
+// passes over tile patterns hand their row sums through it); -1 on an error.
+long long sparse_scratch_floats(void* h, const int* Offsets, const int* Columns, int nnz, bool backward) {
+    SparseAttn* a = as_sparse(h, "spion_attn_scratch");
+    if (!a) return -1;
+    if (a->is_bf16 || !Offsets || (nnz > 0 && !Columns)) {
+        set_error("spion_attn_scratch: an index and a handle of the fp32 family expected");
+        return -1;
+    }
+    if (!ensure_pattern(a, Offsets, Columns, nnz)) return -1;
+    if (a->pat.tiled) return 0;
+    if (!backward) return a->pat.hybrid ? (long long)hyb_forward_floats(a) : 0;
+    const size_t ds = (size_t)a->NB * (size_t)std::max(nnz, 1);
+    return (long long)(a->pat.hybrid ? std::max(ds, hyb_backward_floats(a)) : ds);
 }
 
 int transpose_last2(const float* in, float* out, int batch, int rows, int cols, hipStream_t stream);
@@ -1585,12 +1605,16 @@ static int rem_per_quad(const SparseAttn* a) {
 // ocopy (contiguous heads only): where a second copy of O goes, or null.
 template <bool ST>
 static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const float* V, const KeyTerms& Mask,
-                           float* Attn, float* Out, float* ocopy, const int* Offsets, int nnz, const Layouts& ly) {
+                           float* Attn, float* Out, float* ocopy, const int* Offsets, int nnz, const Layouts& ly,
+                           HybForwardWork work) {
     PhaseRange phase("spion forward (hybrid kernels)");
-    if (!ensure_ws(&a->ws_stats, (size_t)a->NB * a->L * 2)) return;
     // the remainder's raw logits between the first and the third launch: a compact list of their own (written and
     // read in full lines) rather than their places inside P, where every four-byte store would pull in a line
-    if (!ensure_ws_grow(a, &a->ws_raw, &a->ws_raw_count, rem_list(a), "attn_forward")) return;
+    if (!work.raw) {
+        if (!ensure_ws(&a->ws_stats, (size_t)a->NB * a->L * 2)) return;
+        if (!ensure_ws_grow(a, &a->ws_raw, &a->ws_raw_count, rem_list(a), "attn_forward")) return;
+        work = HybForwardWork{reinterpret_cast<float2*>(a->ws_stats), a->ws_raw};
+    }
     a->last_path = a->pat.hyb_dense ? 3 : 2;
     const int nbr = a->L / 32;
     const long long rows = (long long)a->NB * a->L;
@@ -1598,14 +1622,15 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
     const bool one = a->pat.max_row_tiles <= HYB_MAXT1;
     const dim3 grid_t(nbr * a->NB), block_t(one ? 64 : 256);
     const dim3 grid_g((unsigned)((rows + HYB_GWAVES - 1) / HYB_GWAVES)), block_g(64 * HYB_GWAVES);
-    float2* stats = reinterpret_cast<float2*>(a->ws_stats);
+    float2* stats = work.stats;
+    float* raw = work.raw;
     const bool lds = a->pat.rem_lds, two = lds && rem_per_quad(a) == 2;
 #define SPION_HYB_TILES(MASKED, WAVES_, MAXT_, REM_)                                                                  \
     hipLaunchKernelGGL((hyb_tile_fwd_kernel<MASKED, WAVES_, MAXT_, ST, REM_>), grid_t, block_t, 0, a->hdr.stream, Q,  \
                        K, V, Mask, Attn, Out, REM_ ? ocopy : nullptr, stats, Offsets, a->pat.hyb, a->L, nbr, a->NB,   \
                        nnz, a->scale, ly)
 #define SPION_REM_FWD(MASKED, NO_)                                                                                     \
-    SPION_REM_LAUNCH((rem_fwd_kernel<MASKED, ST, NO_>), NO_, Q, K, V, Mask, a->ws_raw, stats, Out, a->pat.rem, a->L, \
+    SPION_REM_LAUNCH((rem_fwd_kernel<MASKED, ST, NO_>), NO_, Q, K, V, Mask, raw, stats, Out, a->pat.rem, a->L, \
                      a->NB, a->scale, ly)
 #define SPION_HYB_FWD(MASKED)                                                                                        \
     do {                                                                                                             \
@@ -1613,7 +1638,7 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
         else if (lds) SPION_REM_FWD(MASKED, 1);                                                                      \
         else                                                                                                         \
             hipLaunchKernelGGL((hyb_rem_logits_kernel<MASKED, ST>), grid_g, block_g, 0, a->hdr.stream, Q, K, Mask,   \
-                               a->ws_raw, stats, a->pat.hyb, a->L, a->NB, a->scale, ly);                             \
+                               raw, stats, a->pat.hyb, a->L, a->NB, a->scale, ly);                                   \
         if (one && lds) SPION_HYB_TILES(MASKED, 1, HYB_MAXT1, true);                                                 \
         else if (one) SPION_HYB_TILES(MASKED, 1, HYB_MAXT1, false);                                                  \
         else if (lds) SPION_HYB_TILES(MASKED, 4, HYB_MAXT4, true);                                                   \
@@ -1627,53 +1652,54 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
 #undef SPION_REM_FWD
 #undef SPION_HYB_TILES
     if (lds)
-        hipLaunchKernelGGL(rem_prob_kernel, grid_t, dim3(REM_PROB_THREADS), 0, a->hdr.stream, (const float*)a->ws_raw, Attn,
+        hipLaunchKernelGGL(rem_prob_kernel, grid_t, dim3(REM_PROB_THREADS), 0, a->hdr.stream, (const float*)raw, Attn,
                            (const float2*)stats, Offsets, a->pat.rem, a->L, nbr, a->NB, nnz);
     else
-        hipLaunchKernelGGL(hyb_rem_pv_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, V, (const float*)a->ws_raw, Attn,
+        hipLaunchKernelGGL(hyb_rem_pv_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, V, (const float*)raw, Attn,
                            Out, ocopy, (const float2*)stats, a->pat.hyb, a->L, a->NB, nnz, ly);
     check_launch("hybrid forward kernels");
 }
 
-// o: the forward's output (same layout as dO).  dS: scratch for the remainder's {dS, P} pairs, [NB][nr].
+// o: the forward's output (same layout as dO).
 template <bool ST>
 static void launch_hyb_bwd(SparseAttn* a, const float* Q, const float* K, const float* V, const float* P,
-                           const float* dO, const float* o, float* dS, float* dQ, float* dK, float* dV,
+                           const float* dO, const float* o, const HybBackwardWork& work, float* dQ, float* dK, float* dV,
                            const int* Offsets, int nnz, const Layouts& ly) {
     PhaseRange phase("spion backward (hybrid kernels)");
-    if (!ensure_ws(&a->ws_rowsum, (size_t)a->NB * a->L)) return;
+    if (!work.rowsum && !ensure_ws(&a->ws_rowsum, (size_t)a->NB * a->L)) return;
+    float* rowsum = work.rowsum ? work.rowsum : a->ws_rowsum;
+    float2* pairs = work.pairs;
     a->last_path = a->pat.hyb_dense ? 3 : 2;
     const int nbr = a->L / 32;
     const long long rows = (long long)a->NB * a->L;
     const bool one_r = a->pat.max_row_tiles <= 2 * HYB_MAXT1, one_c = a->pat.max_col_tiles <= 2 * HYB_MAXT1;
     const dim3 grid_t(nbr * a->NB);
     const dim3 grid_g((unsigned)((rows + HYB_GWAVES - 1) / HYB_GWAVES)), block_g(64 * HYB_GWAVES);
-    float2* pairs = reinterpret_cast<float2*>(dS);
     const bool lds = a->pat.rem_lds, two = lds && rem_per_quad(a) == 2;
     if (a->bwd_passes & 1) {
         if (one_r)
             hipLaunchKernelGGL((hyb_tile_bwd_row_kernel<1, ST>), grid_t, dim3(64), 0, a->hdr.stream, K, V, P, dO, o,
-                               a->ws_rowsum, dQ, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
+                               rowsum, dQ, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
         else
             hipLaunchKernelGGL((hyb_tile_bwd_row_kernel<4, ST>), grid_t, dim3(256), 0, a->hdr.stream, K, V, P, dO, o,
-                               a->ws_rowsum, dQ, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
+                               rowsum, dQ, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
 #define SPION_REM_ROW(NO_)                                                                                            \
-    SPION_REM_LAUNCH((rem_bwd_row_kernel<ST, NO_>), NO_, K, V, P, dO, (const float*)a->ws_rowsum, pairs, dQ, Offsets, \
+    SPION_REM_LAUNCH((rem_bwd_row_kernel<ST, NO_>), NO_, K, V, P, dO, (const float*)rowsum, pairs, dQ, Offsets, \
                      a->pat.rem, a->L, a->NB, nnz, a->scale, ly)
         if (two) SPION_REM_ROW(2);
         else if (lds) SPION_REM_ROW(1);
         else
             hipLaunchKernelGGL(hyb_rem_bwd_row_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, K, V, P, dO,
-                               (const float*)a->ws_rowsum, pairs, dQ, a->pat.hyb, a->L, a->NB, nnz, a->scale, ly);
+                               (const float*)rowsum, pairs, dQ, a->pat.hyb, a->L, a->NB, nnz, a->scale, ly);
 #undef SPION_REM_ROW
     }
     if (a->bwd_passes & 2) {
         if (one_c)
             hipLaunchKernelGGL((hyb_tile_bwd_col_kernel<1, ST>), grid_t, dim3(64), 0, a->hdr.stream, Q, V, P, dO,
-                               (const float*)a->ws_rowsum, dK, dV, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
+                               (const float*)rowsum, dK, dV, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
         else
             hipLaunchKernelGGL((hyb_tile_bwd_col_kernel<4, ST>), grid_t, dim3(256), 0, a->hdr.stream, Q, V, P, dO,
-                               (const float*)a->ws_rowsum, dK, dV, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
+                               (const float*)rowsum, dK, dV, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
 #define SPION_REM_COL(NO_)                                                                                          \
     SPION_REM_LAUNCH((rem_bwd_col_kernel<ST, NO_>), NO_, Q, dO, (const float2*)pairs, dK, dV, a->pat.rem, a->L, a->NB, \
                      ly)
@@ -1739,7 +1765,8 @@ static void launch_elem_bwd(SparseAttn* a, const float* Q, const float* K, const
 
 // krow: Kt is K itself, row-major [NB][L][d], not the transposed copy of the reference's ABI.
 void sparse_forward(void* h, const float* Q, const float* Kt, const float* V, const KeyTerms& Mask, float* Attn,
-                    float* Out, const int* Offsets, const int* Columns, int nnz, bool mask_entry, bool krow) {
+                    float* Out, const int* Offsets, const int* Columns, int nnz, bool mask_entry, bool krow,
+                    const CallScratch& scratch) {
     SparseAttn* a = as_sparse(h, "attn_forward");
     if (!a) return;
     if (a->has_mask != mask_entry || a->is_bf16) {
@@ -1789,7 +1816,8 @@ void sparse_forward(void* h, const float* Q, const float* Kt, const float* V, co
         return;
     }
     a->last_path = 2;
-    const bool hybrid = take_hybrid_forward(a, {Q, Kt, V, Out});  // (a transposed copy of Kt is aligned as well)
+    HybForwardWork work;
+    const bool hybrid = take_hybrid_forward(a, {Q, Kt, V, Out}, scratch, &work);  // (a transposed copy of Kt is aligned as well)
     float* hyb_ocopy = hybrid ? ocache_for_forward(a, Attn) : nullptr;
     if (!hyb_ocopy) ocache_drop(a, Attn);
     const float* Krm = Kt;  // the element kernels read K row-major
@@ -1799,7 +1827,7 @@ void sparse_forward(void* h, const float* Q, const float* Kt, const float* V, co
         Krm = a->ws_trans;
     }
     if (hybrid) {
-        launch_hyb_fwd<false>(a, Q, Krm, V, Mask, Attn, Out, hyb_ocopy, Offsets, nnz, Layouts{});
+        launch_hyb_fwd<false>(a, Q, Krm, V, Mask, Attn, Out, hyb_ocopy, Offsets, nnz, Layouts{}, work);
         return;
     }
     switch (a->d) {
@@ -1815,7 +1843,7 @@ void sparse_forward(void* h, const float* Q, const float* Kt, const float* V, co
 // from it and no kept copy is looked up.  vrow: Vt is V itself, row-major [NB][L][d].
 void sparse_backward(void* h, const float* Q, const float* K, const float* Vt, const float* P, const float* dO,
                      float* dP, float* dS, float* dQ, float* dK, float* dV, const int* Offsets, const int* Columns,
-                     int nnz, const float* Out, bool vrow) {
+                     int nnz, const float* Out, bool vrow, const CallScratch& scratch) {
     SparseAttn* a = as_sparse(h, "attn_backward");
     if (!a) return;
     (void)dP;
@@ -1843,6 +1871,7 @@ void sparse_backward(void* h, const float* Q, const float* K, const float* Vt, c
         return;
     }
     a->last_path = 2;
+    if (!dS) dS = scratch.floats >= (size_t)a->NB * (size_t)std::max(nnz, 1) ? scratch.p : nullptr;
     if (!dS) {
         set_error("attn_backward: the element path needs the dS scratch buffer");
         return;
@@ -1857,9 +1886,9 @@ void sparse_backward(void* h, const float* Q, const float* K, const float* Vt, c
         // the hybrid kernels take the row sums from the forward's output (the caller's, or the handle's kept copy);
         // without it the gather kernels below serve the same P
         const float* o = Out ? Out : ocache_for_backward(a, P);
-        float* pairs;
-        if (o && take_hybrid_backward(a, {Q, K, Vrm, dO, o, dQ, dK, dV}, dS, nnz, &pairs)) {
-            launch_hyb_bwd<false>(a, Q, K, Vrm, P, dO, o, pairs, dQ, dK, dV, Offsets, nnz, Layouts{});
+        HybBackwardWork work;
+        if (o && take_hybrid_backward(a, {Q, K, Vrm, dO, o, dQ, dK, dV}, dS, scratch, &work)) {
+            launch_hyb_bwd<false>(a, Q, K, Vrm, P, dO, o, work, dQ, dK, dV, Offsets, nnz, Layouts{});
             return;
         }
     }
@@ -2002,7 +2031,7 @@ static SparseAttn* strided_handle(void* h, const char* who, const int* Offsets, 
 
 void sparse_forward_strided(void* h, const float* Q, const float* K, const float* V, const KeyTerms& Mask, float* Attn,
                             float* Out, const int* Offsets, const int* Columns, int nnz, int heads,
-                            const HeadLayout& in, const HeadLayout& out) {
+                            const HeadLayout& in, const HeadLayout& out, const CallScratch& scratch) {
     const char* who = "attn_forward_strided";
     SparseAttn* a = strided_handle(h, who, Offsets, Columns, nnz, heads);
     if (!a) return;
@@ -2030,8 +2059,9 @@ void sparse_forward_strided(void* h, const float* Q, const float* K, const float
     ly.H = heads;
     if (!a->pat.tiled) {
         ocache_drop(a, Attn);  // the backward of these entry points is handed Out
-        if (take_hybrid_forward(a, {Q, K, V, Out})) {
-            launch_hyb_fwd<true>(a, Q, K, V, Mask, Attn, Out, nullptr, Offsets, nnz, ly);
+        HybForwardWork work;
+        if (take_hybrid_forward(a, {Q, K, V, Out}, scratch, &work)) {
+            launch_hyb_fwd<true>(a, Q, K, V, Mask, Attn, Out, nullptr, Offsets, nnz, ly, work);
             return;
         }
         a->last_path = 2;
@@ -2057,7 +2087,8 @@ void sparse_forward_strided(void* h, const float* Q, const float* K, const float
 
 void sparse_backward_strided(void* h, const float* Q, const float* K, const float* V, const float* P, const float* Out,
                              const float* dO, float* dQ, float* dK, float* dV, const int* Offsets, const int* Columns,
-                             int nnz, int heads, const HeadLayout& in, const HeadLayout& out, const HeadLayout& grad) {
+                             int nnz, int heads, const HeadLayout& in, const HeadLayout& out, const HeadLayout& grad,
+                             const CallScratch& scratch) {
     const char* who = "attn_backward_strided";
     SparseAttn* a = strided_handle(h, who, Offsets, Columns, nnz, heads);
     if (!a) return;
@@ -2077,31 +2108,34 @@ void sparse_backward_strided(void* h, const float* Q, const float* K, const floa
         set_error("%s: the gradient layout maps two elements to one address", who);
         return;
     }
-    if (!ensure_ws(&a->ws_rowsum, (size_t)a->NB * a->L)) return;
     Layouts ly{};
     ly.in = in;
     ly.out = out;
     ly.grad = grad;
     ly.H = heads;
     if (!a->pat.tiled) {
-        // these entry points have no dS argument: the scratch is the handle's (grown outside graph capture only)
-        if (!ensure_ws_grow(a, &a->ws_ds, &a->ws_ds_count, (size_t)a->NB * (size_t)std::max(nnz, 1), who)) return;
-        float* pairs;
-        if (take_hybrid_backward(a, {Q, K, V, dO, Out, dQ, dK, dV}, a->ws_ds, nnz, &pairs)) {
-            launch_hyb_bwd<true>(a, Q, K, V, P, dO, Out, pairs, dQ, dK, dV, Offsets, nnz, ly);
+        // dS lies in the caller's scratch; without one that holds it in the handle's (grown outside graph capture only)
+        const size_t ds_floats = (size_t)a->NB * (size_t)std::max(nnz, 1);
+        const bool callers = scratch.floats >= ds_floats;
+        if (!callers && !ensure_ws_grow(a, &a->ws_ds, &a->ws_ds_count, ds_floats, who)) return;
+        float* ds = callers ? scratch.p : a->ws_ds;
+        HybBackwardWork work;
+        if (take_hybrid_backward(a, {Q, K, V, dO, Out, dQ, dK, dV}, ds, callers ? scratch : CallScratch{}, &work)) {
+            launch_hyb_bwd<true>(a, Q, K, V, P, dO, Out, work, dQ, dK, dV, Offsets, nnz, ly);
             return;
         }
         a->last_path = 2;
         switch (a->d) {
-            case 16: launch_elem_bwd<16, true>(a, Q, K, V, P, dO, a->ws_ds, dQ, dK, dV, Offsets, Columns, nnz, ly); break;
-            case 32: launch_elem_bwd<32, true>(a, Q, K, V, P, dO, a->ws_ds, dQ, dK, dV, Offsets, Columns, nnz, ly); break;
-            case 64: launch_elem_bwd<64, true>(a, Q, K, V, P, dO, a->ws_ds, dQ, dK, dV, Offsets, Columns, nnz, ly); break;
-            default: launch_elem_bwd<128, true>(a, Q, K, V, P, dO, a->ws_ds, dQ, dK, dV, Offsets, Columns, nnz, ly); break;
+            case 16: launch_elem_bwd<16, true>(a, Q, K, V, P, dO, ds, dQ, dK, dV, Offsets, Columns, nnz, ly); break;
+            case 32: launch_elem_bwd<32, true>(a, Q, K, V, P, dO, ds, dQ, dK, dV, Offsets, Columns, nnz, ly); break;
+            case 64: launch_elem_bwd<64, true>(a, Q, K, V, P, dO, ds, dQ, dK, dV, Offsets, Columns, nnz, ly); break;
+            default: launch_elem_bwd<128, true>(a, Q, K, V, P, dO, ds, dQ, dK, dV, Offsets, Columns, nnz, ly); break;
         }
         check_launch("elem_bwd kernels");
         return;
     }
     a->last_path = 1;
+    if (!ensure_ws(&a->ws_rowsum, (size_t)a->NB * a->L)) return;
     if (a->d == 32) launch_tile_bwd<32, true, true>(a, Q, K, V, P, dO, dQ, dK, dV, Offsets, nnz, Out, ly);
     else launch_tile_bwd<64, true, true>(a, Q, K, V, P, dO, dQ, dK, dV, Offsets, nnz, Out, ly);
     check_launch("tile_bwd kernels");

@@ -106,68 +106,126 @@ def test_infinities_stay_in_their_rows():
     cpp.destroy(handle)
 
 
-def test_scattered_patterns_and_capture():
-    """A pattern without dense structure: float64 agrees; a graph recorded before the handle has its workspaces holds the
-    element kernels, one recorded after a step the kernels by ranges."""
-    B, H, L = 32, 2, 576
-    gen = torch.Generator(device="cuda").manual_seed(3)
-    pattern = (torch.rand(L, L, generator=gen, device="cuda") < 0.05).float()
+def _scattered(L, gen, share=0.05):
+    """A pattern without dense structure, a long row and an empty one."""
+    pattern = (torch.rand(L, L, generator=gen, device="cuda") < share).float()
     pattern[17, ::2] = 1.0
     pattern[9] = 0.0
-    q, k, v, do = (torch.randn(B, H, L, 32, generator=gen, device="cuda") for _ in range(4))
-    where = pattern.bool()
+    return pattern
+
+
+def _registered(handle, pattern):
+    """The index of a pattern on file with a handle: (device tensors, number of entries)."""
+    where, L = pattern.bool(), pattern.shape[0]
     off = torch.zeros(L + 1, dtype=torch.int32)
     off[1:] = where.sum(1).cumsum(0).cpu()
     col = where.nonzero()[:, 1].to(torch.int32).cpu()
-    d_off, d_col, count = off.cuda(), col.cuda(), where.sum(1).to(torch.int32)
+    index = off.cuda(), col.cuda(), where.sum(1).to(torch.int32)
     nnz = int(off[-1])
     core = _lib.core()
+    assert core.spion_register_pattern(handle, index[0].data_ptr(), index[1].data_ptr(), nnz, off.data_ptr(), col.data_ptr()) == 0
+    return index, nnz
+
+
+def test_scattered_patterns_and_capture():
+    """A pattern without dense structure, without scratch (the element kernels) and with (the kernels by ranges): float64 agrees,
+    and graphs of both give the eager bits, recorded before the handle has run anything."""
+    B, H, L = 32, 2, 576
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    pattern = _scattered(L, gen)
+    q, k, v, do = (torch.randn(B, H, L, 32, generator=gen, device="cuda") for _ in range(4))
+    where = pattern.bool()
+    core = _lib.core()
     cpp, handle, _ = _module(B, H, L, False)
-    assert core.spion_register_pattern(handle, d_off.data_ptr(), d_col.data_ptr(), nnz, off.data_ptr(), col.data_ptr()) == 0
+    (d_off, d_col, row_counts), nnz = _registered(handle, pattern)
     ds = torch.empty(B * H * nnz, device="cuda")
     out = torch.empty_like(q)
     p = torch.empty(B * H, nnz, device="cuda")
     grads = [torch.empty_like(q) for _ in range(3)]
+    need = [core.spion_attn_scratch(handle, d_off.data_ptr(), d_col.data_ptr(), nnz, back) for back in (0, 1)]
+    assert need[0] > 0 and need[1] >= B * H * nnz
+    scratch = torch.empty(max(need), device="cuda")
 
-    def step():
-        core.spion_set_stream(handle, torch.cuda.current_stream().cuda_stream)
-        at = (d_off.data_ptr(), d_col.data_ptr(), count.data_ptr(), nnz)
+    def plain():
+        at = (d_off.data_ptr(), d_col.data_ptr(), row_counts.data_ptr(), nnz)
         core.spion_attn_forward_rowmajor(handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), None, p.data_ptr(), out.data_ptr(), *at)
         core.spion_attn_backward_rowmajor(handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), p.data_ptr(), out.data_ptr(),
                                           do.data_ptr(), ds.data_ptr(), *(g.data_ptr() for g in grads), *at)
 
-    def record():
+    def with_scratch():
+        at = (d_off.data_ptr(), d_col.data_ptr(), nnz, H)
+        core.spion_attn_forward_scratch(handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), None, 0, p.data_ptr(), out.data_ptr(), *at,
+                                        None, None, scratch.data_ptr(), need[0])
+        core.spion_attn_backward_scratch(handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), p.data_ptr(), out.data_ptr(), do.data_ptr(),
+                                         *(g.data_ptr() for g in grads), *at, None, None, None, scratch.data_ptr(), need[1])
+
+    def record(step):
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
+            core.spion_set_stream(handle, torch.cuda.current_stream().cuda_stream)
             step()
         _lib.check_error("capture")
         return graph
 
-    def replayed(graph):
-        for t in (out, p, *grads):
+    def results(run):
+        for t in (out, p, *grads, scratch):
             t.fill_(float("nan"))
-        graph.replay()
+        run()
         torch.cuda.synchronize()
         return [t.clone() for t in (out, p, *grads)]
 
-    before = record()
-    first = replayed(before)
-    for t in (out, p, *grads):
-        t.fill_(float("nan"))
-    step()
-    torch.cuda.synchronize()
+    steps = plain, with_scratch
+    graphs = [record(step) for step in steps]
+    core.spion_set_stream(handle, torch.cuda.current_stream().cuda_stream)
+    eager = [results(step) for step in steps]
+    _lib.check_error("steps")
     assert core.spion_last_path(handle) == 2
-    eager = [t.clone() for t in (out, p, *grads)]
-    after = record()
+    assert not torch.equal(eager[0][0], eager[1][0])  # other kernels, other roundings
     for _ in range(3):
-        assert all(torch.equal(x, y) for x, y in zip(replayed(after), eager))
-        assert all(torch.equal(x, y) for x, y in zip(replayed(before), first))
+        for graph, want in zip(graphs, eager):
+            assert all(torch.equal(x, y) for x, y in zip(results(graph.replay), want))
     at = lambda t: t[B // 2, 1][None]
     ref = _reference(at(q), at(k), at(v), at(do), pattern.double()[None], None)
-    for results in (first, eager):
-        got = (results[1][(B // 2) * H + 1],) + tuple(at(results[i]) for i in (0, 2, 3, 4))
+    for got in eager:
+        got = (got[1][(B // 2) * H + 1],) + tuple(at(got[i]) for i in (0, 2, 3, 4))
         for name, x, y in zip(("P", "out", "dQ", "dK", "dV"), got, (ref[0][0][where],) + ref[1:]):
             tol = 2e-5 * (y.abs() + y.pow(2).mean().sqrt())
             assert float(((x.double() - y).abs() / tol).max()) <= 1.0, name
     core.spion_set_stream(handle, 0)
+    cpp.destroy(handle)
+
+
+@pytest.mark.parametrize("kind", ["scattered", "window"])
+@pytest.mark.parametrize("views", [False, True])
+def test_calls_share_nothing_in_the_handle(kind, views):
+    """Two steps of one module on two streams at a time: the bits of the same steps one after the other."""
+    B, H, L = 32, 2, 1024
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    pattern = _scattered(L, gen) if kind == "scattered" else _pattern(L, gen)
+    shape = (B, L, H, 32) if views else (B, H, L, 32)
+    make = lambda: torch.randn(*shape, generator=gen, device="cuda")
+    inputs = [[make().transpose(1, 2) if views else make() for _ in range(4)] for _ in range(2)]
+    ones = torch.ones(B, L, device="cuda")
+    cpp, handle, module = _module(B, H, L, False)
+
+    def step(which):
+        q, k, v = (t.detach().requires_grad_() for t in inputs[which][:3])
+        out, p = module(q, k, v, ones, pattern)
+        out.backward(inputs[which][3])
+        return out.detach(), p.detach(), q.grad, k.grad, v.grad
+
+    want = [step(0), step(1)]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for s in streams:
+        s.wait_stream(torch.cuda.current_stream())
+    got = [[], []]
+    for _ in range(4):
+        for which, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                got[which].append(step(which))
+    torch.cuda.synchronize()
+    for which in range(2):
+        for results in got[which]:
+            assert all(torch.equal(x, y) for x, y in zip(results, want[which]))
     cpp.destroy(handle)
