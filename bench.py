@@ -64,13 +64,6 @@ def _roof_of(kernel, ms, flops, ceiling, nbytes):
     return dict(bound=bound, kernel=kernel, achieved=work, peak=peak, unit=unit, traffic=None)
 
 
-def _remainder_in_lds(L, NB):
-    """Whether the remainder's kernels of the hybrid path take their operands from LDS (the library's rule)."""
-    if L < 512 or L > 1 << 18 or "SPION_HYB_GATHER" in os.environ:
-        return False
-    return NB * -(-L // 256) * 4 >= torch.cuda.get_device_properties(0).multi_processor_count
-
-
 def _event_ms(fn, iters, warm=3):
     """Average duration of fn() in ms from HIP events on the current (= the library's) stream."""
     for _ in range(warm):
@@ -799,7 +792,7 @@ def bench_sparse_layer(args, dev, workload, full=True):
     # launches
     ranges = ("rem_fwd_kernel + hyb_tile_fwd_kernel + rem_prob_kernel", "hyb_tile_bwd_row_kernel + rem_bwd_row_kernel",
               "hyb_tile_bwd_col_kernel + rem_bwd_col_kernel")
-    by_ranges = d == 32 and L % 32 == 0 and _remainder_in_lds(L, NB)
+    by_ranges = _lib.core().spion_debug_counter(handle, 3) == 1
     names = {1: ("tile_fwd_kernel", "tile_bwd_row_kernel", "tile_bwd_col_kernel"),
              2: ranges if by_ranges else ("elem_fwd_kernel", "elem_bwd_row_kernel", "elem_bwd_col_kernel"),
              3: ranges if by_ranges else ("hyb_rem_logits_kernel + hyb_tile_fwd_kernel + hyb_rem_pv_kernel",

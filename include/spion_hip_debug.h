@@ -21,8 +21,13 @@ void spion_set_backward_passes(void* handle, int mask);
 /* Counters of a sparse handle: which = 0 -> pattern analyses that copied the index back from the device (and
  * waited for the stream), which = 1 -> analyses made from host arrays (spion_register_pattern), which = 2 ->
  * workspace buffers that a larger pattern has outgrown and that stay allocated until the handle is destroyed (a HIP
- * graph recorded before the growth still points at them).  -1 otherwise. */
+ * graph recorded before the growth still points at them), which = 3 -> 1 if the remainder of the pattern last used goes by
+ * ranges whose rows lie in LDS.  -1 otherwise. */
 int spion_debug_counter(void* handle, int which);
+
+/* Whether the library lets the remainder of an element pattern (`entries` a head) go by ranges (1) or gathers it (0), on a
+ * device of so many compute units (host only: needs no device); -1 on bad arguments. */
+int spion_debug_remainder_by_ranges(int num_batches, int seq_len, long long entries, int compute_units);
 
 /* Whether the backward of row-major heads of a dense handle runs as work-groups that share their tiles on the current
  * device (1), or with four wavefronts to a strip (0); -1 for other handles. */
@@ -54,11 +59,9 @@ int spion_debug_bf16_plan(const int* tile_ptr, int nstrips, int pairs, int num_b
  *   SPION_BF16_NO_PAIRS  the bf16 forward and row pass take one strip per wavefront on every pattern (default: two
  *                        strips per wavefront on masks of 64 x 64 blocks and larger, contiguous heads);
  *   SPION_BF16_ROW_PAIRS=0  the same for the row pass alone.
- *   SPION_HYB_GATHER     hybrid patterns: the remainder's column pass gathers its Q and dO rows from L2, one wavefront
- *                        per column (default, when seq_len is a multiple of 1024 and num_batches * seq_len / 256 >= 256:
- *                        work-groups of 1024, 512 or 256 columns with the rows of a range of the sequence in LDS; the
- *                        element kernels' column pass at emb_dim 32 likewise), and so do the forward's two remainder
- *                        kernels (default: operands in LDS when num_batches * seq_len / 512, resp. / 1024, >= 256);
+ *   SPION_HYB_GATHER     element and hybrid patterns: the remainder's kernels, and the element kernels' column pass, gather
+ *                        their rows from L2, one wavefront per row or column (default: rows of a range of the sequence in
+ *                        LDS where that is the faster way, which depends on heads, length and entries);
  * Read whenever a bf16 handle indexes a pattern (tests):
  *   SPION_BF16_LANES     number of persistent wavefronts the bf16 kernels are launched with (default: eight per
  *                        compute unit); a handful makes each one walk many strips of several heads in a row.

@@ -94,6 +94,7 @@ int sparse_sizes(void*, int*, int*, int*);
 void sparse_force_element(void*, int);
 void sparse_set_bwd_passes(void*, int);
 int sparse_debug_counter(void*, int);
+int sparse_debug_rem_by_ranges(int, int, long long, int);
 int sparse_debug_bf16_plan(const int*, int, int, int, int, int*, int, int*, int, int*, int, int*, int, int*);
 void sparse_use_ocache(void*, int);
 void* sparse_bf16_init(int, int, int, int);
@@ -396,6 +397,9 @@ void spion_force_element_path(void* h, int on) { sparse_force_element(h, on); }
 void spion_set_backward_passes(void* h, int mask) { sparse_set_bwd_passes(h, mask); }
 int spion_debug_dense_groups(void* h) { return dense_groups(h); }
 int spion_debug_counter(void* h, int which) { return sparse_debug_counter(h, which); }
+int spion_debug_remainder_by_ranges(int num_batches, int seq_len, long long entries, int compute_units) {
+    return num_batches > 0 && seq_len > 0 && compute_units > 0 ? sparse_debug_rem_by_ranges(num_batches, seq_len, entries, compute_units) : -1;
+}
 int spion_debug_bf16_plan(const int* tile_ptr, int nstrips, int pairs, int num_batches, int lanes, int* items,
                           int cap_items, int* lane_ptr, int cap_ptr, int* lane_ent, int cap_ent, int* longs,
                           int cap_longs, int* counts) {

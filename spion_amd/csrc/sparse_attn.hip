@@ -706,18 +706,39 @@ static int bf16_lanes() {
     return device_cus() * 8;
 }
 
-// Whether the remainder of an element pattern keeps its rows in LDS (remainder_kernels.h), lists by ranges instead of by
-// whole rows and columns; SPION_HYB_GATHER: never.  With a quarter of the machine's compute units at work the two are level
-// (16 heads of 1024 with 17 remainder entries a row: forward 12 us against 17 gathered from L2, row pass 12 / 11, column pass
-// 13 / 14), with more the gathers are behind everywhere (32 of 1024 with 27: 18 / 28, 17 / 21, 17 / 26; 16 of 4096 with 80:
-// 53 / 93, 55 / 76, 50 / 93).  A list's word holds the position in a row of the pattern in 18 bits.
+// Rows (columns) per quad of the remainder's kernels by ranges, work-groups of 256 or 512, one per CU and round: a round of the
+// larger ones takes 1.6 times one of the smaller (64 heads of 4096: two of 87 us against four of 54; 32 of 2048: 56 against 37 in all).
+struct RemRounds {
+    int per_quad;
+    double rounds;  // of the smaller work-groups' length
+};
+static RemRounds rem_rounds(int NB, int L, int cus) {
+    const auto rounds = [&](int per) { return ((long long)NB * ((L + per - 1) / per) + cus - 1) / cus; };
+    const long long one = rounds(REM_QUADS), two = rounds(2 * REM_QUADS);
+    return 10 * one > 16 * two ? RemRounds{2, 1.6 * two} : RemRounds{1, (double)one};
+}
+// Whether the remainder of an element pattern, nr entries a head, goes by ranges whose rows lie in LDS (remainder_kernels.h) or
+// entry by entry from L2.  Gathers cost by rows and entries, ranges by work-groups times ranges, whatever is in them, and one CU
+// takes one work-group however few there are.  Forward + backward on 256 CUs in us, nr / L = r entries a row:
+//     by ranges  10 + rounds (11 L / 512 + 0.8 r)        gathers  NB L / 65536 (115 + 2.2 r)
+// (r from 2 to 300, 1 to 256 heads of 512 to 32768: the rule takes the faster side, or one at most 17 % behind.)  Measured, by ranges /
+// gathers: 64 heads of 4096, r = 16: 354 / 403, 128: 956 / 1382; 16 of 1024, 8: 42 / 35; 64 of 1024, 16: 71 / 97; 4 of 4096, 16: 92 / 36;
+// 8 of 8192, 16: 188 / 148, 300: 493 / 715; 1 of 16384, 16: 300 / 43; 4 of 32768, 16: 895 / 532, 300: 1565 / 2458.  It also bounds the
+// lists' offsets, L / 512 for every row and column, to a few tens and a fraction of the entries.  A list's word holds the position in a row
+// of the pattern in 18 bits.
+static bool rem_by_ranges(int NB, int L, long long nr, int cus) {
+    if (L < REM_RANGE || L > (1 << 18) || nr <= 0) return false;
+    const double ranges = (L + REM_RANGE - 1) / REM_RANGE, r = (double)nr / L;
+    return 10 + rem_rounds(NB, L, cus).rounds * (11 * ranges + 0.8 * r) < (double)NB * L / (256.0 * cus) * (115 + 2.2 * r);
+}
+int sparse_debug_rem_by_ranges(int NB, int L, long long nr, int cus) { return rem_by_ranges(NB, L, nr, cus); }
+// SPION_HYB_GATHER: never by ranges
 static bool rem_gather_forced() {
     static const bool gather = getenv("SPION_HYB_GATHER") != nullptr;
     return gather;
 }
-static bool rem_in_lds(const SparseAttn* a) {
-    return !rem_gather_forced() && a->L >= REM_RANGE && a->L <= (1 << 18) &&
-           (long long)a->NB * ((a->L + REM_QUADS - 1) / REM_QUADS) * 4 >= device_cus();
+static bool rem_in_lds(const SparseAttn* a, long long nr) {
+    return !rem_gather_forced() && rem_by_ranges(a->NB, a->L, nr, device_cus());
 }
 
 // Copy the index to the host once (unless the caller hands over host copies), validate it, detect the tile
@@ -922,8 +943,8 @@ static bool analyse_pattern(SparseAttn* a, const int* Offsets, const int* Column
         pi.max_col_tiles = mc;
     } else {
         // ---- hybrid split: aligned 32x32 tiles with at least HYB_MIN_FILL entries become dense tiles (at most
-        // HYB_MAX_ROW_TILES per block row, the fullest first), everything else is the remainder.  Where the remainder's rows
-        // lie in LDS every pattern goes this way, whatever part of it the tiles hold (no tiles at all: 32 heads of 4096, 300
+        // HYB_MAX_ROW_TILES per block row, the fullest first), everything else is the remainder.  Where the remainder goes by
+        // ranges (rem_by_ranges) every pattern is split, whatever part of it the tiles hold (no tiles at all: 32 heads of 4096, 300
         // random entries a row, forward 542 us gathered from L2 / 213, row pass 548 / 384, column pass 690 / 252); with gathers
         // only patterns that are mostly tiles.
         if (!a->force_element && a->d == 32 && L % 32 == 0 && nnz > 0) {
@@ -954,7 +975,7 @@ static bool analyse_pattern(SparseAttn* a, const int* Offsets, const int* Column
             }
             int nt = (int)t_col.size();
             pi.hyb_dense = nt > 0 && dense_entries * 2 >= (long long)nnz;
-            if (pi.hyb_dense || rem_in_lds(a)) {
+            if (pi.hyb_dense || rem_in_lds(a, nnz - dense_entries)) {
                 if (nt == 0) {  // one that no block row or column lists: what the kernels' clamped look-ups find
                     t_col.push_back(0);
                     t_row.push_back(0);
@@ -993,7 +1014,7 @@ static bool analyse_pattern(SparseAttn* a, const int* Offsets, const int* Column
                 }
                 std::vector<int> t_ci(t_ct.size());
                 for (size_t e = 0; e < t_ct.size(); ++e) t_ci[e] = t_row[t_ct[e]];
-                pi.rem_lds = rem_in_lds(a);
+                pi.rem_lds = rem_in_lds(a, nr);
                 if (pi.rem_lds) {
                     // by ranges of REM_RANGE columns, then rows, columns ascending; and by ranges of rows, then columns
                     const int nk = (L + REM_RANGE - 1) / REM_RANGE;
@@ -1590,13 +1611,6 @@ static int elem_lds_columns(const SparseAttn* a) {
 #define SPION_ELEM_COL_LDS(ST_, NC_, ...)                                                                       \
     hipLaunchKernelGGL((elem_bwd_col_lds_kernel<ST_, NC_>), dim3(a->NB * hyb_groups(a->L, 128 * NC_)),          \
                        dim3(HYB_CL_THREADS), 0, a->hdr.stream, __VA_ARGS__)
-// Rows (columns) per quad of the remainder's kernels, work-groups of 256 or 512, one per CU and round: a round of the larger
-// ones takes 1.6 times one of the smaller (64 heads of 4096: two of 87 us against four of 54; 32 of 2048: 56 against 37 in all).
-static int rem_per_quad(const SparseAttn* a) {
-    const long long cus = device_cus();
-    const auto rounds = [&](int per) { return ((long long)a->NB * hyb_groups(a->L, per) + cus - 1) / cus; };
-    return 10 * rounds(REM_QUADS) > 16 * rounds(2 * REM_QUADS) ? 2 : 1;
-}
 #define SPION_REM_LAUNCH(KERNEL_, NO_, ...)                                                                                 \
     hipLaunchKernelGGL((KERNEL_), dim3(a->NB * hyb_groups(a->L, (NO_) * REM_QUADS)), dim3(REM_THREADS), 0, a->hdr.stream, \
                        __VA_ARGS__)
@@ -1624,7 +1638,7 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
     const dim3 grid_g((unsigned)((rows + HYB_GWAVES - 1) / HYB_GWAVES)), block_g(64 * HYB_GWAVES);
     float2* stats = work.stats;
     float* raw = work.raw;
-    const bool lds = a->pat.rem_lds, two = lds && rem_per_quad(a) == 2;
+    const bool lds = a->pat.rem_lds, two = lds && rem_rounds(a->NB, a->L, device_cus()).per_quad == 2;
 #define SPION_HYB_TILES(MASKED, WAVES_, MAXT_, REM_)                                                                  \
     hipLaunchKernelGGL((hyb_tile_fwd_kernel<MASKED, WAVES_, MAXT_, ST, REM_>), grid_t, block_t, 0, a->hdr.stream, Q,  \
                        K, V, Mask, Attn, Out, REM_ ? ocopy : nullptr, stats, Offsets, a->pat.hyb, a->L, nbr, a->NB,   \
@@ -1675,7 +1689,7 @@ static void launch_hyb_bwd(SparseAttn* a, const float* Q, const float* K, const 
     const bool one_r = a->pat.max_row_tiles <= 2 * HYB_MAXT1, one_c = a->pat.max_col_tiles <= 2 * HYB_MAXT1;
     const dim3 grid_t(nbr * a->NB);
     const dim3 grid_g((unsigned)((rows + HYB_GWAVES - 1) / HYB_GWAVES)), block_g(64 * HYB_GWAVES);
-    const bool lds = a->pat.rem_lds, two = lds && rem_per_quad(a) == 2;
+    const bool lds = a->pat.rem_lds, two = lds && rem_rounds(a->NB, a->L, device_cus()).per_quad == 2;
     if (a->bwd_passes & 1) {
         if (one_r)
             hipLaunchKernelGGL((hyb_tile_bwd_row_kernel<1, ST>), grid_t, dim3(64), 0, a->hdr.stream, K, V, P, dO, o,
@@ -2506,7 +2520,7 @@ int sparse_debug_counter(void* h, int which) {
     SparseAttn* a = as_sparse(h, "spion_debug_counter");
     if (!a) return -1;
     return which == 0 ? a->analyses_from_device : which == 1 ? a->analyses_from_host
-         : which == 2 ? (int)a->retired.size() : -1;
+         : which == 2 ? (int)a->retired.size() : which == 3 ? (int)a->pat.rem_lds : -1;
 }
 void sparse_set_bwd_passes(void* h, int mask) {
     SparseAttn* a = as_sparse(h, "spion_set_backward_passes");

@@ -44,7 +44,7 @@ def _module(B, H, L, masked):
 
 
 # one range; a second one of 32 rows; work-groups of 256 rows whose last is partial; work-groups of 512, the last partial
-@pytest.mark.parametrize("B,H,L,masked", [(32, 2, 512, False), (16, 2, 544, True), (11, 2, 1056, False), (35, 2, 1056, True),
+@pytest.mark.parametrize("B,H,L,masked", [(32, 2, 512, False), (24, 2, 544, True), (14, 2, 1056, False), (35, 2, 1056, True),
                                           (35, 2, 1056, False), (32, 2, 2048, False)])
 @pytest.mark.parametrize("views", [False, True])
 def test_ranges_and_batches(B, H, L, masked, views):
@@ -62,6 +62,7 @@ def test_ranges_and_batches(B, H, L, masked, views):
     out.backward(do)
     torch.cuda.synchronize()
     assert _lib.core().spion_last_path(handle) == 3
+    assert _lib.core().spion_debug_counter(handle, 3) == 1
     where = pattern.bool()
     p = None if masked else p.detach().reshape(B, H, -1)  # the masked module does not return it
     for b, h in ((0, 0), (B // 2, H - 1), (B - 1, H - 1)):
@@ -91,6 +92,7 @@ def test_infinities_stay_in_their_rows():
     out, p = module(q, k, v, torch.ones(B, L, device="cuda"), pattern)
     out.backward(do)
     assert _lib.core().spion_last_path(handle) == 3
+    assert _lib.core().spion_debug_counter(handle, 3) == 1
     i = torch.arange(L, device="cuda")
     near = (i - far).abs() < 128  # the window's tiles
     reads_v = near | (pattern[:, far] > 0)
@@ -143,7 +145,7 @@ def test_scattered_patterns_and_capture():
     p = torch.empty(B * H, nnz, device="cuda")
     grads = [torch.empty_like(q) for _ in range(3)]
     need = [core.spion_attn_scratch(handle, d_off.data_ptr(), d_col.data_ptr(), nnz, back) for back in (0, 1)]
-    assert need[0] > 0 and need[1] >= B * H * nnz
+    assert need[0] > 0 and need[1] >= B * H * nnz and core.spion_debug_counter(handle, 3) == 1
     scratch = torch.empty(max(need), device="cuda")
 
     def plain():
@@ -215,6 +217,7 @@ def test_calls_share_nothing_in_the_handle(kind, views):
         return out.detach(), p.detach(), q.grad, k.grad, v.grad
 
     want = [step(0), step(1)]
+    assert _lib.core().spion_debug_counter(handle, 3) == 1
     torch.cuda.synchronize()
     streams = [torch.cuda.Stream() for _ in range(2)]
     for s in streams:
@@ -228,4 +231,32 @@ def test_calls_share_nothing_in_the_handle(kind, views):
     for which in range(2):
         for results in got[which]:
             assert all(torch.equal(x, y) for x, y in zip(results, want[which]))
+    cpp.destroy(handle)
+
+
+# long patterns of few entries, few heads: gathered, whether mostly tiles or not; an empty remainder
+@pytest.mark.parametrize("B,L,kind", [(4, 4096, "scattered"), (1, 8192, "scattered"), (4, 4096, "window"), (64, 1024, "tiles")])
+def test_patterns_that_are_gathered(B, L, kind):
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    i = torch.arange(L, device="cuda")
+    if kind == "tiles":  # whole tiles but for one entry of each
+        pattern = ((i[:, None] // 32 - i[None, :] // 32).abs() <= 1).float()
+        pattern[::32, ::32] = 0.0
+    else:
+        pattern = (torch.rand(L, L, generator=gen, device="cuda") < 16 / L).float()
+        if kind == "window":
+            pattern[(i[:, None] - i[None, :]).abs() <= 40] = 1.0
+    q, k, v, do = (torch.randn(B, 1, L, 32, generator=gen, device="cuda") for _ in range(4))
+    q, k, v = (t.requires_grad_() for t in (q, k, v))
+    cpp, handle, module = _module(B, 1, L, False)
+    out, p = module(q, k, v, torch.ones(B, L, device="cuda"), pattern)
+    out.backward(do)
+    core = _lib.core()
+    assert core.spion_debug_counter(handle, 3) == 0 and core.spion_last_path(handle) == (2 if kind == "scattered" else 3)
+    at = lambda t: t.detach()[B - 1]
+    ref = _reference(at(q), at(k), at(v), at(do), pattern.double()[None], None)
+    got = (p.detach().reshape(B, -1)[B - 1],) + tuple(at(t) for t in (out, q.grad, k.grad, v.grad))
+    for name, x, y in zip(("P", "out", "dQ", "dK", "dV"), got, (ref[0][0][pattern.bool()],) + ref[1:]):
+        tol = 2e-5 * (y.abs() + y.pow(2).mean().sqrt())
+        assert float(((x.double() - y).abs() / tol).max()) <= 1.0, name
     cpp.destroy(handle)
