@@ -725,9 +725,9 @@ static RemRounds rem_rounds(int NB, int L, int cus) {
 // gathers: 64 heads of 4096, r = 16: 354 / 403, 128: 956 / 1382; 16 of 1024, 8: 42 / 35; 64 of 1024, 16: 71 / 97; 4 of 4096, 16: 92 / 36;
 // 8 of 8192, 16: 188 / 148, 300: 493 / 715; 1 of 16384, 16: 300 / 43; 4 of 32768, 16: 895 / 532, 300: 1565 / 2458.  It also bounds the
 // lists' offsets, L / 512 for every row and column, to a few tens and a fraction of the entries.  A list's word holds the position in a row
-// of the pattern in 18 bits.
+// of the pattern in 18 bits, and the kernels find the pairs {dS, P} of an entry by a signed 32-bit byte offset.
 static bool rem_by_ranges(int NB, int L, long long nr, int cus) {
-    if (L < REM_RANGE || L > (1 << 18) || nr <= 0) return false;
+    if (L < REM_RANGE || L > (1 << 18) || nr <= 0 || nr >= (1 << 28)) return false;
     const double ranges = (L + REM_RANGE - 1) / REM_RANGE, r = (double)nr / L;
     return 10 + rem_rounds(NB, L, cus).rounds * (11 * ranges + 0.8 * r) < (double)NB * L / (256.0 * cus) * (115 + 2.2 * r);
 }

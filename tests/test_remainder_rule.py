@@ -34,5 +34,7 @@ def test_limits():
     core = _lib.core()
     assert _by_ranges(64, 480, 16) == 0 and _by_ranges(64, (1 << 18) + 32, 4096) == 0
     assert core.spion_debug_remainder_by_ranges(64, 4096, 0, 256) == 0  # an empty remainder
+    # {dS, P} of an entry are found by a signed 32-bit byte offset, 8 bytes an entry
+    assert [core.spion_debug_remainder_by_ranges(16, 32768, n, 256) for n in ((1 << 28) - 1, 1 << 28, (1 << 29) - 1)] == [1, 0, 0]
     for bad in ((0, 4096, 1, 256), (64, 0, 1, 256), (64, 4096, 1, 0)):
         assert core.spion_debug_remainder_by_ranges(*bad) == -1
