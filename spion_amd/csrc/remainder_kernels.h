@@ -358,6 +358,7 @@ __global__ __launch_bounds__(REM_THREADS) void rem_bwd_row_kernel(
     f32x4 acc[NO][2], go[NO][2];
     float g0[NO];
     int pbase[NO];
+    int entries[NO];  // 0: the row has none
 #pragma unroll
     for (int c = 0; c < NO; ++c) {
         const int row = min(row0 + c * REM_QUADS, L - 1);
@@ -368,6 +369,7 @@ __global__ __launch_bounds__(REM_THREADS) void rem_bwd_row_kernel(
         }
         g0[c] = qi == 0 ? G[(size_t)bh * L + row] : 0.f;  // one lane's sum starts from -g
         pbase[c] = offs[row];
+        entries[c] = 0;
     }
 
     int addr[4], first = 0, left = 0, cnt = 0;  // the present batch: LDS rows, first entry of the lane, entries from it on
@@ -438,6 +440,7 @@ __global__ __launch_bounds__(REM_THREADS) void rem_bwd_row_kernel(
             bool more;
             do {
                 take();
+                entries[c] = max(entries[c], cnt);
                 more = __any(cnt > REM_BATCH);  // a row with more entries in the range: the rest of it is the next batch
                 if (more) span.x += REM_BATCH;
                 else span = ahead;
@@ -455,7 +458,9 @@ __global__ __launch_bounds__(REM_THREADS) void rem_bwd_row_kernel(
 #pragma unroll
     for (int c = 0; c < NO; ++c) {
         const int row = row0 + c * REM_QUADS;
-        if (row >= L) continue;
+        // Slots without an entry are walked with the row's dO and g: where these are not finite, a row of no entries at all has
+        // NaN for a sum.  (Clearing the product of every such slot instead took 34 us of the launch at the shape above.)
+        if (row >= L || !entries[c]) continue;
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             f32x4* o = reinterpret_cast<f32x4*>(dQ + gb + (size_t)row * gld) + (k ^ j) * 4 + qi;

@@ -108,6 +108,30 @@ def test_infinities_stay_in_their_rows():
     cpp.destroy(handle)
 
 
+@pytest.mark.parametrize("kind", ["window", "scattered"])
+def test_rows_without_entries_take_nothing_from_infinities(kind):
+    """A row of the pattern without entries: its gradient of Q stays zero whatever its dO (and dO . O) is."""
+    B, H, L = 16, 2, 1024
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    pattern = _pattern(L, gen) if kind == "window" else _scattered(L, gen)
+    empty = (pattern.sum(1) == 0).nonzero()[:, 0].tolist()
+    assert empty
+    if kind == "window":  # neither do the block row's dense tiles hold the row
+        for i in empty:
+            pattern[i // 32 * 32: i // 32 * 32 + 32] *= (torch.rand(32, L, generator=gen, device="cuda") < 0.1).float()
+    q, k, v, do = (torch.randn(B, H, L, 32, generator=gen, device="cuda") for _ in range(4))
+    do[..., empty, 5] = float("inf")
+    q, k, v = (t.requires_grad_() for t in (q, k, v))
+    cpp, handle, module = _module(B, H, L, False)
+    out, p = module(q, k, v, torch.ones(B, L, device="cuda"), pattern)
+    out.backward(do)
+    assert _lib.core().spion_debug_counter(handle, 3) == 1
+    assert (out[..., empty, :] == 0).all() and (q.grad[..., empty, :] == 0).all()
+    for t in (out, q.grad, k.grad, v.grad):
+        assert torch.isfinite(t).all()
+    cpp.destroy(handle)
+
+
 def _scattered(L, gen, share=0.05):
     """A pattern without dense structure, a long row and an empty one."""
     pattern = (torch.rand(L, L, generator=gen, device="cuda") < share).float()
