@@ -153,6 +153,53 @@ __device__ __forceinline__ void hyb_mma_add(const float (&w)[16], const float (&
     acc[0] += part[0];
 }
 
+// A matrix product multiplies what a tile lacks by zero: an infinity or NaN of one row or column of an operand reaches all of the
+// tile, while an entry of the pattern should take it to its own row and column only.  The kernels look at their sums at the end
+// (sixteen instructions a strip) and form those that are not finite again, entry by entry.
+__device__ __forceinline__ bool hyb_not_finite(const f32x16& acc) {
+    float s = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s = fmaf(acc[r], 0.f, s);
+    return __any(s != s);
+}
+// What the wavefront itself (or an earlier kernel) stored: past the caches of the CU.
+__device__ __forceinline__ float hyb_stored(const float* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The sum over a half-wave, in all of its lanes.
+__device__ __forceinline__ float hyb_half_sum(float x) {
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    return x;
+}
+// Rows of a strip from the entries of n tiles: sums of weight(row of the strip, column, position in P) X[column], a half-wave to a
+// row and a lane to a feature, back in the layout of the accumulators.  tile(u): the u-th tile; T: the wavefront's own LDS.
+template <class Tile, class Weight>
+__device__ __forceinline__ void hyb_rows_by_entries(float* T, int l, int n, const HybIndex& ix, const float* __restrict__ X, int ld,
+                                                    Tile tile, Weight weight, f32x16& acc) {
+    const int h = l >> 5, li = l & 31;
+#pragma unroll 1
+    for (int rr = 0; rr < 16; ++rr) {
+        const int row = 2 * rr + h;
+        const auto entry_weight = weight(row);
+        float s = 0.f;
+#pragma unroll 1
+        for (int u = 0; u < n; ++u) {
+            const int t = tile(u), col0 = ix.t_col[t] * 32;
+            int pos = ix.t_pos[(size_t)t * 32 + row];
+            unsigned bits = ix.t_bits[(size_t)t * 32 + row];
+            while (bits) {
+                const int col = col0 + __builtin_ctz(bits);
+                bits &= bits - 1;
+                s = fmaf(entry_weight(col, pos++), X[(size_t)col * ld + li], s);
+            }
+        }
+        T[row * TS + li] = s;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = T[acc_row(r, h) * TS + li];
+}
+
 // Two-deep software pipeline over n tiles with two register sets: while tile i is computed, the operands and P of
 // tile i + 1 are in flight and so is the index of tile i + 2 (requested first, so that waiting for it leaves the
 // younger requests outstanding).  Positions past the end are clamped by the callers (valid, redundant requests).
@@ -418,6 +465,12 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
         }
         __builtin_amdgcn_sched_barrier(0);
     }
+    if (hyb_not_finite(o[0])) {
+        __threadfence();  // P of these tiles, just stored
+        hyb_rows_by_entries(
+            T, l, nu, ix, V + ib, ild, [&](int u) { return t0 + w + u * WAVES; },
+            [&](int) { return [&](int, int pos) { return hyb_stored(Ph + pos); }; }, o[0]);
+    }
     float add[16];
     if constexpr (REM) {
         const float share = __builtin_amdgcn_exp2f(rem.x - Mx) * zinv;  // of the remainder's own sums
@@ -554,6 +607,16 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_row_kernel(const float* __restrict__ K
             for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
             hyb_mma_add(ds, kb, acc);
         });
+    if (hyb_not_finite(acc[0]))
+        hyb_rows_by_entries(
+            T, l, n, ix, K + ib, ild, [&](int u) { return t0 + w + u * WAVES; },
+            [&](int row) {
+                const float go_i = dO[ob + (size_t)(I * 32 + row) * old_ + li], g_i = __shfl(g, row, 64);
+                return [=](int col, int pos) {
+                    return (hyb_half_sum(go_i * V[ib + (size_t)col * ild + li]) - g_i) * P[(size_t)bh * nnz + pos];
+                };
+            },
+            acc[0]);
     if constexpr (WAVES > 1) __syncthreads();
     hyb_reduce_store<WAVES>(acc[0], scale, dQ + gb, gld, I * 32, w, li, h, lds);
 }
@@ -698,6 +761,35 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_col_kernel(const float* __restrict__ Q
         const int l2 = second_walk(l);
         load_vt(vt, l2);
         walk(whole(vt), l2);
+    }
+    if (hyb_not_finite(ak[0]) || hyb_not_finite(av[0])) {
+#pragma unroll 1
+        for (int jj = 0; jj < 16; ++jj) {
+            const int j = 2 * jj + h;
+            const float v_j = V[ib + (size_t)(J * 32 + j) * ild + li];
+            float sk = 0.f, sv = 0.f;
+#pragma unroll 1
+            for (int u = 0; u < n; ++u) {
+                const int e = e0 + w + u * WAVES, t = ix.t_ct[e], row0 = ix.t_ci[e] * 32;
+#pragma unroll 1
+                for (int i = 0; i < 32; ++i) {
+                    const unsigned bits = ix.t_bits[(size_t)t * 32 + i];
+                    if (!((bits >> j) & 1u)) continue;
+                    const float p = P[(size_t)bh * nnz + ix.t_pos[(size_t)t * 32 + i] + __popc(bits & ((1u << j) - 1u))];
+                    const float go_i = dO[ob + (size_t)(row0 + i) * old_ + li];
+                    const float ds = (hyb_half_sum(go_i * v_j) + G[(size_t)bh * L + row0 + i]) * p;
+                    sk = fmaf(ds, Q[ib + (size_t)(row0 + i) * ild + li], sk);
+                    sv = fmaf(p, go_i, sv);
+                }
+            }
+            Tq[j * TS + li] = sk;
+            To[j * TS + li] = sv;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            ak[0][r] = Tq[acc_row(r, h) * TS + li];
+            av[0][r] = To[acc_row(r, h) * TS + li];
+        }
     }
     if constexpr (WAVES > 1) __syncthreads();
     hyb_reduce_store<WAVES>(ak[0], scale, dK + gb, gld, J * 32, w, li, h, lds);

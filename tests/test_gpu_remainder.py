@@ -132,6 +132,71 @@ def test_rows_without_entries_take_nothing_from_infinities(kind):
     cpp.destroy(handle)
 
 
+def _holed(L, half, gen):
+    """A window of the given half width that lacks a fifth of its entries, and random columns; half 0: whole and holed tiles that
+    hold less than half of the entries."""
+    i = torch.arange(L, device="cuda")
+    pattern = (torch.rand(L, L, generator=gen, device="cuda") < (0.02 if half else 0.06)).float()
+    holes = (torch.rand(L, L, generator=gen, device="cuda") < 0.8).float()
+    if half:
+        near = (i[:, None] - i[None, :]).abs() <= half
+        return torch.where(near, holes, pattern)
+    for n in range(0, L, 128):
+        pattern[n: n + 32, n: n + 32] = holes[n: n + 32, n: n + 32] if n % 256 else 1.0
+        pattern[n: n + 32, (n + 512) % L: (n + 512) % L + 32] = 1.0
+    return pattern
+
+
+# tiles of one and of four wavefronts a strip; the remainder by ranges and gathered
+@pytest.mark.parametrize("half,B,masked", [(0, 16, False), (40, 16, False), (40, 16, True), (100, 16, False), (230, 16, False), (40, 1, False),
+                                           (230, 1, True)])
+def test_infinities_stay_with_their_entries(half, B, masked):
+    """An infinity or NaN of a row or column reaches the rows and columns it has an entry with and no other, also where a well-filled
+    tile lacks the entry."""
+    H, L = 2, 1024
+    gen = torch.Generator(device="cuda").manual_seed(9 + half)
+    pattern = _holed(L, half, gen)
+    row, col = 128 + 11, 128 + 7
+    heads = [torch.randn(B, H, L, 32, generator=gen, device="cuda") for _ in range(4)]
+    cpp, handle, module = _module(B, H, L, masked)
+    ones = torch.ones(B, L, device="cuda")
+    core = _lib.core()
+
+    def run(q, k, v, do):
+        q, k, v = (t.requires_grad_() for t in (q, k, v))
+        out, _ = module(q, k, v, ones, pattern)
+        out.backward(do)
+        assert core.spion_last_path(handle) == (3 if half else 2) and core.spion_debug_counter(handle, 3) == (B > 1)
+        return out.detach(), q.grad, k.grad, v.grad
+
+    clean = run(*(t.clone() for t in heads))
+
+    def step(which, at, feature):
+        """Which rows are finite.  They are those of the run without the infinity, to rounding."""
+        inputs = [t.clone() for t in heads]
+        inputs[which][..., at, feature] = float("nan" if which < 2 else "inf")  # (a logit of -inf is a probability of 0)
+        finite = []
+        for x, y in zip(run(*inputs), clean):
+            ok = torch.isfinite(x).all(-1)
+            # a few hundred terms of 2^-24 of a typical element each, in another order
+            assert ((x - y).abs() <= 2e-5 * (y.abs() + y.pow(2).mean().sqrt()))[ok].all()
+            finite.append(ok)
+        return finite
+
+    in_col, in_row, others = pattern[:, col] > 0, pattern[row] > 0, torch.arange(L, device="cuda") != row
+    same = lambda finite, reached: torch.equal(finite, (~reached).expand_as(finite))
+    for which in (1, 2):  # K, V: the rows that have the column
+        out, dq, dk, dv = step(which, col, 3)
+        reached = (pattern[in_col] > 0).any(0)  # dK and dV take {dS, P} of those rows
+        assert same(out, in_col) and same(dq, in_col) and same(dk, reached)
+        assert same(dv, reached if which == 1 else torch.zeros_like(reached))
+    for which in (0, 3):  # Q, dO: the row itself and the columns that it has
+        out, dq, dk, dv = step(which, row, 5)
+        assert same(out, ~others if which == 0 else torch.zeros_like(others)) and same(dq, ~others)
+        assert same(dk, in_row) and same(dv, in_row)
+    cpp.destroy(handle)
+
+
 def _scattered(L, gen, share=0.05):
     """A pattern without dense structure, a long row and an empty one."""
     pattern = (torch.rand(L, L, generator=gen, device="cuda") < share).float()
