@@ -643,9 +643,12 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
     //
     // Heads that eight does not divide: each die has NB / 8 heads to itself and an eighth of the work of the others, in the order of
     // the strips, so that it sees two of them at most.  (All of them dealt among all lanes, every die's L2 saw every head.  Steps in us,
-    // so / now: 83 of 5600, blocks of 32, 5 %, 480 / 329; 12 of 16384 266 / 226; 30 of 9952, d = 32, 220 / 184; 61 of 14080, d = 32, 697 / 615; 10 of
-    // 6144, up to two items a lane, 88 / 83, which dealt among all lanes longest first; so did forwards of 9 of 8192, 44.0 / 31.7, and of
-    // 20 of 4096, 28.6 / 25.0.)
+    // so / now: 83 of 5600, blocks of 32, 5 %, 480 / 329; 12 of 16384 266 / 226; 30 of 9952, d = 32, 220 / 184; 61 of 14080, d = 32, 697 / 615.)
+    // With up to two items a lane of these, a die's are dealt longest first instead, whatever they are: a lane has no order of heads to
+    // keep.  All lanes and heads longest first / by dies, chunks first / by dies, longest first, forward + backward kernels: 4 of 16384, 3.7 %,
+    // 121 / 124 / 120; 4 of 11712, d = 32, 8.3 %, 90 / 96 / 90; 3 of 16256, 6.3 %, 147 / 144 / 137; 9 of 8192 115 / 93 / 93; 10 of 6144 87 / 82 / 80;
+    // 30 of 2048 82 / 78 / 73; 45 of 3200 161 / 139 / 132; 36 of 3072, d = 32, 80.5 / 76.6 / 80.0 (blocks of 64); 1 of 16384 78 / 77 / 77.
+    const bool few = even == 1 && (long long)its.size() * NB <= 2LL * lanes;
     const int groups = lanes % 8 == 0 && lanes >= 64 ? 8 : even;  // dies
     const int per_group = lanes / groups, heads_per_group = NB / groups, whole_heads = heads_per_group * groups;
     std::vector<std::vector<std::pair<int, int>>> lane_list(lanes);  // {head, item}
@@ -679,6 +682,11 @@ static Bf16PlanHost build_bf16_plan(const std::vector<int>& ptr, int nstrips, bo
             top.first += weight(its[o]);
             heap.push(top);
         };
+        if (few) {
+            for (int o : order)
+                for (int head : heads) deal(head, o);
+            continue;
+        }
         for (int o : order)
             if (its[o].kind >= 0)
                 for (int head : heads) deal(head, o);

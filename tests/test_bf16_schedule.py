@@ -106,6 +106,27 @@ def test_schedule_walks_every_tile_once(kind, pairs, NB, lanes):
         assert mine.max() <= mine.mean() + w.max() + 1e-9
 
 
+@pytest.mark.parametrize("pairs", [False, True])
+@pytest.mark.parametrize("NB,nstrips", [(1, 256), (3, 64), (4, 128), (9, 64)])
+def test_few_items_are_dealt_longest_first(NB, nstrips, pairs):
+    """Numbers of heads that eight does not divide, at most an item a lane: the lanes of a die, which start in this order, have
+    its items by length, chunks of long strips among whole ones."""
+    rng = np.random.default_rng(NB + nstrips)
+    cnt = rng.integers(3, 30, nstrips)
+    cnt[0] = nstrips
+    if pairs:
+        cnt = np.repeat(cnt[::2], 2)
+    plan = _plan(np.concatenate([[0], np.cumsum(cnt)]), pairs, NB, 2048)
+    items, ents, lane_ptr = plan["items"], plan["ents"], plan["lane_ptr"]
+    assert len(plan["longs"]) and len(items) * NB <= 2 * plan["lanes"]
+    w = np.where(items[:, 3] == -2, 2, 1) * items[:, 2] + 2
+    for die in range(8):
+        load = [w[ents[lane_ptr[lane]: lane_ptr[lane + 1], 1]].sum() for lane in range(die, plan["lanes"], 8)]
+        used = np.count_nonzero(load)
+        assert used == len(set(map(tuple, np.concatenate([ents[lane_ptr[l]: lane_ptr[l + 1]] for l in range(die, plan["lanes"], 8)]))))
+        assert np.all(np.diff(load) <= 0)
+
+
 def test_schedule_rejects_bad_arguments():
     core = _lib.core()
     core.spion_debug_bf16_plan.restype = ctypes.c_int
