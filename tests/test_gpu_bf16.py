@@ -210,6 +210,27 @@ def test_bf16_with_key_mask(d):
     abi.close()
 
 
+# chunks of eight tiles: up to eight of them, one more, and both sides of every further sixteen
+@pytest.mark.parametrize("tiles", [64, 65, 72, 73, 128, 129, 192, 193, 320])
+@pytest.mark.parametrize("d", [32, 64])
+def test_bf16_global_row_of_many_chunks(tiles, d):
+    """One head: the strip of a global row is cut into tiles / 8 chunks, whose results the merge kernel combines."""
+    L = 32 * tiles
+    i = torch.arange(tiles)
+    mat = ((i[:, None] - i[None, :]).abs() <= 1).float()
+    mat[3] = 1.0
+    mod = BlockAttentionBF16(dict(head_dim=d, num_head=1, max_seq_len=L, batch_size=1, block_size=32))
+    q, k, v, _ = (t[:, None] for t in _bf16_inputs(1, L, d, seed=tiles))
+    q = q * torch.linspace(0.2, 4.0, L, device="cuda", dtype=torch.bfloat16)[:, None]  # chunks of unlike maxima
+    with torch.no_grad():
+        out, _ = mod(q, k, v, torch.ones(1, L, device="cuda"), mat.cuda())
+    rows = slice(96, 128)
+    logits = q[0, 0, rows].double() @ k[0, 0].double().t() / d ** 0.5
+    want = torch.softmax(logits, -1) @ v[0, 0].double()
+    assert_close_bf16(out[0, 0, rows].double().cpu().numpy(), want.cpu().numpy(), f"{tiles} tiles")
+    _lib.core().spion_block_bf16_destroy(mod.attn_handle)
+
+
 @pytest.mark.parametrize("d", [32, 64])
 def test_bf16_long_strips_with_key_mask_and_large_logits(d):
     """A global block row and column are cut into chunks whose partial results a merge kernel combines: the
