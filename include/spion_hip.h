@@ -445,7 +445,7 @@ void spion_block_bf16_attn_forward_strided_keys(void* handle, const void* Q, con
  * Each returns 0 on success. */
 int spion_project_forward(const float* X, const float* const* W, const float* const* b, float* Y, long long rows, int n,
                           int segs, int dim, void* stream);
-/* The same, and in the same launch what spion_key_penalty makes of a key mask. */
+/* The same, and then what spion_key_penalty makes of a key mask. */
 int spion_project_forward_keys(const float* X, const float* const* W, const float* const* b, float* Y, long long rows, int n,
                                int segs, int dim, const float* mask, float* penalty, int batch, int heads, int seq_len,
                                void* stream);

@@ -116,8 +116,9 @@ void dense_backward(void*, const float*, const float*, const float*, const float
                     float*);
 int dense_groups(void*);
 int pattern_generate(const float*, int, int, int, int, int, double, float*, float*, float*, hipStream_t);
-int project_forward(const float*, const float* const*, const float* const*, float*, long long, int, int, int, const float*, float*, int,
-                    int, int, hipStream_t);
+int project_forward(const float*, const float* const*, const float* const*, float*, long long, int, int, int, hipStream_t);
+int project_forward_keys(const float*, const float* const*, const float* const*, float*, long long, int, int, int, const float*, float*,
+                         int, int, int, hipStream_t);
 int project_backward_input(const float*, const float* const*, float*, long long, int, int, int, hipStream_t);
 long long project_workspace(long long, int, int);
 int project_backward_weight(const float*, const float*, float*, float*, float*, long long, int, int, hipStream_t);
@@ -267,7 +268,7 @@ void spion_densemask_destroy(void* h) { destroy_handle(h, KIND_DENSE); }
 int spion_project_forward(const float* X, const float* const* W, const float* const* b, float* Y, long long rows, int n,
                           int segs, int dim, void* stream) {
     note_current_handle(nullptr);
-    return project_forward(X, W, b, Y, rows, n, segs, dim, nullptr, nullptr, 0, 0, 0, static_cast<hipStream_t>(stream));
+    return project_forward(X, W, b, Y, rows, n, segs, dim, static_cast<hipStream_t>(stream));
 }
 int spion_project_forward_keys(const float* X, const float* const* W, const float* const* b, float* Y, long long rows, int n,
                                int segs, int dim, const float* mask, float* penalty, int batch, int heads, int seq_len,
@@ -277,7 +278,7 @@ int spion_project_forward_keys(const float* X, const float* const* W, const floa
         set_error("spion_project_forward_keys: null mask");
         return 1;
     }
-    return project_forward(X, W, b, Y, rows, n, segs, dim, mask, penalty, batch, heads, seq_len, static_cast<hipStream_t>(stream));
+    return project_forward_keys(X, W, b, Y, rows, n, segs, dim, mask, penalty, batch, heads, seq_len, static_cast<hipStream_t>(stream));
 }
 int spion_project_backward_input(const float* dY, const float* const* W, float* dX, long long rows, int n, int segs, int dim,
                                  void* stream) {

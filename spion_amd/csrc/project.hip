@@ -141,24 +141,6 @@ struct OperandLds {
 // the work-groups of the first column of tiles also leave sum_r A[r][m] in Csum[z][m].
 // A wavefront whose sums are not finite, or all too small for split operands (Split3, tile_ops.h), forms them again from
 // the operands in memory, one fp32 term after the other: some 30 us at 256 terms, and rare.
-// Forward: work-groups past the last item turn a key mask into penalties, which an attention layer needs right after its
-// projections (KeyMask::total 0: none).  us, projections of two heads of d = 32 alone / penalties in their launch / in one of
-// their own: one sample of 2048 tokens 4.9 / 4.9 / 7.7, 32 of 1024 12.4 / 12.4 / 14.9, 64 of 2048 39.2 / 39.4 / 40.6, 64 of 4096 74.6 / 79.5 /
-// 79.2, 256 of 1024 74.0 / 77.3 / 79.7; 16 heads of d = 64, 8 samples of 4096 1370 / 1370 / 1376.
-struct KeyMask {
-    const float* mask;
-    float* pen;
-    long long L, total;
-    int H, groups;
-};
-// [B][L] key mask (1 valid, 0 padded) -> [B*H][L] additive penalties 1e6 (1 - mask), one copy per head
-// (models/attention_blockcuda_mask.py:42-43): the elements of work-group g of `groups`.
-__device__ __forceinline__ void key_penalties(const KeyMask& k, int g) {
-    for (long long i = (long long)g * 256 + threadIdx.x; i < k.total; i += (long long)k.groups * 256) {
-        const long long bh = i / k.L;
-        k.pen[i] = 1e6f * (1.0f - k.mask[bh / k.H * k.L + (i - bh * k.L)]);
-    }
-}
 struct Product {
     SegRows A, B;
     SegBias bias;
@@ -333,17 +315,9 @@ __device__ __forceinline__ void project_item(const Product& y, int item, char* s
 }
 // consecutive items share the rows of A (the larger operand) and run on one die
 template <bool A_ACROSS, bool B_ACROSS, int WM, int WN, bool COLSUM>
-__global__ __launch_bounds__(256, 2) void project_kernel(Product y, KeyMask keys) {
+__global__ __launch_bounds__(256, 2) void project_kernel(Product y) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    int items = gridDim.x;
-    if constexpr (!A_ACROSS && !B_ACROSS) {
-        items -= keys.groups;
-        if ((int)blockIdx.x >= items) {
-            key_penalties(keys, blockIdx.x - items);
-            return;
-        }
-    }
-    project_item<A_ACROSS, B_ACROSS, WM, WN, COLSUM>(y, xcd_remap(blockIdx.x, items), smem);
+    project_item<A_ACROSS, B_ACROSS, WM, WN, COLSUM>(y, xcd_remap(blockIdx.x, gridDim.x), smem);
 }
 // Both products of a backward, which read the same dY, in one launch: the pieces of dW (and db) first, whose work-groups live
 // longest, then the tiles of dX, which fill what those leave idle.  By themselves both wait for memory most of their time (3.3
@@ -388,7 +362,7 @@ static Product product(const SegRows& A, const SegRows& B, const SegBias& bias, 
 }
 template <bool AA, bool BA, int WM, int WN, bool CS>
 static bool launch_project(const SegRows& A, const SegRows& B, const SegBias& bias, float* C, int ldc, float* Csum, int M,
-                           int N, int R, int pieces, int chunks, hipStream_t stream, const KeyMask& keys = KeyMask{}) {
+                           int N, int R, int pieces, int chunks, hipStream_t stream) {
     constexpr int lds = OperandLds<AA, WM>::BYTES + OperandLds<BA, WN>::BYTES;
     if (lds > 64 * 1024) {  // beyond what a launch may ask for without saying so first
         static const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(project_kernel<AA, BA, WM, WN, CS>),
@@ -396,8 +370,8 @@ static bool launch_project(const SegRows& A, const SegRows& B, const SegBias& bi
         if (!SPION_HIP_OK(err)) return false;
     }
     const Product y = product<WM, WN>(A, B, bias, C, ldc, Csum, M, N, R, chunks);
-    hipLaunchKernelGGL((project_kernel<AA, BA, WM, WN, CS>), dim3((unsigned)y.mtiles * y.ntiles * pieces + keys.groups), dim3(256),
-                       lds, stream, y, keys);
+    hipLaunchKernelGGL((project_kernel<AA, BA, WM, WN, CS>), dim3((unsigned)y.mtiles * y.ntiles * pieces), dim3(256), lds, stream,
+                       y);
     return check_launch("project_kernel");
 }
 
@@ -421,24 +395,8 @@ static SegRows weight_rows(const float* const* W, int segs, int n, int K) {
     return SegRows{{W[0], W[segs > 1 ? 1 : 0], W[segs > 2 ? 2 : 0]}, segs > 1 ? n : ONE_PIECE, K};
 }
 
-static bool key_mask(const char* who, const float* mask, float* pen, int B, int H, int L, KeyMask& keys) {
-    if (!mask || !pen || B <= 0 || H <= 0 || L <= 0) {
-        set_error("%s: bad arguments", who);
-        return false;
-    }
-    keys.mask = mask;
-    keys.pen = pen;
-    keys.L = L;
-    keys.total = (long long)B * H * L;
-    keys.H = H;
-    keys.groups = (int)std::min<long long>((keys.total + 255) / 256, 2048);
-    return true;
-}
-
 int project_forward(const float* X, const float* const* W, const float* const* b, float* Y, long long M, int n, int segs,
-                    int K, const float* mask, float* pen, int B, int H, int L, hipStream_t stream) {
-    KeyMask keys{};
-    if (mask && !key_mask("spion_project_forward_keys", mask, pen, B, H, L, keys)) return 1;
+                    int K, hipStream_t stream) {
     if (!W || !b || !project_args("spion_project_forward", M, n, segs, K, {X, Y})) {
         if (!W || !b) set_error("spion_project_forward: null weights");
         return 1;
@@ -448,8 +406,8 @@ int project_forward(const float* X, const float* const* W, const float* const* b
     const SegBias bias{{b[0], b[segs > 1 ? 1 : 0], b[segs > 2 ? 2 : 0]}, segs > 1 ? n : ONE_PIECE};
     const int N = segs * n;
     const bool ok = wide_tiles(M, N)
-        ? launch_project<false, false, 2, 2, false>(plain_rows(X, K), weight_rows(W, segs, n, K), bias, Y, N, nullptr, (int)M, N, K, 1, K / 32, stream, keys)
-        : launch_project<false, false, 1, 1, false>(plain_rows(X, K), weight_rows(W, segs, n, K), bias, Y, N, nullptr, (int)M, N, K, 1, K / 32, stream, keys);
+        ? launch_project<false, false, 2, 2, false>(plain_rows(X, K), weight_rows(W, segs, n, K), bias, Y, N, nullptr, (int)M, N, K, 1, K / 32, stream)
+        : launch_project<false, false, 1, 1, false>(plain_rows(X, K), weight_rows(W, segs, n, K), bias, Y, N, nullptr, (int)M, N, K, 1, K / 32, stream);
     return ok ? 0 : 1;
 }
 
@@ -532,12 +490,31 @@ int project_backward(const float* dY, const float* const* W, const float* X, flo
     return check_launch("project_backward_kernel") && add_pieces(ws, dW, db, N, K, pieces, stream) ? 0 : 1;
 }
 
-__global__ __launch_bounds__(256) void key_penalty_kernel(KeyMask keys) { key_penalties(keys, blockIdx.x); }
+// [B][L] key mask (1 valid, 0 padded) -> [B*H][L] additive penalties 1e6 (1 - mask), one copy per head
+// (models/attention_blockcuda_mask.py:42-43).
+__global__ __launch_bounds__(256) void key_penalty_kernel(const float* __restrict__ mask, float* __restrict__ pen, long long total,
+                                                          long long L, int H) {
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {
+        const long long bh = i / L;
+        pen[i] = 1e6f * (1.0f - mask[bh / H * L + (i - bh * L)]);
+    }
+}
+static bool key_mask_args(const char* who, const float* mask, const float* pen, int B, int H, int L) {
+    if (mask && pen && B > 0 && H > 0 && L > 0) return true;
+    set_error("%s: bad arguments", who);
+    return false;
+}
 int key_penalty(const float* mask, float* pen, int B, int H, int L, hipStream_t stream) {
-    KeyMask keys;
-    if (!key_mask("spion_key_penalty", mask, pen, B, H, L, keys)) return 1;
-    hipLaunchKernelGGL(key_penalty_kernel, dim3(keys.groups), dim3(256), 0, stream, keys);
+    if (!key_mask_args("spion_key_penalty", mask, pen, B, H, L)) return 1;
+    const long long total = (long long)B * H * L;
+    hipLaunchKernelGGL(key_penalty_kernel, dim3((unsigned)std::min<long long>((total + 255) / 256, 2048)), dim3(256), 0, stream, mask,
+                       pen, total, (long long)L, H);
     return check_launch("key_penalty_kernel") ? 0 : 1;
+}
+int project_forward_keys(const float* X, const float* const* W, const float* const* b, float* Y, long long M, int n, int segs, int K,
+                         const float* mask, float* pen, int B, int H, int L, hipStream_t stream) {
+    if (!key_mask_args("spion_project_forward_keys", mask, pen, B, H, L)) return 1;
+    return project_forward(X, W, b, Y, M, n, segs, K, stream) || key_penalty(mask, pen, B, H, L, stream) ? 1 : 0;
 }
 
 }  // namespace spion
