@@ -43,9 +43,9 @@ def _module(B, H, L, masked):
     return cpp, handle, cls(cfg, cpp, handle)
 
 
-# one range; a second one of 32 rows; work-groups of 256 rows whose last is partial; work-groups of 512, the last partial
+# one range; a second one of 32 rows; work-groups of 256 rows whose last is partial; work-groups of 512, the last partial; nine ranges
 @pytest.mark.parametrize("B,H,L,masked", [(32, 2, 512, False), (24, 2, 544, True), (14, 2, 1056, False), (35, 2, 1056, True),
-                                          (35, 2, 1056, False), (32, 2, 2048, False)])
+                                          (35, 2, 1056, False), (32, 2, 2048, False), (24, 2, 4128, True)])
 @pytest.mark.parametrize("views", [False, True])
 def test_ranges_and_batches(B, H, L, masked, views):
     gen = torch.Generator(device="cuda").manual_seed(L + B)
@@ -72,16 +72,18 @@ def test_ranges_and_batches(B, H, L, masked, views):
         for name, x, y in zip(("P", "out", "dQ", "dK", "dV"), got, (ref[0][0][where],) + ref[1:]):
             if x is None:
                 continue
-            # a few hundred terms each: 2^-24 of a typical element per rounding, with a wide margin
-            tol = 2e-5 * (y.abs() + y.pow(2).mean().sqrt())
-            worst = float(((x.double() - y).abs() / tol).max())
-            assert worst <= 1.0, f"{name}, head {(b, h)}: {worst}"
+            # A hundred to some thousand terms each, of unlike signs: their roundings, 2^-24 each, add up as the terms do, to a few
+            # 2^-24 of a typical element (2.3e-7 seen), ten times that for the furthest of 30,000 to 400,000 (2.6e-6 seen).
+            diff, typical = x.double() - y, y.pow(2).mean().sqrt()
+            assert float(diff.pow(2).mean().sqrt() / typical) <= 1e-6, f"{name}, head {(b, h)}"
+            worst = float((diff.abs() / (y.abs() + typical)).max())
+            assert worst <= 1e-5, f"{name}, head {(b, h)}: {worst}"
     cpp.destroy(handle)
 
 
 def test_infinities_stay_in_their_rows():
-    """The slots of a batch that hold no entry read a row of zeros: an infinity reaches the rows that have its column (or whose
-    dense tiles do) and no other."""
+    """The slots of a batch that hold no entry read a row of zeros, and tiles are taken by their entries: an infinity reaches the
+    rows that have its column and no other."""
     B, H, L, far = 16, 2, 1024, 900
     gen = torch.Generator(device="cuda").manual_seed(1)
     pattern = _pattern(L, gen)
@@ -93,18 +95,12 @@ def test_infinities_stay_in_their_rows():
     out.backward(do)
     assert _lib.core().spion_last_path(handle) == 3
     assert _lib.core().spion_debug_counter(handle, 3) == 1
-    i = torch.arange(L, device="cuda")
-    near = (i - far).abs() < 128  # the window's tiles
-    reads_v = near | (pattern[:, far] > 0)
-    assert torch.isfinite(out[..., ~reads_v, :]).all() and torch.isfinite(q.grad[..., ~reads_v, :]).all()
-    assert not torch.isfinite(out[..., pattern[:, far] > 0, 3]).any()
-    reads_q = near | (pattern[far] > 0)
-    # dK and dV also take {dS, P} of rows whose own results are not finite
-    bad_rows = (pattern[reads_v] > 0).any(0)
-    clean = ~(reads_q | bad_rows)
-    if clean.any():
-        assert torch.isfinite(k.grad[..., clean, :]).all()
-    assert torch.isfinite(v.grad[..., ~reads_q & ~near, :]).all()
+    # Q of row far: that row; V: the rows that have the column; dO of row far: as Q.  dK takes {dS, P} of all of them, dV those of row far
+    bad_rows = pattern[:, far] > 0
+    bad_rows[far] = True
+    exactly = lambda t, reached: torch.equal(torch.isfinite(t).all(-1), (~reached).expand(B, H, L))
+    assert exactly(out, bad_rows) and exactly(q.grad, bad_rows)
+    assert exactly(k.grad, (pattern[bad_rows] > 0).any(0)) and exactly(v.grad, pattern[far] > 0)
     cpp.destroy(handle)
 
 
@@ -179,7 +175,7 @@ def test_infinities_stay_with_their_entries(half, B, masked):
         for x, y in zip(run(*inputs), clean):
             ok = torch.isfinite(x).all(-1)
             # a few hundred terms of 2^-24 of a typical element each, in another order
-            assert ((x - y).abs() <= 2e-5 * (y.abs() + y.pow(2).mean().sqrt()))[ok].all()
+            assert ((x - y).abs() <= 1e-5 * (y.abs() + y.pow(2).mean().sqrt()))[ok].all()
             finite.append(ok)
         return finite
 
@@ -280,7 +276,7 @@ def test_scattered_patterns_and_capture():
     for got in eager:
         got = (got[1][(B // 2) * H + 1],) + tuple(at(got[i]) for i in (0, 2, 3, 4))
         for name, x, y in zip(("P", "out", "dQ", "dK", "dV"), got, (ref[0][0][where],) + ref[1:]):
-            tol = 2e-5 * (y.abs() + y.pow(2).mean().sqrt())
+            tol = 1e-5 * (y.abs() + y.pow(2).mean().sqrt())
             assert float(((x.double() - y).abs() / tol).max()) <= 1.0, name
     core.spion_set_stream(handle, 0)
     cpp.destroy(handle)
@@ -346,6 +342,6 @@ def test_patterns_that_are_gathered(B, L, kind):
     ref = _reference(at(q), at(k), at(v), at(do), pattern.double()[None], None)
     got = (p.detach().reshape(B, -1)[B - 1],) + tuple(at(t) for t in (out, q.grad, k.grad, v.grad))
     for name, x, y in zip(("P", "out", "dQ", "dK", "dV"), got, (ref[0][0][pattern.bool()],) + ref[1:]):
-        tol = 2e-5 * (y.abs() + y.pow(2).mean().sqrt())
+        tol = 1e-5 * (y.abs() + y.pow(2).mean().sqrt())
         assert float(((x.double() - y).abs() / tol).max()) <= 1.0, name
     cpp.destroy(handle)
