@@ -758,15 +758,18 @@ def bench_sparse_layer(args, dev, workload, full=True):
                           idx.offsets.data_ptr(), idx.columns.data_ptr(), idx.sum_mat.data_ptr(), nnz)
 
     # what the module runs: every operand row-major, the forward's output handed to the backward
+    need = [core.spion_attn_scratch(handle, idx.offsets.data_ptr(), idx.columns.data_ptr(), nnz, back) for back in (0, 1)]
+    scratch = torch.empty(max(*need, 1), device=dev)
+
     def fwd_rm():
-        core.spion_attn_forward_rowmajor(handle, Q.data_ptr(), K.data_ptr(), V.data_ptr(),
-                                         pen.data_ptr() if with_mask else None, P.data_ptr(), O.data_ptr(),
-                                         idx.offsets.data_ptr(), idx.columns.data_ptr(), idx.sum_mat.data_ptr(), nnz)
+        core.spion_attn_forward_scratch(handle, Q.data_ptr(), K.data_ptr(), V.data_ptr(), key_mask.data_ptr() if with_mask else None,
+                                        H if with_mask else 0, P.data_ptr(), O.data_ptr(), idx.offsets.data_ptr(),
+                                        idx.columns.data_ptr(), nnz, H, None, None, scratch.data_ptr(), need[0])
 
     def bwd_rm():
-        core.spion_attn_backward_rowmajor(handle, Q.data_ptr(), K.data_ptr(), V.data_ptr(), P.data_ptr(), O.data_ptr(),
-                                          dO.data_ptr(), dS.data_ptr(), dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(),
-                                          idx.offsets.data_ptr(), idx.columns.data_ptr(), idx.sum_mat.data_ptr(), nnz)
+        core.spion_attn_backward_scratch(handle, Q.data_ptr(), K.data_ptr(), V.data_ptr(), P.data_ptr(), O.data_ptr(), dO.data_ptr(),
+                                         dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(), idx.offsets.data_ptr(),
+                                         idx.columns.data_ptr(), nnz, H, None, None, None, scratch.data_ptr(), need[1])
 
     it = max(10, args.steps)
     # the reference's ABI (transposed K / V operands, no output in the backward: the library keeps copies)
@@ -850,10 +853,11 @@ def bench_sparse_layer(args, dev, workload, full=True):
         "config": {"workload": f"{wl['name']}: sparse attention fwd+bwd, B={B} H={H} L={L} d={d}, "
                                f"block {bs}, nnz/head={nnz}, block density="
                                f"{wl['block_density'] if wl['block_density'] is None else round(wl['block_density'], 4)}",
-                   "kernel_path": {1: "mfma-tile", 2: "element", 3: "hybrid (mfma tiles + gathered remainder)"}[path]},
+                   "kernel_path": {1: "mfma-tile", 2: "element",
+                                   3: f"hybrid (mfma tiles + remainder {'by ranges' if by_ranges else 'gathered'})"}[path]},
         "rowmajor_abi_ms": {"attn_forward": round(t_fwd, 4), "attn_backward": round(t_bwd, 4),
                             "fwd_plus_bwd": round(t_fwd + t_bwd, 4), "fwd_then_bwd_sequence": round(t_seq, 4),
-                            "what": "spion_attn_forward_rowmajor / spion_attn_backward_rowmajor, the entry points "
+                            "what": "spion_attn_forward_scratch / spion_attn_backward_scratch, the entry points "
                                     "the module calls; kernel_ms are these kernels"},
         "abi_ms": {"attn_forward": round(t_fwd_abi, 4), "attn_backward": round(t_bwd_abi, 4),
                    "fwd_plus_bwd": round(t_fwd_abi + t_bwd_abi, 4), "fwd_then_bwd_sequence": round(t_seq_abi, 4),
