@@ -175,8 +175,9 @@ __device__ __forceinline__ float hyb_half_sum(float x) {
 // Rows of a strip from the entries of n tiles: sums of weight(row of the strip, column, position in P) X[column], a half-wave to a
 // row and a lane to a feature, back in the layout of the accumulators.  tile(u): the u-th tile; T: the wavefront's own LDS.
 template <class Tile, class Weight>
-__device__ __forceinline__ void hyb_rows_by_entries(float* T, int l, int n, const HybIndex& ix, const float* __restrict__ X, int ld,
-                                                    Tile tile, Weight weight, f32x16& acc) {
+__device__ __forceinline__ void hyb_rows_by_entries(float* T, int l, int n, const HybIndex& ix, rsrc_t X, int ld, Tile tile,
+                                                    Weight weight, f32x16& acc) {
+    l = second_walk(l);
     const int h = l >> 5, li = l & 31;
 #pragma unroll 1
     for (int rr = 0; rr < 16; ++rr) {
@@ -191,7 +192,7 @@ __device__ __forceinline__ void hyb_rows_by_entries(float* T, int l, int n, cons
             while (bits) {
                 const int col = col0 + __builtin_ctz(bits);
                 bits &= bits - 1;
-                s = fmaf(entry_weight(col, pos++), X[(size_t)col * ld + li], s);
+                s = fmaf(entry_weight(col, pos++), ld1(X, (col * ld + li) * 4, 0), s);
             }
         }
         T[row * TS + li] = s;
@@ -468,7 +469,7 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_fwd_kernel(const float* __restrict__ Q, co
     if (hyb_not_finite(o[0])) {
         __threadfence();  // P of these tiles, just stored
         hyb_rows_by_entries(
-            T, l, nu, ix, V + ib, ild, [&](int u) { return t0 + w + u * WAVES; },
+            T, l, nu, ix, rV, ild, [&](int u) { return t0 + w + u * WAVES; },
             [&](int) { return [&](int, int pos) { return hyb_stored(Ph + pos); }; }, o[0]);
     }
     float add[16];
@@ -609,11 +610,12 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_row_kernel(const float* __restrict__ K
         });
     if (hyb_not_finite(acc[0]))
         hyb_rows_by_entries(
-            T, l, n, ix, K + ib, ild, [&](int u) { return t0 + w + u * WAVES; },
+            T, l, n, ix, rK, ild, [&](int u) { return t0 + w + u * WAVES; },
             [&](int row) {
-                const float go_i = dO[ob + (size_t)(I * 32 + row) * old_ + li], g_i = __shfl(g, row, 64);
+                const int at = ((I * 32 + row) * old_ + li) * 4;
+                const float go_i = ld1(rdO, at, 0), g_i = hyb_half_sum(go_i * ld1(rO, at, 0));
                 return [=](int col, int pos) {
-                    return (hyb_half_sum(go_i * V[ib + (size_t)col * ild + li]) - g_i) * P[(size_t)bh * nnz + pos];
+                    return (hyb_half_sum(go_i * ld1(rV, (col * ild + li) * 4, 0)) - g_i) * ld1(rP, pos * 4, 0);
                 };
             },
             acc[0]);
@@ -763,10 +765,11 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_col_kernel(const float* __restrict__ Q
         walk(whole(vt), l2);
     }
     if (hyb_not_finite(ak[0]) || hyb_not_finite(av[0])) {
+        const int l2 = second_walk(l), h = l2 >> 5, li = l2 & 31;
 #pragma unroll 1
         for (int jj = 0; jj < 16; ++jj) {
             const int j = 2 * jj + h;
-            const float v_j = V[ib + (size_t)(J * 32 + j) * ild + li];
+            const float v_j = ld1(rV, ((J * 32 + j) * ild + li) * 4, 0);
             float sk = 0.f, sv = 0.f;
 #pragma unroll 1
             for (int u = 0; u < n; ++u) {
@@ -775,10 +778,10 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_col_kernel(const float* __restrict__ Q
                 for (int i = 0; i < 32; ++i) {
                     const unsigned bits = ix.t_bits[(size_t)t * 32 + i];
                     if (!((bits >> j) & 1u)) continue;
-                    const float p = P[(size_t)bh * nnz + ix.t_pos[(size_t)t * 32 + i] + __popc(bits & ((1u << j) - 1u))];
-                    const float go_i = dO[ob + (size_t)(row0 + i) * old_ + li];
-                    const float ds = (hyb_half_sum(go_i * v_j) + G[(size_t)bh * L + row0 + i]) * p;
-                    sk = fmaf(ds, Q[ib + (size_t)(row0 + i) * ild + li], sk);
+                    const float p = ld1(rP, (ix.t_pos[(size_t)t * 32 + i] + __popc(bits & ((1u << j) - 1u))) * 4, 0);
+                    const float go_i = ld1(rdO, ((row0 + i) * old_ + li) * 4, 0);
+                    const float ds = (hyb_half_sum(go_i * v_j) + ld1(rG, (row0 + i) * 4, 0)) * p;
+                    sk = fmaf(ds, ld1(rQ, ((row0 + i) * ild + li) * 4, 0), sk);
                     sv = fmaf(p, go_i, sv);
                 }
             }
