@@ -1,7 +1,7 @@
 // Hybrid kernels for element-sparse patterns (d = 32): the well-filled aligned 32 x 32 tiles of the pattern (the
 // local window of a "window + random columns" pattern, say) run as dense MFMA tiles with a bit mask for the entries
-// that are absent, the remaining entries as per-row gathers; the softmax statistics are merged across the two
-// parts, and P stays in CSR order exactly as the reference's kernels leave it (models/block_attn_mask.cu:88-140):
+// that are absent, the remaining entries by ranges of rows in LDS (remainder_kernels.h) or as per-row gathers; the softmax
+// statistics are merged across the two parts, and P stays in CSR order exactly as the reference's kernels leave it (models/block_attn_mask.cu:88-140):
 // a tile's entries of one row are consecutive in that row's CSR run, so `first position + number of present
 // columns to the left` addresses them.
 //
@@ -10,10 +10,12 @@
 //
 // The two parts run as separate launches, each at the occupancy that suits it: the tile kernels (one wavefront per
 // strip of 32 rows or columns when strips hold few dense tiles, else a work-group of four wavefronts, wavefront w
-// taking the strip's dense tiles w, w+4, ...) and the gather kernels (one wavefront per row or column of the
-// remainder, sixteen wavefronts per CU, because the gathers are bound by the number of requests in flight).
-// Forward: remainder logits and their row statistics, then the tiles (which merge the statistics and fix the row's
-// maximum and denominator), then the remainder's probabilities and share of O.  Backward: tile part then remainder
+// taking the strip's dense tiles w, w+4, ...) and the remainder's: work-groups of sixteen wavefronts that walk ranges
+// of the sequence in LDS, or where that costs more (rem_by_ranges, sparse_attn.hip) gathers, one wavefront per row or column,
+// sixteen per CU, because they are bound by the number of requests in flight.
+// Forward: remainder logits and their row statistics (by ranges: the remainder's share of O as well), then the tiles (which
+// merge the statistics, fix the row's maximum and denominator and rescale and add that share), then the remainder's
+// probabilities (gathered: and its share of O).  Backward: tile part then remainder
 // part of the row pass, the same for the column pass; the remainder kernels add to what the tile kernels wrote
 // (each row or column has exactly one writer per launch).
 #pragma once

@@ -111,7 +111,7 @@ __device__ __forceinline__ rsrc_t rem_word_rsrc(const int* w, int nr) { return m
 // tiles'; rem_prob_kernel then makes the probabilities.
 // A batch's maximum first, then its exponentials, each by the lane that owns the entry; the sums of the batches before are
 // rescaled once a batch.  64 heads of 4096 rows with 76 entries: 139 us (logits) + 205 (P.V, probabilities) -> 174 + 75
-// (rem_prob_kernel); vector ALU 73 % busy.
+// (rem_prob_kernel); vector ALU 79 % busy.
 // -------------------------------------------------------------------------------------------------
 template <bool MASK, bool ST, int NO>
 __global__ __launch_bounds__(REM_THREADS) void rem_fwd_kernel(const float* __restrict__ Q, const float* __restrict__ K,
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(REM_PROB_THREADS) void rem_prob_kernel(const float*
 // -------------------------------------------------------------------------------------------------
 // Backward, row pass: dS = (dO_i . v_j - g_i) * P / sqrt(d), dQ_i += sum dS . K[col]; {dS, P} of every entry to Pairs
 // [NB][nr] in the order of the rb list, where the column pass reads them.
-// 64 heads of 4096 rows with 76 remainder entries each: 337 us (gathering from L2) -> 182; vector ALU 58 % busy, 590 MB of
+// 64 heads of 4096 rows with 76 remainder entries each: 337 us (gathering from L2) -> 180; vector ALU 65 % busy, 595 MB of
 // traffic (P's lines come once per range).
 // -------------------------------------------------------------------------------------------------
 template <bool ST, int NO>
@@ -471,8 +471,8 @@ __global__ __launch_bounds__(REM_THREADS) void rem_bwd_row_kernel(
 
 // -------------------------------------------------------------------------------------------------
 // Backward, column pass: dK_j += sum_i dS_ij Q_i, dV_j += sum_i P_ij dO_i from the {dS, P} pairs of the row pass (dS
-// already carries the 1/sqrt(d)).  As above: 236 us (eight lanes to a column, weights looked up in row order) -> 172; vector ALU
-// 63 % busy.  The look-ups in the pairs cost 30 of them: with the entries in plain row order, not by ranges, 55.
+// already carries the 1/sqrt(d)).  As above: 236 us (eight lanes to a column, weights looked up in row order) -> 171; vector ALU
+// 70 % busy.  The look-ups in the pairs cost 30 of them: with the entries in plain row order, not by ranges, 55.
 // -------------------------------------------------------------------------------------------------
 template <bool ST, int NO>
 __global__ __launch_bounds__(REM_THREADS) void rem_bwd_col_kernel(

@@ -6,9 +6,11 @@
 //                     cores, in fp32 or with operands split into three bf16 parts (tile_kernels.h); tiles go
 //                     from global memory into LDS or the MFMA register layout in whole 128-byte rows, the
 //                     tile list of a block row / block column is walked per wavefront.
-//   * element path -- any other CSR (element-sparse patterns, odd head sizes).  d = 32 and enough rows: well-filled
-//                     32x32 tiles of the pattern on the matrix cores (hybrid_kernels.h), the remainder by ranges
-//                     whose rows lie in LDS (remainder_kernels.h); else one wavefront per row gathers K/V rows.
+//   * element path -- any other CSR (element-sparse patterns, odd head sizes).  d = 32: well-filled 32x32
+//                     tiles of the pattern on the matrix cores (hybrid_kernels.h), the remainder by ranges whose rows
+//                     lie in LDS (remainder_kernels.h), where these are the faster way (rem_by_ranges) and, for patterns with
+//                     less than half of their entries in such tiles, the caller brings scratch; else one wavefront per row
+//                     gathers K/V rows.
 //                     A transposed index built on the host once per pattern makes dK/dV deterministic without
 //                     atomics.
 //
