@@ -114,14 +114,19 @@ def _address(layout):
 
 
 def _scratch(m, index, backward, device):
-    """Scratch of a call of the core: (tensor, pointer, floats)."""
+    """Scratch of a call of the core: (tensor, pointer, floats).  Where there is no memory for it, what the element kernels, or
+    the handle's workspaces, do with."""
     floats = _lib.core().spion_attn_scratch(m.attn_handle, *index.tail[:2], index.nnz, int(backward))
     if floats < 0:
         _lib.check_error("attn_backward" if backward else "attn_forward")
-    if floats <= 0:
-        return None, None, 0
-    t = torch.empty(floats, dtype=torch.float32, device=device)
-    return t, t.data_ptr(), floats
+    least = max(m.num_batches * index.nnz, 1) if backward else 0
+    try:
+        t = torch.empty(max(floats, 0), dtype=torch.float32, device=device)
+    except torch.cuda.OutOfMemoryError:
+        if floats <= least:
+            raise
+        t = torch.empty(least, dtype=torch.float32, device=device)
+    return (t, t.data_ptr(), t.numel()) if t.numel() else (None, None, 0)
 
 
 def _empty_heads(shape, interleaved, device):

@@ -159,11 +159,18 @@ struct CoreResult {
     bool strided = false;
 };
 
-// Scratch of a call of the core, of its stream as every tensor made here is.
-Tensor core_scratch(void* h, const Tensor& offsets, const Tensor& columns, int64_t nnz, bool backward, const torch::TensorOptions& opt) {
+// Scratch of a call of the core, of its stream as every tensor made here is.  Where there is no memory for it, the `least` floats
+// that the element kernels, or the handle's workspaces, do with.
+Tensor core_scratch(void* h, const Tensor& offsets, const Tensor& columns, int64_t nnz, bool backward, int64_t least,
+                    const torch::TensorOptions& opt) {
     const int64_t floats = spion_attn_scratch(h, ip(offsets), ip(columns), (int)nnz, backward);
     if (floats < 0) check_library(backward ? "attn_backward" : "attn_forward");
-    return floats > 0 ? torch::empty({floats}, opt) : Tensor();
+    if (floats <= least) return floats > 0 ? torch::empty({floats}, opt) : Tensor();
+    try {
+        return torch::empty({floats}, opt);
+    } catch (const c10::OutOfMemoryError&) {
+        return least > 0 ? torch::empty({least}, opt) : Tensor();
+    }
 }
 float* fps(Tensor& t) { return t.defined() ? fpm(t) : nullptr; }
 int64_t count(const Tensor& t) { return t.defined() ? t.numel() : 0; }
@@ -192,7 +199,7 @@ CoreResult core_forward(const Tensor& query, const Tensor& key, const Tensor& va
     const auto opt = query.options();
     CoreResult r;
     r.p_flat = torch::empty({B * H * nnz}, opt);
-    Tensor scratch = core_scratch(h, offsets, columns, nnz, false, opt);
+    Tensor scratch = core_scratch(h, offsets, columns, nnz, false, 0, opt);
     spion_head_layout lin{}, lout{}, lk{}, lv{};
     r.strided = reads_views && !(query.is_contiguous() && key.is_contiguous() && value.is_contiguous()) &&
                 head_layout(query, lin) && head_layout(key, lk) && head_layout(value, lv) && same_strides(key, query) &&
@@ -281,7 +288,7 @@ struct SparseAttnNode : public torch::autograd::Function<SparseAttnNode> {
             dv = torch::empty(q.sizes(), opt);
         }
         // (in place of the ABI's two [NB*nnz] scratch arguments, models/attention_blockcuda.py:83-84)
-        Tensor scratch = core_scratch(h, offsets, columns, nnz, true, opt);
+        Tensor scratch = core_scratch(h, offsets, columns, nnz, true, std::max<int64_t>(q.size(0) * q.size(1) * nnz, 1), opt);
         spion_attn_backward_scratch(h, fp(q), fp(k), fp(v), fp(p_flat), fp(out), fp(go), fpm(dq), fpm(dk), fpm(dv), ip(offsets),
                                     ip(columns), (int)nnz, heads, strided ? &lin : nullptr, strided ? &lout : nullptr,
                                     strided ? &lgrad : nullptr, fps(scratch), count(scratch));

@@ -319,6 +319,49 @@ def test_calls_share_nothing_in_the_handle(kind, views):
     cpp.destroy(handle)
 
 
+@pytest.mark.parametrize("node", [True, False])
+def test_no_memory_for_scratch(node, monkeypatch):
+    """What fits without the scratch still runs: the element kernels, in P and dS."""
+    B, H, L = 32, 2, 2048
+    if not node:
+        monkeypatch.setattr(_lib, "autograd_node", lambda: None)
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    pattern = _scattered(L, gen)
+    q, k, v, do = (torch.randn(B, H, L, 32, generator=gen, device="cuda") for _ in range(4))
+    q, k, v = (t.requires_grad_() for t in (q, k, v))
+    ones = torch.ones(B, L, device="cuda")
+    cpp, handle, module = _module(B, H, L, False)
+    core = _lib.core()
+
+    def step(limit):
+        """Forward and backward, with no more than 1.5 times P and the tensors beside the inputs in either."""
+        q.grad = k.grad = v.grad = None
+        with torch.no_grad():
+            p_bytes = 4 * B * H * int(pattern.sum())
+        for part in ("forward", "backward"):
+            torch.cuda.synchronize()
+            torch.cuda.empty_cache()
+            if limit:
+                room = torch.cuda.memory_reserved() + 1.5 * p_bytes + 4 * q.numel() * (1 if part == "forward" else 3)
+                torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(0).total_memory)
+            try:
+                if part == "forward":
+                    out, p = module(q, k, v, ones, pattern)
+                else:
+                    out.backward(do)
+            finally:
+                torch.cuda.set_per_process_memory_fraction(1.0)
+        return out.detach(), p.detach(), q.grad, k.grad, v.grad
+
+    want = step(False)
+    assert core.spion_debug_counter(handle, 3) == 1
+    got = step(True)
+    assert not torch.equal(got[0], want[0])  # other kernels, other roundings
+    for x, y in zip(got, want):
+        assert ((x - y).abs() <= 1e-5 * (y.abs() + y.pow(2).mean().sqrt())).all()
+    cpp.destroy(handle)
+
+
 # long patterns of few entries, few heads: gathered, whether mostly tiles or not; an empty remainder
 @pytest.mark.parametrize("B,L,kind", [(4, 4096, "scattered"), (1, 8192, "scattered"), (4, 4096, "window"), (64, 1024, "tiles")])
 def test_patterns_that_are_gathered(B, L, kind):
