@@ -483,9 +483,10 @@ def bench_dense_phase(args, dev, d=32):
         handle, Qr.data_ptr(), Kr.data_ptr(), Vr.data_ptr(), None, attn.data_ptr(), out_r.data_ptr(), H, A, A),
         max(10, args.steps // 4))
     _lib.check_error("dense forward (row-major)")
-    t_bwd_rm = _event_ms(lambda: core.spion_dense_backward_strided(
+    scratch = torch.empty(core.spion_dense_scratch(handle), device=dev)  # none: the two passes
+    t_bwd_rm = _event_ms(lambda: core.spion_dense_backward_scratch(
         handle, Qr.data_ptr(), Kr.data_ptr(), Vr.data_ptr(), attn.data_ptr(), out_r.data_ptr(), dOr.data_ptr(),
-        gq.data_ptr(), gk.data_ptr(), gv.data_ptr(), H, A, A, A), max(10, args.steps // 4))
+        gq.data_ptr(), gk.data_ptr(), gv.data_ptr(), H, A, A, A, scratch.data_ptr(), scratch.numel()), max(10, args.steps // 4))
     _lib.check_error("dense backward (row-major)")
     # the same forward leaving the mean of all maps as well (what pattern discovery reads)
     mean_map = torch.empty(L, L, device=dev)
@@ -495,7 +496,7 @@ def bench_dense_phase(args, dev, d=32):
             handle, Qr.data_ptr(), Kr.data_ptr(), Vr.data_ptr(), None, attn.data_ptr(), out_r.data_ptr(),
             mean_map.data_ptr(), H, A, A), max(10, args.steps // 4))
         _lib.check_error("dense forward with mean (row-major)")
-    del Qr, Kr, Vr, dOr, out_r, gq, gk, gv, mean_map
+    del Qr, Kr, Vr, dOr, out_r, gq, gk, gv, mean_map, scratch
 
     # forward kernel alone at the C ABI (operands in the layouts it takes: Qt, Vt feature-major)
     Qt = _lib.transpose_last2(q.detach().reshape(NB, L, d))
@@ -517,14 +518,19 @@ def bench_dense_phase(args, dev, d=32):
     alg_flops = 12.0 * L * L * d * NB
     k_fwd = "dense_fwd_reg_kernel" if d == 32 else "dense_fwd_reg64_kernel"
     shared = core.spion_debug_dense_groups(handle) == 1
-    k_bwd = "dense_group_row_kernel + dense_group_col_kernel" if shared else f"dense_bwd_row{d}_kernel + dense_bwd_col{d}_kernel"
+    walk_floats = core.spion_dense_scratch(handle)  # one walk over the map (dense_fused_kernels.h)
+    k_bwd = ("dense_group_col_dq_kernel + dense_group_row_sum_kernel" if walk_floats else
+             "dense_group_row_kernel + dense_group_col_kernel" if shared else f"dense_bwd_row{d}_kernel + dense_bwd_col{d}_kernel")
     ceil_fwd, ceil_row, ceil_col = (_matrix_ceiling(*p) for p in _DENSE_PRODUCTS[d, shared])
     map_bytes, third = 4.0 * NB * L * L, alg_flops / 3.0  # each kernel writes or reads the map once
     roof = _roof_of(k_fwd, t_fwd_rm, third, ceil_fwd, map_bytes + 16.0 * NB * L * d)
     roof["frac"] = roof["achieved"] / roof["peak"]
     roof["kernel_ms"] = {k_fwd: round(t_fwd_rm, 4), k_bwd: round(t_bwd_rm, 4)}
-    roof["backward_frac"] = (max(_floors_ms(third, ceil_row, map_bytes + 20.0 * NB * L * d).values())
-                             + max(_floors_ms(third, ceil_col, map_bytes + 20.0 * NB * L * d).values())) / t_bwd_rm
+    if walk_floats:  # four products; the map and the heads' tensors once
+        roof["backward_frac"] = max(_floors_ms(2 * third, _matrix_ceiling(4, 0, 4), map_bytes + 32.0 * NB * L * d).values()) / t_bwd_rm
+    else:
+        roof["backward_frac"] = (max(_floors_ms(third, ceil_row, map_bytes + 20.0 * NB * L * d).values())
+                                 + max(_floors_ms(third, ceil_col, map_bytes + 20.0 * NB * L * d).values())) / t_bwd_rm
     if t_fwd_mean is not None:
         roof["forward_with_mean_ms"] = round(t_fwd_mean, 4)  # spion_dense_forward_strided_mean: maps + their mean
     # the feature-major ABI: at d = 32 the same forward and a backward whose wavefronts have tiles of their own, at d = 64 the

@@ -395,6 +395,16 @@ void spion_dense_backward_strided(void* handle, const float* Q, const float* K, 
                                   float* dQ, float* dK, float* dV,
                                   int heads, const spion_head_layout* in, const spion_head_layout* out,
                                   const spion_head_layout* grad);
+/* The same backward in scratch of the caller's: launches that fill the machine (emb_dim 32) then take dQ, dK and dV from one
+ * walk over the map, the work-groups' parts of dQ lying in the scratch and nothing in the handle.
+ *   spion_dense_scratch  floats a backward can use (0: none; -1: an error)
+ *   scratch              16-byte aligned, contents unspecified, the caller's again when the call's work on the handle's stream
+ *                        has ended; null or one that is too small: the call is spion_dense_backward_strided. */
+long long spion_dense_scratch(void* handle);
+void spion_dense_backward_scratch(void* handle, const float* Q, const float* K, const float* V, const float* P,
+                                  const float* Out, const float* dO, float* dQ, float* dK, float* dV, int heads,
+                                  const spion_head_layout* in, const spion_head_layout* out,
+                                  const spion_head_layout* grad, float* scratch, long long floats);
 
 /* The dense forward on [B][H][L][d] views (spion_dense_forward_strided) that also leaves the mean of all
  * num_batches maps in Mean [seq_len][seq_len] (queries x keys, the Score input of spion_pattern_generate):

@@ -150,6 +150,10 @@ def core() -> ctypes.CDLL:
     lib.spion_transition_update.restype = c_int
     lib.spion_dense_backward_strided.argtypes = [_P] * 10 + [c_int, _P, _P, _P]
     lib.spion_dense_backward_strided.restype = None
+    lib.spion_dense_scratch.argtypes = [_P]
+    lib.spion_dense_scratch.restype = ctypes.c_longlong
+    lib.spion_dense_backward_scratch.argtypes = [_P] * 10 + [c_int, _P, _P, _P, _P, ctypes.c_longlong]
+    lib.spion_dense_backward_scratch.restype = None
     lib.spion_transpose_last2.argtypes = [_P, _P, c_int, c_int, c_int, _P]
     lib.spion_transpose_last2.restype = c_int
     lib.spion_version.restype = c_char_p

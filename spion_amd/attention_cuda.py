@@ -122,10 +122,14 @@ class _DenseAttnFunction(torch.autograd.Function):
             else:
                 dq, dk, dv = (_empty_heads((B, H, L, d), q.stride(1) < q.stride(2), dev) for _ in range(3))
             lin, lout, lgrad = _lib.taken_layout(q), _lib.taken_layout(out), _lib.head_layout(dq)
-            _lib.core().spion_dense_backward_strided(
+            try:
+                scratch = torch.empty(max(_lib.core().spion_dense_scratch(m.attn_handle), 0), dtype=torch.float32, device=dev)
+            except torch.cuda.OutOfMemoryError:  # the call does without
+                scratch = torch.empty(0, device=dev)
+            _lib.core().spion_dense_backward_scratch(
                 m.attn_handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), attn.data_ptr(), out.data_ptr(),
                 go.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), H, ctypes.addressof(lin),
-                ctypes.addressof(lout), ctypes.addressof(lgrad))
+                ctypes.addressof(lout), ctypes.addressof(lgrad), scratch.data_ptr(), scratch.numel())
             _lib.check_error("attn_backward")
             return dq, dk, dv, None, None
         qt, key, value, attn = saved

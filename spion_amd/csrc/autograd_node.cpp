@@ -411,8 +411,13 @@ struct DenseAttnNode : public torch::autograd::Function<DenseAttnNode> {
         taken_layout(q, lin);
         taken_layout(out, lout);
         head_layout(dq, lgrad);
-        spion_dense_backward_strided(h, fp(q), fp(k), fp(v), fp(attn), fp(out), fp(go), fpm(dq), fpm(dk), fpm(dv), (int)q.size(1),
-                                     &lin, &lout, &lgrad);
+        Tensor scratch;
+        try {
+            if (const int64_t floats = spion_dense_scratch(h); floats > 0) scratch = torch::empty({floats}, opt);
+        } catch (const c10::OutOfMemoryError&) {  // the call does without
+        }
+        spion_dense_backward_scratch(h, fp(q), fp(k), fp(v), fp(attn), fp(out), fp(go), fpm(dq), fpm(dk), fpm(dv), (int)q.size(1),
+                                     &lin, &lout, &lgrad, fps(scratch), count(scratch));
         check_library("attn_backward");
         return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }

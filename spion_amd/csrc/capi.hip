@@ -82,7 +82,8 @@ void sparse_backward_strided(void*, const float*, const float*, const float*, co
 void dense_forward_strided(void*, const float*, const float*, const float*, const KeyTerms&, float*, float*, int,
                            const HeadLayout&, const HeadLayout&);
 void dense_backward_strided(void*, const float*, const float*, const float*, const float*, const float*, const float*,
-                            float*, float*, float*, int, const HeadLayout&, const HeadLayout&, const HeadLayout&);
+                            float*, float*, float*, int, const HeadLayout&, const HeadLayout&, const HeadLayout&,
+                            const CallScratch&);
 void sparse_invalidate(void*);
 int sparse_register_pattern(void*, const int*, const int*, int, const int*, const int*);
 void sparse_forget_pattern(void*, const int*, const int*);
@@ -115,6 +116,7 @@ void dense_forward(void*, const float*, const float*, const float*, const KeyTer
 void dense_backward(void*, const float*, const float*, const float*, const float*, const float*, float*, float*,
                     float*);
 int dense_groups(void*);
+long long dense_scratch_floats(void*);
 int pattern_generate(const float*, int, int, int, int, int, double, float*, float*, float*, hipStream_t);
 int project_forward(const float*, const float* const*, const float* const*, float*, long long, int, int, int, hipStream_t);
 int project_forward_keys(const float*, const float* const*, const float* const*, float*, long long, int, int, int, const float*, float*,
@@ -515,7 +517,20 @@ void spion_dense_backward_strided(void* h, const float* Q, const float* K, const
         set_error("dense attn_backward_strided: null layout argument");
         return;
     }
-    dense_backward_strided(h, Q, K, V, P, Out, dO, dQ, dK, dV, heads, to_layout(in), to_layout(out), to_layout(grad));
+    dense_backward_strided(h, Q, K, V, P, Out, dO, dQ, dK, dV, heads, to_layout(in), to_layout(out), to_layout(grad),
+                           CallScratch{});
+}
+long long spion_dense_scratch(void* h) { return dense_scratch_floats(h); }
+void spion_dense_backward_scratch(void* h, const float* Q, const float* K, const float* V, const float* P, const float* Out,
+                                  const float* dO, float* dQ, float* dK, float* dV, int heads, const spion_head_layout* in,
+                                  const spion_head_layout* out, const spion_head_layout* grad, float* scratch,
+                                  long long floats) {
+    if (!in || !out || !grad) {
+        set_error("dense attn_backward_scratch: null layout argument");
+        return;
+    }
+    dense_backward_strided(h, Q, K, V, P, Out, dO, dQ, dK, dV, heads, to_layout(in), to_layout(out), to_layout(grad),
+                           call_scratch(scratch, floats));
 }
 // The forwards above on a key mask itself.
 static bool key_mask_given(const char* who, const float* mask, int heads) {

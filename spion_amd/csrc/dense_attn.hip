@@ -8,7 +8,7 @@
 // L/32 tiles of the other dimension; see tile_ops.h for the register layout, tile_kernels.h (mma_feat_init) for which
 // products run on the fp32 and which, with split operands, on the bf16 matrix pipe.
 #include "common.h"
-#include "dense_group_kernels.h"
+#include "dense_fused_kernels.h"
 #include "../../include/spion_hip.h"
 
 #include <cmath>
@@ -1558,6 +1558,30 @@ static bool dense_groups_fill(const DenseAttn* a) {
     return filling >= (a->d == 32 ? 0.64 : 0.44);
 }
 
+// Strips to a work-group of the backward in one walk (dense_fused_kernels.h), 0: the passes above.  us of a backward, passes /
+// four strips to a work-group / eight, N: work-groups of four.  Few work-groups leave CUs idle (a CU holds two of four or one of
+// eight): 16 heads of 1024 (N = 128) 55 / 72 / 92, 8 of 2048 (128) 104 / 130 / 172, 20 of 1024 (160) 73 / 69 / 91, 5 of 4096 (160)
+// 243 / 246 / 334, 22 of 1024 (176) 85 / 69 / 91, 12 of 2048 (192) 163 / 130 / 173; above that always behind the passes' time:
+// 512 heads of 96 30 / 21 / 32, 64 of 1024 158 / 131 / 124, 100 of 160 (200) 17 / 17 / 21 being the one exception.  Eight write and
+// add half as many parts but fill the machine in larger steps: one round of CUs, 40 heads of 1024 121 / 104 / 94, 24 of 1504 159
+// / 141 / 131, 32 of 1024 (half of a round) 95 / 78 / 95; more rounds, by the share of places with a strip, 128 of 1024 (1.0) 306 / 255
+// / 247, 100 of 1024 (0.78) 264 / 221 / 215, 90 (0.70) 219 / 190 / 201, 128 of 1056 (0.69) 358 / 313 / 329, 256 of 288 (0.56) 71 / 62 / 72.
+static int dense_fused_strips(const DenseAttn* a) {
+    const long long cus = device_cus(), nbr = a->L / 32, c4 = (nbr + 3) / 4, c8 = (nbr + 7) / 8, n4 = c4 * a->NB, n8 = c8 * a->NB;
+    if (a->d != 32 || a->L > 16384 || nbr < 2 || 8 * n4 <= 5 * cus) return 0;
+    const long long rounds = (n8 + cus - 1) / cus;
+    const bool eight = rounds == 1 ? c8 < c4 && 16 * n8 >= 9 * cus : 4 * nbr * a->NB >= 3 * 8 * cus * rounds;
+    return eight ? 8 : 4;
+}
+static size_t dense_fused_floats(const DenseAttn* a) {
+    const int G = dense_fused_strips(a);
+    return G ? (size_t)((a->L / 32 + G - 1) / G) * a->NB * a->L * a->d : 0;
+}
+long long dense_scratch_floats(void* h) {
+    const DenseAttn* a = as_dense(h, "dense_scratch");
+    return a ? (long long)dense_fused_floats(a) : -1;
+}
+
 int dense_groups(void* h) {
     const DenseAttn* a = as_dense(h, "spion_debug_dense_groups");
     return a ? (int)dense_groups_fill(a) : -1;
@@ -1565,7 +1589,7 @@ int dense_groups(void* h) {
 
 void dense_backward_strided(void* h, const float* Q, const float* K, const float* V, const float* P, const float* Out,
                             const float* dO, float* dQ, float* dK, float* dV, int heads, const HeadLayout& in,
-                            const HeadLayout& out, const HeadLayout& grad) {
+                            const HeadLayout& out, const HeadLayout& grad, const CallScratch& scratch) {
     const char* who = "dense attn_backward_strided";
     const HeadLayout* lays[3] = {&in, &out, &grad};
     DenseAttn* a = dense_strided_handle(h, who, heads, lays, 3);
@@ -1583,13 +1607,26 @@ void dense_backward_strided(void* h, const float* Q, const float* K, const float
         set_error("%s: the gradient layout maps two elements to one address", who);
         return;
     }
-    if (!a->ws_rowsum && !SPION_HIP_OK(hipMalloc((void**)&a->ws_rowsum, sizeof(float) * (size_t)a->NB * a->L))) return;
     Layouts ly{};
     ly.in = in;
     ly.out = out;
     ly.grad = grad;
     ly.H = heads;
     const int nbr = a->L / 32;
+    if (const size_t need = dense_fused_floats(a); need && scratch.p && scratch.floats >= need) {
+        const int G = dense_fused_strips(a), C = (nbr + G - 1) / G;
+        if (G == 8)
+            hipLaunchKernelGGL(dense_group_col_dq_kernel<8>, dim3(C * a->NB), dim3(64 * 8), 0, a->hdr.stream, Q, K, V, P, dO, Out,
+                               dK, dV, scratch.p, a->L, nbr, a->NB, a->scale, ly);
+        else
+            hipLaunchKernelGGL(dense_group_col_dq_kernel<4>, dim3(C * a->NB), dim3(64 * 4), 0, a->hdr.stream, Q, K, V, P, dO, Out,
+                               dK, dV, scratch.p, a->L, nbr, a->NB, a->scale, ly);
+        hipLaunchKernelGGL(dense_group_row_sum_kernel, dim3((nbr * a->NB + 3) / 4), dim3(256), 0, a->hdr.stream, K, V, P, dO,
+                           Out, scratch.p, dQ, C, a->L, nbr, a->NB, a->scale, ly);
+        check_launch("dense_bwd kernels");
+        return;
+    }
+    if (!a->ws_rowsum && !SPION_HIP_OK(hipMalloc((void**)&a->ws_rowsum, sizeof(float) * (size_t)a->NB * a->L))) return;
     const dim3 grid(nbr * a->NB), block4(64 * 4);
     if (dense_groups_fill(a)) {
         const int G = a->d / 8;

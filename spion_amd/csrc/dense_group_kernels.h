@@ -113,6 +113,66 @@ __device__ __forceinline__ void mma_cols(const char* T, const typename DmaTile<D
     }
 }
 
+// The sums of a strip of queries (dQ) or keys (dK, dV) once more with fp32 chains, straight from memory.  l2: the lane, hidden
+// by second_walk; init(I, ..): -g of query tile I (register = query).
+template <int D>
+__device__ __forceinline__ void dense_row_again(const float* K, const float* V, const float* Attn, const float* dO, int L,
+                                                int nbr, int I, int bh, int l2, const f32x16& gneg, size_t ib, int ild,
+                                                size_t hbytes, size_t ob, int old_, size_t obytes, f32x16 (&acc)[D / 32]) {
+    constexpr int KH = D / 2, NC = D / 32;
+    const int h2 = l2 >> 5, li2 = l2 & 31;
+    const rsrc_t rV = make_rsrc(V + ib, hbytes), rK = make_rsrc(K + ib, hbytes);
+    const rsrc_t rP = make_rsrc(Attn + (size_t)bh * L * L, (size_t)L * L * 4);
+    float go[KH];
+    ldr_rows<D>(make_rsrc(dO + ob, obytes), (li2 * old_ + h2 * KH) * 4, I * 32 * old_ * 4, go);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[c] = splat16(0.f);
+#pragma unroll 1
+    for (int J = 0; J < nbr; ++J) {
+        float vt[KH], p[16], kb[NC][16], ds[16];
+        ldr_rows<D>(rV, (li2 * ild + h2 * KH) * 4, J * 32 * ild * 4, vt);
+        ldr_tile_cols(rP, (4 * h2 * L + li2) * 4, (J * 32 * L + I * 32) * 4, L, p);
+        ldr_tile_b<D>(rK, (4 * h2 * ild + li2) * 4, J * 32 * ild * 4, kb, ild);
+        const f32x16 dp = mma_feat_f32<D>(vt, go, gneg);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ds[r] = dp[r] * p[r];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[c] = mma_chain(kb[c], ds, acc[c]);
+    }
+}
+template <int D, class Init>
+__device__ __forceinline__ void dense_col_again(const float* Q, const float* V, const float* Attn, const float* dO, int L,
+                                                int nbr, int J, int bh, int l, size_t ib, int ild, size_t hbytes, size_t ob,
+                                                int old_, size_t obytes, f32x16 (&ak)[D / 32], f32x16 (&av)[D / 32],
+                                                Init init) {
+    constexpr int KH = D / 2, NC = D / 32;
+    const int l2 = second_walk(l), h2 = l2 >> 5, li2 = l2 & 31;
+    const rsrc_t rQ = make_rsrc(Q + ib, hbytes), rdO = make_rsrc(dO + ob, obytes);
+    const rsrc_t rP = make_rsrc(Attn + (size_t)bh * L * L, (size_t)L * L * 4);
+    float v[KH];
+    ldr_rows<D>(make_rsrc(V + ib, hbytes), (li2 * ild + h2 * KH) * 4, J * 32 * ild * 4, v);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        ak[c] = splat16(0.f);
+        av[c] = splat16(0.f);
+    }
+#pragma unroll 1
+    for (int I = 0; I < nbr; ++I) {
+        float go[KH], p[16], b[NC][16], ds[16];
+        ldr_rows<D>(rdO, (li2 * old_ + h2 * KH) * 4, I * 32 * old_ * 4, go);
+        ldr_4x4(rP, (li2 * L + 4 * h2) * 4, (J * 32 * L + I * 32) * 4, p);
+        const f32x16 dp = mma_feat_f32<D>(go, v, init(I, li2, h2, rdO));
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ds[r] = dp[r] * p[r];
+        ldr_tile_b<D>(rdO, (4 * h2 * old_ + li2) * 4, I * 32 * old_ * 4, b, old_);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) av[c] = mma_chain(b[c], p, av[c]);
+        ldr_tile_b<D>(rQ, (4 * h2 * ild + li2) * 4, I * 32 * ild * 4, b, ild);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) ak[c] = mma_chain(b[c], ds, ak[c]);
+    }
+}
+
 // three work-groups of four wavefronts to a CU (d = 32: 50 KB of LDS each), one of eight (d = 64: 135 KB)
 #define SPION_GROUP_KERNEL(D) \
     __global__ __launch_bounds__(8 * (D)) __attribute__((amdgpu_waves_per_eu((D) == 32 ? 3 : 2, (D) == 32 ? 3 : 2)))
@@ -205,27 +265,7 @@ SPION_GROUP_KERNEL(D) void dense_group_row_kernel(
         step(J, std::integral_constant<int, 0>());
         if (J + 1 < nbr) step(J + 1, std::integral_constant<int, 1>());
     }
-    if (split_failed(acc)) {  // once more with fp32 chains, straight from memory
-        const int l2 = second_walk(l), h2 = l2 >> 5, li2 = l2 & 31;
-        const rsrc_t rV = make_rsrc(V + ib, hbytes), rK = make_rsrc(K + ib, hbytes);
-        const rsrc_t rP = make_rsrc(Attn + (size_t)bh * L * L, (size_t)L * L * 4);
-        float go[KH];
-        ldr_rows<D>(rdO, (li2 * old_ + h2 * KH) * 4, I * 32 * old_ * 4, go);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) acc[c] = splat16(0.f);
-#pragma unroll 1
-        for (int J = 0; J < nbr; ++J) {
-            float vt[KH], p[16], kb[NC][16], ds[16];
-            ldr_rows<D>(rV, (li2 * ild + h2 * KH) * 4, J * 32 * ild * 4, vt);
-            ldr_tile_cols(rP, (4 * h2 * L + li2) * 4, (J * 32 * L + I * 32) * 4, L, p);
-            ldr_tile_b<D>(rK, (4 * h2 * ild + li2) * 4, J * 32 * ild * 4, kb, ild);
-            const f32x16 dp = mma_feat_f32<D>(vt, go, gneg);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) ds[r] = dp[r] * p[r];
-#pragma unroll
-            for (int c = 0; c < NC; ++c) acc[c] = mma_chain(kb[c], ds, acc[c]);
-        }
-    }
+    if (split_failed(acc)) dense_row_again<D>(K, V, Attn, dO, L, nbr, I, bh, second_walk(l), gneg, ib, ild, hbytes, ob, old_, obytes, acc);
     if (Iw < nbr) {
 #pragma unroll
         for (int c = 0; c < NC; ++c) reduce_store_rows<1>(acc[c] * scale, dQ + gb + 32 * c, I * 32, w, li, h, nullptr, gld);
@@ -328,36 +368,17 @@ SPION_GROUP_KERNEL(D) void dense_group_col_kernel(
         step(I, std::integral_constant<int, 0>());
         if (I + 1 < nbr) step(I + 1, std::integral_constant<int, 1>());
     }
-    if (split_failed(ak) || split_failed(av)) {  // as above
-        const int l2 = second_walk(l), h2 = l2 >> 5, li2 = l2 & 31;
-        const rsrc_t rQ = make_rsrc(Q + ib, hbytes), rdO = make_rsrc(dO + ob, obytes);
-        const rsrc_t rP = make_rsrc(Attn + (size_t)bh * L * L, (size_t)L * L * 4), rG = make_rsrc(Gs + (size_t)bh * L, (size_t)L * 4);
-        float v[KH];
-        ldr_rows<D>(rV, (li2 * ild + h2 * KH) * 4, J * 32 * ild * 4, v);
+    if (split_failed(ak) || split_failed(av)) {
+        const rsrc_t rG = make_rsrc(Gs + (size_t)bh * L, (size_t)L * 4);
+        dense_col_again<D>(Q, V, Attn, dO, L, nbr, J, bh, l, ib, ild, hbytes, ob, old_, obytes, ak, av,
+                           [&](int I, int, int h2, const rsrc_t&) {
+                               float gi[16];
+                               ldr_4x4(rG, 16 * h2, I * 128, gi);
+                               f32x16 init;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            ak[c] = splat16(0.f);
-            av[c] = splat16(0.f);
-        }
-#pragma unroll 1
-        for (int I = 0; I < nbr; ++I) {
-            float go[KH], p[16], gi[16], b[NC][16], ds[16];
-            ldr_rows<D>(rdO, (li2 * old_ + h2 * KH) * 4, I * 32 * old_ * 4, go);
-            ldr_4x4(rP, (li2 * L + 4 * h2) * 4, (J * 32 * L + I * 32) * 4, p);
-            ldr_4x4(rG, 16 * h2, I * 128, gi);
-            f32x16 init;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) init[r] = gi[r];
-            const f32x16 dp = mma_feat_f32<D>(go, v, init);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) ds[r] = dp[r] * p[r];
-            ldr_tile_b<D>(rdO, (4 * h2 * old_ + li2) * 4, I * 32 * old_ * 4, b, old_);
-#pragma unroll
-            for (int c = 0; c < NC; ++c) av[c] = mma_chain(b[c], p, av[c]);
-            ldr_tile_b<D>(rQ, (4 * h2 * ild + li2) * 4, I * 32 * ild * 4, b, ild);
-#pragma unroll
-            for (int c = 0; c < NC; ++c) ak[c] = mma_chain(b[c], ds, ak[c]);
-        }
+                               for (int r = 0; r < 16; ++r) init[r] = gi[r];
+                               return init;
+                           });
     }
     if (Jw < nbr) {
 #pragma unroll
