@@ -678,7 +678,9 @@ void tile_fwd_kernel(
 #pragma unroll
     for (int c = 0; c < D / 32; ++c) o[c] = splat16(0.f);
 
-    auto two_sweeps = [&]() {
+    constexpr bool FALLBACK = LONG && MAXT > 0;
+    auto two_sweeps = [&](float (&q)[KH], int l) {
+        const int h = l >> 5, li = l & 31;
         // ---- sweep 1: online row maximum and denominator -------------------------------------------
         const int nu = cnt > w ? (cnt - w + WAVES - 1) / WAVES : 0;  // tiles of this wavefront
         struct PreK {
@@ -764,10 +766,15 @@ void tile_fwd_kernel(
             }
         }
     };
-    constexpr bool FALLBACK = LONG && MAXT > 0;
     if constexpr (MAXT > 0) {
       if (FALLBACK && cnt > MAXT * WAVES) {
-        two_sweeps();
+        // Nothing shared with the other branch, whose registers are full: with q shared, the strided kernels at d = 64 spilled 57
+        // registers, and a reload of one waits for all loads in flight (24 heads of 4000 110 -> 86 us, 64 of 2048 with a sixth of the
+        // blocks and key mask 161 -> 114; contiguous heads, which had room, as before).
+        const int l2 = second_walk(l);
+        float q2[KH];
+        load_q(q2, l2);
+        two_sweeps(q2, l2);
       } else {
         const int nu = cnt > w ? (cnt - w + WAVES - 1) / WAVES : 0;  // tiles of this wavefront
         f32x16 S[MAXT];
@@ -1015,7 +1022,7 @@ void tile_fwd_kernel(
         }
       }
     } else {
-        two_sweeps();
+        two_sweeps(q, l);
     }
     if constexpr (SHARE) __syncthreads();  // every wavefront is done with its tiles
     if (!ST && Ocache) reduce_store2<D, WAVES>(o, O + hb, Ocache + hb, I * 32, w, li, h, lds);
@@ -1315,13 +1322,15 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
         const u32x4 wP = rsrc_words(P + (size_t)bh * nnz, (size_t)nnz * 4), wG = rsrc_words(G + (size_t)bh * L, (size_t)L * 4);
         const int ql = DmaTileF32::voff(l, ild), ol = DmaTileF32::voff(l, old_);
         const int qx = DmaTileF32::extra_step(ild), ox = DmaTileF32::extra_step(old_);
-        const int pl0 = 16 * ((l & 7) ^ (l >> 3)), pl1 = (l >> 3) * 4;  // lane offset into a P tile: pl0 + pl1 * row stride
         const auto a_p = DmaTileF32::cols_addr(Tp, li, h);  // the Q tile's are 4 KB on
         const auto a_go = DmaTileF32::own_addr(To, li, 4 * h, 1);
         const char* a_g = Tg + 16 * h;
+        // (Strided heads have two lane offsets in ql and ol; the ones made here are then the registers over 168, and waiting for
+        // the reload of a spilled one is waiting for the tiles in flight: 32 x 2 heads of 4096 165 -> 160 us, 64 x 2 of 1024 38.2 -> 36.6.)
         auto issue_pg = [&](const int4 d) {
-            DmaTileF32::load<true>(wP, lp, pl0 + pl1 * d.z, d.y * 4, DmaTileF32::extra_step(d.z));
-            dma_b32(wG, lg, l * 4, d.x * 128);
+            const int x = ST ? lane_again() : l;
+            DmaTileF32::load<true>(wP, lp, 16 * ((x & 7) ^ (x >> 3)) + (x >> 3) * 4 * d.z, d.y * 4, DmaTileF32::extra_step(d.z));
+            dma_b32(wG, lg, x * 4, d.x * 128);
         };
         auto issue_qo = [&](const int4 d) {
             DmaTileF32::load(wQ, lq, ql, d.x * 32 * ild * 4, qx);

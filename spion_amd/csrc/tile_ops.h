@@ -190,6 +190,13 @@ __device__ __forceinline__ int second_walk(int l) {
     return l;
 }
 
+// The lane once more, two instructions where it is asked for and no register in between.
+__device__ __forceinline__ int lane_again() {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
+    return l;
+}
+
 // acc += A.B over the 16 slots of each half-wave, an fp32 chain
 __device__ __forceinline__ f32x16 mma_chain(const float (&a)[16], const float (&b)[16], f32x16 acc) {
 #pragma unroll
