@@ -46,7 +46,7 @@ def _matrix_ceiling(split, chains, algorithmic=2):
 
 # (split, fp32) products per tile of forward, row pass and column pass (spion_amd/csrc/tile_kernels.h, mma_feat_init, says why);
 # the dense forward in its register-resident form, the dense backward with shared tiles (dense_group_kernels.h) and without
-_TILE_PRODUCTS = {32: ((1, 1), (1, 1), (3, 0)), 64: ((2, 0), (2, 0), (0, 3))}
+_TILE_PRODUCTS = {32: ((1, 1), (1, 1), (3, 0)), 64: ((2, 0), (2, 0), (3, 0))}
 _DENSE_PRODUCTS = {(32, True): ((1, 1), (2, 0), (3, 0)), (64, True): ((2, 0), (2, 0), (3, 0)),
                    (32, False): ((1, 1), (2, 0), (1, 2)), (64, False): ((2, 0), (2, 0), (0, 3))}
 

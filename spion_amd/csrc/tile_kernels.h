@@ -354,6 +354,16 @@ struct DmaTileF32 {
         for (int g = 0; g < 8; ++g) x.a[g] = T + li * 128 + 16 * (g ^ (li & 7));
         return x;
     }
+    __device__ static __forceinline__ void get16(const Own8& o, int half, float (&x)[16]) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(o.a[4 * half + g]);
+            x[4 * g + 0] = v.x;
+            x[4 * g + 1] = v.y;
+            x[4 * g + 2] = v.z;
+            x[4 * g + 3] = v.w;
+        }
+    }
     __device__ static __forceinline__ void get32(const Own8& o, float (&x)[32]) {
 #pragma unroll
         for (int g = 0; g < 8; ++g) {
@@ -407,13 +417,13 @@ struct DmaTileF32 {
 //   * products over the head dimension, whose other operand a wavefront keeps for all its tiles, are split: one
 //     operand per tile;
 //   * products over a tile's rows, which need two operands split, run on the bf16 pipe in the forward at d = 64 (one of the
-//     two serves two products), in the row pass and in the column pass at d = 32 (three wavefronts per SIMD hide the
+//     two serves two products), in the row pass and in the column pass (d = 32: three wavefronts per SIMD hide the
 //     splitting; dO is split once for its two products), on the fp32 pipe in the forward at d = 32 (split there: 32 x 2 heads
 //     of 4096, a tenth kept, whole step 475 -> 488 us; six logit tiles and split operands spill at three wavefronts per SIMD);
-//   * the column pass at d = 64 uses fp32 chains alone: split operands for its five products spill registers, and whole
-//     steps are 1 % slower to 4 % faster without (split / fp32 chains in us, on four machines: 64 x 2 heads of 1024,
-//     14 % kept, 194 to 202 / 187 to 194; 16 x 4 of 2048, 10 %, 262 to 274 / 255 to 265; 3 x 8 of 4000, 8 %, 278 to 291 / 274
-//     to 291).
+//   * the column pass at d = 64 splits an operand where it is used and reads it out of LDS no earlier: all of a tile's held at
+//     once were 16 to 21 registers too many, whose reloads wait for the tiles in flight, and gave away what the products gained.
+//     fp32 chains / split, us: 3 x 8 heads of 4000, 8 % kept, 132 / 103 (whole step 297 / 272), 16 x 4 of 2048, 16 %, 165 / 131
+//     (378 / 352); 2-norm errors against float64 of dK and dV there 4.1e-7 / 3.5e-7 and 3.9e-7 / 3.4e-7.
 // Measured in us per launch in a training loop, all kernels on fp32 chains / as now.  32 x 2 heads of 4096 tokens,
 // d = 32, 32 x 32 blocks, a tenth kept: forward 162 / 155, row pass 141 / 134, column pass 184 / 161; 256 x 2 heads of 1024:
 // 139 / 139, 122 / 121, 148 / 132; 2 x 2 of 8192, a fifth kept (two sweeps): 104 / 97, 76 / 71, 98 / 91; 3 x 8 heads of 4000,
@@ -1406,7 +1416,7 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
             }
         }
     } else {
-        // d = 64, the same schedule: the Q and dO tiles are two 4 KB tiles each (features 0..31 and 32..63), the P
+        // d = 64: the Q and dO tiles are two 4 KB tiles each (features 0..31 and 32..63), the P
         // tile one; twenty instructions a tile.  No room is left for -g: each lane loads the value of query row
         // lane % 32 of the next tile with an ordinary load (the compiler's wait for it falls where everything in
         // flight is waited for anyway, see settle), and one extra MFMA step -- A = that value in the lower half-wave,
@@ -1424,20 +1434,83 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
         const auto a_p = DmaTileF32::cols_addr(Tp, li, h), a_q = DmaTileF32::cols_addr(Tq, li, h),
                    a_o = DmaTileF32::cols_addr(To, li, h);
         const auto a_go = DmaTileF32::own8_addr(To + h * DmaTileF32::TILE, li);  // dO[query li][feature 32h + s]
-        auto issue = [&](const int4 d) {
-            const int I = d.x, rn = d.z;
-            DmaTileF32::load<true>(wP, lp, pl0 + pl1 * rn, d.y * 4, DmaTileF32::extra_step(rn));
-            DmaTileF32::load(wQ, lq, ql, I * 32 * ild * 4, qx);
-            DmaTileF32::load(wQ, lq + DmaTileF32::TILE, ql, I * 32 * ild * 4 + 128, qx);
-            DmaTileF32::load(wO, lo, ol, I * 32 * old_ * 4, ox);
-            DmaTileF32::load(wO, lo + DmaTileF32::TILE, ol, I * 32 * old_ * 4 + 128, ox);
+        auto issue_p = [&](const int4 d) {
+            DmaTileF32::load<true>(wP, lp, pl0 + pl1 * d.z, d.y * 4, DmaTileF32::extra_step(d.z));
+        };
+        auto issue_q = [&](const int4 d) {
+            DmaTileF32::load(wQ, lq, ql, d.x * 32 * ild * 4, qx);
+            DmaTileF32::load(wQ, lq + DmaTileF32::TILE, ql, d.x * 32 * ild * 4 + 128, qx);
+        };
+        auto issue_o = [&](const int4 d) {
+            DmaTileF32::load(wO, lo, ol, d.x * 32 * old_ * 4, ox);
+            DmaTileF32::load(wO, lo + DmaTileF32::TILE, ol, d.x * 32 * old_ * 4 + 128, ox);
         };
         if (nu > 0) {
             int4 dn = desc[w];
-            issue(dn);
             float gl = ld1(rG, li * 4, dn.x * 128);
+            issue_p(dn);
+            issue_o(dn);
+            issue_q(dn);
             dn = desc[w + (nu > 1 ? WAVES : 0)];
             for (int i = 0; i < nu; ++i) {
+                if constexpr (!EXACT) {
+                    // Operands are read out of LDS, split and used one after the other, and a tile's place is requested again
+                    // as soon as it has been read.
+                    const int4 dnn = desc[w + min(i + 2, nu - 1) * WAVES];
+                    wait_vm<0>();
+                    settle(gl);
+                    const float ga = h == 0 ? gl : 0.f;
+                    float p[16];
+                    DmaTileF32::get(a_p, p);
+                    wait_lgkm0();
+                    if (i + 1 < nu) {
+                        gl = ld1(rG, li * 4, dn.x * 128);
+                        issue_p(dn);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    f32x16 dp = __builtin_amdgcn_mfma_f32_32x32x2f32(ga, 1.0f, splat16(0.f), 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        float x[16];
+                        Split3<16> v;
+                        DmaTileF32::get16(a_go, t, x);
+#pragma unroll
+                        for (int k = 0; k < 3; ++k)
+#pragma unroll
+                            for (int j = 0; j < 2; ++j) v.p[k][j] = vk.p[k][2 * t + j];
+                        dp = mma_split(split3(x), v, dp);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    {
+                        const Split3<16> ps = split3(p);
+#pragma unroll
+                        for (int c = 0; c < 2; ++c) {
+                            float x[16];
+                            DmaTileF32::get(a_o, x, c * DmaTileF32::TILE);
+                            if (c == 1) {
+                                wait_lgkm0();
+                                if (i + 1 < nu) issue_o(dn);
+                            }
+                            av[c] = mma_split(ps, split3(x), av[c]);
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    {
+                        float ds[16];
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) ds[r] = dp[r] * p[r];
+                        const Split3<16> dss = split3(ds);
+                        float qb[2][16];
+                        DmaTileF32::get(a_q, qb[0]);
+                        DmaTileF32::get(a_q, qb[1], DmaTileF32::TILE);
+                        wait_lgkm0();
+                        if (i + 1 < nu) issue_q(dn);
+                        dn = dnn;
+#pragma unroll
+                        for (int c = 0; c < 2; ++c) ak[c] = mma_split(dss, split3(qb[c]), ak[c]);
+                    }
+                    continue;
+                } else {
                 const int4 dnn = desc[w + min(i + 2, nu - 1) * WAVES];  // descriptor of the tile after the next
                 wait_vm<0>();
                 settle(gl);
@@ -1451,7 +1524,9 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
                 DmaTileF32::get(a_o, ob[1], DmaTileF32::TILE);
                 wait_lgkm0();
                 if (i + 1 < nu) {
-                    issue(dn);
+                    issue_p(dn);
+                    issue_q(dn);
+                    issue_o(dn);
                     gl = ld1(rG, li * 4, dn.x * 128);
                 }
                 dn = dnn;
@@ -1461,21 +1536,18 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
                 float ds[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pc[r];
-                mma_b_split<D, EXACT>(ds, qb, ak);
-                mma_b_split<D, EXACT>(pc, ob, av);
+                mma_b_f32<D>(ds, qb, ak);
+                mma_b_f32<D>(pc, ob, av);
+                }
             }
         }
     }
     };
-    if constexpr (D == 64) {
-        walk(whole(vt), l);
-    } else {
-        walk(split3(vt), l);
-        if (split_failed(ak) || split_failed(av)) {
-            const int l2 = second_walk(l);
-            load_vt(vt, l2);
-            walk(whole(vt), l2);
-        }
+    walk(split3(vt), l);
+    if (split_failed(ak) || split_failed(av)) {
+        const int l2 = second_walk(l);
+        load_vt(vt, l2);
+        walk(whole(vt), l2);
     }
     if constexpr (WAVES > 1) __syncthreads();  // every wavefront is done with its tiles
 #pragma unroll
