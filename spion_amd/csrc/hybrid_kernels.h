@@ -61,22 +61,6 @@ constexpr int HYB_GWAVES = 4;    // wavefronts (rows / columns) per work-group o
 // two wavefronts per SIMD, each with the next tile's operands in flight while it works on one
 #define SPION_HYB_KERNEL(W) __global__ __launch_bounds__(64 * (W)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 
-// What the tile kernels request ahead of a tile: two operand tiles (raw 16-byte pieces, linear), the tile of P in the
-// col-owner layout, and -- one tile further ahead, because the addresses of P come out of it -- the tile's index:
-// block column (or row), and position and present-column set of tile row li (lane li and lane 32 + li hold the same).
-struct HybPre {
-    f32x4 a[4], b[4];
-    float p[16];
-    float g_l;
-    int pos_l, blk;
-    unsigned bits_l;
-};
-
-__device__ __forceinline__ void hyb_fetch_index(const HybIndex& ix, int t, int li, HybPre& x) {
-    x.pos_l = ix.t_pos[(size_t)t * 32 + li];
-    x.bits_l = ix.t_bits[(size_t)t * 32 + li];
-}
-
 // One value per tile row, held by lane li (and 32 + li) for row li, to the 16 rows acc_row(q, h), q = 0..15, a lane
 // works on: through 32 words of the wavefront's own LDS space.
 __device__ __forceinline__ void hyb_rows_from_lanes(int* xs, int l, int h, int v, int (&out)[16]) {
@@ -86,14 +70,6 @@ __device__ __forceinline__ void hyb_rows_from_lanes(int* xs, int l, int h, int v
         const int4 p = *reinterpret_cast<const int4*>(xs + 8 * g + 4 * h);
         out[4 * g + 0] = p.x, out[4 * g + 1] = p.y, out[4 * g + 2] = p.z, out[4 * g + 3] = p.w;
     }
-}
-__device__ __forceinline__ void hyb_tile_rows(int* xs, int l, int h, const HybPre& x, int (&pos)[16],
-                                              unsigned (&bits)[16]) {
-    int b[16];
-    hyb_rows_from_lanes(xs, l, h, x.pos_l, pos);
-    hyb_rows_from_lanes(xs + 64, l, h, (int)x.bits_l, b);
-#pragma unroll
-    for (int q = 0; q < 16; ++q) bits[q] = (unsigned)b[q];
 }
 // The tile of P in the col-owner layout (lane li = column of the tile, register q = row acc_row(q, h)); absent
 // entries read as 0 (their offset lies past the end of the buffer).  A tile row's entries are consecutive in memory:
@@ -203,32 +179,62 @@ __device__ __forceinline__ void hyb_rows_by_entries(float* T, int l, int n, cons
     for (int r = 0; r < 16; ++r) acc[r] = T[acc_row(r, h) * TS + li];
 }
 
-// Two-deep software pipeline over n tiles with two register sets: while tile i is computed, the operands and P of
-// tile i + 1 are in flight and so is the index of tile i + 2 (requested first, so that waiting for it leaves the
-// younger requests outstanding).  Positions past the end are clamped by the callers (valid, redundant requests).
-template <class FetchIdx, class FetchData, class Compute>
-__device__ __forceinline__ void hyb_pipeline(int n, HybPre& a, HybPre& b, FetchIdx fetch_idx, FetchData fetch_data,
-                                             Compute compute) {
-    if (n <= 0) return;
-    fetch_idx(a, 0);
-    fetch_idx(b, 1);
-    fetch_data(a, 0);
+// A tile's index: block column (or row), and position and present-column set of tile row li (lane li and lane 32 + li hold the
+// same).
+struct HybTile {
+    int pos_l, blk;
+    unsigned bits_l;
+};
+__device__ __forceinline__ void hyb_fetch_index(const HybIndex& ix, int t, int li, HybTile& x) {
+    x.pos_l = ix.t_pos[(size_t)t * 32 + li];
+    x.bits_l = ix.t_bits[(size_t)t * 32 + li];
+}
+// An element of the index that is the same for the wavefront, as a scalar load: the vector loads in flight are counted.
+__device__ __forceinline__ int hyb_scalar(const int* p, int i) {
+    return __builtin_amdgcn_readfirstlane(
+        reinterpret_cast<const __attribute__((address_space(4))) int*>(reinterpret_cast<uintptr_t>(p))[i]);
+}
+// us per launch, operand tiles in two register sets and fp32 chains (row pass; in the column pass the product dO.V^T was split) /
+// so, with all products split: 32 x 2 heads of 4096, 5 tiles a strip, 97 / 90 and 101 / 86; 2-norm errors against float64 of dQ
+// 1.91e-7 / 1.57e-7, dK 1.76e-7 / 1.60e-7, dV 1.57e-7 / 1.41e-7.  (The index of a strip's first tile with its own rows: no
+// difference; three wavefronts per SIMD spill 74 registers in the row pass.)
+// The walk of the backward kernels over n > 0 tiles: while tile i is worked on, its operand tiles' places in LDS, read by then,
+// take those of tile i + 1 (load: buffer loads into LDS), the registers of its P take the gathered entries of tile i + 1, and
+// the index of tile i + 2 is on its way.  fetch(x, i): the index of tile i (two loads, past the end those of the last one);
+// x: the first tile's.  work(p, next): reads tile i's operands out of LDS, calls next() and forms its products.
+template <class Fetch, class Load, class Work>
+__device__ __forceinline__ void hyb_walk(int n, HybTile x, int* X, int l, int h, int li, rsrc_t rP, Fetch fetch, Load load,
+                                         Work work) {
+    HybTile y;
+    float p[16];
+    auto request = [&](const HybTile& t) {
+        int pos[16], bits[16];
+        unsigned set[16];
+        hyb_rows_from_lanes(X, l, h, t.pos_l, pos);
+        hyb_rows_from_lanes(X + 64, l, h, (int)t.bits_l, bits);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) set[q] = (unsigned)bits[q];
+        load(__builtin_amdgcn_readfirstlane(t.blk));
+        hyb_load_p_cols(rP, pos, set, li, p);
+    };
+    auto step = [&](int i, const HybTile& now, HybTile& then) {
+        fetch(then, i + 2);
+        wait_vm<2>();  // all but that index
+        __builtin_amdgcn_sched_barrier(0);
+        work(p, [&] {
+            request(now);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    request(x);
+    fetch(x, 1);
     int i = 0;
     for (; i + 1 < n; i += 2) {
-        fetch_idx(a, i + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_data(b, i + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(a, i);
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_idx(b, i + 3);
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_data(a, i + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(b, i + 1);
-        __builtin_amdgcn_sched_barrier(0);
+        step(i, x, y);
+        step(i + 1, y, x);
     }
-    if (i < n) compute(a, i);
+    wait_vm<0>();
+    if (i < n) work(p, [] {});
 }
 
 // =================================================================================================
@@ -548,9 +554,12 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_row_kernel(const float* __restrict__ K
                                               float* __restrict__ dQ, HybIndex ix, int L, int nbr, int NB, int nnz,
                                               float scale, Layouts ly) {
     constexpr int D = 32, KH = 16;
-    __shared__ __attribute__((aligned(16))) float lds_t[WAVES][64 * TS];
-    __shared__ __attribute__((aligned(16))) int lds_x[WAVES][128];
-    float* lds = &lds_t[0][0];
+    typedef DmaTileF32 DT;
+    // per wavefront: the V and K tiles, a padded tile (layout change of P; the final reduction starts there) and the index
+    constexpr int WB = 2 * DT::TILE + 32 * TS * 4 + 512;
+    static_assert(WAVES == 1 || WAVES * WB >= WAVES * 4096, "the reduction fits in the tile space");
+    __shared__ __attribute__((aligned(16))) char smem[WAVES * WB];
+    float* lds = reinterpret_cast<float*>(smem);
     const int item = xcd_remap(blockIdx.x, nbr * NB);
     const int bh = item / nbr, I = item % nbr;
     const int w = wave_index(), l = threadIdx.x & 63, h = l >> 5, li = l & 31;
@@ -562,13 +571,28 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_row_kernel(const float* __restrict__ K
     const rsrc_t rK = make_rsrc(K + ib, ibytes), rV = make_rsrc(V + ib, ibytes);
     const rsrc_t rdO = make_rsrc(dO + ob, obytes), rO = make_rsrc(Out + ob, obytes);
     const rsrc_t rP = make_rsrc(P + (size_t)bh * nnz, (size_t)nnz * 4);
-    float* T = lds_t[w];
-    float* Tx = T + 32 * TS;
-    int* X = lds_x[w];
-    const int lin = lin_voff(l, ild), tile_bytes = 32 * ild * 4;
+    const u32x4 wV = rsrc_words(V + ib, ibytes), wK = rsrc_words(K + ib, ibytes);
+    const char* Tv = smem + w * WB;
+    const char* Tk = Tv + DT::TILE;
+    float* T = reinterpret_cast<float*>(smem + w * WB + 2 * DT::TILE);
+    int* X = reinterpret_cast<int*>(smem + w * WB + 2 * DT::TILE + 32 * TS * 4);
+    const unsigned lv = lds_address(Tv), lk = lv + DT::TILE;
+    const int tile_bytes = 32 * ild * 4;
 
+    auto load_go = [&](float (&go)[KH], int l) {
+        ldr_rows<D>(rdO, ((l & 31) * old_ + (l >> 5) * KH) * 4, I * 32 * old_ * 4, go);
+    };
+    const int t0 = hyb_scalar(ix.t_rp, I), cnt = hyb_scalar(ix.t_rp, I + 1) - t0;
+    const int n = cnt > w ? (cnt - w + WAVES - 1) / WAVES : 0;
+    auto fetch = [&](HybTile& x, int i, int li) {
+        const int t = t0 + w + max(min(i, n - 1), 0) * WAVES;
+        x.blk = hyb_scalar(ix.t_col, t);
+        hyb_fetch_index(ix, t, li, x);
+    };
+    HybTile x0 = {};
+    if (n > 0) fetch(x0, 0, li);  // on its way with the strip's own rows
     float go[KH], oo[KH];
-    ldr_rows<D>(rdO, (li * old_ + h * KH) * 4, I * 32 * old_ * 4, go);
+    load_go(go, l);
     ldr_rows<D>(rO, (li * old_ + h * KH) * 4, I * 32 * old_ * 4, oo);
     float g = 0.f;
 #pragma unroll
@@ -577,39 +601,45 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_row_kernel(const float* __restrict__ K
     if (w == 0 && h == 0) G[(size_t)bh * L + I * 32 + li] = -g;
     const f32x16 gneg = splat16(-g);
 
-    const int t0 = ix.t_rp[I], cnt = ix.t_rp[I + 1] - t0;
-    const int n = cnt > w ? (cnt - w + WAVES - 1) / WAVES : 0;
-    f32x16 acc[1] = {splat16(0.f)};
-    HybPre xa, xb;
-    hyb_pipeline(
-        n, xa, xb,
-        [&](HybPre& x, int i) {
-            const int t = t0 + w + min(i, n - 1) * WAVES;
-            x.blk = ix.t_col[t];
-            hyb_fetch_index(ix, t, li, x);
-        },
-        [&](HybPre& x, int) {
-            int pos[16];
-            unsigned bits[16];
-            hyb_tile_rows(X, l, h, x, pos, bits);
-            ldr_tile_lin(rV, lin, x.blk * tile_bytes, ild, x.a);
-            hyb_load_p_cols(rP, pos, bits, li, x.p);
-            ldr_tile_lin(rK, lin, x.blk * tile_bytes, ild, x.b);
-        },
-        [&](HybPre& x, int) {
-            float pr[16], vt[KH], kb[1][16];
-            lds_put_lin(Tx, l, x.a);
-            lds_get_feat32(Tx, li, h, vt);
-            lds_put_cols(T, li, h, x.p);
-            lds_get_rows(T, li, h, pr);                        // pr[r] = P[query li][key acc_row(r, h)]
-            const f32x16 dp = mma_feat_f32<D>(vt, go, gneg);  // dp[r] = dO_i . v_j - g_i
-            lds_put_lin(Tx, l, x.b);
-            lds_get_cols(Tx, li, h, kb[0]);
-            float ds[16];
+    f32x16 acc[1];
+    auto walk = [&](const auto& gk, int l) {  // gk: the dO operand, split or whole
+        constexpr bool EXACT = is_whole<std::decay_t<decltype(gk)>>;
+        const int h = l >> 5, li = l & 31;
+        const int il = DT::voff(l, ild), ix_ = DT::extra_step(ild);
+        const auto a_v = DT::own_addr(Tv, li, 4 * h, 1);
+        const auto a_k = DT::cols_addr(Tk, li, h);
+        settle(gk);
+        acc[0] = splat16(0.f);
+        if (n <= 0) return;
+        hyb_walk(
+            n, x0, X, l, h, li, rP, [&](HybTile& x, int i) { fetch(x, i, li); },
+            [&](int blk) {
+                DT::load(wV, lv, il, blk * tile_bytes, ix_);
+                DT::load(wK, lk, il, blk * tile_bytes, ix_);
+            },
+            [&](const float (&p)[16], auto next) {
+                float vt[KH], kb[1][16], pr[16];
+                lds_put_cols(T, li, h, p);
+                DT::get(a_v, vt);
+                DT::get(a_k, kb[0]);
+                lds_get_rows(T, li, h, pr);  // pr[r] = P[query li][key acc_row(r, h)]
+                wait_lgkm0();
+                next();
+                const f32x16 dp = mma_feat_init<D>(vt, gk, gneg);  // dp[r] = dO_i . v_j - g_i
+                float ds[16];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
-            hyb_mma_add(ds, kb, acc);
-        });
+                for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pr[r];
+                f32x16 part[1] = {splat16(0.f)};
+                mma_b_split<D, EXACT>(ds, kb, part);
+                acc[0] += part[0];
+            });
+    };
+    walk(split3(go), l);
+    if (split_failed(acc)) {
+        const int l2 = second_walk(l);
+        load_go(go, l2);
+        walk(whole(go), l2);
+    }
     if (hyb_not_finite(acc[0]))
         hyb_rows_by_entries(
             T, l, n, ix, rK, ild, [&](int u) { return t0 + w + u * WAVES; },
@@ -690,12 +720,17 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_col_kernel(const float* __restrict__ Q
                                               float* __restrict__ dV, HybIndex ix, int L, int nbr, int NB, int nnz,
                                               float scale, Layouts ly) {
     constexpr int D = 32, KH = 16;
-    __shared__ __attribute__((aligned(16))) float lds_t[WAVES][64 * TS];
-    __shared__ __attribute__((aligned(16))) int lds_x[WAVES][128];
-    float* lds = &lds_t[0][0];
+    typedef DmaTileF32 DT;
+    typedef DmaTile<32> Plane;
+    // per wavefront: the Q and dO tiles, the parts of dO (its second product reads them transposed), -g and the index
+    constexpr int WB = 2 * DT::TILE + 3 * Plane::TILE + 256 + 512;
+    static_assert(2 * 32 * TS * 4 <= WB, "the sums by entries fit in the tile space");
+    __shared__ __attribute__((aligned(16))) char smem[WAVES * WB];
+    float* lds = reinterpret_cast<float*>(smem);
     const int item = xcd_remap(blockIdx.x, nbr * NB);
     const int bh = item / nbr, J = item % nbr;
-    const int w = wave_index(), l = threadIdx.x & 63, h = l >> 5, li = l & 31;
+    const int w = wave_index(), l = threadIdx.x & 63;
+    const int h = l >> 5, li = l & 31;
     size_t ib, ob, gb, ibytes, obytes, gbytes;
     int ild, old_, gld;
     head_slice<ST, D>(ly.in, ly.H, bh, L, ib, ild, ibytes);
@@ -705,67 +740,109 @@ SPION_HYB_KERNEL(WAVES) void hyb_tile_bwd_col_kernel(const float* __restrict__ Q
     const rsrc_t rdO = make_rsrc(dO + ob, obytes);
     const rsrc_t rG = make_rsrc(G + (size_t)bh * L, (size_t)L * 4);
     const rsrc_t rP = make_rsrc(P + (size_t)bh * nnz, (size_t)nnz * 4);
-    float* Tq = lds_t[w];
-    float* To = Tq + 32 * TS;
-    int* X = lds_x[w];
+    const u32x4 wQ = rsrc_words(Q + ib, ibytes), wO = rsrc_words(dO + ob, obytes), wG = rsrc_words(G + (size_t)bh * L, (size_t)L * 4);
+    char* const Tq_ = smem + w * WB;
+    char* const To_ = Tq_ + DT::TILE;
+    char* const planes = Tq_ + 2 * DT::TILE;
+    char* const Tg = planes + 3 * Plane::TILE;
+    int* X = reinterpret_cast<int*>(Tg + 256);
+    const unsigned lq = lds_address(Tq_), lo = lq + DT::TILE, lg = lds_address(Tg);
 
     auto load_vt = [&](float (&vt)[KH], int l) {
         ldr_rows<D>(rV, ((l & 31) * ild + (l >> 5) * KH) * 4, J * 32 * ild * 4, vt);
     };
+    f32x16 ak[1], av[1];
+    const int e0 = hyb_scalar(ix.t_cp, J), ecnt = hyb_scalar(ix.t_cp, J + 1) - e0;
+    const int n = ecnt > w ? (ecnt - w + WAVES - 1) / WAVES : 0;
+    auto fetch = [&](HybTile& x, int i, int li) {
+        const int e = e0 + w + max(min(i, n - 1), 0) * WAVES;
+        x.blk = hyb_scalar(ix.t_ci, e);
+        hyb_fetch_index(ix, hyb_scalar(ix.t_ct, e), li, x);
+    };
+    HybTile x0 = {};
+    if (n > 0) fetch(x0, 0, li);
     float vt[KH];
     load_vt(vt, l);
 
-    f32x16 ak[1], av[1];
-    const int e0 = ix.t_cp[J], ecnt = ix.t_cp[J + 1] - e0;
-    const int n = ecnt > w ? (ecnt - w + WAVES - 1) / WAVES : 0;
     auto walk = [&](const auto& vk, int l) {  // vk: the V operand, split or whole
-    const int h = l >> 5, li = l & 31;
-    const int lin_i = lin_voff(l, ild), lin_o = lin_voff(l, old_);
-    ak[0] = splat16(0.f);
-    av[0] = splat16(0.f);
-    HybPre xa, xb;
-    hyb_pipeline(
-        n, xa, xb,
-        [&](HybPre& x, int i) {
-            const int e = e0 + w + min(i, n - 1) * WAVES;
-            x.blk = ix.t_ci[e];
-            hyb_fetch_index(ix, ix.t_ct[e], li, x);
-        },
-        [&](HybPre& x, int) {
-            int pos[16];
-            unsigned bits[16];
-            hyb_tile_rows(X, l, h, x, pos, bits);
-            ldr_tile_lin(rQ, lin_i, x.blk * 32 * ild * 4, ild, x.a);
-            ldr_tile_lin(rdO, lin_o, x.blk * 32 * old_ * 4, old_, x.b);
-            hyb_load_p_cols(rP, pos, bits, li, x.p);  // p[r] = P[query acc_row(r, h)][key li]
-            x.g_l = ld1(rG, li * 4, x.blk * 128);
-        },
-        [&](HybPre& x, int) {
-            float go[KH], qb[1][16], ob[1][16];
-            int gn[16];
-            lds_put_lin(Tq, l, x.a);
-            lds_put_lin(To, l, x.b);
-            hyb_rows_from_lanes(X, l, h, __builtin_bit_cast(int, x.g_l), gn);
-            lds_get_feat32(To, li, h, go);
-            lds_get_cols(Tq, li, h, qb[0]);
-            lds_get_cols(To, li, h, ob[0]);
-            f32x16 init;
+        constexpr bool EXACT = is_whole<std::decay_t<decltype(vk)>>;
+        const int h = l >> 5, li = l & 31;
+        const int ql = DT::voff(l, ild), qx = DT::extra_step(ild), ol = DT::voff(l, old_), ox = DT::extra_step(old_);
+        const auto a_q = DT::cols_addr(Tq_, li, h);  // the dO tile's are 4 KB on
+        const auto a_go = DT::own_addr(To_, li, 4 * h, 1);
+        const auto ra = Plane::row_addr(li, h);
+        const auto ta = Plane::tr_addr(l);
+        settle(vk);
+        ak[0] = splat16(0.f);
+        av[0] = splat16(0.f);
+        if (n <= 0) return;
+        hyb_walk(
+            n, x0, X, l, h, li, rP, [&](HybTile& x, int i) { fetch(x, i, li); },
+            [&](int blk) {
+                DT::load(wQ, lq, ql, blk * 32 * ild * 4, qx);
+                DT::load(wO, lo, ol, blk * 32 * old_ * 4, ox);
+                dma_b32(wG, lg, l * 4, blk * 128);
+            },
+            [&](const float (&p)[16], auto next) {  // p[r] = P[query acc_row(r, h)][key li]
+                float go[KH], qb[1][16], pc[16];
+                f32x16 init;
+                DT::get(a_go, go);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) init[r] = __builtin_bit_cast(float, gn[r]);
-            const f32x16 dp = mma_feat_init<D>(go, vk, init);  // dO_i . v_j - g_i, i = acc_row(r, h), j = li
-            float ds[16];
+                for (int g = 0; g < 4; ++g) {
+                    const f32x4 v = *reinterpret_cast<const f32x4*>(Tg + 16 * h + 32 * g);
+                    init[4 * g + 0] = v.x;
+                    init[4 * g + 1] = v.y;
+                    init[4 * g + 2] = v.z;
+                    init[4 * g + 3] = v.w;
+                }
+                DT::get(a_q, qb[0]);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) ds[r] = dp[r] * x.p[r];
-            hyb_mma_add(ds, qb, ak);
-            hyb_mma_add(x.p, ob, av);
-        });
+                for (int r = 0; r < 16; ++r) pc[r] = p[r];
+                f32x16 dp, part[1] = {splat16(0.f)};
+                if constexpr (EXACT) {
+                    float ot[1][16];
+                    DT::get(a_q, ot[0], DT::TILE);
+                    wait_lgkm0();
+                    next();
+                    dp = mma_feat_init<D>(go, vk, init);  // dO_i . v_j - g_i, i = acc_row(r, h), j = li
+                    mma_b_f32<D>(pc, ot, part);
+                } else {
+                    wait_lgkm0();
+                    next();
+                    const Split3<16> gs = split3(go);
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) *reinterpret_cast<bf16x8*>(planes + k * Plane::TILE + ra.a[t]) = gs.p[k][t];
+                    dp = mma_split(gs, vk, init);
+                    asm volatile("" ::: "memory");  // same-wave LDS accesses complete in order
+                    Split3<16> ot;
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        bf16x8 x[1][2];
+                        Plane::get_tile_t(planes + k * Plane::TILE, ta, x);
+                        ot.p[k][0] = x[0][0];
+                        ot.p[k][1] = x[0][1];
+                    }
+                    part[0] = mma_split(split3(pc), ot, part[0]);
+                }
+                av[0] += part[0];
+                float ds[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) ds[r] = dp[r] * pc[r];
+                part[0] = splat16(0.f);
+                mma_b_split<D, EXACT>(ds, qb, part);
+                ak[0] += part[0];
+            });
     };
     walk(split3(vt), l);
-    if (split_failed(ak)) {  // (dV comes from fp32 chains in any case)
+    if (split_failed(ak) || split_failed(av)) {
         const int l2 = second_walk(l);
         load_vt(vt, l2);
         walk(whole(vt), l2);
     }
+    float* Tq = reinterpret_cast<float*>(Tq_);
+    float* To = Tq + 32 * TS;
     if (hyb_not_finite(ak[0]) || hyb_not_finite(av[0])) {
         const int l2 = second_walk(l), h = l2 >> 5, li = l2 & 31;
 #pragma unroll 1

@@ -432,8 +432,7 @@ struct DmaTileF32 {
 // of 1024 tokens stay where they are (390: memory), 32 x 2 heads of 2048 in 64 x 64 blocks 133 -> 131.  The dense kernels (dense_attn.hip), 64 x 2 heads of 1024, d = 32: forward 180 / 177, row pass 177
 // / 156, column pass 235 / 209 (of its products the first; three splits do not fit the registers of three wavefronts per
 // SIMD: 260); 4 x 2 of 3072: 163 / 136, 108 / 86, 148 / 118; 4 x 8 of 2048, d = 64: 319 / 276, 276 / 240.  The dense
-// tiles of element patterns (hybrid_kernels.h, 32 x 2 heads of 4096): forward 97 / 91, column pass 99 / 96; the row pass (84 / 84)
-// stays on fp32 chains.
+// tiles of element patterns (hybrid_kernels.h, 32 x 2 heads of 4096): forward 97 / 91; their backward has figures of its own there.
 // Against float64 the outputs and gradients of both are as close as the fp32 chains' or closer (2-norms, 1024 to 4096
 // tokens: 1.0e-7 to 5.8e-7 where those gave 2.2e-7 to 6.1e-7).
 // acc = init + A.B over the head dimension; B is an operand the kernel keeps, split or whole.
