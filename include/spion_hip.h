@@ -304,7 +304,8 @@ void spion_attn_backward_rowmajor(void* handle, const float* Q, const float* K, 
  *   the pattern must be a union of aligned 32x32 tiles and must already be analysed on this handle
  *   (by an earlier forward with the same Offsets / Columns / nnz, or by spion_register_pattern).
  * All calls on one GPU share the array: calls that overlap on one GPU (two streams, two threads, two handles)
- * race.  Nothing in it needs clearing between calls: the row pass writes every row sum the column pass reads. */
+ * race.  Nothing in it needs clearing between calls: the row pass writes every row sum the column pass reads.  (Small calls form
+ * the row sums where they are used and touch neither array.) */
 void spion_attn_backward_noalloc(void* handle, const float* Q, const float* K, const float* V, const float* P,
                                  const float* Out, const float* dO,
                                  float* dQ, float* dK, float* dV,

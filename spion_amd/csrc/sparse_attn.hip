@@ -1514,6 +1514,21 @@ static int bwd_waves(const SparseAttn* a, const PatternIndex& pi, int nbr, int s
     return 4;
 }
 
+// Wavefronts per strip of a backward whose passes share one launch (d = 32, eight wavefronts on a CU); 0: one pass after the
+// other.  One launch wins while its tail and start are much of the step: up to 80 tiles per CU over all heads (a fifth to a half
+// of the time at 64 to 2048 strips of four tiles, a tenth at 4096; 91 us each way at 92 tiles per CU; at 200, 177 against 162).
+// A strip is shared by two or four wavefronts where the longest is more than twice or five times what a wavefront's place on
+// the machine has to do (in us with 1, 2 and 4; rows and columns alike, then an eighth of the columns four times as long:
+// 512 strips of 4 tiles 17.7, 15.2, 17.2, then 34, 23, 19; 2048 of them 40, 45, 56, then 57, 53, 60; 256 of 19 tiles 50, 33, 24;
+// 1024 of 13 tiles 54, 51, 57, then 82, 78, 86); four gain nothing where most strips have one tile or two (11.9, 11.2, 13.4).
+static int both_waves(const SparseAttn* a, const PatternIndex& pi, int nbr) {
+    const long long cus = device_cus(), tiles = (long long)pi.ntiles * a->NB, longest = std::max(pi.max_row_tiles, pi.max_col_tiles);
+    if (tiles > 80 * cus) return 0;
+    const double place = (double)tiles / (4 * cus);  // two passes over eight wavefronts per CU
+    if (longest > 5 * place && pi.ntiles > 2 * nbr) return 4;
+    return longest > 2 * place ? 2 : 1;
+}
+
 template <int D, bool VROW, bool ST = false>
 static void launch_tile_bwd(SparseAttn* a, const float* Q, const float* K, const float* Vt, const float* P,
                             const float* dO, float* dQ, float* dK, float* dV, const int* offs, int nnz,
@@ -1580,6 +1595,23 @@ static void launch_tile_bwd(SparseAttn* a, const float* Q, const float* K, const
         }
     } else {
         const int wv = pick_waves(a, pi, nbr, false);
+        if constexpr (D == 32 && VROW) {
+            // (a gradient written over what the other pass still reads needs the two launches one after the other)
+            const bool apart = dQ != ocache && dK != ocache && dV != ocache && dK != K && dV != K;
+            const int bw = a->bwd_passes == 3 && ocache && apart ? both_waves(a, pi, nbr) : 0;
+            if (bw > 0) {
+                PhaseRange range("spion backward: both passes (dQ, dK, dV)");
+#define SPION_BOTH(W)                                                                                                     \
+    hipLaunchKernelGGL((tile_bwd_both_kernel<W, ST>), dim3(2 * nbr * a->NB), dim3(64 * W), 0, a->hdr.stream, Q, K, Vt, P, \
+                       dO, ocache, dQ, dK, dV, pi.d_rdesc, pi.d_tcol, pi.d_cdesc, pi.d_tcdesc, a->L, nbr, a->NB, nnz,     \
+                       a->scale, hc, ly)
+                if (bw == 1) SPION_BOTH(1);
+                else if (bw == 2) SPION_BOTH(2);
+                else SPION_BOTH(4);
+#undef SPION_BOTH
+                return;
+            }
+        }
         if (a->bwd_passes & 1) {
             PhaseRange range("spion backward: row pass (dQ)");
             SPION_BY_WAVES(wv, SPION_ROWS, a->hdr.stream, 0, nbr);

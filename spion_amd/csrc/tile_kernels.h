@@ -1045,12 +1045,15 @@ void tile_fwd_kernel(
 // the 32 x d result.  G receives -g for the column pass.
 // -------------------------------------------------------------------------------------------------
 // VROW: the V operand is row-major [NB][L][D] instead of feature-major [NB][D][L].
-template <int D, int WAVES, bool HAVE_O, bool VROW = false, bool ST = false>
-SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
+template <int D, int WAVES>
+constexpr int tile_bwd_row_lds() { return WAVES * (1 + 2 * (D / 32)) * DmaTileF32::TILE; }
+// BOTH: the columns' strips run in the same launch (they form their own row sums; heads in the same order as theirs).
+template <int D, int WAVES, bool HAVE_O, bool VROW, bool ST, bool BOTH = false>
+__device__ __forceinline__ void tile_bwd_row_item(
     const float* __restrict__ K, const float* __restrict__ Vt, const float* __restrict__ P,
     const float* __restrict__ dO, const float* __restrict__ Ocache, float* __restrict__ G,
     float* __restrict__ dQ, const int* __restrict__ rdesc, const int* __restrict__ tcol,
-    int L, int nbr, int NB, int nnz, float scale, int hc, Layouts ly, int s0, int ns) {
+    int L, int nbr, int NB, int nnz, float scale, int hc, const Layouts& ly, int s0, int ns, int item, char* smem) {
     static_assert(!ST || (VROW && HAVE_O), "strided heads: row-major operands, Out given");
     constexpr int KH = D / 2;
     // LDS of a wavefront: the V, P and K tiles of one pattern tile, 4 KB per 32 features: 12 KB (d = 32, twelve
@@ -1059,16 +1062,14 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
     // a barrier.
     constexpr int WB = (1 + 2 * (D / 32)) * DmaTileF32::TILE;
     constexpr int RED = WAVES > 1 ? WAVES * (D / 32) * 16 * 64 * 4 : 0;
-    static_assert(RED <= WAVES * WB, "the reduction fits in the tile space");
-    __shared__ __attribute__((aligned(16))) char smem[WAVES * WB];
+    static_assert(RED <= WAVES * WB && WAVES * WB == tile_bwd_row_lds<D, WAVES>(), "the reduction fits in the tile space");
     float* lds = reinterpret_cast<float*>(smem);
     auto lds_g = [&](int ww) { return reinterpret_cast<float*>(smem + ww * WB + WB - 128); };
     // Last head first: the forward wrote P front to back, so its tail is what the memory-side cache still holds.
     // This launch covers strips s0 .. s0+ns-1 of every head's strip order.
-    const int item = xcd_remap(blockIdx.x, ns * NB);
     int bh, pos;
     item_to_head_strip(item, ns, hc, bh, pos);
-    bh = NB - 1 - bh;
+    if (!BOTH) bh = NB - 1 - bh;
     const int4 sd = reinterpret_cast<const int4*>(rdesc)[s0 + pos];  // strips longest first: {strip, first tile, tiles, P offset}
     const int I = sd.x, t0 = sd.y, cnt = sd.z;
     const int w = wave_index(), l = threadIdx.x & 63, h = l >> 5, li = l & 31;
@@ -1137,7 +1138,7 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
             __syncthreads();  // the partial sums lie where tiles are about to land
         }
     }
-    if (w == 0 && h == 0) G[(size_t)bh * L + I * 32 + li] = -g;
+    if (!BOTH && w == 0 && h == 0) G[(size_t)bh * L + I * 32 + li] = -g;
     const f32x16 gneg = splat16(-g);
 
     f32x16 acc[D / 32];
@@ -1256,6 +1257,16 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
     for (int c = 0; c < D / 32; ++c) acc[c] *= scale;
     reduce_store<D, WAVES>(acc, dQ + gb, I * 32, w, li, h, lds, gld);
 }
+template <int D, int WAVES, bool HAVE_O, bool VROW = false, bool ST = false>
+SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
+    const float* __restrict__ K, const float* __restrict__ Vt, const float* __restrict__ P,
+    const float* __restrict__ dO, const float* __restrict__ Ocache, float* __restrict__ G,
+    float* __restrict__ dQ, const int* __restrict__ rdesc, const int* __restrict__ tcol,
+    int L, int nbr, int NB, int nnz, float scale, int hc, Layouts ly, int s0, int ns) {
+    __shared__ __attribute__((aligned(16))) char smem[tile_bwd_row_lds<D, WAVES>()];
+    tile_bwd_row_item<D, WAVES, HAVE_O, VROW, ST>(K, Vt, P, dO, Ocache, G, dQ, rdesc, tcol, L, nbr, NB, nnz, scale, hc, ly, s0,
+                                                  ns, xcd_remap(blockIdx.x, ns * NB), smem);
+}
 
 // -------------------------------------------------------------------------------------------------
 // Backward, column pass, one work-group per (head, block column): dK_J = sum_I dS_IJ^T Q_I,
@@ -1263,24 +1274,28 @@ SPION_TILE_KERNEL(WAVES) void tile_bwd_row_kernel(
 // started from the stored -g, the 1/sqrt(d) of dK is applied to the 32 x d result.
 // -------------------------------------------------------------------------------------------------
 // VROW: as in the row pass.
-template <int D, int WAVES, bool VROW = false, bool ST = false>
-SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
+// OWN_G: G is Out, and the row sums g_i = dO_i . O_i of a tile's queries are formed here (d = 32).
+template <int D, int WAVES, bool OWN_G = false>
+constexpr int tile_bwd_col_lds() {
+    return WAVES * (D == 32 ? (OWN_G ? 4 : 3) * DmaTileF32::TILE + 256 : 5 * DmaTileF32::TILE);
+}
+template <int D, int WAVES, bool VROW, bool ST, bool OWN_G = false>
+__device__ __forceinline__ void tile_bwd_col_item(
     const float* __restrict__ Q, const float* __restrict__ Vt, const float* __restrict__ P,
     const float* __restrict__ dO, const float* __restrict__ G, float* __restrict__ dK, float* __restrict__ dV,
     const int* __restrict__ cdesc, const int* __restrict__ tcdesc, int L, int nbr, int NB, int nnz, float scale,
-    int hc, Layouts ly, int s0, int ns) {
+    int hc, const Layouts& ly, int s0, int ns, int item, char* smem) {
     static_assert(!ST || VROW, "strided heads: row-major operands");
+    static_assert(!OWN_G || D == 32);
     constexpr int KH = D / 2;
     // LDS of a wavefront: d = 32, the P, Q and dO tiles and 64 floats of -g; d = 64, the P tile and two tiles each for
     // Q and dO, 20 KB, which eight wavefronts per CU fill to the last byte: -g then travels in a register.  The
     // buffer of the final reductions lies inside the tile space, a barrier in between.
-    constexpr int WB = D == 32 ? 3 * DmaTileF32::TILE + 256 : 5 * DmaTileF32::TILE;
+    constexpr int WB = tile_bwd_col_lds<D, 1, OWN_G>();
     constexpr int RED = WAVES > 1 ? WAVES * (D / 32) * 16 * 64 * 4 : 0;
     static_assert(RED <= WAVES * WB, "the reduction fits in the tile space");
-    __shared__ __attribute__((aligned(16))) char smem[WAVES * WB];
     float* lds = reinterpret_cast<float*>(smem);
-    const int item = xcd_remap(blockIdx.x, ns * NB);  // strips s0 .. s0+ns-1 of every head's strip order
-    int bh, pos;
+    int bh, pos;  // (strips s0 .. s0+ns-1 of every head's strip order)
     item_to_head_strip(item, ns, hc, bh, pos);
     const int4 sd = reinterpret_cast<const int4*>(cdesc)[s0 + pos];  // strips longest first: {strip, first tile, tiles, 0}
     const int J = sd.x, e0 = sd.y, cnt = sd.z;
@@ -1292,7 +1307,7 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
     head_slice<ST, D>(ly.grad, ly.H, bh, L, gb, gld, gbytes);
     const rsrc_t rQ = make_rsrc(Q + ib, hbytes), rV = make_rsrc(Vt + ib, hbytes), rdO = make_rsrc(dO + ob, obytes);
     const rsrc_t rP = make_rsrc(P + (size_t)bh * nnz, (size_t)nnz * 4);
-    const rsrc_t rG = make_rsrc(G + (size_t)bh * L, (size_t)L * 4);
+    const rsrc_t rG = make_rsrc(G + (OWN_G ? 0 : (size_t)bh * L), (size_t)L * 4);
 
     auto load_vt = [&](float (&vt)[KH], int l) {
         if constexpr (VROW) ldr_rows<D>(rV, ((l & 31) * ild + (l >> 5) * KH) * 4, J * 32 * ild * 4, vt);
@@ -1324,11 +1339,12 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
         const char* Tp = reinterpret_cast<const char*>(T);
         const char* Tq = Tp + DmaTileF32::TILE;
         const char* To = Tp + 2 * DmaTileF32::TILE;
-        const char* Tg = Tp + 3 * DmaTileF32::TILE;
+        char* Tg = const_cast<char*>(Tp) + (OWN_G ? 4 : 3) * DmaTileF32::TILE;  // OWN_G: behind the tile of Out
         const unsigned lp = lds_address(Tp), lq = lp + DmaTileF32::TILE, lo = lp + 2 * DmaTileF32::TILE,
                        lg = lp + 3 * DmaTileF32::TILE;
         const u32x4 wQ = rsrc_words(Q + ib, hbytes), wO = rsrc_words(dO + ob, obytes);
-        const u32x4 wP = rsrc_words(P + (size_t)bh * nnz, (size_t)nnz * 4), wG = rsrc_words(G + (size_t)bh * L, (size_t)L * 4);
+        const u32x4 wP = rsrc_words(P + (size_t)bh * nnz, (size_t)nnz * 4);
+        const u32x4 wG = rsrc_words(G + (OWN_G ? ob : (size_t)bh * L), OWN_G ? obytes : (size_t)L * 4);
         const int ql = DmaTileF32::voff(l, ild), ol = DmaTileF32::voff(l, old_);
         const int qx = DmaTileF32::extra_step(ild), ox = DmaTileF32::extra_step(old_);
         const auto a_p = DmaTileF32::cols_addr(Tp, li, h);  // the Q tile's are 4 KB on
@@ -1339,11 +1355,12 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
         auto issue_pg = [&](const int4 d) {
             const int x = ST ? lane_again() : l;
             DmaTileF32::load<true>(wP, lp, 16 * ((x & 7) ^ (x >> 3)) + (x >> 3) * 4 * d.z, d.y * 4, DmaTileF32::extra_step(d.z));
-            dma_b32(wG, lg, x * 4, d.x * 128);
+            if constexpr (!OWN_G) dma_b32(wG, lg, x * 4, d.x * 128);
         };
         auto issue_qo = [&](const int4 d) {
             DmaTileF32::load(wQ, lq, ql, d.x * 32 * ild * 4, qx);
             DmaTileF32::load(wO, lo, ol, d.x * 32 * old_ * 4, ox);
+            if constexpr (OWN_G) DmaTileF32::load(wG, lg, ol, d.x * 32 * old_ * 4, ox);
         };
         if (nu > 0) {
             int4 dn = desc[w];
@@ -1356,6 +1373,14 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
                 float pc[16], qb[1][16], go[KH];
                 f32x16 init;
                 DmaTileF32::get(a_go, go);
+                if constexpr (OWN_G) {
+                    float oo[KH], g = 0.f;
+                    DmaTileF32::get(a_go, oo, DmaTileF32::TILE);
+#pragma unroll
+                    for (int s = 0; s < KH; ++s) g = fmaf(go[s], oo[s], g);
+                    g += __shfl_xor(g, 32, 64);
+                    reinterpret_cast<float*>(Tg)[l] = -g;  // (both halves hold it)
+                }
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const f32x4 v = *reinterpret_cast<const f32x4*>(a_g + 32 * g);
@@ -1554,6 +1579,39 @@ SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
     reduce_store<D, WAVES>(ak, dK + gb, J * 32, w, li, h, lds, gld);
     if (WAVES > 1) __syncthreads();
     reduce_store<D, WAVES>(av, dV + gb, J * 32, w, li, h, lds, gld);
+}
+template <int D, int WAVES, bool VROW = false, bool ST = false>
+SPION_TILE_KERNEL_D(WAVES, D) void tile_bwd_col_kernel(
+    const float* __restrict__ Q, const float* __restrict__ Vt, const float* __restrict__ P,
+    const float* __restrict__ dO, const float* __restrict__ G, float* __restrict__ dK, float* __restrict__ dV,
+    const int* __restrict__ cdesc, const int* __restrict__ tcdesc, int L, int nbr, int NB, int nnz, float scale,
+    int hc, Layouts ly, int s0, int ns) {
+    __shared__ __attribute__((aligned(16))) char smem[tile_bwd_col_lds<D, WAVES>()];
+    tile_bwd_col_item<D, WAVES, VROW, ST>(Q, Vt, P, dO, G, dK, dV, cdesc, tcdesc, L, nbr, NB, nnz, scale, hc, ly, s0, ns,
+                                          xcd_remap(blockIdx.x, ns * NB), smem);
+}
+
+// Both passes of a small backward in one launch (d = 32, row-major operands): the columns' strips form the row sums they need
+// themselves, from a tile of Out beside that of dO, so neither pass waits for the other.  Such a step is bound by latency: a
+// pass of 512 strips of four tiles takes 9 us wherever it runs, a launch's start, one strip's chain and the gap to the next.
+// A row's and a column's strip follow one another, so that what they share of P comes from the same L2.  Two wavefronts per
+// SIMD (176 registers, 16.25 KB of LDS a wavefront).  Backward at 8 x 2 heads of 1024, 4.3 tiles a strip: 21.0 -> 15.2 us; one
+// sample 18.7 -> 8.5; 64 x 2 heads 70 -> 67.
+template <int WAVES, bool ST>
+SPION_TILE_KERNEL(WAVES) void tile_bwd_both_kernel(
+    const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V, const float* __restrict__ P,
+    const float* __restrict__ dO, const float* __restrict__ Out, float* __restrict__ dQ, float* __restrict__ dK,
+    float* __restrict__ dV, const int* __restrict__ rdesc, const int* __restrict__ tcol, const int* __restrict__ cdesc,
+    const int* __restrict__ tcdesc, int L, int nbr, int NB, int nnz, float scale, int hc, Layouts ly) {
+    constexpr int RB = tile_bwd_row_lds<32, WAVES>(), CB = tile_bwd_col_lds<32, WAVES, true>();
+    __shared__ __attribute__((aligned(16))) char smem[RB > CB ? RB : CB];
+    const int item = xcd_remap(blockIdx.x, 2 * nbr * NB);
+    if (item & 1)
+        tile_bwd_row_item<32, WAVES, true, true, ST, true>(K, V, P, dO, Out, nullptr, dQ, rdesc, tcol, L, nbr, NB, nnz, scale, hc,
+                                                           ly, 0, nbr, item >> 1, smem);
+    else
+        tile_bwd_col_item<32, WAVES, true, ST, true>(Q, V, P, dO, Out, dK, dV, cdesc, tcdesc, L, nbr, NB, nnz, scale, hc, ly, 0,
+                                                     nbr, item >> 1, smem);
 }
 
 }  // namespace spion
