@@ -29,6 +29,10 @@ int spion_debug_counter(void* handle, int which);
  * device of so many compute units (host only: needs no device); -1 on bad arguments. */
 int spion_debug_remainder_by_ranges(int num_batches, int seq_len, long long entries, int compute_units);
 
+/* How many heads (a multiple of `unit`) of such a pattern are launched together, bytes_per_head of P and list between their
+ * launches; -1 for sizes that are not positive or heads that are not whole units.  Host logic. */
+int spion_debug_remainder_heads(int num_batches, int seq_len, int unit, double bytes_per_head, int compute_units);
+
 /* Whether the backward of row-major heads of a dense handle runs as work-groups that share their tiles on the current
  * device (1), or with four wavefronts to a strip (0); -1 for other handles. */
 int spion_debug_dense_groups(void* handle);

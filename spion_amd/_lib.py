@@ -110,6 +110,8 @@ def core() -> ctypes.CDLL:
     lib.spion_debug_counter.restype = c_int
     lib.spion_debug_remainder_by_ranges.argtypes = [c_int, c_int, ctypes.c_longlong, c_int]
     lib.spion_debug_remainder_by_ranges.restype = c_int
+    lib.spion_debug_remainder_heads.argtypes = [c_int, c_int, c_int, ctypes.c_double, c_int]
+    lib.spion_debug_remainder_heads.restype = c_int
     lib.spion_use_output_cache.argtypes = [_P, c_int]
     lib.spion_use_output_cache.restype = None
     lib.spion_attn_backward_with_out.argtypes = [_P] * 15 + [c_int]

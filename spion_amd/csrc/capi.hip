@@ -96,6 +96,7 @@ void sparse_force_element(void*, int);
 void sparse_set_bwd_passes(void*, int);
 int sparse_debug_counter(void*, int);
 int sparse_debug_rem_by_ranges(int, int, long long, int);
+int sparse_debug_hyb_heads(int, int, int, double, int);
 int sparse_debug_bf16_plan(const int*, int, int, int, int, int*, int, int*, int, int*, int, int*, int, int*);
 void sparse_use_ocache(void*, int);
 void* sparse_bf16_init(int, int, int, int);
@@ -402,6 +403,11 @@ int spion_debug_dense_groups(void* h) { return dense_groups(h); }
 int spion_debug_counter(void* h, int which) { return sparse_debug_counter(h, which); }
 int spion_debug_remainder_by_ranges(int num_batches, int seq_len, long long entries, int compute_units) {
     return num_batches > 0 && seq_len > 0 && compute_units > 0 ? sparse_debug_rem_by_ranges(num_batches, seq_len, entries, compute_units) : -1;
+}
+int spion_debug_remainder_heads(int num_batches, int seq_len, int unit, double bytes_per_head, int compute_units) {
+    return num_batches > 0 && seq_len > 0 && unit > 0 && num_batches % unit == 0 && compute_units > 0
+               ? sparse_debug_hyb_heads(num_batches, seq_len, unit, bytes_per_head, compute_units)
+               : -1;
 }
 int spion_debug_bf16_plan(const int* tile_ptr, int nstrips, int pairs, int num_batches, int lanes, int* items,
                           int cap_items, int* lane_ptr, int cap_ptr, int* lane_ent, int cap_ent, int* longs,

@@ -741,6 +741,22 @@ static bool rem_by_ranges(int NB, int L, long long nr, int cus) {
     const double ranges = (L + REM_RANGE - 1) / REM_RANGE, r = (double)nr / L;
     return 10 + rem_rounds(NB, L, cus).rounds * (11 * ranges + 0.8 * r) < (double)NB * L / (256.0 * cus) * (115 + 2.2 * r);
 }
+// Heads of an element pattern whose launches go one after the other before the next heads' (the remainder by ranges): what a
+// head's launches leave for each other, `bytes` of it -- its P and the remainder's list --, is then read from the memory-side
+// cache (256 MB) where all heads' would pass through memory.  The fewest groups of at most 192 MB, else the smallest, as long as
+// they take no more rounds of work-groups than all heads at once; a multiple of `unit` heads (a sample, where heads of one share
+// their key mask or are strided).  64 heads of 4096 with 205 entries a row: 867 -> 836 us, probabilities 75 -> 61, the rest
+// 3 % less; 128: 1758, in two groups 1748, in four 1717.  In four groups of 16, twice the rounds, 64 heads take 1000.
+static int hyb_heads(int NB, int L, int unit, double bytes, int cus) {
+    const double rounds = rem_rounds(NB, L, cus).rounds;
+    int best = NB;
+    for (int groups = 2; best * bytes > 192e6 && groups <= rounds; ++groups) {  // (a group takes a round or more)
+        const int n = ((NB + groups - 1) / groups + unit - 1) / unit * unit;
+        if ((NB / n) * rem_rounds(n, L, cus).rounds + (NB % n ? rem_rounds(NB % n, L, cus).rounds : 0) <= rounds) best = n;
+    }
+    return best;
+}
+int sparse_debug_hyb_heads(int NB, int L, int unit, double bytes, int cus) { return hyb_heads(NB, L, unit, bytes, cus); }
 int sparse_debug_rem_by_ranges(int NB, int L, long long nr, int cus) { return rem_by_ranges(NB, L, nr, cus); }
 // SPION_HYB_GATHER: never by ranges
 static bool rem_gather_forced() {
@@ -1653,48 +1669,46 @@ static int elem_lds_columns(const SparseAttn* a) {
 #define SPION_ELEM_COL_LDS(ST_, NC_, ...)                                                                       \
     hipLaunchKernelGGL((elem_bwd_col_lds_kernel<ST_, NC_>), dim3(a->NB * hyb_groups(a->L, 128 * NC_)),          \
                        dim3(HYB_CL_THREADS), 0, a->hdr.stream, __VA_ARGS__)
-#define SPION_REM_LAUNCH(KERNEL_, NO_, ...)                                                                                 \
-    hipLaunchKernelGGL((KERNEL_), dim3(a->NB * hyb_groups(a->L, (NO_) * REM_QUADS)), dim3(REM_THREADS), 0, a->hdr.stream, \
+#define SPION_REM_LAUNCH(KERNEL_, NO_, ...)                                                                              \
+    hipLaunchKernelGGL((KERNEL_), dim3(nh * hyb_groups(a->L, (NO_) * REM_QUADS)), dim3(REM_THREADS), 0, a->hdr.stream, \
                        __VA_ARGS__)
+
+// Where head h0 (the first of a sample, for strided heads) begins
+template <bool ST>
+static size_t head_base(const SparseAttn* a, const HeadLayout& y, int H, int h0) {
+    return ST ? (size_t)(h0 / H) * y.bstride : (size_t)h0 * a->L * a->d;
+}
 
 // Hybrid patterns (dense tiles + remainder, d = 32).  Every operand row-major; ST: heads located by `ly`.
 // ocopy (contiguous heads only): where a second copy of O goes, or null.
+// The launches of nh heads.
 template <bool ST>
-static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const float* V, const KeyTerms& Mask,
-                           float* Attn, float* Out, float* ocopy, const int* Offsets, int nnz, const Layouts& ly,
-                           HybForwardWork work) {
-    PhaseRange phase("spion forward (hybrid kernels)");
-    // the remainder's raw logits between the first and the third launch: a compact list of their own (written and
-    // read in full lines) rather than their places inside P, where every four-byte store would pull in a line
-    if (!work.raw) {
-        if (!ensure_ws(&a->ws_stats, (size_t)a->NB * a->L * 2)) return;
-        if (!ensure_ws_grow(a, &a->ws_raw, &a->ws_raw_count, rem_list(a), "attn_forward")) return;
-        work = HybForwardWork{reinterpret_cast<float2*>(a->ws_stats), a->ws_raw};
-    }
-    a->last_path = a->pat.hyb_dense ? 3 : 2;
+static void launch_hyb_fwd_heads(SparseAttn* a, int nh, const float* Q, const float* K, const float* V, const KeyTerms& Mask,
+                                 float* Attn, float* Out, float* ocopy, const int* Offsets, int nnz, const Layouts& ly,
+                                 const HybForwardWork& work) {
     const int nbr = a->L / 32;
-    const long long rows = (long long)a->NB * a->L;
+    const long long rows = (long long)nh * a->L;
     // strips of few dense tiles: one wavefront walks the whole strip; else four share it
     const bool one = a->pat.max_row_tiles <= HYB_MAXT1;
-    const dim3 grid_t(nbr * a->NB), block_t(one ? 64 : 256);
+    const dim3 grid_t(nbr * nh), block_t(one ? 64 : 256);
     const dim3 grid_g((unsigned)((rows + HYB_GWAVES - 1) / HYB_GWAVES)), block_g(64 * HYB_GWAVES);
     float2* stats = work.stats;
     float* raw = work.raw;
-    const bool lds = a->pat.rem_lds, two = lds && rem_rounds(a->NB, a->L, device_cus()).per_quad == 2;
+    const bool lds = a->pat.rem_lds, two = lds && rem_rounds(nh, a->L, device_cus()).per_quad == 2;
 #define SPION_HYB_TILES(MASKED, WAVES_, MAXT_, REM_)                                                                  \
     hipLaunchKernelGGL((hyb_tile_fwd_kernel<MASKED, WAVES_, MAXT_, ST, REM_>), grid_t, block_t, 0, a->hdr.stream, Q,  \
-                       K, V, Mask, Attn, Out, REM_ ? ocopy : nullptr, stats, Offsets, a->pat.hyb, a->L, nbr, a->NB,   \
+                       K, V, Mask, Attn, Out, REM_ ? ocopy : nullptr, stats, Offsets, a->pat.hyb, a->L, nbr, nh,      \
                        nnz, a->scale, ly)
 #define SPION_REM_FWD(MASKED, NO_)                                                                                     \
     SPION_REM_LAUNCH((rem_fwd_kernel<MASKED, ST, NO_>), NO_, Q, K, V, Mask, raw, stats, Out, a->pat.rem, a->L, \
-                     a->NB, a->scale, ly)
+                     nh, a->scale, ly)
 #define SPION_HYB_FWD(MASKED)                                                                                        \
     do {                                                                                                             \
         if (two) SPION_REM_FWD(MASKED, 2);                                                                           \
         else if (lds) SPION_REM_FWD(MASKED, 1);                                                                      \
         else                                                                                                         \
             hipLaunchKernelGGL((hyb_rem_logits_kernel<MASKED, ST>), grid_g, block_g, 0, a->hdr.stream, Q, K, Mask,   \
-                               raw, stats, a->pat.hyb, a->L, a->NB, a->scale, ly);                                   \
+                               raw, stats, a->pat.hyb, a->L, nh, a->scale, ly);                                   \
         if (one && lds) SPION_HYB_TILES(MASKED, 1, HYB_MAXT1, true);                                                 \
         else if (one) SPION_HYB_TILES(MASKED, 1, HYB_MAXT1, false);                                                  \
         else if (lds) SPION_HYB_TILES(MASKED, 4, HYB_MAXT4, true);                                                   \
@@ -1709,14 +1723,83 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
 #undef SPION_HYB_TILES
     if (lds)
         hipLaunchKernelGGL(rem_prob_kernel, grid_t, dim3(REM_PROB_THREADS), 0, a->hdr.stream, (const float*)raw, Attn,
-                           (const float2*)stats, Offsets, a->pat.rem, a->L, nbr, a->NB, nnz);
+                           (const float2*)stats, Offsets, a->pat.rem, a->L, nbr, nh, nnz);
     else
         hipLaunchKernelGGL(hyb_rem_pv_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, V, (const float*)raw, Attn,
-                           Out, ocopy, (const float2*)stats, a->pat.hyb, a->L, a->NB, nnz, ly);
+                           Out, ocopy, (const float2*)stats, a->pat.hyb, a->L, nh, nnz, ly);
+}
+template <bool ST>
+static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const float* V, const KeyTerms& Mask,
+                           float* Attn, float* Out, float* ocopy, const int* Offsets, int nnz, const Layouts& ly,
+                           HybForwardWork work) {
+    PhaseRange phase("spion forward (hybrid kernels)");
+    // the remainder's raw logits between the first and the third launch: a compact list of their own (written and
+    // read in full lines) rather than their places inside P, where every four-byte store would pull in a line
+    if (!work.raw) {
+        if (!ensure_ws(&a->ws_stats, (size_t)a->NB * a->L * 2)) return;
+        if (!ensure_ws_grow(a, &a->ws_raw, &a->ws_raw_count, rem_list(a), "attn_forward")) return;
+        work = HybForwardWork{reinterpret_cast<float2*>(a->ws_stats), a->ws_raw};
+    }
+    a->last_path = a->pat.hyb_dense ? 3 : 2;
+    const int per = a->pat.rem_lds ? hyb_heads(a->NB, a->L, ST ? ly.H : a->has_mask ? Mask.heads : 1,
+                                               4.0 * ((double)nnz + a->pat.hyb_nr), device_cus())
+                                   : a->NB;
+    for (int h0 = 0; h0 < a->NB; h0 += per) {
+        const size_t in = head_base<ST>(a, ly.in, ly.H, h0), out = head_base<ST>(a, ly.out, ly.H, h0);
+        KeyTerms mask = Mask;
+        if (a->has_mask) mask.p = Mask.row(h0, a->L);
+        launch_hyb_fwd_heads<ST>(a, std::min(per, a->NB - h0), Q + in, K + in, V + in, mask, Attn + (size_t)h0 * nnz, Out + out,
+                                 ocopy ? ocopy + out : nullptr, Offsets, nnz, ly, work);
+    }
     check_launch("hybrid forward kernels");
 }
 
 // o: the forward's output (same layout as dO).
+template <bool ST>
+static void launch_hyb_bwd_heads(SparseAttn* a, int nh, const float* Q, const float* K, const float* V, const float* P,
+                                 const float* dO, const float* o, float* rowsum, float2* pairs, float* dQ, float* dK, float* dV,
+                                 const int* Offsets, int nnz, const Layouts& ly) {
+    const int nbr = a->L / 32;
+    const long long rows = (long long)nh * a->L;
+    const bool one_r = a->pat.max_row_tiles <= 2 * HYB_MAXT1, one_c = a->pat.max_col_tiles <= 2 * HYB_MAXT1;
+    const dim3 grid_t(nbr * nh);
+    const dim3 grid_g((unsigned)((rows + HYB_GWAVES - 1) / HYB_GWAVES)), block_g(64 * HYB_GWAVES);
+    const bool lds = a->pat.rem_lds, two = lds && rem_rounds(nh, a->L, device_cus()).per_quad == 2;
+    if (a->bwd_passes & 1) {
+        if (one_r)
+            hipLaunchKernelGGL((hyb_tile_bwd_row_kernel<1, ST>), grid_t, dim3(64), 0, a->hdr.stream, K, V, P, dO, o,
+                               rowsum, dQ, a->pat.hyb, a->L, nbr, nh, nnz, a->scale, ly);
+        else
+            hipLaunchKernelGGL((hyb_tile_bwd_row_kernel<4, ST>), grid_t, dim3(256), 0, a->hdr.stream, K, V, P, dO, o,
+                               rowsum, dQ, a->pat.hyb, a->L, nbr, nh, nnz, a->scale, ly);
+#define SPION_REM_ROW(NO_)                                                                                            \
+    SPION_REM_LAUNCH((rem_bwd_row_kernel<ST, NO_>), NO_, K, V, P, dO, (const float*)rowsum, pairs, dQ, Offsets, \
+                     a->pat.rem, a->L, nh, nnz, a->scale, ly)
+        if (two) SPION_REM_ROW(2);
+        else if (lds) SPION_REM_ROW(1);
+        else
+            hipLaunchKernelGGL(hyb_rem_bwd_row_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, K, V, P, dO,
+                               (const float*)rowsum, pairs, dQ, a->pat.hyb, a->L, nh, nnz, a->scale, ly);
+#undef SPION_REM_ROW
+    }
+    if (a->bwd_passes & 2) {
+        if (one_c)
+            hipLaunchKernelGGL((hyb_tile_bwd_col_kernel<1, ST>), grid_t, dim3(64), 0, a->hdr.stream, Q, V, P, dO,
+                               (const float*)rowsum, dK, dV, a->pat.hyb, a->L, nbr, nh, nnz, a->scale, ly);
+        else
+            hipLaunchKernelGGL((hyb_tile_bwd_col_kernel<4, ST>), grid_t, dim3(256), 0, a->hdr.stream, Q, V, P, dO,
+                               (const float*)rowsum, dK, dV, a->pat.hyb, a->L, nbr, nh, nnz, a->scale, ly);
+#define SPION_REM_COL(NO_)                                                                                          \
+    SPION_REM_LAUNCH((rem_bwd_col_kernel<ST, NO_>), NO_, Q, dO, (const float2*)pairs, dK, dV, a->pat.rem, a->L, nh, \
+                     ly)
+        if (two) SPION_REM_COL(2);
+        else if (lds) SPION_REM_COL(1);
+        else
+            hipLaunchKernelGGL(hyb_rem_bwd_col_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, Q, dO,
+                               (const float2*)pairs, dK, dV, a->pat.hyb, a->L, nh, ly);
+#undef SPION_REM_COL
+    }
+}
 template <bool ST>
 static void launch_hyb_bwd(SparseAttn* a, const float* Q, const float* K, const float* V, const float* P,
                            const float* dO, const float* o, const HybBackwardWork& work, float* dQ, float* dK, float* dV,
@@ -1726,45 +1809,15 @@ static void launch_hyb_bwd(SparseAttn* a, const float* Q, const float* K, const 
     float* rowsum = work.rowsum ? work.rowsum : a->ws_rowsum;
     float2* pairs = work.pairs;
     a->last_path = a->pat.hyb_dense ? 3 : 2;
-    const int nbr = a->L / 32;
-    const long long rows = (long long)a->NB * a->L;
-    const bool one_r = a->pat.max_row_tiles <= 2 * HYB_MAXT1, one_c = a->pat.max_col_tiles <= 2 * HYB_MAXT1;
-    const dim3 grid_t(nbr * a->NB);
-    const dim3 grid_g((unsigned)((rows + HYB_GWAVES - 1) / HYB_GWAVES)), block_g(64 * HYB_GWAVES);
-    const bool lds = a->pat.rem_lds, two = lds && rem_rounds(a->NB, a->L, device_cus()).per_quad == 2;
-    if (a->bwd_passes & 1) {
-        if (one_r)
-            hipLaunchKernelGGL((hyb_tile_bwd_row_kernel<1, ST>), grid_t, dim3(64), 0, a->hdr.stream, K, V, P, dO, o,
-                               rowsum, dQ, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
-        else
-            hipLaunchKernelGGL((hyb_tile_bwd_row_kernel<4, ST>), grid_t, dim3(256), 0, a->hdr.stream, K, V, P, dO, o,
-                               rowsum, dQ, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
-#define SPION_REM_ROW(NO_)                                                                                            \
-    SPION_REM_LAUNCH((rem_bwd_row_kernel<ST, NO_>), NO_, K, V, P, dO, (const float*)rowsum, pairs, dQ, Offsets, \
-                     a->pat.rem, a->L, a->NB, nnz, a->scale, ly)
-        if (two) SPION_REM_ROW(2);
-        else if (lds) SPION_REM_ROW(1);
-        else
-            hipLaunchKernelGGL(hyb_rem_bwd_row_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, K, V, P, dO,
-                               (const float*)rowsum, pairs, dQ, a->pat.hyb, a->L, a->NB, nnz, a->scale, ly);
-#undef SPION_REM_ROW
-    }
-    if (a->bwd_passes & 2) {
-        if (one_c)
-            hipLaunchKernelGGL((hyb_tile_bwd_col_kernel<1, ST>), grid_t, dim3(64), 0, a->hdr.stream, Q, V, P, dO,
-                               (const float*)rowsum, dK, dV, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
-        else
-            hipLaunchKernelGGL((hyb_tile_bwd_col_kernel<4, ST>), grid_t, dim3(256), 0, a->hdr.stream, Q, V, P, dO,
-                               (const float*)rowsum, dK, dV, a->pat.hyb, a->L, nbr, a->NB, nnz, a->scale, ly);
-#define SPION_REM_COL(NO_)                                                                                          \
-    SPION_REM_LAUNCH((rem_bwd_col_kernel<ST, NO_>), NO_, Q, dO, (const float2*)pairs, dK, dV, a->pat.rem, a->L, a->NB, \
-                     ly)
-        if (two) SPION_REM_COL(2);
-        else if (lds) SPION_REM_COL(1);
-        else
-            hipLaunchKernelGGL(hyb_rem_bwd_col_kernel<ST>, grid_g, block_g, 0, a->hdr.stream, Q, dO,
-                               (const float2*)pairs, dK, dV, a->pat.hyb, a->L, a->NB, ly);
-#undef SPION_REM_COL
+    // (a pass by itself finds the sums and pairs of all heads)
+    const int per = a->pat.rem_lds && a->bwd_passes == 3
+                        ? hyb_heads(a->NB, a->L, ST ? ly.H : 1, 4.0 * ((double)nnz + 2.0 * a->pat.hyb_nr), device_cus())
+                        : a->NB;
+    for (int h0 = (a->NB - 1) / per * per; h0 >= 0; h0 -= per) {  // the forward's last heads are what the cache still holds
+        const size_t in = head_base<ST>(a, ly.in, ly.H, h0), out = head_base<ST>(a, ly.out, ly.H, h0);
+        const size_t gr = head_base<ST>(a, ly.grad, ly.H, h0);
+        launch_hyb_bwd_heads<ST>(a, std::min(per, a->NB - h0), Q + in, K + in, V + in, P + (size_t)h0 * nnz, dO + out, o + out,
+                                 rowsum, pairs, dQ + gr, dK + gr, dV + gr, Offsets, nnz, ly);
     }
     check_launch("hyb_bwd kernels");
 }
