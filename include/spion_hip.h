@@ -400,7 +400,8 @@ void spion_dense_backward_strided(void* handle, const float* Q, const float* K, 
  * walk over the map, the work-groups' parts of dQ lying in the scratch and nothing in the handle.
  *   spion_dense_scratch  floats a backward can use (0: none; -1: an error)
  *   scratch              16-byte aligned, contents unspecified, the caller's again when the call's work on the handle's stream
- *                        has ended; null or one that is too small: the call is spion_dense_backward_strided. */
+ *                        has ended; null or one that is too small, or dK or dV over K, V or Out: the call is
+ *                        spion_dense_backward_strided. */
 long long spion_dense_scratch(void* handle);
 void spion_dense_backward_scratch(void* handle, const float* Q, const float* K, const float* V, const float* P,
                                   const float* Out, const float* dO, float* dQ, float* dK, float* dV, int heads,

@@ -1613,7 +1613,11 @@ void dense_backward_strided(void* h, const float* Q, const float* K, const float
     ly.grad = grad;
     ly.H = heads;
     const int nbr = a->L / 32;
-    if (const size_t need = dense_fused_floats(a); need && scratch.p && scratch.floats >= need) {
+    // (a gradient written over what other work-groups of the one walk, or the addition behind it, still read needs the passes)
+    const long long gs = layout_span(grad, a->NB / heads, heads, a->L, a->d), is = layout_span(in, a->NB / heads, heads, a->L, a->d),
+                    os = layout_span(out, a->NB / heads, heads, a->L, a->d);
+    auto over = [&](const float* g) { return spans_meet(g, gs, K, is) || spans_meet(g, gs, V, is) || spans_meet(g, gs, Out, os); };
+    if (const size_t need = dense_fused_floats(a); need && scratch.p && scratch.floats >= need && !over(dK) && !over(dV)) {
         const int G = dense_fused_strips(a), C = (nbr + G - 1) / G;
         if (G == 8)
             hipLaunchKernelGGL(dense_group_col_dq_kernel<8>, dim3(C * a->NB), dim3(64 * 8), 0, a->hdr.stream, Q, K, V, P, dO, Out,

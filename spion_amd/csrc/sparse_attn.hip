@@ -1545,6 +1545,12 @@ static int both_waves(const SparseAttn* a, const PatternIndex& pi, int nbr) {
     return longest > 2 * place ? 2 : 1;
 }
 
+// Floats that a tensor of all heads spans
+template <bool ST>
+static long long head_span(const SparseAttn* a, const HeadLayout& y, int H) {
+    return ST ? layout_span(y, a->NB / H, H, a->L, a->d) : (long long)a->NB * a->L * a->d;
+}
+
 template <int D, bool VROW, bool ST = false>
 static void launch_tile_bwd(SparseAttn* a, const float* Q, const float* K, const float* Vt, const float* P,
                             const float* dO, float* dQ, float* dK, float* dV, const int* offs, int nnz,
@@ -1613,8 +1619,11 @@ static void launch_tile_bwd(SparseAttn* a, const float* Q, const float* K, const
         const int wv = pick_waves(a, pi, nbr, false);
         if constexpr (D == 32 && VROW) {
             // (a gradient written over what the other pass still reads needs the two launches one after the other)
-            const bool apart = dQ != ocache && dK != ocache && dV != ocache && dK != K && dV != K;
-            const int bw = a->bwd_passes == 3 && ocache && apart ? both_waves(a, pi, nbr) : 0;
+            const long long in = head_span<ST>(a, ly.in, ly.H), out = head_span<ST>(a, ly.out, ly.H), gr = head_span<ST>(a, ly.grad, ly.H);
+            auto over = [&](const float* g) { return spans_meet(g, gr, K, in) || spans_meet(g, gr, Vt, in); };
+            auto over_out = [&](const float* g) { return spans_meet(g, gr, ocache, out); };
+            const bool apart = ocache && !over(dK) && !over(dV) && !over_out(dQ) && !over_out(dK) && !over_out(dV);
+            const int bw = a->bwd_passes == 3 && apart ? both_waves(a, pi, nbr) : 0;
             if (bw > 0) {
                 PhaseRange range("spion backward: both passes (dQ, dK, dV)");
 #define SPION_BOTH(W)                                                                                                     \
@@ -1809,15 +1818,20 @@ static void launch_hyb_bwd(SparseAttn* a, const float* Q, const float* K, const 
     float* rowsum = work.rowsum ? work.rowsum : a->ws_rowsum;
     float2* pairs = work.pairs;
     a->last_path = a->pat.hyb_dense ? 3 : 2;
-    // (a pass by itself finds the sums and pairs of all heads)
-    const int per = a->pat.rem_lds && a->bwd_passes == 3
+    // (a pass by itself finds the sums and pairs of all heads; a gradient over an operand may lie over that of a head still to come)
+    const long long in = head_span<ST>(a, ly.in, ly.H), out = head_span<ST>(a, ly.out, ly.H), gr = head_span<ST>(a, ly.grad, ly.H);
+    bool apart = true;
+    for (const float* g : {dQ, dK, dV})
+        apart = apart && !spans_meet(g, gr, Q, in) && !spans_meet(g, gr, K, in) && !spans_meet(g, gr, V, in) && !spans_meet(g, gr, dO, out) &&
+                !spans_meet(g, gr, o, out) && !spans_meet(g, gr, P, (long long)a->NB * nnz);
+    const int per = a->pat.rem_lds && a->bwd_passes == 3 && apart
                         ? hyb_heads(a->NB, a->L, ST ? ly.H : 1, 4.0 * ((double)nnz + 2.0 * a->pat.hyb_nr), device_cus())
                         : a->NB;
     for (int h0 = (a->NB - 1) / per * per; h0 >= 0; h0 -= per) {  // the forward's last heads are what the cache still holds
-        const size_t in = head_base<ST>(a, ly.in, ly.H, h0), out = head_base<ST>(a, ly.out, ly.H, h0);
-        const size_t gr = head_base<ST>(a, ly.grad, ly.H, h0);
-        launch_hyb_bwd_heads<ST>(a, std::min(per, a->NB - h0), Q + in, K + in, V + in, P + (size_t)h0 * nnz, dO + out, o + out,
-                                 rowsum, pairs, dQ + gr, dK + gr, dV + gr, Offsets, nnz, ly);
+        const size_t i0 = head_base<ST>(a, ly.in, ly.H, h0), o0 = head_base<ST>(a, ly.out, ly.H, h0);
+        const size_t g0 = head_base<ST>(a, ly.grad, ly.H, h0);
+        launch_hyb_bwd_heads<ST>(a, std::min(per, a->NB - h0), Q + i0, K + i0, V + i0, P + (size_t)h0 * nnz, dO + o0, o + o0,
+                                 rowsum, pairs, dQ + g0, dK + g0, dV + g0, Offsets, nnz, ly);
     }
     check_launch("hyb_bwd kernels");
 }

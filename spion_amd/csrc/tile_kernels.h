@@ -544,6 +544,12 @@ struct Layouts {
     HeadLayout in, out, grad;
     int H;
 };
+// Host side: what `n` floats at x and `m` floats at y span has an address in common; layout_span: the floats from a [B][H][L][d] view's
+// first element to its last.
+inline bool spans_meet(const float* x, long long n, const float* y, long long m) { return x < y + m && y < x + n; }
+inline long long layout_span(const HeadLayout& y, int B, int H, int L, int d) {
+    return (B - 1) * y.bstride + (long long)(H - 1) * y.hstride + (long long)(L - 1) * y.ld + d;
+}
 // Host side: true when no two elements of a [B][H][L][d] view with this layout share an address (required of every
 // tensor the kernels write).  Heads either follow one another as whole blocks or are interleaved inside the rows.
 inline bool layout_is_injective(const HeadLayout& y, int B, int H, int L, int d) {

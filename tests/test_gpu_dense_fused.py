@@ -104,7 +104,7 @@ def test_one_walk_near_the_smallest_floats_and_a_small_row():
     compare_by_element(one, p.detach()[0], out.detach()[0], [x.grad[0] for x in leaves], d)
 
 
-def test_calls_without_enough_scratch_run_the_two_passes():
+def test_calls_without_enough_scratch_or_over_an_operand_run_the_two_passes():
     core, NB, L, d = _lib.core(), 100, 288, 32
     gen = torch.Generator(device="cuda").manual_seed(0)
     q, k, v, do = _heads(NB, 1, L, d, "plain", 4, gen)
@@ -118,17 +118,21 @@ def test_calls_without_enough_scratch_run_the_two_passes():
     assert floats == 2 * NB * L * d
     scratch = torch.empty(floats, device="cuda")
 
-    def backward(*tail):
-        grads = [torch.empty_like(q) for _ in range(3)]
+    def backward(*tail, dk=None, dv=None):  # (which operand the gradient lies over)
+        at = {"k": k.clone(), "v": v.clone(), "out": out.clone()}
+        grads = [torch.empty_like(q), at.get(dk, torch.empty_like(q)), at.get(dv, torch.empty_like(q))]
         call = core.spion_dense_backward_scratch if tail else core.spion_dense_backward_strided
-        call(h, q.data_ptr(), k.data_ptr(), v.data_ptr(), attn.data_ptr(), out.data_ptr(), do.data_ptr(),
+        call(h, q.data_ptr(), at["k"].data_ptr(), at["v"].data_ptr(), attn.data_ptr(), at["out"].data_ptr(), do.data_ptr(),
              *(g.data_ptr() for g in grads), 1, lay, lay, lay, *tail)
         _lib.check_error()
+        torch.cuda.synchronize()
         return grads
 
     passes = backward()
     for tail in ((None, 0), (scratch.data_ptr(), floats - 1), (scratch.data_ptr() + 4, floats)):
         assert all(torch.equal(x, y) for x, y in zip(backward(*tail), passes))
+    for over in ({"dk": "k"}, {"dk": "v"}, {"dk": "out"}, {"dv": "k"}, {"dv": "v"}, {"dv": "out"}):
+        assert all(torch.equal(x, y) for x, y in zip(backward(scratch.data_ptr(), floats, **over), passes))
     walk = backward(scratch.data_ptr(), floats)
     assert not torch.equal(walk[0], passes[0])  # (dQ is summed in another order)
     for x, y in zip(walk, passes):

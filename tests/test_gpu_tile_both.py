@@ -81,9 +81,9 @@ def test_a_gradient_over_an_operand_runs_one_pass_after_the_other():
     out, p = abi.forward_rowmajor(q, k, v)
 
     def backward(over):
-        at = {"out": out.clone(), "k": k.clone()}
+        at = {"out": out.clone(), "k": k.clone(), "v": v.clone()}
         grads = [at[over[n]] if n in over else torch.empty_like(q) for n in ("dq", "dk", "dv")]
-        ptr = [t.data_ptr() for t in (q, at["k"], v, p, at["out"], do)]
+        ptr = [t.data_ptr() for t in (q, at["k"], at["v"], p, at["out"], do)]
         names = _kernels(lambda: core.spion_attn_backward_rowmajor(
             abi.handle, *ptr, None, *(t.data_ptr() for t in grads), abi.offsets.data_ptr(), abi.columns.data_ptr(),
             abi.sum_mat.data_ptr(), abi.nnz))
@@ -92,7 +92,7 @@ def test_a_gradient_over_an_operand_runs_one_pass_after_the_other():
 
     names, plain = backward({})
     assert "tile_bwd_both_kernel" in names
-    for over in ({"dq": "out"}, {"dk": "out"}, {"dv": "out"}, {"dk": "k"}, {"dv": "k"}):
+    for over in ({"dq": "out"}, {"dk": "out"}, {"dv": "out"}, {"dk": "k"}, {"dv": "k"}, {"dk": "v"}, {"dv": "v"}):
         names, got = backward(over)
         assert "tile_bwd_row_kernel" in names and "tile_bwd_both_kernel" not in names
         for x, y in zip(got, plain):  # sums of at most L + d + 3 roundings each in another order
