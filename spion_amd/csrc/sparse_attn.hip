@@ -805,11 +805,20 @@ static bool analyse_pattern(SparseAttn* a, const int* Offsets, const int* Column
         set_error("pattern: Offsets[0]=%d, Offsets[L]=%d do not match nnz=%d", off[0], off[L], nnz);
         return false;
     }
-    for (int i = 0; i < L; ++i) {
+    for (int i = 0; i < L; ++i)
         if (off[i + 1] < off[i]) {
             set_error("pattern: Offsets not monotone at row %d", i);
             return false;
         }
+    // A row is in range when its columns increase and its ends are: a loop that vectorises (entry by entry, this was most of the
+    // first call on a pattern); the entries are looked at one by one only to report what is wrong.
+    auto in_order = [&](int b, int e) {
+        int bad = 0;
+        for (int k = b + 1; k < e; ++k) bad |= col[k] <= col[k - 1];
+        return !bad && (b == e || (col[b] >= 0 && col[e - 1] < L));
+    };
+    for (int i = 0; i < L; ++i) {
+        if (in_order(off[i], off[i + 1])) continue;
         for (int k = off[i]; k < off[i + 1]; ++k) {
             if (col[k] < 0 || col[k] >= L) {
                 set_error("pattern: column %d out of range at row %d", col[k], i);

@@ -128,6 +128,27 @@ def test_handle_keeps_several_patterns_and_registration_from_host():
     abi.close()
 
 
+@pytest.mark.parametrize("at,value,message", [
+    (0, -1, "column -1 out of range at row 0"), (-1, 128, "column 128 out of range at row 127"),
+    (-1, 0, "columns of row 127 are not strictly increasing"), (40, 200, "column 200 out of range at row"),
+    (33, -(2 ** 31), "column -2147483648 out of range at row"), (None, None, "Offsets not monotone at row 6")])
+def test_a_malformed_index_is_refused_with_its_first_fault(at, value, message):
+    L, bs, core = 128, 32, _lib.core()
+    abi = SparseABI(32, L, 1, bs, with_mask=False)
+    off, col = (np.array(x, dtype=np.int32) for x in osa.build_csr_from_block_mask(np.eye(L // bs, dtype=np.float32), bs)[1:])
+    if at is None:
+        off[6], off[7] = off[7], off[6]
+    else:
+        col[at] = value
+    dev = [torch.from_numpy(x).cuda() for x in (off, col)]
+    assert core.spion_register_pattern(abi.handle, *(t.data_ptr() for t in dev), len(col), off.ctypes.data, col.ctypes.data) != 0
+    assert message.encode() in core.spion_handle_error(abi.handle)
+    core.spion_clear_handle_error(abi.handle)
+    with pytest.raises(_lib.SpionLibraryError):
+        _lib.check_error()
+    abi.close()
+
+
 def test_kept_output_copy_is_dropped_by_forwards_that_do_not_refresh_it():
     """A forward through the reference ABI files a copy of Out under its P buffer.  A later forward that fills the
     same P buffer without refreshing the copy (strided heads) must drop it: the reference-ABI backward then
