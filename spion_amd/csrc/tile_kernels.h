@@ -1353,14 +1353,18 @@ __device__ __forceinline__ void tile_bwd_col_item(
         const u32x4 wG = rsrc_words(G + (OWN_G ? ob : (size_t)bh * L), OWN_G ? obytes : (size_t)L * 4);
         const int ql = DmaTileF32::voff(l, ild), ol = DmaTileF32::voff(l, old_);
         const int qx = DmaTileF32::extra_step(ild), ox = DmaTileF32::extra_step(old_);
+        const int pl0 = 16 * ((l & 7) ^ (l >> 3)), pl1 = (l >> 3) * 4;
         const auto a_p = DmaTileF32::cols_addr(Tp, li, h);  // the Q tile's are 4 KB on
         const auto a_go = DmaTileF32::own_addr(To, li, 4 * h, 1);
         const char* a_g = Tg + 16 * h;
-        // (Strided heads have two lane offsets in ql and ol; the ones made here are then the registers over 168, and waiting for
-        // the reload of a spilled one is waiting for the tiles in flight: 32 x 2 heads of 4096 165 -> 160 us, 64 x 2 of 1024 38.2 -> 36.6.)
+        // Contiguous heads keep the lane offset into a P tile (pl0 + pl1 * row stride; made anew, they keep one register more than
+        // there is and reload it: column pass of 4 heads of 8192, a tenth kept, 50 -> 53 us).  Strided heads have two lane offsets
+        // in ql and ol and make it where it is used: the ones kept would be the registers over 168, and waiting for the reload of
+        // a spilled one is waiting for the tiles in flight (32 x 2 heads of 4096 165 -> 160 us, 64 x 2 of 1024 38.2 -> 36.6).
         auto issue_pg = [&](const int4 d) {
             const int x = ST ? lane_again() : l;
-            DmaTileF32::load<true>(wP, lp, 16 * ((x & 7) ^ (x >> 3)) + (x >> 3) * 4 * d.z, d.y * 4, DmaTileF32::extra_step(d.z));
+            const int po = ST ? 16 * ((x & 7) ^ (x >> 3)) + (x >> 3) * 4 * d.z : pl0 + pl1 * d.z;
+            DmaTileF32::load<true>(wP, lp, po, d.y * 4, DmaTileF32::extra_step(d.z));
             if constexpr (!OWN_G) dma_b32(wG, lg, x * 4, d.x * 128);
         };
         auto issue_qo = [&](const int4 d) {
