@@ -783,9 +783,12 @@ void tile_fwd_kernel(
     };
     if constexpr (MAXT > 0) {
       if (FALLBACK && cnt > MAXT * WAVES) {
-        // Nothing shared with the other branch, whose registers are full: with q shared, the strided kernels at d = 64 spilled 57
-        // registers, and a reload of one waits for all loads in flight (24 heads of 4000 110 -> 86 us, 64 of 2048 with a sixth of the
-        // blocks and key mask 161 -> 114; contiguous heads, which had room, as before).
+        // Nothing shared with the other branch, whose registers are full.  With q shared, six tiles of strided heads at d = 64 spilled
+        // 57 registers, and a reload of one waits for all loads in flight (24 heads of 4000 110 -> 86 us, 64 of 2048 with a sixth
+        // of the blocks and key mask 161 -> 114); 38 are left (27 with key mask), one or two of which are reloaded in the loop over
+        // the register tiles.  Contiguous heads had room for q: with a key mask they spill one to three registers more than with
+        // it, outside their loops (64 of 2048, a sixth of the blocks, 124 -> 126 us, 24 of 4000 and 128 of 1024 level); both layouts
+        // take the same way, because the split of a q scaled in the same block rounds once less, and so differently.
         const int l2 = second_walk(l);
         float q2[KH];
         load_q(q2, l2);
