@@ -26,6 +26,7 @@
 #include <initializer_list>
 #include <cmath>
 #include <cstdlib>
+#include <numeric>
 #include <queue>
 #include <vector>
 
@@ -1759,9 +1760,11 @@ static void launch_hyb_fwd(SparseAttn* a, const float* Q, const float* K, const 
         work = HybForwardWork{reinterpret_cast<float2*>(a->ws_stats), a->ws_raw};
     }
     a->last_path = a->pat.hyb_dense ? 3 : 2;
-    const int per = a->pat.rem_lds ? hyb_heads(a->NB, a->L, ST ? ly.H : a->has_mask ? Mask.heads : 1,
-                                               4.0 * ((double)nnz + a->pat.hyb_nr), device_cus())
-                                   : a->NB;
+    // (a group starts with a sample of the layout and with a row of the mask, whose heads the caller gives by themselves)
+    const long long unit = std::lcm(ST ? (long long)ly.H : 1ll, a->has_mask ? (long long)Mask.heads : 1ll);
+    const int per = a->pat.rem_lds && unit < a->NB
+                        ? hyb_heads(a->NB, a->L, (int)unit, 4.0 * ((double)nnz + a->pat.hyb_nr), device_cus())
+                        : a->NB;
     for (int h0 = 0; h0 < a->NB; h0 += per) {
         const size_t in = head_base<ST>(a, ly.in, ly.H, h0), out = head_base<ST>(a, ly.out, ly.H, h0);
         KeyTerms mask = Mask;
