@@ -1270,6 +1270,7 @@ static bool ensure_ws_grow(SparseAttn* a, float** p, size_t* have, size_t need, 
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+static bool all_aligned16(std::initializer_list<const void*> ps) { return std::all_of(ps.begin(), ps.end(), aligned16); }
 
 // Whether a call on a hybrid pattern takes the hybrid kernels, and what their launches leave for each other (null: in the
 // handle).  The remainder's kernels by ranges load 16 bytes a lane.  Where the element kernels would do as well (few entries in
@@ -1288,10 +1289,7 @@ static size_t hyb_forward_floats(const SparseAttn* a) { return 2 * (size_t)a->NB
 static size_t hyb_backward_floats(const SparseAttn* a) { return (size_t)a->NB * a->L + 2 * rem_list(a); }
 static bool take_hybrid(const SparseAttn* a, std::initializer_list<const void*> operands) {
     if (!a->pat.hybrid) return false;
-    if (!a->pat.rem_lds) return true;
-    for (const void* p : operands)
-        if (!aligned16(p)) return false;
-    return true;
+    return !a->pat.rem_lds || all_aligned16(operands);
 }
 static bool take_hybrid_forward(const SparseAttn* a, std::initializer_list<const void*> operands, const CallScratch& scratch,
                                 HybForwardWork* work) {
@@ -1301,10 +1299,12 @@ static bool take_hybrid_forward(const SparseAttn* a, std::initializer_list<const
     work->raw = scratch.p + 2 * (size_t)a->NB * a->L;
     return true;
 }
-// dS: [NB][nnz] floats, which hold the pairs of a pattern at least half of which lies in dense tiles; or null.
-static bool take_hybrid_backward(const SparseAttn* a, std::initializer_list<const void*> operands, float* dS,
-                                 const CallScratch& scratch, HybBackwardWork* work) {
-    if (!take_hybrid(a, operands)) return false;
+// dS: [NB][nnz] floats, which hold the pairs of a pattern at least half of which lies in dense tiles; or null.  tiles: Q, K, V and
+// dO, which the tiles' passes take from memory into LDS 16 bytes a lane, whichever kernels the remainder has.
+static bool take_hybrid_backward(const SparseAttn* a, std::initializer_list<const void*> tiles,
+                                 std::initializer_list<const void*> others, float* dS, const CallScratch& scratch,
+                                 HybBackwardWork* work) {
+    if (!take_hybrid(a, others) || !all_aligned16(tiles)) return false;
     if (scratch.floats < hyb_backward_floats(a)) {
         work->pairs = reinterpret_cast<float2*>(dS);
         return a->pat.hyb_dense && dS;
@@ -2022,7 +2022,7 @@ void sparse_backward(void* h, const float* Q, const float* K, const float* Vt, c
         // without it the gather kernels below serve the same P
         const float* o = Out ? Out : ocache_for_backward(a, P);
         HybBackwardWork work;
-        if (o && take_hybrid_backward(a, {Q, K, Vrm, dO, o, dQ, dK, dV}, dS, scratch, &work)) {
+        if (o && take_hybrid_backward(a, {Q, K, Vrm, dO}, {o, dQ, dK, dV}, dS, scratch, &work)) {
             launch_hyb_bwd<false>(a, Q, K, Vrm, P, dO, o, work, dQ, dK, dV, Offsets, nnz, Layouts{});
             return;
         }
@@ -2255,7 +2255,7 @@ void sparse_backward_strided(void* h, const float* Q, const float* K, const floa
         if (!callers && !ensure_ws_grow(a, &a->ws_ds, &a->ws_ds_count, ds_floats, who)) return;
         float* ds = callers ? scratch.p : a->ws_ds;
         HybBackwardWork work;
-        if (take_hybrid_backward(a, {Q, K, V, dO, Out, dQ, dK, dV}, ds, callers ? scratch : CallScratch{}, &work)) {
+        if (take_hybrid_backward(a, {Q, K, V, dO}, {Out, dQ, dK, dV}, ds, callers ? scratch : CallScratch{}, &work)) {
             launch_hyb_bwd<true>(a, Q, K, V, P, dO, Out, work, dQ, dK, dV, Offsets, nnz, ly);
             return;
         }
