@@ -1628,11 +1628,12 @@ static void launch_tile_bwd(SparseAttn* a, const float* Q, const float* K, const
     } else {
         const int wv = pick_waves(a, pi, nbr, false);
         if constexpr (D == 32 && VROW) {
-            // (a gradient written over what the other pass still reads needs the two launches one after the other)
+            // (a gradient written over what the other pass still reads needs the two launches one after the other; so does an Out
+            // off 16 bytes, which the row pass reads into registers and the columns' strips of the one launch into LDS)
             const long long in = head_span<ST>(a, ly.in, ly.H), out = head_span<ST>(a, ly.out, ly.H), gr = head_span<ST>(a, ly.grad, ly.H);
             auto over = [&](const float* g) { return spans_meet(g, gr, K, in) || spans_meet(g, gr, Vt, in); };
             auto over_out = [&](const float* g) { return spans_meet(g, gr, ocache, out); };
-            const bool apart = ocache && !over(dK) && !over(dV) && !over_out(dQ) && !over_out(dK) && !over_out(dV);
+            const bool apart = ocache && aligned16(ocache) && !over(dK) && !over(dV) && !over_out(dQ) && !over_out(dK) && !over_out(dV);
             const int bw = a->bwd_passes == 3 && apart ? both_waves(a, pi, nbr) : 0;
             if (bw > 0) {
                 PhaseRange range("spion backward: both passes (dQ, dK, dV)");

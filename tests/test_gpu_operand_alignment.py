@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from spion_amd import _lib
+from spion_amd import _lib, workloads
 from tests.abi_utils import SparseABI
 from tests.test_gpu_split_products import EPS, _csr
 
@@ -62,5 +62,17 @@ def test_tiles_of_element_patterns(which):
     assert "hyb_tile_bwd" in names
     names, got = _backward(abi, {**t, which: _off(t[which])})
     assert "hyb_tile_bwd" not in names
+    _close(got, want, L)
+    abi.close()
+
+
+def test_output_of_a_small_tile_pattern():
+    """Out enters the one launch of both passes as tiles, the two launches row by row."""
+    L, bs = 512, 32
+    abi, t = _step(L, 6, workloads.band_random_block_mask(L // bs, 1, density=0.25, seed=1), bs)
+    names, want = _backward(abi, t)
+    assert "tile_bwd_both_kernel" in names
+    names, got = _backward(abi, {**t, "out": _off(t["out"])})
+    assert "tile_bwd_row_kernel" in names and "tile_bwd_both_kernel" not in names
     _close(got, want, L)
     abi.close()
