@@ -1617,7 +1617,17 @@ void dense_backward_strided(void* h, const float* Q, const float* K, const float
     const long long gs = layout_span(grad, a->NB / heads, heads, a->L, a->d), is = layout_span(in, a->NB / heads, heads, a->L, a->d),
                     os = layout_span(out, a->NB / heads, heads, a->L, a->d);
     auto over = [&](const float* g) { return spans_meet(g, gs, K, is) || spans_meet(g, gs, V, is) || spans_meet(g, gs, Out, os); };
+    const size_t rowsum_bytes = sizeof(float) * (size_t)a->NB * a->L;
     if (const size_t need = dense_fused_floats(a); need && scratch.p && scratch.floats >= need && !over(dK) && !over(dV)) {
+        if (!a->ws_rowsum) {
+            // What the passes hand on is there after any first backward, as without scratch: a later one that is recorded into a
+            // graph and has none, or lies over an operand, cannot allocate it.
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(a->hdr.stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+                hipMalloc((void**)&a->ws_rowsum, rowsum_bytes) != hipSuccess)
+                a->ws_rowsum = nullptr;
+            (void)hipGetLastError();
+        }
         const int G = dense_fused_strips(a), C = (nbr + G - 1) / G;
         if (G == 8)
             hipLaunchKernelGGL(dense_group_col_dq_kernel<8>, dim3(C * a->NB), dim3(64 * 8), 0, a->hdr.stream, Q, K, V, P, dO, Out,
@@ -1630,7 +1640,7 @@ void dense_backward_strided(void* h, const float* Q, const float* K, const float
         check_launch("dense_bwd kernels");
         return;
     }
-    if (!a->ws_rowsum && !SPION_HIP_OK(hipMalloc((void**)&a->ws_rowsum, sizeof(float) * (size_t)a->NB * a->L))) return;
+    if (!a->ws_rowsum && !SPION_HIP_OK(hipMalloc((void**)&a->ws_rowsum, rowsum_bytes))) return;
     const dim3 grid(nbr * a->NB), block4(64 * 4);
     if (dense_groups_fill(a)) {
         const int G = a->d / 8;
