@@ -398,7 +398,8 @@ void spion_dense_backward_strided(void* handle, const float* Q, const float* K, 
                                   const spion_head_layout* grad);
 /* The same backward in scratch of the caller's: launches that fill the machine (emb_dim 32) then take dQ, dK and dV from one
  * walk over the map, the work-groups' parts of dQ lying in the scratch and nothing in the handle.
- *   spion_dense_scratch  floats a backward can use (0: none; -1: an error)
+ *   spion_dense_scratch  floats a backward can use (0: none; -1: an error): an eighth or a quarter of the map's, rounded up to
+ *                        whole groups of eight or four strips of 32 keys
  *   scratch              16-byte aligned, contents unspecified, the caller's again when the call's work on the handle's stream
  *                        has ended; null or one that is too small, or dK or dV over K, V or Out: the call is
  *                        spion_dense_backward_strided. */

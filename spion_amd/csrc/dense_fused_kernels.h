@@ -5,8 +5,8 @@
 // Why: the row pass and the column pass read the map, 4 L^2 bytes a head, once each and form dO.V^T twice; together they take
 // three operand splits a tile (dS' twice, P).  Here a tile is read once, dS' is formed and split once -- its parts go through LDS
 // to change sides for the product with K -- and the row sums g come from the operand tiles as they are split, so nothing is
-// handed from launch to launch but the parts: ceil(L / 32 G) of [L][32] a head, 4 or 2 bytes written and read per G * 32 of the
-// map's.
+// handed from launch to launch but the parts: ceil(L / 32 G) of [L][32] a head, a quarter (G = 4) or an eighth (G = 8) of the map's
+// bytes, written once and read once.
 // A step (one tile of 32 queries for all G strips) has two barriers: before the first one the products dO.V^T, P^T.dO and K^T.dS'^T,
 // each wavefront by itself; between them the G partial tiles of dQ are added, the next operand tile is split, and the product
 // dS'^T.Q, whose operands are in registers by then, keeps the matrix pipe busy meanwhile.
