@@ -782,10 +782,11 @@ def bench_sparse_layer(args, dev, workload, full=True):
     t_fwd_abi = _event_ms(fwd, it)
     t_bwd_abi = _event_ms(bwd, it)
     t_seq_abi = _event_ms(lambda: (fwd(), bwd()), it)  # the order a training step runs them in
-    # the three kernels as the module launches them
+    # the kernels as the module launches them
     core.spion_use_output_cache(handle, 0)
     t_fwd = _event_ms(fwd_rm, it)
     t_bwd = _event_ms(bwd_rm, it)
+    one_launch = path == 1 and core.spion_debug_counter(handle, 4) == 1  # small calls: both passes of the backward
     t_seq = _event_ms(lambda: (fwd_rm(), bwd_rm()), it)
     core.spion_set_backward_passes(handle, 1)
     t_row = _event_ms(bwd_rm, it)
@@ -807,17 +808,23 @@ def bench_sparse_layer(args, dev, workload, full=True):
              3: ranges if by_ranges else ("hyb_rem_logits_kernel + hyb_tile_fwd_kernel + hyb_rem_pv_kernel",
                                           "hyb_tile_bwd_row_kernel + hyb_rem_bwd_row_kernel",
                                           "hyb_tile_bwd_col_kernel + hyb_rem_bwd_col_kernel")}[path]
-    kernels = dict(zip(names, (t_fwd, t_row, t_col)))
+    if one_launch:
+        names = ("tile_fwd_kernel", "tile_bwd_both_kernel")
+    kernels = dict(zip(names, (t_fwd, t_bwd) if one_launch else (t_fwd, t_row, t_col)))
     dom = max(kernels, key=kernels.get)
     dom_ms = kernels[dom]
     floors = {}
     if path == 1:
         # the matrix pipes a kernel's products run on against the bytes it cannot do without: P once, and Q, K, V, O / K, V,
-        # dO, O, dQ / Q, V, dO, dK, dV
-        ceiling = {k_: _matrix_ceiling(*p) for k_, p in zip(names, _TILE_PRODUCTS[d])}
-        nbytes = {k_: 4.0 * (t_ * L * d + nnz) * NB for k_, t_ in zip(names, (4, 5, 5))}
-        floors = {k_: _floors_ms(third, ceiling[k_], nbytes[k_]) for k_ in names}
-        roof = _roof_of(dom, dom_ms, third, ceiling[dom], nbytes[dom])
+        # dO, O, dQ / Q, V, dO, dK, dV (both passes: all eight)
+        products, tensors, thirds = _TILE_PRODUCTS[d], (4, 5, 5), (1, 1, 1)
+        if one_launch:
+            products, tensors, thirds = (products[0], tuple(map(sum, zip(*products[1:])))), (4, 8), (1, 2)
+        flops = {k_: n * third for k_, n in zip(names, thirds)}
+        ceiling = {k_: _matrix_ceiling(*p, 2 * n) for k_, p, n in zip(names, products, thirds)}
+        nbytes = {k_: 4.0 * (t_ * L * d + nnz) * NB for k_, t_ in zip(names, tensors)}
+        floors = {k_: _floors_ms(flops[k_], ceiling[k_], nbytes[k_]) for k_ in names}
+        roof = _roof_of(dom, dom_ms, flops[dom], ceiling[dom], nbytes[dom])
     else:
         # element path: HBM-bound by design; the slowest kernel's share of the algorithmic bytes
         share = {names[0]: 4.0 * (4 * L * d + nnz) * NB, names[1]: 4.0 * (4 * L * d + nnz) * NB,

@@ -22,7 +22,8 @@ void spion_set_backward_passes(void* handle, int mask);
  * waited for the stream), which = 1 -> analyses made from host arrays (spion_register_pattern), which = 2 ->
  * workspace buffers that a larger pattern has outgrown and that stay allocated until the handle is destroyed (a HIP
  * graph recorded before the growth still points at them), which = 3 -> 1 if the remainder of the pattern last used goes by
- * ranges whose rows lie in LDS.  -1 otherwise. */
+ * ranges whose rows lie in LDS, which = 4 -> 1 if the last backward over a pattern of tiles ran both passes in one launch.  -1
+ * otherwise. */
 int spion_debug_counter(void* handle, int which);
 
 /* Whether the library lets the remainder of an element pattern (`entries` a head) go by ranges (1) or gathers it (0), on a

@@ -499,6 +499,7 @@ struct SparseAttn {
     // recorded earlier on this handle has their addresses in its kernel nodes and may still be replayed.
     std::vector<void*> retired;
     int last_path = 0;
+    bool last_bwd_both = false;  // the last backward over tiles ran both passes in one launch
     bool is_bf16 = false;  // handle of the bf16 family: tile patterns only, P is never materialised
     bool force_element = false;
     int bwd_passes = 3;  // bit 0: row pass (g, dQ), bit 1: column pass (dK, dV); profiling only
@@ -1572,6 +1573,7 @@ static void launch_tile_bwd(SparseAttn* a, const float* Q, const float* K, const
     const int nbr = a->L / 32;
     const int hc = heads_per_group(a);
     const float* ocache = Out ? Out : ocache_for_backward(a, P);
+    a->last_bwd_both = false;
     // A pattern with a few strips far longer than the rest (global rows, global columns): those run four wavefronts
     // to a strip in a small launch of their own, all other strips in a launch with the wavefront count their own
     // number calls for -- instead of four wavefronts to every strip of the pattern because of the few.  The large
@@ -1636,6 +1638,7 @@ static void launch_tile_bwd(SparseAttn* a, const float* Q, const float* K, const
             const bool apart = ocache && aligned16(ocache) && !over(dK) && !over(dV) && !over_out(dQ) && !over_out(dK) && !over_out(dV);
             const int bw = a->bwd_passes == 3 && apart ? both_waves(a, pi, nbr) : 0;
             if (bw > 0) {
+                a->last_bwd_both = true;
                 PhaseRange range("spion backward: both passes (dQ, dK, dV)");
 #define SPION_BOTH(W)                                                                                                     \
     hipLaunchKernelGGL((tile_bwd_both_kernel<W, ST>), dim3(2 * nbr * a->NB), dim3(64 * W), 0, a->hdr.stream, Q, K, Vt, P, \
@@ -2642,7 +2645,8 @@ int sparse_debug_counter(void* h, int which) {
     SparseAttn* a = as_sparse(h, "spion_debug_counter");
     if (!a) return -1;
     return which == 0 ? a->analyses_from_device : which == 1 ? a->analyses_from_host
-         : which == 2 ? (int)a->retired.size() : which == 3 ? (int)a->pat.rem_lds : -1;
+         : which == 2 ? (int)a->retired.size() : which == 3 ? (int)a->pat.rem_lds
+         : which == 4 ? (int)a->last_bwd_both : -1;
 }
 void sparse_set_bwd_passes(void* h, int mask) {
     SparseAttn* a = as_sparse(h, "spion_set_backward_passes");

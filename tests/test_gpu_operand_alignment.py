@@ -71,8 +71,9 @@ def test_output_of_a_small_tile_pattern():
     L, bs = 512, 32
     abi, t = _step(L, 6, workloads.band_random_block_mask(L // bs, 1, density=0.25, seed=1), bs)
     names, want = _backward(abi, t)
-    assert "tile_bwd_both_kernel" in names
+    assert "tile_bwd_both_kernel" in names and _lib.core().spion_debug_counter(abi.handle, 4) == 1
     names, got = _backward(abi, {**t, "out": _off(t["out"])})
     assert "tile_bwd_row_kernel" in names and "tile_bwd_both_kernel" not in names
+    assert _lib.core().spion_debug_counter(abi.handle, 4) == 0
     _close(got, want, L)
     abi.close()
