@@ -747,8 +747,8 @@ static bool rem_by_ranges(int NB, int L, long long nr, int cus) {
 // head's launches leave for each other, `bytes` of it -- its P and the remainder's list --, is then read from the memory-side
 // cache (256 MB) where all heads' would pass through memory.  The fewest groups of at most 192 MB, else the smallest, as long as
 // they take no more rounds of work-groups than all heads at once; a multiple of `unit` heads (a sample, where heads of one share
-// their key mask or are strided).  64 heads of 4096 with 205 entries a row: 867 -> 836 us, probabilities 75 -> 61, the rest
-// 3 % less; 128: 1758, in two groups 1748, in four 1717.  In four groups of 16, twice the rounds, 64 heads take 1000.
+// their key mask or are strided).  64 heads of 4096 with 205 entries a row, a step: 880 -> 857 us, of which the probabilities
+// 75 -> 61; 128: 1758, in two groups 1748, in four 1717.  In four groups of 16, twice the rounds, 64 heads take 1000.
 static int hyb_heads(int NB, int L, int unit, double bytes, int cus) {
     const double rounds = rem_rounds(NB, L, cus).rounds;
     int best = NB;
